@@ -198,8 +198,9 @@ class GroupLimitedMoE(nn.Module):
     Router logits are an fp32 product; scores ``sigmoid(z)``; experts form ``groups`` equal groups of
     neighbours, a group is scored by the sum of its two best experts, only the ``keep`` best groups are
     eligible and the ``top`` best eligible experts are used, weighted by their own scores (no
-    renormalisation).  Token copies are sorted by expert and run through per-expert GEMMs on
-    contiguous segments (the dispatch of :class:`MoEMLP`); the weighted sum is accumulated in fp32."""
+    renormalisation).  On GPUs in bf16 the whole layer runs on the device (:func:`llmctl.ops.hybrid.routed_experts`);
+    otherwise token copies are sorted by expert and run through per-expert GEMMs on contiguous segments (the dispatch
+    of :class:`MoEMLP`).  The weighted sum is accumulated in fp32."""
 
     def __init__(self, width: int, ff: int, experts: int, top: int, groups: int, keep: int, device=None, dtype=None):
         super().__init__()
@@ -220,6 +221,9 @@ class GroupLimitedMoE(nn.Module):
         from llmctl.ops import hybrid as hops
 
         T = x.shape[0]
+        if hops.experts_ok(x, self.experts_up, self.experts_down, self.E, self.top):
+            return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, self.experts_up,
+                                       self.experts_down, "swiglu")
         topi, topw = hops.group_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.top,
                                             self.groups, self.keep)
         flat = topi.reshape(-1)
@@ -242,8 +246,9 @@ class BiasedSoftmaxMoE(nn.Module):
     outputs are experts without weights whose output is their input; ``shared_gate``: the shared expert's output is
     multiplied by ``sigmoid(w_sg . h)``, one number per token, whose row rides on the shared up projection;
     ``select_bias=False``: there is no selection bias.  The experts' down weights are one matrix ``[width, experts * ff]``.
-    Dispatch as in :class:`GroupLimitedMoE`
-    (token copies sorted by expert, per-expert GEMMs on contiguous segments, fp32 weighted sum).  Steps of
+    In bf16 on GPUs the layer runs on the device as a whole (:func:`llmctl.ops.hybrid.routed_experts`: no host
+    synchronisation, one grouped product per projection).  Otherwise (fp32, the CPU, widths that are no multiples of 8): dispatch as in
+    :class:`GroupLimitedMoE` (token copies sorted by expert, per-expert GEMMs on contiguous segments, fp32 weighted sum).  Steps of
     few tokens that between them reach about every expert anyway (decode batches) take the dense form
     instead: all experts on all rows in one up GEMM, one activation pass that multiplies every expert's activations by
     its routing weight (zero for the unchosen ones), and one down GEMM over all experts' activations side by side,
@@ -340,6 +345,14 @@ class BiasedSoftmaxMoE(nn.Module):
                 return hops.glu_act(u, "silu", scale)
             return hops.act_any(u, self.act, scale)
 
+        z = None if self.w_sup is None else torch.nn.functional.linear(x, self.w_sup, self.b_sup)
+        ys = torch.nn.functional.linear(act(z[:, :self.sup_rows]), self.w_sdown) if self.shared_ff else None
+        gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
+        down = self.w_down.view(x.shape[1], self.E, self.ff).transpose(0, 1)  # [E, width, ff]
+        if hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top):
+            out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
+                                      self.act, ys, gate)
+            return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out
         topi, topw = hops.bias_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.bias, self.top,
                                            self.groups, self.keep, self.renorm)
         if self._dense(T):
@@ -368,17 +381,11 @@ class BiasedSoftmaxMoE(nn.Module):
                     ye = torch.cat([ye, xs[real:tok.shape[0]]], 0)
             w = topw.reshape(-1).index_select(0, order).unsqueeze(-1)
             out = torch.zeros(T, x.shape[1], dtype=torch.float32, device=x.device).index_add_(0, tok, ye.float() * w)
-        side = None
-        if self.w_sup is not None:
-            z = torch.nn.functional.linear(x, self.w_sup, self.b_sup)
-            if self.shared_ff:
-                ys = torch.nn.functional.linear(act(z[:, :self.sup_rows]), self.w_sdown)
-                if self.shared_gate:
-                    out = hops.gated_add_f32_(out, ys, z[:, self.sup_rows:self.sup_rows + 1])
-                else:
-                    out += ys
-            side = z[:, self.sup_rows + (1 if self.shared_gate else 0):]
-        return (out, side) if self.side else out
+        if gate is not None:
+            out = hops.gated_add_f32_(out, ys, gate)
+        elif ys is not None:
+            out += ys
+        return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out
 
 
 def expert_param_global_name(name: str, module_e0: int) -> str:

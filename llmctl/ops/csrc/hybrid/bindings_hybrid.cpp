@@ -47,6 +47,10 @@ void mlstm_chunk_combine(const at::Tensor& S, const at::Tensor& n, const at::Ten
 std::tuple<at::Tensor, at::Tensor> group_topk_router(const at::Tensor& logits, int64_t top, int64_t groups, int64_t keep);
 std::tuple<at::Tensor, at::Tensor> bias_topk_router(const at::Tensor& logits, const c10::optional<at::Tensor>& bias, int64_t top, int64_t groups,
                                                     int64_t keep, bool renorm);
+std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t top,
+                                             int64_t groups, int64_t keep, bool softmax, bool renorm);
+at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
+                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate);
 std::tuple<at::Tensor, at::Tensor> hc_embed_norm(const at::Tensor& ids, const at::Tensor& table, int64_t streams, const at::Tensor& c_in,
                                                  const at::Tensor& g, double eps, bool out_bf16);
 at::Tensor hc_update_norm_(at::Tensor X, const at::Tensor& y1, double s1, const c10::optional<at::Tensor>& y2, double s2, const at::Tensor& mix,
@@ -141,6 +145,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("delta_chunk_combine(Tensor(a!) S, Tensor slots, Tensor start, Tensor base, Tensor loc, Tensor P, Tensor(b!) init) -> ()");
   m.def("gated_norm_add_norm_f32_(Tensor(a!) x, Tensor y, Tensor r, Tensor w_post, Tensor? w_next, float eps, bool out_bf16) -> Tensor");
   m.def("embed_rmsnorm_f32(Tensor ids, Tensor pos, Tensor table, Tensor pos_table, Tensor w, float eps, bool out_bf16) -> (Tensor, Tensor)");
+  m.def("moe_route(Tensor x, Tensor w, Tensor? bias, int top, int groups, int keep, bool softmax, bool renorm) -> (Tensor, Tensor)");
+  m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
   m.def("qk_fullnorm_prep(Tensor z, int H, int G, int dk, int dv, Tensor q_norm, Tensor k_norm, float eps, Tensor pos, float temp_coef, int temp_every, Tensor(a!) cache, Tensor slots, Tensor? freq=None, int rot=0, bool interleaved=False, float amp=1.0) -> Tensor");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, float qscale, Tensor(a!) S, Tensor slots, Tensor cu, Tensor start, Tensor(b!)? logd=None, bool write_out=True, bool write_state=True) -> Tensor");
@@ -185,6 +191,8 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("bias_topk_router", &llmctl_hybrid::bias_topk_router);
   m.impl("gated_norm_add_norm_f32_", &llmctl_hybrid::gated_norm_add_norm_f32_);
   m.impl("embed_rmsnorm_f32", &llmctl_hybrid::embed_rmsnorm_f32);
+  m.impl("moe_route", &llmctl_hybrid::moe_route);
+  m.impl("moe_experts", &llmctl_hybrid::moe_experts);
   m.impl("act_any", &llmctl_hybrid::act_any);
   m.impl("qk_fullnorm_prep", &llmctl_hybrid::qk_fullnorm_prep);
   m.impl("gla_scan", &llmctl_hybrid::gla_scan);

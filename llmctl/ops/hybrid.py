@@ -364,6 +364,35 @@ def bias_topk_router(logits, bias, top: int, groups: int = 1, keep: int = 1, ren
     return ref.bias_topk_router(logits, bias, top, groups, keep, renorm)
 
 
+_EXPERT_ACTS = {"relu2": 0, "swiglu": 1, "gelu": 2}
+MAX_EXPERTS = 128  # the expert kernels take the weights' addresses as arguments
+
+
+def experts_ok(x, up, down, outputs: int, top: int = 1) -> bool:
+    """Whether :func:`routed_experts` takes these operands: bf16 GPU rows and weights, widths in multiples of 8 with rows aligned
+    to 16 bytes, at most 128 router outputs, of which at most 64 are chosen.  ``up`` / ``down``: one ``[E, rows, K]`` tensor or a list of ``[rows, K]`` ones."""
+    if not (use_native(x) and x.dtype == torch.bfloat16 and x.dim() == 2 and outputs <= MAX_EXPERTS and top <= 64):
+        return False
+    ups, downs = ([w] if torch.is_tensor(w) else list(w) for w in (up, down))
+    return (x.shape[1] % 8 == 0 and downs[0].shape[-1] % 8 == 0
+            and all(t.dtype == torch.bfloat16 and t.is_cuda and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+                    and all(v % 8 == 0 for v in t.stride()[:-1]) for t in [x] + ups + downs)
+            and all(w.stride() == ws[0].stride() for ws in (ups, downs) for w in ws))
+
+
+def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax: bool, renorm: bool, up, down, act: str, shared=None,
+                   gate=None):
+    """``sum_k w_k expert_k(x_t)`` over the chosen experts of every row of ``x [T, W]`` (bf16) -> fp32 ``[T, W]``, all on the device:
+    router (fp32 scores of the fp32 ``w_router [E, W]``; ``softmax``: :func:`bias_topk_router`'s choice, else
+    :func:`group_topk_router`'s), copies grouped by expert, grouped products, weighted sum.  ``act``: ``relu2`` / ``gelu`` / ``swiglu``
+    (``up`` holds ``[gate ; up]``).  Router outputs beyond the experts are experts that give their input.  ``shared [T, W]`` (times
+    ``sigmoid(gate [T, 1])`` if given) is added.  Operands: :func:`experts_ok`."""
+    nat = native_hybrid()
+    idx, wgt = nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
+    return nat.moe_experts(x, idx, wgt, [up] if torch.is_tensor(up) else list(up), [down] if torch.is_tensor(down) else list(down),
+                           _EXPERT_ACTS[act], shared, gate)
+
+
 def act_any(x, kind: str, scale=None):
     """Elementwise activation of ``x`` (bf16 or fp32, computed in fp32): ``relu2`` = relu(x)^2, ``gelu`` = the
     exact (erf) GELU; ``scale`` (fp32 ``[rows]``): a factor per row."""

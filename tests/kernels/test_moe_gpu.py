@@ -1,0 +1,101 @@
+"""Grouped expert kernels (``llmctl/ops/csrc/hybrid/moe.hip``) against the same layer in float64, at the edges of
+their tiles: single rows, the last small step (64 tokens) and the first tiled one, partial row and column tiles, K tails,
+experts that nobody chose and one that everybody chose, experts without weights, gated shared experts."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(T, W, ff, E, act, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(T, W, generator=g).bfloat16()
+    router = torch.randn(E, W, generator=g) * W ** -0.5
+    rows = 2 * ff if act == "swiglu" else ff
+    up = (torch.randn(E, rows, W, generator=g) * W ** -0.5).bfloat16()
+    down = (torch.randn(W, E * ff, generator=g) * ff ** -0.5).bfloat16()
+    return x.cuda(), router.cuda(), up.cuda(), down.cuda()
+
+
+def _plain(x, idx, w, up, down, act, E):
+    x, up, down = x.double(), up.double(), down.double()
+    out = torch.zeros_like(x)
+    ff = down.shape[-1]
+    for e in range(E):
+        t, k = (idx == e).nonzero(as_tuple=True)
+        u = x[t] @ up[e].t()
+        if act == "swiglu":
+            u = torch.nn.functional.silu(u[:, :ff]) * u[:, ff:]
+        elif act == "relu2":
+            u = torch.relu(u).square()
+        else:
+            u = torch.nn.functional.gelu(u)
+        out.index_add_(0, t, (u @ down[e].t()) * w[t, k].double()[:, None])
+    t, k = (idx >= E).nonzero(as_tuple=True)
+    out.index_add_(0, t, x[t] * w[t, k].double()[:, None])
+    return out
+
+
+@pytest.mark.parametrize("act", ["swiglu", "relu2", "gelu"])
+@pytest.mark.parametrize("T,W,ff,E,top", [
+    (1, 64, 8, 4, 2), (3, 72, 24, 5, 3), (16, 256, 64, 8, 2), (17, 136, 40, 8, 2), (33, 128, 16, 3, 1), (64, 2048, 96, 8, 2),
+    (65, 64, 8, 4, 2), (66, 72, 24, 5, 5), (129, 136, 40, 128, 4), (300, 256, 200, 8, 2), (511, 1024, 512, 4, 2),
+    (1024, 192, 136, 2, 1), (2050, 128, 72, 16, 2)])
+def test_experts_against_float64(T, W, ff, E, top, act):
+    from llmctl.ops import hybrid as hops
+
+    x, router, up, down = _case(T, W, ff, E, act, seed=T)
+    d3 = down.view(W, E, ff).transpose(0, 1)
+    assert hops.experts_ok(x, up, d3, E)
+    nat = hops.native_hybrid()
+    idx, w = nat.moe_route(x, router, None, top, 1, 1, True, True)
+    got = nat.moe_experts(x, idx, w, [up], [d3], hops._EXPERT_ACTS[act])
+    want = _plain(x, idx.long(), w, up, d3, act, E)
+    # two bf16 roundings (activation, expert result) of relative size 2^-9 each, over sums of ff and of top terms
+    assert (got.double() - want).norm() <= 2.0 ** -7 * want.norm()
+    again = nat.moe_experts(x, idx, w, [u.contiguous() for u in up.unbind(0)], [u.contiguous() for u in d3.unbind(0)],
+                            hops._EXPERT_ACTS[act])
+    assert torch.equal(got, again)  # a list of expert weights is the same product, and no atomics: bit for bit
+
+
+@pytest.mark.parametrize("T", [5, 64, 65, 700])
+def test_one_expert_takes_all_and_experts_without_weights(T):
+    from llmctl.ops import hybrid as hops
+
+    W, ff, E = 128, 48, 6  # output 7 is an expert without weights
+    x, _, up, down = _case(T, W, ff, E, "swiglu")
+    d3 = down.view(W, E, ff).transpose(0, 1)
+    nat = hops.native_hybrid()
+    idx = torch.tensor([[3, 7]], dtype=torch.int32, device="cuda").repeat(T, 1)
+    w = torch.rand(T, 2, device="cuda")
+    shared = torch.randn(T, W + 8, device="cuda").bfloat16()
+    got = nat.moe_experts(x, idx, w, [up], [d3], 1, shared[:, :W], shared[:, W:W + 1])
+    want = _plain(x, idx.long(), w, up, d3, "swiglu", E) + torch.sigmoid(shared[:, W:W + 1].double()) * shared[:, :W].double()
+    assert (got.double() - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.parametrize("T,W,E,top,groups,keep", [(1, 64, 8, 2, 1, 1), (7, 72, 8, 2, 4, 2), (130, 256, 128, 8, 8, 3), (1025, 2048, 8, 2, 2, 1),
+                                                   (1030, 136, 9, 9, 3, 3)])
+@pytest.mark.parametrize("kind", ["sigmoid", "softmax", "softmax+bias"])
+def test_route_matches_the_choice_kernels(T, W, E, top, groups, keep, kind):
+    """The fused router chooses and weighs as the choice kernels do on the float64 logits (rows whose choice hangs on less
+    than the fp32 product's rounding are left out)."""
+    from llmctl.ops import hybrid as hops
+
+    x, router, _, _ = _case(T, W, 8, E, "relu2", seed=3)
+    bias = torch.randn(E, device="cuda") * 0.1 if kind == "softmax+bias" else None
+    idx, w = hops.native_hybrid().moe_route(x, router, bias, top, groups, keep, kind != "sigmoid", True if kind != "sigmoid" else False)
+    z = x.double() @ router.double().t()
+    pick = (lambda l: hops.group_topk_router(l, top, groups, keep)) if kind == "sigmoid" else (
+        lambda l: hops.bias_topk_router(l, bias, top, groups, keep, True))
+    ri, rw = pick(z.float().contiguous())
+    # a perturbation of the size of the product's rounding (W terms) that leaves the choice alone marks a safe row
+    eps = 4e-6 * z.abs().max().float()
+    safe = torch.ones(T, dtype=torch.bool, device="cuda")
+    for s in range(4):
+        noise = (torch.rand(z.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(s)) - 0.5) * 2 * eps
+        safe &= (pick((z.float() + noise).contiguous())[0] == ri).all(1)
+    assert safe.float().mean() > 0.9
+    assert torch.equal(idx.long()[safe], ri[safe])
+    assert torch.allclose(w[safe], rw[safe], rtol=1e-4, atol=1e-6)
