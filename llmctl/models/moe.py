@@ -216,6 +216,13 @@ class GroupLimitedMoE(nn.Module):
             for p in list(self.experts_up) + list(self.experts_down):
                 p.normal_(0.0, 0.02)
 
+    def on_device(self, T: int) -> bool:
+        """Whether a step of T rows runs without a host synchronisation."""
+        from llmctl.ops import hybrid as hops
+
+        up = self.experts_up[0]
+        return hops.experts_ok(up[:1], self.experts_up, self.experts_down, self.E, self.top)
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x [T, width] -> fp32 [T, width]."""
         from llmctl.ops import hybrid as hops
@@ -331,6 +338,13 @@ class BiasedSoftmaxMoE(nn.Module):
         a = act(torch.bmm(xg, self.w_up.transpose(1, 2)).view(E * C, self.up_rows))
         y = torch.bmm(a.view(E, C, self.ff), self.w_down.view(W, E, self.ff).permute(1, 2, 0)).view(E * C, W)
         return y.index_select(0, both[E * C:])
+
+    def on_device(self, T: int) -> bool:
+        """Whether a step of T rows runs without a host synchronisation."""
+        from llmctl.ops import hybrid as hops
+
+        down = self.w_down.view(-1, self.E, self.ff).transpose(0, 1)
+        return self._dense(T) or hops.experts_ok(self.w_up[0, :1], self.w_up, down, self.E + self.identity, self.top)
 
     def forward(self, x: torch.Tensor):
         """x [T, width] -> fp32 [T, width] (and the side columns)."""

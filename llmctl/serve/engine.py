@@ -39,6 +39,7 @@ from llmctl.models import DecoderLM
 from llmctl.utils.env import graph_capture_gc_guard
 
 from .block_manager import PagedKVCache, make_kv_manager
+from .decode_graph import MAX_GRAPHS, WARM_STEPS, DecodeGraph, upload_packed
 from .prefix_cache import PrefixCache
 from .scheduler import ContinuousBatchScheduler, PrefillChunk, SamplingParams, Sequence
 from .tokenizer import load_tokenizer
@@ -90,7 +91,7 @@ class InferenceEngine:
         self.hybrid = bool(getattr(self.model, "is_hybrid", False))
         if self.hybrid:
             self._init_hybrid(max_batch_size, max_batch_tokens, kv_cache_fraction, num_kv_blocks, scheduler,
-                              prefix_caching, kv_cache_dtype, weight_dtype, seed)
+                              prefix_caching, kv_cache_dtype, weight_dtype, seed, use_graphs)
             return
         # decode projection weights: the model's ("auto"), or an fp8 (OCP e4m3fn) copy with fp32 row
         # scales ("fp8", W8A16) that the fused decode path streams instead (half the bytes of the
@@ -149,7 +150,7 @@ class InferenceEngine:
                  block_size, self.kv_cache.nbytes / 1e9)
 
     def _init_hybrid(self, max_batch_size, max_batch_tokens, kv_cache_fraction, num_kv_blocks, scheduler,
-                     prefix_caching, kv_cache_dtype, weight_dtype, seed) -> None:
+                     prefix_caching, kv_cache_dtype, weight_dtype, seed, use_graphs) -> None:
         from .block_manager import HybridCache
 
         if self.tp > 1:
@@ -183,8 +184,13 @@ class InferenceEngine:
                                                   scheduler, bs, prefix_cache=self.prefix_cache,
                                                   state_slots=self.kv_cache.slots)
         self.max_batch_size = max_batch_size
-        self.use_graphs = False  # routed experts size their segments on the host
+        self.use_graphs = False  # the transformer's padded, sampled graphs; this family's: _hybrid_decode
         self._graphs = {}
+        # captured decode steps by (rows, context bound); a shape maps to the number of eager steps it has had until then
+        self._decode_graphs: Dict[Tuple[int, int], object] = {}
+        self._decode_capture = use_graphs and self.device.type == "cuda"
+        self._graph_pool = None
+        self._weights_seen = None
         self._np_rng = np.random.default_rng(seed)
         self._pending = None
         self._last_toks = None
@@ -208,8 +214,6 @@ class InferenceEngine:
         d = self.device
         Tp = len(pp["ids"]) if pp is not None else 0
         Td = len(dp["ids"]) if dp is not None else 0
-        i32 = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int32)).to(d, non_blocking=True)
-        i64 = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int64)).to(d, non_blocking=True)
         ids = np.concatenate([np.asarray(pp["ids"], dtype=np.int64) if Tp else np.zeros(0, np.int64),
                               np.asarray(dp["ids"], dtype=np.int64) if Td else np.zeros(0, np.int64)])
         pos = np.concatenate([np.asarray(pp["pos"], dtype=np.int32) if Tp else np.zeros(0, np.int32),
@@ -225,24 +229,76 @@ class InferenceEngine:
             list(dp["positions"]) if Td else [])
         state = (list(pp["state"]) if Tp else []) + (list(dp["state"]) if Td else [])
         seq_of = np.repeat(np.arange(len(cu) - 1, dtype=np.int32), np.diff(np.asarray(cu, dtype=np.int64)))
-        batch = StepBatch(ids=i64(ids), pos=i32(pos), slots=i64(slots), Tp=Tp,
-                          p_cu=i32(p_cu) if Tp else None, p_ctx=i32(pp["ctx"]) if Tp else None,
-                          p_bt=i32(pp["bt"]) if Tp else None, d_ctx=i32(dp["ctx"]) if Td else None,
-                          d_bt=i32(dp["bt"]) if Td else None, cu=i32(cu), start=i32(start), state=i32(state),
-                          max_q=max((b - a for a, b in zip(p_cu[:-1], p_cu[1:])), default=0), cu_host=cu,
-                          seq_of=i32(seq_of), d_max_ctx=int(max(dp["ctx"])) if Td else 0,
-                          carried=any(int(v) > 0 and b - a > 1 for v, a, b in zip(start, p_cu[:-1], p_cu[1:])),
-                          fresh=Td == 0 and all(int(v) == 0 for v in start))
         if rows is None:
             rows = (list(pp["last"]) if Tp else []) + list(range(Tp, Tp + Td))
+        i32, none = (lambda a: np.asarray(a, dtype=np.int32)), np.zeros(0, np.int32)
+        # all index arrays of the step through one copy
+        up = upload_packed([ids, slots, np.asarray(rows, dtype=np.int64), pos, i32(p_cu) if Tp else none,
+                            i32(pp["ctx"]) if Tp else none, i32(pp["bt"]) if Tp else none, i32(dp["ctx"]) if Td else none,
+                            i32(dp["bt"]) if Td else none, i32(cu), i32(start), i32(state), seq_of], d)
+        ids_d, slots_d, rows_d, pos_d, p_cu_d, p_ctx_d, p_bt_d, d_ctx_d, d_bt_d, cu_d, start_d, state_d, seq_d = up
+        batch = StepBatch(ids=ids_d, pos=pos_d, slots=slots_d, Tp=Tp, p_cu=p_cu_d if Tp else None, p_ctx=p_ctx_d if Tp else None,
+                          p_bt=p_bt_d if Tp else None, d_ctx=d_ctx_d if Td else None, d_bt=d_bt_d if Td else None, cu=cu_d,
+                          start=start_d, state=state_d,
+                          max_q=max((b - a for a, b in zip(p_cu[:-1], p_cu[1:])), default=0), cu_host=cu,
+                          seq_of=seq_d, d_max_ctx=int(max(dp["ctx"])) if Td else 0,
+                          carried=any(int(v) > 0 and b - a > 1 for v, a, b in zip(start, p_cu[:-1], p_cu[1:])),
+                          fresh=Td == 0 and all(int(v) == 0 for v in start))
         if count:
             self.stats["prefill_tokens"] += Tp
             self.stats["decode_tokens"] += Td
         if not rows and trail is None:
-            self.model.step(batch, self.kv_cache, rows=i64([]))
+            self.model.step(batch, self.kv_cache, rows=rows_d)
             return torch.empty(0, self.cfg.vocab_size, device=d, dtype=self.dtype)
-        x = self.model.step(batch, self.kv_cache, rows=i64(rows), trail=trail)
+        every = len(rows) == len(ids) and list(rows) == list(range(len(ids)))  # (a decode step reads all of its rows)
+        x = self.model.step(batch, self.kv_cache, rows=None if every else rows_d, trail=trail)
         return self.model.logits(x)
+
+    def _weights_key(self):
+        """What a captured step's kernels were recorded against: the weights' storage and versions (modules keep stacked or
+        transposed copies of them, which an in-place change makes stale)."""
+        ps = getattr(self, "_param_list", None)
+        if ps is None:
+            ps = self._param_list = list(self.model.parameters())
+        return sum(p._version for p in ps), sum(p.data_ptr() for p in ps)
+
+    def _hybrid_decode(self, dp: Dict, count: bool = True, ids_on_device: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """One decode step of a hybrid-mixer model: the first steps of a shape run eagerly, then its captured graph is
+        replayed (:mod:`llmctl.serve.decode_graph`).  ``ids_on_device``: the rows' input tokens as a device tensor."""
+        n = len(dp["positions"])
+        key = (n, 1 << max(int(max(dp["ctx"])) - 1, 0).bit_length()) if n else None
+        g = None
+        if self._decode_capture and n:
+            w = self._weights_key()
+            if w != self._weights_seen:
+                self.release_graphs()
+                self._weights_seen = w
+            g = self._decode_graphs.pop(key, 0)
+            if not isinstance(g, DecodeGraph) and g >= WARM_STEPS and all(
+                    m.on_device(n) for m in self.model.modules() if hasattr(m, "on_device")):
+                if self._graph_pool is None:
+                    self._graph_pool = torch.cuda.graph_pool_handle()
+                while sum(isinstance(v, DecodeGraph) for v in self._decode_graphs.values()) >= MAX_GRAPHS:
+                    old = next(k for k, v in self._decode_graphs.items() if isinstance(v, DecodeGraph))
+                    torch.cuda.synchronize(self.device)
+                    self._decode_graphs.pop(old).graph.reset()
+                dg = DecodeGraph(n, self.max_blocks_per_seq, key[1], self.device)
+                dg.capture(self.model, self.kv_cache, self._graph_pool)
+                g = dg
+            self._decode_graphs[key] = g if isinstance(g, DecodeGraph) else g + 1  # (re-inserted: most recently used last)
+        if not isinstance(g, DecodeGraph):
+            if ids_on_device is not None:
+                dp = dict(dp, ids=ids_on_device.tolist())
+            return self._hybrid_exec(None, dp, count=count)
+        limit = getattr(self.model, "position_limit", None)
+        if limit is not None and max(dp["positions"]) >= limit:
+            raise ValueError(f"position {max(dp['positions'])} is beyond the model's {limit} learned positions")
+        use_knobs(self.knobs)
+        if count:
+            self.stats["decode_tokens"] += n
+        self.stats["graph_replays"] += 1
+        return g.run({"ids": dp.get("ids"), "slots": dp["slots"], "pos": dp["positions"], "ctx": dp["ctx"],
+                      "start": dp["positions"], "state": dp["state"], "bt": dp["bt"]}, ids_on_device)
 
     # ------------------------------------------------------------------ externally driven schedule
     def open_sequence(self, ids: List[int], request_id: str = "", params: Optional[SamplingParams] = None) -> Sequence:
@@ -735,11 +791,17 @@ class InferenceEngine:
     def release_graphs(self) -> None:
         """Drop the captured decode graphs (they hold the RCCL communicator's captured
         collectives: release them before ``destroy_process_group``)."""
-        if self._graphs and self.device.type == "cuda":
+        own = [g for g in getattr(self, "_decode_graphs", {}).values() if isinstance(g, DecodeGraph)]
+        if (self._graphs or own) and self.device.type == "cuda":
             torch.cuda.synchronize(self.device)
         for g, _ in self._graphs.values():
             g.reset()
         self._graphs.clear()
+        for g in own:
+            g.graph.reset()
+        if self.hybrid:
+            self._decode_graphs.clear()
+            self._graph_pool = None
 
     def close(self) -> None:
         """Deterministic teardown, never left to garbage collection: drop an in-flight pipelined
@@ -786,7 +848,7 @@ class InferenceEngine:
     def decode_exec(self, plan: Dict) -> torch.Tensor:
         use_knobs(self.knobs)
         if self.hybrid:
-            return self._hybrid_exec(None, plan)
+            return self._hybrid_decode(plan)
         ids, positions, slots, ctx, bt = plan["ids"], plan["positions"], plan["slots"], plan["ctx"], plan["bt"]
         n = len(ids)
         self.stats["decode_tokens"] += n
@@ -900,9 +962,8 @@ class InferenceEngine:
         d = self.device
         n = len(plan["positions"])
         if self.hybrid:
-            if cont:  # the previous step's sampled ids (this path reads them back: no captured graph)
-                plan = dict(plan, ids=self._last_toks.tolist())
-            logits = self._hybrid_exec(None, plan, count=False)  # counted by _launch_decode
+            # a continued step's input is what the previous one sampled, still on the device; counted by _launch_decode
+            logits = self._hybrid_decode(plan, count=False, ids_on_device=self._last_toks if cont else None)
             toks = self._sample_plan(logits, plan, n)
             self._last_toks = toks
             return toks
