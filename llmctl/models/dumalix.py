@@ -232,7 +232,7 @@ class DumalixLM(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         xn, _ = hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None, self.cfg.layer_norm_eps, True,
                                        self.dtype)
-        return F.linear(xn, self.lm_head)
+        return hops.linear(xn, self.lm_head)
 
     # ------------------------------------------------------------------ checkpoint names
     @torch.no_grad()

@@ -177,7 +177,7 @@ class LenitarLM(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         xn = hops.layernorm_f32(x.contiguous(), self.final_norm_w, self.final_norm_b, self.cfg.layer_norm_eps,
                                 self.dtype)
-        return F.linear(xn, self.lm_head)
+        return hops.linear(xn, self.lm_head)
 
     # ------------------------------------------------------------------ checkpoint names
     @torch.no_grad()

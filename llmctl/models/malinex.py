@@ -226,7 +226,8 @@ class MalinexLM(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         xn, _ = hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None, self.cfg.layer_norm_eps, False,
                                        self.dtype)
-        return F.linear(xn, self.lm_head).float() * self.cfg.logit_scale
+        z = hops.linear_f32(xn, self.lm_head)
+        return z if self.cfg.logit_scale == 1.0 else z * self.cfg.logit_scale
 
     # ------------------------------------------------------------------ checkpoint names
     @torch.no_grad()

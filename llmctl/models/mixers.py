@@ -205,20 +205,20 @@ class LatentAttention(nn.Module):
         if isinstance(cache, tuple):  # (paged rows, recurrent states): this mixer keeps no state
             cache = cache[0]
         T, H = h.shape[0], self.H
-        z = F.linear(h, self.w_in)
+        z = hops.linear(h, self.w_in)
         a, c = self.q_cols, self.q_cols + self.rk + self.dr
         hops.latent_kv_write(z[:, a:c], self.kv_norm, self.eps, b.pos, self.inv_freq, self.rot_dims, cache, b.slots,
                              self.interleaved, self.rot_amp)
         if self.qr:
             cq = hops.rmsnorm_cols(z[:, :a], self.q_norm, self.eps, self.qr, h.dtype)
-            q = F.linear(cq, self.w_uq).view(T, H, self.dn + self.dr)
+            q = hops.linear(cq, self.w_uq).view(T, H, self.dn + self.dr)
         else:
             q = z[:, :a].unflatten(1, (H, self.dn + self.dr))  # a view: rows keep z's pitch
         if self._expand(b):
             o = self._attend_expanded(q, b, cache)
             if self.has_gate:
                 o = hops.sigmoid_gate_mul(o, z[:, c:])
-            return F.linear(o, self.w_o)
+            return hops.linear(o, self.w_o)
         q_lat = torch.bmm(q[:, :, :self.dn].transpose(0, 1), self.w_uk).transpose(0, 1)  # [T, H, rank]
         qa = hops.latent_q_assemble(q_lat, q, b.pos, self.inv_freq, self.rot_dims, self.dn, self.interleaved, self.rot_amp)
         outs = []
@@ -232,7 +232,7 @@ class LatentAttention(nn.Module):
         o = torch.bmm(o_lat.transpose(0, 1), self._w_uv_t()).transpose(0, 1).reshape(T, H * self.dv)
         if self.has_gate:
             o = hops.sigmoid_gate_mul(o, z[:, c:])
-        return F.linear(o, self.w_o)
+        return hops.linear(o, self.w_o)
 
 
 class CausalConv(nn.Module):
@@ -350,7 +350,7 @@ class GroupedAttention(nn.Module):
         rows, states = cache if isinstance(cache, tuple) else (cache, ())
         T = h.shape[0]
         if z is None:
-            z = F.linear(h, self.w_qkv, self.b_qkv)
+            z = hops.linear(h, self.w_qkv, self.b_qkv)
         if self.conv is not None:
             z = self.conv(z, b, states[0])
         v_first = None
@@ -377,7 +377,7 @@ class GroupedAttention(nn.Module):
             outs.append(hops.latent_attention_decode(q[b.Tp:], rows, b.d_bt, b.d_ctx, self.window, self.sink, self.scale,
                                                      self.dv, max_ctx=b.d_max_ctx, **opt))
         o = outs[0] if len(outs) == 1 else torch.cat(outs)
-        return F.linear(o.reshape(T, self.H * self.dv), self.w_o)
+        return hops.linear(o.reshape(T, self.H * self.dv), self.w_o)
 
 
 class ClampedGLU(nn.Module):
@@ -393,7 +393,7 @@ class ClampedGLU(nn.Module):
         _init(self.w_down, 0.02)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(hops.clamped_glu(F.linear(h, self.w_gu), self.limit, self.alpha), self.w_down)
+        return hops.linear(hops.clamped_glu(hops.linear(h, self.w_gu), self.limit, self.alpha), self.w_down)
 
 
 class MLSTM(nn.Module):
@@ -420,7 +420,7 @@ class MLSTM(nn.Module):
 
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         T, H, dk, dv = h.shape[0], self.H, self.dk, self.dv
-        z = F.linear(h, self.w_in)
+        z = hops.linear(h, self.w_in)
         q, k = z[:, :H * dk].view(T, H, dk), z[:, H * dk:2 * H * dk].view(T, H, dk)
         v = z[:, 2 * H * dk:2 * H * dk + H * dv].view(T, H, dv)
         g = z[:, 2 * H * dk + H * dv:]
@@ -428,17 +428,10 @@ class MLSTM(nn.Module):
         S, n, m = state
         o = hops.mlstm_scan(q, k, v, gates, self.b_i, self.b_f, self.cap, 1.0 / math.sqrt(dk), S, n, m, b.state,
                             b.cu, b.start, cu_host=b.cu_host)
-        return F.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
+        return hops.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
 
 
-def _mm_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """``x @ w^T`` with an fp32 result (inputs in their own dtype, fp32 accumulation)."""
-    if x.dtype == torch.float32:
-        return F.linear(x, w)
-    try:
-        return torch.mm(x, w.t(), out_dtype=torch.float32)
-    except (TypeError, RuntimeError):
-        return F.linear(x, w).float()
+_mm_f32 = hops.linear_f32
 
 
 class GatedLinearAttention(nn.Module):
@@ -483,7 +476,7 @@ class GatedLinearAttention(nn.Module):
         if isinstance(state, tuple) and len(state) == 2 and isinstance(state[1], tuple):  # (rows, states)
             state = state[1]
         T, H, dk, dv = h.shape[0], self.H, self.dk, self.dv
-        z = F.linear(h, self.w_in, self.b_in)
+        z = hops.linear(h, self.w_in, self.b_in)
         a, c, e = H * dk, 2 * H * dk, 2 * H * dk + H * dv
         q, k = z[:, :a].unflatten(1, (H, dk)), z[:, a:c].unflatten(1, (H, dk))
         v = z[:, c:e].unflatten(1, (H, dv))
@@ -493,7 +486,7 @@ class GatedLinearAttention(nn.Module):
             b.scratch["gla_plan"] = hops.gla_chunk_plan(b.cu_host, h.device) if h.is_cuda else None
         o = hops.gla_scan(q, k, v, decay, self.b_a2, self.tau, dk ** -0.5, state[0], b.state, b.cu, b.start,
                           plan=b.scratch["gla_plan"])
-        y = F.linear(hops.headnorm_gate(o, self._norm_rows(), g, self.eps, h.dtype, silu=True), self.w_o)
+        y = hops.linear(hops.headnorm_gate(o, self._norm_rows(), g, self.eps, h.dtype, silu=True), self.w_o)
         return (y, z[:, self.cols:]) if self.side else y
 
 
@@ -541,7 +534,7 @@ class SigmoidAttention(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, cache):
         rows = cache[0] if isinstance(cache, tuple) else cache
         T, H, G, dk, dv = h.shape[0], self.H, self.G, self.dk, self.dv
-        z = F.linear(h, self.w_in, self.b_in)
+        z = hops.linear(h, self.w_in, self.b_in)
         q = hops.qk_fullnorm_prep(z, H, G, dk, dv, self.q_norm, self.k_norm, self.eps, b.pos, self.temp_coef,
                                   self.temp_every, rows, b.slots)
         opt = dict(groups=G, koff=dv, sig_bias=self.bias, dist_a=self.dist_a, dist_b=self.dist_b)
@@ -554,7 +547,7 @@ class SigmoidAttention(nn.Module):
                                                      max_ctx=b.d_max_ctx, **opt))
         o = outs[0] if len(outs) == 1 else torch.cat(outs)
         g0 = self.cols - H
-        y = F.linear(hops.sigmoid_gate_mul(o.reshape(T, H * dv), z[:, g0:self.cols]), self.w_o)
+        y = hops.linear(hops.sigmoid_gate_mul(o.reshape(T, H * dv), z[:, g0:self.cols]), self.w_o)
         return (y, z[:, self.cols:]) if self.side else y
 
 
@@ -574,8 +567,13 @@ class DenseFF(nn.Module):
         _init(self.w_down, 0.02)
 
     def forward(self, h: torch.Tensor):
-        z = F.linear(h, self.w_up, self.b_up)
-        y = F.linear(hops.act_any(z[:, :self.ff], self.act), self.w_down, self.b_down)
+        if hops.rows_ok(h, self.w_up, self.b_up):  # the activation in the product's epilogue
+            z = hops.rows_linear(h, self.w_up, self.b_up, self.act, self.ff)
+            a = z[:, :self.ff]
+        else:
+            z = F.linear(h, self.w_up, self.b_up)
+            a = hops.act_any(z[:, :self.ff], self.act)
+        y = hops.linear(a, self.w_down, self.b_down)
         return (y, z[:, self.ff:]) if self.side else y
 
 
@@ -592,7 +590,7 @@ class GatedFF(nn.Module):
         _init(self.w_down, 0.02)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return F.linear(hops.glu_act(F.linear(h, self.w_gu), self.act), self.w_down)
+        return hops.linear(hops.glu_act(hops.linear(h, self.w_gu), self.act), self.w_down)
 
 
 class DifferentialAttention(nn.Module):
@@ -642,7 +640,7 @@ class DifferentialAttention(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, cache) -> torch.Tensor:
         rows = cache[0] if isinstance(cache, tuple) else cache
         T, H, G, dk, dv = h.shape[0], self.H, self.G, self.dk, self.dv
-        z = F.linear(h, self.w_qkv)
+        z = hops.linear(h, self.w_qkv)
         k0, v0 = 2 * H * dk, 2 * (H + G) * dk
         hops.kv_rows_write(z[:, k0:v0], z[:, v0:], rows, b.slots, G)
         o = torch.empty(T, H * dv, device=h.device, dtype=h.dtype)
@@ -651,7 +649,7 @@ class DifferentialAttention(nn.Module):
             hops.diff_attention(z[:b.Tp, :k0], rows, b.p_bt, b.p_cu, b.p_ctx, *a, out=o[:b.Tp], max_q=b.max_q)
         if T > b.Tp:
             hops.diff_attention(z[b.Tp:, :k0], rows, b.d_bt, None, b.d_ctx, *a, out=o[b.Tp:], max_ctx=b.d_max_ctx)
-        return F.linear(o, self.w_o)
+        return hops.linear(o, self.w_o)
 
 
 class MinGRU(nn.Module):
@@ -682,8 +680,8 @@ class MinGRU(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         if isinstance(state, tuple) and len(state) == 2 and isinstance(state[1], tuple):  # (rows, states)
             state = state[1]
-        y = hops.mingru_scan(F.linear(h, self.w_in), self.b_z, self.b_x, state[0], b)
-        return F.linear(y, self.w_o)
+        y = hops.mingru_scan(hops.linear(h, self.w_in), self.b_z, self.b_x, state[0], b)
+        return hops.linear(y, self.w_o)
 
 
 class DeltaRule(nn.Module):
@@ -725,7 +723,7 @@ class DeltaRule(nn.Module):
         T, H, d = h.shape[0], self.H, self.d
         n = H * d
         if z is None:
-            z = F.linear(h, self.w_in)
+            z = hops.linear(h, self.w_in)
         r, k, v = (z[:, i * n:(i + 1) * n].unflatten(1, (H, d)) for i in range(3))
         g, za = z[:, 3 * n:4 * n], z[:, 4 * n:5 * n]
         zw = _mm_f32(hops.tanh_act(z[:, 5 * n:self.cols]), self.w_w2)  # fp32 [T, H * d]
@@ -733,7 +731,7 @@ class DeltaRule(nn.Module):
             b.scratch["gla_plan"] = hops.gla_chunk_plan(b.cu_host, h.device) if h.is_cuda else None
         o = hops.delta_scan(r, k, v, zw, self.w0, za, self.b_a, self.decay_coef, self.key_eps, state[0], b.state, b.cu,
                             b.start, plan=b.scratch["gla_plan"])
-        return F.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
+        return hops.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
 
 
 def _rows8(n: int) -> int:
@@ -788,12 +786,12 @@ class GatedDeltaRule(nn.Module):
         S, carried = _own_states(state)
         H, G, dv = self.H, self.G, self.dv
         if z is None:
-            z = F.linear(h, self.w_in)
+            z = hops.linear(h, self.w_in)
         c, g0 = self.conv.channels, self.conv.channels + H * dv
         qk, v = hops.conv_silu_unit(z[:, :c], self.conv.tap_major(), None, carried, b, G, G, self.dk, self.dk ** -0.5, self.key_eps)
         y = hops.memory_scan(qk[:, :G], qk[:, G:], v.view(-1, H, dv), "delta", S, b, ga=z[:, g0:g0 + H], gb=z[:, g0 + H:g0 + 2 * H],
                              a_log=self.a_log, dt_bias=self.dt_bias, norm=(self._norm_rows(), z[:, c:g0], self.eps))
-        return F.linear(y, self.w_o)
+        return hops.linear(y, self.w_o)
 
 
 class Mamba2(nn.Module):
@@ -836,13 +834,13 @@ class Mamba2(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         S, carried = _own_states(state)
         T, n = h.shape[0], self.inner
-        z = F.linear(h, self.w_in)
+        z = hops.linear(h, self.w_in)
         c = n + self.conv.channels
         _, xbc = hops.conv_silu_unit(z[:, n:c], self.conv.tap_major(), self.conv_bias, carried, b, 0, 0, 0, 1.0)
         B, C = (xbc[:, n + i * self.G * self.N:n + (i + 1) * self.G * self.N].unflatten(1, (self.G, self.N)) for i in range(2))
         o = hops.memory_scan(C, B, xbc[:, :n].unflatten(1, (self.H, self.dv)), "ssm", S, b, ga=z[:, c:c + self.H], a_log=self.a_log,
                              dt_bias=self.dt_bias, skip=self.skip)
-        return F.linear(hops.gate_groupnorm(o.view(T, n), z[:, :n], self.norm, self.norm_groups, self.eps, h.dtype), self.w_o)
+        return hops.linear(hops.gate_groupnorm(o.view(T, n), z[:, :n], self.norm, self.norm_groups, self.eps, h.dtype), self.w_o)
 
 
 class Retention(nn.Module):
@@ -880,12 +878,12 @@ class Retention(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         S = _own_states(state)[0]
         H, dk, dv = self.H, self.dk, self.dv
-        z = F.linear(h, self.w_in)
+        z = hops.linear(h, self.w_in)
         qk = hops.rotary_f32(z, H, H, dk, b.pos, self.inv_freq, self.rot_dims, self.interleaved, self.rot_amp, dk ** -0.5)
         v0, g0 = 2 * H * dk, 2 * H * dk + H * dv
         y = hops.memory_scan(qk[:, :H], qk[:, H:], z[:, v0:g0].unflatten(1, (H, dv)), "fixed", S, b, log_decay=self.log_decay,
                              norm=(None, z[:, g0:g0 + H * dv], self.eps))
-        return F.linear(y, self.w_o)
+        return hops.linear(y, self.w_o)
 
 
 class ParallelMixers(nn.Module):
@@ -931,7 +929,7 @@ class ParallelMixers(nn.Module):
         rows, states = cache
         nl = len(self.left.state_shapes())
         w, bias, c0 = self._stacked()
-        z = F.linear(h, w, bias)
+        z = hops.linear(h, w, bias)
         yl = self.left.step(h, b, (rows, tuple(states[:nl])), z=z[:, :self.left.w_in.shape[0]])
         yr = self.right.step(h, b, (rows, tuple(states[nl:])), z=z[:, c0:c0 + self.right.w_in.shape[0]])
         return (yl, self.left_scale), (yr, self.right_scale)

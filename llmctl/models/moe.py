@@ -359,8 +359,14 @@ class BiasedSoftmaxMoE(nn.Module):
                 return hops.glu_act(u, "silu", scale)
             return hops.act_any(u, self.act, scale)
 
-        z = None if self.w_sup is None else torch.nn.functional.linear(x, self.w_sup, self.b_sup)
-        ys = torch.nn.functional.linear(act(z[:, :self.sup_rows]), self.w_sdown) if self.shared_ff else None
+        z = ys = None
+        if self.w_sup is not None:
+            fused = self.act != "swiglu" and hops.rows_ok(x, self.w_sup, self.b_sup)  # the activation in the product's epilogue
+            z = (hops.rows_linear(x, self.w_sup, self.b_sup, self.act, self.sup_rows) if fused
+                 else hops.linear(x, self.w_sup, self.b_sup))
+            if self.shared_ff:
+                u = z[:, :self.sup_rows]
+                ys = hops.linear(u if fused else act(u), self.w_sdown)
         gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
         down = self.w_down.view(x.shape[1], self.E, self.ff).transpose(0, 1)  # [E, width, ff]
         if hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top):

@@ -272,7 +272,7 @@ class PamazenLM(nn.Module):
     def logits(self, x: torch.Tensor) -> torch.Tensor:
         xn, _ = hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self._final_norm_row(), None, self.cfg.layer_norm_eps, False,
                                        self.dtype)
-        z = F.linear(xn, self.lm_head).float()
+        z = hops.linear_f32(xn, self.lm_head)
         return hops.softcap_(z, self.cfg.logit_softcap) if self.cfg.logit_softcap > 0 else z
 
     # ------------------------------------------------------------------ checkpoint names

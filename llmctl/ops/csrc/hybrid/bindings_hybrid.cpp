@@ -47,6 +47,7 @@ void mlstm_chunk_combine(const at::Tensor& S, const at::Tensor& n, const at::Ten
 std::tuple<at::Tensor, at::Tensor> group_topk_router(const at::Tensor& logits, int64_t top, int64_t groups, int64_t keep);
 std::tuple<at::Tensor, at::Tensor> bias_topk_router(const at::Tensor& logits, const c10::optional<at::Tensor>& bias, int64_t top, int64_t groups,
                                                     int64_t keep, bool renorm);
+at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t act, int64_t act_cols, bool f32);
 std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t top,
                                              int64_t groups, int64_t keep, bool softmax, bool renorm);
 at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
@@ -145,6 +146,7 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("delta_chunk_combine(Tensor(a!) S, Tensor slots, Tensor start, Tensor base, Tensor loc, Tensor P, Tensor(b!) init) -> ()");
   m.def("gated_norm_add_norm_f32_(Tensor(a!) x, Tensor y, Tensor r, Tensor w_post, Tensor? w_next, float eps, bool out_bf16) -> Tensor");
   m.def("embed_rmsnorm_f32(Tensor ids, Tensor pos, Tensor table, Tensor pos_table, Tensor w, float eps, bool out_bf16) -> (Tensor, Tensor)");
+  m.def("rows_linear(Tensor x, Tensor w, Tensor? bias, int act, int act_cols, bool f32) -> Tensor");
   m.def("moe_route(Tensor x, Tensor w, Tensor? bias, int top, int groups, int keep, bool softmax, bool renorm) -> (Tensor, Tensor)");
   m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
@@ -191,6 +193,7 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("bias_topk_router", &llmctl_hybrid::bias_topk_router);
   m.impl("gated_norm_add_norm_f32_", &llmctl_hybrid::gated_norm_add_norm_f32_);
   m.impl("embed_rmsnorm_f32", &llmctl_hybrid::embed_rmsnorm_f32);
+  m.impl("rows_linear", &llmctl_hybrid::rows_linear);
   m.impl("moe_route", &llmctl_hybrid::moe_route);
   m.impl("moe_experts", &llmctl_hybrid::moe_experts);
   m.impl("act_any", &llmctl_hybrid::act_any);

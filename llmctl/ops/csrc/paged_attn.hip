@@ -41,6 +41,28 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const unsigned short* __r
   cache_store8(vc, (slot * row8 + c) * 8, x, fp8);
 }
 
+// qkv rows [T, (nq + 2 nkv) D] without rotation: q out, K and V of the row to its cache slot (-1: nowhere), in one pass
+__global__ __launch_bounds__(256) void qkv_split_cache_kernel(const unsigned short* __restrict__ qkv, long ld,
+                                                              unsigned short* __restrict__ q, void* __restrict__ kc,
+                                                              void* __restrict__ vc, const int64_t* __restrict__ slots,
+                                                              int T, int q8, int kv8, bool fp8) {
+  const int row8 = q8 + 2 * kv8;
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (long)T * row8) return;
+  const int t = i / row8, c = i % row8;
+  const unsigned short* src = qkv + (long)t * ld + c * 8;
+  if (c < q8) {
+    *reinterpret_cast<uint4*>(q + ((long)t * q8 + c) * 8) = *reinterpret_cast<const uint4*>(src);
+    return;
+  }
+  const long slot = slots[t];
+  if (slot < 0) return;
+  const int cc = c - q8;
+  float x[8];
+  load8(src, x);
+  cache_store8(cc < kv8 ? kc : vc, (slot * kv8 + (cc < kv8 ? cc : cc - kv8)) * 8, x, fp8);
+}
+
 // Merge the 4 waves x TPW token groups' online-softmax partials (m, l in the log2 domain, O
 // unnormalised) of one workgroup through LDS; write the normalised row (nsplit 1) or the split's
 // fp32 partial for paged_combine_kernel.
@@ -302,6 +324,26 @@ void kv_cache_write(const at::Tensor& k, const at::Tensor& v, at::Tensor& k_cach
                      kv_fp8(k_cache));
 }
 
+at::Tensor qkv_split_cache(const at::Tensor& qkv, int64_t nq, int64_t nkv, at::Tensor& k_cache, at::Tensor& v_cache,
+                           const at::Tensor& slots) {
+  LLMCTL_CHECK(qkv.dim() == 2 && qkv.is_cuda() && qkv.scalar_type() == at::kBFloat16 && qkv.stride(1) == 1 && qkv.stride(0) % 8 == 0 &&
+                   (reinterpret_cast<uintptr_t>(qkv.data_ptr()) & 15) == 0,
+               "qkv_split_cache: bf16 [T, (nq + 2 nkv) D], aligned rows");
+  LLMCTL_CHECK(k_cache.is_contiguous() && v_cache.is_contiguous() && kv_cache_ok(k_cache) && k_cache.dim() == 4 && v_cache.sizes() == k_cache.sizes() &&
+                   v_cache.scalar_type() == k_cache.scalar_type(),
+               "qkv_split_cache: contiguous bf16 or fp8 (e4m3fn) caches [blocks, block size, heads, D]");
+  const int64_t T = qkv.size(0), D = k_cache.size(3);
+  LLMCTL_CHECK(nq > 0 && nkv > 0 && k_cache.size(2) == nkv && D % 8 == 0 && qkv.size(1) == (nq + 2 * nkv) * D, "qkv_split_cache: heads do not fit the row");
+  LLMCTL_CHECK(slots.is_cuda() && slots.is_contiguous() && slots.scalar_type() == at::kLong && slots.numel() == T, "slots: int64 [T]");
+  const c10::DeviceGuard g(qkv.device());
+  at::Tensor q = at::empty({T, nq, D}, qkv.options());
+  if (T == 0) return q;
+  const long total = T * (nq + 2 * nkv) * D / 8;
+  hipLaunchKernelGGL(qkv_split_cache_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream(), bf_ptr(qkv), (long)qkv.stride(0), bf_mut(q),
+                     k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr<int64_t>(), (int)T, (int)(nq * D / 8), (int)(nkv * D / 8), kv_fp8(k_cache));
+  return q;
+}
+
 namespace {
 // launch the decode kernel (+ combine) for N sequences x Hq query heads
 void launch_paged_decode(const unsigned short* q, const at::Tensor& k_cache,
@@ -386,6 +428,7 @@ at::Tensor paged_attention_decode(const at::Tensor& q, const at::Tensor& k_cache
 
 TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
   m.impl("kv_cache_write", &kv_cache_write);
+  m.impl("qkv_split_cache", &qkv_split_cache);
   m.impl("paged_attention_decode", &paged_attention_decode);
 }
 

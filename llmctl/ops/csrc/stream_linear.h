@@ -1,0 +1,167 @@
+// y[M, N] = act(x[M, K] W[N, K]^T + bias) for few rows (M <= 32): a stream of W over the matrix cores, in one launch.
+//
+// The bound is the weight stream and, below some 20 MB of weights, the latency of one round trip to HBM plus the launch
+// (3.5 us in a graph).  Measured beside the library's product (one MI355X, weights from HBM, 16 rows, us):
+//   N x K        2048 x 2048  4096 x 2048  8192 x 2048  10496 x 2048  32000 x 2048  4096 x 4096  2048 x 4096  768 x 3072  768 x 768
+//   library          11.1         11.7         13.8         16.1          33.1          15.6         14.9         9.1         5.3
+//   here              6.4          7.1          9.7         15.1          27.2          10.4          9.9         7.7         4.0
+// A workgroup owns whole outputs (no partial sums between workgroups), so N / 16 < 256 leaves CUs idle, and a CU draws about 30 GB/s
+// from HBM: 2048 x 8192 takes 17 us against the library's 13, which splits K over the chip.  Callers leave such shapes to it.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <hip/hip_bf16.h>
+
+#include <cstdint>
+
+namespace stream_linear {
+
+using frag_t = __attribute__((ext_vector_type(8))) __bf16;
+using acc_t = __attribute__((ext_vector_type(4))) float;
+
+struct Args {
+  const unsigned short* x;
+  long ldx;
+  const unsigned short* w;
+  long ldw;
+  const unsigned short* bias;  // bf16 [N] or null
+  void* y;                     // [M, N], bf16 or fp32
+  int M, N, K;
+  int act;       // 0 none, 1 gelu (erf), 2 gelu (tanh), 3 relu^2
+  int act_cols;  // of the first that many columns
+  int f32;  // y is fp32
+};
+
+__device__ __forceinline__ uint4 load_or_zero(const unsigned short* p, bool in) {
+  uint4 v = make_uint4(0, 0, 0, 0);
+  if (in) v = *reinterpret_cast<const uint4*>(p);
+  return v;
+}
+
+__device__ __forceinline__ float activate(int act, float v) {
+  if (act == 1) return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f));
+  if (act == 2) {
+    const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
+    return 0.5f * v * (1.0f + tanhf(u));
+  }
+  if (act == 3) {
+    const float r = fmaxf(v, 0.f);
+    return r * r;
+  }
+  return v;
+}
+
+// A workgroup of NW waves owns 16 NT weight rows; the waves split K.  A lane streams 16 bytes of its weight row per 32-deep step,
+// U steps in flight before the first MFMA; the weight fragment is the MFMA row operand, so a lane ends up with four
+// neighbouring outputs of one token.  K is a multiple of 8 (the last step is filled up with zeros), N any.
+template <int NT, int MT, int NW, int U>
+__global__ __launch_bounds__(NW * 64) void kernel(Args g) {
+  __shared__ acc_t red[NW][NT * MT][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, kg = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT;
+  const unsigned short* wp[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) wp[n] = g.w + (long)min(n0 + n * 16 + r, g.N - 1) * g.ldw + 8 * kg;
+  const unsigned short* xp[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xp[m] = g.x + (long)min(m * 16 + r, g.M - 1) * g.ldx + 8 * kg;
+  acc_t acc[NT][MT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[n][m] = acc_t{0.f, 0.f, 0.f, 0.f};
+  const int steps = (g.K + 31) / 32, per = (steps + NW - 1) / NW;
+  const int s0 = wave * per, s1 = min(s0 + per, steps), whole = min(s1, g.K / 32);
+  for (int s = s0; s < s1; s += U) {
+    uint4 wv[U][NT], xv[U][MT];
+    if (s + U <= whole) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) wv[u][n] = *reinterpret_cast<const uint4*>(wp[n] + (s + u) * 32);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xv[u][m] = *reinterpret_cast<const uint4*>(xp[m] + (s + u) * 32);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const bool in = s + u < s1 && (s + u) * 32 + 8 * kg < g.K;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) wv[u][n] = load_or_zero(wp[n] + (s + u) * 32, in);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xv[u][m] = load_or_zero(xp[m] + (s + u) * 32, in);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the whole batch in flight before the first MFMA
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_t, wv[u][n]), __builtin_bit_cast(frag_t, xv[u][m]),
+                                                              acc[n][m], 0, 0, 0);
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) red[wave][n * MT + m][lane] = acc[n][m];
+  __syncthreads();
+  for (int i = tid; i < NT * MT * 64; i += NW * 64) {
+    const int t = i >> 6, l = i & 63, row = (t % MT) * 16 + (l & 15), c = n0 + (t / MT) * 16 + 4 * (l >> 4);
+    if (row >= g.M || c >= g.N) continue;
+    acc_t s = red[0][t][l];
+#pragma unroll
+    for (int v = 1; v < NW; ++v) s += red[v][t][l];
+    const long o = (long)row * g.N + c;
+    const int left = min(4, g.N - c);
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float b = g.bias != nullptr && j < left ? __uint_as_float((unsigned)g.bias[c + j] << 16) : 0.f;
+      v[j] = activate(c + j < g.act_cols ? g.act : 0, s[j] + b);
+    }
+    if (g.f32) {
+      float* y = static_cast<float*>(g.y) + o;
+      if (left == 4 && (g.N & 3) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+      else
+        for (int j = 0; j < left; ++j) y[j] = v[j];
+    } else {
+      unsigned short* y = static_cast<unsigned short*>(g.y) + o;
+      unsigned short h[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) h[j] = __bfloat16_as_ushort(__float2bfloat16(v[j]));
+      if (left == 4 && (g.N & 3) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
+      else
+        for (int j = 0; j < left; ++j) y[j] = h[j];
+    }
+  }
+}
+
+template <int NT, int MT, int NW, int U>
+inline void go(const Args& g, hipStream_t st) {
+  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + 16 * NT - 1) / (16 * NT))), NW * 64, 0, st>>>(g);
+}
+
+// Weight rows per workgroup: a workgroup also reads its rows' x, 16 rows of it per 16 weight rows, so wide outputs take 32 or
+// 64 weight rows per pass over x once that leaves the chip full (16 rows of x, K 2048, us by 16 / 32 / 64 weight rows: N 4096 7.1 /
+// 8.4 / 12.2, N 8192 11.1 / 9.7 / 12.7, N 32000 34.8 / 29.9 / 27.2).  With up to four rows x costs next to nothing and two waves of
+// twice the depth per workgroup are best (N 8192, one row: 8.1 us against 9.5).  17 to 32 rows: 32 weight rows from N 5120.
+inline void launch(const Args& g, hipStream_t st) {
+  if (g.M > 16) {
+    if (g.N < 5120) go<1, 2, 4, 8>(g, st);
+    else go<2, 2, 4, 4>(g, st);
+  } else if (g.M <= 4 && g.N >= 6144) {
+    go<1, 1, 2, 8>(g, st);
+  } else if (g.N < 5120) {
+    go<1, 1, 4, 8>(g, st);
+  } else if (g.N < 24576) {
+    go<2, 1, 4, 8>(g, st);
+  } else {
+    go<4, 1, 4, 4>(g, st);
+  }
+}
+
+}  // namespace stream_linear

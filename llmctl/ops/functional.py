@@ -376,6 +376,19 @@ def kv_cache_write(k, v, k_cache, v_cache, slot_mapping):
         ref.kv_cache_write(k, v, k_cache, v_cache, slot_mapping)
 
 
+def qkv_split_cache(qkv, nq: int, nkv: int, k_cache, v_cache, slots):
+    """``qkv [T, (nq + 2 nkv) D]`` of a model without rotary positions: K and V rows to the paged cache at ``slots`` (-1 =
+    skip), q as ``[T, nq, D]``; returns (q, k, v), k and v as views of ``qkv`` where that is possible."""
+    T = qkv.shape[0]
+    x = qkv.view(T, nq + 2 * nkv, -1)
+    q, k, v = x[:, :nq], x[:, nq:nq + nkv], x[:, nq + nkv:]
+    if use_native(qkv) and qkv.is_contiguous() and x.shape[2] % 8 == 0:
+        return native().qkv_split_cache(qkv, nq, nkv, k_cache, v_cache, slots), k, v
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    kv_cache_write(k, v, k_cache, v_cache, slots)
+    return q, k, v
+
+
 def paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale: Optional[float] = None):
     scale = scale if scale is not None else q.shape[-1] ** -0.5
     if use_native(q):
@@ -419,32 +432,48 @@ def paged_prefill_attention(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, s
 SKINNY_CONFIGS: dict = {}  # (M, N, K) -> tuned config (0 = hipBLASLt), from a tuning cache
 
 
-def decode_linear(x, w, b=None):
-    """``x @ w^T (+ b)`` for decode-shaped inputs: the weight-streaming MFMA kernels
-    (``csrc/skinny_gemm.hip``) where they beat hipBLASLt on uncached weights
-    (``profiles/skinny_sweep_r2*.jsonl``): every projection up to 16 tokens (at 16 tokens the
-    LDS-staged v2 kernel: QKV 3.78 vs 3.55 TB/s, up 3.89 vs 3.35, down 3.16 vs 2.07) and the
-    4096 x 4096 o-projection up to 32; wide projections at 17-32 tokens stay on hipBLASLt, and so
-    does the vocabulary projection (out features >= 16384) from 8 tokens (GPT-7B LM head at 16
-    tokens: 59.7 vs 68.5 us, ``profiles/decode_gemm_nt_r5.txt``).
-    Knob ``skinny_gemm``: ``off`` / ``all`` force the library / kernel path (A/B)."""
+_ROW_ACTS = {None: 0, "gelu": 2}  # the tanh form, as :func:`gelu`
+
+
+def stream_ok(x, w, b=None) -> bool:
+    """Does ``csrc/stream_linear.h`` take this product, and is it the fastest form of it?  At most 32 rows, bf16, K a multiple of 8,
+    aligned rows.  Up to 16 rows every output width; few outputs of a deep product (fewer than 4096 of more than 6144) and, with 17
+    to 32 rows, anything deeper than 2048 or wider than 8192 go to the library, which splits K over the chip (tables beside the
+    kernel)."""
+    if not (x.dim() == 2 and 1 <= x.shape[0] <= 32 and use_native(x)):
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    pays = (K <= 6144 or N >= 4096) if M <= 16 else (K <= 2048 and N <= 8192)
+    return (pays and K % 8 == 0 and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.stride(1) == 1
+            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous())))
+
+
+def decode_linear(x, w, b=None, act: Optional[str] = None):
+    """``act(x @ w^T (+ b))`` for decode-shaped inputs (``act``: None or ``gelu``): the weight-streaming kernels where they beat
+    hipBLASLt on uncached weights, bias and activation in the same launch (``csrc/stream_linear.h``; a tuned configuration
+    or knob ``skinny_gemm`` = ``all`` picks ``csrc/skinny_gemm.hip``, ``off`` the library).  Other inputs: the library and an
+    activation pass."""
     from llmctl.exec.linear import forward_linear
 
     mode = knobs().skinny_gemm
     M = x.shape[0] if x.dim() == 2 else 0
+    y = None
     tuned = SKINNY_CONFIGS.get((M, w.shape[0], w.shape[1])) if SKINNY_CONFIGS and x.dim() == 2 else None
     if tuned is not None and mode == "auto" and use_native(x):
         if tuned == 0:
-            return torch.nn.functional.linear(x, w, b)
-        if x.is_contiguous() and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16:
-            return native().skinny_linear_cfg(x, w, b, tuned)
-    if (mode != "off" and use_native(x) and x.dim() == 2 and M <= 32 and x.dtype == torch.bfloat16
+            y = torch.nn.functional.linear(x, w, b)
+        elif x.is_contiguous() and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16:
+            y = native().skinny_linear_cfg(x, w, b, tuned)
+    if y is None and mode == "auto" and stream_ok(x, w, b):
+        return native().stream_linear(x, w, b, _ROW_ACTS[act])
+    if (y is None and mode == "all" and use_native(x) and x.dim() == 2 and M <= 32 and x.dtype == torch.bfloat16
             and w.dtype == torch.bfloat16 and w.shape[0] % 16 == 0 and x.shape[1] % 128 == 0
-            and x.is_contiguous() and w.is_contiguous() and (b is None or b.is_contiguous())
-            and (mode == "all" or (M <= 16 and not (M >= 8 and w.shape[0] >= 16384))
-                 or (w.shape[0] <= 4096 and x.shape[1] <= 4096))):
-        return native().skinny_linear(x, w, b)
-    return forward_linear(x, w, b)
+            and x.is_contiguous() and w.is_contiguous() and (b is None or b.is_contiguous())):
+        y = native().skinny_linear(x, w, b)
+    if y is None:
+        y = forward_linear(x, w, b)
+    return gelu(y) if act == "gelu" else y
 
 
 def _dequant(w, w_scale, dtype):
@@ -597,7 +626,7 @@ __all__ = [
     "transpose_",
     "rmsnorm", "add_rmsnorm", "layernorm", "add_layernorm", "rope_qkv", "flash_attention", "rope_flash_attention",
     "swiglu",
-    "gelu", "cross_entropy", "adamw_step_", "l2norm_sq", "kv_cache_write", "paged_attention_decode",
+    "gelu", "cross_entropy", "adamw_step_", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
     "sample", "decode_linear", "decode_linear_fp8", "decode_fused_ok", "decode_qkv_rope_cache", "decode_up_swiglu", "decode_attention_qkv", "up_swiglu",
     "decode_linear_add_rmsnorm", "rope_qkv_cache", "paged_prefill_attention", "prefill_work_list", "attn_merge_",
     "rms_rstd", "rowscale_ok", "linear_rowscale", "up_swiglu_rowscale", "linear_acc_",

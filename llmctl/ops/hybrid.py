@@ -364,6 +364,42 @@ def bias_topk_router(logits, bias, top: int, groups: int = 1, keep: int = 1, ren
     return ref.bias_topk_router(logits, bias, top, groups, keep, renorm)
 
 
+_ROW_ACTS = {None: 0, "gelu": 1, "relu2": 3}
+
+
+def rows_ok(x, w, b=None) -> bool:
+    """Whether :func:`rows_linear` takes this product of a few rows and is the fastest form of it (the rule of
+    :func:`llmctl.ops.functional.stream_ok`)."""
+    if x.dim() != 2 or x.shape[0] > 32:
+        return False
+    from .functional import stream_ok
+
+    return stream_ok(x, w, b)
+
+
+def rows_linear(x, w, b=None, act=None, act_cols=None, f32: bool = False):
+    """``x @ w^T (+ b)`` of at most 32 bf16 rows in one launch, ``act`` (``gelu`` / ``relu2``) on the first ``act_cols`` columns (None:
+    all), in bf16 or fp32 (``f32``).  Operands: :func:`rows_ok`."""
+    return native_hybrid().rows_linear(x, w, b, _ROW_ACTS[act], w.shape[0] if act_cols is None else act_cols, f32)
+
+
+def linear(x, w, b=None):
+    """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), others are the library's product."""
+    return rows_linear(x, w, b) if rows_ok(x, w, b) else torch.nn.functional.linear(x, w, b)
+
+
+def linear_f32(x, w):
+    """``x @ w^T`` with an fp32 result (inputs in their own dtype, fp32 accumulation)."""
+    if x.dtype == torch.float32:
+        return torch.nn.functional.linear(x, w)
+    if rows_ok(x, w):
+        return rows_linear(x, w, f32=True)
+    try:
+        return torch.mm(x, w.t(), out_dtype=torch.float32)
+    except (TypeError, RuntimeError):
+        return torch.nn.functional.linear(x, w).float()
+
+
 _EXPERT_ACTS = {"relu2": 0, "swiglu": 1, "gelu": 2}
 MAX_EXPERTS = 128  # the expert kernels take the weights' addresses as arguments
 

@@ -441,12 +441,14 @@ class InferenceEngine:
         if self.rope is not None:
             return ops.rope_qkv_cache(qkv, self.rope[0], self.rope[1], layer.nq, layer.nkv, seq_len, positions,
                                       kc, vc, slots)
-        T = qkv.shape[0]
-        x = qkv.view(T, layer.nq + 2 * layer.nkv, layer.D)
-        q, k, v = (x[:, :layer.nq].contiguous(), x[:, layer.nq:layer.nq + layer.nkv].contiguous(),
-                   x[:, layer.nq + layer.nkv:].contiguous())
-        ops.kv_cache_write(k, v, kc, vc, slots)
-        return q, k, v
+        return ops.qkv_split_cache(qkv, layer.nq, layer.nkv, kc, vc, slots)
+
+    def _row_linear(self, x, w, b):
+        """A row-parallel projection with its bias: in the product's epilogue when nothing is reduced in between."""
+        if self.tp == 1:
+            return ops.decode_linear(x, w, b)
+        y = self._reduce(ops.decode_linear(x, w))
+        return y if b is None else y + b
 
     def _mlp(self, layer, xn):
         if layer.moe is not None:  # routed experts (host-side split sizes: eager, no graphs)
@@ -455,13 +457,9 @@ class InferenceEngine:
             # prefill-sized (T % 256 == 0): the SwiGLU rides on the gate/up GEMM's epilogue
             act = (ops.up_swiglu(xn, layer.w_up, layer.b_up) if xn.shape[0] >= 256 and xn.shape[0] % 256 == 0
                    else ops.swiglu(ops.decode_linear(xn, layer.w_up, layer.b_up)))
-            out = ops.decode_linear(act, layer.w_down)
         else:
-            out = ops.decode_linear(ops.gelu(ops.decode_linear(xn, layer.w_up, layer.b_up)), layer.w_down)
-        out = self._reduce(out)  # row-parallel down projection
-        if layer.b_down is not None:
-            out = out + layer.b_down
-        return out
+            act = ops.decode_linear(xn, layer.w_up, layer.b_up, act="gelu")
+        return self._row_linear(act, layer.w_down, layer.b_down)
 
     def _final(self, x, res):
         m = self.model
@@ -548,9 +546,7 @@ class InferenceEngine:
             else:
                 o = ops.paged_prefill_attention(q.view(T, layer.nq, layer.D), kc[li], vc[li], bt, cu, ctx,
                                                 work=work)
-            a = self._reduce(ops.decode_linear(o.view(T, -1), layer.wo))
-            if layer.bo is not None:
-                a = a + layer.bo
+            a = self._row_linear(o.view(T, -1), layer.wo, layer.bo)
             xn, res = self._norm(layer, a, res, "mlp")
             x = self._mlp(layer, xn)
         self.stats["prefill_tokens"] += T
@@ -611,9 +607,7 @@ class InferenceEngine:
             od = ops.paged_attention_decode(q[Tp:].reshape(Td, layer.nq, layer.D).contiguous(), kc[li], vc[li], bt_d,
                                             ctx_d)
             o = torch.cat([op.reshape(Tp, -1), od.reshape(Td, -1)])
-            a = self._reduce(ops.decode_linear(o, layer.wo))
-            if layer.bo is not None:
-                a = a + layer.bo
+            a = self._row_linear(o, layer.wo, layer.bo)
             xn, res = self._norm(layer, a, res, "mlp")
             x = self._mlp(layer, xn)
         self.stats["prefill_tokens"] += Tp
@@ -651,9 +645,7 @@ class InferenceEngine:
             xn, res = self._norm(layer, x, res, "attn")
             q, k, v = self._qkv(layer, xn, positions, self.max_model_len, kc[li], vc[li], slots)
             o = ops.paged_attention_decode(q, kc[li], vc[li], block_tables, ctx_lens)
-            a = self._reduce(ops.decode_linear(o.view(o.shape[0], -1), layer.wo))
-            if layer.bo is not None:
-                a = a + layer.bo
+            a = self._row_linear(o.view(o.shape[0], -1), layer.wo, layer.bo)
             xn, res = self._norm(layer, a, res, "mlp")
             x = self._mlp(layer, xn)
         return self._final(x, res)

@@ -1,0 +1,55 @@
+"""Few-row projections (``csrc/stream_linear.h``) against float64: row counts at the edges of the row tiles and of the launch rule,
+outputs that are no multiple of 4, 16 or 64, K tails, strided rows, bias, activations on some of the columns; and the split of
+an unrotated QKV row into q and the paged cache."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _act(name, y):
+    F = torch.nn.functional
+    return {None: lambda v: v, "gelu": F.gelu, "gelu_tanh": lambda v: F.gelu(v, approximate="tanh"), "relu2": lambda v: torch.relu(v).square()}[name](y)
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(3, 8), (17, 40), (64, 768), (200, 2056), (5119, 96), (5120, 64), (6150, 136), (24570, 72), (24600, 200), (2048, 4096)])
+def test_rows_linear_against_float64(M, N, K):
+    from llmctl.ops._lib import native, native_hybrid
+
+    g = torch.Generator(device="cuda").manual_seed(M * 7 + N)
+    x = torch.randn(M, K + 16, device="cuda", generator=g).bfloat16()[:, 8:8 + K]  # strided rows, 16-byte aligned
+    w = (torch.randn(N, K, device="cuda", generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    y = x.double() @ w.double().t() + b.double()
+    cols = N // 2 + 1
+    for act, code in ((None, 0), ("gelu", 1), ("relu2", 3)):
+        want = torch.cat([_act(act, y[:, :cols]), y[:, cols:]], 1)
+        got = native_hybrid().rows_linear(x, w, b, code, cols, True)
+        # fp32 sums of K bf16 products and an fp32 activation: K ulp at most, far less in practice
+        assert (got.double() - want).norm() <= 1e-5 * want.norm()
+        half = native_hybrid().rows_linear(x, w, b, code, cols, False)
+        assert torch.equal(half, got.bfloat16())  # bf16 results are the fp32 ones, rounded once
+    want = _act("gelu_tanh", x.double() @ w.double().t())
+    got = native().stream_linear(x, w, None, 2)
+    assert (got.double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("T,nq,nkv,D", [(1, 12, 12, 64), (5, 4, 2, 64), (33, 3, 1, 128)])
+def test_qkv_split_cache(T, nq, nkv, D, dtype):
+    from llmctl import ops
+
+    g = torch.Generator(device="cuda").manual_seed(T)
+    qkv = torch.randn(T, (nq + 2 * nkv) * D, device="cuda", generator=g).bfloat16()
+    caches = [torch.zeros(6, 16, nkv, D, device="cuda").to(dtype) for _ in range(4)]
+    slots = torch.randperm(96, device="cuda", generator=g)[:T]
+    slots[T // 2] = -1
+    q, k, v = ops.qkv_split_cache(qkv, nq, nkv, caches[0], caches[1], slots)
+    x = qkv.view(T, nq + 2 * nkv, D)
+    ops.kv_cache_write(x[:, nq:nq + nkv].contiguous(), x[:, nq + nkv:].contiguous(), caches[2], caches[3], slots)
+    assert torch.equal(q, x[:, :nq]) and q.is_contiguous()
+    assert torch.equal(k, x[:, nq:nq + nkv]) and torch.equal(v, x[:, nq + nkv:])
+    for a, b in ((0, 2), (1, 3)):
+        assert torch.equal(caches[a].view(torch.uint8), caches[b].view(torch.uint8))
