@@ -303,14 +303,17 @@ __global__ __launch_bounds__(256) void latent_attn_decode_kernel(const T* __rest
   }
 }
 
-// latent_attn_mfma.hip: the matrix-core form for bf16 shapes that fit it
+// latent_attn_mfma.hip: the matrix-core form for bf16 shapes that fit it (the check holds for both forms)
 bool latent_attn_mfma_ok(const at::Tensor& qa, int64_t rk, int64_t rs, int64_t koff, bool turn_back);
 // capped scores are built into the plain softmax form only, for keys up to 256 wide
 static bool mfma_cap_ok(const RowAttnOpts& x, int64_t R) {
   return x.softcap == 0.0 || (x.ofreq == nullptr && x.sig_bias == nullptr && x.hscale == nullptr && R <= 256);
 }
-void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor* cu, const at::Tensor& ctx,
+void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu, const at::Tensor& ctx,
                       int64_t window, const float* sink, double scale, int64_t rk, int64_t max_q, at::Tensor& out, const RowAttnOpts& x);
+// one query row per sequence (row_decode.hip)
+void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
+                double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x);
 
 // ------------------------------------------------------------------------------------------ host
 static void check_cache(const at::Tensor& cache, const at::Tensor& like, int64_t R) {
@@ -452,7 +455,7 @@ at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, co
   at::Tensor out = at::empty({T, H, rk}, qa.options());
   if (T == 0 || ns == 0) return out;
   if (mfma && mfma_cap_ok(x, R) && (x.dist_a == nullptr || x.sig_bias != nullptr) && latent_attn_mfma_ok(qa, rk, cache.size(2) / groups, koff, x.ofreq != nullptr || x.sig_bias != nullptr)) {
-    latent_attn_mfma(qa, cache, bt, &cu, ctx, window, sink_p, scale, rk, max_q, out, x);
+    latent_attn_mfma(qa, cache, bt, cu, ctx, window, sink_p, scale, rk, max_q, out, x);
     return out;
   }
   const int VT = rk <= 32 ? 32 : (rk <= 64 ? 64 : 128);
@@ -499,7 +502,7 @@ at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, con
   at::Tensor out = at::empty({ns, H, rk}, qa.options());
   if (ns == 0) return out;
   if (mfma && mfma_cap_ok(x, R) && (x.dist_a == nullptr || x.sig_bias != nullptr) && latent_attn_mfma_ok(qa, rk, cache.size(2) / groups, koff, x.ofreq != nullptr || x.sig_bias != nullptr)) {
-    latent_attn_mfma(qa, cache, bt, nullptr, ctx, window, sink_p, scale, rk, 1, out, x);
+    row_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
     return out;
   }
   HYB_CHECK(rk <= 512, "generic decode kernel: value width <= 512");

@@ -1,10 +1,10 @@
-// Latent attention on the matrix cores (bf16; MFMA 32x32x16), prompt portions and decode rows alike.
+// Latent attention on the matrix cores (bf16; MFMA 32x32x16) for prompt portions; decode rows: row_decode.hip.
 //
 // The cache row [latent | rotary key] of width R is key and, in its first ``rank`` entries, value; the
 // queries come in the same layout (see latent_attn.hip).  This is the flash-attention forward of the
 // framework's paged prefill kernel re-cut for that layout:
 //   * a workgroup (4 waves) owns 128 query rows = TB tokens x HB heads of one sequence (HB = 1 for
-//     long portions, = the head count for decode rows and short portions, where the heads of a token
+//     long portions, = the head count for short portions, where the heads of a token
 //     fill the tile and share every key row);
 //   * tiles of 64 keys, gathered through the block table into LDS once per workgroup: a "row image"
 //     of all of R (in column blocks of 128) for S^T = K Q^T, and a "transposed-read image" of the
@@ -32,7 +32,7 @@ struct LArgs {
   const unsigned short* cache;
   unsigned short* out;
   const int* bt;
-  const int* cu;   // nullptr: one query row per sequence (decode)
+  const int* cu;
   const int* ctx;
   const float* sink;    // nullptr: no sink
   const float* hscale;  // nullptr or a factor on every head's scores
@@ -45,17 +45,11 @@ struct LArgs {
   int keep;                     // the window spares the keys at positions below this
   float scale_log2;
   float cap_log2, cap_inv2;     // CAP forms: x (log2 domain) = cap_log2 * tanh(s * scale); cap_inv2 = 2 log2(e) scale / cap
-  // decode rows with the key range split over blockIdx.x (few sequences would otherwise leave the chip
-  // idle): each split writes its unnormalised fp32 output and (running maximum, denominator) here
-  int nsplit;
-  float* ws_o;   // [rows, nsplit, rk]
-  float* ws_ml;  // [rows, nsplit, 2]
 };
 
 // ROT: the output's neighbour pairs are turned back by the query's position (a.ofreq); a template flag
 // so that the forms without it keep their register budget.  SIG: the weights are sigmoids of the scores
-// (after the distance penalty), not a softmax: no running maximum, no rescale, no denominator; the splits
-// of decode rows are merged as a plain sum (m = 0 everywhere, l = 1 in the first split only).  CAP: the scaled score
+// (after the distance penalty), not a softmax: no running maximum, no rescale, no denominator (l = 1).  CAP: the scaled score
 // s becomes cap tanh(s / cap) before masks and softmax (tanh y = 1 - 2 / (1 + e^(2y))).
 template <int NCB, int NDB, bool ROT, bool SIG = false, bool CAP = false>
 __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
@@ -74,12 +68,11 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
   const int hg = blockIdx.z / a.nvt, v0 = (blockIdx.z % a.nvt) * (NDB * 32);
   const int P = a.H / a.G;                       // query heads per kv group
   const int grp = hg / a.hpg, hsub = (hg % a.hpg) * a.HB;  // this workgroup's kv group, its first head inside it
-  const int q_begin = a.cu ? a.cu[n] : n;
-  const int qlen = a.cu ? a.cu[n + 1] - q_begin : 1;
+  const int q_begin = a.cu[n];
+  const int qlen = a.cu[n + 1] - q_begin;
   const int HB = a.HB, TB = 128 / HB;
-  const int split = a.nsplit > 1 ? blockIdx.x : 0;
   // prompt portions: the last query blocks of a sequence see the most keys; they are dispatched first
-  const int tok0 = a.nsplit > 1 ? 0 : (int)(gridDim.x - 1 - blockIdx.x) * TB;
+  const int tok0 = (int)(gridDim.x - 1 - blockIdx.x) * TB;
   if (tok0 >= qlen) return;
   const int ctx = a.ctx[n];
   const int pos0 = ctx - qlen;
@@ -112,14 +105,10 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
     l_i = 1.0f;
   }
   const float my_scale = a.scale_log2 * (a.hscale != nullptr ? a.hscale[headc] : 1.0f);
-  if (split > 0) {                                 // (the sink is counted by the first split only)
-    m_i = -INFINITY;
-    l_i = 0.f;
-  }
   float pen_a = 0.f, pen_b = 0.f, sig_b2 = 0.f;
   if constexpr (SIG) {
     m_i = 0.f;
-    l_i = split == 0 ? 1.f : 0.f;
+    l_i = 1.f;
     if (a.dist_a != nullptr) pen_a = a.dist_a[headc], pen_b = a.dist_b[headc];
     sig_b2 = a.sig_bias[headc] * kLog2e;
   }
@@ -134,12 +123,7 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
   const int kept0 = ((first_pos / a.chunk) * a.chunk) / LKB;
   const int n_kept = a.keep > 0 ? max(min((a.keep + LKB - 1) / LKB, t_first) - kept0, 0) : 0;
   auto tile_of = [&](int i) { return i < n_kept ? kept0 + i : t_first + i - n_kept; };
-  int t_lo = 0, t_hi = n_kept + t_end - t_first;
-  if (a.nsplit > 1) {
-    const int per = (t_hi - t_lo + a.nsplit - 1) / a.nsplit;
-    t_lo += split * per;
-    t_hi = min(t_hi, t_lo + per);
-  }
+  const int t_lo = 0, t_hi = n_kept + t_end - t_first;
   // this wave's rows: positions [w_first, w_last]
   const int w_first = pos0 + min(tok0 + (wave * 32) / HB, qlen - 1);
   const int w_last = pos0 + min(tok0 + (wave * 32 + 31) / HB, qlen - 1);
@@ -317,21 +301,7 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
         }
   }
 
-  if (valid && a.nsplit > 1) {
-    const long rowi = (long)(q_begin + my_tok) * a.H + my_head;
-    float* Wp = a.ws_o + (rowi * a.nsplit + split) * a.rk;
-#pragma unroll
-    for (int d = 0; d < NDB; ++d)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int col = v0 + d * 32 + 8 * g + 4 * hh;
-        if (col < a.rk) *reinterpret_cast<float4*>(Wp + col) = make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
-      }
-    if (v0 == 0 && hh == 0) {
-      a.ws_ml[(rowi * a.nsplit + split) * 2] = m_i;
-      a.ws_ml[(rowi * a.nsplit + split) * 2 + 1] = l_i;
-    }
-  } else if (valid) {
+  if (valid) {
     const float inv = 1.f / l_i;
     unsigned short* Op = a.out + ((long)(q_begin + my_tok) * a.H + my_head) * a.rk;
 #pragma unroll
@@ -360,34 +330,6 @@ __global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
   }
 }
 
-// out[row] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M = max_s m_s (splits that saw nothing: m = -inf, l = 0)
-__global__ void latent_split_merge_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, unsigned short* __restrict__ out,
-                                          int nsplit, int rk, const float* __restrict__ ofreq, const int* __restrict__ ctx, int H) {
-  const long row = blockIdx.x;
-  const float pos = ofreq != nullptr ? (float)(ctx[row / H] - 1) : 0.f;  // one row per sequence: its last position
-  const float* ml = ws_ml + row * nsplit * 2;
-  float M = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) M = fmaxf(M, ml[2 * s]);
-  float L = 0.f;
-  for (int s = 0; s < nsplit; ++s) L += ml[2 * s + 1] * (ml[2 * s] == -INFINITY ? 0.f : fast_exp2(ml[2 * s] - M));
-  const float inv = 1.f / L;
-  for (int c = threadIdx.x; c < rk; c += blockDim.x) {
-    float v = 0.f, w = 0.f;  // column c and, for the turn back, its pair partner c ^ 1
-    for (int s = 0; s < nsplit; ++s)
-      if (ml[2 * s] != -INFINITY) {
-        const float f = fast_exp2(ml[2 * s] - M);
-        v += ws_o[(row * nsplit + s) * rk + c] * f;
-        if (ofreq != nullptr) w += ws_o[(row * nsplit + s) * rk + (c ^ 1)] * f;
-      }
-    if (ofreq != nullptr) {
-      float sn, cs;
-      sincosf(pos * ofreq[c >> 1], &sn, &cs);
-      v = (c & 1) ? v * cs - w * sn : v * cs + w * sn;
-    }
-    out[row * rk + c] = __bfloat16_as_ushort(__float2bfloat16(v * inv));
-  }
-}
-
 template <int NCB, bool ROT, bool SIG = false, bool CAP = false>
 void launch_ncb(const LArgs& a, int ndb, dim3 grid, hipStream_t st) {
   auto go = [&](auto kern, int NDBv) {
@@ -409,8 +351,8 @@ bool latent_attn_mfma_ok(const at::Tensor& qa, int64_t rk, int64_t rs, int64_t k
   return qa.scalar_type() == at::kBFloat16 && R % 8 == 0 && rk % 8 == 0 && rs % 8 == 0 && koff % 8 == 0 && R <= (turn_back ? 256 : 640) && qa.size(1) >= 1;
 }
 
-// cu == nullptr: one query row per sequence.  ``x`` carries the optional parts (see RowAttnOpts).
-void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor* cu, const at::Tensor& ctx,
+// ``x`` carries the optional parts (see RowAttnOpts).
+void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu, const at::Tensor& ctx,
                       int64_t window, const float* sink, double scale, int64_t rk, int64_t max_q, at::Tensor& out, const RowAttnOpts& x) {
   const int64_t H = qa.size(1), R = qa.size(2), ns = ctx.numel();
   const int64_t G = x.groups, P = H / G, rs = cache.size(2) / G;
@@ -425,27 +367,13 @@ void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::T
   const int hpg = (int)((P + HB - 1) / HB);  // head tiles per kv group
   const int hgroups = (int)G * hpg;
   HYB_CHECK(ns <= 65535 && hgroups * nvt <= 65535, "grid too large");
-  // decode rows: split the visible key tiles over workgroups until the launch has a few hundred of them
-  int nsplit = 1;
-  at::Tensor ws_o, ws_ml;
-  if (cu == nullptr && rk % 4 == 0) {
-    const int64_t span = std::min<int64_t>(std::min<int64_t>(window, x.chunk), x.max_ctx > 0 ? x.max_ctx : (int64_t)1 << 30);
-    const int tiles = (int)std::min<int64_t>((span + LKB - 1) / LKB + 1 + (x.keep_first + LKB - 1) / LKB, 1 << 20);
-    const long blocks = (long)ns * hgroups * nvt;
-    while (nsplit < tiles && nsplit < 32 && blocks * nsplit < 512) nsplit *= 2;
-    if (nsplit > 1) {
-      ws_o = at::empty({ns * H, nsplit, rk}, qa.options().dtype(at::kFloat));
-      ws_ml = at::empty({ns * H, nsplit, 2}, qa.options().dtype(at::kFloat));
-    }
-  }
   LArgs a{reinterpret_cast<const unsigned short*>(qa.data_ptr()), reinterpret_cast<const unsigned short*>(cache.data_ptr()),
-          reinterpret_cast<unsigned short*>(out.data_ptr()), bt.data_ptr<int>(), cu ? cu->data_ptr<int>() : nullptr, ctx.data_ptr<int>(),
+          reinterpret_cast<unsigned short*>(out.data_ptr()), bt.data_ptr<int>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
           sink, x.hscale, x.ofreq, x.dist_a, x.dist_b, x.sig_bias, (int)H, (int)R, (int)rk, (int)cache.size(1), (int)bt.size(1), (int)window, HB, nvt,
           (int)G, (int)rs, (int)x.koff, (int)x.chunk, hpg, (int)x.keep_first,
           (float)(scale * 1.4426950408889634), (float)(x.softcap * 1.4426950408889634),
-          x.softcap > 0.0 ? (float)(2.0 * 1.4426950408889634 * scale / x.softcap) : 0.f, nsplit, nsplit > 1 ? ws_o.data_ptr<float>() : nullptr,
-          nsplit > 1 ? ws_ml.data_ptr<float>() : nullptr};
-  dim3 grid(nsplit > 1 ? (unsigned)nsplit : (unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)(hgroups * nvt));
+          x.softcap > 0.0 ? (float)(2.0 * 1.4426950408889634 * scale / x.softcap) : 0.f};
+  dim3 grid((unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)(hgroups * nvt));
   hipStream_t st = cur_stream();
   if (x.softcap > 0.0) {  // built for keys up to 256 wide, plain softmax form (the caller checks)
     HYB_CHECK(x.hscale == nullptr && ncb <= 2, "capped scores: no per-head factor, keys up to 256 wide");
@@ -466,10 +394,6 @@ void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::T
       default: launch_ncb<5, false>(a, ndb, grid, st); break;
     }
   }
-  if (nsplit > 1)
-    latent_split_merge_kernel<<<dim3((unsigned)(ns * H)), 128, 0, st>>>(ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(),
-                                                                        reinterpret_cast<unsigned short*>(out.data_ptr()), nsplit, (int)rk,
-                                                                        x.ofreq, ctx.data_ptr<int>(), (int)H);
 }
 
 }  // namespace llmctl_hybrid
