@@ -27,7 +27,7 @@ than gemm64 for all of them (knob ``dgrad64``, see ``dgrad64_shape_ok``).
 
 from __future__ import annotations
 
-from typing import Callable, List, Optional
+from typing import Callable, List, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -320,6 +320,18 @@ class GradSink:
         for cb in self.callbacks:
             cb(p)
 
+    def open(self, p: torch.nn.Parameter) -> Tuple[torch.Tensor, bool]:
+        """A vector's flat gradient for a kernel to write, and whether it adds to it; ``close`` follows the launch."""
+        return self._target(p), not p._llmctl_fresh
+
+    close = _written
+
+    def add(self, p: torch.nn.Parameter, g: torch.Tensor) -> None:
+        """A gradient computed elsewhere (CPU and fp32 paths)."""
+        t = self._target(p)
+        t.copy_(g) if p._llmctl_fresh else t.add_(g)
+        self._written(p)
+
     def write(self, p: torch.nn.Parameter, dy2: torch.Tensor, x2: torch.Tensor) -> None:
         wgrad_into(self._target(p), dy2, x2, accumulate=not p._llmctl_fresh)
         self._written(p)
@@ -334,14 +346,28 @@ class GradSink:
         return dgu
 
 
+def bias_grad(b: torch.nn.Parameter, dy2: torch.Tensor) -> Optional[torch.Tensor]:
+    """Column sums of ``dy2``: into ``b``'s flat gradient if it has a sink (returns None), else as an ordinary gradient."""
+    from llmctl import ops
+
+    sink: Optional[GradSink] = getattr(b, "_llmctl_grad_sink", None)
+    if sink is not None:
+        g, add = sink.open(b)
+        ops.col_sum_(dy2, g, add)
+        sink.close(b)
+        return None
+    db = torch.empty(b.shape, dtype=dy2.dtype, device=dy2.device)
+    ops.col_sum_(dy2, db, False)
+    return db
+
+
 class _Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, b):
         ctx.save_for_backward(x, w)
         # keep the Parameter object itself: tensors coming back from saved_tensors can be
         # aliases (e.g. under activation checkpointing) that do not carry the sink
-        ctx.wparam = w
-        ctx.has_b = b is not None
+        ctx.wparam, ctx.bparam = w, b
         sink = getattr(w, "_llmctl_grad_sink", None)
         ctx.wt = None
         if sink is not None and ctx.needs_input_grad[0] and not dgrad64_shape_ok(x.numel() // x.shape[-1], w):
@@ -375,7 +401,7 @@ class _Linear(torch.autograd.Function):
                 dx = F.linear(dy, ctx.wt)
             else:
                 dx = dy.matmul(w)
-        db = dy2.sum(0) if (ctx.has_b and ctx.needs_input_grad[2]) else None
+        db = bias_grad(ctx.bparam, dy2) if (ctx.bparam is not None and ctx.needs_input_grad[2]) else None
         return dx, dw, db
 
 

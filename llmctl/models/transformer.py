@@ -367,6 +367,8 @@ class DecoderLayer(nn.Module):
             o = ops.rope_flash_attention(qkv, rope[0], rope[1], self.nq, self.nkv, B, S, positions, doc_start,
                                          inplace=True)
             return self._attn_out(o, B, S)
+        if rope is None and self.pc.cp_size == 1:
+            return self._attn_out(ops.qkv_flash_attention(qkv, self.nq, self.nkv, B, S, doc_start), B, S)
         if rope is not None:
             q, k, v = ops.rope_qkv(qkv, rope[0], rope[1], self.nq, self.nkv, S, positions)
         else:
@@ -388,6 +390,8 @@ class DecoderLayer(nn.Module):
         return self._attn_out(o, B, S)
 
     def _attn_out(self, o, B, S):
+        if self.pc.tp_size == 1:  # the bias in the GEMM
+            return linear(o.reshape(B * S, self.nq * self.D), self.wo, self.bo)
         if self._async_sp():  # o-proj GEMM with the SP reduce-scatter overlapped
             out = async_tp.row_parallel_sp(o.reshape(B * S, self.nq * self.D), self.wo, self.pc.tp_group)
         else:
@@ -416,6 +420,8 @@ class DecoderLayer(nn.Module):
                 out = _SwiGLUDown.apply(gu, self.w_down, self.pc.activation_checkpoint == "selective")
             else:
                 hdn = ops.gelu(linear(x, self.w_up, self.b_up))
+                if self.pc.tp_size == 1:  # the bias in the GEMM
+                    return linear(hdn, self.w_down, self.b_down)
                 out = linear(hdn, self.w_down)
             out = self._row_out(out)
         if self.b_down is not None:

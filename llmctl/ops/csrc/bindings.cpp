@@ -22,6 +22,9 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("layernorm_fwd(Tensor x, Tensor w, Tensor b, float eps) -> (Tensor, Tensor, Tensor)");
   m.def("add_layernorm_fwd(Tensor x, Tensor residual, Tensor w, Tensor b, float eps) -> (Tensor, Tensor, Tensor, Tensor)");
   m.def("layernorm_bwd(Tensor dy, Tensor x, Tensor w, Tensor mu, Tensor rstd, Tensor? dres) -> (Tensor, Tensor, Tensor)");
+  m.def("norm_bwd_into(Tensor dy, Tensor x, Tensor w, Tensor? mu, Tensor rstd, Tensor? dres, Tensor(a!) dw, bool add_w, Tensor(b!)? db, bool add_b) -> Tensor");
+  // bias gradients (col_sum.hip)
+  m.def("col_sum_(Tensor x, Tensor(a!) out, bool add) -> ()");
   // elementwise (elementwise.hip)
   m.def("rope_qkv_fwd(Tensor qkv, Tensor cos, Tensor sin, int nq, int nkv, int seq_len, Tensor? positions) -> (Tensor, Tensor, Tensor)");
   m.def("rope_qk_inplace_(Tensor(a!) qkv, Tensor cos, Tensor sin, int nq, int nkv, int seq_len, Tensor? positions) -> ()");
@@ -40,7 +43,7 @@ TORCH_LIBRARY(llmctl, m) {
   // attention (flash_attn_fwd.hip / flash_attn_bwd.hip)
   m.def("flash_attn_fwd(Tensor q, Tensor k, Tensor v, float scale, bool causal, Tensor? doc_start=None) -> (Tensor, Tensor)");
   m.def("flash_attn_bwd(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, float scale, bool causal, Tensor? doc_start=None) -> (Tensor, Tensor, Tensor)");
-  m.def("flash_attn_bwd_qkv(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, float scale, bool causal, Tensor? doc_start, Tensor cos, Tensor sin, Tensor? positions, int seq_len) -> Tensor");
+  m.def("flash_attn_bwd_qkv(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor o, Tensor lse, float scale, bool causal, Tensor? doc_start, Tensor? cos, Tensor? sin, Tensor? positions, int seq_len) -> Tensor");
   m.def("fa_bwd_ablate(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor delta, Tensor lse, Tensor(a!) dq, Tensor(b!) dk, Tensor(c!) dv, int abl) -> ()");
   // serving (paged_attn.hip, sampling.hip)
   m.def("qkv_split_cache(Tensor qkv, int nq, int nkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slots) -> Tensor");

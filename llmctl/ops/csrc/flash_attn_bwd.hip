@@ -1568,11 +1568,13 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> flash_attn_bwd(const at::Tensor& 
 // Attention backward with the RoPE backward fused into the dQ / dK stores: returns the gradient of
 // the QKV projection output dqkv [B*S, (Hq + 2 Hkv) * D] directly (dq / dk rotated back by their
 // positions, dv copied), the layout ``rope_qkv`` split the projection from.  cos / sin: fp32
-// [>= max position, D/2]; positions: int32 [B*S] or none (position = token % seq_len).
+// [>= max position, D/2]; positions: int32 [B*S] or none (position = token % seq_len).  Without cos / sin
+// nothing is rotated: the gradient of a projection that was attended as it is.
 at::Tensor flash_attn_bwd_qkv(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
                               const at::Tensor& o, const at::Tensor& lse, double scale, bool causal,
-                              const c10::optional<at::Tensor>& doc_start, const at::Tensor& cos_t,
-                              const at::Tensor& sin_t, const c10::optional<at::Tensor>& positions, int64_t seq_len) {
+                              const c10::optional<at::Tensor>& doc_start, const c10::optional<at::Tensor>& cos_o,
+                              const c10::optional<at::Tensor>& sin_o, const c10::optional<at::Tensor>& positions,
+                              int64_t seq_len) {
   LLMCTL_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4 && o.dim() == 4 && dout.dim() == 4,
                "flash_attn_bwd_qkv: [B,S,H,D] tensors");
   const int B = q.size(0), S = q.size(1), Hq = q.size(2), D = q.size(3);
@@ -1589,17 +1591,22 @@ at::Tensor flash_attn_bwd_qkv(const at::Tensor& dout, const at::Tensor& q, const
                      t->stride(1) % 8 == 0 && t->stride(2) % 8 == 0 &&
                      (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0,
                  "flash_attn_bwd_qkv: bf16, d-contiguous, 16-B aligned rows");
-  LLMCTL_CHECK(cos_t.is_cuda() && sin_t.is_cuda() && cos_t.scalar_type() == at::kFloat &&
-                   sin_t.scalar_type() == at::kFloat && cos_t.is_contiguous() && sin_t.is_contiguous() &&
-                   cos_t.dim() == 2 && cos_t.size(1) == D / 2 && sin_t.sizes() == cos_t.sizes(),
-               "flash_attn_bwd_qkv: cos/sin fp32 contiguous [P, D/2]");
-  const bool has_pos = positions.has_value() && positions->defined();
-  if (has_pos) {
-    LLMCTL_CHECK(positions->is_cuda() && positions->scalar_type() == at::kInt && positions->is_contiguous() &&
-                     positions->numel() == (long)B * S,
-                 "flash_attn_bwd_qkv: positions int32 [B*S]");
-  } else {
-    LLMCTL_CHECK(seq_len > 0 && seq_len <= cos_t.size(0), "flash_attn_bwd_qkv: seq_len within the tables");
+  const bool rope = cos_o.has_value() && cos_o->defined();
+  LLMCTL_CHECK(rope == (sin_o.has_value() && sin_o->defined()), "flash_attn_bwd_qkv: cos and sin together");
+  const bool has_pos = rope && positions.has_value() && positions->defined();
+  if (rope) {
+    const at::Tensor &cos_t = *cos_o, &sin_t = *sin_o;
+    LLMCTL_CHECK(cos_t.is_cuda() && sin_t.is_cuda() && cos_t.scalar_type() == at::kFloat &&
+                     sin_t.scalar_type() == at::kFloat && cos_t.is_contiguous() && sin_t.is_contiguous() &&
+                     cos_t.dim() == 2 && cos_t.size(1) == D / 2 && sin_t.sizes() == cos_t.sizes(),
+                 "flash_attn_bwd_qkv: cos/sin fp32 contiguous [P, D/2]");
+    if (has_pos) {
+      LLMCTL_CHECK(positions->is_cuda() && positions->scalar_type() == at::kInt && positions->is_contiguous() &&
+                       positions->numel() == (long)B * S,
+                   "flash_attn_bwd_qkv: positions int32 [B*S]");
+    } else {
+      LLMCTL_CHECK(seq_len > 0 && seq_len <= cos_t.size(0), "flash_attn_bwd_qkv: seq_len within the tables");
+    }
   }
   const c10::DeviceGuard g(q.device());
   const long W = (long)(Hq + 2 * Hkv) * D;
@@ -1613,8 +1620,8 @@ at::Tensor flash_attn_bwd_qkv(const at::Tensor& dout, const at::Tensor& q, const
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), dout.stride(0), dout.stride(1), dout.stride(2),
             (float)scale, (float)(scale * 1.4426950408889634), nullptr, W, W, W,
-            cos_t.data_ptr<float>(), sin_t.data_ptr<float>(), has_pos ? positions->data_ptr<int>() : nullptr,
-            (int)(has_pos ? 1 : seq_len), bf_ptr(o), o.stride(0), o.stride(1), o.stride(2),
+            rope ? cos_o->data_ptr<float>() : nullptr, rope ? sin_o->data_ptr<float>() : nullptr,
+            has_pos ? positions->data_ptr<int>() : nullptr, (int)(has_pos ? 1 : seq_len), bf_ptr(o), o.stride(0), o.stride(1), o.stride(2),
             delta.data_ptr<float>(), nullptr, 0};
   auto rck = row_consts(a, lse);
   bool doc = false;

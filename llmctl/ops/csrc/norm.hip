@@ -9,7 +9,7 @@
 //
 // Replaces: the reference's HF RMSNorm (library op, SURVEY §2.5 "fused_rmsnorm" declared
 // plugin name, USER_GUIDE.md:268).
-#include "common.h"
+#include "col_reduce.h"
 
 namespace llmctl {
 namespace {
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void rstd_kernel(const unsigned short* __restr
 }
 
 template <int NV, bool LN, bool DRES>
-__global__ __launch_bounds__(256, LN ? 1 : 2) void norm_bwd_kernel(const unsigned short* __restrict__ dy,
+__global__ __launch_bounds__(256, LN && NV > 4 ? 1 : 2) void norm_bwd_kernel(const unsigned short* __restrict__ dy,
                                                                     const unsigned short* __restrict__ x,
                                                                     const unsigned short* __restrict__ w,
                                                                     const float* __restrict__ mu,
@@ -348,30 +348,6 @@ __global__ __launch_bounds__(256) void norm_bwd_wide_kernel(const unsigned short
   }
 }
 
-
-// sum partial rows [P, H] -> out[H] (bf16).  Block = 64 columns x 4 waves; wave w sums rows
-// w, w+4, ... (4 independent loads in flight per lane), then the 4 waves combine via LDS.
-__global__ __launch_bounds__(256) void col_reduce_kernel(const float* __restrict__ part, int P, int H,
-                                                          unsigned short* __restrict__ out) {
-  __shared__ float red[4][64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + lane;
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  if (c < H) {
-    int p = w;
-    for (; p + 12 < P; p += 16) {
-      s0 += part[(size_t)p * H + c];
-      s1 += part[(size_t)(p + 4) * H + c];
-      s2 += part[(size_t)(p + 8) * H + c];
-      s3 += part[(size_t)(p + 12) * H + c];
-    }
-    for (; p < P; p += 4) s0 += part[(size_t)p * H + c];
-  }
-  red[w][lane] = (s0 + s1) + (s2 + s3);
-  __syncthreads();
-  if (w == 0 && c < H) out[c] = f2bf(red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane]);
-}
-
 int fwd_grid(int T) {
   int blocks = (T + kWaves - 1) / kWaves;
   return std::max(1, std::min(blocks, num_cus() * 8));
@@ -405,12 +381,14 @@ void launch_fwd(const at::Tensor& x, const at::Tensor* res, const at::Tensor& w,
 
 template <bool LN>
 void launch_bwd(const at::Tensor& dy, const at::Tensor& x, const at::Tensor& w, const at::Tensor* mu,
-                const at::Tensor& rstd, const c10::optional<at::Tensor>& dres, at::Tensor& dx, at::Tensor& dw,
-                at::Tensor* db) {
+                const at::Tensor& rstd, const c10::optional<at::Tensor>& dres, at::Tensor& dx, const at::Tensor& dw,
+                const at::Tensor* db, bool add_w = false, bool add_b = false) {
   const int T = x.size(0), H = x.size(1);
   const int nv = (H + 511) / 512;
-  // pipelined kernel (H <= 4096): 2 blocks per CU for RMSNorm (LDS dW slabs, 64 KB each)
-  const int per_cu = (nv <= 8 && !LN) ? 2 : 1;
+  // blocks per CU, the pipelined kernel: its dW slab is 64 KB at H = 4096 (RMSNorm: two fit LDS), and LayerNorm holds two slabs.  More
+  // blocks than that cost more in slabs cleared and reduced than they hide (LayerNorm with residual, 8192 rows, kernel and
+  // reduction in us at 1 / 2 / 3 / 4 blocks: 768 columns 20.9 / 18.2 / 18.5 / 19.9, 1600 columns 33.4 / 29.2 / 34.6 / 36.1)
+  const int per_cu = nv <= (LN ? 4 : 8) ? 2 : 1;
   const int grid = std::max(1, std::min((T + kWaves - 1) / kWaves, per_cu * num_cus()));
   auto opts = x.options().dtype(at::kFloat);
   at::Tensor dw_part = at::empty({grid, H}, opts);
@@ -450,11 +428,9 @@ void launch_bwd(const at::Tensor& dy, const at::Tensor& x, const at::Tensor& w, 
   }
 #undef LAUNCH
 #undef LAUNCHW
-  hipLaunchKernelGGL(col_reduce_kernel, dim3((H + 63) / 64), dim3(256), 0, s, dw_part.data_ptr<float>(), grid, H,
-                     bf_mut(dw));
-  if (LN)
-    hipLaunchKernelGGL(col_reduce_kernel, dim3((H + 63) / 64), dim3(256), 0, s, db_part.data_ptr<float>(), grid, H,
-                       bf_mut(*db));
+  launch_col_reduce(ColReduceArgs{{dw_part.data_ptr<float>(), LN ? db_part.data_ptr<float>() : nullptr},
+                                  {dw.data_ptr(), LN ? db->data_ptr() : nullptr}, {add_w, add_b}, grid, H},
+                    LN ? 2 : 1, dw.scalar_type() == at::kFloat, s);
 }
 
 void check2d(const at::Tensor& t, const char* n) {
@@ -539,6 +515,25 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> layernorm_bwd(const at::Tensor& d
   return {dx, dw, db};
 }
 
+// The same with the weights' gradients stored (or added, ``add_w`` / ``add_b``) into existing vectors (bf16, or fp32 main
+// gradients); mu and db belong to LayerNorm.  Returns dx.
+at::Tensor norm_bwd_into(const at::Tensor& dy, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& mu,
+                         const at::Tensor& rstd, const c10::optional<at::Tensor>& dres, at::Tensor dw, bool add_w,
+                         const c10::optional<at::Tensor>& db, bool add_b) {
+  check2d(dy, "dy");
+  check2d(x, "x");
+  if (dres.has_value() && dres->defined()) check2d(*dres, "dres");
+  const bool ln = mu.has_value() && mu->defined();
+  LLMCTL_CHECK(ln == (db.has_value() && db->defined()), "norm_bwd_into: mean and bias gradient together");
+  LLMCTL_CHECK(col_out_ok(dw, x.size(1)) && (!ln || (col_out_ok(*db, x.size(1)) && db->scalar_type() == dw.scalar_type())),
+               "norm_bwd_into: gradients are contiguous bf16 or fp32 vectors of one type");
+  const c10::DeviceGuard g(x.device());
+  auto dx = at::empty_like(x);
+  if (ln) launch_bwd<true>(dy, x, w, &*mu, rstd, dres, dx, dw, &*db, add_w, add_b);
+  else launch_bwd<false>(dy, x, w, nullptr, rstd, dres, dx, dw, nullptr, add_w);
+  return dx;
+}
+
 at::Tensor rms_rstd(const at::Tensor& x, double eps) {
   check2d(x, "x");
   const int T = x.size(0), H = x.size(1);
@@ -570,6 +565,7 @@ TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
   m.impl("layernorm_fwd", &layernorm_fwd);
   m.impl("add_layernorm_fwd", &add_layernorm_fwd);
   m.impl("layernorm_bwd", &layernorm_bwd);
+  m.impl("norm_bwd_into", &norm_bwd_into);
 }
 
 }  // namespace llmctl

@@ -260,11 +260,16 @@ class TrainingEngine:
             solo = ("embed", "lm_head") if (pp > 1 and mc.tie_word_embeddings) else ()
             self.flat = FlatParameters(named, bucket_numel=bucket_numel, align=align, solo=solo,
                                        grad_dtype=grad_dtype)
-            # GEMM-written weight gradients (no AccumulateGrad pass); tied embeddings excluded
+            # kernel-written gradients (no AccumulateGrad pass); tied embeddings excluded
             from llmctl.exec.linear import GradSink
 
             tied = mc.tie_word_embeddings
             leafs = ("wqkv", "wo", "w_up", "w_down") + (() if tied else ("lm_head",))
+            # norm weights and biases too (their kernels write the flat gradient: no add and no fill per vector), the biases
+            # where every one of them goes through ``linear``
+            leafs += ("attn_norm_w", "mlp_norm_w", "final_norm_w", "attn_norm_b", "mlp_norm_b", "final_norm_b")
+            if pg.layout.tp == 1 and not mc.is_moe and not mc.gated_mlp:
+                leafs += ("bqkv", "bo", "b_up", "b_down")
             self.grad_sink = GradSink()
             self.flat.install_sinks(self.grad_sink, lambda n, p: n.split(".")[-1] in leafs)
         if pp > 1 and mc.tie_word_embeddings:

@@ -168,7 +168,7 @@ class FlatParameters:
     def install_sinks(self, sink, predicate) -> int:
         """Attach a :class:`llmctl.exec.linear.GradSink` to every parameter for which
         ``predicate(name, p)`` holds; their gradients are then written (beta=0 first) by
-        the backward GEMM, so ``zero_grad`` skips them."""
+        the backward's kernels, so ``zero_grad`` skips them."""
         n = 0
         for p in self.params:
             if predicate(self.names[id(p)], p):
@@ -193,7 +193,7 @@ class FlatParameters:
                 if g is None or g.data_ptr() != self.grad[off:].data_ptr():
                     p.grad = g = self.grad[off:off + p.numel()].view_as(p)
             if sink is not None:
-                if getattr(p, "_llmctl_grad_sink", None) is sink:
+                if getattr(p, "_llmctl_grad_sink", None) is sink and p.requires_grad:
                     sink.reset(p)
                 else:
                     g.zero_()
