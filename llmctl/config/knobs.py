@@ -40,7 +40,7 @@ class PerfKnobs:
     gemm64: bool = True            # in-house MFMA GEMMs (False: hipBLASLt everywhere -- A/B only)
     gemm64_config: int = 304       # gemm64 config: tile-order group + 100 * schedule variant + 1000 * split
     fwd64: str = "auto"            # forward x W^T on gemm64: auto (small-M / wide shapes) | all | off
-    dgrad64: str = "fused"         # data gradients on gemm64: fused (down projection) | all | off
+    dgrad64: str = "auto"          # data gradients on gemm64: auto (by tokens) | fused (down projection) | all | off
     wgrad_kernel: bool = True      # weight gradients on the MFMA kernels (False: hipBLASLt)
     swiglu_bwd: str = "side"       # SwiGLU backward: side (wgrad side job) | epilogue | separate
     dgrad_transpose: bool = True   # hipBLASLt data gradients through a W^T copy

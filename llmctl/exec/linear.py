@@ -10,19 +10,15 @@ beta = 1 epilogue, free accumulation) on later gradient-accumulation micro-steps
 then notifies the DP overlap engine that the parameter's gradient is ready — the same
 signal ``register_post_accumulate_grad_hook`` gives for ordinary parameters.
 
-Data gradient through a transposed weight copy: ``dX = dY W`` (the "NN" GEMM) runs ~13 %
-slower on hipBLASLt than the forward's "TN" layout at the GPT-7B shapes
-(``profiles/gemm_tunable_dgradT_r1.log``: 7.27 -> 6.37 ms per layer).  Sinked weights therefore
-keep a bf16 ``W^T`` copy, refreshed by the transpose HIP kernel the first time the weight is
-used after an optimizer step (``GradSink.epoch``; under ZeRO-1/2 that is after the layer's
-all-gather has landed), and the backward computes ``dX = F.linear(dY, W^T)``.  Cost: one
-bf16 copy of the projection weights and ~2 x 13.5 GB of HBM transpose traffic per step.
-
-Round 2: weight gradients run on the in-house 64-deep MFMA kernel (``gemm64_ex``,
-llmctl/ops/csrc/gemm64.hip; 20-40 % over hipBLASLt on the GPT-7B shapes).  Data gradients: the
-down projection's runs on gemm64 with the SwiGLU backward in its epilogue; the others run on
-hipBLASLt's forward layout through the ``W^T`` copies, which measured 0.7 % faster per step
-than gemm64 for all of them (knob ``dgrad64``, see ``dgrad64_shape_ok``).
+Data gradients: up to 16384 tokens a step they run on the in-house 64-deep MFMA kernel, which reads W as it is (``gemm64_ex``,
+llmctl/ops/csrc/gemm64.hip), as the weight gradients do (20-40 % over hipBLASLt on the GPT-7B shapes).  Beyond that, and for
+shapes it does not take, large weights go through a transposed copy: ``dX = dY W`` (the "NN" GEMM) runs ~13 % slower on
+hipBLASLt than the forward's "TN" layout at the GPT-7B shapes (``profiles/gemm_tunable_dgradT_r1.log``: 7.27 -> 6.37 ms per
+layer).  Such weights keep a bf16 ``W^T`` copy, refreshed by the transpose HIP kernel the first time the weight is used after an
+optimizer step (``GradSink.epoch``; under ZeRO-1/2 that is after the layer's all-gather has landed), and the backward
+computes ``dX = F.linear(dY, W^T)``.  Cost: one bf16 copy of the projection weights and ~2 x 13.5 GB of HBM transpose traffic per
+step.  The down projection's data gradient can carry the SwiGLU backward in its epilogue.  Knob ``dgrad64``, see
+``dgrad64_shape_ok`` and ``weight_t_ok``.
 """
 
 from __future__ import annotations
@@ -37,6 +33,7 @@ from llmctl.config.knobs import knobs
 
 # gemm64_ex config: knob gemm64_config (see gemm64_config below).  A tuning cache
 # (llmctl.plugins.tuning_cache) can override it per layout or per exact shape.
+DGRAD64_TOKENS = 16384  # see dgrad64_shape_ok
 GEMM64_CONFIGS: dict = {}  # layout -> config
 GEMM64_SHAPE_CONFIGS: dict = {}  # (layout, M, N, K) -> config
 
@@ -113,16 +110,28 @@ def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     """Will ``dx = dy W`` for ``tokens`` rows run on gemm64?  (Decided at forward time: the
     weight's W^T copy is only kept for layers whose data gradient cannot.)  ``fused``: the
     down-projection data gradient with the SwiGLU backward in its epilogue.
-    Knob ``dgrad64``: fused (default) = only the SwiGLU-fused down-projection data gradient on
-    gemm64, the rest on hipBLASLt's forward layout through the W^T copies; all = every data
-    gradient on gemm64 (no W^T copies, ~10 GB less memory for GPT-7B); off = none.  Same-box GPT-7B
-    step A/B (profiles/bench_r2_dgrad_modes.txt): fused 832.0 / 833.9 ms, 0 833.9 / 832.7 ms,
-    1 837.7 / 839.7 ms."""
+    Knob ``dgrad64``: auto (default) = every data gradient that fits up to ``DGRAD64_TOKENS`` rows, beyond that as fused; fused = only
+    the SwiGLU-fused down-projection data gradient on gemm64, the rest on hipBLASLt's forward layout through the W^T copies; all =
+    every data gradient on gemm64 (no W^T copies, ~10 GB less memory for GPT-7B); off = none.  Whole steps, ms, gemm64 / W^T copies:
+    tiny model, 256 tokens 1.89 / 2.84; gpt2-125m 1024 tokens 8.31 / 12.24, 8192 13.0 / 13.2; two GPT-7B layers 1024 tokens
+    8.02 / 8.69, 8192 25.9 / 26.4, 16384 46.7 / 47.1, 24576 67.0 / 67.1 (a copy costs a pass over the weight, a launch and an event whatever
+    the batch); the full GPT-7B at 24576 tokens 837.7 / 832.0."""
     out, inn = w.shape
     mode = knobs().dgrad64
-    if mode == "off" or (mode == "fused" and not fused):
+    if mode == "off" or (not fused and (mode == "fused" or (mode == "auto" and tokens > DGRAD64_TOKENS))):
         return False
     return _gemm64_ok(tokens, inn, out, w) and out * w.stride(0) * 2 < 2**31
+
+
+def weight_t_ok(tokens: int, w: torch.Tensor) -> bool:
+    """Does the data gradient of a sinked ``w`` for ``tokens`` rows go through a W^T copy?  Where it does not run on gemm64, and
+    (knob dgrad64 = auto, unless its sink was made to keep copies) the layout's gain on the product covers the copy: weights of 2^24 entries at 8192 rows and more.  Whole steps,
+    ms, W^T copies / hipBLASLt reading W as it is: two GPT-7B layers 1024 tokens 8.69 / 8.51, 4096 16.2 / 16.0, 8192 26.4 / 26.7, 16384
+    47.1 / 48.2; gpt2-125m (weights of at most 2^21.2 entries) 1024 tokens 12.2 / 8.8, 8192 13.2 / 12.9, 32768 37.5 / 37.1."""
+    sink = getattr(w, "_llmctl_grad_sink", None)
+    if sink is None or dgrad64_shape_ok(tokens, w):
+        return False
+    return sink.always_transpose or knobs().dgrad64 != "auto" or (tokens >= 8192 and w.numel() >= 1 << 24)
 
 
 def dgrad64_ok(dy2: torch.Tensor, w: torch.Tensor, fused: bool = False) -> bool:
@@ -242,6 +251,7 @@ def wgrad_swiglu_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accu
 class GradSink:
     def __init__(self, transpose_dgrad: Optional[bool] = None):
         self.callbacks: List[Callable[[torch.nn.Parameter], None]] = []
+        self.always_transpose = bool(transpose_dgrad)  # asked for here: whatever the sizes
         if transpose_dgrad is None:
             transpose_dgrad = knobs().dgrad_transpose
         self.transpose_dgrad = transpose_dgrad
@@ -370,7 +380,7 @@ class _Linear(torch.autograd.Function):
         ctx.wparam, ctx.bparam = w, b
         sink = getattr(w, "_llmctl_grad_sink", None)
         ctx.wt = None
-        if sink is not None and ctx.needs_input_grad[0] and not dgrad64_shape_ok(x.numel() // x.shape[-1], w):
+        if ctx.needs_input_grad[0] and weight_t_ok(x.numel() // x.shape[-1], w):
             ctx.wt = sink.weight_t(w)
         return forward_linear(x, w, b)
 
@@ -423,8 +433,7 @@ def data_grad(dy: torch.Tensor, w: torch.nn.Parameter) -> torch.Tensor:
     dy2 = dy.reshape(-1, dy.shape[-1])
     if dgrad64_ok(dy2, w):
         return dgrad64(dy2, w).view(*dy.shape[:-1], w.shape[1])
-    sink = getattr(w, "_llmctl_grad_sink", None)
-    wt = sink.weight_t(w) if sink is not None else None
+    wt = w._llmctl_grad_sink.weight_t(w) if weight_t_ok(dy2.shape[0], w) else None
     if wt is not None:
         GradSink.wait_weight_t(w)
         return F.linear(dy, wt)

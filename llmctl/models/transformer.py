@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from llmctl import ops
 from llmctl.config.knobs import knobs
-from llmctl.exec.linear import data_grad, dgrad64, linear, swiglu_data_grad, weight_grad
+from llmctl.exec.linear import data_grad, linear, swiglu_data_grad, weight_grad
 from llmctl.parallel import async_tp
 from llmctl.parallel import context_parallel as cp
 from llmctl.parallel import tensor_parallel as tp
@@ -92,10 +92,7 @@ class _SwiGLUDown(torch.autograd.Function):
         out = F.linear(act, w_down)
         T = gu.numel() // gu.shape[-1]
         ctx.side = gu.requires_grad and wgrad_swiglu_ok(w_down, T, w_down.shape[1])
-        # the plain data gradient: gemm64 reading W K-major when knob dgrad64 = all, else
-        # hipBLASLt's forward layout through the W^T copy
-        ctx.dgrad_g64 = ctx.side and knobs().dgrad64 == "all"
-        if ctx.side and not ctx.dgrad_g64:
+        if ctx.side:
             _prep_weight_t(w_down, T)
         ctx.recompute = recompute
         if recompute:
@@ -120,10 +117,7 @@ class _SwiGLUDown(torch.autograd.Function):
         if ctx.side:
             # plain data gradient, then the weight gradient computing dgu on the side (gemm64.hip
             # "side job"): the HBM-bound SwiGLU backward streams under the wgrad's MFMAs
-            if ctx.dgrad_g64 and _gemm64_dgrad_ok(dout2, w_down):
-                dact = dgrad64(dout2, w_down)
-            else:
-                dact = data_grad(dout2, ctx.wparam)
+            dact = data_grad(dout2, ctx.wparam)
             dgu = ctx.wparam._llmctl_grad_sink.write_swiglu(ctx.wparam, dout2, act2, dact, gu.reshape(-1, gu.shape[-1]))
             if dgu is not None:
                 return dgu.view(gu.shape), None, None
@@ -134,14 +128,6 @@ class _SwiGLUDown(torch.autograd.Function):
         dw = weight_grad(ctx.wparam, dout2, act2)
         dgu = swiglu_data_grad(dout, ctx.wparam, gu)
         return dgu, dw, None
-
-
-def _gemm64_dgrad_ok(dy2: torch.Tensor, w: torch.Tensor) -> bool:
-    """``dy2 @ w`` on gemm64 (shape / alignment / 32-bit offset limits of ``gemm64_ex``)."""
-    from llmctl.exec.linear import _gemm64_ok
-
-    T, H = dy2.shape
-    return (_gemm64_ok(T, w.shape[1], H, dy2, w) and w.is_contiguous() and H * w.stride(0) * 2 < 2**31)
 
 
 def _fused_fwd_enabled() -> bool:
@@ -165,13 +151,12 @@ def _gemm64_rows(x2: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def _prep_weight_t(w: nn.Parameter, tokens: int) -> None:
-    """Start the side-stream W^T refresh now (forward) if this weight's data gradient will not
-    run on gemm64 — as ``_Linear.forward`` does."""
-    from llmctl.exec.linear import dgrad64_shape_ok
+    """Start the side-stream W^T refresh now (forward) if this weight's data gradient will go
+    through the copy — as ``_Linear.forward`` does."""
+    from llmctl.exec.linear import weight_t_ok
 
-    sink = getattr(w, "_llmctl_grad_sink", None)
-    if sink is not None and not dgrad64_shape_ok(tokens, w):
-        sink.weight_t(w)
+    if weight_t_ok(tokens, w):
+        w._llmctl_grad_sink.weight_t(w)
 
 
 class _QKVRopeAttention(torch.autograd.Function):
@@ -238,8 +223,7 @@ class _UpSwiGLUDown(torch.autograd.Function):
         # is needed comes from the inputs -- round 4 read gu.requires_grad and never took the side
         # path, running the down dgrad on the slower fused-epilogue kernel instead)
         ctx.side = (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]) and wgrad_swiglu_ok(w_down, T, w_down.shape[1])
-        ctx.dgrad_g64 = ctx.side and knobs().dgrad64 == "all"
-        if ctx.side and not ctx.dgrad_g64:
+        if ctx.side:
             _prep_weight_t(w_down, T)
         ctx.save_for_backward(x2, gu, act)
         ctx.w_up, ctx.w_down, ctx.xshape = w_up, w_down, x.shape
@@ -251,10 +235,7 @@ class _UpSwiGLUDown(torch.autograd.Function):
         dout2 = dout.reshape(-1, dout.shape[-1])
         dgu = None
         if ctx.side:
-            if ctx.dgrad_g64 and _gemm64_dgrad_ok(dout2, ctx.w_down):
-                dact = dgrad64(dout2, ctx.w_down)
-            else:
-                dact = data_grad(dout2, ctx.w_down)
+            dact = data_grad(dout2, ctx.w_down)
             dgu = ctx.w_down._llmctl_grad_sink.write_swiglu(ctx.w_down, dout2, act, dact, gu)
             dw_down = None
             if dgu is None:  # operands the side kernel cannot take: weight gradient + elementwise pass
