@@ -39,11 +39,10 @@ at::Tensor attn_qkv_prep(const at::Tensor& z, int64_t H, int64_t G, int64_t dk, 
                          bool v_from_k, const c10::optional<at::Tensor>& v_first, const c10::optional<at::Tensor>& v_lambda);
 at::Tensor mlstm_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& gates, const at::Tensor& b_i,
                       const at::Tensor& b_f, double cap, double qscale, at::Tensor S, at::Tensor n, at::Tensor m,
-                      const at::Tensor& slots, const at::Tensor& cu, const at::Tensor& start, bool slab,
-                      const c10::optional<at::Tensor>& fsum, bool write_out);
-void mlstm_chunk_combine(const at::Tensor& S, const at::Tensor& n, const at::Tensor& m, const at::Tensor& slots, const at::Tensor& start,
-                         const at::Tensor& base, const at::Tensor& locS, const at::Tensor& locn, const at::Tensor& locm,
-                         const at::Tensor& fsum, at::Tensor iS, at::Tensor in_, at::Tensor im);
+                      const at::Tensor& slots, const at::Tensor& cu, const at::Tensor& start, bool slab);
+at::Tensor mlstm_chunked(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& raw, const at::Tensor& b_i,
+                         const at::Tensor& b_f, double cap, double qscale, at::Tensor S, at::Tensor n, at::Tensor m, const at::Tensor& slots,
+                         const at::Tensor& start, const at::Tensor& cu, const at::Tensor& seq, const at::Tensor& base);
 std::tuple<at::Tensor, at::Tensor> group_topk_router(const at::Tensor& logits, int64_t top, int64_t groups, int64_t keep);
 std::tuple<at::Tensor, at::Tensor> bias_topk_router(const at::Tensor& logits, const c10::optional<at::Tensor>& bias, int64_t top, int64_t groups,
                                                     int64_t keep, bool renorm);
@@ -133,8 +132,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("clamped_glu(Tensor gu, float limit, float alpha) -> Tensor");
   m.def("causal_conv(Tensor u, Tensor w, Tensor(a!) state, Tensor seq_of, Tensor cu, Tensor start, Tensor sslot, bool add_input, int max_len=0) -> Tensor");
   m.def("attn_qkv_prep(Tensor z, int H, int G, int dk, int dv, Tensor? q_norm, Tensor? k_norm, float eps, Tensor pos, Tensor freq, int rot_dims, bool interleaved, float amp, Tensor? vfreq, Tensor(a!) cache, Tensor slots, bool v_from_k=False, Tensor? v_first=None, Tensor? v_lambda=None) -> Tensor");
-  m.def("mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor gates, Tensor b_i, Tensor b_f, float cap, float qscale, Tensor(a!) S, Tensor(b!) n, Tensor(c!) m, Tensor slots, Tensor cu, Tensor start, bool slab=False, Tensor(d!)? fsum=None, bool write_out=True) -> Tensor");
-  m.def("mlstm_chunk_combine(Tensor S, Tensor n, Tensor m, Tensor slots, Tensor start, Tensor base, Tensor locS, Tensor locn, Tensor locm, Tensor fsum, Tensor(a!) iS, Tensor(b!) in_, Tensor(c!) im) -> ()");
+  m.def("mlstm_scan(Tensor q, Tensor k, Tensor v, Tensor gates, Tensor b_i, Tensor b_f, float cap, float qscale, Tensor(a!) S, Tensor(b!) n, Tensor(c!) m, Tensor slots, Tensor cu, Tensor start, bool slab=False) -> Tensor");
+  m.def("mlstm_chunked(Tensor q, Tensor k, Tensor v, Tensor raw, Tensor b_i, Tensor b_f, float cap, float qscale, Tensor(a!) S, Tensor(b!) n, Tensor(c!) m, Tensor slots, Tensor start, Tensor cu, Tensor seq, Tensor base) -> Tensor");
   m.def("group_topk_router(Tensor logits, int top, int groups, int keep) -> (Tensor, Tensor)");
   m.def("bias_topk_router(Tensor logits, Tensor? bias, int top, int groups=1, int keep=1, bool renorm=True) -> (Tensor, Tensor)");
   m.def("hc_embed_norm(Tensor ids, Tensor table, int streams, Tensor c_in, Tensor g, float eps, bool out_bf16) -> (Tensor, Tensor)");
@@ -188,7 +187,7 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("causal_conv", &llmctl_hybrid::causal_conv);
   m.impl("attn_qkv_prep", &llmctl_hybrid::attn_qkv_prep);
   m.impl("mlstm_scan", &llmctl_hybrid::mlstm_scan);
-  m.impl("mlstm_chunk_combine", &llmctl_hybrid::mlstm_chunk_combine);
+  m.impl("mlstm_chunked", &llmctl_hybrid::mlstm_chunked);
   m.impl("group_topk_router", &llmctl_hybrid::group_topk_router);
   m.impl("bias_topk_router", &llmctl_hybrid::bias_topk_router);
   m.impl("gated_norm_add_norm_f32_", &llmctl_hybrid::gated_norm_add_norm_f32_);

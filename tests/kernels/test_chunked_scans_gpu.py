@@ -1,0 +1,69 @@
+"""The chunked recurrences on the fp32 matrix cores (``llmctl/ops/csrc/hybrid/mlstm_chunk.hip``) against the
+token-by-token formulas in float64: chunk edges, one-token and empty portions beside long ones, carried and fresh states, key and value
+sizes that fill no tile, strided rows, weak and strong gates (decays from nearly one to nearly nothing within a chunk)."""
+
+import pytest
+import torch
+
+from llmctl.ops import hybrid as hops
+
+pytestmark = pytest.mark.gpu
+LENS = [[41], [256], [300, 1, 0, 63, 64, 65], [17, 513, 128]]
+
+
+def _cu(lens):
+    cu = [0]
+    for n in lens:
+        cu.append(cu[-1] + n)
+    return cu
+
+
+def _rows(T, H, dk, dv, dtype, g):
+    z = torch.randn(T, 2 * H * dk + H * dv + 8, generator=g).to(dtype)  # q | k | v | other columns
+    q, k = z[:, :H * dk].unflatten(1, (H, dk)), z[:, H * dk:2 * H * dk].unflatten(1, (H, dk))
+    return z, q, k, z[:, 2 * H * dk:2 * H * dk + H * dv].unflatten(1, (H, dv))
+
+
+def _check(got, want, terms):
+    """``terms``: the magnitude of what each result sums up; fp32 sums and exponentials of pairwise exact differences, relative 2^-17."""
+    assert ((got.double().cpu() - want).abs() <= 2.0 ** -17 * terms + 1e-7).all(), ((got.double().cpu() - want).abs() / (terms + 1e-7)).max()
+
+
+@pytest.mark.parametrize("lens", LENS)
+@pytest.mark.parametrize("H,dk,dv,dtype,gain", [(2, 8, 8, torch.float32, 1.0), (3, 64, 128, torch.bfloat16, 1.0), (2, 24, 40, torch.bfloat16, 20.0),
+                                                (1, 128, 72, torch.float32, 20.0), (2, 100, 136, torch.bfloat16, 4.0), (2, 33, 16, torch.float32, 1.0)])
+def test_mlstm_chunks(H, dk, dv, dtype, gain, lens):
+    g = torch.Generator().manual_seed(dk + dv)
+    cu, T, ns = _cu(lens), sum(lens), len(lens)
+    z, q, k, v = _rows(T, H, dk, dv, dtype, g)
+    raw, b_i, b_f = torch.randn(T, 2 * H, generator=g) * gain, torch.randn(H, generator=g), torch.randn(H, generator=g) + 2
+    cap, qs = 15.0, dk ** -0.5
+    slots = torch.randperm(ns + 2, generator=g)[:ns].int()
+    start = torch.tensor([0 if i % 2 else 9 for i in range(ns)], dtype=torch.int32)
+    S, n, m = (torch.randn(s, generator=g) for s in ((ns + 2, H, dk, dv), (ns + 2, H, dk), (ns + 2, H)))
+    Sd, nd, md, zd = S.cuda(), n.cuda(), m.cuda(), z.cuda()
+    d = lambda t, a, w: zd[:, a:a + H * w].unflatten(1, (H, w))
+    got = hops.mlstm_scan(d(z, 0, dk), d(z, H * dk, dk), d(z, 2 * H * dk, dv), raw.cuda(), b_i.cuda(), b_f.cuda(), cap, qs, Sd, nd, md,
+                          slots.cuda(), torch.tensor(cu, dtype=torch.int32).cuda(), start.cuda(), cu_host=cu)
+    i = cap * torch.tanh((raw[:, :H].double() + b_i) / cap)
+    f = torch.nn.functional.logsigmoid(cap * torch.tanh((raw[:, H:].double() + b_f) / cap))
+    for s in range(ns):
+        sl, fresh = int(slots[s]), int(start[s]) == 0
+        if lens[s] == 0:
+            assert torch.equal(Sd[sl].cpu(), S[sl]) and torch.equal(md[sl].cpu(), m[sl])
+            continue
+        C, N, M = (torch.zeros_like(t[sl]).double() if fresh else t[sl].double() for t in (S, n, m))
+        Ca, Na = C.abs(), N.abs()  # the magnitudes behind them
+        for t in range(cu[s], cu[s + 1]):
+            Mn = torch.maximum(f[t] + M, i[t])
+            a, b = torch.exp(f[t] + M - Mn), torch.exp(i[t] - Mn)
+            kt, vt, qt = k[t].double(), v[t].double(), q[t].double() * qs
+            C, N = a[:, None, None] * C + b[:, None, None] * kt[:, :, None] * vt[:, None, :], a[:, None] * N + b[:, None] * kt
+            Ca = a[:, None, None] * Ca + b[:, None, None] * kt[:, :, None].abs() * vt[:, None, :].abs()
+            Na = a[:, None] * Na + b[:, None] * kt.abs()
+            M = Mn
+            den = torch.maximum((N * qt).sum(-1).abs(), torch.exp(-M)) + 1e-6
+            num, numa = torch.einsum("hkv,hk->hv", C, qt), torch.einsum("hkv,hk->hv", Ca, qt.abs())
+            want = num / den[:, None]
+            _check(got[t], want, numa / den[:, None] + want.abs() * ((Na * qt.abs()).sum(-1) / den)[:, None])
+        _check(Sd[sl], C, Ca), _check(nd[sl], N, Na), _check(md[sl], M, M.abs() + 1)
