@@ -482,10 +482,12 @@ class GatedLinearAttention(nn.Module):
         v = z[:, c:e].unflatten(1, (H, dv))
         g = z[:, e:e + H * dv]
         decay = _mm_f32(z[:, e + H * dv:self.cols], self.w_a2)  # fp32 [T, H * dk]
-        if "gla_plan" not in b.scratch:
-            b.scratch["gla_plan"] = hops.gla_chunk_plan(b.cu_host, h.device) if h.is_cuda else None
+        least = hops.gla_least(dk)
+        plan = f"gla_plan{least}"
+        if plan not in b.scratch:
+            b.scratch[plan] = hops.gla_chunk_plan(b.cu_host, h.device, least) if h.is_cuda else None
         o = hops.gla_scan(q, k, v, decay, self.b_a2, self.tau, dk ** -0.5, state[0], b.state, b.cu, b.start,
-                          plan=b.scratch["gla_plan"])
+                          plan=b.scratch[plan])
         y = hops.linear(hops.headnorm_gate(o, self._norm_rows(), g, self.eps, h.dtype, silu=True), self.w_o)
         return (y, z[:, self.cols:]) if self.side else y
 

@@ -258,13 +258,20 @@ def embed_rmsnorm_f32(ids, pos, table, pos_table, w, eps: float, out_dtype):
 
 
 GLA_CHUNK = 64  # tokens per chunk of the chunk-parallel scan; portions of >= 4 chunks take it
+GLA_MIN = 64  # keys up to 128 wide, whose chunks are matrix products (us, token by token / chunks, 16 heads of 64 x 128: 32 tokens
+# 41 / 34, 64 76 / 37, 256 288 / 40; 8 heads of 128 x 128: 32 tokens 95 / 43; and a plan costs one upload per step)
 
 
-def gla_chunk_plan(cu_host, device):
+def gla_least(dk: int) -> int:
+    """The shortest portion for which :func:`gla_scan` takes a chunk plan, by key size."""
+    return GLA_MIN if dk <= 128 else 4 * GLA_CHUNK
+
+
+def gla_chunk_plan(cu_host, device, least: int = 4 * GLA_CHUNK):
     """The chunks of a step's portions for the chunk-parallel scan, or None when no portion is long enough:
     (chunk row offsets, first chunk of every sequence, 0 .. P-1, P zeros, P ones) on ``device`` and P.  It
     depends on the step only, so the layers of a model share one."""
-    if cu_host is None or max((b - a for a, b in zip(cu_host[:-1], cu_host[1:])), default=0) < 4 * GLA_CHUNK:
+    if cu_host is None or max((b - a for a, b in zip(cu_host[:-1], cu_host[1:])), default=0) < least:
         return None
     pcu, base = [0], [0]
     for a, b in zip(cu_host[:-1], cu_host[1:]):
@@ -291,7 +298,7 @@ def gla_scan(q, k, v, z, z_bias, tau: float, qscale: float, S, state_slots, cu, 
     if use_native(q):
         nat = native_hybrid()
         if plan is None and cu_host is not None:
-            plan = gla_chunk_plan(cu_host, q.device)
+            plan = gla_chunk_plan(cu_host, q.device, gla_least(q.shape[-1]))
         if plan is not None:
             return _gla_scan_chunked(nat, q, k, v, z, z_bias, tau, qscale, S, state_slots, start, plan)
         return nat.gla_scan(q, k, v, z, z_bias, tau, qscale, S, state_slots, cu, start, None, True, True)
@@ -304,14 +311,20 @@ def _gla_scan_chunked(nat, q, k, v, z, z_bias, tau, qscale, S, state_slots, star
     chunk run from zeros), S_end = diag(D) S_begin + S_loc.  Three passes: (1) every chunk from zeros, all at
     once, no outputs, giving (S_loc, log D); (2) the memory at every chunk's first token, chunk after chunk
     (elementwise), and the sequence's new carried memory; (3) every chunk again from its true memory, all at
-    once, writing outputs token by token."""
+    once, writing outputs."""
     pcu_d, base_d, ident, zeros, ones, P = plan
     H, dk, dv = q.shape[1], q.shape[2], v.shape[2]
     f32 = dict(dtype=torch.float32, device=q.device)
     loc, logd = torch.empty(P, H, dk, dv, **f32), torch.empty(P, H, dk, **f32)
-    nat.gla_scan(q, k, v, z, z_bias, tau, qscale, loc, ident, pcu_d, zeros, logd, False, True)
+    matrix = dk <= 128  # the chunks as matrix products (csrc/hybrid/gla_chunk.hip), else scanned token by token
+    if matrix:
+        nat.gla_chunk_local(k, v, z, z_bias, tau, pcu_d, loc, logd)
+    else:
+        nat.gla_scan(q, k, v, z, z_bias, tau, qscale, loc, ident, pcu_d, zeros, logd, False, True)
     init = torch.empty_like(loc)
     nat.gla_chunk_combine(S, state_slots, start, base_d, loc, logd, init)
+    if matrix:
+        return nat.gla_chunk_out(q, k, v, z, z_bias, tau, qscale, pcu_d, init)
     return nat.gla_scan(q, k, v, z, z_bias, tau, qscale, init, ident, pcu_d, ones, None, True, False)
 
 

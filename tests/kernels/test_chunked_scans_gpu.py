@@ -1,4 +1,4 @@
-"""The chunked recurrences on the fp32 matrix cores (``llmctl/ops/csrc/hybrid/mlstm_chunk.hip``) against the
+"""The chunked recurrences on the fp32 matrix cores (``llmctl/ops/csrc/hybrid/mlstm_chunk.hip``, ``gla_chunk.hip``) against the
 token-by-token formulas in float64: chunk edges, one-token and empty portions beside long ones, carried and fresh states, key and value
 sizes that fill no tile, strided rows, weak and strong gates (decays from nearly one to nearly nothing within a chunk)."""
 
@@ -67,3 +67,35 @@ def test_mlstm_chunks(H, dk, dv, dtype, gain, lens):
             want = num / den[:, None]
             _check(got[t], want, numa / den[:, None] + want.abs() * ((Na * qt.abs()).sum(-1) / den)[:, None])
         _check(Sd[sl], C, Ca), _check(nd[sl], N, Na), _check(md[sl], M, M.abs() + 1)
+
+
+@pytest.mark.parametrize("lens", LENS[1:])
+@pytest.mark.parametrize("H,dk,dv,dtype,gain", [(2, 8, 8, torch.float32, 1.0), (3, 64, 128, torch.bfloat16, 1.0), (2, 24, 40, torch.bfloat16, 100.0),
+                                                (1, 128, 72, torch.float32, 3000.0), (2, 100, 136, torch.bfloat16, 10.0), (2, 33, 16, torch.float32, 1.0),
+                                                (1, 136, 16, torch.float32, 1.0)])
+def test_gla_chunks(H, dk, dv, dtype, gain, lens):
+    g = torch.Generator().manual_seed(dk + dv)
+    cu, T, ns = _cu(lens), sum(lens), len(lens)
+    z, q, k, v = _rows(T, H, dk, dv, dtype, g)
+    zl, zb, tau, qs = torch.randn(T, H * dk, generator=g) * gain, torch.randn(H * dk, generator=g), 16.0, dk ** -0.5
+    slots = torch.randperm(ns + 2, generator=g)[:ns].int()
+    start = torch.tensor([0 if i % 2 else 9 for i in range(ns)], dtype=torch.int32)
+    S = torch.randn(ns + 2, H, dk, dv, generator=g)
+    Sd, zd = S.cuda(), z.cuda()
+    d = lambda a, w: zd[:, a:a + H * w].unflatten(1, (H, w))
+    got = hops.gla_scan(d(0, dk), d(H * dk, dk), d(2 * H * dk, dv), zl.cuda(), zb.cuda(), tau, qs, Sd, slots.cuda(),
+                        torch.tensor(cu, dtype=torch.int32).cuda(), start.cuda(), cu_host=cu)
+    la = (torch.nn.functional.logsigmoid((zl + zb).double()) / tau).view(T, H, dk)
+    for s in range(ns):
+        sl = int(slots[s])
+        if lens[s] == 0:
+            assert torch.equal(Sd[sl].cpu(), S[sl])
+            continue
+        C = torch.zeros_like(S[sl]).double() if int(start[s]) == 0 else S[sl].double()
+        Ca = C.abs()
+        for t in range(cu[s], cu[s + 1]):
+            a, kt, vt, qt = torch.exp(la[t]), k[t].double(), v[t].double(), q[t].double() * qs
+            C = a[:, :, None] * C + kt[:, :, None] * vt[:, None, :]
+            Ca = a[:, :, None] * Ca + kt[:, :, None].abs() * vt[:, None, :].abs()
+            _check(got[t], torch.einsum("hkv,hk->hv", C, qt), torch.einsum("hkv,hk->hv", Ca, qt.abs()))
+        _check(Sd[sl], C, Ca)
