@@ -123,15 +123,29 @@ def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     return _gemm64_ok(tokens, inn, out, w) and out * w.stride(0) * 2 < 2**31
 
 
+def dgrad64_rows(tokens: int, w: torch.Tensor) -> int:
+    """Rows of a large weight's data gradient that gemm64 takes when ``tokens`` is no multiple of its 256-row tiles (knob dgrad64 = auto;
+    else 0): whole tiles, the library multiplies the rest, which streams the weight once more and so takes 1536 rows to pay.  One
+    GPT-7B layer, whole step, ms, this / W^T copies / W as it is: 540 tokens 5.36 / 5.36 / 5.14, 1000 6.10 / 6.06 / 5.91, 1710 7.54 / 7.81
+    / 7.59, 3414 10.1 / 10.4 / 10.8, 8196 19.0 / 21.2 / 21.1."""
+    rows = tokens // 256 * 256
+    if knobs().dgrad64 != "auto" or tokens < 1536 or rows == tokens or w.numel() < 1 << 24 or not dgrad64_shape_ok(rows, w):
+        return 0
+    return rows
+
+
 def weight_t_ok(tokens: int, w: torch.Tensor) -> bool:
     """Does the data gradient of a sinked ``w`` for ``tokens`` rows go through a W^T copy?  Where it does not run on gemm64, and
-    (knob dgrad64 = auto, unless its sink was made to keep copies) the layout's gain on the product covers the copy: weights of 2^24 entries at 8192 rows and more.  Whole steps,
-    ms, W^T copies / hipBLASLt reading W as it is: two GPT-7B layers 1024 tokens 8.69 / 8.51, 4096 16.2 / 16.0, 8192 26.4 / 26.7, 16384
-    47.1 / 48.2; gpt2-125m (weights of at most 2^21.2 entries) 1024 tokens 12.2 / 8.8, 8192 13.2 / 12.9, 32768 37.5 / 37.1."""
+    (knob dgrad64 = auto, unless its sink was made to keep copies) the layout's gain on the product covers the copy: weights of 2^24
+    entries at 8192 rows and more.  Whole steps, ms, W^T copies / hipBLASLt reading W as it is: two GPT-7B layers 1024 tokens 8.69 /
+    8.51, 4096 16.2 / 16.0, 8192 26.4 / 26.7, 16384 47.1 / 48.2; gpt2-125m (weights of at most 2^21.2 entries) 1024 tokens 12.2 /
+    8.8, 8192 13.2 / 12.9, 32768 37.5 / 37.1."""
     sink = getattr(w, "_llmctl_grad_sink", None)
     if sink is None or dgrad64_shape_ok(tokens, w):
         return False
-    return sink.always_transpose or knobs().dgrad64 != "auto" or (tokens >= 8192 and w.numel() >= 1 << 24)
+    if sink.always_transpose or knobs().dgrad64 != "auto":
+        return True
+    return not dgrad64_rows(tokens, w) and tokens >= 8192 and w.numel() >= 1 << 24
 
 
 def dgrad64_ok(dy2: torch.Tensor, w: torch.Tensor, fused: bool = False) -> bool:
@@ -140,13 +154,26 @@ def dgrad64_ok(dy2: torch.Tensor, w: torch.Tensor, fused: bool = False) -> bool:
             and dy2.is_cuda and dy2.dtype == torch.bfloat16 and _rows_ok(dy2))
 
 
-def dgrad64(dy2: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+def dgrad64(dy2: torch.Tensor, w: torch.Tensor, rows: Optional[int] = None) -> torch.Tensor:
+    """``dy2 @ w`` on gemm64, rows from ``rows`` on (``dgrad64_rows``) in the library."""
     from llmctl.ops._lib import native
 
-    dx = torch.empty(dy2.shape[0], w.shape[1], dtype=dy2.dtype, device=dy2.device)
-    cfg = gemm64_config("dgrad", dy2.shape[0], w.shape[1], w.shape[0])
-    native().gemm64_ex(dy2, w, dx, False, True, False, cfg)
+    T = dy2.shape[0]
+    rows = T if rows is None else rows
+    dx = torch.empty(T, w.shape[1], dtype=dy2.dtype, device=dy2.device)
+    cfg = gemm64_config("dgrad", rows, w.shape[1], w.shape[0])
+    native().gemm64_ex(dy2[:rows], w, dx[:rows], False, True, False, cfg)
+    if rows < T:
+        torch.mm(dy2[rows:], w, out=dx[rows:])
     return dx
+
+
+def dgrad64_part(dy2: torch.Tensor, w: torch.Tensor) -> int:
+    """``dgrad64_rows`` for these operands (0: not this way); weights whose sink keeps W^T copies stay with them."""
+    sink = getattr(w, "_llmctl_grad_sink", None)
+    if sink is None or sink.always_transpose or not (dy2.is_cuda and dy2.dtype == torch.bfloat16 and _rows_ok(dy2)):
+        return 0
+    return dgrad64_rows(dy2.shape[0], w)
 
 
 def _gemm_ex_ok(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> bool:
@@ -406,6 +433,8 @@ class _Linear(torch.autograd.Function):
                                       and _gemm64_ok(dy2.shape[0], w.shape[1], w.shape[0], w)
                                       and w.shape[0] * w.stride(0) * 2 < 2**31):
                 dx = dgrad64(dy2, w).view(*dy.shape[:-1], w.shape[1])
+            elif dgrad64_part(dy2, ctx.wparam):
+                dx = dgrad64(dy2, w, dgrad64_part(dy2, ctx.wparam)).view(*dy.shape[:-1], w.shape[1])
             elif ctx.wt is not None:
                 GradSink.wait_weight_t(ctx.wparam)
                 dx = F.linear(dy, ctx.wt)
@@ -433,6 +462,8 @@ def data_grad(dy: torch.Tensor, w: torch.nn.Parameter) -> torch.Tensor:
     dy2 = dy.reshape(-1, dy.shape[-1])
     if dgrad64_ok(dy2, w):
         return dgrad64(dy2, w).view(*dy.shape[:-1], w.shape[1])
+    if dgrad64_part(dy2, w):
+        return dgrad64(dy2, w, dgrad64_part(dy2, w)).view(*dy.shape[:-1], w.shape[1])
     wt = w._llmctl_grad_sink.weight_t(w) if weight_t_ok(dy2.shape[0], w) else None
     if wt is not None:
         GradSink.wait_weight_t(w)
