@@ -51,6 +51,8 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("attn_merge_(Tensor(a!) o_acc, Tensor(b!) lse_acc, Tensor o_j, Tensor lse_j) -> ()");
   m.def("paged_prefill_attention(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_q, Tensor ctx_lens, Tensor work, float scale) -> Tensor");
   m.def("paged_attention_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale) -> Tensor");
+  m.def("norm_linear(Tensor x, Tensor? res, Tensor nw, Tensor nb, float eps, Tensor w, Tensor? bias, int act) -> (Tensor, Tensor)");
+  m.def("norm_qkv_cache(Tensor x, Tensor? res, Tensor nw, Tensor nb, float eps, Tensor w, Tensor? bias, int nq, int nkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slots) -> (Tensor, Tensor)");
   m.def("stream_linear(Tensor x, Tensor w, Tensor? bias, int act) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w, Tensor? bias) -> Tensor");
   m.def("skinny_linear_cfg(Tensor x, Tensor w, Tensor? bias, int config) -> Tensor");

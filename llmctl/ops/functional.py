@@ -542,6 +542,39 @@ def decode_linear(x, w, b=None, act: Optional[str] = None):
     return gelu(y) if act == "gelu" else y
 
 
+def norm_linear_ok(x, res, nw, nb, w, b, split: bool = False) -> bool:
+    """Does ``csrc/norm_linear.hip`` take this LayerNorm and product, and does it pay?  Every workgroup repeats the norm, so for few and
+    short rows and up to 8192 outputs: up to 12 rows of 1024 (8 of 2048); ``split``: four more, as the launch that splits QKV goes too.
+    us in a graph, fused / separate: K 768, N 3072: 1 row 4.8 / 6.7, 8 rows 6.3 / 7.2, 12 rows 7.3 / 7.4, 16 rows 8.3 / 7.6; K 2048, N 3072:
+    1 row 8.0 / 9.8, 8 rows 10.0 / 10.8, 12 rows 11.8 / 11.0; N 16384, K 768: 1 row 11.8 / 10.8."""
+    if nb is None or not (x.dim() == 2 and stream_ok(x, w, b)):
+        return False
+    (M, K), N = x.shape, w.shape[0]
+    bf = all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, nw, nb) + (() if res is None else (res,)))
+    return (bf and K <= 2048 and M <= (12 if K <= 1024 else 8) + 4 * split and N <= 8192 and N % 4 == 0 and knobs().skinny_gemm == "auto"
+            and (M, N, K) not in SKINNY_CONFIGS)
+
+
+def decode_norm_linear(x, res, nw, nb, eps: float, w, b=None, act: Optional[str] = None):
+    """``act(LN(x + res) w^T (+ b))`` of a decode step (``res`` None: nothing is added); returns it and the new residual ``x +
+    res``.  Few short rows take one launch."""
+    if norm_linear_ok(x, res, nw, nb, w, b):
+        y, r = native().norm_linear(x, res, nw, nb, eps, w, b, _ROW_ACTS[act])
+        return y, (x if res is None else r)
+    xn, r = (layernorm(x, nw, nb, eps), x) if res is None else add_layernorm(x, res, nw, nb, eps)
+    return decode_linear(xn, w, b, act=act), r
+
+
+def decode_norm_qkv_cache(x, res, nw, nb, eps: float, w, b, nq: int, nkv: int, k_cache, v_cache, slots):
+    """``decode_norm_linear`` for the QKV projection of a model without rotary positions, K and V rows written to the paged cache at
+    ``slots``; returns (q ``[T, nq, D]``, the new residual)."""
+    if norm_linear_ok(x, res, nw, nb, w, b, True) and w.shape[0] // (nq + 2 * nkv) % 8 == 0:
+        q, r = native().norm_qkv_cache(x, res, nw, nb, eps, w, b, nq, nkv, k_cache, v_cache, slots)
+        return q, (x if res is None else r)
+    xn, r = (layernorm(x, nw, nb, eps), x) if res is None else add_layernorm(x, res, nw, nb, eps)
+    return qkv_split_cache(decode_linear(xn, w, b), nq, nkv, k_cache, v_cache, slots)[0], r
+
+
 def _dequant(w, w_scale, dtype):
     """bf16 image of an fp8 (e4m3fn) weight with fp32 row scales (fallback paths)."""
     return w if w_scale is None else (w.float() * w_scale.float().unsqueeze(1)).to(dtype)

@@ -642,12 +642,21 @@ class InferenceEngine:
         res = None
         kc, vc = self.kv_cache.k, self.kv_cache.v
         for li, layer in enumerate(self.model.layers):
-            xn, res = self._norm(layer, x, res, "attn")
-            q, k, v = self._qkv(layer, xn, positions, self.max_model_len, kc[li], vc[li], slots)
+            eps = self.cfg.layer_norm_eps
+            if self.rope is None and layer.attn_norm_b is not None:
+                q, res = ops.decode_norm_qkv_cache(x, res, layer.attn_norm_w, layer.attn_norm_b, eps, layer.wqkv, layer.bqkv, layer.nq,
+                                                   layer.nkv, kc[li], vc[li], slots)
+            else:
+                xn, res = self._norm(layer, x, res, "attn")
+                q, k, v = self._qkv(layer, xn, positions, self.max_model_len, kc[li], vc[li], slots)
             o = ops.paged_attention_decode(q, kc[li], vc[li], block_tables, ctx_lens)
             a = self._row_linear(o.view(o.shape[0], -1), layer.wo, layer.bo)
-            xn, res = self._norm(layer, a, res, "mlp")
-            x = self._mlp(layer, xn)
+            if layer.moe is None and not self.cfg.gated_mlp and layer.mlp_norm_b is not None:
+                h, res = ops.decode_norm_linear(a, res, layer.mlp_norm_w, layer.mlp_norm_b, eps, layer.w_up, layer.b_up, act="gelu")
+                x = self._row_linear(h, layer.w_down, layer.b_down)
+            else:
+                xn, res = self._norm(layer, a, res, "mlp")
+                x = self._mlp(layer, xn)
         return self._final(x, res)
 
     _W8_NAMES = ("wqkv", "wo", "w_up", "w_down")
