@@ -59,6 +59,11 @@ __device__ __forceinline__ float expert_act(int act, float u, float g) {
   return 0.5f * u * (1.0f + erff(u * 0.70710678118654752440f));
 }
 
+// The tiled form rounds the first projection's results to the activation's type before the activation, as a product and an
+// activation pass give them: over thousands of tokens a later router then sees the same numbers as behind per-expert products, and
+// the same choices where two experts are nearly equal (unrounded, one token in some 3000 chose otherwise).
+__device__ __forceinline__ float bf16_of(float v) { return __bfloat162float(__float2bfloat16(v)); }
+
 // (a conditional expression on two lvalues selects between addresses, one of them a stack slot)
 __device__ __forceinline__ uint4 load_or_zero(const bf16_t* p, bool in) {
   uint4 v = make_uint4(0, 0, 0, 0);
@@ -386,7 +391,7 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
         if (c >= g.cols) continue;
         float v[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = expert_act(1, acc[i][j + NI / 2][t], acc[i][j][t]);
+        for (int t = 0; t < 4; ++t) v[t] = expert_act(1, bf16_of(acc[i][j + NI / 2][t]), bf16_of(acc[i][j][t]));
         *reinterpret_cast<uint2*>(o + c) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
       }
     } else {
@@ -396,7 +401,7 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
         if (c >= g.cols) continue;
         float v[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = MODE == DOWN ? acc[i][j][t] : expert_act(g.act, acc[i][j][t], 0.f);
+        for (int t = 0; t < 4; ++t) v[t] = MODE == DOWN ? acc[i][j][t] : expert_act(g.act, bf16_of(acc[i][j][t]), 0.f);
         *reinterpret_cast<uint2*>(o + c) = make_uint2(pack2(v[0], v[1]), pack2(v[2], v[3]));
       }
     }
