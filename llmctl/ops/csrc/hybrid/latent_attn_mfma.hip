@@ -51,8 +51,11 @@ struct LArgs {
 // so that the forms without it keep their register budget.  SIG: the weights are sigmoids of the scores
 // (after the distance penalty), not a softmax: no running maximum, no rescale, no denominator (l = 1).  CAP: the scaled score
 // s becomes cap tanh(s / cap) before masks and softmax (tanh y = 1 - 2 / (1 + e^(2y))).
+// Keys and values up to 128 wide: two workgroups per CU (64.5 KB of images each; held to 256 registers, one's softmax runs beside the
+// other's products).  16 heads over 4 kv groups, portions of 2048 and 1331 tokens: 156 us at one per CU (200 + 96 registers),
+// 100 so.  Wider keys stay at one: 192-wide keys took 108 us against 99, with one set of images instead of two 107.
 template <int NCB, int NDB, bool ROT, bool SIG = false, bool CAP = false>
-__global__ __launch_bounds__(256, 1) void latent_attn_mfma_kernel(LArgs a) {
+__global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
   constexpr int NKS = NCB * 8;
   constexpr int NTB = (NDB + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
