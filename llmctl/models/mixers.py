@@ -219,8 +219,7 @@ class LatentAttention(nn.Module):
             if self.has_gate:
                 o = hops.sigmoid_gate_mul(o, z[:, c:])
             return hops.linear(o, self.w_o)
-        q_lat = torch.bmm(q[:, :, :self.dn].transpose(0, 1), self.w_uk).transpose(0, 1)  # [T, H, rank]
-        qa = hops.latent_q_assemble(q_lat, q, b.pos, self.inv_freq, self.rot_dims, self.dn, self.interleaved, self.rot_amp)
+        qa = hops.latent_queries(q, self.w_uk, b.pos, self.inv_freq, self.rot_dims, self.interleaved, self.rot_amp)
         outs = []
         if b.Tp:
             outs.append(hops.latent_attention_prefill(qa[:b.Tp], cache, b.p_bt, b.p_cu, b.p_ctx, self.window,
@@ -229,10 +228,7 @@ class LatentAttention(nn.Module):
             outs.append(hops.latent_attention_decode(qa[b.Tp:], cache, b.d_bt, b.d_ctx, self.window, self.sink,
                                                      self.scale, self.rk, max_ctx=b.d_max_ctx))
         o_lat = outs[0] if len(outs) == 1 else torch.cat(outs)
-        o = torch.bmm(o_lat.transpose(0, 1), self._w_uv_t()).transpose(0, 1).reshape(T, H * self.dv)
-        if self.has_gate:
-            o = hops.sigmoid_gate_mul(o, z[:, c:])
-        return hops.linear(o, self.w_o)
+        return hops.linear(hops.latent_values(o_lat, self._w_uv_t(), z[:, c:] if self.has_gate else None), self.w_o)
 
 
 class CausalConv(nn.Module):

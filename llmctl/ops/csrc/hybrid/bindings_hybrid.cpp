@@ -75,6 +75,9 @@ at::Tensor qk_fullnorm_prep(const at::Tensor& z, int64_t H, int64_t G, int64_t d
 at::Tensor gla_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& z, const at::Tensor& z_bias,
                     double tau, double qscale, at::Tensor S, const at::Tensor& slots, const at::Tensor& cu, const at::Tensor& start,
                     const c10::optional<at::Tensor>& logd, bool write_out, bool write_state);
+at::Tensor latent_q_rows(const at::Tensor& q, const at::Tensor& w_uk, const at::Tensor& pos, const at::Tensor& inv_freq, int64_t rot_dims,
+                         bool interleaved, double amp);
+at::Tensor latent_out_rows(const at::Tensor& o, const at::Tensor& w, const c10::optional<at::Tensor>& gate);
 void gla_chunk_local(const at::Tensor& k, const at::Tensor& v, const at::Tensor& z, const at::Tensor& z_bias, double tau, const at::Tensor& cu,
                      at::Tensor loc, at::Tensor logd);
 at::Tensor gla_chunk_out(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& z, const at::Tensor& z_bias, double tau,
@@ -155,6 +158,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
   m.def("qk_fullnorm_prep(Tensor z, int H, int G, int dk, int dv, Tensor q_norm, Tensor k_norm, float eps, Tensor pos, float temp_coef, int temp_every, Tensor(a!) cache, Tensor slots, Tensor? freq=None, int rot=0, bool interleaved=False, float amp=1.0) -> Tensor");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, float qscale, Tensor(a!) S, Tensor slots, Tensor cu, Tensor start, Tensor(b!)? logd=None, bool write_out=True, bool write_state=True) -> Tensor");
+  m.def("latent_q_rows(Tensor q, Tensor w_uk, Tensor pos, Tensor inv_freq, int rot_dims, bool interleaved, float amp) -> Tensor");
+  m.def("latent_out_rows(Tensor o, Tensor w, Tensor? gate=None) -> Tensor");
   m.def("gla_chunk_local(Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, Tensor cu, Tensor(a!) loc, Tensor(b!) logd) -> ()");
   m.def("gla_chunk_out(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, float qscale, Tensor cu, Tensor init) -> Tensor");
   m.def("gla_chunk_combine(Tensor(a!) S, Tensor slots, Tensor start, Tensor base, Tensor loc, Tensor logd, Tensor(b!) init) -> ()");
@@ -204,6 +209,8 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("act_any", &llmctl_hybrid::act_any);
   m.impl("qk_fullnorm_prep", &llmctl_hybrid::qk_fullnorm_prep);
   m.impl("gla_scan", &llmctl_hybrid::gla_scan);
+  m.impl("latent_q_rows", &llmctl_hybrid::latent_q_rows);
+  m.impl("latent_out_rows", &llmctl_hybrid::latent_out_rows);
   m.impl("gla_chunk_local", &llmctl_hybrid::gla_chunk_local);
   m.impl("gla_chunk_out", &llmctl_hybrid::gla_chunk_out);
   m.impl("gla_chunk_combine", &llmctl_hybrid::gla_chunk_combine);

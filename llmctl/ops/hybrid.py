@@ -166,6 +166,32 @@ def attn_qkv_prep(z, H: int, G: int, dk: int, dv: int, q_norm, k_norm, eps: floa
                              v_from_k, v_first, v_lambda)
 
 
+def head_rows_ok(x, w) -> bool:
+    """Does ``csrc/hybrid/head_rows.hip`` take the per-head products ``x [T, H, K] @ w [H, K, N]``?  Up to 32 rows in bf16, K a
+    multiple of 4, N of 8, aligned rows."""
+    return (use_native(x) and 1 <= x.shape[0] <= 32 and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 4 == 0
+            and w.shape[2] % 8 == 0 and x.stride(2) == 1 and x.stride(0) % 4 == 0 and x.stride(1) % 4 == 0 and x.data_ptr() % 8 == 0
+            and w.data_ptr() % 16 == 0)
+
+
+def latent_queries(q, w_uk, pos, inv_freq, rot_dims: int, interleaved: bool = False, amp: float = 1.0):
+    """Queries ``q [T, H, dn + rot]`` in the layout of a latent cache row, ``[q[.., :dn] W_uk | turned q[.., dn:]]`` with ``w_uk [H, dn,
+    rank]``: one launch for few rows, else a batched product and :func:`latent_q_assemble`."""
+    dn = w_uk.shape[1]
+    if head_rows_ok(q, w_uk) and (w_uk.shape[2] + q.shape[2] - dn) % 4 == 0:
+        return native_hybrid().latent_q_rows(q, w_uk, pos, inv_freq, rot_dims, interleaved, amp)
+    q_lat = torch.bmm(q[:, :, :dn].transpose(0, 1), w_uk).transpose(0, 1)  # [T, H, rank]
+    return latent_q_assemble(q_lat, q, pos, inv_freq, rot_dims, dn, interleaved, amp)
+
+
+def latent_values(o, w, gate=None):
+    """``[T, H dv]``: latent outputs ``o [T, H, rank]`` through ``w [H, rank, dv]``, times ``sigmoid(gate)`` if given."""
+    if head_rows_ok(o, w) and (gate is None or (gate.dtype == torch.bfloat16 and gate.shape[1] == w.shape[0] * w.shape[2] and gate.stride(1) == 1)):
+        return native_hybrid().latent_out_rows(o, w, gate)
+    y = torch.bmm(o.transpose(0, 1), w).transpose(0, 1).reshape(o.shape[0], -1)
+    return y if gate is None else sigmoid_gate_mul(y, gate)
+
+
 def sigmoid_gate_mul(o, g):
     """``o * sigmoid(g)`` -> g's dtype.  ``g`` may have fewer columns than ``o [T, C]``: ``g [T, H]`` gates
     every run of ``C / H`` neighbouring columns (one number per head)."""
