@@ -64,6 +64,51 @@ __global__ __launch_bounds__(NT) void gated_norm_add_norm_kernel(float* __restri
   for (int c = threadIdx.x + KEEP * NT; c < W; c += NT) stf(h + row * W + c, xr[c] * rstd2 * wn[c]);
 }
 
+// The same for rows of up to 4 * NT * VQ values in quads, all of a row's loads in flight at once (2048 wide, 16
+// rows: 10.5 us as above, 4.5 so; 2911 rows 27.3 and 18.4).
+template <typename TY, typename TR, typename TH, int VQ>
+__global__ __launch_bounds__(NT) void gated_norm_add_norm_quads_kernel(float* __restrict__ x, const TY* __restrict__ y, int64_t y_st,
+                                                                       const TR* __restrict__ r, int64_t r_st, const float* __restrict__ wp,
+                                                                       const float* __restrict__ wn, TH* __restrict__ h, int W, float eps) {
+  __shared__ float red[NW];
+  const int64_t row = blockIdx.x;
+  float4 g[VQ], rv[VQ], xv[VQ], pv[VQ], nv[VQ];
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
+    g[i] = ld4(y + row * y_st + c);
+    rv[i] = ld4(r + row * r_st + c);
+    xv[i] = ld4(x + row * W + c);
+    pv[i] = ld4(wp + c);
+    nv[i] = wn != nullptr ? ld4(wn + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    g[i] = make_float4(g[i].x * sigmoidf_(rv[i].x), g[i].y * sigmoidf_(rv[i].y), g[i].z * sigmoidf_(rv[i].z), g[i].w * sigmoidf_(rv[i].w));
+    if ((int)(threadIdx.x + i * NT) * 4 < W) q += (g[i].x * g[i].x + g[i].y * g[i].y) + (g[i].z * g[i].z + g[i].w * g[i].w);
+  }
+  const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+  float q2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    g[i] = make_float4(xv[i].x + g[i].x * rstd * pv[i].x, xv[i].y + g[i].y * rstd * pv[i].y, xv[i].z + g[i].z * rstd * pv[i].z,
+                       xv[i].w + g[i].w * rstd * pv[i].w);
+    if (c < W) {
+      st4(x + row * W + c, g[i]);
+      q2 += (g[i].x * g[i].x + g[i].y * g[i].y) + (g[i].z * g[i].z + g[i].w * g[i].w);
+    }
+  }
+  if (h == nullptr) return;
+  const float rstd2 = 1.0f / sqrtf(block_sum<NW>(q2, red) / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    if (c < W) st4(h + row * W + c, make_float4(g[i].x * rstd2 * nv[i].x, g[i].y * rstd2 * nv[i].y, g[i].z * rstd2 * nv[i].z, g[i].w * rstd2 * nv[i].w));
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pos,
                                                            const T* __restrict__ table, const T* __restrict__ ptable, const float* __restrict__ w,
@@ -281,9 +326,16 @@ at::Tensor gated_norm_add_norm_f32_(at::Tensor x, const at::Tensor& y, const at:
     using TY = std::remove_pointer_t<decltype(ty)>;
     using TR = std::remove_pointer_t<decltype(tr)>;
     using TH = std::remove_pointer_t<decltype(th)>;
-    gated_norm_add_norm_kernel<TY, TR, TH><<<dim3((unsigned)T), NT, 0, st>>>(x.data_ptr<float>(), (const TY*)y.data_ptr(), y.stride(0),
-                                                                           (const TR*)r.data_ptr(), r.stride(0), w_post.data_ptr<float>(), wn,
-                                                                           wn != nullptr ? (TH*)h.data_ptr() : (TH*)nullptr, (int)W, (float)eps);
+    auto launch = [&](auto kern) {
+      kern<<<dim3((unsigned)T), NT, 0, st>>>(x.data_ptr<float>(), (const TY*)y.data_ptr(), y.stride(0), (const TR*)r.data_ptr(), r.stride(0),
+                                             w_post.data_ptr<float>(), wn, wn != nullptr ? (TH*)h.data_ptr() : (TH*)nullptr, (int)W, (float)eps);
+    };
+    const bool quads = W <= 16 * NT && quads_ok((const TY*)y.data_ptr(), y.stride(0), W) && quads_ok((const TR*)r.data_ptr(), r.stride(0), W) &&
+                       quads_ok(x.data_ptr<float>(), W, W) && quads_ok(w_post.data_ptr<float>(), W, W) && (wn == nullptr || quads_ok(wn, W, W));
+    if (quads && W <= 4 * NT) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 1>);
+    else if (quads && W <= 8 * NT) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 2>);
+    else if (quads) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 4>);
+    else launch(gated_norm_add_norm_kernel<TY, TR, TH>);
   };
   dispatch_act(y, [&](auto* ty) {
     dispatch_act(r, [&](auto* tr) {

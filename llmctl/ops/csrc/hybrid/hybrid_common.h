@@ -74,6 +74,25 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 
 // Sum over a block of NW waves; every thread gets the result.  ``red`` holds NW floats; two barriers.
+// four neighbouring values (16-byte aligned fp32, 8-byte aligned bf16)
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 ld4(const bf16_t* p) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+}
+__device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+__device__ __forceinline__ void st4(bf16_t* p, float4 v) {
+  auto pack = [](float a, float b) {
+    return (unsigned)__bfloat16_as_ushort(__float2bfloat16(a)) | ((unsigned)__bfloat16_as_ushort(__float2bfloat16(b)) << 16);
+  };
+  *reinterpret_cast<uint2*>(p) = make_uint2(pack(v.x, v.y), pack(v.z, v.w));
+}
+// rows of W values, ``stride`` apart, that ld4 / st4 may walk
+template <typename T>
+inline bool quads_ok(const T* p, int64_t stride, int64_t W) {
+  return W % 4 == 0 && stride % 4 == 0 && reinterpret_cast<uintptr_t>(p) % (4 * sizeof(T)) == 0;
+}
+
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
