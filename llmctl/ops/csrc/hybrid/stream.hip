@@ -51,10 +51,9 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
   for (int i = 0; i < VQ; ++i) {
     const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
     v[i] = ld4(x + r * W + c);
-    av[i] = ld4(a + r * a_stride + c);
+    av[i] = a != nullptr ? ld4(a + r * a_stride + c) : make_float4(0.f, 0.f, 0.f, 0.f);
     bv[i] = b != nullptr ? ld4(b + r * W + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-    wv[i] = ld4(w + c);
-    cv[i] = ld4(bias + c);
+    if (h != nullptr) wv[i] = ld4(w + c), cv[i] = ld4(bias + c);
   }
   float s = 0.f;
 #pragma unroll
@@ -63,10 +62,11 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
     v[i].x = v[i].x + av[i].x + bv[i].x, v[i].y = v[i].y + av[i].y + bv[i].y;
     v[i].z = v[i].z + av[i].z + bv[i].z, v[i].w = v[i].w + av[i].w + bv[i].w;
     if (c < W) {
-      st4(x + r * W + c, v[i]);
+      if (a != nullptr) st4(x + r * W + c, v[i]);
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
   }
+  if (h == nullptr) return;
   const float mean = block_sum<NW>(s, red) / (float)W;
   float q = 0.f;
 #pragma unroll
@@ -270,6 +270,19 @@ static at::Tensor out_like(const at::Tensor& ref, at::IntArrayRef shape, bool bf
   return at::empty(shape, ref.options().dtype(bf16 ? at::kBFloat16 : at::kFloat));
 }
 
+// x += a (+ b) where a is given, h = LN(x) where h is: rows in quads where widths and addresses allow
+template <typename T>
+static void launch_add_layernorm(float* x, const T* a, int64_t a_st, const float* b, const float* w, const float* bias, T* h, int64_t rows, int W,
+                                 double eps) {
+  auto go = [&](auto kern) { kern<<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps); };
+  const bool quads = W <= 16 * NT && quads_ok(x, W, W) && (a == nullptr || quads_ok(a, a_st, W)) && (b == nullptr || quads_ok(b, W, W)) &&
+                     (h == nullptr || (quads_ok(w, W, W) && quads_ok(bias, W, W)));
+  if (quads && W <= 4 * NT) go(add_layernorm_quads_kernel<T, 1>);
+  else if (quads && W <= 8 * NT) go(add_layernorm_quads_kernel<T, 2>);
+  else if (quads) go(add_layernorm_quads_kernel<T, 4>);
+  else go(add_layernorm_kernel<T>);
+}
+
 at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, double eps, bool out_bf16) {
   HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kFloat, "x: contiguous fp32 [T, W]");
   const int W = (int)x.size(1);
@@ -279,8 +292,7 @@ at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Ten
   if (x.size(0) == 0) return h;
   dispatch_act(h, [&](auto* tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
-    add_layernorm_kernel<T><<<dim3((unsigned)x.size(0)), NT, 0, cur_stream()>>>(
-        x.data_ptr<float>(), (const T*)nullptr, 0, nullptr, w.data_ptr<float>(), b.data_ptr<float>(), (T*)h.data_ptr(), W, (float)eps);
+    launch_add_layernorm<T>(x.data_ptr<float>(), nullptr, 0, nullptr, w.data_ptr<float>(), b.data_ptr<float>(), (T*)h.data_ptr(), x.size(0), W, eps);
   });
   return h;
 }
@@ -298,9 +310,8 @@ void residual_add_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Te
   c10::DeviceGuard guard(x.device());
   dispatch_act(a, [&](auto* tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
-    add_layernorm_kernel<T><<<dim3((unsigned)x.size(0)), NT, 0, cur_stream()>>>(
-        x.data_ptr<float>(), (const T*)a.data_ptr(), a.stride(0), b.has_value() ? b->data_ptr<float>() : nullptr, nullptr, nullptr,
-        (T*)nullptr, (int)x.size(1), 0.f);
+    launch_add_layernorm<T>(x.data_ptr<float>(), (const T*)a.data_ptr(), a.stride(0), b.has_value() ? b->data_ptr<float>() : nullptr, nullptr, nullptr,
+                            nullptr, x.size(0), (int)x.size(1), 0.0);
   });
 }
 
@@ -315,17 +326,8 @@ at::Tensor add_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::opti
   if (x.size(0) == 0) return h;
   dispatch_act(a, [&](auto* tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
-    const float* bp = b.has_value() ? b->data_ptr<float>() : nullptr;
-    auto go = [&](auto kern) {
-      kern<<<dim3((unsigned)x.size(0)), NT, 0, cur_stream()>>>(x.data_ptr<float>(), (const T*)a.data_ptr(), a.stride(0), bp, w.data_ptr<float>(),
-                                                              bias.data_ptr<float>(), (T*)h.data_ptr(), W, (float)eps);
-    };
-    const bool quads = W <= 16 * NT && quads_ok((const T*)a.data_ptr(), a.stride(0), W) && quads_ok(x.data_ptr<float>(), W, W) &&
-                       (bp == nullptr || quads_ok(bp, W, W)) && quads_ok(w.data_ptr<float>(), W, W) && quads_ok(bias.data_ptr<float>(), W, W);
-    if (quads && W <= 4 * NT) go(add_layernorm_quads_kernel<T, 1>);
-    else if (quads && W <= 8 * NT) go(add_layernorm_quads_kernel<T, 2>);
-    else if (quads) go(add_layernorm_quads_kernel<T, 4>);
-    else go(add_layernorm_kernel<T>);
+    launch_add_layernorm<T>(x.data_ptr<float>(), (const T*)a.data_ptr(), a.stride(0), b.has_value() ? b->data_ptr<float>() : nullptr,
+                            w.data_ptr<float>(), bias.data_ptr<float>(), (T*)h.data_ptr(), x.size(0), W, eps);
   });
   return h;
 }

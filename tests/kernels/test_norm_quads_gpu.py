@@ -28,6 +28,12 @@ def test_add_layernorm_rows(W, bf16, pad, second):
     h = hops.add_layernorm_f32_(x, a, z, w, b, 1e-5, a.dtype)
     _near(x, want, want.abs() + 4, False)
     _near(h, y, w.double().abs() * 8 + b.double().abs(), bf16)
+    x2 = x.clone()
+    h2 = hops.layernorm_f32(x2, w, b, 1e-5, a.dtype)  # the norm alone leaves x as it is
+    _near(h2, y, w.double().abs() * 8 + b.double().abs(), bf16)
+    assert torch.equal(x2, x)
+    hops.residual_add_(x2, a, z)  # the sum alone
+    _near(x2, want + a.double() + (z.double() if second else 0), want.abs() + 8, False)
 
 
 @pytest.mark.parametrize("W", WIDTHS)
