@@ -93,6 +93,7 @@ class GradSyncEngine:
     def finish(self) -> None:
         """Issue any bucket not yet launched (unused params) and wait for all comms."""
         if self.enabled:
+            self.flat.settle_grads()
             while self._next < len(self._ready):
                 self._launch(self.flat.buckets[self._next])
                 self._next += 1

@@ -24,29 +24,33 @@ from ._lib import native, use_native
 
 # =============================================================================== norms
 def _norm_grads(ctx, dy2, x2, w, mu, rstd, dres2):
-    """(dx, dw, db) of a norm over the rows ``x2`` (``mu`` None: RMS norm, db None).  Weights with a gradient sink
-    (``llmctl.exec.linear.GradSink``) have their gradients written into the flat gradient by the kernel and get None."""
-    params = [p for p in ctx.norm_params if p is not None]
-    sink = getattr(params[0], "_llmctl_grad_sink", None)
-    if sink is not None and not all(p.requires_grad and getattr(p, "_llmctl_grad_sink", None) is sink for p in params):
-        sink = None
-    if sink is not None and use_native(dy2):
-        (dw, add_w), (db, add_b) = sink.open(params[0]), (sink.open(params[1]) if mu is not None else (None, False))
+    """(dx, dw, db) of a norm over the rows ``x2`` (``mu`` None: RMS norm, db None).  Every vector for itself: one that needs a gradient
+    and has a sink (``llmctl.exec.linear.GradSink``) has it written into the flat gradient, by the kernel, and gets None; one without a
+    sink gets an ordinary gradient; a frozen one gets None and leaves the other as it is."""
+    params, needed = ctx.norm_params, ctx.needs_input_grad[ctx.norm_at:ctx.norm_at + len(ctx.norm_params)]
+    sinks = [getattr(p, "_llmctl_grad_sink", None) if need else None for p, need in zip(params, needed)]
+    if use_native(dy2) and any(s is not None for s in sinks):
+        outs = [s.open(p) if s is not None else None for p, s in zip(params, sinks)]
+        kind = next(o[0].dtype for o in outs if o is not None)  # (the kernel's two sums share a type)
+        outs = [(torch.empty(p.shape, dtype=kind, device=dy2.device), False) if o is None else o for p, o in zip(params, outs)]
+        (dw, add_w), (db, add_b) = outs[0], (outs[1] if mu is not None else (None, False))
         dx = native().norm_bwd_into(dy2, x2, w, mu, rstd, dres2, dw, add_w, db, add_b)
-        for p in params:
-            sink.close(p)
-        return dx, None, None
-    k = native() if use_native(dy2) else ref
-    if mu is None:
-        dx, dw = k.rmsnorm_bwd(dy2, x2, w, rstd, dres2)
-        db = None
+        grads = [None if s is not None or not need else o[0].to(p.dtype) for p, s, need, o in zip(params, sinks, needed, outs)]
+        for p, s in zip(params, sinks):
+            if s is not None:
+                s.close(p)
     else:
-        dx, dw, db = k.layernorm_bwd(dy2, x2, w, mu, rstd, dres2)
-    if sink is not None:
-        for p, g in zip(params, (dw, db)):
-            sink.add(p, g)
-        return dx, None, None
-    return dx, dw, db
+        k = native() if use_native(dy2) else ref
+        if mu is None:
+            dx, *sums = k.rmsnorm_bwd(dy2, x2, w, rstd, dres2)
+        else:
+            dx, *sums = k.layernorm_bwd(dy2, x2, w, mu, rstd, dres2)
+        grads = []
+        for p, s, need, g in zip(params, sinks, needed, sums):
+            if s is not None:
+                s.add(p, g)
+            grads.append(g if need and s is None else None)
+    return dx, grads[0], grads[1] if mu is not None else None
 
 
 class _RMSNorm(torch.autograd.Function):
@@ -58,7 +62,7 @@ class _RMSNorm(torch.autograd.Function):
         else:
             y, rstd = ref.rmsnorm_fwd(x2, w, eps)
         ctx.save_for_backward(x2, w, rstd)
-        ctx.shape, ctx.norm_params = x.shape, (w,)
+        ctx.shape, ctx.norm_params, ctx.norm_at = x.shape, (w,), 1
         return y.view(x.shape)
 
     @staticmethod
@@ -82,7 +86,7 @@ class _AddRMSNorm(torch.autograd.Function):
             res_out = (x2.float() + r2.float()).to(x.dtype)
             y, rstd = ref.rmsnorm_fwd(res_out, w, eps)
         ctx.save_for_backward(res_out, w, rstd)
-        ctx.shape, ctx.norm_params = x.shape, (w,)
+        ctx.shape, ctx.norm_params, ctx.norm_at = x.shape, (w,), 2
         return y.view(x.shape), res_out.view(x.shape)
 
     @staticmethod
@@ -105,7 +109,7 @@ class _LayerNorm(torch.autograd.Function):
         else:
             y, mu, rstd = ref.layernorm_fwd(x2, w, b, eps)
         ctx.save_for_backward(x2, w, mu, rstd)
-        ctx.shape, ctx.norm_params = x.shape, (w, b)
+        ctx.shape, ctx.norm_params, ctx.norm_at = x.shape, (w, b), 1
         return y.view(x.shape)
 
     @staticmethod
@@ -127,7 +131,7 @@ class _AddLayerNorm(torch.autograd.Function):
             res_out = (x2.float() + r2.float()).to(x.dtype)
             y, mu, rstd = ref.layernorm_fwd(res_out, w, b, eps)
         ctx.save_for_backward(res_out, w, mu, rstd)
-        ctx.shape, ctx.norm_params = x.shape, (w, b)
+        ctx.shape, ctx.norm_params, ctx.norm_at = x.shape, (w, b), 2
         return y.view(x.shape), res_out.view(x.shape)
 
     @staticmethod

@@ -169,13 +169,19 @@ class FlatParameters:
         """Attach a :class:`llmctl.exec.linear.GradSink` to every parameter for which
         ``predicate(name, p)`` holds; their gradients are then written (beta=0 first) by
         the backward's kernels, so ``zero_grad`` skips them."""
-        n = 0
-        for p in self.params:
-            if predicate(self.names[id(p)], p):
-                sink.attach(p)
-                n += 1
+        self.sinked = [p for p in self.params if predicate(self.names[id(p)], p)]
+        for p in self.sinked:
+            sink.attach(p)
         self.sink = sink
-        return n
+        return len(self.sinked)
+
+    def settle_grads(self) -> None:
+        """After the last backward of a step: zeros for every parameter with a sink that took no part in it, whose gradient
+        ``zero_grad`` left as the last step wrote it."""
+        for p in getattr(self, "sinked", ()):
+            if p._llmctl_fresh:
+                grad_view(p).zero_()
+                p._llmctl_fresh = False
 
     def zero_grad(self) -> None:
         if self.grad is None:
@@ -193,10 +199,13 @@ class FlatParameters:
                 if g is None or g.data_ptr() != self.grad[off:].data_ptr():
                     p.grad = g = self.grad[off:off + p.numel()].view_as(p)
             if sink is not None:
-                if getattr(p, "_llmctl_grad_sink", None) is sink and p.requires_grad:
+                owned = getattr(p, "_llmctl_grad_sink", None) is sink
+                if owned and p.requires_grad:
                     sink.reset(p)
                 else:
                     g.zero_()
+                    if owned:
+                        p._llmctl_fresh = False  # whatever writes it (it may be trainable again by then) adds to zeros
 
     def view(self, start: int, end: int, which: str = "grad") -> torch.Tensor:
         buf = self.grad if which == "grad" else self.data
