@@ -67,7 +67,8 @@ def file_flags(src: Path, flags):
 
 
 def _headers(src: Path):
-    return sorted(list(src.parent.glob("*.h")) + list(src.parent.glob("*.inc")))
+    """The headers that a source may include: its folder's, and those of ``csrc`` that both groups share."""
+    return sorted(h for d in {src.parent, CSRC} for e in ("*.h", "*.inc") for h in d.glob(e))
 
 
 def _digest(src: Path, flags) -> str:

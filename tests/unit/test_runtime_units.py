@@ -539,3 +539,16 @@ def test_token_loader_property(tmp_path):
             assert torch.equal(torch.cat(sk.next_batch(), 1), want[k]), (use_native, "skip resume")
 
     check()
+
+
+# ---------------------------------------------------------------- kernel build
+def test_objects_depend_on_the_headers_they_include():
+    """Every header that a source names in quotes is part of its object's content key."""
+    import re
+
+    from llmctl.ops import build
+
+    for src in sorted(build.CSRC.rglob("*.hip")) + sorted(build.CSRC.rglob("*.cpp")):
+        known = {h.name for h in build._headers(src)}
+        named = {n.rsplit("/", 1)[-1] for n in re.findall(r'^#include "([^"]+)"', src.read_text(), re.M)}
+        assert named <= known, (src.name, named - known)
