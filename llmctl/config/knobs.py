@@ -65,7 +65,7 @@ class PerfKnobs:
     decode_fused: bool = True      # decode projections with fused epilogues
     decode_splits: int = 0         # paged-attention context splits (0: auto)
     decode_v3: int = 1             # skinny decode GEMM v3 schedule
-    skinny_gemm: str = "auto"      # decode-size GEMMs on the skinny kernel: auto | all | off
+    skinny_gemm: str = "auto"      # decode-size GEMMs: auto (weight stream, skinny kernel or library by size) | all (skinny) | off
     prefill_swiglu: bool = True    # serving prefill gate/up GEMM with the SwiGLU epilogue
     prefill_fa: bool = True        # fresh prompts through the packed flash-attention kernel
     prefill_norm_fold: bool = True  # prefill RMSNorms folded into the QKV / gate-up GEMMs (row-scaled epilogue)

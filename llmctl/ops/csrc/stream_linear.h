@@ -3,10 +3,11 @@
 // The bound is the weight stream and, below some 20 MB of weights, the latency of one round trip to HBM plus the launch
 // (3.5 us in a graph).  Measured beside the library's product (one MI355X, weights from HBM, 16 rows, us):
 //   N x K        2048 x 2048  4096 x 2048  8192 x 2048  10496 x 2048  32000 x 2048  4096 x 4096  2048 x 4096  768 x 3072  768 x 768
-//   library          11.1         11.7         13.8         16.1          33.1          15.6         14.9         9.1         5.3
-//   here              6.4          7.1          9.7         15.1          27.2          10.4          9.9         7.7         4.0
+//   library          11.1         10.8         12.3         14.0          31.6          15.0         14.3         9.1         5.2
+//   here              6.2          6.9          9.6         15.0          27.5          10.4           9.8        7.7         4.0
 // A workgroup owns whole outputs (no partial sums between workgroups), so N / 16 < 256 leaves CUs idle, and a CU draws about 30 GB/s
-// from HBM: 2048 x 8192 takes 17 us against the library's 13, which splits K over the chip.  Callers leave such shapes to it.
+// from HBM: 2048 x 8192 takes 17 us against the library's 13, which splits K over the chip; and tiles that fill the CUs one and a half
+// times (10496) cost as much as two rounds.  The callers' rules (llmctl/ops/functional.py: stream_pays, decode_form) leave such shapes.
 #pragma once
 
 #include <hip/hip_runtime.h>

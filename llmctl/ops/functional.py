@@ -505,42 +505,73 @@ SKINNY_CONFIGS: dict = {}  # (M, N, K) -> tuned config (0 = hipBLASLt), from a t
 _ROW_ACTS = {None: 0, "gelu": 2}  # the tanh form, as :func:`gelu`
 
 
-def stream_ok(x, w, b=None) -> bool:
-    """Does ``csrc/stream_linear.h`` take this product, and is it the fastest form of it?  At most 32 rows, bf16, K a multiple of 8,
-    aligned rows.  Up to 16 rows every output width; few outputs of a deep product (fewer than 4096 of more than 6144) and, with 17
-    to 32 rows, anything deeper than 2048 or wider than 8192 go to the library, which splits K over the chip (tables beside the
-    kernel)."""
-    if not (x.dim() == 2 and 1 <= x.shape[0] <= 32 and use_native(x)):
-        return False
-    (M, K), N = x.shape, w.shape[0]
-    pays = (K <= 6144 or N >= 4096) if M <= 16 else (K <= 2048 and N <= 8192)
-    return (pays and K % 8 == 0 and x.dtype == w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.stride(1) == 1
+def stream_takes(x, w, b=None) -> bool:
+    """Does ``csrc/stream_linear.h`` take this product?  At most 32 rows, bf16, K a multiple of 8, aligned rows."""
+    return (x.dim() == 2 and 1 <= x.shape[0] <= 32 and use_native(x) and x.shape[1] % 8 == 0 and x.dtype == w.dtype == torch.bfloat16
+            and x.stride(1) == 1 and w.stride(1) == 1
             and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous())))
 
 
+def stream_ok(x, w, b=None) -> bool:
+    """``stream_takes``, and it is faster than the library's product (:func:`stream_pays`)."""
+    return x.dim() == 2 and 1 <= x.shape[0] <= 32 and stream_pays(x.shape[0], w.shape[0], x.shape[1]) and stream_takes(x, w, b)
+
+
+def stream_pays(M: int, N: int, K: int) -> bool:
+    """Is the weight stream faster than the library's product?  In a graph, weights from HBM, us, library / here, beside each line.  (The
+    library splits K over the chip at some sizes and not at others: 4096 x 8192 15.2, 4096 x 11008 37.5.)"""
+    if M > 16:  # 32 rows 4096 x 2048 11.4 / 8.9, 2048 x 4096 11.7 / 13.3, 10240 x 2048 14.6 / 17.7; 24 rows 4240 x 2048 11.1 / 12.5, 4128 x 1024 11.3 / 7.8
+        return N <= 8192 and K <= 2048 and not (4096 < N < 5120 and K > 1024)
+    if K > 4096:  # only where the tiles fill the 256 CUs evenly, and up to 8 rows: 8 rows 4096 x 8192 15.2 / 16.1, 4096 x 11008 37.3 / 21.6, 32000 x 6144
+        # 86 / 74; 5120 x 8192 19.4 / 22.6, 2048 x 6144 11.0 / 11.8; 16 rows 4096 x 8192 15.8 / 17.9
+        tiles = (N + 15) // 16 if N < 5120 or (M <= 4 and N >= 6144) else (N + 31) // 32 if N < 24576 else (N + 63) // 64
+        return M <= 8 and tiles >= 0.95 * (-(-tiles // 256) * 256)
+    if M > 8 and 8192 < N <= 16384:  # 32 outputs a tile fill the CUs one and a half times: 16 rows 8192 x 2048 12.3 / 9.6, 8256 x 2048 13.5 / 14.5, 10240 x 3072
+        return False  # 19.3 / 20.7
+    return M <= 4 or N <= 40960  # 16 rows 32000 x 2048 31.6 / 27.5, 50304 x 768 18.2 / 21.7, 50304 x 3072 57.5 / 70.2; 4 rows 50304 x 768 18.0 / 17.5
+
+
+def decode_form(M: int, N: int, K: int) -> str:
+    """The form of :func:`decode_linear` by size: ``stream``, ``skinny`` (``csrc/skinny_gemm.hip``) or ``library``.  Beside
+    :func:`stream_pays`, us in a graph, stream / skinny:"""
+    if M > 16:  # 32 rows 3072 x 768 5.0 / 4.7, 4096 x 2048 8.9 / 10.5
+        return "skinny" if K < 1024 and N <= 4096 else "stream" if stream_pays(M, N, K) else "library"
+    if M <= 4:  # 4 rows 3072 x 768 3.8 / 3.5, 4096 x 4096 9.0 / 9.1, 5120 x 10240 26.7 / 40.8
+        return "skinny" if K < 1024 and N <= 16384 else "stream"
+    if (K > 4096 and N <= 2048) or (2048 <= K < 3072 and N <= 4096) or (8192 < N <= 12288 and not 1024 < K < 3072):
+        return "skinny"  # 8 rows 1024 x 11008 18.8 / 12.9, 4096 x 2048 6.6 / 6.1, 10240 x 4096 23.6 / 21.1; 16 rows 2048 x 6144 13.4 / 11.8
+    return "stream" if N < (16384 if M >= 8 else 40961) or stream_pays(M, N, K) else "library"  # 8 rows 4096 x 11008 21.6 / 27.4
+
+
 def decode_linear(x, w, b=None, act: Optional[str] = None):
-    """``act(x @ w^T (+ b))`` for decode-shaped inputs (``act``: None or ``gelu``): the weight-streaming kernels where they beat
-    hipBLASLt on uncached weights, bias and activation in the same launch (``csrc/stream_linear.h``; a tuned configuration
-    or knob ``skinny_gemm`` = ``all`` picks ``csrc/skinny_gemm.hip``, ``off`` the library).  Other inputs: the library and an
-    activation pass."""
+    """``act(x @ w^T (+ b))`` for decode-shaped inputs (``act``: None or ``gelu``): the form that is fastest on uncached weights
+    (``decode_form``): a stream of the weight with bias and activation in the same launch (``csrc/stream_linear.h``),
+    ``csrc/skinny_gemm.hip``, or the library.  A tuned configuration or knob ``skinny_gemm`` = ``all`` picks
+    ``csrc/skinny_gemm.hip``, ``off`` the library.  Other inputs: the library and an activation pass."""
     from llmctl.exec.linear import forward_linear
 
     mode = knobs().skinny_gemm
-    M = x.shape[0] if x.dim() == 2 else 0
+    (M, K), N = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
     y = None
-    tuned = SKINNY_CONFIGS.get((M, w.shape[0], w.shape[1])) if SKINNY_CONFIGS and x.dim() == 2 else None
+    tuned = SKINNY_CONFIGS.get((M, N, w.shape[1])) if SKINNY_CONFIGS and x.dim() == 2 else None
     if tuned is not None and mode == "auto" and use_native(x):
         if tuned == 0:
             y = torch.nn.functional.linear(x, w, b)
         elif x.is_contiguous() and w.is_contiguous() and x.dtype == w.dtype == torch.bfloat16:
             y = native().skinny_linear_cfg(x, w, b, tuned)
-    if y is None and mode == "auto" and stream_ok(x, w, b):
+    form = "skinny" if mode == "all" else "library" if mode == "off" or not 1 <= M <= 32 else decode_form(M, N, K)
+    if y is None and form == "skinny":
+        if (use_native(x) and M <= 32 and x.dtype == w.dtype == torch.bfloat16 and N % 16 == 0 and K % 128 == 0
+                and x.is_contiguous() and w.is_contiguous() and (b is None or b.is_contiguous())
+                and not (mode == "auto" and act is not None)):  # (an activation pass of its own costs more than the kernels differ by)
+            y = native().skinny_linear(x, w, b)
+        elif mode == "auto":
+            form = "stream"
+    if form == "library" and mode == "auto" and act is not None and M * N % 8:
+        form = "stream"  # (the activation pass takes multiples of 8)
+    if y is None and form == "stream" and stream_takes(x, w, b):
         return native().stream_linear(x, w, b, _ROW_ACTS[act])
-    if (y is None and mode == "all" and use_native(x) and x.dim() == 2 and M <= 32 and x.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and w.shape[0] % 16 == 0 and x.shape[1] % 128 == 0
-            and x.is_contiguous() and w.is_contiguous() and (b is None or b.is_contiguous())):
-        y = native().skinny_linear(x, w, b)
     if y is None:
         y = forward_linear(x, w, b)
     return gelu(y) if act == "gelu" else y
