@@ -12,6 +12,7 @@ copies are needed between kernels:
 
 from __future__ import annotations
 
+import functools
 from typing import List, Optional, Tuple
 
 import torch
@@ -506,11 +507,13 @@ _ROW_ACTS = {None: 0, "gelu": 2}  # the tanh form, as :func:`gelu`
 
 
 def stream_takes(x, w, b=None) -> bool:
-    """Does ``csrc/stream_linear.h`` take this product?  At most 32 rows, bf16, K a multiple of 8, aligned rows."""
-    return (x.dim() == 2 and 1 <= x.shape[0] <= 32 and use_native(x) and x.shape[1] % 8 == 0 and x.dtype == w.dtype == torch.bfloat16
-            and x.stride(1) == 1 and w.stride(1) == 1
-            and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous())))
+    """Does ``csrc/stream_linear.h`` take this product?  At most 32 rows, bf16, K a multiple of 8, aligned rows.  (Asked for every
+    projection of an eager step: one look at each property.)"""
+    if not (x.is_cuda and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16):
+        return False
+    xs, ws, (M, K) = x.stride(), w.stride(), x.shape
+    return (1 <= M <= 32 and xs[1] == 1 and ws[1] == 1 and (xs[0] | ws[0] | K) & 7 == 0 and (x.data_ptr() | w.data_ptr()) & 15 == 0
+            and (b is None or (b.dtype is torch.bfloat16 and b.is_contiguous())) and use_native(x))
 
 
 def stream_ok(x, w, b=None) -> bool:
@@ -518,6 +521,7 @@ def stream_ok(x, w, b=None) -> bool:
     return x.dim() == 2 and 1 <= x.shape[0] <= 32 and stream_pays(x.shape[0], w.shape[0], x.shape[1]) and stream_takes(x, w, b)
 
 
+@functools.lru_cache(maxsize=4096)
 def stream_pays(M: int, N: int, K: int) -> bool:
     """Is the weight stream faster than the library's product?  In a graph, weights from HBM, us, library / here, beside each line.  (The
     library splits K over the chip at some sizes and not at others: 4096 x 8192 15.2, 4096 x 11008 37.5.)"""
@@ -527,11 +531,13 @@ def stream_pays(M: int, N: int, K: int) -> bool:
         # 86 / 74; 5120 x 8192 19.4 / 22.6, 2048 x 6144 11.0 / 11.8; 16 rows 4096 x 8192 15.8 / 17.9
         tiles = (N + 15) // 16 if N < 5120 or (M <= 4 and N >= 6144) else (N + 31) // 32 if N < 24576 else (N + 63) // 64
         return M <= 8 and tiles >= 0.95 * (-(-tiles // 256) * 256)
-    if M > 8 and 8192 < N <= 16384:  # 32 outputs a tile fill the CUs one and a half times: 16 rows 8192 x 2048 12.3 / 9.6, 8256 x 2048 13.5 / 14.5, 10240 x 3072
-        return False  # 19.3 / 20.7
+    # (8193 to 16384 outputs at more than 8 rows fill the CUs one and a half times with tiles of 32: 16 rows 8192 x 2048 12.3 / 9.6, but
+    # 8256 x 2048 13.5 / 14.5 and 10240 x 3072 19.3 / 20.7.  They stay here: in a step that is not captured the library's call takes 18 us of
+    # the host and this one 7.)
     return M <= 4 or N <= 40960  # 16 rows 32000 x 2048 31.6 / 27.5, 50304 x 768 18.2 / 21.7, 50304 x 3072 57.5 / 70.2; 4 rows 50304 x 768 18.0 / 17.5
 
 
+@functools.lru_cache(maxsize=4096)
 def decode_form(M: int, N: int, K: int) -> str:
     """The form of :func:`decode_linear` by size: ``stream``, ``skinny`` (``csrc/skinny_gemm.hip``) or ``library``.  Beside
     :func:`stream_pays`, us in a graph, stream / skinny:"""
@@ -570,7 +576,7 @@ def decode_linear(x, w, b=None, act: Optional[str] = None):
             form = "stream"
     if form == "library" and mode == "auto" and act is not None and M * N % 8:
         form = "stream"  # (the activation pass takes multiples of 8)
-    if y is None and form == "stream" and stream_takes(x, w, b):
+    if y is None and form == "stream" and x.dim() == 2 and stream_takes(x, w, b):
         return native().stream_linear(x, w, b, _ROW_ACTS[act])
     if y is None:
         y = forward_linear(x, w, b)

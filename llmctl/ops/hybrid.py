@@ -21,6 +21,7 @@ import torch
 
 from . import ref_hybrid as ref
 from ._lib import native_hybrid, use_native
+from .functional import stream_ok
 
 
 def layernorm_f32(x, w, b, eps: float, out_dtype):
@@ -384,11 +385,7 @@ _ROW_ACTS = {None: 0, "gelu": 1, "relu2": 3}
 def rows_ok(x, w, b=None) -> bool:
     """Whether :func:`rows_linear` takes this product of a few rows and is the fastest form of it (the rule of
     :func:`llmctl.ops.functional.stream_ok`)."""
-    if x.dim() != 2 or x.shape[0] > 32:
-        return False
-    from .functional import stream_ok
-
-    return stream_ok(x, w, b)
+    return x.shape[0] <= 32 and stream_ok(x, w, b)
 
 
 def rows_linear(x, w, b=None, act=None, act_cols=None, f32: bool = False):
