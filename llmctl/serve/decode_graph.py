@@ -1,15 +1,23 @@
 """A captured decode step of a hybrid-mixer model: static device inputs behind one staged copy, the model's step over
 ``n`` rows and its logits as one HIP graph.
 
-Recurrent states live in the step itself, so nothing may run twice: there are no warm-up passes and no padded rows.  The
+Recurrent states live in the step itself, so nothing may run twice: there are no warm-up passes, and the pools have no scratch
+slot that a padded row could write.  The
 engine runs the first steps of a shape eagerly (:data:`WARM_STEPS`: they load the kernels and build what the modules
 derive from their weights once), then records the same calls and replays them.  A shape is the number of rows and the
 power of two that holds the longest context, which sizes the split of the keys over workgroups; the kernels read every
-sequence's own length from device memory, so any context runs through any split."""
+sequence's own length from device memory, so any context runs through any split.
+
+Batches change shape all the time, so a recording must be cheap: it takes the host's time for the step's launches, without the
+synchronisation, the collection of garbage and the emptied allocator that ``torch.cuda.graph`` starts with.  The step that records and its
+first replay, one MI355X, 9 to 15 rows, with / without those three: Malinex (3 layers) 26.4 / 1.1 ms, Lenitar (4) 29 / 1.7, Dumazen (6) 28 / 1.6; their
+eager steps take 0.7, 0.9 and 1.0.  Sixteen row counts in turn, 12 rounds: Malinex 1405 / 346 us a step, Lenitar 1515 / 486.
+What does not record (no memory left, a module that waits for the device) runs eagerly, as the first steps do."""
 
 from __future__ import annotations
 
-from typing import Dict, List, Sequence, Tuple
+import threading
+from typing import Callable, Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -17,7 +25,8 @@ import torch
 from llmctl.utils.env import graph_capture_gc_guard
 
 WARM_STEPS = 2  # eager steps of a shape before it is captured
-MAX_GRAPHS = 32  # shapes kept per engine; the least recently used one goes first
+CROWDED_STEPS = 16  # the same once another shape's graph has to go for it: what a recording costs is then a small part of these steps
+MAX_GRAPHS = 64  # shapes kept per engine; the least recently used one goes first
 STAGES = 4  # pinned input sets: the host runs at most this many steps ahead of the copies
 
 
@@ -62,20 +71,36 @@ class DecodeGraph:
         self.batch = StepBatch(ids=v["ids"], pos=v["pos"], slots=v["slots"], Tp=0, p_cu=None, p_ctx=None, p_bt=None,
                                d_ctx=v["ctx"], d_bt=v["bt"], cu=cu, start=v["start"], state=v["state"], max_q=0,
                                cu_host=list(range(n + 1)), seq_of=cu[:n], d_max_ctx=max_ctx, carried=False, fresh=False)
-        self.stages = []
-        for _ in range(STAGES):
-            host = torch.zeros(size, dtype=torch.uint8, pin_memory=True)
-            ev = torch.cuda.Event()
-            self.stages.append((host, host.numpy(), ev))
+        # one pinned block for all input sets (each pinned allocation is a call into the driver)
+        hosts = torch.zeros(STAGES, size, dtype=torch.uint8, pin_memory=True)
+        self.stages = [(h, h.numpy(), torch.cuda.Event()) for h in hosts]
         self.turn = 0
         self.graph = self.logits = None
 
     def capture(self, model, cache, pool) -> None:
+        """Record the step.  Nothing runs, so a failure (raised) leaves caches and states as they were."""
         g = torch.cuda.CUDAGraph()
-        with graph_capture_gc_guard(), torch.cuda.graph(g, pool=pool):
-            self.batch.scratch.clear()
-            self.logits = model.logits(model.step(self.batch, cache))
-        self.graph = g
+        with _capturing, graph_capture_gc_guard(collect=False), torch.cuda.stream(_capture_stream(self.buf.device)):
+            # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
+            g.capture_begin(pool=pool, capture_error_mode="thread_local")
+            try:
+                self.batch.scratch.clear()
+                logits = model.logits(model.step(self.batch, cache))
+            except BaseException:
+                try:
+                    g.capture_end()
+                except RuntimeError:
+                    pass  # (the first error is the one to tell)
+                self.batch.scratch.clear()
+                g.reset()
+                raise
+            g.capture_end()
+        self.graph, self.logits = g, logits
+
+    def release(self) -> None:
+        torch.cuda.synchronize(self.buf.device)  # its last replay, on whatever stream
+        self.graph.reset()
+        self.graph = self.logits = None
 
     def run(self, values: Dict[str, np.ndarray], ids_on_device=None) -> torch.Tensor:
         """Stage the step's inputs, copy them over, replay.  ``ids_on_device``: the input tokens, already sampled there.
@@ -95,3 +120,49 @@ class DecodeGraph:
         ev.record()
         self.graph.replay()
         return self.logits.clone()
+
+
+_capturing = threading.Lock()  # one recording at a time: they share a stream
+_capture_streams: Dict[torch.device, "torch.cuda.Stream"] = {}
+
+
+def _capture_stream(device: torch.device) -> "torch.cuda.Stream":
+    s = _capture_streams.get(device)
+    if s is None:
+        s = _capture_streams[device] = torch.cuda.Stream(device=device)
+    return s
+
+
+class GraphTable:
+    """The shapes of an engine's decode steps: how many eager steps each has had, or its graph, or that it does not record."""
+
+    def __init__(self):
+        self._shapes: Dict[Tuple[int, int], object] = {}  # least recently used first
+        self._graphs = 0
+
+    def __len__(self) -> int:
+        return self._graphs
+
+    def step(self, shape: Tuple[int, int], record: Callable[[Tuple[int, int]], Optional[DecodeGraph]]) -> Optional[DecodeGraph]:
+        """The graph that runs the next step of ``shape``; None: it runs eagerly.  ``record(shape)``: its graph, or None where it
+        cannot be recorded."""
+        e = self._shapes.pop(shape, 0)
+        if isinstance(e, int):
+            if e >= (WARM_STEPS if self._graphs < MAX_GRAPHS else CROWDED_STEPS):
+                if self._graphs >= MAX_GRAPHS:
+                    old = next(k for k, v in self._shapes.items() if v is not None and not isinstance(v, int))
+                    self._shapes.pop(old).release()
+                    self._graphs -= 1
+                e = record(shape)
+                self._graphs += e is not None
+            else:
+                e += 1
+        self._shapes[shape] = e
+        return None if isinstance(e, int) else e
+
+    def clear(self) -> None:
+        for e in self._shapes.values():
+            if e is not None and not isinstance(e, int):
+                e.release()
+        self._shapes.clear()
+        self._graphs = 0

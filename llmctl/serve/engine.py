@@ -39,7 +39,7 @@ from llmctl.models import DecoderLM
 from llmctl.utils.env import graph_capture_gc_guard
 
 from .block_manager import PagedKVCache, make_kv_manager
-from .decode_graph import MAX_GRAPHS, WARM_STEPS, DecodeGraph, upload_packed
+from .decode_graph import DecodeGraph, GraphTable, upload_packed
 from .prefix_cache import PrefixCache
 from .scheduler import ContinuousBatchScheduler, PrefillChunk, SamplingParams, Sequence
 from .tokenizer import load_tokenizer
@@ -186,11 +186,10 @@ class InferenceEngine:
         self.max_batch_size = max_batch_size
         self.use_graphs = False  # the transformer's padded, sampled graphs; this family's: _hybrid_decode
         self._graphs = {}
-        # captured decode steps by (rows, context bound); a shape maps to the number of eager steps it has had until then
-        self._decode_graphs: Dict[Tuple[int, int], object] = {}
+        self._decode_graphs = GraphTable()  # captured decode steps by (rows, context bound)
         self._decode_capture = use_graphs and self.device.type == "cuda"
         self._graph_pool = None
-        self._weights_seen = None
+        self._weights_seen = self._key_modules = None
         self._np_rng = np.random.default_rng(seed)
         self._pending = None
         self._last_toks = None
@@ -255,38 +254,56 @@ class InferenceEngine:
         return self.model.logits(x)
 
     def _weights_key(self):
-        """What a captured step's kernels were recorded against: the weights' storage and versions (modules keep stacked or
-        transposed copies of them, which an in-place change makes stale)."""
-        ps = getattr(self, "_param_list", None)
-        if ps is None:
-            ps = self._param_list = list(self.model.parameters())
-        return sum(p._version for p in ps), sum(p.data_ptr() for p in ps)
+        """What a captured step's kernels were recorded against, in the model's order: its modules, and every parameter's and
+        buffer's identity, storage and version (modules keep stacked or transposed copies of them, which an in-place change makes
+        stale)."""
+        seen = self._key_modules  # (children dicts of the modules, the children, their dicts of tensors)
+        if seen is None or seen[1] != [c for d in seen[0] for c in d.values()]:  # first use, or a module was exchanged
+            live = list(self.model.modules())
+            kids = [m._modules for m in live]
+            seen = self._key_modules = (kids, [c for d in kids for c in d.values()], [d for m in live for d in (m._parameters, m._buffers)])
+        ts = [t for d in seen[2] for t in d.values() if t is not None]
+        try:
+            versions = [t._version for t in ts]
+        except RuntimeError:  # tensors made in inference mode keep no version (and cannot be changed outside of it)
+            versions = [0 if t.is_inference() else t._version for t in ts]
+        return list(map(id, ts)), list(map(torch.Tensor.data_ptr, ts)), versions
+
+    def _record_decode(self, shape: Tuple[int, int]) -> Optional[DecodeGraph]:
+        """The captured decode step of ``shape`` = (rows, context bound), or None where it cannot be recorded: its steps stay eager."""
+        n, max_ctx = shape
+        if not all(m.on_device(n) for m in self.model.modules() if hasattr(m, "on_device")):
+            return None
+        for last in (False, True):
+            if not self._decode_graphs:  # (a pool ends with its last graph)
+                self._graph_pool = torch.cuda.graph_pool_handle()
+            try:
+                g = DecodeGraph(n, self.max_blocks_per_seq, max_ctx, self.device)
+                g.capture(self.model, self.kv_cache, self._graph_pool)
+                return g
+            except torch.OutOfMemoryError as e:
+                if last:
+                    log.warning("decode steps of %d rows stay eager: no memory to record them (%s)", n, e)
+                else:  # once more with what the allocator keeps for later
+                    torch.cuda.synchronize(self.device)
+                    torch.cuda.empty_cache()
+            except RuntimeError as e:
+                log.warning("decode steps of %d rows stay eager: %s", n, e)
+                break
+        return None
 
     def _hybrid_decode(self, dp: Dict, count: bool = True, ids_on_device: Optional[torch.Tensor] = None) -> torch.Tensor:
         """One decode step of a hybrid-mixer model: the first steps of a shape run eagerly, then its captured graph is
         replayed (:mod:`llmctl.serve.decode_graph`).  ``ids_on_device``: the rows' input tokens as a device tensor."""
         n = len(dp["positions"])
-        key = (n, 1 << max(int(max(dp["ctx"])) - 1, 0).bit_length()) if n else None
         g = None
         if self._decode_capture and n:
             w = self._weights_key()
             if w != self._weights_seen:
                 self.release_graphs()
                 self._weights_seen = w
-            g = self._decode_graphs.pop(key, 0)
-            if not isinstance(g, DecodeGraph) and g >= WARM_STEPS and all(
-                    m.on_device(n) for m in self.model.modules() if hasattr(m, "on_device")):
-                if self._graph_pool is None:
-                    self._graph_pool = torch.cuda.graph_pool_handle()
-                while sum(isinstance(v, DecodeGraph) for v in self._decode_graphs.values()) >= MAX_GRAPHS:
-                    old = next(k for k, v in self._decode_graphs.items() if isinstance(v, DecodeGraph))
-                    torch.cuda.synchronize(self.device)
-                    self._decode_graphs.pop(old).graph.reset()
-                dg = DecodeGraph(n, self.max_blocks_per_seq, key[1], self.device)
-                dg.capture(self.model, self.kv_cache, self._graph_pool)
-                g = dg
-            self._decode_graphs[key] = g if isinstance(g, DecodeGraph) else g + 1  # (re-inserted: most recently used last)
-        if not isinstance(g, DecodeGraph):
+            g = self._decode_graphs.step((n, 1 << max(int(max(dp["ctx"])) - 1, 0).bit_length()), self._record_decode)
+        if g is None:
             if ids_on_device is not None:
                 dp = dict(dp, ids=ids_on_device.tolist())
             return self._hybrid_exec(None, dp, count=count)
@@ -792,16 +809,14 @@ class InferenceEngine:
     def release_graphs(self) -> None:
         """Drop the captured decode graphs (they hold the RCCL communicator's captured
         collectives: release them before ``destroy_process_group``)."""
-        own = [g for g in getattr(self, "_decode_graphs", {}).values() if isinstance(g, DecodeGraph)]
+        own = getattr(self, "_decode_graphs", None)
         if (self._graphs or own) and self.device.type == "cuda":
             torch.cuda.synchronize(self.device)
         for g, _ in self._graphs.values():
             g.reset()
         self._graphs.clear()
-        for g in own:
-            g.graph.reset()
-        if self.hybrid:
-            self._decode_graphs.clear()
+        if own is not None:
+            own.clear()
             self._graph_pool = None
 
     def close(self) -> None:

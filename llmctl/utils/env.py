@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import os
+import threading
 from dataclasses import dataclass
 
 
@@ -91,9 +92,13 @@ def install_hang_dump() -> None:
         faulthandler.dump_traceback_later(float(s), repeat=True, exit=False)
 
 
+_gc_guards = {"open": 0, "was": False, "lock": threading.Lock()}
+
+
 @contextlib.contextmanager
-def graph_capture_gc_guard():
-    """Collect garbage before a hipGraph capture and keep the cyclic collector off during it.
+def graph_capture_gc_guard(collect: bool = True):
+    """Collect garbage before a hipGraph capture (``collect``: 20 ms in a serving process) and keep the cyclic collector off during
+    it; captures of several threads may overlap.
 
     A collection inside a capture can run the destructor of an unrelated, unreachable engine
     whose captured graphs then free their executable graphs and pools on a capturing device;
@@ -102,11 +107,17 @@ def graph_capture_gc_guard():
     beforehand under ``force_cudagraph_gc``."""
     import gc
 
-    gc.collect()
-    was = gc.isenabled()
-    gc.disable()
+    if collect:
+        gc.collect()
+    with _gc_guards["lock"]:
+        if not _gc_guards["open"]:
+            _gc_guards["was"] = gc.isenabled()
+            gc.disable()
+        _gc_guards["open"] += 1
     try:
         yield
     finally:
-        if was:
-            gc.enable()
+        with _gc_guards["lock"]:
+            _gc_guards["open"] -= 1
+            if not _gc_guards["open"] and _gc_guards["was"]:
+                gc.enable()

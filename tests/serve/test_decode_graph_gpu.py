@@ -1,6 +1,7 @@
 """Captured decode steps of the hybrid families against the eager ones: the same sequences through an engine with graphs and
 one without, over several replays with eager work in between, sequences that come and go (other row counts, reused state
-slots and pages), a context that passes a power of two, tokens fed back on the device, and weights changed in place."""
+slots and pages), a context that passes a power of two, tokens fed back on the device, weights changed in place or exchanged, shapes
+that are given up or do not record, and other threads at work during a recording."""
 
 import pytest
 import torch
@@ -82,6 +83,174 @@ def test_captured_steps_match_eager_ones(name, dtype):
     assert es[1].stats["graph_replays"] == 0
     for e in es:
         e.close()
+
+
+class _Pair:
+    """The same sequences in an engine with graphs and one without."""
+
+    def __init__(self, name, dtype=torch.bfloat16):
+        self.es, self.dtype = [_engine(name, g, dtype) for g in (True, False)], dtype
+        self.gen = torch.Generator().manual_seed(1)
+        self.live = []
+
+    def admit(self, n):
+        from llmctl.serve.scheduler import PrefillChunk
+
+        ids, out = torch.randint(0, 500, (n,), generator=self.gen).tolist(), []
+        for e in self.es:
+            s = e.open_sequence(ids)
+            e.prefill([PrefillChunk(s, 0, n)])
+            e.scheduler.computed(s, n)
+            out.append(s)
+        self.live.append(out)
+
+    def step(self, rows):
+        new, got = torch.randint(0, 500, (rows,), generator=self.gen).tolist(), []
+        for k, e in enumerate(self.es):
+            seqs = [p[k] for p in self.live[:rows]]
+            for s, t in zip(seqs, new):
+                e.scheduler.extend(s, [t])
+                s._decode_slot = int(e.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+            got.append(e.decode(seqs))
+            for s in seqs:
+                e.scheduler.computed(s, 1)
+        _close(got[0], got[1], self.dtype)
+
+    def check_caches(self):
+        """Rows and states of the live sequences."""
+        for i in range(len(self.es[0].kv_cache._layers)):
+            flat = lambda v: [t for w in (v if isinstance(v, tuple) else (v,)) for t in (w if isinstance(w, tuple) else (w,))]
+            for a, b in zip(*(flat(e.kv_cache.layer(i)) for e in self.es)):
+                if b.float().norm() > 0:
+                    _close(a, b, self.dtype)
+
+    def replays(self):
+        return self.es[0].stats["graph_replays"]
+
+    def close(self):
+        for e in self.es:
+            e.close()
+
+
+def test_shapes_come_and_go(monkeypatch):
+    from llmctl.serve import decode_graph as dg
+
+    monkeypatch.setattr(dg, "MAX_GRAPHS", 2)
+    monkeypatch.setattr(dg, "CROWDED_STEPS", 3)
+    p = _Pair("dumazen-w128-l4-h4-g2")
+    for n in (40, 41, 36, 38):
+        p.admit(n)
+    for rows in (4, 4, 4, 3, 3, 3, 2, 2, 2, 2, 4, 4, 4, 4, 3, 1, 1, 2, 1, 1, 4, 4):
+        p.step(rows)
+    p.check_caches()
+    assert p.replays() == 6 and len(p.es[0]._decode_graphs) == 2  # recorded: 4, 3, 2 (4 goes), 4 (3 goes), 1 (4 goes); one more of 2
+    p.close()
+
+
+@pytest.mark.parametrize("error,stays", [(RuntimeError, 0), (torch.OutOfMemoryError, 3)])
+def test_a_step_that_does_not_record_runs_eagerly(monkeypatch, error, stays):
+    """A failure inside the recording (memory: once) leaves caches, states and later recordings as they should be."""
+    p = _Pair("malinex-w128-l4-h4-g2-e4-s1")
+    for n in (20, 7, 40):
+        p.admit(n)
+    model, failures = p.es[0].model, []
+    logits = type(model).logits
+
+    def fail(self, x):
+        if torch.cuda.is_current_stream_capturing() and x.shape[0] == 3 and not (stays and failures):
+            failures.append(1)
+            raise error("no room")
+        return logits(self, x)
+
+    monkeypatch.setattr(type(model), "logits", fail)
+    for _ in range(5):
+        p.step(3)
+    assert len(failures) == 1 and p.replays() == stays
+    for _ in range(5):
+        p.step(2)
+    p.check_caches()
+    assert p.replays() == stays + 3
+    p.close()
+
+
+def test_exchanged_weights_are_used():
+    """Two parameters that change places, one that is another object (a checkpoint assigned), a module that is another one."""
+    p = _Pair("dumazen-w128-l4-h4-g2")
+    p.admit(20)
+    p.admit(9)
+    models = [e.model for e in p.es]
+
+    def change_places(m):
+        a, b = (m.layers[i].ff.w_down for i in (0, 1))
+        a.data, b.data = b.data, a.data
+
+    def assign(m):
+        m.load_state_dict({k: v * 0.9 if v.is_floating_point() else v for k, v in m.state_dict().items()}, assign=True)
+
+    def exchange(m):
+        m.layers[0].ff, m.layers[1].ff = m.layers[1].ff, m.layers[0].ff
+
+    for change in (None, change_places, assign, exchange):
+        before = p.replays()
+        if change is not None:
+            for m in models:
+                change(m)
+        for _ in range(4):
+            p.step(2)
+        assert p.replays() == before + 2
+    p.close()
+
+
+def test_other_threads_work_during_recordings():
+    import threading
+
+    stop, errors = threading.Event(), []
+
+    def work():
+        try:
+            s = torch.cuda.Stream()
+            with torch.cuda.stream(s):
+                k = 0
+                while not stop.is_set():
+                    k = k % 64 + 1
+                    t = torch.full((k << 14,), float(k), device="cuda")
+                    assert float(t.sum().cpu()) == k * (k << 14)
+                    torch.from_numpy(t[:8].cpu().numpy()).cuda()
+                    s.synchronize()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    th = threading.Thread(target=work)
+    th.start()
+    try:
+        p = _Pair("dumazen-w128-l4-h4-g2")
+        for n in (36, 37, 38, 39):
+            p.admit(n)
+        for rows in (4, 3, 2, 1):
+            for _ in range(4):
+                p.step(rows)
+        assert p.replays() == 8
+    finally:
+        stop.set()
+        th.join()
+    assert not errors, errors
+    p.close()
+
+
+def test_the_position_limit_holds_for_replays(monkeypatch):
+    p = _Pair("malinex-w128-l4-h4-g2-e4-s1")
+    p.admit(20)
+    for _ in range(4):
+        p.step(1)
+    assert p.replays() == 2
+    monkeypatch.setattr(type(p.es[0].model), "position_limit", 24)
+    for e in p.es:
+        with pytest.raises(ValueError, match="beyond the model's 24"):
+            s = p.live[0][p.es.index(e)]
+            e.scheduler.extend(s, [1])
+            s._decode_slot = int(e.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+            e.decode([s])
+    p.close()
 
 
 @pytest.mark.parametrize("name", ["malinex-w128-l4-h4-g2-e4-s1", "dumazen-w128-l4-h4-g2"])
