@@ -506,14 +506,19 @@ SKINNY_CONFIGS: dict = {}  # (M, N, K) -> tuned config (0 = hipBLASLt), from a t
 _ROW_ACTS = {None: 0, "gelu": 2}  # the tanh form, as :func:`gelu`
 
 
+def wants_grad(*ts) -> bool:
+    """Will autograd want a gradient through an op of these operands?  (The kernels of serving have no backward.)"""
+    return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
+
+
 def stream_takes(x, w, b=None) -> bool:
-    """Does ``csrc/stream_linear.h`` take this product?  At most 32 rows, bf16, K a multiple of 8, aligned rows.  (Asked for every
+    """Does ``csrc/stream_linear.h`` take this product?  At most 32 rows, bf16, K a multiple of 8, aligned rows, no gradient.  (Asked for every
     projection of an eager step: one look at each property.)"""
     if not (x.is_cuda and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16):
         return False
     xs, ws, (M, K) = x.stride(), w.stride(), x.shape
     return (1 <= M <= 32 and xs[1] == 1 and ws[1] == 1 and (xs[0] | ws[0] | K) & 7 == 0 and (x.data_ptr() | w.data_ptr()) & 15 == 0
-            and (b is None or (b.dtype is torch.bfloat16 and b.is_contiguous())) and use_native(x))
+            and (b is None or (b.dtype is torch.bfloat16 and b.is_contiguous())) and use_native(x) and not wants_grad(x, w, b))
 
 
 def stream_ok(x, w, b=None) -> bool:
@@ -588,7 +593,7 @@ def norm_linear_ok(x, res, nw, nb, w, b, split: bool = False) -> bool:
     short rows and up to 8192 outputs: up to 12 rows of 1024 (8 of 2048); ``split``: four more, as the launch that splits QKV goes too.
     us in a graph, fused / separate: K 768, N 3072: 1 row 4.8 / 6.7, 8 rows 6.3 / 7.2, 12 rows 7.3 / 7.4, 16 rows 8.3 / 7.6; K 2048, N 3072:
     1 row 8.0 / 9.8, 8 rows 10.0 / 10.8, 12 rows 11.8 / 11.0; N 16384, K 768: 1 row 11.8 / 10.8."""
-    if nb is None or not (x.dim() == 2 and stream_ok(x, w, b)):
+    if nb is None or not (x.dim() == 2 and stream_ok(x, w, b)) or wants_grad(res, nw, nb):
         return False
     (M, K), N = x.shape, w.shape[0]
     bf = all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, nw, nb) + (() if res is None else (res,)))

@@ -21,7 +21,7 @@ import torch
 
 from . import ref_hybrid as ref
 from ._lib import native_hybrid, use_native
-from .functional import stream_ok
+from .functional import stream_ok, wants_grad
 
 
 def layernorm_f32(x, w, b, eps: float, out_dtype):
@@ -172,7 +172,7 @@ def head_rows_ok(x, w) -> bool:
     multiple of 4, N of 8, aligned rows."""
     return (use_native(x) and 1 <= x.shape[0] <= 32 and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 4 == 0
             and w.shape[2] % 8 == 0 and x.stride(2) == 1 and x.stride(0) % 4 == 0 and x.stride(1) % 4 == 0 and x.data_ptr() % 8 == 0
-            and w.data_ptr() % 16 == 0)
+            and w.data_ptr() % 16 == 0 and not wants_grad(x, w))
 
 
 def latent_queries(q, w_uk, pos, inv_freq, rot_dims: int, interleaved: bool = False, amp: float = 1.0):
@@ -405,6 +405,8 @@ def linear_f32(x, w):
         return torch.nn.functional.linear(x, w)
     if rows_ok(x, w):
         return rows_linear(x, w, f32=True)
+    if wants_grad(x, w):  # (the library's product with another output type has no derivative)
+        return torch.nn.functional.linear(x, w).float()
     try:
         return torch.mm(x, w.t(), out_dtype=torch.float32)
     except (TypeError, RuntimeError):
