@@ -99,3 +99,26 @@ def test_route_matches_the_choice_kernels(T, W, E, top, groups, keep, kind):
     assert safe.float().mean() > 0.9
     assert torch.equal(idx.long()[safe], ri[safe])
     assert torch.allclose(w[safe], rw[safe], rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("layout", ["off by four bytes", "transposed"])
+@pytest.mark.parametrize("T", [6, 80])
+@pytest.mark.parametrize("kind", ["group", "softmax"])
+def test_routers_in_other_layouts(kind, T, layout):
+    """A router that is a slice of a larger buffer, or a transposed matrix: the layer's general form takes it."""
+    from llmctl.models.moe import BiasedSoftmaxMoE, GroupLimitedMoE
+
+    torch.manual_seed(0)
+    kw = dict(device="cuda", dtype=torch.bfloat16)
+    m = GroupLimitedMoE(64, 32, 4, 2, 2, 1, **kw) if kind == "group" else BiasedSoftmaxMoE(64, 32, 4, 2, "relu2", **kw)
+    x = torch.randn(T, 64, device="cuda").bfloat16()
+    with torch.no_grad():
+        want = m(x)
+        w = m.w_router.detach()
+        buf = torch.zeros(w.numel() + 1, device="cuda")
+        other = buf[1:].view_as(w) if layout != "transposed" else torch.empty(64, 4, device="cuda").t()
+        other.copy_(w)
+        m.w_router.data = other
+        assert not m.w_router.is_contiguous() or m.w_router.data_ptr() % 16
+        got = m(x)
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()  # the general form rounds every expert's result to bf16
