@@ -393,6 +393,8 @@ def bias_grad(b: torch.nn.Parameter, dy2: torch.Tensor) -> Optional[torch.Tensor
         ops.col_sum_(dy2, g, add)
         sink.close(b)
         return None
+    if torch.is_grad_enabled():  # a backward that is differentiated itself (create_graph)
+        return dy2.sum(0)
     db = torch.empty(b.shape, dtype=dy2.dtype, device=dy2.device)
     ops.col_sum_(dy2, db, False)
     return db

@@ -74,3 +74,16 @@ def test_unrotated_qkv_attention(B, S, nq, nkv, D, docs):
     o2 = ops.flash_attention(q, k, v, causal=True, doc_start=ds)
     o2.backward(do)
     assert torch.equal(o, o2) and torch.equal(qkv.grad, ref.grad)  # the same kernels on other strides
+
+
+def test_a_bias_gradient_can_be_differentiated():
+    from llmctl.exec.linear import linear
+
+    g = torch.Generator().manual_seed(0)
+    r = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
+    x, w, b = r(24, 64), r(32, 64), r(32).requires_grad_()
+    y = linear(x, w, b)
+    (gb,) = torch.autograd.grad((y.float() ** 3).sum(), b, create_graph=True)  # sum over rows of 3 y^2
+    (ggb,) = torch.autograd.grad(gb.float().sum(), b)  # sum over rows of 6 y
+    want = 6 * (x.double() @ w.double().t() + b.double()).sum(0)
+    assert (ggb.double() - want).norm() <= 2.0 ** -5 * want.norm()
