@@ -422,8 +422,10 @@ class MLSTM(nn.Module):
         g = z[:, 2 * H * dk + H * dv:]
         gates = F.linear(h.float(), self.w_if)  # fp32 [T, 2H]
         S, n, m = state
+        if "mlstm_plan" not in b.scratch:
+            b.scratch["mlstm_plan"] = hops.mlstm_chunk_plan(b.cu_host, h.device) if h.is_cuda and dk <= 128 else None
         o = hops.mlstm_scan(q, k, v, gates, self.b_i, self.b_f, self.cap, 1.0 / math.sqrt(dk), S, n, m, b.state,
-                            b.cu, b.start, cu_host=b.cu_host)
+                            b.cu, b.start, plan=b.scratch["mlstm_plan"])
         return hops.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
 
 

@@ -206,32 +206,41 @@ MLSTM_MIN = 40  # portions from here on take it (us, scan / chunks, 16 heads of 
 # 256 329 / 53; 8 heads of 128 x 128: 16 tokens 60 / 55, 32 97 / 56)
 
 
-def mlstm_scan(q, k, v, if_raw, b_i, b_f, cap: float, qscale: float, S, n, m, state_slots, cu, start, slab: bool = False,
-               cu_host=None):
-    """mLSTM recurrence over the step's tokens; returns the un-normalised head outputs fp32
-    ``[T, H, dv]`` and updates the state pools in place.  ``slab`` forces the block-per-tile kernel
-    (the form for key dims above 128) where the wave-per-tile one would run.  ``cu_host`` (the row
-    offsets as a host list) lets long portions run chunk-parallel (:func:`_mlstm_chunked`)."""
-    if use_native(q):
-        if (cu_host is not None and not slab and q.shape[-1] <= 128
-                and max((b - a for a, b in zip(cu_host[:-1], cu_host[1:])), default=0) >= MLSTM_MIN):
-            return _mlstm_chunked(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, start, cu_host)
-        return native_hybrid().mlstm_scan(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, cu, start, slab)
-    return ref.mlstm_scan(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, cu, start)
-
-
-def _mlstm_chunked(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, start, cu_host):
-    """The same recurrence in chunks of 64 tokens as matrix products (``csrc/hybrid/mlstm_chunk.hip``): every chunk's own contribution,
-    the states at the chunks' first tokens in order (and the new carried states), every chunk's outputs from its state."""
+def mlstm_chunk_plan(cu_host, device):
+    """The chunks of a step's portions for :func:`mlstm_scan`, or None when no portion is long enough: (chunk row offsets, sequence of
+    every chunk, first chunk of every sequence) on ``device``.  It depends on the step only, so the layers of a model share one (with
+    a plan of its own, uploaded with a wait, a Lenitar prompt of 2048 tokens took 1727 us where it takes 1585 so, with one such layer in
+    four)."""
+    if cu_host is None or max((b - a for a, b in zip(cu_host[:-1], cu_host[1:])), default=0) < MLSTM_MIN:
+        return None
     cu, base, seq = [0], [0], []
     for s, (a, b) in enumerate(zip(cu_host[:-1], cu_host[1:])):
         cu += [min(t + MLSTM_CHUNK, b) for t in range(a, b, MLSTM_CHUNK)]
         seq += [s] * (len(cu) - 1 - len(seq))
         base.append(len(seq))
     P = len(seq)
-    plan = torch.tensor(cu + seq + base, dtype=torch.int32).to(q.device)  # blocking: the host tensor is a temporary
-    return native_hybrid().mlstm_chunked(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, start, plan[:P + 1],
-                                         plan[P + 1:2 * P + 1], plan[2 * P + 1:])
+    # pinned (the allocator keeps it until the copy is over): the host does not wait for what is queued
+    plan = torch.tensor(cu + seq + base, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+    return plan[:P + 1], plan[P + 1:2 * P + 1], plan[2 * P + 1:]
+
+
+def mlstm_scan(q, k, v, if_raw, b_i, b_f, cap: float, qscale: float, S, n, m, state_slots, cu, start, slab: bool = False,
+               cu_host=None, plan=None):
+    """mLSTM recurrence over the step's tokens; returns the un-normalised head outputs fp32
+    ``[T, H, dv]`` and updates the state pools in place.  ``slab`` forces the block-per-tile kernel
+    (the form for key dims above 128) where the wave-per-tile one would run.  ``cu_host`` (the row
+    offsets as a host list) or ``plan`` (:func:`mlstm_chunk_plan` of them) lets long portions run in chunks of 64 tokens as matrix products
+    (``csrc/hybrid/mlstm_chunk.hip``): every chunk's own contribution, the states at the chunks' first tokens in order (and the new
+    carried states), every chunk's outputs from its state."""
+    if use_native(q):
+        if not slab and q.shape[-1] <= 128:
+            if plan is None and cu_host is not None:
+                plan = mlstm_chunk_plan(cu_host, q.device)
+            if plan is not None:
+                chunks, seq, base = plan
+                return native_hybrid().mlstm_chunked(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, start, chunks, seq, base)
+        return native_hybrid().mlstm_scan(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, cu, start, slab)
+    return ref.mlstm_scan(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, cu, start)
 
 
 def headnorm_gate(o, w, g, eps: float, out_dtype, silu: bool = False):

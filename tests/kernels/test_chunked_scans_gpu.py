@@ -99,3 +99,18 @@ def test_gla_chunks(H, dk, dv, dtype, gain, lens):
             Ca = a[:, :, None] * Ca + kt[:, :, None].abs() * vt[:, None, :].abs()
             _check(got[t], torch.einsum("hkv,hk->hv", C, qt), torch.einsum("hkv,hk->hv", Ca, qt.abs()))
         _check(Sd[sl], C, Ca)
+
+
+def test_the_layers_of_a_step_share_one_plan(monkeypatch):
+    from llmctl.serve.engine import InferenceEngine
+    from llmctl.serve.scheduler import PrefillChunk
+
+    e = InferenceEngine("lenitar-w128-l8", device="cuda", max_batch_size=2, num_kv_blocks=32, block_size=16, max_model_len=256, prefix_caching=False)
+    assert sum(type(m).__name__ == "MLSTM" for m in e.model.modules()) >= 2
+    calls, plan = [], hops.mlstm_chunk_plan
+    monkeypatch.setattr(hops, "mlstm_chunk_plan", lambda *a: calls.append(1) or plan(*a))
+    for _ in range(2):
+        s = e.open_sequence(list(range(1, 90)))
+        e.prefill([PrefillChunk(s, 0, 89)])
+    assert len(calls) == 2  # one a step
+    e.close()
