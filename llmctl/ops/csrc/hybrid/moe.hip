@@ -14,10 +14,11 @@
 //     (64-wide tiles: the next three) in registers under the MFMAs of this one.  16-byte chunks are swizzled by the row, so a wave's fragment
 //     reads touch every bank slot equally.  The weight fragment is the MFMA row operand: a lane ends up with four neighbouring
 //     columns of one token.  Gate and up columns of the same place belong to the same wave, which makes the gated activation
-//     lane-local.  Consecutive tiles of one expert go to one XCD, whose L2 then holds that expert's weights once.
+//     lane-local.  Consecutive tiles go to one XCD, in bands of eight row tiles that walk the columns together.
 //   * moe_small_kernel (steps of at most 64 tokens: decode): weight streaming.  A workgroup owns 16 output rows of one expert
 //     (gate and up: 2 x 16), its four waves split K; it finds its rows by scanning the choices itself, so no grouping pass
-//     runs; experts that no token chose are never read.
+//     runs.  Below two copies per expert, experts that no token chose are not read; from there on, where nearly every one has some, a wave
+//     asks for its first steps (8, or 4 from 33 tokens on) before it knows.
 //   * moe_combine_kernel: out_t = sum_k w_tk y_tk (+ w x_t for experts without weights) (+ the shared expert), fp32.
 //
 // A row tile has 128 rows when the experts get 96 or more on average, else 64 (and 64 columns): below that the grid
@@ -267,6 +268,10 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 
 // ------------------------------------------------------------------------------------------------ tiles
 enum { UP_GLU = 0, UP_PLAIN = 1, DOWN = 2 };
+// Row tiles that walk the columns together: an XCD's neighbouring workgroups then share weights as well as rows.  One at a time, every row tile read its
+// expert's weights from the memory side again.  Whole layer, us, one / eight at a time (2, 4, 16 and 32 lie between): 8 gated experts of 4096 x 8192, top 2,
+// 2048 tokens 1476 / 1136, 16384 tokens 11072 / 7517; 2048 x 4096 at 2048 340 / 325, 16384 2138 / 1979; 2048 x 1024 at 2048 118 / 119.
+constexpr int BAND = 8;
 
 struct TileArgs {
   const bf16_t* a;  // UP: the step's rows [T, K]; DOWN: the activations by sorted row [N, K]
@@ -292,7 +297,8 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
   if (id >= real) return;
   const int q8 = real >> 3, r8 = real & 7, xcd = id & 7;
   const int tile = xcd * q8 + min(xcd, r8) + (id >> 3);
-  const int mt = tile / g.ntile, nt = tile - mt * g.ntile;
+  const int first = tile / (BAND * g.ntile) * BAND, in = tile - first * g.ntile, high = min(BAND, g.tiles[0] - first);
+  const int nt = in / high, mt = first + in - nt * high;
   const int e = g.tiles[1 + 3 * mt], row0 = g.tiles[2 + 3 * mt], rows = g.tiles[3 + 3 * mt];
   const bf16_t* __restrict__ w = g.w.p[e];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
