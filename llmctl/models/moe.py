@@ -221,14 +221,16 @@ class GroupLimitedMoE(nn.Module):
         from llmctl.ops import hybrid as hops
 
         up = self.experts_up[0]
-        return hops.experts_ok(up[:1], self.experts_up, self.experts_down, self.E, self.top, self.w_router)
+        return (hops.experts_pay(T, self.top, self.E, *up.shape)
+                and hops.experts_ok(up[:1], self.experts_up, self.experts_down, self.E, self.top, self.w_router))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x [T, width] -> fp32 [T, width]."""
         from llmctl.ops import hybrid as hops
 
         T = x.shape[0]
-        if hops.experts_ok(x, self.experts_up, self.experts_down, self.E, self.top, self.w_router):
+        if (hops.experts_pay(T, self.top, self.E, 2 * self.ff, x.shape[1])
+                and hops.experts_ok(x, self.experts_up, self.experts_down, self.E, self.top, self.w_router)):
             return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, self.experts_up,
                                        self.experts_down, "swiglu")
         topi, topw = hops.group_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.top,
@@ -344,7 +346,8 @@ class BiasedSoftmaxMoE(nn.Module):
         from llmctl.ops import hybrid as hops
 
         down = self.w_down.view(-1, self.E, self.ff).transpose(0, 1)
-        return self._dense(T) or hops.experts_ok(self.w_up[0, :1], self.w_up, down, self.E + self.identity, self.top, self.w_router)
+        return self._dense(T) or (hops.experts_pay(T, self.top, self.E, *self.w_up.shape[1:]) and hops.experts_ok(
+            self.w_up[0, :1], self.w_up, down, self.E + self.identity, self.top, self.w_router))
 
     def forward(self, x: torch.Tensor):
         """x [T, width] -> fp32 [T, width] (and the side columns)."""
@@ -369,7 +372,8 @@ class BiasedSoftmaxMoE(nn.Module):
                 ys = hops.linear(u if fused else act(u), self.w_sdown)
         gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
         down = self.w_down.view(x.shape[1], self.E, self.ff).transpose(0, 1)  # [E, width, ff]
-        if hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router):
+        if (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1])
+                and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
             out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
                                       self.act, ys, gate)
             return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out

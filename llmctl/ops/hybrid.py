@@ -440,6 +440,16 @@ def experts_ok(x, up, down, outputs: int, top: int = 1, w_router=None) -> bool:
             and all(w.stride() == ws[0].stride() for ws in (ups, downs) for w in ws))
 
 
+def experts_pay(T: int, top: int, E: int, rows: int, width: int) -> bool:
+    """Is :func:`routed_experts` faster than a pair of library products per expert?  Unless the experts are large (``rows`` x ``width`` of
+    the first projection from 7 * 2^23 on) and get many rows each (2048 of that size, fewer of larger ones): there the library's tiles
+    win back the host's wait and the extra passes.  Whole layer, 8 experts, top 2, ms, grouped / per expert: gated 4096 x 14336 at 2048 tokens
+    2.0 / 2.0, 8192 6.7 / 5.7; gated 4096 x 8192 at 4096 2.0 / 2.1, 16384 7.2 / 6.5; plain 4096 x 14336 at 4096 2.47 / 2.49, 8192 4.6 / 4.0; plain
+    4096 x 8192 at 16384 4.8 / 5.2; gated 2048 x 8192 at 32768 7.4 / 7.7."""
+    size = rows * width
+    return size < 7 << 23 or T * top // E * size < 7 << 34
+
+
 def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax: bool, renorm: bool, up, down, act: str, shared=None,
                    gate=None):
     """``sum_k w_k expert_k(x_t)`` over the chosen experts of every row of ``x [T, W]`` (bf16) -> fp32 ``[T, W]``, all on the device:

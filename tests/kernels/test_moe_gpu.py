@@ -122,3 +122,26 @@ def test_routers_in_other_layouts(kind, T, layout):
         assert not m.w_router.is_contiguous() or m.w_router.data_ptr() % 16
         got = m(x)
     assert (got - want).norm() <= 2.0 ** -7 * want.norm()  # the general form rounds every expert's result to bf16
+
+
+@pytest.mark.parametrize("kind", ["group", "softmax"])
+def test_large_experts_with_many_rows_take_library_products(kind, monkeypatch):
+    """On either side of the line, with it moved to a size for tests: the same results, and the form that the rule names."""
+    from llmctl.models.moe import BiasedSoftmaxMoE, GroupLimitedMoE
+    from llmctl.ops import hybrid as hops
+
+    assert hops.experts_pay(1 << 20, 2, 8, 16384, 2048) and hops.experts_pay(4096, 2, 8, 16384, 4096)
+    assert not hops.experts_pay(16384, 2, 8, 16384, 4096) and not hops.experts_pay(4096, 2, 8, 28672, 4096) and hops.experts_pay(4095, 2, 8, 28672, 4096)
+    torch.manual_seed(0)
+    kw = dict(device="cuda", dtype=torch.bfloat16)
+    m = GroupLimitedMoE(64, 32, 4, 2, 2, 1, **kw) if kind == "group" else BiasedSoftmaxMoE(64, 32, 4, 2, "relu2", **kw)
+    x = torch.randn(80, 64, device="cuda").bfloat16()
+    grouped, calls = hops.routed_experts, []
+    monkeypatch.setattr(hops, "routed_experts", lambda *a: calls.append(1) or grouped(*a))
+    with torch.no_grad():
+        want = m(x)
+        assert calls and m.on_device(80)
+        monkeypatch.setattr(hops, "experts_pay", lambda *a: False)
+        got = m(x)
+        assert len(calls) == 1 and (kind == "softmax" or not m.on_device(80))
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()
