@@ -18,11 +18,19 @@ namespace llmctl_hybrid {
 
 __device__ __forceinline__ float log_sigmoid(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
 
-// raw [T, 2H] -> (i, f): i = cap tanh((z_i + b_i) / cap), f = logsigmoid(cap tanh((z_f + b_f) / cap))
+// raw [T, 2H] -> (i, f): i = cap tanh((z_i + b_i) / cap), f = logsigmoid(cap tanh((z_f + b_f) / cap)).  And the carried normalisers and log-scales of
+// the step's sequences to n0 [ns, H, dk] and m0 [ns, H]: every value tile of a head starts from them, and the first one to end stores the new ones
+// while others may not have begun (65 sequences of 16 heads and two tiles: results 3 % off).
 __global__ void mlstm_gates_kernel(const float* __restrict__ raw, const float* __restrict__ b_i, const float* __restrict__ b_f,
-                                   float cap, float* __restrict__ out, int64_t T, int H) {
+                                   float cap, float* __restrict__ out, int64_t T, int H, const float* __restrict__ np, const float* __restrict__ mp,
+                                   const int* __restrict__ slots, float* __restrict__ n0, float* __restrict__ m0, int ns, int dk) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= T * 2 * H) return;
+  if (i >= T * 2 * H) {
+    const int64_t j = i - T * 2 * H, nn = (int64_t)ns * H * dk, hd = (int64_t)H * dk;
+    if (j < nn) n0[j] = np[slots[j / hd] * hd + j % hd];
+    else if (j < nn + (int64_t)ns * H) m0[j - nn] = mp[(int64_t)slots[(j - nn) / H] * H + (j - nn) % H];
+    return;
+  }
   const int c = (int)(i % (2 * H));
   if (c < H) out[i] = cap * tanhf((raw[i] + b_i[c]) / cap);
   else out[i] = log_sigmoid(cap * tanhf((raw[i] + b_f[c - H]) / cap));
@@ -48,6 +56,7 @@ template <typename T, int DK>
 __global__ __launch_bounds__(64) void mlstm_scan_wave_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                              int64_t row_stride, const float* __restrict__ gates, float qscale,
                                                              float* __restrict__ Sp, float* __restrict__ np, float* __restrict__ mp,
+                                                             const float* __restrict__ n0, const float* __restrict__ m0,
                                                              const int* __restrict__ slots, const int* __restrict__ cu,
                                                              const int* __restrict__ start, float* __restrict__ out, int H, int dk,
                                                              int dv) {
@@ -68,8 +77,8 @@ __global__ __launch_bounds__(64) void mlstm_scan_wave_kernel(const T* __restrict
 #pragma unroll
   for (int d = 0; d < DK; ++d) S[d] = (!fresh && cok && d < dk) ? Sb[(int64_t)d * dv + col] : 0.f;
 #pragma unroll
-  for (int i = 0; i < NR; ++i) nr[i] = (!fresh && lane + 64 * i < dk) ? nb[lane + 64 * i] : 0.f;
-  float m = fresh ? 0.f : mp[slot * H + h];
+  for (int i = 0; i < NR; ++i) nr[i] = (!fresh && lane + 64 * i < dk) ? n0[((int64_t)sq * H + h) * dk + lane + 64 * i] : 0.f;
+  float m = fresh ? 0.f : m0[(int64_t)sq * H + h];
   // operands of TBATCH tokens are loaded ahead, one batch in flight while the previous one is processed
   // (a single wave has nothing else to hide a load behind)
   constexpr int TBATCH = 8;
@@ -161,8 +170,8 @@ template <typename T, int DS>  // DS: rows per slab held in registers (>= ceil(d
 __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v,
                                                          int64_t row_stride, const float* __restrict__ gates,
                                                          float qscale, float* __restrict__ Sp, float* __restrict__ np,
-                                                         float* __restrict__ mp, const int* __restrict__ slots,
-                                                         const int* __restrict__ cu, const int* __restrict__ start,
+                                                         float* __restrict__ mp, const float* __restrict__ n0, const float* __restrict__ m0,
+                                                         const int* __restrict__ slots, const int* __restrict__ cu, const int* __restrict__ start,
                                                          float* __restrict__ out, int H, int dk, int dv) {
   extern __shared__ float sm[];
   float* qk = sm;                    // [2][2 dk]
@@ -186,9 +195,9 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ q
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int r = lane + 64 * i;
-    nr[i] = (!fresh && r < rows && d0 + r < dk) ? nb[d0 + r] : 0.f;
+    nr[i] = (!fresh && r < rows && d0 + r < dk) ? n0[((int64_t)sq * H + h) * dk + d0 + r] : 0.f;
   }
-  float m = fresh ? 0.f : mp[slot * H + h];
+  float m = fresh ? 0.f : m0[(int64_t)sq * H + h];
   for (int t = a; t < b; ++t) {
     const int buf = (t - a) & 1;
     float* qs = qk + buf * 2 * dk;
@@ -273,11 +282,13 @@ at::Tensor mlstm_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor
   c10::DeviceGuard guard(q.device());
   at::Tensor out = at::empty({T, H, dv}, q.options().dtype(at::kFloat));
   if (T == 0 || ns == 0) return out;
-  at::Tensor act = at::empty_like(gates);
+  at::Tensor act = at::empty_like(gates), n0 = at::empty({ns, H, dk}, out.options()), m0 = at::empty({ns, H}, out.options());
   {
-    const int64_t ng = T * 2 * H;
-    mlstm_gates_kernel<<<dim3((unsigned)((ng + 255) / 256)), 256, 0, cur_stream()>>>(gates.data_ptr<float>(), b_i.data_ptr<float>(),
-                                                                                    b_f.data_ptr<float>(), (float)cap, act.data_ptr<float>(), T, (int)H);
+    const int64_t ng = T * 2 * H + ns * H * (dk + 1);
+    HYB_CHECK((ng + 255) / 256 < ((int64_t)1 << 31), "grid too large");
+    mlstm_gates_kernel<<<dim3((unsigned)((ng + 255) / 256)), 256, 0, cur_stream()>>>(
+        gates.data_ptr<float>(), b_i.data_ptr<float>(), b_f.data_ptr<float>(), (float)cap, act.data_ptr<float>(), T, (int)H, n.data_ptr<float>(),
+        m.data_ptr<float>(), slots.data_ptr<int>(), n0.data_ptr<float>(), m0.data_ptr<float>(), (int)ns, (int)dk);
   }
   const int rows = (int)((dk + 3) / 4);
   const size_t lds = (size_t)(4 * dk + 2 * 4 * 65) * sizeof(float);
@@ -289,8 +300,8 @@ at::Tensor mlstm_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor
     auto go = [&](auto kern, int threads, size_t shm) {
       kern<<<grid, threads, shm, cur_stream()>>>((const Tt*)q.data_ptr(), (const Tt*)k.data_ptr(), (const Tt*)v.data_ptr(), row_stride,
                                                 act.data_ptr<float>(), (float)qscale, S.data_ptr<float>(), n.data_ptr<float>(),
-                                                m.data_ptr<float>(), slots.data_ptr<int>(), cu.data_ptr<int>(), start.data_ptr<int>(),
-                                                out.data_ptr<float>(), (int)H, (int)dk, (int)dv);
+                                                m.data_ptr<float>(), n0.data_ptr<float>(), m0.data_ptr<float>(), slots.data_ptr<int>(),
+                                                cu.data_ptr<int>(), start.data_ptr<int>(), out.data_ptr<float>(), (int)H, (int)dk, (int)dv);
     };
     auto launch = [&](auto kern) { go(kern, 256, lds); };
     if (!slab && dk <= 16) go(mlstm_scan_wave_kernel<Tt, 16>, 64, 0);

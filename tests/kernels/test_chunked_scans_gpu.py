@@ -114,3 +114,37 @@ def test_the_layers_of_a_step_share_one_plan(monkeypatch):
         e.prefill([PrefillChunk(s, 0, 89)])
     assert len(calls) == 2  # one a step
     e.close()
+
+
+@pytest.mark.parametrize("slab", [False, True])
+@pytest.mark.parametrize("ns,H,dk,dv", [(300, 16, 64, 256), (128, 16, 32, 200), (64, 8, 16, 64)])
+def test_mlstm_decode_rows_of_many_sequences(ns, H, dk, dv, slab):
+    """One token each: every value tile of a head starts from the carried normaliser and log-scale, however late it begins."""
+    from llmctl.ops._lib import native_hybrid
+
+    g = torch.Generator(device="cuda").manual_seed(ns)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    q, k, v = r(ns, H, dk), r(ns, H, dk), r(ns, H, dv)
+    z = torch.cat([t.reshape(ns, -1) for t in (q, k, v)], 1).contiguous()  # rows of one projection
+    q, k, v = (z[:, a:a + H * w].unflatten(1, (H, w)) for a, w in ((0, dk), (H * dk, dk), (2 * H * dk, dv)))
+    raw, b_i, b_f, cap, qs = r(ns, 2 * H), r(H), r(H) + 2, 15.0, dk ** -0.5
+    S, n, m = r(ns, H, dk, dv), r(ns, H, dk), r(ns, H)
+    slots = torch.randperm(ns, generator=torch.Generator().manual_seed(1)).int().cuda()
+    i32 = lambda n: torch.arange(n, dtype=torch.int32, device="cuda")
+    for _ in range(4):
+        i = cap * torch.tanh((raw[:, :H].double() + b_i) / cap)
+        f = torch.nn.functional.logsigmoid(cap * torch.tanh((raw[:, H:].double() + b_f) / cap))
+        S0, n0, m0 = S[slots.long()].double(), n[slots.long()].double(), m[slots.long()].double()
+        m1 = torch.maximum(f + m0, i)
+        a, b = torch.exp(f + m0 - m1), torch.exp(i - m1)
+        S1 = a[..., None, None] * S0 + b[..., None, None] * k.double()[..., None] * v.double()[:, :, None]
+        n1 = a[..., None] * n0 + b[..., None] * k.double()
+        den = torch.maximum((n1 * q.double() * qs).sum(-1).abs(), torch.exp(-m1)) + 1e-6
+        num = (S1 * q.double()[..., None] * qs).sum(2)
+        got = native_hybrid().mlstm_scan(q, k, v, raw, b_i, b_f, cap, qs, S, n, m, slots, i32(ns + 1), torch.ones_like(slots), slab)
+        # the quotient's parts are fp32 sums of dk products: 2^-17 of their terms' size each
+        size = (S1.abs() * q.double().abs()[..., None] * qs).sum(2) / den[..., None]
+        rel = (n1.abs() * q.double().abs() * qs).sum(-1) / den
+        assert ((got.double() - num / den[..., None]).abs() <= 2.0 ** -16 * (size + rel[..., None] * (num / den[..., None]).abs()) + 1e-6).all()
+        for pool, want in ((S, S1), (n, n1), (m, m1)):
+            assert (pool[slots.long()].double() - want).norm() <= 2.0 ** -18 * want.norm()
