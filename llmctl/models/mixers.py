@@ -422,10 +422,11 @@ class MLSTM(nn.Module):
         g = z[:, 2 * H * dk + H * dv:]
         gates = F.linear(h.float(), self.w_if)  # fp32 [T, 2H]
         S, n, m = state
-        if "mlstm_plan" not in b.scratch:
-            b.scratch["mlstm_plan"] = hops.mlstm_chunk_plan(b.cu_host, h.device) if h.is_cuda and dk <= 128 else None
+        key = ("mlstm_plan", H, dk, dv)
+        if key not in b.scratch:
+            b.scratch[key] = hops.mlstm_chunk_plan(b.cu_host, h.device, H, dk, dv) if h.is_cuda else None
         o = hops.mlstm_scan(q, k, v, gates, self.b_i, self.b_f, self.cap, 1.0 / math.sqrt(dk), S, n, m, b.state,
-                            b.cu, b.start, plan=b.scratch["mlstm_plan"])
+                            b.cu, b.start, plan=b.scratch[key])
         return hops.linear(hops.headnorm_gate(o, self.norm, g, self.eps, h.dtype), self.w_o)
 
 
@@ -480,12 +481,11 @@ class GatedLinearAttention(nn.Module):
         v = z[:, c:e].unflatten(1, (H, dv))
         g = z[:, e:e + H * dv]
         decay = _mm_f32(z[:, e + H * dv:self.cols], self.w_a2)  # fp32 [T, H * dk]
-        least = hops.gla_least(dk)
-        plan = f"gla_plan{least}"
-        if plan not in b.scratch:
-            b.scratch[plan] = hops.gla_chunk_plan(b.cu_host, h.device, least) if h.is_cuda else None
+        key = ("gla_plan", H, dk, dv)
+        if key not in b.scratch:
+            b.scratch[key] = hops.gla_plan(b.cu_host, h.device, H, dk, dv) if h.is_cuda else None
         o = hops.gla_scan(q, k, v, decay, self.b_a2, self.tau, dk ** -0.5, state[0], b.state, b.cu, b.start,
-                          plan=b.scratch[plan])
+                          plan=b.scratch[key])
         y = hops.linear(hops.headnorm_gate(o, self._norm_rows(), g, self.eps, h.dtype, silu=True), self.w_o)
         return (y, z[:, self.cols:]) if self.side else y
 

@@ -202,16 +202,34 @@ def sigmoid_gate_mul(o, g):
 
 
 MLSTM_CHUNK = 64  # tokens per chunk of the chunked form
-MLSTM_MIN = 40  # portions from here on take it (us, scan / chunks, 16 heads of 64 x 128: 16 tokens 29 / 48, 32 49 / 47, 64 91 / 50,
-# 256 329 / 53; 8 heads of 128 x 128: 16 tokens 60 / 55, 32 97 / 56)
 
 
-def mlstm_chunk_plan(cu_host, device):
-    """The chunks of a step's portions for :func:`mlstm_scan`, or None when no portion is long enough: (chunk row offsets, sequence of
-    every chunk, first chunk of every sequence) on ``device``.  It depends on the step only, so the layers of a model share one (with
-    a plan of its own, uploaded with a wait, a Lenitar prompt of 2048 tokens took 1727 us where it takes 1585 so, with one such layer in
-    four)."""
-    if cu_host is None or max((b - a for a, b in zip(cu_host[:-1], cu_host[1:])), default=0) < MLSTM_MIN:
+def _chunks_pay(cu_host, H: int, dk: int, dv: int, scan, chunks) -> bool:
+    """Are a step's portions faster in chunks of 64 tokens than scanned token by token?  A scan lasts as long as its longest portion (L
+    tokens), whatever else runs beside it; every chunk, a one-token portion's too, costs its workgroups and passes over a state.  ``scan``:
+    us = a + L (b + c dk), ``chunks``: us = a + P H (b + c dk dv) for P chunks, fitted to 231 steps each (1 to 64 portions of 24 to 255 tokens
+    beside 0 to 64 of one, 4 to 64 heads of 16 x 16 to 128 x 256).  A quarter in favour of the scan: the choice is then 2 to 3 % off the
+    faster form on average, and at no such step more than 4 us slower than the scan."""
+    lens = [b - a for a, b in zip(cu_host[:-1], cu_host[1:])]
+    L = max(lens, default=0)
+    if L < 16 or L >= 256:
+        return L >= 256
+    P = sum((n + 63) // 64 for n in lens)
+    return 1.25 * (chunks[0] + P * H * (chunks[1] + chunks[2] * dk * dv)) < scan[0] + L * (scan[1] + scan[2] * dk)
+
+
+def _upload_ints(values, device):
+    """int32 on ``device``.  From pinned memory, which its allocator keeps until the copy is over: the host does not wait for what is queued."""
+    return torch.tensor(values, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+
+
+def mlstm_chunk_plan(cu_host, device, H: int, dk: int, dv: int):
+    """The chunks of a step's portions for :func:`mlstm_scan` of ``H`` heads of ``dk`` x ``dv``, or None where the scan is faster (16 heads of 64 x
+    128, us, scan / chunks: one portion of 24 tokens 40 / 24, of 255 328 / 29, 64 of 40 tokens 81 / 114, one of 64 beside 64 of one
+    token 105 / 120): (chunk row offsets, sequence of every chunk, first chunk of every sequence) on ``device``.  It depends on the step
+    only, so the layers of a model share one (with a plan of its own, uploaded with a wait, a Lenitar prompt of 2048 tokens took 1727 us
+    where it takes 1585 so, with one such layer in four)."""
+    if cu_host is None or dk > 128 or not _chunks_pay(cu_host, H, dk, dv, (15.0, 0.28, 0.021), (22.0, 0.005, 1.1e-5)):
         return None
     cu, base, seq = [0], [0], []
     for s, (a, b) in enumerate(zip(cu_host[:-1], cu_host[1:])):
@@ -219,8 +237,7 @@ def mlstm_chunk_plan(cu_host, device):
         seq += [s] * (len(cu) - 1 - len(seq))
         base.append(len(seq))
     P = len(seq)
-    # pinned (the allocator keeps it until the copy is over): the host does not wait for what is queued
-    plan = torch.tensor(cu + seq + base, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+    plan = _upload_ints(cu + seq + base, device)
     return plan[:P + 1], plan[P + 1:2 * P + 1], plan[2 * P + 1:]
 
 
@@ -235,7 +252,7 @@ def mlstm_scan(q, k, v, if_raw, b_i, b_f, cap: float, qscale: float, S, n, m, st
     if use_native(q):
         if not slab and q.shape[-1] <= 128:
             if plan is None and cu_host is not None:
-                plan = mlstm_chunk_plan(cu_host, q.device)
+                plan = mlstm_chunk_plan(cu_host, q.device, *q.shape[1:], v.shape[2])
             if plan is not None:
                 chunks, seq, base = plan
                 return native_hybrid().mlstm_chunked(q, k, v, if_raw, b_i, b_f, cap, qscale, S, n, m, state_slots, start, chunks, seq, base)
@@ -294,13 +311,15 @@ def embed_rmsnorm_f32(ids, pos, table, pos_table, w, eps: float, out_dtype):
 
 
 GLA_CHUNK = 64  # tokens per chunk of the chunk-parallel scan; portions of >= 4 chunks take it
-GLA_MIN = 64  # keys up to 128 wide, whose chunks are matrix products (us, token by token / chunks, 16 heads of 64 x 128: 32 tokens
-# 41 / 34, 64 76 / 37, 256 288 / 40; 8 heads of 128 x 128: 32 tokens 95 / 43; and a plan costs one upload per step)
 
 
-def gla_least(dk: int) -> int:
-    """The shortest portion for which :func:`gla_scan` takes a chunk plan, by key size."""
-    return GLA_MIN if dk <= 128 else 4 * GLA_CHUNK
+def gla_plan(cu_host, device, H: int, dk: int, dv: int):
+    """The plan of :func:`gla_scan` for a step's portions (:func:`gla_chunk_plan`), or None where scanning them is faster.  Keys up to 128
+    wide, whose chunks are matrix products (16 heads of 64 x 128, us, scan / chunks: one portion of 40 tokens 50 / 35, of 255 288 / 40, 64 of
+    64 tokens 101 / 126, one of 64 beside 64 of one token 91 / 113); wider ones from 256 tokens on."""
+    if cu_host is None or dk > 128:
+        return gla_chunk_plan(cu_host, device)
+    return gla_chunk_plan(cu_host, device, 1) if _chunks_pay(cu_host, H, dk, dv, (9.7, 0.28, 0.0197), (32.0, 0.02, 1.03e-5)) else None
 
 
 def gla_chunk_plan(cu_host, device, least: int = 4 * GLA_CHUNK):
@@ -317,7 +336,7 @@ def gla_chunk_plan(cu_host, device, least: int = 4 * GLA_CHUNK):
             pcu.append(t)
         base.append(len(pcu) - 1)
     P = len(pcu) - 1
-    both = torch.tensor(pcu + base, dtype=torch.int32).to(device)  # blocking: the host tensor is a temporary
+    both = _upload_ints(pcu + base, device)
     ident = torch.arange(P, dtype=torch.int32, device=device)
     return (both[:P + 1], both[P + 1:], ident, torch.zeros(P, dtype=torch.int32, device=device),
             torch.ones(P, dtype=torch.int32, device=device), P)
@@ -330,11 +349,11 @@ def gla_scan(q, k, v, z, z_bias, tau: float, qscale: float, S, state_slots, cu, 
     (row-strided views allowed), ``z [T, H*dk]`` fp32, ``z_bias`` fp32 ``[H*dk]``.
     Returns fp32 ``[T, H, dv]`` and updates the state pool ``S [slots, H, dk, dv]`` in place at
     ``state_slots[seq]`` (a sequence with ``start == 0`` begins from zeros).  ``cu_host`` (the row offsets on
-    the host) or ``plan`` (:func:`gla_chunk_plan` of them) lets long portions run chunk-parallel."""
+    the host) or ``plan`` (:func:`gla_plan` of them) lets long portions run chunk-parallel."""
     if use_native(q):
         nat = native_hybrid()
         if plan is None and cu_host is not None:
-            plan = gla_chunk_plan(cu_host, q.device, gla_least(q.shape[-1]))
+            plan = gla_plan(cu_host, q.device, *q.shape[1:], v.shape[2])
         if plan is not None:
             return _gla_scan_chunked(nat, q, k, v, z, z_bias, tau, qscale, S, state_slots, start, plan)
         return nat.gla_scan(q, k, v, z, z_bias, tau, qscale, S, state_slots, cu, start, None, True, True)
@@ -698,7 +717,7 @@ def _memory_plan(b, device):
             for lo, hi in zip(b.cu_host[:n], b.cu_host[1:n + 1]):
                 pcu += list(range(lo + MEMORY_CHUNK, hi, MEMORY_CHUNK)) + ([hi] if hi > lo else [])
                 base.append(len(pcu) - 1)
-            both = torch.tensor(pcu + base, dtype=torch.int32).to(device)  # blocking: the host tensor is a temporary
+            both = _upload_ints(pcu + base, device)
             plan = (both[:len(pcu)], both[len(pcu):], len(pcu) - 1)
         b.scratch["memory_plan"] = plan
     return b.scratch["memory_plan"]

@@ -148,3 +148,34 @@ def test_mlstm_decode_rows_of_many_sequences(ns, H, dk, dv, slab):
         assert ((got.double() - num / den[..., None]).abs() <= 2.0 ** -16 * (size + rel[..., None] * (num / den[..., None]).abs()) + 1e-6).all()
         for pool, want in ((S, S1), (n, n1), (m, m1)):
             assert (pool[slots.long()].double() - want).norm() <= 2.0 ** -18 * want.norm()
+
+
+@pytest.mark.parametrize("lens,chunks", [([255], True), ([40], True), ([100] + [1] * 16, True), ([64] + [1] * 64, False), ([40] * 64, False), ([1] * 8, False),
+                                         ([256] + [1] * 64, True)])
+@pytest.mark.parametrize("op", ["mlstm", "gla"])
+def test_short_portions_of_many_sequences_are_scanned(op, lens, chunks):
+    """Which form a step takes, and that both agree there (the same recurrence, in chunks or token by token)."""
+    from llmctl.ops._lib import native_hybrid
+
+    H, dk, dv, nat = 16, 64, 128, native_hybrid()
+    plan = (hops.mlstm_chunk_plan if op == "mlstm" else hops.gla_plan)(_cu(lens), torch.device("cuda"), H, dk, dv)
+    assert (plan is not None) == chunks
+    g = torch.Generator().manual_seed(len(lens))
+    T, ns = sum(lens), len(lens)
+    z, q, k, v = _rows(T, H, dk, dv, torch.bfloat16, g)
+    zd = z.cuda()
+    q, k, v = (zd[:, a:a + H * w].unflatten(1, (H, w)) for a, w in ((0, dk), (H * dk, dk), (2 * H * dk, dv)))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32).cuda()
+    slots, start, cu = i32(list(range(ns))), i32([5] * ns), i32(_cu(lens))
+    S, n, m = (torch.randn(s, generator=g).cuda() for s in ((ns, H, dk, dv), (ns, H, dk), (ns, H)))
+    S2, n2, m2 = S.clone(), n.clone(), m.clone()
+    if op == "mlstm":
+        raw, b_i, b_f = torch.randn(T, 2 * H, generator=g).cuda(), torch.zeros(H).cuda(), torch.full((H,), 2.0).cuda()
+        got = hops.mlstm_scan(q, k, v, raw, b_i, b_f, 15.0, dk ** -0.5, S, n, m, slots, cu, start, cu_host=_cu(lens))
+        want = nat.mlstm_scan(q, k, v, raw, b_i, b_f, 15.0, dk ** -0.5, S2, n2, m2, slots, cu, start, False)
+    else:
+        zl, zb = torch.randn(T, H * dk, generator=g).cuda(), torch.zeros(H * dk).cuda()
+        got = hops.gla_scan(q, k, v, zl, zb, 16.0, dk ** -0.5, S, slots, cu, start, cu_host=_cu(lens))
+        want = nat.gla_scan(q, k, v, zl, zb, 16.0, dk ** -0.5, S2, slots, cu, start, None, True, True)
+    for a, b in ((got, want), (S, S2)):  # fp32 sums of some hundred terms in another order (the mLSTM's quotient may cancel)
+        assert (a - b).norm() <= 1e-4 * b.norm()
