@@ -219,8 +219,9 @@ def _chunks_pay(cu_host, H: int, dk: int, dv: int, scan, chunks) -> bool:
 
 
 def _upload_ints(values, device):
-    """int32 on ``device``.  From pinned memory, which its allocator keeps until the copy is over: the host does not wait for what is queued."""
-    return torch.tensor(values, dtype=torch.int32, pin_memory=True).to(device, non_blocking=True)
+    """int32 on ``device``.  For a GPU from pinned memory, which its allocator keeps until the copy is over: the host does not wait for what is
+    queued."""
+    return torch.tensor(values, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda").to(device, non_blocking=True)
 
 
 def mlstm_chunk_plan(cu_host, device, H: int, dk: int, dv: int):
