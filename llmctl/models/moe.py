@@ -372,7 +372,7 @@ class BiasedSoftmaxMoE(nn.Module):
                 ys = hops.linear(u if fused else act(u), self.w_sdown)
         gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
         down = self.w_down.view(x.shape[1], self.E, self.ff).transpose(0, 1)  # [E, width, ff]
-        if (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1])
+        if (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
                 and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
             out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
                                       self.act, ys, gate)

@@ -448,13 +448,13 @@ MAX_EXPERTS = 128  # the expert kernels take the weights' addresses as arguments
 
 def experts_ok(x, up, down, outputs: int, top: int = 1, w_router=None) -> bool:
     """Whether :func:`routed_experts` takes these operands: bf16 GPU rows and weights, widths in multiples of 8 with rows aligned
-    to 16 bytes, at most 128 router outputs, of which at most 64 are chosen, a contiguous, aligned router.  ``up`` / ``down``: one ``[E,
-    rows, K]`` tensor or a list of ``[rows, K]`` ones."""
+    to 16 bytes, at most 128 router outputs, of which at most 64 are chosen, a contiguous, aligned router, no gradient wanted.  ``up`` /
+    ``down``: one ``[E, rows, K]`` tensor or a list of ``[rows, K]`` ones."""
     if not (use_native(x) and x.dtype == torch.bfloat16 and x.dim() == 2 and outputs <= MAX_EXPERTS and top <= 64
             and (w_router is None or (w_router.is_contiguous() and w_router.data_ptr() % 16 == 0))):
         return False
     ups, downs = ([w] if torch.is_tensor(w) else list(w) for w in (up, down))
-    return (x.shape[1] % 8 == 0 and downs[0].shape[-1] % 8 == 0
+    return (not wants_grad(x, *ups, *downs) and x.shape[1] % 8 == 0 and downs[0].shape[-1] % 8 == 0
             and all(t.dtype == torch.bfloat16 and t.is_cuda and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
                     and all(v % 8 == 0 for v in t.stride()[:-1]) for t in [x] + ups + downs)
             and all(w.stride() == ws[0].stride() for ws in (ups, downs) for w in ws))
