@@ -297,7 +297,7 @@ class InferenceEngine:
         replayed (:mod:`llmctl.serve.decode_graph`).  ``ids_on_device``: the rows' input tokens as a device tensor."""
         n = len(dp["positions"])
         g = None
-        if self._decode_capture and n:
+        if self._decode_capture and n and np.shape(dp["bt"])[1:] == (self.max_blocks_per_seq,):  # (tables of another width: eagerly)
             w = self._weights_key()
             if w != self._weights_seen:
                 self.release_graphs()

@@ -3,6 +3,7 @@ one without, over several replays with eager work in between, sequences that com
 slots and pages), a context that passes a power of two, tokens fed back on the device, weights changed in place or exchanged, shapes
 that are given up or do not record, and other threads at work during a recording."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -144,6 +145,34 @@ def test_shapes_come_and_go(monkeypatch):
         p.step(rows)
     p.check_caches()
     assert p.replays() == 6 and len(p.es[0]._decode_graphs) == 2  # recorded: 4, 3, 2 (4 goes), 4 (3 goes), 1 (4 goes); one more of 2
+    p.close()
+
+
+@pytest.mark.parametrize("width", [5, 20])
+def test_plans_with_block_tables_of_another_width(width):
+    """A caller's own plan may hold just the blocks that are in use, or more columns than the engine's."""
+    p = _Pair("malinex-w128-l4-h4-g2-e4-s1")
+    for n in (40, 45):  # (no context passes a power of two)
+        p.admit(n)
+    for _ in range(4):
+        p.step(2)
+    assert p.replays() == 2
+    got = []
+    for k, e in enumerate(p.es):
+        seqs = [s[k] for s in p.live]
+        for s in seqs:
+            e.scheduler.extend(s, [7])
+            s._decode_slot = int(e.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+        plan = e.decode_plan(seqs)
+        assert plan["bt"].shape[1] == 16 and all(c <= 5 * 16 for c in plan["ctx"])
+        plan["bt"] = np.pad(plan["bt"], ((0, 0), (0, 4)))[:, :width].copy()
+        got.append(e.decode_exec(plan))
+        for s in seqs:
+            e.scheduler.computed(s, 1)
+    _close(got[0], got[1], p.dtype)
+    p.step(2)
+    p.check_caches()
+    assert p.replays() == 3
     p.close()
 
 
