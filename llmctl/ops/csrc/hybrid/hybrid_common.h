@@ -73,7 +73,6 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// Sum over a block of NW waves; every thread gets the result.  ``red`` holds NW floats; two barriers.
 // four neighbouring values (16-byte aligned fp32, 8-byte aligned bf16)
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 ld4(const bf16_t* p) {
@@ -93,6 +92,7 @@ inline bool quads_ok(const T* p, int64_t stride, int64_t W) {
   return W % 4 == 0 && stride % 4 == 0 && reinterpret_cast<uintptr_t>(p) % (4 * sizeof(T)) == 0;
 }
 
+// Sum over a block of NW waves; every thread gets the result.  ``red`` holds NW floats; two barriers.
 template <int NW>
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
