@@ -115,7 +115,8 @@ def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     every data gradient on gemm64 (no W^T copies, ~10 GB less memory for GPT-7B); off = none.  Whole steps, ms, gemm64 / W^T copies:
     tiny model, 256 tokens 1.89 / 2.84; gpt2-125m 1024 tokens 8.31 / 12.24, 8192 13.0 / 13.2; two GPT-7B layers 1024 tokens
     8.02 / 8.69, 8192 25.9 / 26.4, 16384 46.7 / 47.1, 24576 67.0 / 67.1 (a copy costs a pass over the weight, a launch and an event whatever
-    the batch); the full GPT-7B at 24576 tokens 837.7 / 832.0."""
+    the batch).  Beyond the limit nothing is gained: the full GPT-7B, two runs each, 24576 tokens 816.6, 818.0 / 816.5, 817.6, 32768 1073.8,
+    1075.0 / 1071.1, 1071.3 (``profiles/dgrad_routes_full_model.txt``)."""
     out, inn = w.shape
     mode = knobs().dgrad64
     if mode == "off" or (not fused and (mode == "fused" or (mode == "auto" and tokens > DGRAD64_TOKENS))):

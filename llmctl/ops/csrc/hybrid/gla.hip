@@ -1,7 +1,7 @@
 // Gated linear attention: per (sequence, head) a memory S [dk, dv] (fp32) whose key rows decay by a
 // data-dependent factor, S_t = diag(a_t) S_(t-1) + k_t v_t^T, read out as o_t = S_t^T q_t.
 //
-// (Portions from 64 tokens with dk <= 128: gla_chunk.hip for the two passes over the chunks.)
+// (Portions in chunks with dk <= 128: gla_chunk.hip for the two passes over the chunks; which portions: gla_plan in llmctl/ops/hybrid.py.)
 //   gla_scan           token by token; one wave per (sequence, head, 64 value columns): a lane owns one
 //                      value column and keeps its dk state entries in registers, so update and read-out are
 //                      lane-local; a_t, k_t, q_t reach all lanes through a wave-private LDS line.  The decay

@@ -3,7 +3,7 @@
 //   i = cap tanh((zi + bi) / cap),   f = logsigmoid(cap tanh((zf + bf) / cap)):
 //   m' = max(f + m, i);  S = e^(f + m - m') S + e^(i - m') k v^T;  n likewise with k alone;
 //   o = S^T q / (max(|n . q|, e^(-m')) + 1e-6),  q already scaled.
-// (Long portions with dk <= 128: mlstm_chunk.hip.)  A pre-pass turns the gate pre-activations into i and f for all tokens at once.  The scan has two forms:
+// (Portions in chunks, dk <= 128: mlstm_chunk.hip; which ones: mlstm_chunk_plan in llmctl/ops/hybrid.py.)  A pre-pass turns the gate pre-activations into i and f for all tokens at once.  The scan has two forms:
 //   * dk <= 128: one wave per (sequence, head, tile of 64 value columns), a lane owns one column of S
 //     (all dk rows in registers); k and q are spread over the lanes and reach the column update as
 //     scalar operands (v_readlane), n is spread over the lanes and n . q is one wave reduction: no LDS

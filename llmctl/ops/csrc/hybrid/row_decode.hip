@@ -20,6 +20,8 @@
 //   576 / 512, 1                                         12.4 (21.5)   18.0 (55.2)   35.1 (97.3)   87.5 (259, 3.5 TB/s now)
 //   256 / 256, 2                                          8.3 (13.7)   13.7 (33.5)   33.2 (60.9)   106 (156, 5.1 TB/s now)
 //   128 / 128, 4                                          7.1 (9.0)    11.9 (22.0)   30.6 (48.3)   99.6 (146, 5.4 TB/s now)
+// (The form for keys of 257 to 576 columns fills its 256 registers and spills one vector and eleven scalar registers, 8 bytes of scratch a lane; the
+// first row was measured with that.)
 #include "attn_common.h"
 #include "hybrid_common.h"
 

@@ -311,7 +311,7 @@ def embed_rmsnorm_f32(ids, pos, table, pos_table, w, eps: float, out_dtype):
     return ref.embed_rmsnorm_f32(ids, pos, table, pos_table, w, eps, out_dtype)
 
 
-GLA_CHUNK = 64  # tokens per chunk of the chunk-parallel scan; portions of >= 4 chunks take it
+GLA_CHUNK = 64  # tokens per chunk of the chunk-parallel scan; which portions take it: gla_plan, gla_chunk_plan
 
 
 def gla_plan(cu_host, device, H: int, dk: int, dv: int):
