@@ -138,4 +138,9 @@ struct RowAttnOpts {
   int64_t keep_first = 0;             // the window does not hide the keys at positions below this
 };
 
+// How a launch over decode rows is cut: its workgroups before a row's keys are split, the splits, and the 64-key steps of a row at most
+struct DecodeCut {
+  int64_t groups, nsplit, steps;
+};
+
 }  // namespace llmctl_hybrid

@@ -311,7 +311,10 @@ static bool mfma_cap_ok(const RowAttnOpts& x, int64_t R) {
 }
 void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu, const at::Tensor& ctx,
                       int64_t window, const float* sink, double scale, int64_t rk, int64_t max_q, at::Tensor& out, const RowAttnOpts& x);
-// one query row per sequence (row_decode.hip)
+// one query row per sequence: 16 heads of a kv group per workgroup (row_decode.hip), or up to 128 (latent_attn_mfma.hip)
+bool decode_tiles_pay(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x, int64_t most);
+void latent_attn_mfma_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
+                             double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x);
 void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
                 double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x);
 
@@ -502,7 +505,8 @@ at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, con
   at::Tensor out = at::empty({ns, H, rk}, qa.options());
   if (ns == 0) return out;
   if (mfma && mfma_cap_ok(x, R) && (x.dist_a == nullptr || x.sig_bias != nullptr) && latent_attn_mfma_ok(qa, rk, cache.size(2) / groups, koff, x.ofreq != nullptr || x.sig_bias != nullptr)) {
-    row_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
+    if (decode_tiles_pay(ns, H, R, rk, window, x, bt.size(1) * cache.size(1))) latent_attn_mfma_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
+    else row_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
     return out;
   }
   HYB_CHECK(rk <= 512, "generic decode kernel: value width <= 512");

@@ -1,10 +1,11 @@
-// Latent attention on the matrix cores (bf16; MFMA 32x32x16) for prompt portions; decode rows: row_decode.hip.
+// Latent attention on the matrix cores (bf16; MFMA 32x32x16) for prompt portions, and for decode rows whose many heads share their
+// keys (decode_tiles_pay); other decode rows: row_decode.hip.
 //
 // The cache row [latent | rotary key] of width R is key and, in its first ``rank`` entries, value; the
 // queries come in the same layout (see latent_attn.hip).  This is the flash-attention forward of the
 // framework's paged prefill kernel re-cut for that layout:
 //   * a workgroup (4 waves) owns 128 query rows = TB tokens x HB heads of one sequence (HB = 1 for
-//     long portions, = the head count for short portions, where the heads of a token
+//     long portions, = the head count for decode rows and short portions, where the heads of a token
 //     fill the tile and share every key row);
 //   * tiles of 64 keys, gathered through the block table into LDS once per workgroup: a "row image"
 //     of all of R (in column blocks of 128) for S^T = K Q^T, and a "transposed-read image" of the
@@ -45,16 +46,22 @@ struct LArgs {
   int keep;                     // the window spares the keys at positions below this
   float scale_log2;
   float cap_log2, cap_inv2;     // CAP forms: x (log2 domain) = cap_log2 * tanh(s * scale); cap_inv2 = 2 log2(e) scale / cap
+  // SPLIT forms: the key range of a decode row is spread over blockIdx.x (few sequences would otherwise leave the chip idle): each split
+  // writes its unnormalised fp32 output and (running maximum, denominator) here, and row_merge joins them
+  int nsplit;
+  float* ws_o;   // [rows, nsplit, rk]
+  float* ws_ml;  // [rows, nsplit, 2]
 };
 
 // ROT: the output's neighbour pairs are turned back by the query's position (a.ofreq); a template flag
 // so that the forms without it keep their register budget.  SIG: the weights are sigmoids of the scores
 // (after the distance penalty), not a softmax: no running maximum, no rescale, no denominator (l = 1).  CAP: the scaled score
-// s becomes cap tanh(s / cap) before masks and softmax (tanh y = 1 - 2 / (1 + e^(2y))).
+// s becomes cap tanh(s / cap) before masks and softmax (tanh y = 1 - 2 / (1 + e^(2y))).  SPLIT: decode rows, one query per sequence (no
+// a.cu), nsplit workgroups for a row's keys.
 // Keys and values up to 128 wide: two workgroups per CU (64.5 KB of images each; held to 256 registers, one's softmax runs beside the
 // other's products).  16 heads over 4 kv groups, portions of 2048 and 1331 tokens: 156 us at one per CU (200 + 96 registers),
 // 100 so.  Wider keys stay at one: 192-wide keys took 108 us against 99, with one set of images instead of two 107.
-template <int NCB, int NDB, bool ROT, bool SIG = false, bool CAP = false>
+template <int NCB, int NDB, bool ROT, bool SIG = false, bool CAP = false, bool SPLIT = false>
 __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
   constexpr int NKS = NCB * 8;
   constexpr int NTB = (NDB + 3) / 4;
@@ -71,11 +78,12 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   const int hg = blockIdx.z / a.nvt, v0 = (blockIdx.z % a.nvt) * (NDB * 32);
   const int P = a.H / a.G;                       // query heads per kv group
   const int grp = hg / a.hpg, hsub = (hg % a.hpg) * a.HB;  // this workgroup's kv group, its first head inside it
-  const int q_begin = a.cu[n];
-  const int qlen = a.cu[n + 1] - q_begin;
+  const int q_begin = SPLIT ? n : a.cu[n];
+  const int qlen = SPLIT ? 1 : a.cu[n + 1] - q_begin;
   const int HB = a.HB, TB = 128 / HB;
   // prompt portions: the last query blocks of a sequence see the most keys; they are dispatched first
-  const int tok0 = (int)(gridDim.x - 1 - blockIdx.x) * TB;
+  const int split = SPLIT ? blockIdx.x : 0;
+  const int tok0 = SPLIT ? 0 : (int)(gridDim.x - 1 - blockIdx.x) * TB;
   if (tok0 >= qlen) return;
   const int ctx = a.ctx[n];
   const int pos0 = ctx - qlen;
@@ -103,7 +111,7 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
   float m_i = -INFINITY, l_i = 0.f;
-  if (a.sink != nullptr) {  // the sink: one unit of mass at its own logit
+  if (a.sink != nullptr && split == 0) {  // the sink: one unit of mass at its own logit, counted by the first split
     m_i = a.sink[headc] * kLog2e;
     l_i = 1.0f;
   }
@@ -111,7 +119,7 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   float pen_a = 0.f, pen_b = 0.f, sig_b2 = 0.f;
   if constexpr (SIG) {
     m_i = 0.f;
-    l_i = 1.f;
+    l_i = split == 0 ? 1.f : 0.f;
     if (a.dist_a != nullptr) pen_a = a.dist_a[headc], pen_b = a.dist_b[headc];
     sig_b2 = a.sig_bias[headc] * kLog2e;
   }
@@ -126,7 +134,12 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   const int kept0 = ((first_pos / a.chunk) * a.chunk) / LKB;
   const int n_kept = a.keep > 0 ? max(min((a.keep + LKB - 1) / LKB, t_first) - kept0, 0) : 0;
   auto tile_of = [&](int i) { return i < n_kept ? kept0 + i : t_first + i - n_kept; };
-  const int t_lo = 0, t_hi = n_kept + t_end - t_first;
+  int t_lo = 0, t_hi = n_kept + t_end - t_first;
+  if constexpr (SPLIT) {
+    const int per = (t_hi + a.nsplit - 1) / a.nsplit;
+    t_lo = split * per;
+    t_hi = min(t_hi, t_lo + per);
+  }
   // this wave's rows: positions [w_first, w_last]
   const int w_first = pos0 + min(tok0 + (wave * 32) / HB, qlen - 1);
   const int w_last = pos0 + min(tok0 + (wave * 32 + 31) / HB, qlen - 1);
@@ -304,7 +317,21 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
         }
   }
 
-  if (valid) {
+  if (SPLIT && valid && a.nsplit > 1) {
+    const long rowi = (long)n * a.H + my_head;
+    float* Wp = a.ws_o + (rowi * a.nsplit + split) * a.rk;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int col = v0 + d * 32 + 8 * g + 4 * hh;
+        if (col < a.rk) *reinterpret_cast<float4*>(Wp + col) = make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
+      }
+    if (v0 == 0 && hh == 0) {
+      a.ws_ml[(rowi * a.nsplit + split) * 2] = m_i;
+      a.ws_ml[(rowi * a.nsplit + split) * 2 + 1] = l_i;
+    }
+  } else if (valid) {
     const float inv = 1.f / l_i;
     unsigned short* Op = a.out + ((long)(q_begin + my_tok) * a.H + my_head) * a.rk;
 #pragma unroll
@@ -333,7 +360,7 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   }
 }
 
-template <int NCB, bool ROT, bool SIG = false, bool CAP = false>
+template <int NCB, bool SPLIT, bool ROT, bool SIG = false, bool CAP = false>
 void launch_ncb(const LArgs& a, int ndb, dim3 grid, hipStream_t st) {
   auto go = [&](auto kern, int NDBv) {
     const size_t one = (size_t)(NCB + (NDBv + 3) / 4) * LIMG;
@@ -341,9 +368,62 @@ void launch_ncb(const LArgs& a, int ndb, dim3 grid, hipStream_t st) {
     HYB_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess, "LDS size");
     kern<<<grid, 256, lds, st>>>(a);
   };
-  if (ndb == 2) go(latent_attn_mfma_kernel<NCB, 2, ROT, SIG, CAP>, 2);
-  else if (ndb == 4) go(latent_attn_mfma_kernel<NCB, 4, ROT, SIG, CAP>, 4);
-  else go(latent_attn_mfma_kernel<NCB, 8, ROT, SIG, CAP>, 8);
+  if (ndb == 2) go(latent_attn_mfma_kernel<NCB, 2, ROT, SIG, CAP, SPLIT>, 2);
+  else if (ndb == 4) go(latent_attn_mfma_kernel<NCB, 4, ROT, SIG, CAP, SPLIT>, 4);
+  else go(latent_attn_mfma_kernel<NCB, 8, ROT, SIG, CAP, SPLIT>, 8);
+}
+
+template <bool SPLIT>
+void launch_form(const LArgs& a, int ncb, int ndb, dim3 grid, const RowAttnOpts& x) {
+  hipStream_t st = cur_stream();
+  if (x.softcap > 0.0) {  // built for keys up to 256 wide, plain softmax form (the caller checks)
+    HYB_CHECK(x.hscale == nullptr && ncb <= 2, "capped scores: no per-head factor, keys up to 256 wide");
+    if (ncb == 1) launch_ncb<1, SPLIT, false, false, true>(a, ndb, grid, st);
+    else launch_ncb<2, SPLIT, false, false, true>(a, ndb, grid, st);
+  } else if (x.sig_bias != nullptr) {  // built for keys up to 256 wide (latent_attn_mfma_ok)
+    if (ncb == 1) launch_ncb<1, SPLIT, false, true>(a, ndb, grid, st);
+    else launch_ncb<2, SPLIT, false, true>(a, ndb, grid, st);
+  } else if (x.ofreq != nullptr) {
+    if (ncb == 1) launch_ncb<1, SPLIT, true>(a, ndb, grid, st);
+    else launch_ncb<2, SPLIT, true>(a, ndb, grid, st);
+  } else {
+    switch (ncb) {
+      case 1: launch_ncb<1, SPLIT, false>(a, ndb, grid, st); break;
+      case 2: launch_ncb<2, SPLIT, false>(a, ndb, grid, st); break;
+      case 3: launch_ncb<3, SPLIT, false>(a, ndb, grid, st); break;
+      case 4: launch_ncb<4, SPLIT, false>(a, ndb, grid, st); break;
+      default: launch_ncb<5, SPLIT, false>(a, ndb, grid, st); break;
+    }
+  }
+}
+
+// The cut of a call: column blocks of the keys and value tiles, heads and tokens of a workgroup's 128 rows.
+struct Cut {
+  int ncb, ndb, nvt, HB, hpg;
+  Cut(int64_t R, int64_t rk, int64_t P, bool heads) {
+    ncb = (int)((R + 127) / 128);
+    ndb = rk <= 64 ? 2 : (rk <= 128 ? 4 : 8);
+    nvt = (int)((rk + ndb * 32 - 1) / (ndb * 32));
+    HB = 1;
+    while (heads && HB < P && HB < 128) HB *= 2;
+    hpg = (int)((P + HB - 1) / HB);
+  }
+};
+
+LArgs make_args(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const int* cu, const at::Tensor& ctx, int64_t window, const float* sink,
+                double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x, const Cut& c) {
+  LArgs a = {};
+  a.qa = reinterpret_cast<const unsigned short*>(qa.data_ptr()), a.cache = reinterpret_cast<const unsigned short*>(cache.data_ptr());
+  a.out = reinterpret_cast<unsigned short*>(out.data_ptr());
+  a.bt = bt.data_ptr<int>(), a.cu = cu, a.ctx = ctx.data_ptr<int>();
+  a.sink = sink, a.hscale = x.hscale, a.ofreq = x.ofreq, a.dist_a = x.dist_a, a.dist_b = x.dist_b, a.sig_bias = x.sig_bias;
+  a.H = (int)qa.size(1), a.R = (int)qa.size(2), a.rk = (int)rk, a.bs = (int)cache.size(1), a.maxb = (int)bt.size(1), a.window = (int)window;
+  a.HB = c.HB, a.nvt = c.nvt, a.G = (int)x.groups, a.rs = (int)(cache.size(2) / x.groups), a.koff = (int)x.koff, a.chunk = (int)x.chunk, a.hpg = c.hpg;
+  a.keep = (int)x.keep_first;
+  a.scale_log2 = (float)(scale * 1.4426950408889634), a.cap_log2 = (float)(x.softcap * 1.4426950408889634);
+  a.cap_inv2 = x.softcap > 0.0 ? (float)(2.0 * 1.4426950408889634 * scale / x.softcap) : 0.f;
+  a.nsplit = 1;
+  return a;
 }
 }  // namespace
 
@@ -357,46 +437,45 @@ bool latent_attn_mfma_ok(const at::Tensor& qa, int64_t rk, int64_t rs, int64_t k
 // ``x`` carries the optional parts (see RowAttnOpts).
 void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu, const at::Tensor& ctx,
                       int64_t window, const float* sink, double scale, int64_t rk, int64_t max_q, at::Tensor& out, const RowAttnOpts& x) {
-  const int64_t H = qa.size(1), R = qa.size(2), ns = ctx.numel();
-  const int64_t G = x.groups, P = H / G, rs = cache.size(2) / G;
-  const int ncb = (int)((R + 127) / 128);
-  const int ndb = rk <= 64 ? 2 : (rk <= 128 ? 4 : 8);
-  const int nvt = (int)((rk + ndb * 32 - 1) / (ndb * 32));
-  int HB = 1;
-  if (max_q < 64) {
-    while (HB < P && HB < 128) HB *= 2;
+  const int64_t ns = ctx.numel();
+  const Cut c(qa.size(2), rk, qa.size(1) / x.groups, max_q < 64);
+  const int TB = 128 / c.HB, z = (int)x.groups * c.hpg * c.nvt;
+  HYB_CHECK(ns <= 65535 && z <= 65535, "grid too large");
+  const LArgs a = make_args(qa, cache, bt, cu.data_ptr<int>(), ctx, window, sink, scale, rk, out, x, c);
+  launch_form<false>(a, c.ncb, c.ndb, dim3((unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)z), x);
+}
+
+void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const float* ofreq);  // row_decode.hip
+
+// The decode form's cut: the visible key tiles are split over workgroups until the launch has a few hundred of them.  ``images``: 128-column
+// images of a tile's keys and values in LDS.
+DecodeCut tile_cut(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x, int* images) {
+  const Cut c(R, rk, H / x.groups, true);
+  *images = c.ncb + (c.ndb + 3) / 4;
+  const int64_t span = std::min<int64_t>(std::min<int64_t>(window, x.chunk), x.max_ctx > 0 ? x.max_ctx : (int64_t)1 << 30);
+  DecodeCut d = {ns * x.groups * c.hpg * c.nvt, 1, std::min<int64_t>((span + LKB - 1) / LKB + 1 + (x.keep_first + LKB - 1) / LKB, 1 << 20)};
+  while (d.nsplit < d.steps && d.nsplit < 32 && d.groups * d.nsplit < 512) d.nsplit *= 2;
+  return d;
+}
+
+// Decode rows: up to 128 heads of a kv group in one tile.
+void latent_attn_mfma_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
+                             double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x) {
+  const int64_t H = qa.size(1), ns = ctx.numel();
+  const Cut c(qa.size(2), rk, H / x.groups, true);
+  const int z = (int)x.groups * c.hpg * c.nvt;
+  HYB_CHECK(ns <= 65535 && z <= 65535, "grid too large");
+  LArgs a = make_args(qa, cache, bt, nullptr, ctx, window, sink, scale, rk, out, x, c);
+  int images;
+  a.nsplit = (int)tile_cut(ns, H, qa.size(2), rk, window, x, &images).nsplit;
+  at::Tensor ws_o, ws_ml;
+  if (a.nsplit > 1) {
+    ws_o = at::empty({ns * H, a.nsplit, rk}, qa.options().dtype(at::kFloat));
+    ws_ml = at::empty({ns * H, a.nsplit, 2}, qa.options().dtype(at::kFloat));
+    a.ws_o = ws_o.data_ptr<float>(), a.ws_ml = ws_ml.data_ptr<float>();
   }
-  const int TB = 128 / HB;
-  const int hpg = (int)((P + HB - 1) / HB);  // head tiles per kv group
-  const int hgroups = (int)G * hpg;
-  HYB_CHECK(ns <= 65535 && hgroups * nvt <= 65535, "grid too large");
-  LArgs a{reinterpret_cast<const unsigned short*>(qa.data_ptr()), reinterpret_cast<const unsigned short*>(cache.data_ptr()),
-          reinterpret_cast<unsigned short*>(out.data_ptr()), bt.data_ptr<int>(), cu.data_ptr<int>(), ctx.data_ptr<int>(),
-          sink, x.hscale, x.ofreq, x.dist_a, x.dist_b, x.sig_bias, (int)H, (int)R, (int)rk, (int)cache.size(1), (int)bt.size(1), (int)window, HB, nvt,
-          (int)G, (int)rs, (int)x.koff, (int)x.chunk, hpg, (int)x.keep_first,
-          (float)(scale * 1.4426950408889634), (float)(x.softcap * 1.4426950408889634),
-          x.softcap > 0.0 ? (float)(2.0 * 1.4426950408889634 * scale / x.softcap) : 0.f};
-  dim3 grid((unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)(hgroups * nvt));
-  hipStream_t st = cur_stream();
-  if (x.softcap > 0.0) {  // built for keys up to 256 wide, plain softmax form (the caller checks)
-    HYB_CHECK(x.hscale == nullptr && ncb <= 2, "capped scores: no per-head factor, keys up to 256 wide");
-    if (ncb == 1) launch_ncb<1, false, false, true>(a, ndb, grid, st);
-    else launch_ncb<2, false, false, true>(a, ndb, grid, st);
-  } else if (x.sig_bias != nullptr) {  // built for keys up to 256 wide (latent_attn_mfma_ok)
-    if (ncb == 1) launch_ncb<1, false, true>(a, ndb, grid, st);
-    else launch_ncb<2, false, true>(a, ndb, grid, st);
-  } else if (x.ofreq != nullptr) {
-    if (ncb == 1) launch_ncb<1, true>(a, ndb, grid, st);
-    else launch_ncb<2, true>(a, ndb, grid, st);
-  } else {
-    switch (ncb) {
-      case 1: launch_ncb<1, false>(a, ndb, grid, st); break;
-      case 2: launch_ncb<2, false>(a, ndb, grid, st); break;
-      case 3: launch_ncb<3, false>(a, ndb, grid, st); break;
-      case 4: launch_ncb<4, false>(a, ndb, grid, st); break;
-      default: launch_ncb<5, false>(a, ndb, grid, st); break;
-    }
-  }
+  launch_form<true>(a, c.ncb, c.ndb, dim3((unsigned)a.nsplit, (unsigned)ns, (unsigned)z), x);
+  if (a.nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x.ofreq);
 }
 
 }  // namespace llmctl_hybrid

@@ -284,21 +284,60 @@ __global__ __launch_bounds__(128) void row_merge_kernel(const float* __restrict_
 }
 }  // namespace
 
+// Joins the splits of decode rows: ws_o [ns H, nsplit, rk], ws_ml [ns H, nsplit, 2] -> out [ns, H, rk]; at most 64 splits
+void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const float* ofreq) {
+  row_merge_kernel<<<dim3((unsigned)ws_o.size(0)), 128, 0, cur_stream()>>>(ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(),
+                                                                         reinterpret_cast<unsigned short*>(out.data_ptr()), (int)ws_o.size(1), (int)ws_o.size(2), ofreq,
+                                                                         ctx.data_ptr<int>(), (int)out.size(1));
+}
+
+namespace {
+int value_tiles(int64_t R, int64_t rk) { return R <= 128 && rk <= 128 ? 8 : (R <= 256 && rk <= 256 ? 16 : 32); }
+
+// The key steps go to further workgroups until the launch has two per CU: a CU draws about 30 GB/s of a chain of dependent loads,
+// and the merge of 64 splits costs 2 to 3 us (unrolled: its loads run together).
+DecodeCut row_cut(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x) {
+  const int64_t nv = value_tiles(R, rk), span = std::min<int64_t>(std::min<int64_t>(window, x.chunk), x.max_ctx > 0 ? x.max_ctx : (int64_t)1 << 30) + x.keep_first;
+  DecodeCut d = {ns * x.groups * ((H / x.groups + 15) / 16) * ((rk + nv * 16 - 1) / (nv * 16)), 1, (span + KEYS - 1) / KEYS};
+  while (d.nsplit < d.steps && d.nsplit < 64 && d.groups * d.nsplit < 512) d.nsplit *= 2;
+  return d;
+}
+}  // namespace
+
+DecodeCut tile_cut(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x, int* images);  // latent_attn_mfma.hip
+
+// Are decode rows faster in tiles of up to 128 heads (latent_attn_mfma_decode) than 16 heads at a time?  More than 32 heads of a kv group read each
+// key row three times and more here, which costs more than the tiles' idle rows and longer chain once there are enough keys.  ``most``: keys that a row's block table holds.
+// us, here / in tiles, one kv group, 128 heads: 576 / 512 wide, 16 rows x 1000 39 / 59, x 4000 101 / 100, x 32000 735 / 527, 64 x 4000 372 / 289, 256 x 500
+// 214 / 152; 128 / 128 wide, 16 x 4000 36 / 21, 64 x 8000 216 / 66; 320 / 256 wide, 64 x 500 49 / 54, 64 x 8000 576 / 199.  64 heads: 576 / 512 64 x 8000 394 / 489, 256 /
+// 256 64 x 8000 181 / 145.  Both costs are estimated, us = launches + steps in all (at the rate of a full chip) + the steps of one workgroup + the merge, fitted to
+// 896 calls each (1 to 256 rows of 128 to 128000 keys, 40 to 256 heads of 64 to 640 wide keys); the choice is 0.7 % off the faster form on average.
+bool decode_tiles_pay(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x, int64_t most) {
+  if (H / x.groups <= 32) return false;
+  int images;
+  const DecodeCut r = row_cut(ns, H, R, rk, window, x), t = tile_cut(ns, H, R, rk, window, x, &images);
+  const int64_t steps = std::min<int64_t>(r.steps, (most + KEYS - 1) / KEYS);
+  const double merge = 2e-6 * (double)(ns * H * rk);  // per split
+  const int nv = value_tiles(R, rk);
+  double row = nv == 8 ? 7.0 : (nv == 16 ? 9.5 : 13.0);
+  row += (nv == 8 ? 0.93 : (nv == 16 ? 2.4 : (R <= 576 ? 3.2 + 0.005 * (double)R : 11.0))) * (double)(r.groups * steps) / 512.0;
+  row += (nv == 8 ? 0.65 : 0.0) * (double)((steps + r.nsplit - 1) / r.nsplit) + (r.nsplit > 1 ? merge * (double)r.nsplit : 0.0);
+  static const double all[6] = {0.42, 1.5, 2.3, 3.1, 4.1, 5.4}, chain[6] = {1.75, 2.1, 3.2, 3.6, 3.6, 4.2};  // by images, 2 to 7
+  const int i = std::min(std::max(images, 2), 7) - 2;
+  const double tile = 5.5 + 1.7 * images + all[i] * (double)(t.groups * steps) / 256.0 + chain[i] * (double)((steps + t.nsplit - 1) / t.nsplit) +
+                      (t.nsplit > 1 ? merge * (double)t.nsplit : 0.0);
+  return row > tile;
+}
+
 // Keys up to 640 wide; keys, values, sub-rows and the key offset in multiples of 8 (latent_attn_mfma_ok).
 void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
                 double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x) {
   const int64_t ns = qa.size(0), H = qa.size(1), R = qa.size(2), G = x.groups, P = H / G, rs = cache.size(2) / G;
   const int htiles = (int)((P + 15) / 16);
-  const int nv = R <= 128 && rk <= 128 ? 8 : (R <= 256 && rk <= 256 ? 16 : 32);
+  const int nv = value_tiles(R, rk);
   const int nvt = (int)((rk + nv * 16 - 1) / (nv * 16));
   HYB_CHECK(ns <= 65535 && G * htiles * nvt <= 65535, "grid too large");
-  // the key steps go to further workgroups until the launch has two per CU: a CU draws about 30 GB/s of a chain of dependent loads,
-  // and the merge of 64 splits costs 2 to 3 us (unrolled: its loads run together)
-  const int64_t span = std::min<int64_t>(std::min<int64_t>(window, x.chunk), x.max_ctx > 0 ? x.max_ctx : (int64_t)1 << 30) + x.keep_first;
-  const int64_t steps = (span + KEYS - 1) / KEYS;
-  const int64_t blocks = ns * G * htiles * nvt;
-  int nsplit = 1;
-  while (nsplit < steps && nsplit < 64 && blocks * nsplit < 512) nsplit *= 2;
+  const int nsplit = (int)row_cut(ns, H, R, rk, window, x).nsplit;
   at::Tensor ws_o, ws_ml;
   if (nsplit > 1) {
     ws_o = at::empty({ns * H, nsplit, rk}, qa.options().dtype(at::kFloat));
@@ -325,9 +364,7 @@ void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor&
   else if (nv == 16) go(row_decode_kernel<8, 16>, 16);
   else if (R <= 576) go(row_decode_kernel<18, 32>, 32);
   else go(row_decode_kernel<20, 32>, 32);
-  if (nsplit > 1)
-    row_merge_kernel<<<dim3((unsigned)(ns * H)), 128, 0, st>>>(ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(), reinterpret_cast<unsigned short*>(out.data_ptr()),
-                                                              nsplit, (int)rk, x.ofreq, ctx.data_ptr<int>(), (int)H);
+  if (nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x.ofreq);
 }
 
 }  // namespace llmctl_hybrid

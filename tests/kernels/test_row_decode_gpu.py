@@ -107,3 +107,73 @@ def test_empty_splits_and_long_context():
     want = _plain(qa, cache, bt, ctx, NO, None, 0.09, 128, 1, 0, NO, None, None, None, None, None, 0.0, 0)
     got = hops.latent_attention_decode(qa.cuda(), cache.cuda(), bt.cuda(), ctx.cuda(), NO, None, 0.09, 128, max_ctx=5000).double().cpu()
     assert ((got - want).abs() <= 2.0 ** -7 * want.abs().amax(-1, keepdim=True).clamp(min=1.0)).all()
+
+
+def _plain_rows(qa, cache, bt, ctx, window, sink, scale, rk, groups, koff, chunk, hscale, ofreq, sig_bias, dist_a, dist_b, softcap, keep):
+    """``_plain`` with a row's heads at once, float64 on the operands' device."""
+    ns, H, R = qa.shape
+    P, rs = H // groups, cache.shape[2] // groups
+    out = torch.empty(ns, H, rk, dtype=torch.float64, device=qa.device)
+    up = lambda t: None if t is None else t.double()[:, None]
+    sink, hscale, sig_bias, dist_a, dist_b = map(up, (sink, hscale, sig_bias, dist_a, dist_b))
+    for n in range(ns):
+        c = int(ctx[n])
+        rows = cache[bt[n, :(c + cache.shape[1] - 1) // cache.shape[1]].long()].reshape(-1, groups, rs)[:c].double()
+        j, pos = torch.arange(c, device=qa.device), c - 1
+        seen = (j >= (pos // chunk) * chunk) & ((pos - j < window) | (j < keep))
+        k, v = rows[:, :, koff:koff + R].permute(1, 2, 0).contiguous(), rows[:, :, :rk].transpose(0, 1).contiguous()
+        s = torch.bmm(qa[n].double().view(groups, P, R), k).view(H, c) * scale * (1.0 if hscale is None else hscale)
+        if softcap:
+            s = softcap * torch.tanh(s / softcap)
+        if sig_bias is not None:
+            w = torch.sigmoid(s - dist_a * torch.log1p(dist_b * (pos - j).double()) + sig_bias) * seen
+        else:
+            s = s.masked_fill(~seen, float("-inf"))
+            top = s.amax(1, keepdim=True) if sink is None else torch.maximum(s.amax(1, keepdim=True), sink)
+            e = torch.exp(s - top)
+            w = e / (e.sum(1, keepdim=True) + (0 if sink is None else torch.exp(sink - top)))
+        o = torch.bmm(w.view(groups, P, c), v).view(H, rk)
+        if ofreq is not None:
+            a = pos * ofreq.double()
+            u, t = o[:, 0::2].clone(), o[:, 1::2].clone()
+            o[:, 0::2], o[:, 1::2] = u * a.cos() + t * a.sin(), t * a.cos() - u * a.sin()
+        out[n] = o
+    return out
+
+
+@pytest.mark.parametrize("H,R,rk,groups,koff,rs,bs,ns", [
+    (128, 64, 64, 1, 0, 64, 16, 260), (72, 136, 64, 2, 72, 208, 16, 290), (130, 40, 24, 1, 0, 40, 8, 200), (96, 320, 256, 1, 0, 320, 16, 70),
+    (128, 576, 512, 1, 0, 576, 64, 40), (40, 640, 600, 1, 0, 640, 12, 90)])
+@pytest.mark.parametrize("form", ["plain", "sink", "window", "keep", "scale", "cap", "turn", "sigmoid"])
+def test_many_heads_of_a_group(H, R, rk, groups, koff, rs, bs, ns, form):
+    """Many heads over the same keys in many rows, at contexts around the edges of a tile and over splits, some of them empty: sizes that run in
+    tiles of up to 128 heads (``decode_tiles_pay``), and the same rows few at a time, which do not."""
+    if form in ("cap", "turn", "sigmoid") and R > 256:
+        pytest.skip("keys this wide take these options in the generic kernel")
+    g = torch.Generator().manual_seed(H * R + rk)
+    qa, cache, bt, ctx = (t.cuda() for t in _case(H, R, rk, groups, koff, rs, [EDGES[i % len(EDGES)] + 64 * (i // 64) for i in range(ns)], bs, seed=R))
+    bt = torch.nn.functional.pad(bt, (0, 8192 // bs))  # room for longer contexts
+    opt = dict(window=NO, sink=None, chunk=NO, hscale=None, ofreq=None, sig_bias=None, dist_a=None, dist_b=None, softcap=0.0, keep=0)
+    rnd = lambda n: torch.rand(n, generator=g).cuda()
+    if form in ("sink", "turn"):
+        opt["sink"] = torch.randn(H, generator=g).cuda()
+    if form == "window":
+        opt.update(window=130, chunk=192)
+    elif form == "keep":
+        opt.update(window=100, keep=70)
+    elif form == "scale":
+        opt["hscale"] = rnd(H) + 0.5
+    elif form == "cap":
+        opt["softcap"] = 2.0
+    elif form == "turn":
+        opt["ofreq"] = rnd(rk // 2) * 0.1
+    elif form == "sigmoid":
+        opt.update(sig_bias=-4 * rnd(H), dist_a=rnd(H), dist_b=rnd(H))
+    o, scale = opt, R ** -0.5
+    want = _plain_rows(qa, cache, bt, ctx, o["window"], o["sink"], scale, rk, groups, koff, o["chunk"], o["hscale"], o["ofreq"], o["sig_bias"], o["dist_a"],
+                       o["dist_b"], o["softcap"], o["keep"])
+    run = lambda q, t, c, m: hops.latent_attention_decode(q, cache, t, c, o["window"], o["sink"], scale, rk, True, groups, koff, o["chunk"], o["hscale"], o["ofreq"], m,
+                                                          o["sig_bias"], o["dist_a"], o["dist_b"], o["softcap"], o["keep"]).double()
+    size = want.abs().amax(-1, keepdim=True).clamp(min=1.0)  # (the bound: see above)
+    for got in (run(qa, bt, ctx, 0), run(qa, bt, ctx, int(ctx.max())), torch.cat([run(qa[i:i + 3], bt[i:i + 3], ctx[i:i + 3], int(ctx.max())) for i in range(0, ns, 3)])):
+        assert ((got - want).abs() <= 2.0 ** -7 * size).all(), ((got - want).abs() / size).amax((1, 2))
