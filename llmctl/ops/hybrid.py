@@ -204,15 +204,15 @@ def sigmoid_gate_mul(o, g):
 MLSTM_CHUNK = 64  # tokens per chunk of the chunked form
 
 
-def _chunks_pay(cu_host, H: int, dk: int, dv: int, scan, chunks) -> bool:
+def _chunks_pay(cu_host, H: int, dk: int, dv: int, scan, chunks, least: int = 16) -> bool:
     """Are a step's portions faster in chunks of 64 tokens than scanned token by token?  A scan lasts as long as its longest portion (L
     tokens), whatever else runs beside it; every chunk, a one-token portion's too, costs its workgroups and passes over a state.  ``scan``:
     us = a + L (b + c dk), ``chunks``: us = a + P H (b + c dk dv) for P chunks, fitted to 231 steps each (1 to 64 portions of 24 to 255 tokens
     beside 0 to 64 of one, 4 to 64 heads of 16 x 16 to 128 x 256).  A quarter in favour of the scan: the choice is then 2 to 3 % off the
-    faster form on average, and at no such step more than 4 us slower than the scan."""
+    faster form on average, and at no such step more than 4 us slower than the scan.  Portions below ``least`` tokens are scanned."""
     lens = [b - a for a, b in zip(cu_host[:-1], cu_host[1:])]
     L = max(lens, default=0)
-    if L < 16 or L >= 256:
+    if L < least or L >= 256:
         return L >= 256
     P = sum((n + 63) // 64 for n in lens)
     return 1.25 * (chunks[0] + P * H * (chunks[1] + chunks[2] * dk * dv)) < scan[0] + L * (scan[1] + scan[2] * dk)
@@ -316,11 +316,13 @@ GLA_CHUNK = 64  # tokens per chunk of the chunk-parallel scan; which portions ta
 
 def gla_plan(cu_host, device, H: int, dk: int, dv: int):
     """The plan of :func:`gla_scan` for a step's portions (:func:`gla_chunk_plan`), or None where scanning them is faster.  Keys up to 128
-    wide, whose chunks are matrix products (16 heads of 64 x 128, us, scan / chunks: one portion of 40 tokens 50 / 35, of 255 288 / 40, 64 of
-    64 tokens 101 / 126, one of 64 beside 64 of one token 91 / 113); wider ones from 256 tokens on."""
+    wide, whose chunks are matrix products, from 64 tokens on (16 heads of 64 x 128, us, scan / chunks: one portion of 255 288 / 40, 64 of
+    64 tokens 101 / 126, one of 64 beside 64 of one token 91 / 113); wider ones from 256 tokens on.  Shorter ones, too, take the GPU less time in
+    chunks (40 tokens 50 / 35), but such steps are bound by the host, whom the plan and three launches in place of one cost more: Malinex
+    prompts of width 1024, 24 tokens 573 / 639, 48 tokens 833 / 905."""
     if cu_host is None or dk > 128:
         return gla_chunk_plan(cu_host, device)
-    return gla_chunk_plan(cu_host, device, 1) if _chunks_pay(cu_host, H, dk, dv, (9.7, 0.28, 0.0197), (32.0, 0.02, 1.03e-5)) else None
+    return gla_chunk_plan(cu_host, device, 1) if _chunks_pay(cu_host, H, dk, dv, (9.7, 0.28, 0.0197), (32.0, 0.02, 1.03e-5), GLA_CHUNK) else None
 
 
 def gla_chunk_plan(cu_host, device, least: int = 4 * GLA_CHUNK):
