@@ -229,10 +229,10 @@ class GroupLimitedMoE(nn.Module):
         from llmctl.ops import hybrid as hops
 
         T = x.shape[0]
-        if (hops.experts_pay(T, self.top, self.E, 2 * self.ff, x.shape[1])
-                and hops.experts_ok(x, self.experts_up, self.experts_down, self.E, self.top, self.w_router)):
-            return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, self.experts_up,
-                                       self.experts_down, "swiglu")
+        if hops.experts_pay(T, self.top, self.E, 2 * self.ff, x.shape[1]):
+            ups, downs = hops.expert_list(self.experts_up), hops.expert_list(self.experts_down)
+            if hops.experts_ok(x, ups, downs, self.E, self.top, self.w_router):
+                return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, ups, downs, "swiglu")
         topi, topw = hops.group_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.top,
                                             self.groups, self.keep)
         flat = topi.reshape(-1)

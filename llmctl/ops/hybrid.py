@@ -448,6 +448,15 @@ _EXPERT_ACTS = {"relu2": 0, "swiglu": 1, "gelu": 2}
 MAX_EXPERTS = 128  # the expert kernels take the weights' addresses as arguments
 
 
+def expert_list(w) -> list:
+    """The weights of a layer's experts as a list: of one stacked tensor, a list of tensors, or a ParameterList (whose own iterator takes a
+    microsecond an entry)."""
+    if torch.is_tensor(w):
+        return [w]
+    own = w._parameters if isinstance(w, torch.nn.ParameterList) else ()
+    return list(own.values()) if own and len(own) == len(w) else list(w)
+
+
 def experts_ok(x, up, down, outputs: int, top: int = 1, w_router=None) -> bool:
     """Whether :func:`routed_experts` takes these operands: bf16 GPU rows and weights, widths in multiples of 8 with rows aligned
     to 16 bytes, at most 128 router outputs, of which at most 64 are chosen, a contiguous, aligned router, no gradient wanted.  ``up`` /
@@ -455,11 +464,17 @@ def experts_ok(x, up, down, outputs: int, top: int = 1, w_router=None) -> bool:
     if not (use_native(x) and x.dtype == torch.bfloat16 and x.dim() == 2 and outputs <= MAX_EXPERTS and top <= 64
             and (w_router is None or (w_router.is_contiguous() and w_router.data_ptr() % 16 == 0))):
         return False
-    ups, downs = ([w] if torch.is_tensor(w) else list(w) for w in (up, down))
-    return (not wants_grad(x, *ups, *downs) and x.shape[1] % 8 == 0 and downs[0].shape[-1] % 8 == 0
-            and all(t.dtype == torch.bfloat16 and t.is_cuda and t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-                    and all(v % 8 == 0 for v in t.stride()[:-1]) for t in [x] + ups + downs)
-            and all(w.stride() == ws[0].stride() for ws in (ups, downs) for w in ws))
+    ups, downs, xs = expert_list(up), expert_list(down), x.stride()
+    if x.shape[1] & 7 or downs[0].shape[-1] & 7 or xs[1] != 1 or xs[0] & 7 or x.data_ptr() & 15:
+        return False
+    for ws in (ups, downs):
+        st = ws[0].stride()
+        if st[-1] != 1 or any(v & 7 for v in st[:-1]):
+            return False
+        for w in ws:
+            if w.dtype is not torch.bfloat16 or not w.is_cuda or w.data_ptr() & 15 or w.stride() != st:
+                return False
+    return not (torch.is_grad_enabled() and wants_grad(x, *ups, *downs))
 
 
 def experts_pay(T: int, top: int, E: int, rows: int, width: int) -> bool:
@@ -481,8 +496,7 @@ def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax:
     ``sigmoid(gate [T, 1])`` if given) is added.  Operands: :func:`experts_ok`."""
     nat = native_hybrid()
     idx, wgt = nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
-    return nat.moe_experts(x, idx, wgt, [up] if torch.is_tensor(up) else list(up), [down] if torch.is_tensor(down) else list(down),
-                           _EXPERT_ACTS[act], shared, gate)
+    return nat.moe_experts(x, idx, wgt, expert_list(up), expert_list(down), _EXPERT_ACTS[act], shared, gate)
 
 
 def act_any(x, kind: str, scale=None):
