@@ -295,3 +295,24 @@ def test_generated_tokens_are_the_same(name):
         assert (e.stats["graph_replays"] > 0) == graphs
         e.close()
     assert outs[0] == outs[1]
+
+
+def test_the_upload_of_a_step_does_not_wait():
+    """The index arrays are on their way while earlier kernels still run, and arrive as they were when the call was made."""
+    from llmctl.serve.decode_graph import upload_packed
+
+    arrays = [np.arange(700, dtype=np.int64), np.zeros(0, np.int32), np.arange(300, dtype=np.int32).reshape(3, 100)]
+    upload_packed(arrays, torch.device("cuda"))  # (the first pinned block of this size is an allocation)
+    a = torch.randn(8192, 8192, device="cuda").bfloat16()
+    torch.cuda.synchronize()
+    for _ in range(40):  # some 30 ms
+        b = a @ a
+    done = torch.cuda.Event()
+    done.record()
+    got = upload_packed(arrays, torch.device("cuda"))
+    want = [x.copy() for x in arrays]
+    for x in arrays:
+        x[...] = -1
+    assert not done.query()
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and torch.equal(g.cpu(), torch.from_numpy(w))
