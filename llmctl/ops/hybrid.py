@@ -170,7 +170,7 @@ def attn_qkv_prep(z, H: int, G: int, dk: int, dv: int, q_norm, k_norm, eps: floa
 def head_rows_ok(x, w) -> bool:
     """Does ``csrc/hybrid/head_rows.hip`` take the per-head products ``x [T, H, K] @ w [H, K, N]``?  Up to 32 rows in bf16, K a
     multiple of 4, N of 8, aligned rows."""
-    return (use_native(x) and 1 <= x.shape[0] <= 32 and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 4 == 0
+    return (1 <= x.shape[0] <= 32 and use_native(x) and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous() and w.shape[1] % 4 == 0
             and w.shape[2] % 8 == 0 and x.stride(2) == 1 and x.stride(0) % 4 == 0 and x.stride(1) % 4 == 0 and x.data_ptr() % 8 == 0
             and w.data_ptr() % 16 == 0 and not wants_grad(x, w))
 
@@ -427,7 +427,7 @@ def rows_linear(x, w, b=None, act=None, act_cols=None, f32: bool = False):
 
 def linear(x, w, b=None):
     """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), others are the library's product."""
-    return rows_linear(x, w, b) if rows_ok(x, w, b) else torch.nn.functional.linear(x, w, b)
+    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else torch.nn.functional.linear(x, w, b)
 
 
 def linear_f32(x, w):
