@@ -58,7 +58,8 @@ def test_qkv_split_cache(T, nq, nkv, D, dtype):
 
 @pytest.mark.parametrize("M,N,K", [(4, 1040, 6144), (4, 1040, 6272), (5, 2048, 8192), (16, 1024, 6144), (8, 3072, 4224), (16, 8192, 256), (16, 8208, 256),
                                    (8, 8200, 256), (16, 16400, 128), (12, 40976, 128), (6, 50257, 64), (4, 3072, 768), (3, 17, 40), (17, 768, 896),
-                                   (20, 4240, 1152), (32, 5120, 2048), (24, 2048, 2176), (32, 8208, 128), (33, 64, 128), (8, 64, 20)])
+                                   (12, 2048, 768), (5, 4112, 768), (5, 1024, 1024), (4, 4096, 1536), (4, 4112, 1536), (24, 4096, 1536), (24, 4096, 1664),
+                                   (16, 61440, 64), (16, 61424, 64), (8, 4096, 8192), (4, 4096, 8192), (4, 4096, 12288), (8, 4096, 12288), (20, 4240, 1152), (32, 5120, 2048), (24, 2048, 2176), (32, 8208, 128), (33, 64, 128), (8, 64, 20)])
 def test_every_form_of_a_few_row_product(M, N, K):
     """The products on either side of every line of the rules, contiguous and strided, with bias and activation, against float64."""
     from llmctl import ops
