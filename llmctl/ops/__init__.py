@@ -9,6 +9,7 @@ from . import ref
 from ._lib import available as native_available
 from .functional import (
     adamw_step_,
+    clip_scale,
     add_layernorm,
     add_rmsnorm,
     col_sum_,
@@ -48,7 +49,7 @@ from .functional import (
 )
 
 __all__ = [
-    "ref", "native_available", "adamw_step_", "add_layernorm", "add_rmsnorm", "col_sum_", "cross_entropy", "decode_linear",
+    "ref", "native_available", "adamw_step_", "add_layernorm", "add_rmsnorm", "clip_scale", "col_sum_", "cross_entropy", "decode_linear",
     "decode_attention_qkv", "decode_fused_ok", "decode_linear_add_rmsnorm", "decode_norm_linear", "decode_norm_qkv_cache", "decode_qkv_rope_cache", "decode_up_swiglu",
     "flash_attention", "gelu", "kv_cache_write", "qkv_flash_attention", "qkv_split_cache", "l2norm_sq", "layernorm", "paged_attention_decode",
     "paged_prefill_attention", "prefill_work_list", "attn_merge_",

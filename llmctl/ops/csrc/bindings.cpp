@@ -39,6 +39,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("cross_entropy_bwd(Tensor dloss, Tensor logits, Tensor lse, Tensor labels, int ignore_index, bool inplace) -> Tensor");
   // optimizer (optim.hip)
   m.def("adamw_step_(Tensor(a!) param, Tensor(b!) master, Tensor grad, Tensor(c!) exp_avg, Tensor(d!) exp_avg_sq, float lr, float beta1, float beta2, float eps, float weight_decay, float bc1, float bc2, Tensor? grad_scale) -> ()");
+  m.def("clip_scale(Tensor nsq, Tensor skipped, float divisor, float max_norm) -> (Tensor, Tensor, Tensor)");
   m.def("l2norm_sq_(Tensor x, Tensor(a!) out) -> ()");
   // attention (flash_attn_fwd.hip / flash_attn_bwd.hip)
   m.def("flash_attn_fwd(Tensor q, Tensor k, Tensor v, float scale, bool causal, Tensor? doc_start=None) -> (Tensor, Tensor)");

@@ -402,6 +402,22 @@ def adamw_step_(param, master, grad, exp_avg, exp_avg_sq, *, lr: float, beta1: f
         ref.adamw_step_(param, master, grad, exp_avg, exp_avg_sq, lr, beta1, beta2, eps, weight_decay, step, gs)
 
 
+def clip_scale(nsq: torch.Tensor, skipped: torch.Tensor, divisor: float, max_norm: float):
+    """``(norm, scale, skipped)`` of an optimizer step from the summed squares of its gradients, on the device: ``norm = sqrt(nsq) /
+    divisor``; ``scale = min(1, max_norm / (norm + 1e-6)) / divisor`` (``1 / divisor`` with ``max_norm`` 0), NaN for a norm that is not
+    finite, which leaves everything untouched in ``adamw_step_``; ``skipped`` counts such steps."""
+    if use_native(nsq):
+        return native().clip_scale(nsq, skipped, divisor, max_norm)
+    norm = torch.sqrt(nsq) / divisor
+    if max_norm > 0:
+        coef = torch.clamp(max_norm / (norm + 1e-6), max=1.0) / divisor
+    else:
+        coef = torch.ones_like(norm) / divisor
+    finite = torch.isfinite(norm)
+    coef = torch.where(finite, coef, torch.full_like(coef, float("nan")))
+    return norm, coef, skipped + (~finite).to(torch.int32).reshape(skipped.shape)
+
+
 def col_sum_ok(x, out) -> bool:
     """Whether ``col_sum_`` (csrc/col_sum.hip) takes these rows and this output; the rest is a plain sum."""
     return (use_native(x) and x.dim() == 2 and x.dtype == torch.bfloat16 and x.shape[0] > 0 and x.stride(1) == 1 and x.shape[1] % 8 == 0
@@ -779,7 +795,7 @@ __all__ = [
     "transpose_",
     "rmsnorm", "add_rmsnorm", "layernorm", "add_layernorm", "rope_qkv", "flash_attention", "rope_flash_attention",
     "swiglu",
-    "gelu", "cross_entropy", "adamw_step_", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
+    "gelu", "cross_entropy", "adamw_step_", "clip_scale", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
     "sample", "decode_linear", "decode_linear_fp8", "decode_fused_ok", "decode_qkv_rope_cache", "decode_up_swiglu", "decode_attention_qkv", "up_swiglu",
     "decode_linear_add_rmsnorm", "rope_qkv_cache", "paged_prefill_attention", "prefill_work_list", "attn_merge_",
     "rms_rstd", "rowscale_ok", "linear_rowscale", "up_swiglu_rowscale", "linear_acc_",

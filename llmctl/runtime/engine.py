@@ -437,7 +437,7 @@ class TrainingEngine:
                 with ctx, ectx:
                     losses.append(self._forward_backward(x, y, denom, before_backward=(
                         self._late_zero_grad if late_zero and i == 0 else None)))
-            loss = torch.stack(losses).sum()
+            loss = losses[0] if n == 1 else torch.stack(losses).sum()
         if self.zero3 is not None:
             self.zero3.finish_grad_sync()
         elif self.sync is not None:

@@ -185,16 +185,9 @@ class FlatAdamW:
             nsq = self.grad_norm_sq()
             if extra_norm_sq is not None:
                 nsq = nsq + extra_norm_sq
-            norm = torch.sqrt(nsq) / grad_divisor
-            if self.max_grad_norm and self.max_grad_norm > 0:
-                coef = torch.clamp(self.max_grad_norm / (norm + 1e-6), max=1.0) / grad_divisor
-            else:
-                coef = torch.ones_like(norm) / grad_divisor
             # skip-step policy: a non-finite global norm (identical on every rank) turns the scale
             # into NaN, which the fused kernel treats as "leave everything untouched"
-            finite = torch.isfinite(norm)
-            coef = torch.where(finite, coef, torch.full_like(coef, float("nan")))
-            self.skipped_steps = self.skipped_steps + (~finite).to(torch.int32)
+            norm, coef, self.skipped_steps = ops.clip_scale(nsq, self.skipped_steps, grad_divisor, self.max_grad_norm or 0.0)
         else:
             norm = self.last_grad_norm if self.last_grad_norm is not None else torch.zeros_like(coef)
         self.last_coef = coef
