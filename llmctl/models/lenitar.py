@@ -23,7 +23,6 @@ from typing import Any, Dict, List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from llmctl.ops import hybrid as hops
 
@@ -157,8 +156,7 @@ class LenitarLM(nn.Module):
         the paged latent pool or the state pools of layer i).  Returns the fp32 residual stream of
         ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer."""
         cfg, eps, dt = self.cfg, self.cfg.layer_norm_eps, self.dtype
-        x = F.embedding(b.ids, self.embed).float() * cfg.embedding_scale  # fp32 residual stream
-        h = hops.layernorm_f32(x, self.layers[0].norm_w, self.layers[0].norm_b, eps, dt)
+        x, h = hops.embed_layernorm_f32(b.ids, self.embed, cfg.embedding_scale, self.layers[0].norm_w, self.layers[0].norm_b, eps)  # fp32 stream
         n = len(self.layers)
         for i, layer in enumerate(self.layers):
             y = layer.mixer.step(h, b, cache.layer(i))

@@ -26,6 +26,7 @@ TORCH_LIBRARY(llmctl, m) {
   // bias gradients (col_sum.hip)
   m.def("col_sum_(Tensor x, Tensor(a!) out, bool add) -> ()");
   // elementwise (elementwise.hip)
+  m.def("embed_rows(Tensor ids, Tensor table, Tensor? pos, Tensor? pos_table) -> Tensor");
   m.def("rope_qkv_fwd(Tensor qkv, Tensor cos, Tensor sin, int nq, int nkv, int seq_len, Tensor? positions) -> (Tensor, Tensor, Tensor)");
   m.def("rope_qk_inplace_(Tensor(a!) qkv, Tensor cos, Tensor sin, int nq, int nkv, int seq_len, Tensor? positions) -> ()");
   m.def("rope_qkv_cache_fwd(Tensor qkv, Tensor cos, Tensor sin, int nq, int nkv, int seq_len, Tensor? positions, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slots) -> (Tensor, Tensor, Tensor)");

@@ -4,6 +4,8 @@
 #include <ATen/ATen.h>
 
 namespace llmctl_hybrid {
+std::tuple<at::Tensor, at::Tensor> embed_layernorm_f32(const at::Tensor& ids, const at::Tensor& table, double scale, const at::Tensor& w,
+                                                       const at::Tensor& b, double eps);
 at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, double eps, bool out_bf16);
 void residual_add_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& b);
 at::Tensor add_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& b, const at::Tensor& w,
@@ -124,6 +126,7 @@ at::Tensor rotary_f32(const at::Tensor& z, int64_t nq, int64_t nk, int64_t dk, c
 }  // namespace llmctl_hybrid
 
 TORCH_LIBRARY(llmctl_hybrid, m) {
+  m.def("embed_layernorm_f32(Tensor ids, Tensor table, float scale, Tensor w, Tensor b, float eps) -> (Tensor, Tensor)");
   m.def("layernorm_f32(Tensor x, Tensor w, Tensor b, float eps, bool out_bf16) -> Tensor");
   m.def("residual_add_(Tensor(a!) x, Tensor a, Tensor? b) -> ()");
   m.def("add_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? b, Tensor w, Tensor bias, float eps, bool out_bf16) -> Tensor");
@@ -182,6 +185,7 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
 }
 
 TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
+  m.impl("embed_layernorm_f32", &llmctl_hybrid::embed_layernorm_f32);
   m.impl("layernorm_f32", &llmctl_hybrid::layernorm_f32);
   m.impl("residual_add_", &llmctl_hybrid::residual_add_);
   m.impl("add_layernorm_f32_", &llmctl_hybrid::add_layernorm_f32_);

@@ -127,6 +127,42 @@ __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __rest
   for (int c = threadIdx.x; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
 }
 
+// The same in quads, all of a row's loads in flight at once (16 rows of 2048: 9.7 us as above, 5.5 so; 2911 rows 24.9 and 16.6).
+template <typename T, int VQ>
+__global__ __launch_bounds__(NT) void embed_rmsnorm_quads_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pos,
+                                                                 const T* __restrict__ table, const T* __restrict__ ptable,
+                                                                 const float* __restrict__ w, float* __restrict__ x, T* __restrict__ h, int W,
+                                                                 float eps) {
+  __shared__ float red[NW];
+  const int64_t row = blockIdx.x;
+  const T* e = table + ids[row] * (int64_t)W;
+  const T* p = ptable + (int64_t)pos[row] * W;
+  float4 v[VQ], pv[VQ], wv[VQ];
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
+    v[i] = ld4(e + c);
+    pv[i] = ld4(p + c);
+    wv[i] = ld4(w + c);
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    v[i].x += pv[i].x, v[i].y += pv[i].y, v[i].z += pv[i].z, v[i].w += pv[i].w;
+    if (c < W) {
+      st4(x + row * W + c, v[i]);
+      q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+  }
+  const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    if (c < W) st4(h + row * W + c, make_float4(v[i].x * rstd * wv[i].x, v[i].y * rstd * wv[i].y, v[i].z * rstd * wv[i].z, v[i].w * rstd * wv[i].w));
+  }
+}
+
 template <int KIND>
 __device__ __forceinline__ float act_one(float v) {
   if constexpr (KIND == 0) {
@@ -362,9 +398,16 @@ std::tuple<at::Tensor, at::Tensor> embed_rmsnorm_f32(const at::Tensor& ids, cons
   if (T == 0) return {x, h};
   dispatch_act(table, [&](auto* tag) {
     using Tt = std::remove_pointer_t<decltype(tag)>;
-    embed_rmsnorm_kernel<Tt><<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), (const Tt*)table.data_ptr(),
-                                                                        (const Tt*)pos_table.data_ptr(), w.data_ptr<float>(), x.data_ptr<float>(),
-                                                                        (Tt*)h.data_ptr(), (int)W, (float)eps);
+    const Tt *tp = (const Tt*)table.data_ptr(), *pp = (const Tt*)pos_table.data_ptr();
+    auto go = [&](auto kern) {
+      kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), tp, pp, w.data_ptr<float>(), x.data_ptr<float>(),
+                                                       (Tt*)h.data_ptr(), (int)W, (float)eps);
+    };
+    const bool quads = W <= 16 * NT && quads_ok(tp, W, W) && quads_ok(pp, W, W) && quads_ok(w.data_ptr<float>(), W, W);
+    if (quads && W <= 4 * NT) go(embed_rmsnorm_quads_kernel<Tt, 1>);
+    else if (quads && W <= 8 * NT) go(embed_rmsnorm_quads_kernel<Tt, 2>);
+    else if (quads) go(embed_rmsnorm_quads_kernel<Tt, 4>);
+    else go(embed_rmsnorm_kernel<Tt>);
   });
   return {x, h};
 }

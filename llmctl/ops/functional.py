@@ -402,6 +402,18 @@ def adamw_step_(param, master, grad, exp_avg, exp_avg_sq, *, lr: float, beta1: f
         ref.adamw_step_(param, master, grad, exp_avg, exp_avg_sq, lr, beta1, beta2, eps, weight_decay, step, gs)
 
 
+def embed_rows(ids: torch.Tensor, table: torch.Tensor, pos: Optional[torch.Tensor] = None,
+               pos_table: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``table[ids]`` (``+ pos_table[pos]``) of a serving step's tokens (no gradients)."""
+    if (use_native(table) and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape[1] % 8 == 0 and t.data_ptr() % 16 == 0
+                                  for t in (table, pos_table) if t is not None)
+            and ids.dim() == 1 and ids.is_contiguous() and ids.dtype == torch.int64
+            and (pos_table is None or (pos.is_contiguous() and pos.dtype in (torch.int32, torch.int64)))):
+        return native().embed_rows(ids, table, pos if pos_table is not None else None, pos_table)
+    x = torch.nn.functional.embedding(ids, table)
+    return x if pos_table is None else x + pos_table[pos]
+
+
 def clip_scale(nsq: torch.Tensor, skipped: torch.Tensor, divisor: float, max_norm: float):
     """``(norm, scale, skipped)`` of an optimizer step from the summed squares of its gradients, on the device: ``norm = sqrt(nsq) /
     divisor``; ``scale = min(1, max_norm / (norm + 1e-6)) / divisor`` (``1 / divisor`` with ``max_norm`` 0), NaN for a norm that is not
@@ -795,7 +807,7 @@ __all__ = [
     "transpose_",
     "rmsnorm", "add_rmsnorm", "layernorm", "add_layernorm", "rope_qkv", "flash_attention", "rope_flash_attention",
     "swiglu",
-    "gelu", "cross_entropy", "adamw_step_", "clip_scale", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
+    "gelu", "cross_entropy", "adamw_step_", "clip_scale", "embed_rows", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
     "sample", "decode_linear", "decode_linear_fp8", "decode_fused_ok", "decode_qkv_rope_cache", "decode_up_swiglu", "decode_attention_qkv", "up_swiglu",
     "decode_linear_add_rmsnorm", "rope_qkv_cache", "paged_prefill_attention", "prefill_work_list", "attn_merge_",
     "rms_rstd", "rowscale_ok", "linear_rowscale", "up_swiglu_rowscale", "linear_acc_",

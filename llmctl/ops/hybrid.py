@@ -31,6 +31,14 @@ def layernorm_f32(x, w, b, eps: float, out_dtype):
     return ref.layernorm_f32(x, w, b, eps, out_dtype)
 
 
+def embed_layernorm_f32(ids, table, scale: float, w, b, eps: float):
+    """``x = table[ids] * scale`` as the fp32 residual stream, and its LayerNorm in the table's dtype.  Returns (x, h)."""
+    if use_native(table) and table.is_contiguous():
+        return native_hybrid().embed_layernorm_f32(ids, table, scale, w, b, eps)
+    x = torch.nn.functional.embedding(ids, table).float() * scale
+    return x, layernorm_f32(x, w, b, eps, table.dtype)
+
+
 def residual_add_(x, a, b=None):
     """``x += a (+ b)`` on the fp32 residual stream (a, b: any float dtype)."""
     if use_native(x):

@@ -437,11 +437,8 @@ class InferenceEngine:
             ok = (local >= 0) & (local < m.embed.shape[0])
             x = F.embedding(local.clamp(0, m.embed.shape[0] - 1), m.embed) * ok.unsqueeze(-1).to(m.embed.dtype)
             x = self._reduce(x)
-        else:
-            x = F.embedding(ids, m.embed)
-        if m.pos_embed is not None:
-            x = x + m.pos_embed[positions]
-        return x
+            return x if m.pos_embed is None else x + m.pos_embed[positions]
+        return ops.embed_rows(ids, m.embed, positions, m.pos_embed)
 
     def _norm(self, layer, x, res, which: str):
         w = layer.attn_norm_w if which == "attn" else layer.mlp_norm_w
@@ -543,7 +540,7 @@ class InferenceEngine:
             doc = torch.from_numpy(plan["doc"]).to(d, non_blocking=True).view(1, T)
         # (one prompt: plain causal attention, which also lets the kernel split the K/V range of
         # its few q-blocks over two workgroups — the split is off for packed documents)
-        x = self._embed(ids, pos.long())
+        x = self._embed(ids, pos)
         if self._norm_fold_ok(T):
             h = self._prefill_layers_folded(x, pos, slots, fa, doc, bt, cu, ctx, work)
             self.stats["prefill_tokens"] += T
@@ -608,7 +605,7 @@ class InferenceEngine:
         ctx_d = torch.tensor(dp["ctx"], dtype=torch.int32).to(d, non_blocking=True)
         fa = pp.get("doc") is not None and d.type == "cuda" and self.knobs.prefill_fa
         doc = torch.from_numpy(pp["doc"]).to(d, non_blocking=True).view(1, Tp) if fa and len(pp["cu"]) > 2 else None
-        x = self._embed(ids, pos.long())
+        x = self._embed(ids, pos)
         res = None
         kc, vc = self.kv_cache.k, self.kv_cache.v
         for li, layer in enumerate(self.model.layers):
