@@ -39,7 +39,7 @@ from llmctl.models import DecoderLM
 from llmctl.utils.env import graph_capture_gc_guard
 
 from .block_manager import PagedKVCache, make_kv_manager
-from .decode_graph import DecodeGraph, GraphTable, upload_packed
+from .decode_graph import STAGES, DecodeGraph, GraphTable, packed_layout, packed_views, upload_packed
 from .prefix_cache import PrefixCache
 from .scheduler import ContinuousBatchScheduler, PrefillChunk, SamplingParams, Sequence
 from .tokenizer import load_tokenizer
@@ -524,20 +524,18 @@ class InferenceEngine:
         use_knobs(self.knobs)
         d = self.device
         T = len(plan["ids"])
-        ids = torch.from_numpy(plan["ids"]).to(d, non_blocking=True)
-        pos = torch.from_numpy(plan["pos"]).to(d, non_blocking=True)
-        slots = torch.from_numpy(plan["slots"]).to(d, non_blocking=True)
-        bt = torch.from_numpy(plan["bt"]).to(d, non_blocking=True)
-        cu = torch.tensor(plan["cu"], dtype=torch.int32).to(d, non_blocking=True)
-        ctx = torch.tensor(plan["ctx"], dtype=torch.int32).to(d, non_blocking=True)
-        work = torch.tensor(plan["work"], dtype=torch.int32).to(d, non_blocking=True)
         # fresh prompts: the training flash-attention kernel over packed documents, K/V straight
         # from the RoPE pass (16 x 2k burst TTFT p50 224.6 -> 218.6 ms, single 2k prompt 27.5 ->
         # 26.2 ms, profiles/serve_r2_session6.txt); knob prefill_fa off keeps the paged kernel
-        doc = None
         fa = plan.get("doc") is not None and d.type == "cuda" and self.knobs.prefill_fa
-        if fa and len(plan["cu"]) > 2:  # several prompts packed: document boundaries
-            doc = torch.from_numpy(plan["doc"]).to(d, non_blocking=True).view(1, T)
+        docs = fa and len(plan["cu"]) > 2  # several prompts packed: document boundaries
+        i64, i32 = (lambda a: np.asarray(a, dtype=np.int64)), (lambda a: np.asarray(a, dtype=np.int32))
+        # all index arrays of the step through one copy, for which the host does not wait (four GPT-7B layers, 2048 tokens among
+        # others: 3266 -> 3105 us)
+        ids, slots, last, pos, bt, cu, ctx, work, doc = upload_packed(
+            [i64(plan["ids"]), i64(plan["slots"]), i64(plan["last"]), i32(plan["pos"]), i32(plan["bt"]), i32(plan["cu"]), i32(plan["ctx"]),
+             i32(plan["work"]), i32(plan["doc"]) if docs else np.zeros(0, np.int32)], d)
+        doc = doc.view(1, T) if docs else None
         # (one prompt: plain causal attention, which also lets the kernel split the K/V range of
         # its few q-blocks over two workgroups — the split is off for packed documents)
         x = self._embed(ids, pos)
@@ -546,7 +544,7 @@ class InferenceEngine:
             self.stats["prefill_tokens"] += T
             if not plan["last"]:
                 return torch.empty(0, self.cfg.vocab_size, device=d, dtype=h.dtype)
-            hl = h.index_select(0, torch.tensor(plan["last"], device=d))
+            hl = h.index_select(0, last)
             xn = ops.rmsnorm(hl, self.model.final_norm_w, self.cfg.layer_norm_eps)
             return self._gather_vocab(ops.decode_linear(xn, self.model.head_weight()))
         res = None
@@ -566,7 +564,6 @@ class InferenceEngine:
         self.stats["prefill_tokens"] += T
         if not plan["last"]:
             return torch.empty(0, self.cfg.vocab_size, device=d, dtype=x.dtype)
-        last = torch.tensor(plan["last"], device=d)
         return self._final(x.index_select(0, last), res.index_select(0, last))
 
     # ------------------------------------------------------------------ mixed prefill + decode
@@ -754,28 +751,29 @@ class InferenceEngine:
 
     def _static(self, nb: int) -> Dict:
         d = self.device
-        bufs = {"ids": torch.zeros(nb, dtype=torch.long, device=d),
-                "positions": torch.zeros(nb, dtype=torch.int32, device=d),
-                "slots": torch.full((nb,), -1, dtype=torch.long, device=d),
-                "block_tables": torch.zeros(nb, self.max_blocks_per_seq, dtype=torch.int32, device=d),
-                "ctx_lens": torch.ones(nb, dtype=torch.int32, device=d),
-                # in-graph sampling: per-row parameters (rewritten when the batch's change) and uniforms
-                "u": torch.zeros(nb, dtype=torch.float32, device=d),
-                "temp": torch.zeros(nb, dtype=torch.float32, device=d),
-                "topk": torch.zeros(nb, dtype=torch.int32, device=d),
-                "topp": torch.ones(nb, dtype=torch.float32, device=d)}
-        # pinned host staging of the step inputs, two sets: an asynchronous step refills one while
-        # the other's H2D copies may still be queued behind the step in flight (a non_blocking
-        # copy from pageable memory would be synchronous)
-        pin = self.device.type == "cuda"
+        pin = d.type == "cuda"
+        # the step's inputs: views of one buffer, the ids first, so that a step takes one copy (of six, each took 3 us of the
+        # device's time and a gap: one row of gpt2-125m, 12 layers, 413 -> 392 us a step with the embedding in one launch)
+        arrays = [np.zeros(nb, np.int64), np.zeros(nb, np.int32), np.full(nb, -1, np.int64), np.zeros((nb, self.max_blocks_per_seq), np.int32),
+                  np.ones(nb, np.int32), np.zeros(nb, np.int32)]
+        offs, size = packed_layout(arrays)
+        # pinned host sets, of which the host fills one while the others' copies may still be queued behind the steps in flight.  They start
+        # as the defaults: rows past the live batch are copied too and must stay valid (block id 0, context 1) for the padded graph rows
+        hosts = torch.zeros(STAGES, size, dtype=torch.uint8, pin_memory=pin)
         stage = []
-        for _ in range(2):
-            # initialised from the device defaults: rows past the live batch are copied too and
-            # must stay valid (block id 0, context 1) for the padded graph rows
-            h = {k: bufs[k].to("cpu") for k in self._STAGED}
-            stage.append({k: (v.pin_memory() if pin else v) for k, v in h.items()})
-        bufs["stage"] = stage
-        bufs["flip"] = 0
+        for h in hosts:
+            hn = dict(zip(self._STAGED, (v.numpy() for v in packed_views(h, offs, arrays))))
+            hn["u"] = hn["u"].view(np.float32)
+            for v, a in zip(hn.values(), arrays):
+                v[...] = a
+            stage.append((h, hn, torch.cuda.Event() if pin else None))
+        buf = hosts[0].to(d)
+        bufs = dict(zip(self._STAGED, packed_views(buf, offs, arrays)))
+        bufs["u"] = bufs["u"].view(torch.float32)
+        bufs.update(inputs=buf, ids_end=offs[1], stage=stage, turn=0,
+                    # in-graph sampling: per-row parameters (rewritten when the batch's change)
+                    temp=torch.zeros(nb, dtype=torch.float32, device=d), topk=torch.zeros(nb, dtype=torch.int32, device=d),
+                    topp=torch.ones(nb, dtype=torch.float32, device=d))
         toks = torch.zeros(nb, dtype=torch.long)
         bufs["host_toks"] = [toks.pin_memory() if pin else toks, toks.clone().pin_memory() if pin else toks.clone()]
         bufs["tflip"] = 0
@@ -886,9 +884,10 @@ class InferenceEngine:
         if nb not in self._graphs:
             self._capture(nb)
         g, b = self._graphs[nb]
-        h = b["stage"][b["flip"]]
-        b["flip"] ^= 1
-        hn = {k: v.numpy() for k, v in h.items()}
+        h, hn, ev = b["stage"][b["turn"]]
+        b["turn"] = (b["turn"] + 1) % STAGES
+        if ev is not None:
+            ev.synchronize()  # the copy that last read this set
         if not cont:
             hn["ids"][:n] = plan["ids"]
         hn["positions"][:n] = plan["positions"]
@@ -910,10 +909,10 @@ class InferenceEngine:
                 b["topk"][:n].copy_(torch.from_numpy(np.frombuffer(key[1], dtype=np.int32).copy()).to(d))
                 b["topp"][:n].copy_(torch.from_numpy(np.frombuffer(key[2], dtype=np.float32).copy()).to(d))
                 b["params_key"] = key
-        for k in self._STAGED:
-            if cont and k == "ids":
-                continue
-            b[k].copy_(h[k], non_blocking=True)
+        at = b["ids_end"] if cont else 0
+        b["inputs"][at:].copy_(h[at:], non_blocking=True)
+        if ev is not None:
+            ev.record()
         g.replay()
         self.stats["graph_replays"] += 1
         return g, b
