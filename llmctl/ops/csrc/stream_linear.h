@@ -2,12 +2,15 @@
 //
 // The bound is the weight stream and, below some 20 MB of weights, the latency of one round trip to HBM plus the launch
 // (3.5 us in a graph).  Measured beside the library's product (one MI355X, weights from HBM, 16 rows, us):
-//   N x K        2048 x 2048  4096 x 2048  8192 x 2048  10496 x 2048  32000 x 2048  4096 x 4096  2048 x 4096  768 x 3072  768 x 768
-//   library          11.1         10.8         12.3         14.0          31.6          15.0         14.3         9.1         5.2
-//   here              6.2          6.9          9.6         15.0          27.5          10.4           9.8        7.7         4.0
-// A workgroup owns whole outputs (no partial sums between workgroups), so N / 16 < 256 leaves CUs idle, and a CU draws about 30 GB/s
-// from HBM: 2048 x 8192 takes 17 us against the library's 13, which splits K over the chip; and tiles that fill the CUs one and a half
-// times (10496) cost as much as two rounds.  The callers' rules (llmctl/ops/functional.py: stream_pays, decode_form) leave such shapes.
+//   N x K        768 x 768  768 x 3072  2048 x 2048  2048 x 4096  4240 x 2048  8256 x 2048  9248 x 2048  10496 x 2048  32000 x 2048
+//   library          5.2         9.1        11.0         14.8         12.1         13.9         15.9         15.0          35
+//   whole tiles      4.0         7.7         6.5         10.0         10.5         15.0         15.5         15.0          29
+//   here             3.9         6.6         6.1          9.0          7.8         10.8         11.6         12.6          29
+// A workgroup owns whole outputs (no partial sums between workgroups) and draws some 30 GB/s, so all 256 CUs must have the same number of them:
+// it owns N / 256 outputs (or an even part, see launch), whatever that is, and the MFMA tiles' other rows repeat its last one (``whole tiles``:
+// 16 or 32 outputs each, which left CUs idle below 4096 outputs and made two uneven rounds above 8192).  With K beyond 4096 a
+// workgroup's own read of x weighs as much as its weights: 2048 x 8192 takes 15 us against the library's 13.6, which splits K over the
+// chip.  The callers' rules (llmctl/ops/functional.py: stream_pays, decode_form) leave such shapes.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -31,6 +34,7 @@ struct Args {
   int act;       // 0 none, 1 gelu (erf), 2 gelu (tanh), 3 relu^2
   int act_cols;  // of the first that many columns
   int f32;  // y is fp32
+  int rows = 0;  // outputs of a workgroup, at most 16 NT
 };
 
 __device__ __forceinline__ uint4 load_or_zero(const unsigned short* p, bool in) {
@@ -52,7 +56,7 @@ __device__ __forceinline__ float activate(int act, float v) {
   return v;
 }
 
-// A workgroup of NW waves owns 16 NT weight rows; the waves split K.  A lane streams 16 bytes of its weight row per 32-deep step,
+// A workgroup of NW waves owns ``rows`` weight rows, at most 16 NT; the waves split K.  A lane streams 16 bytes of its weight row per 32-deep step,
 // U steps in flight before the first MFMA; the weight fragment is the MFMA row operand, so a lane ends up with four
 // neighbouring outputs of one token.  K is a multiple of 8 (the last step is filled up with zeros), N any.
 template <int NT, int MT, int NW, int U>
@@ -60,10 +64,10 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
   __shared__ acc_t red[NW][NT * MT][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, kg = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT;
+  const int n0 = blockIdx.x * g.rows, n1 = min(n0 + g.rows, g.N);
   const unsigned short* wp[NT];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) wp[n] = g.w + (long)min(n0 + n * 16 + r, g.N - 1) * g.ldw + 8 * kg;
+  for (int n = 0; n < NT; ++n) wp[n] = g.w + (long)min(n0 + n * 16 + r, n1 - 1) * g.ldw + 8 * kg;
   const unsigned short* xp[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) xp[m] = g.x + (long)min(m * 16 + r, g.M - 1) * g.ldx + 8 * kg;
@@ -112,12 +116,12 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
   __syncthreads();
   for (int i = tid; i < NT * MT * 64; i += NW * 64) {
     const int t = i >> 6, l = i & 63, row = (t % MT) * 16 + (l & 15), c = n0 + (t / MT) * 16 + 4 * (l >> 4);
-    if (row >= g.M || c >= g.N) continue;
+    if (row >= g.M || c >= n1) continue;
     acc_t s = red[0][t][l];
 #pragma unroll
     for (int v = 1; v < NW; ++v) s += red[v][t][l];
     const long o = (long)row * g.N + c;
-    const int left = min(4, g.N - c);
+    const int left = min(4, n1 - c);
     float v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -126,7 +130,7 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
     }
     if (g.f32) {
       float* y = static_cast<float*>(g.y) + o;
-      if (left == 4 && (g.N & 3) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+      if (left == 4 && (o & 3) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
       else
         for (int j = 0; j < left; ++j) y[j] = v[j];
     } else {
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
       unsigned short h[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) h[j] = __bfloat16_as_ushort(__float2bfloat16(v[j]));
-      if (left == 4 && (g.N & 3) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
+      if (left == 4 && (o & 3) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
       else
         for (int j = 0; j < left; ++j) y[j] = h[j];
     }
@@ -142,26 +146,35 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
 }
 
 template <int NT, int MT, int NW, int U>
-inline void go(const Args& g, hipStream_t st) {
-  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + 16 * NT - 1) / (16 * NT))), NW * 64, 0, st>>>(g);
+inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
+  g.rows = rows;
+  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + rows - 1) / rows)), NW * 64, 0, st>>>(g);
 }
 
-// Weight rows per workgroup: a workgroup also reads its rows' x, 16 rows of it per 16 weight rows, so wide outputs take 32 or
-// 64 weight rows per pass over x once that leaves the chip full (16 rows of x, K 2048, us by 16 / 32 / 64 weight rows: N 4096 7.1 /
-// 8.4 / 12.2, N 8192 11.1 / 9.7 / 12.7, N 32000 34.8 / 29.9 / 27.2).  With up to four rows x costs next to nothing and two waves of
-// twice the depth per workgroup are best (N 8192, one row: 8.1 us against 9.5).  17 to 32 rows: 32 weight rows from N 5120.
+// Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to
+// nothing, and smaller workgroups in more rounds hide the latency better (one row, K 2048, one round / rounds of at most 16 weight rows:
+// N 5152 7.8 / 7.3 us, N 8192 9.9 / 8.5, N 12288 13.0 / 12.0; from K 3072 on the other way: N 9248 x 4096 17.7 / 18.3, so rounds of 32 there).  Waves
+// and depth: 16 rows of x, 8 waves of 4 steps / 4 of 8: N 2048 6.00 / 6.06 us, N 4096 7.16 / 7.26; one row 768 x 3072 4.42 / 4.51.
 inline void launch(const Args& g, hipStream_t st) {
+  const int tall = g.M > 4 || g.N <= 4096 ? 64 : g.N > 16384 || g.K <= 2048 ? 16 : 32;  // rows of a workgroup at most
+  const int rounds = (g.N + 256 * tall - 1) / (256 * tall);                             // of 256 workgroups
+  int rows = (g.N + 256 * rounds - 1) / (256 * rounds);
+  if (g.N > 16384) rows = g.M > 4 ? (rows + 3) / 4 * 4 : 16;  // (whole quads are stored at once)
   if (g.M > 16) {
-    if (g.N < 5120) go<1, 2, 4, 8>(g, st);
-    else go<2, 2, 4, 4>(g, st);
-  } else if (g.M <= 4 && g.N >= 6144) {
-    go<1, 1, 2, 8>(g, st);
-  } else if (g.N < 5120) {
-    go<1, 1, 4, 8>(g, st);
-  } else if (g.N < 24576) {
-    go<2, 1, 4, 8>(g, st);
+    if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
+    else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);
+    else if (rows <= 48) go<3, 2, 4, 4>(g, st, rows);
+    else go<4, 2, 4, 4>(g, st, rows);
+  } else if (rows <= 16) {
+    if (rounds > 1 && g.N <= 16384) go<1, 1, 2, 8>(g, st, rows);
+    else go<1, 1, 8, 4>(g, st, rows);
+  } else if (rows <= 32) {
+    if (g.M <= 4) go<2, 1, 4, 4>(g, st, rows);
+    else go<2, 1, 4, 8>(g, st, rows);
+  } else if (rows <= 48) {
+    go<3, 1, 4, 4>(g, st, rows);
   } else {
-    go<4, 1, 4, 4>(g, st);
+    go<4, 1, 4, 4>(g, st, rows);
   }
 }
 

@@ -557,22 +557,20 @@ def stream_ok(x, w, b=None) -> bool:
 @functools.lru_cache(maxsize=4096)
 def stream_pays(M: int, N: int, K: int) -> bool:
     """Is the weight stream faster than the library's product?  In a graph, weights from HBM, us, library / here, beside each line.  (The
-    library splits K over the chip at some sizes and not at others: 4096 x 8192 15.2, 4096 x 11008 37.5.)"""
-    if M > 16:  # 32 rows 4096 x 2048 11.4 / 8.9, 2048 x 4096 11.7 / 13.3, 10240 x 2048 14.6 / 17.7; 24 rows 4240 x 2048 11.1 / 12.5, 4128 x 1024 11.3 / 7.8
-        return N <= 8192 and K <= 2048 and not (4096 < N < 5120 and K > 1024)
-    if K > 4096:  # only where the tiles fill the 256 CUs evenly, and up to 8 rows: 8 rows 4096 x 8192 15.2 / 16.1, 4096 x 11008 37.3 / 21.6, 32000 x 6144
-        # 86 / 74; 5120 x 8192 19.4 / 22.6, 2048 x 6144 11.0 / 11.8; 16 rows 4096 x 8192 15.8 / 17.9.  Rows of W that lie a multiple of 8192 entries apart (up to
-        # four rows, whose workgroups hold fewer of them: of 4096) crowd the same channels: 8 rows 16384 x 16384 98 / 109, 128256 x 8192 352 / 435, 4 rows
-        # 12288 x 12288 59 / 68, 8192 x 28672 84 / 91; 16384 x 8192 61 / 52
-        if K % 8192 == 0 if M > 4 else K % 4096 == 0 and K != 8192:
-            return False
-        tiles = (N + 15) // 16 if N < 5120 or (M <= 4 and N >= 6144) else (N + 31) // 32 if N < 24576 else (N + 63) // 64
-        return M <= 8 and tiles >= 0.95 * (-(-tiles // 256) * 256)
-    # (8193 to 16384 outputs at more than 8 rows fill the CUs one and a half times with tiles of 32: 16 rows 8192 x 2048 12.3 / 9.6, but
-    # 8256 x 2048 13.5 / 14.5 and 10240 x 3072 19.3 / 20.7.  They stay here: in a step that is not captured the library's call takes 18 us of
-    # the host and this one 7.)
-    # 16 rows 32000 x 2048 31.6 / 27.5, 50304 x 768 18.2 / 21.7, 50304 x 3072 57.5 / 70.2, 102400 x 2048 145 / 83, 65024 x 3072 71 / 77, 152064 x 3072 287 / 177; 4 rows
-    # 50304 x 768 18.0 / 17.5
+    library splits K over the chip at some sizes and not at others: 16 rows 4096 x 8192 15.0, 4096 x 11008 37.)"""
+    if M > 16:  # a fragment of x more for every one of W: 32 rows 4240 x 2048 12.2 / 9.7, 12288 x 2048 15.7 / 15.5, 14336 x 1024 21.5 / 10.8, but 14336 x 2048
+        # 16.7 / 17.2, 6144 x 3072 13.1 / 14.2, 50304 x 768 20.7 / 25.2; 152064 x 3072 295 / 202; 24 rows 4096 x 4096 13.6 / 13.1
+        return K <= (2048 if N <= 12288 else 1024 if N <= 32000 else 0) or (N >= 102400 and K <= 4096) or (M <= 24 and N <= 4096 and K <= 4096)
+    if K > 4096 and K % 8192 == 0:  # rows of W that lie a multiple of 8192 entries apart crowd the same channels: 8 rows 2048 x 8192 13.0 / 12.4, 6144 x 8192
+        # 23.7 / 25.6, 16384 x 16384 101 / 129; 4 rows 32000 x 8192 111 / 94; 16 rows 2048 x 8192 13.6 / 15.4
+        return (M <= 8 and N <= (4096 if K == 8192 else 2304)) or (M <= 4 and K == 8192 and N >= 20480)
+    if K > 4096 and M > 8:  # a workgroup reads all of x for its few rows of W: 16 rows 3648 x 6144 13.2 / 14.8, 2304 x 5120 12.3 / 11.7, 12288 x 10240 58 / 51, 32000 x
+        # 6144 86 / 77, 50304 x 12288 220 / 237
+        return 4096 < N <= 40960 or (N <= 2304 and K < 6144)
+    if K > 4096:  # 8 rows 2048 x 6144 11.2 / 10.1, 4096 x 12288 23.0 / 24.5, 12288 x 12288 61 / 57, 50304 x 5120 94 / 102
+        return M <= 4 or ((N <= 40960 or N >= 61440) and not (K % 4096 == 0 and K < 16384 and 2304 < N <= 4096))
+    # 16 rows 2048 x 2048 11.1 / 6.1, 8256 x 2048 14.2 / 11.0, 32000 x 2048 35 / 30, 50304 x 768 20.0 / 21.8, 50304 x 3072 62 / 68, 102400 x 2048 147 / 86, 65024 x 3072
+    # 76 / 81, 152064 x 3072 295 / 183; 4 rows 50304 x 768 19.7 / 19.3
     return M <= 4 or N <= 40960 or N >= 61440
 
 
@@ -580,15 +578,16 @@ def stream_pays(M: int, N: int, K: int) -> bool:
 def decode_form(M: int, N: int, K: int) -> str:
     """The form of :func:`decode_linear` by size: ``stream``, ``skinny`` (``csrc/skinny_gemm.hip``) or ``library``.  Beside
     :func:`stream_pays`, us in a graph, stream / skinny:"""
-    if M > 16:  # 32 rows 3072 x 768 5.6 / 5.2, 4096 x 1024 6.4 / 5.9, 4096 x 1536 7.8 / 7.6, 4096 x 2048 8.9 / 10.5
-        return "skinny" if K <= 1536 and N <= 4096 else "stream" if stream_pays(M, N, K) else "library"
-    if M <= 4:  # 4 rows 3072 x 768 4.4 / 4.0, 4096 x 1536 5.8 / 5.5, 8192 x 1536 7.8 / 8.7, 4096 x 4096 9.0 / 9.1, 5120 x 10240 26.7 / 40.8
-        return "skinny" if (K < 1024 and N <= 16384) or (K <= 1536 and N <= 4096) else "stream"
-    if K < 1024 and N <= 4096:  # 16 rows 768 x 768 4.2 / 3.7, 2304 x 768 4.75 / 4.52, 6144 x 768 5.75 / 7.71; 5 rows 1024 x 1024 4.38 / 4.68
+    # short rows: 1 row 2304 x 768 3.63 / 3.32, 8192 x 768 5.66 / 5.30; 16 rows 768 x 512 3.48 / 3.07, 5152 x 512 4.51 / 4.08, but 2304 x 768 4.10 / 4.06 and 768 x 768
+    # 3.88 / 3.97; 24 rows 4096 x 768 4.87 / 4.57
+    if K < (768 if 4 < M <= 16 and N < 3072 else 1024) and N <= (16384 if M <= 4 else 5152 if M <= 16 else 4096):
         return "skinny"
-    if (K > 4096 and N <= 2048) or (2048 <= K < 3072 and N <= 4096) or (8192 < N <= 12288 and not 1024 < K < 3072):
-        return "skinny"  # 8 rows 1024 x 11008 18.8 / 12.9, 4096 x 2048 6.6 / 6.1, 10240 x 4096 23.6 / 21.1; 16 rows 2048 x 6144 13.4 / 11.8
-    return "stream" if N < (16384 if M >= 8 else 40961) or stream_pays(M, N, K) else "library"  # 8 rows 4096 x 11008 21.6 / 27.4
+    # few long rows, of which skinny splits K over the chip: 8 rows 1024 x 12288 15.0 / 13.3, 16 rows 768 x 10240 15.5 / 13.6, 12 rows 2048 x 28672 42.6 / 37.1,
+    # 16 rows 2048 x 14336 24.7 / 21.5
+    if 4 < M <= 16 and K > (8192 if N <= 1024 else 12288) and N <= (2048 if M >= 8 else 1024):
+        return "skinny"
+    # (the library's own times jump here: 12 rows 2048 x 11008 35.8, stream 18.2; 2048 x 10240 13.1 and 13.1)
+    return "stream" if stream_pays(M, N, K) or (M <= 16 and N <= 4096 and K % 8192) else "library"
 
 
 def decode_linear(x, w, b=None, act: Optional[str] = None):
