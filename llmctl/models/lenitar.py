@@ -160,7 +160,7 @@ class LenitarLM(nn.Module):
         n = len(self.layers)
         for i, layer in enumerate(self.layers):
             y = layer.mixer.step(h, b, cache.layer(i))
-            z = layer.ff(h) if layer.ff is not None else None
+            z = layer.ff(h, late=True) if layer.ff is not None else None
             if i + 1 < n and trail is None:
                 nxt = self.layers[i + 1]
                 h = hops.add_layernorm_f32_(x, y, z, nxt.norm_w, nxt.norm_b, eps, dt)

@@ -217,7 +217,7 @@ class MalinexLM(nn.Module):
             y, r = layer.mixer.step(h, b, cache.layer(i))
             h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm1b, layer.norm2 if layer.ff is not None else nxt, eps, dt)
             if layer.ff is not None:
-                y, r = layer.ff(h)
+                y, r = layer.ff(h, late=True) if isinstance(layer.ff, BiasedSoftmaxMoE) else layer.ff(h)
                 h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm2b, nxt, eps, dt)
             if trail is not None:
                 trail.append(x.clone())

@@ -224,15 +224,16 @@ class GroupLimitedMoE(nn.Module):
         return (hops.experts_pay(T, self.top, self.E, *up.shape)
                 and hops.experts_ok(up[:1], self.experts_up, self.experts_down, self.E, self.top, self.w_router))
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        """x [T, width] -> fp32 [T, width]."""
+    def forward(self, x: torch.Tensor, late: bool = False):
+        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it)."""
         from llmctl.ops import hybrid as hops
 
         T = x.shape[0]
         if hops.experts_pay(T, self.top, self.E, 2 * self.ff, x.shape[1]):
             ups, downs = hops.expert_list(self.experts_up), hops.expert_list(self.experts_down)
             if hops.experts_ok(x, ups, downs, self.E, self.top, self.w_router):
-                return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, ups, downs, "swiglu")
+                return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, ups, downs, "swiglu",
+                                           **({"late": True} if late else {}))
         topi, topw = hops.group_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.top,
                                             self.groups, self.keep)
         flat = topi.reshape(-1)
@@ -349,8 +350,8 @@ class BiasedSoftmaxMoE(nn.Module):
         return self._dense(T) or (hops.experts_pay(T, self.top, self.E, *self.w_up.shape[1:]) and hops.experts_ok(
             self.w_up[0, :1], self.w_up, down, self.E + self.identity, self.top, self.w_router))
 
-    def forward(self, x: torch.Tensor):
-        """x [T, width] -> fp32 [T, width] (and the side columns)."""
+    def forward(self, x: torch.Tensor, late: bool = False):
+        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it) (and the side columns)."""
         from llmctl.ops import hybrid as hops
 
         from .mixers import _mm_f32
@@ -375,7 +376,7 @@ class BiasedSoftmaxMoE(nn.Module):
         if (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
                 and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
             out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
-                                      self.act, ys, gate)
+                                      self.act, ys, gate, **({"late": True} if late else {}))
             return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out
         topi, topw = hops.bias_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.bias, self.top,
                                            self.groups, self.keep, self.renorm)

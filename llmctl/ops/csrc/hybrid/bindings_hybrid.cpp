@@ -51,8 +51,17 @@ std::tuple<at::Tensor, at::Tensor> bias_topk_router(const at::Tensor& logits, co
 at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t act, int64_t act_cols, bool f32);
 std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t top,
                                              int64_t groups, int64_t keep, bool softmax, bool renorm);
+at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act);
 at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
                        const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate);
+at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
+                   const c10::optional<at::Tensor>& gate, int64_t experts);
+at::Tensor add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
+                                      double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
+                                      const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts);
+at::Tensor gated_norm_add_experts_f32_(at::Tensor x, const at::Tensor& r, const at::Tensor& w_post, const c10::optional<at::Tensor>& w_next, double eps,
+                                       const at::Tensor& ye, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
+                                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts);
 std::tuple<at::Tensor, at::Tensor> hc_embed_norm(const at::Tensor& ids, const at::Tensor& table, int64_t streams, const at::Tensor& c_in,
                                                  const at::Tensor& g, double eps, bool out_bf16);
 at::Tensor hc_update_norm_(at::Tensor X, const at::Tensor& y1, double s1, const c10::optional<at::Tensor>& y2, double s2, const at::Tensor& mix,
@@ -157,7 +166,11 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("embed_rmsnorm_f32(Tensor ids, Tensor pos, Tensor table, Tensor pos_table, Tensor w, float eps, bool out_bf16) -> (Tensor, Tensor)");
   m.def("rows_linear(Tensor x, Tensor w, Tensor? bias, int act, int act_cols, bool f32) -> Tensor");
   m.def("moe_route(Tensor x, Tensor w, Tensor? bias, int top, int groups, int keep, bool softmax, bool renorm) -> (Tensor, Tensor)");
+  m.def("moe_expert_rows(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act) -> Tensor");
   m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
+  m.def("moe_sum(Tensor y, Tensor idx, Tensor wgt, Tensor x, Tensor? shared, Tensor? gate, int experts) -> Tensor");
+  m.def("add_experts_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? w, Tensor? bias, float eps, Tensor y, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts) -> Tensor");
+  m.def("gated_norm_add_experts_f32_(Tensor(a!) x, Tensor r, Tensor w_post, Tensor? w_next, float eps, Tensor ye, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts) -> Tensor");
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
   m.def("qk_fullnorm_prep(Tensor z, int H, int G, int dk, int dv, Tensor q_norm, Tensor k_norm, float eps, Tensor pos, float temp_coef, int temp_every, Tensor(a!) cache, Tensor slots, Tensor? freq=None, int rot=0, bool interleaved=False, float amp=1.0) -> Tensor");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, float qscale, Tensor(a!) S, Tensor slots, Tensor cu, Tensor start, Tensor(b!)? logd=None, bool write_out=True, bool write_state=True) -> Tensor");
@@ -209,7 +222,11 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("embed_rmsnorm_f32", &llmctl_hybrid::embed_rmsnorm_f32);
   m.impl("rows_linear", &llmctl_hybrid::rows_linear);
   m.impl("moe_route", &llmctl_hybrid::moe_route);
+  m.impl("moe_expert_rows", &llmctl_hybrid::moe_expert_rows);
   m.impl("moe_experts", &llmctl_hybrid::moe_experts);
+  m.impl("moe_sum", &llmctl_hybrid::moe_sum);
+  m.impl("add_experts_layernorm_f32_", &llmctl_hybrid::add_experts_layernorm_f32_);
+  m.impl("gated_norm_add_experts_f32_", &llmctl_hybrid::gated_norm_add_experts_f32_);
   m.impl("act_any", &llmctl_hybrid::act_any);
   m.impl("qk_fullnorm_prep", &llmctl_hybrid::qk_fullnorm_prep);
   m.impl("gla_scan", &llmctl_hybrid::gla_scan);

@@ -6,7 +6,7 @@
 //   qk_fullnorm_prep          queries and keys normed as whole rows, turned by their position, keys and values to the cache
 //   glu_act                   act(gate) * up of rows [gate | up] (silu or the tanh GELU), times an optional factor per row
 // All arithmetic fp32; y, r, h in the activation dtype or fp32.
-#include "hybrid_common.h"
+#include "expert_rows.h"
 
 namespace llmctl_hybrid {
 
@@ -66,22 +66,26 @@ __global__ __launch_bounds__(NT) void gated_norm_add_norm_kernel(float* __restri
 
 // The same for rows of up to 4 * NT * VQ values in quads, all of a row's loads in flight at once (2048 wide, 16
 // rows: 10.5 us as above, 4.5 so; 2911 rows 27.3 and 18.4).
-template <typename TY, typename TR, typename TH, int VQ>
+// ``Y``: y is the weighted sum of the routed experts' rows of that type (expert_rows.h) instead of a tensor (16 rows, two experts each and a shared
+// one: 4.7 us for the sum and 4.7 here, together 4.9; 2911 rows 12.8 + 17.1, together 19.0).
+template <typename TY, typename TR, typename TH, int VQ, typename Y = void>
 __global__ __launch_bounds__(NT) void gated_norm_add_norm_quads_kernel(float* __restrict__ x, const TY* __restrict__ y, int64_t y_st,
                                                                        const TR* __restrict__ r, int64_t r_st, const float* __restrict__ wp,
-                                                                       const float* __restrict__ wn, TH* __restrict__ h, int W, float eps) {
+                                                                       const float* __restrict__ wn, TH* __restrict__ h, int W, float eps,
+                                                                       ExpertRows m) {
   __shared__ float red[NW];
   const int64_t row = blockIdx.x;
   float4 g[VQ], rv[VQ], xv[VQ], pv[VQ], nv[VQ];
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
-    g[i] = ld4(y + row * y_st + c);
+    if constexpr (std::is_void_v<Y>) g[i] = ld4(y + row * y_st + c);
     rv[i] = ld4(r + row * r_st + c);
     xv[i] = ld4(x + row * W + c);
     pv[i] = ld4(wp + c);
     nv[i] = wn != nullptr ? ld4(wn + c) : make_float4(0.f, 0.f, 0.f, 0.f);
   }
+  if constexpr (!std::is_void_v<Y>) expert_sum_quads<Y, NT, VQ>(m, row, W, g);
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
@@ -362,16 +366,19 @@ at::Tensor gated_norm_add_norm_f32_(at::Tensor x, const at::Tensor& y, const at:
     using TY = std::remove_pointer_t<decltype(ty)>;
     using TR = std::remove_pointer_t<decltype(tr)>;
     using TH = std::remove_pointer_t<decltype(th)>;
+    TH* hp = wn != nullptr ? (TH*)h.data_ptr() : nullptr;
     auto launch = [&](auto kern) {
       kern<<<dim3((unsigned)T), NT, 0, st>>>(x.data_ptr<float>(), (const TY*)y.data_ptr(), y.stride(0), (const TR*)r.data_ptr(), r.stride(0),
-                                             w_post.data_ptr<float>(), wn, wn != nullptr ? (TH*)h.data_ptr() : (TH*)nullptr, (int)W, (float)eps);
+                                             w_post.data_ptr<float>(), wn, hp, (int)W, (float)eps, ExpertRows{});
     };
     const bool quads = W <= 16 * NT && quads_ok((const TY*)y.data_ptr(), y.stride(0), W) && quads_ok((const TR*)r.data_ptr(), r.stride(0), W) &&
                        quads_ok(x.data_ptr<float>(), W, W) && quads_ok(w_post.data_ptr<float>(), W, W) && (wn == nullptr || quads_ok(wn, W, W));
     if (quads && W <= 4 * NT) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 1>);
     else if (quads && W <= 8 * NT) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 2>);
     else if (quads) launch(gated_norm_add_norm_quads_kernel<TY, TR, TH, 4>);
-    else launch(gated_norm_add_norm_kernel<TY, TR, TH>);
+    else
+      gated_norm_add_norm_kernel<TY, TR, TH><<<dim3((unsigned)T), NT, 0, st>>>(x.data_ptr<float>(), (const TY*)y.data_ptr(), y.stride(0), (const TR*)r.data_ptr(),
+                                                                               r.stride(0), w_post.data_ptr<float>(), wn, hp, (int)W, (float)eps);
   };
   dispatch_act(y, [&](auto* ty) {
     dispatch_act(r, [&](auto* tr) {
@@ -379,6 +386,41 @@ at::Tensor gated_norm_add_norm_f32_(at::Tensor x, const at::Tensor& y, const at:
       else go(ty, tr, (float*)nullptr);
     });
   });
+  return h;
+}
+
+at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
+                   const c10::optional<at::Tensor>& gate, int64_t experts);
+
+// gated_norm_add_norm_f32_ with y = the weighted sum of the routed experts' rows ye (moe_sum)
+at::Tensor gated_norm_add_experts_f32_(at::Tensor x, const at::Tensor& r, const at::Tensor& w_post, const c10::optional<at::Tensor>& w_next, double eps,
+                                       const at::Tensor& ye, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
+                                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts) {
+  HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kFloat, "x: contiguous fp32 [T, W]");
+  check_rows(r, "r");
+  const int64_t T = x.size(0), W = x.size(1);
+  HYB_CHECK(r.sizes() == x.sizes() && xin.sizes() == x.sizes(), "r and the experts' rows must have x's shape");
+  HYB_CHECK(f32w(w_post, W) && (!w_next.has_value() || f32w(*w_next, W)), "norm weights: fp32 [W]");
+  const ExpertRows m = expert_rows_of(ye, idx, wgt, xin, shared, gate, experts);
+  const float* wn = w_next.has_value() ? w_next->data_ptr<float>() : nullptr;
+  const bool quads = r.scalar_type() == at::kBFloat16 && W <= 16 * NT && quads_ok((const bf16_t*)r.data_ptr(), r.stride(0), W) &&
+                     quads_ok(x.data_ptr<float>(), W, W) && quads_ok(w_post.data_ptr<float>(), W, W) && (wn == nullptr || quads_ok(wn, W, W));
+  if (!quads) return gated_norm_add_norm_f32_(x, moe_sum(ye, idx, wgt, xin, shared, gate, experts), r, w_post, w_next, eps, true);
+  c10::DeviceGuard guard(x.device());
+  at::Tensor h = w_next.has_value() ? at::empty({T, W}, x.options().dtype(at::kBFloat16)) : at::empty({0}, x.options());
+  if (T == 0) return h;
+  auto go = [&](auto kern) {
+    kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(x.data_ptr<float>(), (const float*)nullptr, 0, (const bf16_t*)r.data_ptr(), r.stride(0), w_post.data_ptr<float>(), wn,
+                                                     wn != nullptr ? (bf16_t*)h.data_ptr() : (bf16_t*)nullptr, (int)W, (float)eps, m);
+  };
+  auto pick = [&](auto* tag) {
+    using Y = std::remove_pointer_t<decltype(tag)>;
+    if (W <= 4 * NT) go(gated_norm_add_norm_quads_kernel<float, bf16_t, bf16_t, 1, Y>);
+    else if (W <= 8 * NT) go(gated_norm_add_norm_quads_kernel<float, bf16_t, bf16_t, 2, Y>);
+    else go(gated_norm_add_norm_quads_kernel<float, bf16_t, bf16_t, 4, Y>);
+  };
+  if (ye.scalar_type() == at::kFloat) pick((float*)nullptr);
+  else pick((bf16_t*)nullptr);
   return h;
 }
 

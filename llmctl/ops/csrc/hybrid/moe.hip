@@ -19,7 +19,8 @@
 //     (gate and up: 2 x 16), its four waves split K; it finds its rows by scanning the choices itself, so no grouping pass
 //     runs.  Below two copies per expert, experts that no token chose are not read; from there on, where nearly every one has some, a wave
 //     asks for its first steps (8, or 4 from 33 tokens on) before it knows.
-//   * moe_combine_kernel: out_t = sum_k w_tk y_tk (+ w x_t for experts without weights) (+ the shared expert), fp32.
+//   * moe_combine_kernel: out_t = sum_k w_tk y_tk (+ w x_t for experts without weights) (+ the shared expert), fp32; where the
+//     result goes straight into the residual stream and a norm, their kernel sums instead (expert_rows.h).
 //
 // A row tile has 128 rows when the experts get 96 or more on average, else 64 (and 64 columns): below that the grid
 // of 128 x 128 tiles does not fill the chip and the K loop of every workgroup is a chain of load latencies.  The large tile
@@ -32,7 +33,7 @@
 //   router      9           9         10         10         10         10         10         10         12
 // up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from 2048 the LDS reads of 64 x 64 wave tiles and the
 // last round of tiles.  A layer of 2048 tokens took 700 us before (sort, per-expert GEMMs, copies), 16 tokens 350 us.
-#include "hybrid_common.h"
+#include "expert_rows.h"
 
 namespace llmctl_hybrid {
 namespace {
@@ -622,10 +623,9 @@ std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tens
   return {idx, wgt};
 }
 
-// sum_k wgt[t, k] expert_(idx[t, k])(x_t) (+ sigmoid(gate_t) shared_t), fp32 [T, W].  ``act``: 0 relu^2, 1 silu-gated (up weights
-// hold [gate ; up]), 2 gelu.  idx >= the number of experts: an expert that gives its input.
-at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
-                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate) {
+// Results of the chosen experts of every row of x, [T * top, W] by entry: fp32 for few tokens, else bf16.  ``act``: 0 relu^2, 1 silu-gated
+// (up weights hold [gate ; up]), 2 gelu.  idx >= the number of experts: an expert that gives its input, whose entries are not written.
+at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act) {
   int64_t E, R, W, E2, W2, ff;
   long ldu, ldd;
   const ExpertPtrs pu = expert_ptrs(up, E, R, W, ldu, "up"), pd = expert_ptrs(down, E2, W2, ff, ldd, "down");
@@ -636,18 +636,12 @@ at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Ten
   HYB_CHECK(idx.is_cuda() && idx.is_contiguous() && idx.scalar_type() == at::kInt && idx.dim() == 2 && idx.size(0) == T, "idx: int32 [T, top]");
   HYB_CHECK(wgt.is_cuda() && wgt.is_contiguous() && wgt.scalar_type() == at::kFloat && wgt.sizes() == idx.sizes(), "weights: fp32 [T, top]");
   HYB_CHECK(N < ((int64_t)1 << 30), "too many token copies");
-  if (shared.has_value())
-    HYB_CHECK(shared->is_cuda() && shared->dim() == 2 && shared->scalar_type() == at::kBFloat16 && shared->size(0) == T && shared->size(1) == W && rows16(*shared),
-              "shared: bf16 [T, W], aligned rows");
-  if (gate.has_value())
-    HYB_CHECK(shared.has_value() && gate->is_cuda() && gate->scalar_type() == at::kBFloat16 && gate->dim() == 2 && gate->size(0) == T, "gate: bf16 [T, 1]");
   c10::DeviceGuard guard(x.device());
   const hipStream_t st = cur_stream();
-  at::Tensor out = at::empty({T, W}, x.options().dtype(at::kFloat));
-  if (T == 0) return out;
   const bool small = T <= SMALL_ROWS;
-  at::Tensor a = at::empty({N, ff}, x.options());
   at::Tensor y = at::empty({N, W}, x.options().dtype(small ? at::kFloat : at::kBFloat16));
+  if (T == 0) return y;
+  at::Tensor a = at::empty({N, ff}, x.options());
   const bf16_t* xp = reinterpret_cast<const bf16_t*>(x.data_ptr());
   bf16_t* ap = reinterpret_cast<bf16_t*>(a.data_ptr());
   if (small) {
@@ -685,18 +679,51 @@ at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Ten
       moe_tile_kernel<64, 64, DOWN, 3, 2, 3><<<gd, 256, 0, st>>>(d);
     }
   }
-  const dim3 gc((unsigned)((T * (W / 8) + 255) / 256));
-  const bf16_t* sp = shared.has_value() ? reinterpret_cast<const bf16_t*>(shared->data_ptr()) : nullptr;
-  const bf16_t* gp = gate.has_value() ? reinterpret_cast<const bf16_t*>(gate->data_ptr()) : nullptr;
-  const long ls = shared.has_value() ? shared->stride(0) : 0, lg = gate.has_value() ? gate->stride(0) : 0;
+  return y;
+}
+
+ExpertRows expert_rows_of(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x,
+                          const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts) {
+  HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.scalar_type() == at::kBFloat16 && rows16(x), "x: bf16 [T, W], aligned rows");
+  const int64_t T = x.size(0), W = x.size(1);
+  HYB_CHECK(idx.is_cuda() && idx.is_contiguous() && idx.scalar_type() == at::kInt && idx.dim() == 2 && idx.size(0) == T, "idx: int32 [T, top]");
+  HYB_CHECK(wgt.is_cuda() && wgt.is_contiguous() && wgt.scalar_type() == at::kFloat && wgt.sizes() == idx.sizes(), "weights: fp32 [T, top]");
+  HYB_CHECK(y.is_cuda() && y.is_contiguous() && y.dim() == 2 && y.size(0) == idx.numel() && y.size(1) == W && W % 8 == 0 &&
+                (y.scalar_type() == at::kFloat || y.scalar_type() == at::kBFloat16) && reinterpret_cast<uintptr_t>(y.data_ptr()) % 16 == 0,
+            "experts' rows: contiguous fp32 or bf16 [T * top, W]");
+  if (shared.has_value())
+    HYB_CHECK(shared->is_cuda() && shared->dim() == 2 && shared->scalar_type() == at::kBFloat16 && shared->size(0) == T && shared->size(1) == W && rows16(*shared),
+              "shared: bf16 [T, W], aligned rows");
+  if (gate.has_value())
+    HYB_CHECK(shared.has_value() && gate->is_cuda() && gate->scalar_type() == at::kBFloat16 && gate->dim() == 2 && gate->size(0) == T, "gate: bf16 [T, 1]");
+  return ExpertRows{y.data_ptr(), idx.data_ptr<int>(), wgt.data_ptr<float>(), reinterpret_cast<const bf16_t*>(x.data_ptr()), (long)x.stride(0),
+                    shared.has_value() ? reinterpret_cast<const bf16_t*>(shared->data_ptr()) : nullptr, shared.has_value() ? (long)shared->stride(0) : 0,
+                    gate.has_value() ? reinterpret_cast<const bf16_t*>(gate->data_ptr()) : nullptr, gate.has_value() ? (long)gate->stride(0) : 0,
+                    (int)experts, (int)idx.size(1)};
+}
+
+// sum_k wgt[t, k] y[t, k] (+ sigmoid(gate_t) shared_t) of moe_expert_rows' results, fp32 [T, W]
+at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
+                   const c10::optional<at::Tensor>& gate, int64_t experts) {
+  const ExpertRows m = expert_rows_of(y, idx, wgt, x, shared, gate, experts);
+  const int64_t T = x.size(0), W = x.size(1);
+  c10::DeviceGuard guard(x.device());
+  at::Tensor out = at::empty({T, W}, x.options().dtype(at::kFloat));
+  if (T == 0) return out;
   auto sum = [&](auto* tag) {
     using Y = std::remove_pointer_t<decltype(tag)>;
-    moe_combine_kernel<Y><<<gc, 256, 0, st>>>(reinterpret_cast<const Y*>(y.data_ptr()), idx.data_ptr<int>(), wgt.data_ptr<float>(), xp,
-                                             (long)x.stride(0), sp, ls, gp, lg, out.data_ptr<float>(), (long)T, (int)W, (int)E, (int)top);
+    moe_combine_kernel<Y><<<dim3((unsigned)((T * (W / 8) + 255) / 256)), 256, 0, cur_stream()>>>(
+        static_cast<const Y*>(m.y), m.idx, m.wgt, m.x, m.ldx, m.shared, m.ld_shared, m.gate, m.ld_gate, out.data_ptr<float>(), (long)T, (int)W, m.E, m.top);
   };
-  if (small) sum((float*)nullptr);
+  if (y.scalar_type() == at::kFloat) sum((float*)nullptr);
   else sum((bf16_t*)nullptr);
   return out;
+}
+
+at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
+                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate) {
+  const at::Tensor y = moe_expert_rows(x, idx, wgt, up, down, act);
+  return moe_sum(y, idx, wgt, x, shared, gate, up.size() == 1 && up[0].dim() == 3 ? up[0].size(0) : (int64_t)up.size());
 }
 
 }  // namespace llmctl_hybrid

@@ -1,7 +1,7 @@
 // The fp32 residual stream of parallel layers and the small row-wise passes around the mixers:
 // LayerNorm (two-pass mean / variance), residual update fused with the next LayerNorm, RMS norm of a
 // column range, sigmoid gating, SwiGLU, per-head unit-RMS with weight and gate.
-#include "hybrid_common.h"
+#include "expert_rows.h"
 
 namespace llmctl_hybrid {
 
@@ -40,10 +40,13 @@ __global__ __launch_bounds__(NT) void add_layernorm_kernel(float* __restrict__ x
 
 // The same for rows of up to 4 * NT * VQ values in quads: all of a row's loads in flight at once, the row in registers from then on.  A decode
 // step's rows are a chain of latencies (16 rows of 2048: 8.9 us as above, 8 dependent loads deep, 4.4 so; 2048 rows 14.5 and 13.3).
-template <typename T, int VQ>
+// ``Y``: b is the weighted sum of the routed experts' rows of that type (expert_rows.h) instead of a tensor; as a pass of its own that sum
+// cost a launch and its own traffic (16 rows of 2048, two experts each: 4.7 + 4.7 us, together 5.0; 2048 rows 8.6 + 14.3, together 11.7).
+template <typename T, int VQ, typename Y = void>
 __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restrict__ x, const T* __restrict__ a, int64_t a_stride,
                                                                  const float* __restrict__ b, const float* __restrict__ w,
-                                                                 const float* __restrict__ bias, T* __restrict__ h, int W, float eps) {
+                                                                 const float* __restrict__ bias, T* __restrict__ h, int W, float eps,
+                                                                 ExpertRows m) {
   __shared__ float red[NW];
   const int64_t r = blockIdx.x;
   float4 v[VQ], av[VQ], bv[VQ], wv[VQ], cv[VQ];
@@ -52,9 +55,10 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
     const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
     v[i] = ld4(x + r * W + c);
     av[i] = a != nullptr ? ld4(a + r * a_stride + c) : make_float4(0.f, 0.f, 0.f, 0.f);
-    bv[i] = b != nullptr ? ld4(b + r * W + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (std::is_void_v<Y>) bv[i] = b != nullptr ? ld4(b + r * W + c) : make_float4(0.f, 0.f, 0.f, 0.f);
     if (h != nullptr) wv[i] = ld4(w + c), cv[i] = ld4(bias + c);
   }
+  if constexpr (!std::is_void_v<Y>) expert_sum_quads<Y, NT, VQ>(m, r, W, bv);
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
@@ -327,13 +331,13 @@ static at::Tensor out_like(const at::Tensor& ref, at::IntArrayRef shape, bool bf
 template <typename T>
 static void launch_add_layernorm(float* x, const T* a, int64_t a_st, const float* b, const float* w, const float* bias, T* h, int64_t rows, int W,
                                  double eps) {
-  auto go = [&](auto kern) { kern<<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps); };
+  auto go = [&](auto kern) { kern<<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps, ExpertRows{}); };
   const bool quads = W <= 16 * NT && quads_ok(x, W, W) && (a == nullptr || quads_ok(a, a_st, W)) && (b == nullptr || quads_ok(b, W, W)) &&
                      (h == nullptr || (quads_ok(w, W, W) && quads_ok(bias, W, W)));
   if (quads && W <= 4 * NT) go(add_layernorm_quads_kernel<T, 1>);
   else if (quads && W <= 8 * NT) go(add_layernorm_quads_kernel<T, 2>);
   else if (quads) go(add_layernorm_quads_kernel<T, 4>);
-  else go(add_layernorm_kernel<T>);
+  else add_layernorm_kernel<T><<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps);
 }
 
 at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, double eps, bool out_bf16) {
@@ -412,6 +416,45 @@ at::Tensor add_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::opti
     launch_add_layernorm<T>(x.data_ptr<float>(), (const T*)a.data_ptr(), a.stride(0), b.has_value() ? b->data_ptr<float>() : nullptr,
                             w.data_ptr<float>(), bias.data_ptr<float>(), (T*)h.data_ptr(), x.size(0), W, eps);
   });
+  return h;
+}
+
+at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
+                   const c10::optional<at::Tensor>& gate, int64_t experts);
+
+// add_layernorm_f32_ with b = the weighted sum of the routed experts' rows y (moe_sum); without w: the sum alone, no norm.
+at::Tensor add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
+                                      double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
+                                      const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts) {
+  check_add(x, a, c10::nullopt);
+  HYB_CHECK(a.scalar_type() == at::kBFloat16 && xin.sizes() == x.sizes() && w.has_value() == bias.has_value(), "routed experts: bf16 rows of x's shape; a norm has both vectors");
+  const int64_t T = x.size(0);
+  const int W = (int)x.size(1);
+  if (w.has_value())
+    HYB_CHECK(w->scalar_type() == at::kFloat && bias->scalar_type() == at::kFloat && w->numel() == W && bias->numel() == W && w->is_contiguous() && bias->is_contiguous(),
+              "norm weight / bias: fp32 [W]");
+  const ExpertRows m = expert_rows_of(y, idx, wgt, xin, shared, gate, experts);
+  c10::DeviceGuard guard(x.device());
+  at::Tensor h = w.has_value() ? out_like(x, x.sizes(), true) : at::empty({0}, x.options());
+  if (T == 0) return h;
+  const float *wp = w.has_value() ? w->data_ptr<float>() : nullptr, *bp = w.has_value() ? bias->data_ptr<float>() : nullptr;
+  bf16_t* hp = w.has_value() ? (bf16_t*)h.data_ptr() : nullptr;
+  const bf16_t* ap = (const bf16_t*)a.data_ptr();
+  float* xp = x.data_ptr<float>();
+  auto go = [&](auto kern) { kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(xp, ap, a.stride(0), nullptr, wp, bp, hp, W, (float)eps, m); };
+  auto pick = [&](auto* tag) {
+    using Y = std::remove_pointer_t<decltype(tag)>;
+    if (W <= 4 * NT) go(add_layernorm_quads_kernel<bf16_t, 1, Y>);
+    else if (W <= 8 * NT) go(add_layernorm_quads_kernel<bf16_t, 2, Y>);
+    else go(add_layernorm_quads_kernel<bf16_t, 4, Y>);
+  };
+  if (W <= 16 * NT && quads_ok(xp, W, W) && quads_ok(ap, a.stride(0), W) && (wp == nullptr || (quads_ok(wp, W, W) && quads_ok(bp, W, W)))) {
+    if (y.scalar_type() == at::kFloat) pick((float*)nullptr);
+    else pick((bf16_t*)nullptr);
+  } else {  // rows that the quads do not take
+    const at::Tensor b = moe_sum(y, idx, wgt, xin, shared, gate, experts);
+    launch_add_layernorm<bf16_t>(xp, ap, a.stride(0), b.data_ptr<float>(), wp, bp, hp, T, W, eps);
+  }
   return h;
 }
 

@@ -39,8 +39,24 @@ def embed_layernorm_f32(ids, table, scale: float, w, b, eps: float):
     return x, layernorm_f32(x, w, b, eps, table.dtype)
 
 
+class ExpertSum:
+    """The weighted sum of the routed experts' results (``routed_experts(..., late=True)``) that is still to be taken: the residual
+    updates below take it in their own pass; :meth:`total` is the sum as a tensor."""
+
+    def __init__(self, rows, idx, wgt, x, shared, gate, experts: int):
+        self.parts = (rows, idx, wgt, x, shared, gate, experts)
+
+    def total(self):
+        return native_hybrid().moe_sum(*self.parts)
+
+
 def residual_add_(x, a, b=None):
-    """``x += a (+ b)`` on the fp32 residual stream (a, b: any float dtype)."""
+    """``x += a (+ b)`` on the fp32 residual stream (a, b: any float dtype; b may be an :class:`ExpertSum`)."""
+    if isinstance(b, ExpertSum):
+        if a.dtype == torch.bfloat16:
+            native_hybrid().add_experts_layernorm_f32_(x, a, None, None, 0.0, *b.parts)
+            return x
+        b = b.total()
     if use_native(x):
         native_hybrid().residual_add_(x, a, b)
         return x
@@ -49,7 +65,11 @@ def residual_add_(x, a, b=None):
 
 def add_layernorm_f32_(x, a, b, w, bias, eps: float, out_dtype):
     """``x += a (+ b)`` in place, then LayerNorm(x) -> ``out_dtype``: the parallel layer's residual
-    update and the next layer's norm in one pass over the stream."""
+    update and the next layer's norm in one pass over the stream.  b may be an :class:`ExpertSum`."""
+    if isinstance(b, ExpertSum):
+        if a.dtype == out_dtype == torch.bfloat16:
+            return native_hybrid().add_experts_layernorm_f32_(x, a, w, bias, eps, *b.parts)
+        b = b.total()
     if use_native(x):
         return native_hybrid().add_layernorm_f32_(x, a, b, w, bias, eps, out_dtype == torch.bfloat16)
     ref.residual_add_(x, a, b)
@@ -304,7 +324,12 @@ def gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps: float, out_dtype):
     """A sublayer's result into the fp32 residual stream of a layer with norms on both sides and a
     gated residual, in one pass: ``g = y sigmoid(r)``; ``x += g / rms(g) * w_post`` in place; returns
     ``x / rms(x) * w_next`` -> ``out_dtype`` (the next sublayer's input), or None when ``w_next`` is None.
-    ``y`` and ``r`` are ``[T, W]`` in the activation dtype or fp32 (row-strided views allowed)."""
+    ``y`` and ``r`` are ``[T, W]`` in the activation dtype or fp32 (row-strided views allowed); y may be an :class:`ExpertSum`."""
+    if isinstance(y, ExpertSum):
+        if out_dtype == torch.bfloat16:
+            h = native_hybrid().gated_norm_add_experts_f32_(x, r, w_post, w_next, eps, *y.parts)
+            return h if w_next is not None else None
+        y = y.total()
     if use_native(x):
         h = native_hybrid().gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps, out_dtype == torch.bfloat16)
         return h if w_next is not None else None
@@ -496,15 +521,18 @@ def experts_pay(T: int, top: int, E: int, rows: int, width: int) -> bool:
 
 
 def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax: bool, renorm: bool, up, down, act: str, shared=None,
-                   gate=None):
+                   gate=None, late: bool = False):
     """``sum_k w_k expert_k(x_t)`` over the chosen experts of every row of ``x [T, W]`` (bf16) -> fp32 ``[T, W]``, all on the device:
     router (fp32 scores of the fp32 ``w_router [E, W]``; ``softmax``: :func:`bias_topk_router`'s choice, else
     :func:`group_topk_router`'s), copies grouped by expert, grouped products, weighted sum.  ``act``: ``relu2`` / ``gelu`` / ``swiglu``
     (``up`` holds ``[gate ; up]``).  Router outputs beyond the experts are experts that give their input.  ``shared [T, W]`` (times
-    ``sigmoid(gate [T, 1])`` if given) is added.  Operands: :func:`experts_ok`."""
+    ``sigmoid(gate [T, 1])`` if given) is added.  ``late``: an :class:`ExpertSum` instead of the sum.  Operands: :func:`experts_ok`."""
     nat = native_hybrid()
     idx, wgt = nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
-    return nat.moe_experts(x, idx, wgt, expert_list(up), expert_list(down), _EXPERT_ACTS[act], shared, gate)
+    ups = expert_list(up)
+    rows = nat.moe_expert_rows(x, idx, wgt, ups, expert_list(down), _EXPERT_ACTS[act])
+    out = ExpertSum(rows, idx, wgt, x, shared, gate, ups[0].shape[0] if ups[0].dim() == 3 else len(ups))
+    return out if late else out.total()
 
 
 def act_any(x, kind: str, scale=None):
