@@ -156,14 +156,16 @@ class LenitarLM(nn.Module):
         the paged latent pool or the state pools of layer i).  Returns the fp32 residual stream of
         ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer."""
         cfg, eps, dt = self.cfg, self.cfg.layer_norm_eps, self.dtype
-        x, h = hops.embed_layernorm_f32(b.ids, self.embed, cfg.embedding_scale, self.layers[0].norm_w, self.layers[0].norm_b, eps)  # fp32 stream
-        n = len(self.layers)
+        n, T = len(self.layers), b.ids.shape[0]
+        routers = [l.ff.few_router(T) if l.ff is not None and trail is None else None for l in self.layers]
+        x, h, routed = hops.embed_layernorm_route(b.ids, self.embed, cfg.embedding_scale, self.layers[0].norm_w, self.layers[0].norm_b, eps,
+                                                  routers[0])  # fp32 residual stream
         for i, layer in enumerate(self.layers):
             y = layer.mixer.step(h, b, cache.layer(i))
-            z = layer.ff(h, late=True) if layer.ff is not None else None
+            z = layer.ff(h, late=True, routed=routed) if layer.ff is not None else None
             if i + 1 < n and trail is None:
                 nxt = self.layers[i + 1]
-                h = hops.add_layernorm_f32_(x, y, z, nxt.norm_w, nxt.norm_b, eps, dt)
+                h, routed = hops.add_layernorm_route_(x, y, z, nxt.norm_w, nxt.norm_b, eps, dt, routers[i + 1])
             else:
                 hops.residual_add_(x, y, z)
                 if trail is not None:

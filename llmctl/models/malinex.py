@@ -215,9 +215,11 @@ class MalinexLM(nn.Module):
             layer = self.block(i)
             nxt = self.block(i + 1).norm1 if i + 1 < n else None
             y, r = layer.mixer.step(h, b, cache.layer(i))
-            h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm1b, layer.norm2 if layer.ff is not None else nxt, eps, dt)
+            experts = layer.ff if isinstance(layer.ff, BiasedSoftmaxMoE) else None
+            h, routed = hops.gated_norm_add_norm_route_(x, y, r, layer.norm1b, layer.norm2 if layer.ff is not None else nxt, eps, dt,
+                                                        experts.few_router(x.shape[0]) if experts is not None else None)
             if layer.ff is not None:
-                y, r = layer.ff(h, late=True) if isinstance(layer.ff, BiasedSoftmaxMoE) else layer.ff(h)
+                y, r = experts(h, late=True, routed=routed) if experts is not None else layer.ff(h)
                 h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm2b, nxt, eps, dt)
             if trail is not None:
                 trail.append(x.clone())

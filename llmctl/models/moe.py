@@ -224,16 +224,23 @@ class GroupLimitedMoE(nn.Module):
         return (hops.experts_pay(T, self.top, self.E, *up.shape)
                 and hops.experts_ok(up[:1], self.experts_up, self.experts_down, self.E, self.top, self.w_router))
 
-    def forward(self, x: torch.Tensor, late: bool = False):
-        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it)."""
+    def few_router(self, T: int):
+        """The router of a step of T rows for the kernel that norms them, or None: this layer routes them itself."""
+        from llmctl.ops import hybrid as hops
+
+        return (self.w_router, None, self.top, self.groups, self.keep, False, False) if T <= hops.ROUTED_ROWS and self.on_device(T) else None
+
+    def forward(self, x: torch.Tensor, late: bool = False, routed=None):
+        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it).  ``routed``: the rows' experts
+        and weights where their norm has found them (:meth:`few_router`)."""
         from llmctl.ops import hybrid as hops
 
         T = x.shape[0]
         if hops.experts_pay(T, self.top, self.E, 2 * self.ff, x.shape[1]):
             ups, downs = hops.expert_list(self.experts_up), hops.expert_list(self.experts_down)
-            if hops.experts_ok(x, ups, downs, self.E, self.top, self.w_router):
+            if routed or hops.experts_ok(x, ups, downs, self.E, self.top, self.w_router):
                 return hops.routed_experts(x, self.w_router, None, self.top, self.groups, self.keep, False, False, ups, downs, "swiglu",
-                                           **({"late": True} if late else {}))
+                                           **({"late": late, "routed": routed} if late else {}))
         topi, topw = hops.group_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.top,
                                             self.groups, self.keep)
         flat = topi.reshape(-1)
@@ -346,12 +353,24 @@ class BiasedSoftmaxMoE(nn.Module):
         """Whether a step of T rows runs without a host synchronisation."""
         from llmctl.ops import hybrid as hops
 
-        down = self.w_down.view(-1, self.E, self.ff).transpose(0, 1)
         return self._dense(T) or (hops.experts_pay(T, self.top, self.E, *self.w_up.shape[1:]) and hops.experts_ok(
-            self.w_up[0, :1], self.w_up, down, self.E + self.identity, self.top, self.w_router))
+            self.w_up[0, :1], self.w_up, self._down_list(), self.E + self.identity, self.top, self.w_router))
 
-    def forward(self, x: torch.Tensor, late: bool = False):
-        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it) (and the side columns)."""
+    def few_router(self, T: int):
+        """The router of a step of T rows for the kernel that norms them, or None: this layer routes them itself."""
+        from llmctl.ops import hybrid as hops
+
+        if T > hops.ROUTED_ROWS or not hops.experts_pay(T, self.top, self.E, self.up_rows, self.w_up.shape[2]) or not hops.experts_ok(
+                self.w_up[0, :1], self.w_up, self._down_list(), self.E + self.identity, self.top, self.w_router):
+            return None
+        return self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm
+
+    def _down_list(self):
+        return self.w_down.view(-1, self.E, self.ff).transpose(0, 1)  # [E, width, ff]
+
+    def forward(self, x: torch.Tensor, late: bool = False, routed=None):
+        """x [T, width] -> fp32 [T, width] (``late``: or a :class:`llmctl.ops.hybrid.ExpertSum` of it) (and the side columns).  ``routed``: the
+        rows' experts and weights where their norm has found them (:meth:`few_router`)."""
         from llmctl.ops import hybrid as hops
 
         from .mixers import _mm_f32
@@ -372,11 +391,11 @@ class BiasedSoftmaxMoE(nn.Module):
                 u = z[:, :self.sup_rows]
                 ys = hops.linear(u if fused else act(u), self.w_sdown)
         gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
-        down = self.w_down.view(x.shape[1], self.E, self.ff).transpose(0, 1)  # [E, width, ff]
-        if (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
-                and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
+        down = self._down_list()
+        if routed or (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
+                      and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
             out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
-                                      self.act, ys, gate, **({"late": True} if late else {}))
+                                      self.act, ys, gate, **({"late": late, "routed": routed} if late else {}))
             return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out
         topi, topw = hops.bias_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.bias, self.top,
                                            self.groups, self.keep, self.renorm)

@@ -4,8 +4,9 @@
 #include <ATen/ATen.h>
 
 namespace llmctl_hybrid {
-std::tuple<at::Tensor, at::Tensor> embed_layernorm_f32(const at::Tensor& ids, const at::Tensor& table, double scale, const at::Tensor& w,
-                                                       const at::Tensor& b, double eps);
+std::vector<at::Tensor> embed_layernorm_f32(const at::Tensor& ids, const at::Tensor& table, double scale, const at::Tensor& w, const at::Tensor& b, double eps,
+    const c10::optional<at::Tensor>& router, const c10::optional<at::Tensor>& rbias, int64_t top,
+    int64_t groups, int64_t keep, bool softmax, bool renorm);
 at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, double eps, bool out_bf16);
 void residual_add_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& b);
 at::Tensor add_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& b, const at::Tensor& w,
@@ -56,9 +57,12 @@ at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Ten
                        const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate);
 at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
                    const c10::optional<at::Tensor>& gate, int64_t experts);
-at::Tensor add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
-                                      double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
-                                      const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts);
+std::vector<at::Tensor> add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
+    double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin, const c10::optional<at::Tensor>& shared,
+    const c10::optional<at::Tensor>& gate, int64_t experts, const c10::optional<at::Tensor>& router, const c10::optional<at::Tensor>& rbias, int64_t top,
+    int64_t groups, int64_t keep, bool softmax, bool renorm);
+std::vector<at::Tensor> gated_norm_add_norm_route_(at::Tensor x, const at::Tensor& y, const at::Tensor& r, const at::Tensor& w_post, const at::Tensor& w_next,
+    double eps, const at::Tensor& router, const c10::optional<at::Tensor>& rbias, int64_t top, int64_t groups, int64_t keep, bool softmax, bool renorm);
 at::Tensor gated_norm_add_experts_f32_(at::Tensor x, const at::Tensor& r, const at::Tensor& w_post, const c10::optional<at::Tensor>& w_next, double eps,
                                        const at::Tensor& ye, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
                                        const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts);
@@ -135,7 +139,7 @@ at::Tensor rotary_f32(const at::Tensor& z, int64_t nq, int64_t nk, int64_t dk, c
 }  // namespace llmctl_hybrid
 
 TORCH_LIBRARY(llmctl_hybrid, m) {
-  m.def("embed_layernorm_f32(Tensor ids, Tensor table, float scale, Tensor w, Tensor b, float eps) -> (Tensor, Tensor)");
+  m.def("embed_layernorm_f32(Tensor ids, Tensor table, float scale, Tensor w, Tensor b, float eps, Tensor? router=None, Tensor? rbias=None, int top=0, int groups=1, int keep=1, bool softmax=False, bool renorm=False) -> Tensor[]");
   m.def("layernorm_f32(Tensor x, Tensor w, Tensor b, float eps, bool out_bf16) -> Tensor");
   m.def("residual_add_(Tensor(a!) x, Tensor a, Tensor? b) -> ()");
   m.def("add_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? b, Tensor w, Tensor bias, float eps, bool out_bf16) -> Tensor");
@@ -169,7 +173,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("moe_expert_rows(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act) -> Tensor");
   m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
   m.def("moe_sum(Tensor y, Tensor idx, Tensor wgt, Tensor x, Tensor? shared, Tensor? gate, int experts) -> Tensor");
-  m.def("add_experts_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? w, Tensor? bias, float eps, Tensor y, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts) -> Tensor");
+  m.def("add_experts_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? w, Tensor? bias, float eps, Tensor y, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts, Tensor? router=None, Tensor? rbias=None, int top=0, int groups=1, int keep=1, bool softmax=False, bool renorm=False) -> Tensor[]");
+  m.def("gated_norm_add_norm_route_(Tensor(a!) x, Tensor y, Tensor r, Tensor w_post, Tensor w_next, float eps, Tensor router, Tensor? rbias, int top, int groups, int keep, bool softmax, bool renorm) -> Tensor[]");
   m.def("gated_norm_add_experts_f32_(Tensor(a!) x, Tensor r, Tensor w_post, Tensor? w_next, float eps, Tensor ye, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts) -> Tensor");
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
   m.def("qk_fullnorm_prep(Tensor z, int H, int G, int dk, int dv, Tensor q_norm, Tensor k_norm, float eps, Tensor pos, float temp_coef, int temp_every, Tensor(a!) cache, Tensor slots, Tensor? freq=None, int rot=0, bool interleaved=False, float amp=1.0) -> Tensor");
@@ -226,6 +231,7 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("moe_experts", &llmctl_hybrid::moe_experts);
   m.impl("moe_sum", &llmctl_hybrid::moe_sum);
   m.impl("add_experts_layernorm_f32_", &llmctl_hybrid::add_experts_layernorm_f32_);
+  m.impl("gated_norm_add_norm_route_", &llmctl_hybrid::gated_norm_add_norm_route_);
   m.impl("gated_norm_add_experts_f32_", &llmctl_hybrid::gated_norm_add_experts_f32_);
   m.impl("act_any", &llmctl_hybrid::act_any);
   m.impl("qk_fullnorm_prep", &llmctl_hybrid::qk_fullnorm_prep);

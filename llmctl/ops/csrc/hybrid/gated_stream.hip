@@ -7,6 +7,7 @@
 //   glu_act                   act(gate) * up of rows [gate | up] (silu or the tanh GELU), times an optional factor per row
 // All arithmetic fp32; y, r, h in the activation dtype or fp32.
 #include "expert_rows.h"
+#include "router_rows.h"
 
 namespace llmctl_hybrid {
 
@@ -68,11 +69,12 @@ __global__ __launch_bounds__(NT) void gated_norm_add_norm_kernel(float* __restri
 // rows: 10.5 us as above, 4.5 so; 2911 rows 27.3 and 18.4).
 // ``Y``: y is the weighted sum of the routed experts' rows of that type (expert_rows.h) instead of a tensor (16 rows, two experts each and a shared
 // one: 4.7 us for the sum and 4.7 here, together 4.9; 2911 rows 12.8 + 17.1, together 19.0).
-template <typename TY, typename TR, typename TH, int VQ, typename Y = void>
+// ``ROUTE``: h goes through a router too (router_rows.h).
+template <typename TY, typename TR, typename TH, int VQ, typename Y = void, bool ROUTE = false>
 __global__ __launch_bounds__(NT) void gated_norm_add_norm_quads_kernel(float* __restrict__ x, const TY* __restrict__ y, int64_t y_st,
                                                                        const TR* __restrict__ r, int64_t r_st, const float* __restrict__ wp,
                                                                        const float* __restrict__ wn, TH* __restrict__ h, int W, float eps,
-                                                                       ExpertRows m) {
+                                                                       ExpertRows m, RouteOut route) {
   __shared__ float red[NW];
   const int64_t row = blockIdx.x;
   float4 g[VQ], rv[VQ], xv[VQ], pv[VQ], nv[VQ];
@@ -109,10 +111,14 @@ __global__ __launch_bounds__(NT) void gated_norm_add_norm_quads_kernel(float* __
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
-    if (c < W) st4(h + row * W + c, make_float4(g[i].x * rstd2 * nv[i].x, g[i].y * rstd2 * nv[i].y, g[i].z * rstd2 * nv[i].z, g[i].w * rstd2 * nv[i].w));
+    g[i] = make_float4(g[i].x * rstd2 * nv[i].x, g[i].y * rstd2 * nv[i].y, g[i].z * rstd2 * nv[i].z, g[i].w * rstd2 * nv[i].w);
+    if (c < W) st4(h + row * W + c, g[i]);
   }
+  if constexpr (ROUTE) route.row<NW, VQ>(g, row, W);
 }
 
+// A thread's first KEEP columns are all asked for before the first is used (one after another 16 rows of 2048 took 9.7 us, so 4.9; 2911 rows 24.9 and
+// 18.3).  The columns stay with their threads, and so the order of the sum, on which near ties of the first layer's experts hang.
 template <typename T>
 __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pos,
                                                            const T* __restrict__ table, const T* __restrict__ ptable, const float* __restrict__ w,
@@ -121,50 +127,35 @@ __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __rest
   const int64_t row = blockIdx.x;
   const T* e = table + ids[row] * (int64_t)W;
   const T* p = ptable + (int64_t)pos[row] * W;
-  float q = 0.f;
-  for (int c = threadIdx.x; c < W; c += NT) {
-    const float v = ldf(e + c) + ldf(p + c);
-    x[row * W + c] = v;
-    q += v * v;
-  }
-  const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
-  for (int c = threadIdx.x; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
-}
-
-// The same in quads, all of a row's loads in flight at once (16 rows of 2048: 9.7 us as above, 5.5 so; 2911 rows 24.9 and 16.6).
-template <typename T, int VQ>
-__global__ __launch_bounds__(NT) void embed_rmsnorm_quads_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pos,
-                                                                 const T* __restrict__ table, const T* __restrict__ ptable,
-                                                                 const float* __restrict__ w, float* __restrict__ x, T* __restrict__ h, int W,
-                                                                 float eps) {
-  __shared__ float red[NW];
-  const int64_t row = blockIdx.x;
-  const T* e = table + ids[row] * (int64_t)W;
-  const T* p = ptable + (int64_t)pos[row] * W;
-  float4 v[VQ], pv[VQ], wv[VQ];
+  float v[KEEP], pv[KEEP], wv[KEEP];
 #pragma unroll
-  for (int i = 0; i < VQ; ++i) {
-    const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
-    v[i] = ld4(e + c);
-    pv[i] = ld4(p + c);
-    wv[i] = ld4(w + c);
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = min((int)(threadIdx.x + i * NT), W - 1);
+    v[i] = ldf(e + c);
+    pv[i] = ldf(p + c);
+    wv[i] = w[c];
   }
   float q = 0.f;
 #pragma unroll
-  for (int i = 0; i < VQ; ++i) {
-    const int c = (int)(threadIdx.x + i * NT) * 4;
-    v[i].x += pv[i].x, v[i].y += pv[i].y, v[i].z += pv[i].z, v[i].w += pv[i].w;
-    if (c < W) {
-      st4(x + row * W + c, v[i]);
-      q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
-    }
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c >= W) break;
+    v[i] += pv[i];
+    x[row * W + c] = v[i];
+    q += v[i] * v[i];
+  }
+  for (int c = threadIdx.x + KEEP * NT; c < W; c += NT) {
+    const float u = ldf(e + c) + ldf(p + c);
+    x[row * W + c] = u;
+    q += u * u;
   }
   const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
 #pragma unroll
-  for (int i = 0; i < VQ; ++i) {
-    const int c = (int)(threadIdx.x + i * NT) * 4;
-    if (c < W) st4(h + row * W + c, make_float4(v[i].x * rstd * wv[i].x, v[i].y * rstd * wv[i].y, v[i].z * rstd * wv[i].z, v[i].w * rstd * wv[i].w));
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < W) stf(h + row * W + c, v[i] * rstd * wv[i]);
   }
+  for (int c = threadIdx.x + KEEP * NT; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
 }
 
 template <int KIND>
@@ -369,7 +360,7 @@ at::Tensor gated_norm_add_norm_f32_(at::Tensor x, const at::Tensor& y, const at:
     TH* hp = wn != nullptr ? (TH*)h.data_ptr() : nullptr;
     auto launch = [&](auto kern) {
       kern<<<dim3((unsigned)T), NT, 0, st>>>(x.data_ptr<float>(), (const TY*)y.data_ptr(), y.stride(0), (const TR*)r.data_ptr(), r.stride(0),
-                                             w_post.data_ptr<float>(), wn, hp, (int)W, (float)eps, ExpertRows{});
+                                             w_post.data_ptr<float>(), wn, hp, (int)W, (float)eps, ExpertRows{}, RouteOut{});
     };
     const bool quads = W <= 16 * NT && quads_ok((const TY*)y.data_ptr(), y.stride(0), W) && quads_ok((const TR*)r.data_ptr(), r.stride(0), W) &&
                        quads_ok(x.data_ptr<float>(), W, W) && quads_ok(w_post.data_ptr<float>(), W, W) && (wn == nullptr || quads_ok(wn, W, W));
@@ -387,6 +378,40 @@ at::Tensor gated_norm_add_norm_f32_(at::Tensor x, const at::Tensor& y, const at:
     });
   });
   return h;
+}
+
+// gated_norm_add_norm_f32_ on bf16 rows, and the router of its result: h, the chosen experts and their weights.
+std::vector<at::Tensor> gated_norm_add_norm_route_(at::Tensor x, const at::Tensor& y, const at::Tensor& r, const at::Tensor& w_post, const at::Tensor& w_next,
+                                                   double eps, const at::Tensor& router, const c10::optional<at::Tensor>& rbias, int64_t top, int64_t groups,
+                                                   int64_t keep, bool softmax, bool renorm) {
+  HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kFloat, "x: contiguous fp32 [T, W]");
+  check_rows(y, "y");
+  check_rows(r, "r");
+  const int64_t T = x.size(0), W = x.size(1);
+  HYB_CHECK(y.sizes() == x.sizes() && r.sizes() == x.sizes(), "y and r must have x's shape");
+  HYB_CHECK(f32w(w_post, W) && f32w(w_next, W), "norm weights: fp32 [W]");
+  const bool quads = y.scalar_type() == at::kBFloat16 && r.scalar_type() == at::kBFloat16 && W <= 16 * NT && quads_ok((const bf16_t*)y.data_ptr(), y.stride(0), W) &&
+                     quads_ok((const bf16_t*)r.data_ptr(), r.stride(0), W) && quads_ok(x.data_ptr<float>(), W, W) && quads_ok(w_post.data_ptr<float>(), W, W) &&
+                     quads_ok(w_next.data_ptr<float>(), W, W);
+  std::vector<at::Tensor> out;
+  if (!quads) {
+    out.push_back(gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps, true));
+    add_routed(out, out[0], router, rbias, top, groups, keep, softmax, renorm);
+    return out;
+  }
+  c10::DeviceGuard guard(x.device());
+  out.push_back(at::empty({T, W}, x.options().dtype(at::kBFloat16)));
+  const RouteOut route = route_out(router, W, rbias, top, groups, keep, softmax, renorm, T, out);
+  if (T == 0) return out;
+  auto go = [&](auto kern) {
+    kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(x.data_ptr<float>(), (const bf16_t*)y.data_ptr(), y.stride(0), (const bf16_t*)r.data_ptr(), r.stride(0),
+                                                     w_post.data_ptr<float>(), w_next.data_ptr<float>(), (bf16_t*)out[0].data_ptr(), (int)W, (float)eps,
+                                                     ExpertRows{}, route);
+  };
+  if (W <= 4 * NT) go(gated_norm_add_norm_quads_kernel<bf16_t, bf16_t, bf16_t, 1, void, true>);
+  else if (W <= 8 * NT) go(gated_norm_add_norm_quads_kernel<bf16_t, bf16_t, bf16_t, 2, void, true>);
+  else go(gated_norm_add_norm_quads_kernel<bf16_t, bf16_t, bf16_t, 4, void, true>);
+  return out;
 }
 
 at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
@@ -411,7 +436,7 @@ at::Tensor gated_norm_add_experts_f32_(at::Tensor x, const at::Tensor& r, const 
   if (T == 0) return h;
   auto go = [&](auto kern) {
     kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(x.data_ptr<float>(), (const float*)nullptr, 0, (const bf16_t*)r.data_ptr(), r.stride(0), w_post.data_ptr<float>(), wn,
-                                                     wn != nullptr ? (bf16_t*)h.data_ptr() : (bf16_t*)nullptr, (int)W, (float)eps, m);
+                                                     wn != nullptr ? (bf16_t*)h.data_ptr() : (bf16_t*)nullptr, (int)W, (float)eps, m, RouteOut{});
   };
   auto pick = [&](auto* tag) {
     using Y = std::remove_pointer_t<decltype(tag)>;
@@ -440,16 +465,9 @@ std::tuple<at::Tensor, at::Tensor> embed_rmsnorm_f32(const at::Tensor& ids, cons
   if (T == 0) return {x, h};
   dispatch_act(table, [&](auto* tag) {
     using Tt = std::remove_pointer_t<decltype(tag)>;
-    const Tt *tp = (const Tt*)table.data_ptr(), *pp = (const Tt*)pos_table.data_ptr();
-    auto go = [&](auto kern) {
-      kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), tp, pp, w.data_ptr<float>(), x.data_ptr<float>(),
-                                                       (Tt*)h.data_ptr(), (int)W, (float)eps);
-    };
-    const bool quads = W <= 16 * NT && quads_ok(tp, W, W) && quads_ok(pp, W, W) && quads_ok(w.data_ptr<float>(), W, W);
-    if (quads && W <= 4 * NT) go(embed_rmsnorm_quads_kernel<Tt, 1>);
-    else if (quads && W <= 8 * NT) go(embed_rmsnorm_quads_kernel<Tt, 2>);
-    else if (quads) go(embed_rmsnorm_quads_kernel<Tt, 4>);
-    else go(embed_rmsnorm_kernel<Tt>);
+    embed_rmsnorm_kernel<Tt><<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), (const Tt*)table.data_ptr(),
+                                                                        (const Tt*)pos_table.data_ptr(), w.data_ptr<float>(), x.data_ptr<float>(),
+                                                                        (Tt*)h.data_ptr(), (int)W, (float)eps);
   });
   return {x, h};
 }

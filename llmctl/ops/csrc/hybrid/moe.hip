@@ -7,7 +7,7 @@
 // the bottom of this comment, with the sizes.
 //
 //   * moe_route_kernel: 16 tokens per workgroup, logits on the fp32 matrix cores, scores and choice in the same kernel: no
-//     logits tensor, no fp32 copy of the rows.
+//     logits tensor, no fp32 copy of the rows.  Steps of up to 64 tokens whose norm is at hand are routed there (router_rows.h).
 //   * moe_group_kernel: one workgroup per expert scans the choices twice (histogram, then ballot prefix): a stable counting
 //     sort, and the list of row tiles that the grouped product walks.
 //   * moe_tile_kernel: BM x BN tiles of one expert's rows, K in 64-deep steps through LDS, the global loads of the next step
@@ -34,6 +34,7 @@
 // up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from 2048 the LDS reads of 64 x 64 wave tiles and the
 // last round of tiles.  A layer of 2048 tokens took 700 us before (sort, per-expert GEMMs, copies), 16 tokens 350 us.
 #include "expert_rows.h"
+#include "router_rows.h"
 
 namespace llmctl_hybrid {
 namespace {
@@ -41,7 +42,7 @@ namespace {
 using bfrag = __attribute__((ext_vector_type(8))) __bf16;
 using facc = __attribute__((ext_vector_type(4))) float;
 
-constexpr int MAX_EXPERTS = 128;  // pointers travel as kernel arguments
+constexpr int MAX_EXPERTS = MAX_ROUTED;  // pointers travel as kernel arguments
 constexpr int SMALL_ROWS = 64;    // tokens of a step that take the weight-streaming form
 
 struct ExpertPtrs {
@@ -78,15 +79,6 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
 }
 
 // ------------------------------------------------------------------------------------------------ router
-// The lowest index of the largest of up to 128 values, two per lane (indices lane and lane + 64), among those with ``in``; the
-// lowest index with ``in`` where no value compares (NaN).  At least one must have it.
-__device__ __forceinline__ int wave_argmax2(const float (&v)[2], const bool (&in)[2]) {
-  const float m = wave_max(fmaxf(in[0] ? v[0] : -INFINITY, in[1] ? v[1] : -INFINITY));
-  unsigned long long m0 = __ballot(in[0] && v[0] == m), m1 = __ballot(in[1] && v[1] == m);
-  if (!(m0 | m1)) m0 = __ballot(in[0]), m1 = __ballot(in[1]);
-  return m0 ? __ffsll(m0) - 1 : 63 + __ffsll(m1);
-}
-
 // 16 tokens per workgroup on the fp32 matrix cores (bf16 rows are exact in fp32): lane (r, kg) loads eight neighbouring k of
 // token r and of router output r, and MFMA step j multiplies element j of every lane's eight, so four k that lie 8 apart.  The sixteen
 // waves take every sixteenth 32-deep block of the row, four of their blocks in flight; then every wave chooses for one token, its
@@ -94,9 +86,8 @@ __device__ __forceinline__ int wave_argmax2(const float (&v)[2], const bool (&in
 // 22 us for 2048 and 43 us for 4096, where this one takes 10 and 12.)
 constexpr int ROUTE_T = 16, ROUTE_WAVES = 16;
 __global__ __launch_bounds__(ROUTE_WAVES * 64) void moe_route_kernel(const bf16_t* __restrict__ x, long ldx, const float* __restrict__ w,
-                                                                     const float* __restrict__ bias, int* __restrict__ idx,
-                                                                     float* __restrict__ wgt, int T, int W, int E, int top, int G, int keep,
-                                                                     int softmax, int renorm) {
+                                                                     RouterChoice c, int* __restrict__ idx, float* __restrict__ wgt, int T, int W) {
+  const int E = c.E;
   constexpr int U = 4;
   __shared__ facc part[ROUTE_WAVES][4][ROUTE_T];  // [wave][outputs 4 kg ..][token]
   __shared__ float logits[ROUTE_T][MAX_EXPERTS];
@@ -145,72 +136,7 @@ __global__ __launch_bounds__(ROUTE_WAVES * 64) void moe_route_kernel(const bf16_
     __syncthreads();
   }
   for (int t = wave; t < ROUTE_T && t0 + t < T; t += ROUTE_WAVES) {
-    float* lg = logits[t];
-    // lane holds router outputs lane and lane + 64
-    float p[2], s[2];
-    bool in[2];  // may still be chosen
-    float mx = 0.f, inv = 1.f;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) p[h] = lane + 64 * h < E ? lg[lane + 64 * h] : -INFINITY;
-    if (softmax) {
-      mx = wave_max(fmaxf(p[0], p[1]));
-      inv = 1.0f / wave_sum(expf(p[0] - mx) + expf(p[1] - mx));
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int e = lane + 64 * h;
-      in[h] = e < E;
-      p[h] = softmax ? expf(p[h] - mx) * inv : 1.0f / (1.0f + expf(-p[h]));
-      s[h] = p[h] + (bias != nullptr && in[h] ? bias[e] : 0.f);
-      if (in[h]) lg[e] = s[h];
-    }
-    if (G > 1) {
-      // a group's score: the sum of its two best (sigmoid router) or its best choice score; the ``keep`` best groups stay open
-      const int per = E / G;
-      float gs[2];
-      bool gin[2];
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int gi = lane + 64 * h;
-        gin[h] = gi < G;
-        float a = -INFINITY, b = -INFINITY;
-        if (gin[h])
-          for (int e = gi * per; e < (gi + 1) * per; ++e) {
-            const float v = lg[e];
-            b = fmaxf(b, fminf(a, v));
-            a = fmaxf(a, v);
-          }
-        gs[h] = softmax || per == 1 ? a : a + b;
-      }
-      unsigned long long open[2] = {0ull, 0ull};
-      for (int kk = 0; kk < keep; ++kk) {
-        const int best = wave_argmax2(gs, gin);
-        if (best < 64) open[0] |= 1ull << best;
-        else open[1] |= 1ull << (best - 64);
-#pragma unroll
-        for (int h = 0; h < 2; ++h) gin[h] = gin[h] && best != lane + 64 * h;
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int gi = min((lane + 64 * h) / per, G - 1);
-        in[h] = in[h] && (((gi < 64 ? open[0] >> gi : open[1] >> (gi - 64)) & 1ull) != 0ull);
-      }
-    }
-    float sum = 0.f, minew = 0.f;
-    int mine = 0;
-    for (int kk = 0; kk < top; ++kk) {  // top <= 64: lane kk keeps choice kk
-      const int best = wave_argmax2(s, in);
-      const float pw = __shfl(best < 64 ? p[0] : p[1], best & 63);
-      sum += pw;
-      if (lane == kk) mine = best, minew = pw;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) in[h] = in[h] && best != lane + 64 * h;
-    }
-    if (lane < top) {
-      idx[(long)(t0 + t) * top + lane] = mine;
-      wgt[(long)(t0 + t) * top + lane] = renorm ? minew * (1.0f / (sum + 1e-20f)) : minew;
-    }
+    choose_experts(logits[t], lane, c, idx + (long)(t0 + t) * c.top, wgt + (long)(t0 + t) * c.top);
   }
 }
 
@@ -603,23 +529,28 @@ bool rows16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr
 
 }  // namespace
 
+RouterChoice router_choice(const at::Tensor& w, int64_t W, const c10::optional<at::Tensor>& bias, int64_t top, int64_t groups, int64_t keep, bool softmax,
+                           bool renorm) {
+  HYB_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous() && w.scalar_type() == at::kFloat && w.size(1) == W && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+            "router: contiguous fp32 [E, W]");
+  const int64_t E = w.size(0);
+  HYB_CHECK(E >= 1 && E <= MAX_EXPERTS && top >= 1 && top <= E && top <= 64, "1 .. 128 router outputs, top in 1 .. min(E, 64)");
+  HYB_CHECK(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (E / groups), "experts split into equal groups; top fits the kept groups");
+  if (bias.has_value()) HYB_CHECK(bias->is_cuda() && bias->is_contiguous() && bias->scalar_type() == at::kFloat && bias->numel() == E, "bias: fp32 [E]");
+  return RouterChoice{bias.has_value() ? bias->data_ptr<float>() : nullptr, (int)E, (int)top, (int)groups, (int)keep, softmax ? 1 : 0, renorm ? 1 : 0};
+}
+
 // The chosen experts (int32 [T, top]) and their weights (fp32 [T, top]) of rows x [T, W] under the fp32 router weight [E, W].
 std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t top,
                                              int64_t groups, int64_t keep, bool softmax, bool renorm) {
   HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.scalar_type() == at::kBFloat16 && x.size(1) % 8 == 0 && rows16(x), "x: bf16 [T, W], aligned rows");
-  HYB_CHECK(w.is_cuda() && w.dim() == 2 && w.is_contiguous() && w.scalar_type() == at::kFloat && w.size(1) == x.size(1) &&
-                reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
-            "router: contiguous fp32 [E, W]");
-  const int64_t T = x.size(0), W = x.size(1), E = w.size(0);
-  HYB_CHECK(E >= 1 && E <= MAX_EXPERTS && top >= 1 && top <= E && top <= 64, "1 .. 128 router outputs, top in 1 .. min(E, 64)");
-  HYB_CHECK(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (E / groups), "experts split into equal groups; top fits the kept groups");
-  if (bias.has_value()) HYB_CHECK(bias->is_cuda() && bias->is_contiguous() && bias->scalar_type() == at::kFloat && bias->numel() == E, "bias: fp32 [E]");
+  const RouterChoice c = router_choice(w, x.size(1), bias, top, groups, keep, softmax, renorm);
+  const int64_t T = x.size(0), W = x.size(1);
   c10::DeviceGuard guard(x.device());
   at::Tensor idx = at::empty({T, top}, x.options().dtype(at::kInt)), wgt = at::empty({T, top}, x.options().dtype(at::kFloat));
   if (T == 0) return {idx, wgt};
   moe_route_kernel<<<dim3((unsigned)((T + ROUTE_T - 1) / ROUTE_T)), ROUTE_WAVES * 64, 0, cur_stream()>>>(
-      reinterpret_cast<const bf16_t*>(x.data_ptr()), x.stride(0), w.data_ptr<float>(), bias.has_value() ? bias->data_ptr<float>() : nullptr,
-      idx.data_ptr<int>(), wgt.data_ptr<float>(), (int)T, (int)W, (int)E, (int)top, (int)groups, (int)keep, softmax ? 1 : 0, renorm ? 1 : 0);
+      reinterpret_cast<const bf16_t*>(x.data_ptr()), x.stride(0), w.data_ptr<float>(), c, idx.data_ptr<int>(), wgt.data_ptr<float>(), (int)T, (int)W);
   return {idx, wgt};
 }
 

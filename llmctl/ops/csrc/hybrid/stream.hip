@@ -2,6 +2,7 @@
 // LayerNorm (two-pass mean / variance), residual update fused with the next LayerNorm, RMS norm of a
 // column range, sigmoid gating, SwiGLU, per-head unit-RMS with weight and gate.
 #include "expert_rows.h"
+#include "router_rows.h"
 
 namespace llmctl_hybrid {
 
@@ -42,11 +43,12 @@ __global__ __launch_bounds__(NT) void add_layernorm_kernel(float* __restrict__ x
 // step's rows are a chain of latencies (16 rows of 2048: 8.9 us as above, 8 dependent loads deep, 4.4 so; 2048 rows 14.5 and 13.3).
 // ``Y``: b is the weighted sum of the routed experts' rows of that type (expert_rows.h) instead of a tensor; as a pass of its own that sum
 // cost a launch and its own traffic (16 rows of 2048, two experts each: 4.7 + 4.7 us, together 5.0; 2048 rows 8.6 + 14.3, together 11.7).
-template <typename T, int VQ, typename Y = void>
+// ``ROUTE``: the rows go through a router too (router_rows.h).
+template <typename T, int VQ, typename Y = void, bool ROUTE = false>
 __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restrict__ x, const T* __restrict__ a, int64_t a_stride,
                                                                  const float* __restrict__ b, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, T* __restrict__ h, int W, float eps,
-                                                                 ExpertRows m) {
+                                                                 ExpertRows m, RouteOut route) {
   __shared__ float red[NW];
   const int64_t r = blockIdx.x;
   float4 v[VQ], av[VQ], bv[VQ], wv[VQ], cv[VQ];
@@ -82,18 +84,19 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
-    if (c < W)
-      st4(h + r * W + c, make_float4(v[i].x * rstd * wv[i].x + cv[i].x, v[i].y * rstd * wv[i].y + cv[i].y, v[i].z * rstd * wv[i].z + cv[i].z,
-                                     v[i].w * rstd * wv[i].w + cv[i].w));
+    v[i] = make_float4(v[i].x * rstd * wv[i].x + cv[i].x, v[i].y * rstd * wv[i].y + cv[i].y, v[i].z * rstd * wv[i].z + cv[i].z,
+                       v[i].w * rstd * wv[i].w + cv[i].w);
+    if (c < W) st4(h + r * W + c, v[i]);
   }
+  if constexpr (ROUTE) route.row<NW, VQ>(v, r, W);
 }
 
 // The first of a step: x = table[id] * scale, h = LayerNorm(x) * w + bias; the product in fp32, as a cast and a multiplication give it.  One
 // launch for the gather, the cast, the scale and the norm (16 rows of 2048: four launches, 27.1 us -> 6.5; 2048 rows 27.4 -> 13.0).
-template <typename T, int VQ>
+template <typename T, int VQ, bool ROUTE>
 __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t* __restrict__ ids, const T* __restrict__ table, int64_t rows,
                                                                    float scale, const float* __restrict__ w, const float* __restrict__ bias,
-                                                                   float* __restrict__ x, T* __restrict__ h, int W, float eps) {
+                                                                   float* __restrict__ x, T* __restrict__ h, int W, float eps, RouteOut route) {
   __shared__ float red[NW];
   const int64_t r = blockIdx.x, id = ids[r];
   CUDA_KERNEL_ASSERT(id >= 0 && id < rows);
@@ -126,10 +129,11 @@ __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
-    if (c < W)
-      st4(h + r * W + c, make_float4(v[i].x * rstd * wv[i].x + cv[i].x, v[i].y * rstd * wv[i].y + cv[i].y, v[i].z * rstd * wv[i].z + cv[i].z,
-                                     v[i].w * rstd * wv[i].w + cv[i].w));
+    v[i] = make_float4(v[i].x * rstd * wv[i].x + cv[i].x, v[i].y * rstd * wv[i].y + cv[i].y, v[i].z * rstd * wv[i].z + cv[i].z,
+                       v[i].w * rstd * wv[i].w + cv[i].w);
+    if (c < W) st4(h + r * W + c, v[i]);
   }
+  if constexpr (ROUTE) route.row<NW, VQ>(v, r, W);
 }
 
 // Rows that the quads do not take: x alone, its LayerNorm by add_layernorm_kernel.
@@ -331,7 +335,7 @@ static at::Tensor out_like(const at::Tensor& ref, at::IntArrayRef shape, bool bf
 template <typename T>
 static void launch_add_layernorm(float* x, const T* a, int64_t a_st, const float* b, const float* w, const float* bias, T* h, int64_t rows, int W,
                                  double eps) {
-  auto go = [&](auto kern) { kern<<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps, ExpertRows{}); };
+  auto go = [&](auto kern) { kern<<<dim3((unsigned)rows), NT, 0, cur_stream()>>>(x, a, a_st, b, w, bias, h, W, (float)eps, ExpertRows{}, RouteOut{}); };
   const bool quads = W <= 16 * NT && quads_ok(x, W, W) && (a == nullptr || quads_ok(a, a_st, W)) && (b == nullptr || quads_ok(b, W, W)) &&
                      (h == nullptr || (quads_ok(w, W, W) && quads_ok(bias, W, W)));
   if (quads && W <= 4 * NT) go(add_layernorm_quads_kernel<T, 1>);
@@ -354,34 +358,50 @@ at::Tensor layernorm_f32(const at::Tensor& x, const at::Tensor& w, const at::Ten
   return h;
 }
 
-std::tuple<at::Tensor, at::Tensor> embed_layernorm_f32(const at::Tensor& ids, const at::Tensor& table, double scale, const at::Tensor& w,
-                                                       const at::Tensor& b, double eps) {
+// x and h; with a router (bf16 rows) the chosen experts of every row of h and their weights too.
+std::vector<at::Tensor> embed_layernorm_f32(const at::Tensor& ids, const at::Tensor& table, double scale, const at::Tensor& w, const at::Tensor& b,
+                                            double eps, const c10::optional<at::Tensor>& router, const c10::optional<at::Tensor>& rbias, int64_t top,
+                                            int64_t groups, int64_t keep, bool softmax, bool renorm) {
   HYB_CHECK(table.is_cuda() && table.dim() == 2 && table.is_contiguous(), "table: contiguous [vocab, W]");
   HYB_CHECK(ids.is_cuda() && ids.is_contiguous() && ids.scalar_type() == at::kLong && ids.dim() == 1, "ids: int64 [T]");
   const int64_t T = ids.numel(), W = table.size(1);
   HYB_CHECK(w.scalar_type() == at::kFloat && b.scalar_type() == at::kFloat && w.numel() == W && b.numel() == W && w.is_contiguous() && b.is_contiguous(), "norm weight / bias: fp32 [W]");
+  HYB_CHECK(!router.has_value() || table.scalar_type() == at::kBFloat16, "a router takes bf16 rows");
   c10::DeviceGuard guard(table.device());
   at::Tensor x = at::empty({T, W}, table.options().dtype(at::kFloat)), h = at::empty({T, W}, table.options());
-  if (T == 0) return {x, h};
-  dispatch_act(table, [&](auto* tag) {
-    using Tt = std::remove_pointer_t<decltype(tag)>;
-    const Tt* tp = (const Tt*)table.data_ptr();
-    float* xp = x.data_ptr<float>();
-    const float *wp = w.data_ptr<float>(), *bp = b.data_ptr<float>();
-    auto go = [&](auto kern) {
-      kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), tp, table.size(0), (float)scale, wp, bp, xp, (Tt*)h.data_ptr(), (int)W,
-                                                       (float)eps);
-    };
-    if (W <= 16 * NT && quads_ok(tp, W, W) && quads_ok(wp, W, W) && quads_ok(bp, W, W)) {
-      if (W <= 4 * NT) go(embed_layernorm_quads_kernel<Tt, 1>);
-      else if (W <= 8 * NT) go(embed_layernorm_quads_kernel<Tt, 2>);
-      else go(embed_layernorm_quads_kernel<Tt, 4>);
-    } else {
-      embed_scale_kernel<Tt><<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), tp, table.size(0), (float)scale, xp, (int)W);
-      launch_add_layernorm<Tt>(xp, nullptr, 0, nullptr, wp, bp, (Tt*)h.data_ptr(), T, (int)W, eps);
-    }
-  });
-  return {x, h};
+  const float *wp = w.data_ptr<float>(), *bp = b.data_ptr<float>();
+  float* xp = x.data_ptr<float>();
+  const bool quads = W <= 16 * NT && W % 4 == 0 && quads_ok(wp, W, W) && quads_ok(bp, W, W) &&
+                     reinterpret_cast<uintptr_t>(table.data_ptr()) % (4 * table.element_size()) == 0;
+  std::vector<at::Tensor> out = {x, h};
+  RouteOut route{};
+  if (router.has_value() && quads) route = route_out(*router, W, rbias, top, groups, keep, softmax, renorm, T, out);
+  if (T > 0)
+    dispatch_act(table, [&](auto* tag) {
+      using Tt = std::remove_pointer_t<decltype(tag)>;
+      const Tt* tp = (const Tt*)table.data_ptr();
+      auto go = [&](auto kern) {
+        kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), tp, table.size(0), (float)scale, wp, bp, xp, (Tt*)h.data_ptr(), (int)W,
+                                                         (float)eps, route);
+      };
+      auto pick = [&](auto on) {
+        constexpr bool R = decltype(on)::value;
+        if (W <= 4 * NT) go(embed_layernorm_quads_kernel<Tt, 1, R>);
+        else if (W <= 8 * NT) go(embed_layernorm_quads_kernel<Tt, 2, R>);
+        else go(embed_layernorm_quads_kernel<Tt, 4, R>);
+      };
+      if (quads) {
+        if constexpr (std::is_same_v<Tt, bf16_t>) {
+          if (router.has_value()) return pick(std::true_type{});
+        }
+        pick(std::false_type{});
+      } else {
+        embed_scale_kernel<Tt><<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), tp, table.size(0), (float)scale, xp, (int)W);
+        launch_add_layernorm<Tt>(xp, nullptr, 0, nullptr, wp, bp, (Tt*)h.data_ptr(), T, (int)W, eps);
+      }
+    });
+  if (router.has_value() && !quads) add_routed(out, h, *router, rbias, top, groups, keep, softmax, renorm);
+  return out;
 }
 
 static void check_add(const at::Tensor& x, const at::Tensor& a, const c10::optional<at::Tensor>& b) {
@@ -422,12 +442,16 @@ at::Tensor add_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::opti
 at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
                    const c10::optional<at::Tensor>& gate, int64_t experts);
 
-// add_layernorm_f32_ with b = the weighted sum of the routed experts' rows y (moe_sum); without w: the sum alone, no norm.
-at::Tensor add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
-                                      double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
-                                      const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts) {
+// add_layernorm_f32_ with b = the weighted sum of the routed experts' rows y (moe_sum); without w: the sum alone, no norm.  With a router the chosen
+// experts of every row of the result and their weights too.
+std::vector<at::Tensor> add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
+                                                   double eps, const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& xin,
+                                                   const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t experts,
+                                                   const c10::optional<at::Tensor>& router, const c10::optional<at::Tensor>& rbias, int64_t top,
+                                                   int64_t groups, int64_t keep, bool softmax, bool renorm) {
   check_add(x, a, c10::nullopt);
   HYB_CHECK(a.scalar_type() == at::kBFloat16 && xin.sizes() == x.sizes() && w.has_value() == bias.has_value(), "routed experts: bf16 rows of x's shape; a norm has both vectors");
+  HYB_CHECK(!router.has_value() || w.has_value(), "a router reads normed rows");
   const int64_t T = x.size(0);
   const int W = (int)x.size(1);
   if (w.has_value())
@@ -436,26 +460,32 @@ at::Tensor add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c
   const ExpertRows m = expert_rows_of(y, idx, wgt, xin, shared, gate, experts);
   c10::DeviceGuard guard(x.device());
   at::Tensor h = w.has_value() ? out_like(x, x.sizes(), true) : at::empty({0}, x.options());
-  if (T == 0) return h;
   const float *wp = w.has_value() ? w->data_ptr<float>() : nullptr, *bp = w.has_value() ? bias->data_ptr<float>() : nullptr;
   bf16_t* hp = w.has_value() ? (bf16_t*)h.data_ptr() : nullptr;
   const bf16_t* ap = (const bf16_t*)a.data_ptr();
   float* xp = x.data_ptr<float>();
-  auto go = [&](auto kern) { kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(xp, ap, a.stride(0), nullptr, wp, bp, hp, W, (float)eps, m); };
-  auto pick = [&](auto* tag) {
+  const bool quads = W <= 16 * NT && quads_ok(xp, W, W) && quads_ok(ap, a.stride(0), W) && (wp == nullptr || (quads_ok(wp, W, W) && quads_ok(bp, W, W)));
+  std::vector<at::Tensor> out = {h};
+  RouteOut route{};
+  if (router.has_value() && quads) route = route_out(*router, W, rbias, top, groups, keep, softmax, renorm, T, out);
+  auto go = [&](auto kern) { kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(xp, ap, a.stride(0), nullptr, wp, bp, hp, W, (float)eps, m, route); };
+  auto pick = [&](auto* tag, auto on) {
     using Y = std::remove_pointer_t<decltype(tag)>;
-    if (W <= 4 * NT) go(add_layernorm_quads_kernel<bf16_t, 1, Y>);
-    else if (W <= 8 * NT) go(add_layernorm_quads_kernel<bf16_t, 2, Y>);
-    else go(add_layernorm_quads_kernel<bf16_t, 4, Y>);
+    constexpr bool R = decltype(on)::value;
+    if (W <= 4 * NT) go(add_layernorm_quads_kernel<bf16_t, 1, Y, R>);
+    else if (W <= 8 * NT) go(add_layernorm_quads_kernel<bf16_t, 2, Y, R>);
+    else go(add_layernorm_quads_kernel<bf16_t, 4, Y, R>);
   };
-  if (W <= 16 * NT && quads_ok(xp, W, W) && quads_ok(ap, a.stride(0), W) && (wp == nullptr || (quads_ok(wp, W, W) && quads_ok(bp, W, W)))) {
-    if (y.scalar_type() == at::kFloat) pick((float*)nullptr);
-    else pick((bf16_t*)nullptr);
-  } else {  // rows that the quads do not take
+  if (quads && T > 0) {
+    const bool f32 = y.scalar_type() == at::kFloat;
+    if (router.has_value()) f32 ? pick((float*)nullptr, std::true_type{}) : pick((bf16_t*)nullptr, std::true_type{});
+    else f32 ? pick((float*)nullptr, std::false_type{}) : pick((bf16_t*)nullptr, std::false_type{});
+  } else if (T > 0) {  // rows that the quads do not take
     const at::Tensor b = moe_sum(y, idx, wgt, xin, shared, gate, experts);
     launch_add_layernorm<bf16_t>(xp, ap, a.stride(0), b.data_ptr<float>(), wp, bp, hp, T, W, eps);
   }
-  return h;
+  if (router.has_value() && !quads) add_routed(out, h, *router, rbias, top, groups, keep, softmax, renorm);
+  return out;
 }
 
 at::Tensor rmsnorm_cols(const at::Tensor& x, const at::Tensor& w, double eps, int64_t n, bool out_bf16) {

@@ -31,12 +31,21 @@ def layernorm_f32(x, w, b, eps: float, out_dtype):
     return ref.layernorm_f32(x, w, b, eps, out_dtype)
 
 
+ROUTED_ROWS = 64  # steps of at most so many rows are routed by the kernels that norm them: a row reads all of the router's weight
+
+
 def embed_layernorm_f32(ids, table, scale: float, w, b, eps: float):
     """``x = table[ids] * scale`` as the fp32 residual stream, and its LayerNorm in the table's dtype.  Returns (x, h)."""
+    return embed_layernorm_route(ids, table, scale, w, b, eps, None)[:2]
+
+
+def embed_layernorm_route(ids, table, scale: float, w, b, eps: float, router):
+    """:func:`embed_layernorm_f32` and the router of its rows: (x, h, routed), see :func:`add_layernorm_route_`."""
     if use_native(table) and table.is_contiguous():
-        return native_hybrid().embed_layernorm_f32(ids, table, scale, w, b, eps)
+        x, h, *routed = native_hybrid().embed_layernorm_f32(ids, table, scale, w, b, eps, *(router or ()))
+        return x, h, routed or None
     x = torch.nn.functional.embedding(ids, table).float() * scale
-    return x, layernorm_f32(x, w, b, eps, table.dtype)
+    return x, layernorm_f32(x, w, b, eps, table.dtype), None
 
 
 class ExpertSum:
@@ -66,14 +75,21 @@ def residual_add_(x, a, b=None):
 def add_layernorm_f32_(x, a, b, w, bias, eps: float, out_dtype):
     """``x += a (+ b)`` in place, then LayerNorm(x) -> ``out_dtype``: the parallel layer's residual
     update and the next layer's norm in one pass over the stream.  b may be an :class:`ExpertSum`."""
+    return add_layernorm_route_(x, a, b, w, bias, eps, out_dtype, None)[0]
+
+
+def add_layernorm_route_(x, a, b, w, bias, eps: float, out_dtype, router):
+    """:func:`add_layernorm_f32_` and the router of its result in the same pass: (h, routed).  ``router``: ``few_router`` of the layer that reads
+    h, or None; ``routed``: what its forward takes, None where it has to route itself."""
     if isinstance(b, ExpertSum):
         if a.dtype == out_dtype == torch.bfloat16:
-            return native_hybrid().add_experts_layernorm_f32_(x, a, w, bias, eps, *b.parts)
+            h, *routed = native_hybrid().add_experts_layernorm_f32_(x, a, w, bias, eps, *b.parts, *(router or ()))
+            return h, routed or None
         b = b.total()
     if use_native(x):
-        return native_hybrid().add_layernorm_f32_(x, a, b, w, bias, eps, out_dtype == torch.bfloat16)
+        return native_hybrid().add_layernorm_f32_(x, a, b, w, bias, eps, out_dtype == torch.bfloat16), None
     ref.residual_add_(x, a, b)
-    return ref.layernorm_f32(x, w, bias, eps, out_dtype)
+    return ref.layernorm_f32(x, w, bias, eps, out_dtype), None
 
 
 def rmsnorm_cols(x, w, eps: float, n: int, out_dtype):
@@ -336,6 +352,14 @@ def gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps: float, out_dtype):
     return ref.gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps, out_dtype)
 
 
+def gated_norm_add_norm_route_(x, y, r, w_post, w_next, eps: float, out_dtype, router):
+    """:func:`gated_norm_add_norm_f32_` and the router of its result: (h, routed), see :func:`add_layernorm_route_`."""
+    if router is None or w_next is None or out_dtype != torch.bfloat16 or isinstance(y, ExpertSum):
+        return gated_norm_add_norm_f32_(x, y, r, w_post, w_next, eps, out_dtype), None
+    h, *routed = native_hybrid().gated_norm_add_norm_route_(x, y, r, w_post, w_next, eps, *router)
+    return h, routed
+
+
 def embed_rmsnorm_f32(ids, pos, table, pos_table, w, eps: float, out_dtype):
     """``x = table[ids] + pos_table[pos]`` (learned absolute positions) as the fp32 residual stream, and
     its RMS norm with weight ``w`` -> ``out_dtype``.  Returns (x, h)."""
@@ -521,14 +545,15 @@ def experts_pay(T: int, top: int, E: int, rows: int, width: int) -> bool:
 
 
 def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax: bool, renorm: bool, up, down, act: str, shared=None,
-                   gate=None, late: bool = False):
+                   gate=None, late: bool = False, routed=None):
     """``sum_k w_k expert_k(x_t)`` over the chosen experts of every row of ``x [T, W]`` (bf16) -> fp32 ``[T, W]``, all on the device:
     router (fp32 scores of the fp32 ``w_router [E, W]``; ``softmax``: :func:`bias_topk_router`'s choice, else
     :func:`group_topk_router`'s), copies grouped by expert, grouped products, weighted sum.  ``act``: ``relu2`` / ``gelu`` / ``swiglu``
     (``up`` holds ``[gate ; up]``).  Router outputs beyond the experts are experts that give their input.  ``shared [T, W]`` (times
-    ``sigmoid(gate [T, 1])`` if given) is added.  ``late``: an :class:`ExpertSum` instead of the sum.  Operands: :func:`experts_ok`."""
+    ``sigmoid(gate [T, 1])`` if given) is added.  ``late``: an :class:`ExpertSum` instead of the sum; ``routed``: the
+    choice and its weights, where the rows' norm has made them.  Operands: :func:`experts_ok`."""
     nat = native_hybrid()
-    idx, wgt = nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
+    idx, wgt = routed or nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
     ups = expert_list(up)
     rows = nat.moe_expert_rows(x, idx, wgt, ups, expert_list(down), _EXPERT_ACTS[act])
     out = ExpertSum(rows, idx, wgt, x, shared, gate, ups[0].shape[0] if ups[0].dim() == 3 else len(ups))
