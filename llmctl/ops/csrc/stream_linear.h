@@ -152,24 +152,26 @@ inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
 }
 
 // Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to
-// nothing, and smaller workgroups in more rounds hide the latency better (one row, K 2048, one round / rounds of at most 16 weight rows:
-// N 5152 7.8 / 7.3 us, N 8192 9.9 / 8.5, N 12288 13.0 / 12.0; from K 3072 on the other way: N 9248 x 4096 17.7 / 18.3, so rounds of 32 there).  Waves
-// and depth: 16 rows of x, 8 waves of 4 steps / 4 of 8: N 2048 6.00 / 6.06 us, N 4096 7.16 / 7.26; one row 768 x 3072 4.42 / 4.51.
+// nothing, and from 6144 outputs on smaller workgroups in more rounds hide the latency better (one row, K 2048, one round / rounds of at most 16
+// weight rows: N 8192 9.9 / 8.5 us, N 12288 13.0 / 12.0; from K 3072 on the other way: N 9248 x 4096 17.7 / 18.3, so rounds of 32 there).  The
+// waves and so the order of a sum depend on M, N and K alone, not on who owns an output (8 waves of 4 steps instead of 4 of 8: N 2048 6.00 /
+// 6.06 us, N 4096 7.16 / 7.26, not worth other results).
 inline void launch(const Args& g, hipStream_t st) {
-  const int tall = g.M > 4 || g.N <= 4096 ? 64 : g.N > 16384 || g.K <= 2048 ? 16 : 32;  // rows of a workgroup at most
-  const int rounds = (g.N + 256 * tall - 1) / (256 * tall);                             // of 256 workgroups
+  const bool few = g.M <= 4 && g.N >= 6144;
+  const int tall = !few ? 64 : g.N > 16384 || g.K <= 2048 ? 16 : 32;         // rows of a workgroup at most
+  const int rounds = (g.N + 256 * tall - 1) / (256 * tall);                  // of 256 workgroups
   int rows = (g.N + 256 * rounds - 1) / (256 * rounds);
-  if (g.N > 16384) rows = g.M > 4 ? (rows + 3) / 4 * 4 : 16;  // (whole quads are stored at once)
+  if (g.N > 16384) rows = few ? 16 : (rows + 3) / 4 * 4;  // (whole quads are stored at once)
   if (g.M > 16) {
     if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
     else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);
     else if (rows <= 48) go<3, 2, 4, 4>(g, st, rows);
     else go<4, 2, 4, 4>(g, st, rows);
   } else if (rows <= 16) {
-    if (rounds > 1 && g.N <= 16384) go<1, 1, 2, 8>(g, st, rows);
-    else go<1, 1, 8, 4>(g, st, rows);
+    if (few) go<1, 1, 2, 8>(g, st, rows);
+    else go<1, 1, 4, 8>(g, st, rows);
   } else if (rows <= 32) {
-    if (g.M <= 4) go<2, 1, 4, 4>(g, st, rows);
+    if (few) go<2, 1, 4, 4>(g, st, rows);
     else go<2, 1, 4, 8>(g, st, rows);
   } else if (rows <= 48) {
     go<3, 1, 4, 4>(g, st, rows);
