@@ -786,7 +786,7 @@ class GatedDeltaRule(nn.Module):
         S, carried = _own_states(state)
         H, G, dv = self.H, self.G, self.dv
         if z is None:
-            z = hops.linear(h, self.w_in)
+            z = hops.odd_linear(h, self.w_in)
         c, g0 = self.conv.channels, self.conv.channels + H * dv
         qk, v = hops.conv_silu_unit(z[:, :c], self.conv.tap_major(), None, carried, b, G, G, self.dk, self.dk ** -0.5, self.key_eps)
         y = hops.memory_scan(qk[:, :G], qk[:, G:], v.view(-1, H, dv), "delta", S, b, ga=z[:, g0:g0 + H], gb=z[:, g0 + H:g0 + 2 * H],
@@ -834,7 +834,7 @@ class Mamba2(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         S, carried = _own_states(state)
         T, n = h.shape[0], self.inner
-        z = hops.linear(h, self.w_in)
+        z = hops.odd_linear(h, self.w_in)
         c = n + self.conv.channels
         _, xbc = hops.conv_silu_unit(z[:, n:c], self.conv.tap_major(), self.conv_bias, carried, b, 0, 0, 0, 1.0)
         B, C = (xbc[:, n + i * self.G * self.N:n + (i + 1) * self.G * self.N].unflatten(1, (self.G, self.N)) for i in range(2))
@@ -878,7 +878,7 @@ class Retention(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
         S = _own_states(state)[0]
         H, dk, dv = self.H, self.dk, self.dv
-        z = hops.linear(h, self.w_in)
+        z = hops.odd_linear(h, self.w_in)
         qk = hops.rotary_f32(z, H, H, dk, b.pos, self.inv_freq, self.rot_dims, self.interleaved, self.rot_amp, dk ** -0.5)
         v0, g0 = 2 * H * dk, 2 * H * dk + H * dv
         y = hops.memory_scan(qk[:, :H], qk[:, H:], z[:, v0:g0].unflatten(1, (H, dv)), "fixed", S, b, log_decay=self.log_decay,
@@ -929,7 +929,7 @@ class ParallelMixers(nn.Module):
         rows, states = cache
         nl = len(self.left.state_shapes())
         w, bias, c0 = self._stacked()
-        z = hops.linear(h, w, bias)
+        z = hops.odd_linear(h, w, bias)
         yl = self.left.step(h, b, (rows, tuple(states[:nl])), z=z[:, :self.left.w_in.shape[0]])
         yr = self.right.step(h, b, (rows, tuple(states[nl:])), z=z[:, c0:c0 + self.right.w_in.shape[0]])
         return (yl, self.left_scale), (yr, self.right_scale)

@@ -83,6 +83,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("hbm_copy(Tensor src, Tensor(a!) dst) -> ()");
   m.def("gemm64_ex(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, int config=4) -> ()");
   m.def("gemm64_swiglu_fwd(Tensor x, Tensor w, int config, Tensor? rstd=None) -> Tensor");
+  m.def("gemm64_fwd(Tensor x, Tensor w, Tensor? bias=None, bool gated=False) -> Tensor");
   m.def("gemm64_rs(Tensor x, Tensor w, Tensor rstd, int config=304) -> Tensor");
   m.def("rms_rstd(Tensor x, float eps) -> Tensor");
   m.def("gemm64_swiglu_dgrad(Tensor dy, Tensor w, Tensor gu, int config=104) -> Tensor");

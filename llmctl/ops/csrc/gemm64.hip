@@ -849,7 +849,8 @@ __device__ __forceinline__ void g2p_fence(f32x4_t (&acc)[8][8]) {
 
 // 4-wave epilogues (lane holds C[wr*128 + 16 i + (l & 15)][wc*128 + 16 j + 4 (l >> 4) + r]): split
 // partial, fp32 store / accumulate, bf16 store / accumulate, fused RoPE-QKV / SwiGLU forward
-template <int EPI, bool RS = false>
+// RAG (forward layout of any M, and N in multiples of 8): the last tiles' rows past M and columns past N are not stored
+template <int EPI, bool RS = false, bool RAG = false>
 __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)[8][8], int tm, int tn, int wr, int wc,
                                              int lane, int sp, int u, const float* rsl = nullptr) {
   constexpr bool PAIRED_B = EPI == EPI_UP_SWIGLU || EPI == EPI_SWIGLU_FWD;
@@ -939,6 +940,7 @@ __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)
     for (int i = 0; i < 8; ++i) {
       const long t = (long)tm * TM + wr * 128 + 16 * i + i16;
       const float ri = row_scale(i);
+      if (RAG && t >= args.M) break;  // (rows grow with i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int col = tn * 128 + wc * 64 + 16 * j + 4 * g;
@@ -1003,13 +1005,26 @@ __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)
   // epilogue must allow for
   const int cs = 16 * (g & 1) + 8 * (g >> 1);
   unsigned short* Cb = args.c + (long)(tm * TM + wr * 128 + i16) * args.ldc + tn * TN + wc * 128 + cs;
+  f32x4_t bias[RAG ? 8 : 1];  // of the lane's columns 16 j + 4 g ..
+  if constexpr (RAG) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int col = tn * TN + wc * 128 + 16 * j + 4 * g;
+      s2_t b = {0, 0};
+      if (args.aux != nullptr && col < args.N) b = *reinterpret_cast<const s2_t*>(args.aux + col);
+      bias[j] = f32x4_t{bf2f(b[0] & 0xffff), bf2f(b[0] >> 16), bf2f(b[1] & 0xffff), bf2f(b[1] >> 16)};
+    }
+  }
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     uint4 old[4];
     const float ri = row_scale(i);
+    const bool row_in = !RAG || tm * TM + wr * 128 + 16 * i + i16 < args.M;
+    auto in = [&](int jp) __attribute__((always_inline)) { return !RAG || (row_in && tn * TN + wc * 128 + cs + 32 * jp < args.N); };
     if constexpr (EPI == EPI_ACC) {
 #pragma unroll
-      for (int jp = 0; jp < 4; ++jp) old[jp] = *reinterpret_cast<const uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp);
+      for (int jp = 0; jp < 4; ++jp)
+        old[jp] = in(jp) ? *reinterpret_cast<const uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp) : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int jp = 0; jp < 4; ++jp) {
@@ -1036,6 +1051,10 @@ __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)
           c0 *= ri;
           c1 *= ri;
         }
+        if constexpr (RAG) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) c0[e] += bias[j][e], c1[e] += bias[j + 1][e];
+        }
         const unsigned x0 = (unsigned)f2bf(c0[0]) | ((unsigned)f2bf(c0[1]) << 16);
         const unsigned x1 = (unsigned)f2bf(c0[2]) | ((unsigned)f2bf(c0[3]) << 16);
         const unsigned y0 = (unsigned)f2bf(c1[0]) | ((unsigned)f2bf(c1[1]) << 16);
@@ -1044,7 +1063,7 @@ __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)
         const auto r1 = __builtin_amdgcn_permlane16_swap(x1, y1, false, false);
         o = make_uint4(r0[0], r1[0], r0[1], r1[1]);
       }
-      *reinterpret_cast<uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp) = o;
+      if (in(jp)) *reinterpret_cast<uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp) = o;
     }
     __builtin_amdgcn_sched_barrier(0);  // one row's conversions live at a time (no spills)
   }
@@ -1351,7 +1370,7 @@ constexpr int EXP = 0;
 #else
 constexpr int STAMP = 0, EXP = 0;
 #endif
-template <bool AT, bool BT, int EPI, int GROUP, bool RS = false>
+template <bool AT, bool BT, int EPI, int GROUP, bool RS = false, bool RAG = false>
 __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm4wp_kernel(G64Args args,
                                                                                                   int n_items) {
   // RS: two 1 KB slots (item parity) of the tile rows' rs values behind the operand buffers
@@ -1396,8 +1415,18 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     const unsigned short* Ab = AT ? args.a + (long)tm * TM : args.a + (long)tm * TM * lda;
     const unsigned short* Bb = PAIRED_B ? args.b + (long)tn * (TN / 2) * ldb
                                : BT ? args.b + (long)tn * TN : args.b + (long)tn * TN * ldb;
-    ra = make_rsrc(Ab);
-    rb = make_rsrc(Bb);
+    if constexpr (RAG) {
+      // range-checked to the operand's end: rows past it are never addressed (whatever the LDS holds for them, they are not stored).  A row past the
+      // end starts past the range by itself, so this holds whether or not the check counts the K offset in soffset.
+      auto bytes = [](long rows, long ld, int K) __attribute__((always_inline)) {
+        return (unsigned)min(((rows - 1) * ld + K) * 2, 0x7fffffffL);
+      };
+      ra = make_rsrc_n(Ab, bytes(args.M - (long)tm * TM, lda, args.K));
+      rb = PAIRED_B ? make_rsrc(Bb) : make_rsrc_n(Bb, bytes(args.N - (long)tn * TN, ldb, args.K));
+    } else {
+      ra = make_rsrc(Ab);
+      rb = make_rsrc(Bb);
+    }
     rb_hi = PAIRED_B ? make_rsrc(args.b + ((long)args.N + (long)tn * (TN / 2) - TN / 2) * ldb) : rb;
   };
 
@@ -1534,7 +1563,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto rs_issue = [&]() __attribute__((always_inline)) {
     if constexpr (RS) {
       if (wave == 0)
-        bdma16(make_rsrc(args.rs + (long)c_tm * TM), (unsigned)(tid & 63) * 16u, 0u,
+        bdma16(RAG ? make_rsrc_n(args.rs + (long)c_tm * TM, (unsigned)(min(args.M - c_tm * TM, TM) * 4)) : make_rsrc(args.rs + (long)c_tm * TM), (unsigned)(tid & 63) * 16u, 0u,
                lds_addr(smem) + 2 * BUF + (it & 1) * 1024);
     }
   };
@@ -1571,7 +1600,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     g4w_fence(acc);
     if (!has_next) wait_vm<0>();  // the re-loads of the last item's K-tiles 0 / 1 are still landing
     stamp();
-    g4w_epilogue<EPI, RS>(args, acc, c_tm, c_tn, wr, wc, lane, c_sp, c_u,
+    g4w_epilogue<EPI, RS, RAG>(args, acc, c_tm, c_tn, wr, wc, lane, c_sp, c_u,
                           reinterpret_cast<const float*>(smem + 2 * BUF + (it & 1) * 1024));
     if constexpr (STAMP) {
       wait_vm<0>();
@@ -1606,7 +1635,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 
 // sum of the split partials of tail tile u (grouped-order position n_main + u) + epilogue;
 // thread = 8 consecutive columns of one row
-template <int EPI, int GROUP, bool RS = false>
+template <int EPI, int GROUP, bool RS = false, bool RAG = false>
 __global__ __launch_bounds__(256) void gemm64_split_reduce(G64Args args) {
   const int u = blockIdx.x / (TM * TN / 8 / 256);
   const int e = (blockIdx.x % (TM * TN / 8 / 256)) * 256 + threadIdx.x;  // 8-column chunk in the tile
@@ -1617,6 +1646,7 @@ __global__ __launch_bounds__(256) void gemm64_split_reduce(G64Args args) {
   const int gsz = min(GROUP, args.tiles_m - grp * GROUP);
   const int inner = wg - grp * per_group;
   const int tm = grp * GROUP + inner % gsz, tn = inner / gsz;
+  if (RAG && (tm * TM + row >= args.M || (EPI != EPI_SWIGLU_FWD && tn * TN + col >= args.N))) return;
   float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const float* W = args.ws + (long)u * args.splits * (TM * TN) + row * TN + col;
   for (int sp = 0; sp < args.splits; ++sp) {
@@ -1740,6 +1770,10 @@ __global__ __launch_bounds__(256) void gemm64_split_reduce(G64Args args) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] += old[j];
   }
+  if (RAG && args.aux != nullptr) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += bf2f(args.aux[tn * TN + col + j]);
+  }
   store8(p, v);
 }
 
@@ -1783,6 +1817,17 @@ void launch(const G64Args& g, int config) {
   const int group = config % 100, variant = (config / 100) % 10;
   if (group == 8) launch_g<AT, BT, EPI, 8, RS>(g, variant);
   else launch_g<AT, BT, EPI, 4, RS>(g, variant);
+}
+
+// Rows and columns that fill no whole tile (RAG): the persistent kernel only.  An erf GELU in the epilogue was no gain: one wave per SIMD runs it with
+// nothing beside it (2911 x 8192 x 2048: 140 us, against 87 and a pass of 28).
+template <int EPI>
+void launch_ragged(const G64Args& g) {
+  const int n_items = g.n_main + (g.tiles_m * g.tiles_n - g.n_main) * g.splits;
+  hipLaunchKernelGGL((gemm4wp_kernel<false, false, EPI, 4, false, true>), dim3(min(n_items, num_cus())), dim3(NT4), 0, stream(), g, n_items);
+  const int n_tail = g.tiles_m * g.tiles_n - g.n_main;
+  if (n_tail > 0)
+    hipLaunchKernelGGL((gemm64_split_reduce<EPI, 4, false, true>), dim3(n_tail * (TM * TN / 8 / 256)), dim3(256), 0, stream(), g);
 }
 
 // Tail split plan: tiles of the last, partial round (when it is at most half full) are cut into
@@ -2170,7 +2215,45 @@ at::Tensor gemm64_rs(const at::Tensor& x, const at::Tensor& w, const at::Tensor&
   return y;
 }
 
+// y = x w^T (+ bias) of any number of rows, w [N, K] with N a multiple of 8; gated: w = [W_gate; W_up] [2F, K], F a multiple of 128, y = silu(g) * u.  K
+// a multiple of 128, at least 256.
+at::Tensor gemm64_fwd(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, bool gated) {
+  LLMCTL_CHECK(x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.is_cuda() && w.is_cuda() &&
+                   x.stride(1) == 1 && w.stride(1) == 1,
+               "gemm64_fwd: bf16 GPU x [M, K] and w [N, K] with unit inner strides");
+  const long M = x.size(0), K = x.size(1), N = gated ? w.size(0) / 2 : w.size(0);
+  LLMCTL_CHECK(w.size(1) == K && K % (2 * TK) == 0 && K >= 4 * TK && (gated ? w.size(0) == 2 * N && N % (TN / 2) == 0 : N % 8 == 0),
+               "gemm64_fwd: K a multiple of 128 from 256 on, N of 8 (gated: of 256)");
+  LLMCTL_CHECK(x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 &&
+                   (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0 && (M <= 1 || x.stride(0) >= K) && w.stride(0) >= K,
+               "gemm64_fwd: 16-byte aligned operand rows that do not overlap");
+  const bool has_bias = bias.has_value() && bias->defined();
+  if (has_bias)
+    LLMCTL_CHECK(!gated && bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N &&
+                     (reinterpret_cast<uintptr_t>(bias->data_ptr()) & 7) == 0,
+                 "gemm64_fwd: bias bf16 [N], aligned to 8 bytes");
+  const long lda = M <= 1 ? K : x.stride(0);
+  LLMCTL_CHECK((long)TM * lda * 2 < (1L << 31) && (long)TN * w.stride(0) * 2 < (1L << 31), "gemm64_fwd: operand too large for 32-bit offsets");
+  const c10::DeviceGuard dg(x.device());
+  auto y = at::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return y;
+  const int tn = gated ? TN / 2 : TN;
+  G64Args g{reinterpret_cast<const unsigned short*>(x.data_ptr()), reinterpret_cast<const unsigned short*>(w.data_ptr()),
+            reinterpret_cast<unsigned short*>(y.data_ptr()), lda, w.stride(0), N,
+            (int)M, (int)N, (int)K, (int)((M + TM - 1) / TM), (int)((N + tn - 1) / tn), 0, 1, 0, nullptr, has_bias ? bf_ptr(*bias) : nullptr};
+  plan_split(g, 0);
+  at::Tensor ws;
+  if (g.splits > 1) {
+    ws = at::empty({(long)(g.tiles_m * g.tiles_n - g.n_main) * g.splits * TM * TN}, x.options().dtype(at::kFloat));
+    g.ws = ws.data_ptr<float>();
+  }
+  if (gated) launch_ragged<EPI_SWIGLU_FWD>(g);
+  else launch_ragged<EPI_STORE>(g);
+  return y;
+}
+
 TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
+  m.impl("gemm64_fwd", &gemm64_fwd);
   m.impl("gemm64_rs", &gemm64_rs);
   m.impl("gemm64_qkv_rope", &gemm64_qkv_rope);
   m.impl("gemm64_up_swiglu", &gemm64_up_swiglu);

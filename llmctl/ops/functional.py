@@ -704,12 +704,32 @@ def decode_attention_qkv(x, w, b, cos, sin, nq: int, nkv: int, positions, k_cach
     return paged_attention_decode(q, k_cache, v_cache, block_tables, ctx_lens, scale)
 
 
+def _gemm64_fwd_takes(x, w, b=None) -> bool:
+    """The operands of ``gemm64_fwd`` (csrc/gemm64.hip), which takes any number of rows."""
+    return (x.dim() == 2 and x.dtype is torch.bfloat16 and w.dtype is torch.bfloat16 and x.shape[1] % 128 == 0 and x.shape[1] >= 256 and x.stride(1) == 1
+            and w.stride(1) == 1 and x.stride(0) % 8 == 0 and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.stride(0) >= x.shape[1] and w.stride(0) >= w.shape[1] and 512 * max(x.stride(0), w.stride(0)) < 2**31
+            and (b is None or (b.dtype is torch.bfloat16 and b.is_contiguous() and b.data_ptr() % 8 == 0)) and use_native(x) and not wants_grad(x, w, b))
+
+
+def odd_linear(x, w, b=None):
+    """``x @ w^T (+ b)`` for layers whose outputs fill no whole tiles of 256: the in-house kernel where the library's products lose to it, else the
+    library's.  From 9 * 2^20 outputs on, us, library / here: K 2048 2300 x 4240 44.8 / 40.6, 3379 x 4240 64.5 / 49.2, 3379 x 9248 132 / 114, 4090 x 12008
+    201 / 145, 2911 x 8256 93 / 87; K 1024 2911 x 4240 42 / 28; K 4096 2300 x 4240 74 / 70; below: 1331 x 4240 29 / 39, 1800 x 5152 44 / 42.  (Outputs in
+    whole tiles: 3379 x 6144 73 / 86, 3379 x 8192 88 / 95.)"""
+    N = w.shape[0]
+    if N % 256 and N % 8 == 0 and x.shape[0] * N >= 9 << 20 and x.shape[1] >= 1024 and _gemm64_fwd_takes(x, w, b):
+        return native().gemm64_fwd(x, w, b)
+    return torch.nn.functional.linear(x, w, b)
+
+
 def up_swiglu(x, w, b=None):
     """``silu(gate) * up`` of the gate/up projection ``x @ w^T (+ b)`` (w = [W_gate; W_up]).
     Serving prefill: tokens a multiple of 256 run the gemm64 kernel with the SwiGLU in its
     epilogue (``gemm64_swiglu_fwd``: gate and matching up rows in one output tile, only the
-    [T, F] activation stored — no gu tensor, no SwiGLU pass).  Knob ``prefill_swiglu`` off
-    disables (A/B)."""
+    [T, F] activation stored — no gu tensor, no SwiGLU pass), and so do other numbers of tokens from 11 * 2^20 entries of the projection on (us,
+    library and SwiGLU pass / here: 4096 -> 2 x 11008 500 tokens 93 / 85, 700 144 / 118, 1331 308 / 210, 2911 503 / 394, 4095 680 / 528; 4096 -> 2 x 8192 700
+    86 / 84, 1331 159 / 172, 2911 296 / 288; 2048 -> 2 x 4096 1500 50 / 46, but 1023 40 / 43).  Knob ``prefill_swiglu`` off disables (A/B)."""
     x2 = x.reshape(-1, x.shape[-1])
     T, F = x2.shape[0], w.shape[0] // 2
     if (b is None and knobs().prefill_swiglu and use_native(x) and T % 256 == 0
@@ -720,6 +740,8 @@ def up_swiglu(x, w, b=None):
 
         act = native().gemm64_swiglu_fwd(x2, w, gemm64_config("fwd", T, 2 * F, x2.shape[1]) % 1000)
         return act.view(*x.shape[:-1], F)
+    if b is None and knobs().prefill_swiglu and F % 128 == 0 and w.shape[0] % 2 == 0 and T * w.shape[0] >= 11 << 20 and _gemm64_fwd_takes(x2, w):
+        return native().gemm64_fwd(x2, w, None, True).view(*x.shape[:-1], F)
     from llmctl.exec.linear import forward_linear
 
     return swiglu(forward_linear(x, w, b))

@@ -21,6 +21,7 @@ import torch
 
 from . import ref_hybrid as ref
 from ._lib import native_hybrid, use_native
+from .functional import odd_linear as wide_linear
 from .functional import stream_ok, wants_grad
 
 
@@ -485,6 +486,12 @@ def rows_linear(x, w, b=None, act=None, act_cols=None, f32: bool = False):
 def linear(x, w, b=None):
     """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), others are the library's product."""
     return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else torch.nn.functional.linear(x, w, b)
+
+
+def odd_linear(x, w, b=None):
+    """:func:`linear` where the outputs may fill no whole tiles and no expert choice hangs on the order of the sums: prompts take
+    :func:`llmctl.ops.functional.odd_linear`'s form."""
+    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else wide_linear(x, w, b)
 
 
 def linear_f32(x, w):

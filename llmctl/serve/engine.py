@@ -468,8 +468,8 @@ class InferenceEngine:
         if layer.moe is not None:  # routed experts (host-side split sizes: eager, no graphs)
             return layer.moe(xn)
         if self.cfg.gated_mlp:
-            # prefill-sized (T % 256 == 0): the SwiGLU rides on the gate/up GEMM's epilogue
-            act = (ops.up_swiglu(xn, layer.w_up, layer.b_up) if xn.shape[0] >= 256 and xn.shape[0] % 256 == 0
+            # prefill-sized: the SwiGLU rides on the gate/up GEMM's epilogue
+            act = (ops.up_swiglu(xn, layer.w_up, layer.b_up) if xn.shape[0] >= 256
                    else ops.swiglu(ops.decode_linear(xn, layer.w_up, layer.b_up)))
         else:
             act = ops.decode_linear(xn, layer.w_up, layer.b_up, act="gelu")
