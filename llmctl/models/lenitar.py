@@ -157,7 +157,8 @@ class LenitarLM(nn.Module):
         ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer."""
         cfg, eps, dt = self.cfg, self.cfg.layer_norm_eps, self.dtype
         n, T = len(self.layers), b.ids.shape[0]
-        routers = [l.ff.few_router(T) if l.ff is not None and trail is None else None for l in self.layers]
+        # decode steps: the norms find the rows' experts (a prompt's checks would cost the host more than its launch of a router)
+        routers = [l.ff.few_router(T) if l.ff is not None and trail is None and b.Tp == 0 else None for l in self.layers]
         x, h, routed = hops.embed_layernorm_route(b.ids, self.embed, cfg.embedding_scale, self.layers[0].norm_w, self.layers[0].norm_b, eps,
                                                   routers[0])  # fp32 residual stream
         for i, layer in enumerate(self.layers):

@@ -217,7 +217,7 @@ class MalinexLM(nn.Module):
             y, r = layer.mixer.step(h, b, cache.layer(i))
             experts = layer.ff if isinstance(layer.ff, BiasedSoftmaxMoE) else None
             h, routed = hops.gated_norm_add_norm_route_(x, y, r, layer.norm1b, layer.norm2 if layer.ff is not None else nxt, eps, dt,
-                                                        experts.few_router(x.shape[0]) if experts is not None else None)
+                                                        experts.few_router(x.shape[0]) if experts is not None and b.Tp == 0 else None)
             if layer.ff is not None:
                 y, r = experts(h, late=True, routed=routed) if experts is not None else layer.ff(h)
                 h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm2b, nxt, eps, dt)

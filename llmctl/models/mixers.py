@@ -188,34 +188,43 @@ class LatentAttention(nn.Module):
             self._uvt, self._uvt_key = self.w_uv.detach().transpose(1, 2).contiguous(), key
         return self._uvt
 
-    def _attend_expanded(self, q: torch.Tensor, b: StepBatch, cache: torch.Tensor) -> torch.Tensor:
+    def _attend_expanded(self, q: torch.Tensor, b: StepBatch, lat: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
+        """``lat``: the step's cache rows [latent | rotary key]; ``rows [T, H, dv + dn + dr]``, which hold the rotary key already."""
         T, H, dn, dr, dv = q.shape[0], self.H, self.dn, self.dr, self.dv
-        lat = cache.view(-1, self.rk + dr).index_select(0, b.slots)  # the rows just written: [latent | rotary key]
-        rows = torch.empty(T, H, dv + dn + dr, device=q.device, dtype=q.dtype)  # per head [v | k | shared rotary key]
-        rows[:, :, :dv + dn] = F.linear(lat[:, :self.rk], self._w_uvk()).view(T, H, dv + dn)
-        rows[:, :, dv + dn:] = lat[:, None, self.rk:]
-        qa = hops.latent_q_assemble(q[:, :, :dn], q, b.pos, self.inv_freq, self.rot_dims, dn, self.interleaved, self.rot_amp)
+        rows[:, :, :dv + dn] = F.linear(lat[:, :self.rk], self._w_uvk()).view(T, H, dv + dn)  # per head [v | k | shared rotary key]
+        if self.qr:  # (a product of its own)
+            qa = hops.rotary_tail_(q, b.pos, self.inv_freq, self.rot_dims, dn, self.interleaved, self.rot_amp)
+        else:
+            qa = hops.latent_q_assemble(q[:, :, :dn], q, b.pos, self.inv_freq, self.rot_dims, dn, self.interleaved, self.rot_amp)
         # the step's rows as a cache of one-token pages: sequence n's position j is row p_cu[n] + j
-        bt = (b.p_cu[:-1, None] + torch.arange(b.max_q, device=q.device, dtype=torch.int32)[None, :]).clamp_(max=T - 1)
-        o = hops.latent_attention_prefill(qa, rows.view(T, 1, -1), bt.contiguous(), b.p_cu, b.p_ctx, self.window, self.sink,
+        if "own_rows" not in b.scratch:
+            b.scratch["own_rows"] = (b.p_cu[:-1, None] + torch.arange(b.max_q, device=q.device, dtype=torch.int32)[None, :]).clamp_(max=T - 1).contiguous()
+        o = hops.latent_attention_prefill(qa, rows.view(T, 1, -1), b.scratch["own_rows"], b.p_cu, b.p_ctx, self.window, self.sink,
                                           self.scale, dv, b.max_q, groups=H, koff=dv)
         return o.reshape(T, H * dv)
 
     def step(self, h: torch.Tensor, b: StepBatch, cache) -> torch.Tensor:
         if isinstance(cache, tuple):  # (paged rows, recurrent states): this mixer keeps no state
             cache = cache[0]
-        T, H = h.shape[0], self.H
+        T, H, dv, dn = h.shape[0], self.H, self.dv, self.dn
         z = hops.linear(h, self.w_in)
         a, c = self.q_cols, self.q_cols + self.rk + self.dr
-        hops.latent_kv_write(z[:, a:c], self.kv_norm, self.eps, b.pos, self.inv_freq, self.rot_dims, cache, b.slots,
-                             self.interleaved, self.rot_amp)
+        rows = lat = None
+        if self._expand(b):
+            rows = torch.empty(T, H, dv + dn + self.dr, device=h.device, dtype=h.dtype)
         if self.qr:
-            cq = hops.rmsnorm_cols(z[:, :a], self.q_norm, self.eps, self.qr, h.dtype)
+            cq, lat = hops.latent_prep(z, self.q_norm, self.kv_norm, self.dr, self.eps, b.pos, self.inv_freq, self.rot_dims, cache, b.slots,
+                                       self.interleaved, self.rot_amp, rows, dv + dn)
             q = hops.linear(cq, self.w_uq).view(T, H, self.dn + self.dr)
         else:
+            hops.latent_kv_write(z[:, a:c], self.kv_norm, self.eps, b.pos, self.inv_freq, self.rot_dims, cache, b.slots,
+                                 self.interleaved, self.rot_amp)
             q = z[:, :a].unflatten(1, (H, self.dn + self.dr))  # a view: rows keep z's pitch
-        if self._expand(b):
-            o = self._attend_expanded(q, b, cache)
+            if rows is not None:
+                lat = cache.view(-1, self.rk + self.dr).index_select(0, b.slots)  # the rows just written
+                rows[:, :, dv + dn:] = lat[:, None, self.rk:]
+        if rows is not None:
+            o = self._attend_expanded(q, b, lat, rows)
             if self.has_gate:
                 o = hops.sigmoid_gate_mul(o, z[:, c:])
             return hops.linear(o, self.w_o)

@@ -16,6 +16,10 @@ at::Tensor sigmoid_gate_mul(const at::Tensor& o, const at::Tensor& g);
 at::Tensor headnorm_gate(const at::Tensor& o, const c10::optional<at::Tensor>& w, const at::Tensor& g, double eps, bool out_bf16, bool silu);
 void latent_kv_write(const at::Tensor& dkv, const at::Tensor& norm_w, double eps, const at::Tensor& pos, const at::Tensor& inv_freq,
                      int64_t rot_dims, at::Tensor cache, const at::Tensor& slots, bool interleaved, double amp);
+std::tuple<at::Tensor, at::Tensor> latent_prep(const at::Tensor& z, int64_t nq, const at::Tensor& q_w, const at::Tensor& kv_w, int64_t dr, double eps,
+                                               const at::Tensor& pos, const at::Tensor& inv_freq, int64_t rot_dims, at::Tensor cache, const at::Tensor& slots,
+                                               bool interleaved, double amp, const c10::optional<at::Tensor>& rows, int64_t kcol);
+void rotary_tail_(at::Tensor q, const at::Tensor& pos, const at::Tensor& inv_freq, int64_t rot_dims, int64_t dn, bool interleaved, double amp);
 at::Tensor latent_q_assemble(const at::Tensor& q_lat, const at::Tensor& q, const at::Tensor& pos, const at::Tensor& inv_freq,
                              int64_t rot_dims, int64_t dn, bool interleaved, double amp);
 at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& cu,
@@ -147,6 +151,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("sigmoid_gate_mul(Tensor o, Tensor g) -> Tensor");
   m.def("headnorm_gate(Tensor o, Tensor? w, Tensor g, float eps, bool out_bf16, bool silu=False) -> Tensor");
   m.def("latent_kv_write(Tensor dkv, Tensor norm_w, float eps, Tensor pos, Tensor inv_freq, int rot_dims, Tensor(a!) cache, Tensor slots, bool interleaved=False, float amp=1.0) -> ()");
+  m.def("latent_prep(Tensor z, int nq, Tensor q_w, Tensor kv_w, int dr, float eps, Tensor pos, Tensor inv_freq, int rot_dims, Tensor(a!) cache, Tensor slots, bool interleaved, float amp, Tensor(b!)? rows, int kcol) -> (Tensor, Tensor)");
+  m.def("rotary_tail_(Tensor(a!) q, Tensor pos, Tensor inv_freq, int rot_dims, int dn, bool interleaved, float amp) -> ()");
   m.def("latent_q_assemble(Tensor q_lat, Tensor q, Tensor pos, Tensor inv_freq, int rot_dims, int dn, bool interleaved=False, float amp=1.0) -> Tensor");
   m.def("latent_attn_prefill(Tensor qa, Tensor cache, Tensor bt, Tensor cu, Tensor ctx, int window, Tensor? sink, float scale, int rk, int max_q, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0) -> Tensor");
   m.def("latent_attn_decode(Tensor qa, Tensor cache, Tensor bt, Tensor ctx, int window, Tensor? sink, float scale, int rk, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, int max_ctx=0, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0) -> Tensor");
@@ -211,6 +217,8 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("sigmoid_gate_mul", &llmctl_hybrid::sigmoid_gate_mul);
   m.impl("headnorm_gate", &llmctl_hybrid::headnorm_gate);
   m.impl("latent_kv_write", &llmctl_hybrid::latent_kv_write);
+  m.impl("latent_prep", &llmctl_hybrid::latent_prep);
+  m.impl("rotary_tail_", &llmctl_hybrid::rotary_tail_);
   m.impl("latent_q_assemble", &llmctl_hybrid::latent_q_assemble);
   m.impl("latent_attn_prefill", &llmctl_hybrid::latent_attn_prefill);
   m.impl("latent_attn_decode", &llmctl_hybrid::latent_attn_decode);

@@ -47,6 +47,96 @@ __global__ __launch_bounds__(256) void latent_kv_write_kernel(const T* __restric
   for (int i = rot_dims + threadIdx.x; i < dr; i += 256) stf(out + rk + i, ldf(xr + rk + i));
 }
 
+// What follows latent attention's input product z = [q latent (nq) | kv latent (rk) | rotary key (dr) | ..] in one launch: blockIdx.y 0 does what
+// latent_kv_write does, and where ``lat`` is given leaves the cache row in lat [T, rk + dr] too and the turned rotary key in every head's key rows
+// (rows [T, H, R], from column kcol on); blockIdx.y 1 norms the q latent (rmsnorm_cols).  Both sides are a latency and little else (16 rows 4.7
+// us each, 2048 rows 5.3), and a prompt read the rows it had just written back through a gather (3.2) and spread the key with a copy of its own (6.8); together 4.9 and 11.4.
+template <typename T>
+__global__ __launch_bounds__(256) void latent_prep_kernel(const T* __restrict__ z, int64_t z_st, const float* __restrict__ qw, T* __restrict__ cq, int nq,
+                                                          const float* __restrict__ w, const int* __restrict__ pos, const float* __restrict__ inv_freq,
+                                                          T* __restrict__ cache, const int64_t* __restrict__ slots, int rk, int dr, int rot_dims, float eps,
+                                                          int inter, float amp, T* __restrict__ lat, T* __restrict__ rows, int H, int R, int kcol) {
+  extern __shared__ float tail[];  // the rotary key as it is stored
+  __shared__ float red[4];
+  const int64_t t = blockIdx.x;
+  if (blockIdx.y == 1) {
+    const T* x = z + t * z_st;
+    float q = 0.f;
+    for (int c = threadIdx.x; c < nq; c += 256) {
+      const float v = ldf(x + c);
+      q += v * v;
+    }
+    const float rstd = 1.0f / sqrtf(block_sum<4>(q, red) / (float)nq + eps);
+    for (int c = threadIdx.x; c < nq; c += 256) stf(cq + t * nq + c, ldf(x + c) * rstd * qw[c]);
+    return;
+  }
+  const int64_t slot = slots[t];
+  if (slot < 0 && lat == nullptr) return;
+  const T* xr = z + t * z_st + nq;
+  T* out = slot < 0 ? nullptr : cache + slot * (int64_t)(rk + dr);
+  T* lr = lat == nullptr ? nullptr : lat + t * (int64_t)(rk + dr);
+  auto put = [&](int c, float v) {
+    if (out != nullptr) stf(out + c, v);
+    if (lr != nullptr) {
+      stf(lr + c, v);
+      if (c >= rk) tail[c - rk] = v;
+    }
+  };
+  float q = 0.f;
+  for (int c = threadIdx.x; c < rk; c += 256) {
+    const float v = ldf(xr + c);
+    q += v * v;
+  }
+  const float rstd = 1.0f / sqrtf(block_sum<4>(q, red) / (float)rk + eps);
+  for (int c = threadIdx.x; c < rk; c += 256) put(c, ldf(xr + c) * rstd * w[c]);
+  const int half = rot_dims / 2;
+  const float p = (float)pos[t];
+  for (int i = threadIdx.x; i < half; i += 256) {
+    float s, c;
+    sincosf(p * inv_freq[i], &s, &c);
+    s *= amp;
+    c *= amp;
+    const int i0 = inter ? 2 * i : i, i1 = inter ? 2 * i + 1 : i + half;  // neighbours or halves
+    const float u = ldf(xr + rk + i0), v = ldf(xr + rk + i1);
+    put(rk + i0, u * c - v * s);
+    put(rk + i1, v * c + u * s);
+  }
+  for (int i = rot_dims + threadIdx.x; i < dr; i += 256) put(rk + i, ldf(xr + rk + i));
+  if (lat == nullptr) return;
+  __syncthreads();
+  for (int i = threadIdx.x; i < H * dr; i += 256) {
+    const int h = i / dr, c = i - h * dr;
+    stf(rows + (t * H + h) * (int64_t)R + kcol + c, tail[c]);
+  }
+}
+
+// The rotary part of queries [T, H, dn + dr] turned where it is (latent_q_assemble on a product that nothing else reads: 2048 rows, 16 heads of 128
+// + 64: 11.3 us with the copy of the plain part, 5.0 so).
+template <typename T>
+__global__ __launch_bounds__(256) void rotary_tail_kernel(T* __restrict__ q, const int* __restrict__ pos, const float* __restrict__ inv_freq, int H, int dn,
+                                                          int dr, int rot_dims, int inter, float amp) {
+  extern __shared__ float cs_tab[];
+  const int64_t t = blockIdx.x;
+  const int half = rot_dims / 2;
+  const float p = (float)pos[t];
+  for (int i = threadIdx.x; i < half; i += 256) {
+    float s, co;
+    sincosf(p * inv_freq[i], &s, &co);
+    cs_tab[2 * i] = co * amp;
+    cs_tab[2 * i + 1] = s * amp;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < H * half; i += 256) {
+    const int h = i / half, c = i - h * half;
+    const float co = cs_tab[2 * c], s = cs_tab[2 * c + 1];
+    T* qr = q + (t * H + h) * (int64_t)(dn + dr) + dn;
+    const int i0 = inter ? 2 * c : c, i1 = inter ? 2 * c + 1 : c + half;
+    const float u = ldf(qr + i0), v = ldf(qr + i1);
+    stf(qr + i0, u * co - v * s);
+    stf(qr + i1, v * co + u * s);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void latent_q_assemble_kernel(const T* __restrict__ ql, int64_t ql_st, int64_t ql_sh,
                                                                 const T* __restrict__ q, int64_t q_st, const int* __restrict__ pos,
@@ -349,6 +439,52 @@ void latent_kv_write(const at::Tensor& dkv, const at::Tensor& norm_w, double eps
     latent_kv_write_kernel<Tt><<<dim3((unsigned)T), 256, 0, cur_stream()>>>(
         (const Tt*)dkv.data_ptr(), dkv.stride(0), norm_w.data_ptr<float>(), pos.data_ptr<int>(), inv_freq.data_ptr<float>(),
         (Tt*)cache.data_ptr(), slots.data_ptr<int64_t>(), (int)rk, (int)dr, (int)rot_dims, (float)eps, interleaved ? 1 : 0, (float)amp);
+  });
+}
+
+// latent_kv_write of z[:, nq:] and rmsnorm_cols of z[:, :nq]; with rows [T, H, R] (a prompt that attends its own rows expanded) also the cache rows as a
+// tensor and the turned rotary key in rows[.., kcol:].  Returns (normed q latent, cache rows or an empty tensor).
+std::tuple<at::Tensor, at::Tensor> latent_prep(const at::Tensor& z, int64_t nq, const at::Tensor& q_w, const at::Tensor& kv_w, int64_t dr, double eps,
+                                               const at::Tensor& pos, const at::Tensor& inv_freq, int64_t rot_dims, at::Tensor cache, const at::Tensor& slots,
+                                               bool interleaved, double amp, const c10::optional<at::Tensor>& rows, int64_t kcol) {
+  check_rows(z, "z");
+  const int64_t T = z.size(0), rk = kv_w.numel();
+  HYB_CHECK(nq >= 1 && rk >= 1 && dr >= 0 && nq + rk + dr <= z.size(1), "z: [q latent | kv latent | rotary key | ..]");
+  HYB_CHECK(f32_vec(q_w, nq) && f32_vec(kv_w, rk), "norm weights: fp32 [q rank], [rank]");
+  HYB_CHECK(rot_dims % 2 == 0 && rot_dims <= dr && f32_vec(inv_freq, rot_dims / 2), "rotary: even dims <= rot part, fp32 inverse frequencies [dims/2]");
+  check_cache(cache, z, rk + dr);
+  check_i32(pos, "pos");
+  HYB_CHECK(pos.numel() == T && slots.is_cuda() && slots.is_contiguous() && slots.scalar_type() == at::kLong && slots.numel() == T, "pos int32 [T], slots int64 [T]");
+  if (rows.has_value())
+    HYB_CHECK(rows->is_cuda() && rows->is_contiguous() && rows->dim() == 3 && rows->size(0) == T && rows->scalar_type() == z.scalar_type() && kcol >= 0 &&
+                  kcol + dr <= rows->size(2) && dr <= 8192,
+              "rows: contiguous [T, H, R] of z's dtype with room for the rotary key");
+  c10::DeviceGuard guard(z.device());
+  at::Tensor cq = at::empty({T, nq}, z.options()), lat = at::empty({rows.has_value() ? T : 0, rk + dr}, z.options());
+  if (T == 0) return {cq, lat};
+  dispatch_act(z, [&](auto* tag) {
+    using Tt = std::remove_pointer_t<decltype(tag)>;
+    const bool ex = rows.has_value();
+    latent_prep_kernel<Tt><<<dim3((unsigned)T, 2), 256, ex ? (size_t)dr * sizeof(float) : 0, cur_stream()>>>(
+        (const Tt*)z.data_ptr(), z.stride(0), q_w.data_ptr<float>(), (Tt*)cq.data_ptr(), (int)nq, kv_w.data_ptr<float>(), pos.data_ptr<int>(),
+        inv_freq.data_ptr<float>(), (Tt*)cache.data_ptr(), slots.data_ptr<int64_t>(), (int)rk, (int)dr, (int)rot_dims, (float)eps, interleaved ? 1 : 0, (float)amp,
+        ex ? (Tt*)lat.data_ptr() : (Tt*)nullptr, ex ? (Tt*)rows->data_ptr() : (Tt*)nullptr, ex ? (int)rows->size(1) : 0, ex ? (int)rows->size(2) : 0, (int)kcol);
+  });
+  return {cq, lat};
+}
+
+void rotary_tail_(at::Tensor q, const at::Tensor& pos, const at::Tensor& inv_freq, int64_t rot_dims, int64_t dn, bool interleaved, double amp) {
+  HYB_CHECK(q.is_cuda() && q.dim() == 3 && q.is_contiguous(), "q: contiguous [T, H, dn + rot]");
+  const int64_t T = q.size(0), H = q.size(1), dr = q.size(2) - dn;
+  HYB_CHECK(dn >= 0 && dr >= 0 && rot_dims % 2 == 0 && rot_dims <= dr && f32_vec(inv_freq, rot_dims / 2), "rotary: even dims <= rot part");
+  check_i32(pos, "pos");
+  HYB_CHECK(pos.numel() == T, "pos: int32 [T]");
+  if (T == 0 || rot_dims == 0) return;
+  c10::DeviceGuard guard(q.device());
+  dispatch_act(q, [&](auto* tag) {
+    using Tt = std::remove_pointer_t<decltype(tag)>;
+    rotary_tail_kernel<Tt><<<dim3((unsigned)T), 256, (size_t)rot_dims * sizeof(float), cur_stream()>>>(
+        (Tt*)q.data_ptr(), pos.data_ptr<int>(), inv_freq.data_ptr<float>(), (int)H, (int)dn, (int)dr, (int)rot_dims, interleaved ? 1 : 0, (float)amp);
   });
 }
 

@@ -261,6 +261,30 @@ __global__ void gate_mul_kernel(const TO* __restrict__ o, const TG* __restrict__
   stf(y + i, ldf(o + i) * (1.0f / (1.0f + expf(-gv))));
 }
 
+// The same 16 bytes at a time: rows whose pieces share one gate (per a multiple of N) or have one each (per 1).  2048 x 2048 with a gate each 11.3 us element by
+// element, 7.8 so; 2911 rows with a gate per head 16.5 and 9.3.
+template <typename T>
+__global__ __launch_bounds__(256) void gate_mul_vec_kernel(const T* __restrict__ o, const T* __restrict__ g, int64_t g_stride, T* __restrict__ y, int64_t rows,
+                                                           int W, int per) {
+  constexpr int N = Vec16<T>::N;
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * N;
+  if (i >= rows * W) return;
+  const int64_t r = i / W;
+  const int c = (int)(i - r * W);
+  float v[N], gv[N];
+  Vec16<T>::load(o + i, v);
+  if (per == 1) {
+    Vec16<T>::load(g + r * g_stride + c, gv);
+  } else {
+    const float one = ldf(g + r * g_stride + c / per);
+#pragma unroll
+    for (int j = 0; j < N; ++j) gv[j] = one;
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) v[j] *= 1.0f / (1.0f + expf(-gv[j]));
+  Vec16<T>::store(y + i, v);
+}
+
 // o [T, H, dv] fp32 -> y [T, H*dv]: o / rms(o over dv) * w (if given) * sigmoid(g) (silu: * g sigmoid(g)); one wave per (token, head).
 template <typename T>
 __global__ __launch_bounds__(NT) void headnorm_gate_kernel(const float* __restrict__ o, const float* __restrict__ w,
@@ -514,8 +538,14 @@ at::Tensor sigmoid_gate_mul(const at::Tensor& o, const at::Tensor& g) {
   if (n == 0) return y;
   dispatch_act(g, [&](auto* tag) {
     using T = std::remove_pointer_t<decltype(tag)>;
-    gate_mul_kernel<T, T><<<dim3((unsigned)((n + 255) / 256)), 256, 0, cur_stream()>>>((const T*)o.data_ptr(), (const T*)g.data_ptr(),
-                                                                                     g.stride(0), (T*)y.data_ptr(), o.size(0), (int)o.size(1), (int)(o.size(1) / g.size(1)));
+    constexpr int N = Vec16<T>::N;
+    const T *op = (const T*)o.data_ptr(), *gp = (const T*)g.data_ptr();
+    const int W = (int)o.size(1), per = (int)(o.size(1) / g.size(1));
+    auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    if (W % N == 0 && at16(op) && at16(y.data_ptr()) && (per % N == 0 || (per == 1 && at16(gp) && g.stride(0) % N == 0)))
+      gate_mul_vec_kernel<T><<<dim3((unsigned)((n / N + 255) / 256)), 256, 0, cur_stream()>>>(op, gp, g.stride(0), (T*)y.data_ptr(), o.size(0), W, per);
+    else
+      gate_mul_kernel<T, T><<<dim3((unsigned)((n + 255) / 256)), 256, 0, cur_stream()>>>(op, gp, g.stride(0), (T*)y.data_ptr(), o.size(0), W, per);
   });
   return y;
 }

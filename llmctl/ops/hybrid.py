@@ -111,6 +111,32 @@ def latent_kv_write(dkv, norm_w, eps: float, pos, inv_freq, rot_dims: int, cache
         ref.latent_kv_write(dkv, norm_w, eps, pos, inv_freq, rot_dims, cache, slots, interleaved, amp)
 
 
+def latent_prep(z, q_norm, kv_norm, dr: int, eps: float, pos, inv_freq, rot_dims: int, cache, slots, interleaved: bool = False, amp: float = 1.0,
+                rows=None, kcol: int = 0):
+    """What follows the product ``z = [q latent | kv latent | rotary key | ..]``: :func:`rmsnorm_cols` of the q latent (returned first) and
+    :func:`latent_kv_write` of the rest.  ``rows [T, H, R]``: the turned rotary key goes to every head's ``rows[.., kcol : kcol + dr]`` too, and
+    the written cache rows are returned second (else None)."""
+    nq, rk = q_norm.numel(), kv_norm.numel()
+    if use_native(z):
+        cq, lat = native_hybrid().latent_prep(z, nq, q_norm, kv_norm, dr, eps, pos, inv_freq, rot_dims, cache, slots, interleaved, amp, rows, kcol)
+        return cq, lat if rows is not None else None
+    latent_kv_write(z[:, nq:nq + rk + dr], kv_norm, eps, pos, inv_freq, rot_dims, cache, slots, interleaved, amp)
+    lat = None
+    if rows is not None:
+        lat = cache.view(-1, rk + dr).index_select(0, slots)
+        rows[:, :, kcol:kcol + dr] = lat[:, None, rk:]
+    return rmsnorm_cols(z[:, :nq], q_norm, eps, nq, z.dtype), lat
+
+
+def rotary_tail_(q, pos, inv_freq, rot_dims: int, dn: int, interleaved: bool = False, amp: float = 1.0):
+    """The rotary part of contiguous queries ``q [T, H, dn + rot]`` turned in place."""
+    if use_native(q):
+        native_hybrid().rotary_tail_(q, pos, inv_freq, rot_dims, dn, interleaved, amp)
+    else:
+        q.copy_(latent_q_assemble(q[:, :, :dn], q, pos, inv_freq, rot_dims, dn, interleaved, amp))
+    return q
+
+
 def latent_q_assemble(q_lat, q, pos, inv_freq, rot_dims: int, dn: int, interleaved: bool = False, amp: float = 1.0):
     """Query rows in the cache's layout: ``[q_lat | rotary(q[..., dn:])]`` per head, where ``q_lat
     [T, H, rank]`` is the unrotated query part carried into the latent space (q W_uk)."""
