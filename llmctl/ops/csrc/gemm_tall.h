@@ -1,0 +1,8 @@
+// Products on 256 x 128 tiles (gemm_tall.hip), for gemm64's dispatch
+#pragma once
+#include <ATen/ATen.h>
+
+namespace llmctl {
+int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits);
+void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits);
+}  // namespace llmctl

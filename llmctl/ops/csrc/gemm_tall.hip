@@ -1,0 +1,318 @@
+// Backward products on 256 x 128 tiles: data gradients dy W (W read K-major) and weight gradients dy^T x, bf16 in, for the sizes that leave the 256 x 256
+// tiles of gemm64.hip short of workgroups.
+//
+// Bound: the MFMAs where the tiles fill the chip; below that the fill.  8192 x 768 is 96 tiles of 256 x 256 for 256 CUs and 192 of 256 x 128; a 768 x 3072
+// weight gradient over 8192 tokens is 36, cut in K to get to 144 at four partial sums an entry, against 72 and three.
+//
+// Layout: four waves, one per SIMD, 128 x 64 each (acc 8 x 4), a ring of three K-tiles of 64 in LDS (48 KB each: the images A_lo, A_hi and B_h0 of
+// gemm64_tiles.h) filled by LDS-DMA.  A K-tile is two phases of 32 MFMAs; fragments are read in the phase before their use, one to a statement of two MFMAs,
+// b twice, by K-tile parity; the DMA pieces go out every third statement; one barrier:
+//   P0(t)  MFMA rows 0-3 [a_lo(t), b(t)]   read a_hi(t), b(t+1) first half      issue A_lo(t+2) second half, A_hi(t+2)
+//   P1(t)  MFMA rows 4-7 [a_hi(t), b(t)]   read a_lo(t+1), b(t+1) second half   issue B(t+3), A_lo(t+3) first half
+//          vmcnt(10) + barrier: B, A_lo(t+2) and A_hi(t+1) have landed
+// Each piece's slot was last read before the barrier that precedes it: B, A_lo(t) by P1(t-1), A_hi(t) by P0(t).  The last three K-tiles issue nothing that does
+// not exist and wait for what is left.  Pieces eight to a half phase queued up in the address unit (a 768 x 3072 product over 8192 tokens in 72 workgroups: 89.2
+// us, so 79.7); twelve in P1, a longer time to arrive, 106.7.
+// LDS moves (128 + 64) x 64 operand entries per wave and K-tile and takes in the 48 KB of another: 1.1 times the MFMAs' 1024 clocks at 128 bytes a clock, where
+// the 256 x 256 tiles are at 0.75; on a full chip those are a fifth faster (8192 x 4096 x 4096: 190 us, here 234).  gemm_tall_splits weighs the two.
+// Measured on one MI355X, us, 256 x 256 tiles / these: data gradients of 8192 tokens 768 x 768 21.6 / 14.0, 2304 x 768 44.7 / 29.5, 3072 x 768 52.6 / 46.5,
+// 2048 x 4096 x 4096 71.0 / 54.3; weight gradients 768 x 768 30.1 / 23.1, 2304 x 768 42.3 / 35.9, 768 x 3072 56.5 / 46.2.
+#include "gemm_tall.h"
+#include "gemm64_tiles.h"
+
+namespace llmctl {
+using namespace attn;
+namespace {
+
+constexpr int TALL_N = 128, SLOT = 3 * HALF;
+enum : int { OUT_STORE = 0, OUT_ADD = 1, OUT_STORE_F32 = 2, OUT_ADD_F32 = 3 };
+
+struct TallArgs {
+  const unsigned short* a;
+  const unsigned short* b;
+  void* c;
+  float* ws;  // [splits][M][N] fp32 partial sums (splits > 1)
+  long lda, ldb, ldc;
+  int M, N, K;
+  int tiles_m, tiles_n, splits;
+};
+
+// 16 wait states between what wrote four rows of accumulators (their zeroes, the last phase's 32 MFMAs) and what reads them
+template <int R>
+__device__ __forceinline__ void fence_rows(f32x4_t (&acc)[8][4]) {
+  asm volatile("s_nop 7\n\ts_nop 7"
+               : "+a"(acc[R][0]), "+a"(acc[R][1]), "+a"(acc[R][2]), "+a"(acc[R][3]), "+a"(acc[R + 1][0]), "+a"(acc[R + 1][1]), "+a"(acc[R + 1][2]),
+                 "+a"(acc[R + 1][3]), "+a"(acc[R + 2][0]), "+a"(acc[R + 2][1]), "+a"(acc[R + 2][2]), "+a"(acc[R + 2][3]), "+a"(acc[R + 3][0]),
+                 "+a"(acc[R + 3][1]), "+a"(acc[R + 3][2]), "+a"(acc[R + 3][3]));
+}
+
+template <bool AT, int OUT>
+__global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_tall_kernel(TallArgs args) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 1, wc = wave & 1;
+  const long lda = args.lda, ldb = args.ldb;
+
+  // item: split outermost, then groups of four tile rows, row innermost; each XCD takes a contiguous run of them, so its L2 holds the panels that it shares
+  const int n_items = args.tiles_m * args.tiles_n * args.splits;
+  const int q8 = n_items / 8, r8 = n_items % 8, x = blockIdx.x % 8;
+  const int item = (x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8) + blockIdx.x / 8;
+  const int tiles = args.tiles_m * args.tiles_n;
+  const int sp = item / tiles, wg = item - sp * tiles;
+  const int grp = wg / (4 * args.tiles_n), gsz = min(4, args.tiles_m - grp * 4), inner = wg - grp * 4 * args.tiles_n;
+  const int tm = grp * 4 + inner % gsz, tn = inner / gsz;
+  const int pairs = args.K / (2 * TK);
+  const int k0 = 2 * (int)((long)pairs * sp / args.splits), KT = 2 * (int)((long)pairs * (sp + 1) / args.splits) - k0;
+
+  i32x4_t ra = make_rsrc(AT ? args.a + (long)tm * TM : args.a + (long)tm * TM * lda);
+  i32x4_t rb = make_rsrc(args.b + (long)tn * TALL_N);
+  asm volatile("s_nop 7" : "+s"(ra), "+s"(rb));  // lane-read scalars to the first DMA piece that uses them
+  const unsigned a_step = AT ? (unsigned)(TK * lda * 2) : (unsigned)(TK * 2), b_step = (unsigned)(TK * ldb * 2);
+  unsigned vo[3][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    vo[A_LO][i] = stage_voff<AT, A_LO, NT4>(i, tid, lda);
+    vo[A_HI][i] = stage_voff<AT, A_HI, NT4>(i, tid, lda);
+    vo[B_H0][i] = stage_voff<true, B_H0, NT4>(i, tid, ldb);
+  }
+  const unsigned lds0 = lds_addr(smem) + wave * 1024;
+  auto issue = [&](auto kind_c, int t, int slot, auto n_c) __attribute__((always_inline)) {
+    constexpr int kind = decltype(kind_c)::value, n = decltype(n_c)::value;
+    const unsigned so = (unsigned)(k0 + t) * (kind == B_H0 ? b_step : a_step);
+#pragma unroll
+    for (int i = 0; i < n; ++i) bdma16(kind == B_H0 ? rb : ra, vo[kind][i], so, lds0 + slot + kind * HALF + i * 4096);
+  };
+
+  f32x4_t acc[8][4];
+  bf16x8_t a_lo[4][2], a_hi[4][2], b[2][4][2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  fence_rows<0>(acc);
+  fence_rows<4>(acc);
+
+  issue(K_<B_H0>{}, 0, 0, K_<4>{});
+  issue(K_<A_LO>{}, 0, 0, K_<4>{});
+  issue(K_<A_HI>{}, 0, 0, K_<4>{});
+  issue(K_<B_H0>{}, 1, SLOT, K_<4>{});
+  issue(K_<A_LO>{}, 1, SLOT, K_<4>{});
+  issue(K_<A_HI>{}, 1, SLOT, K_<4>{});
+  issue(K_<B_H0>{}, 2, 2 * SLOT, K_<4>{});
+  issue(K_<A_LO>{}, 2, 2 * SLOT, K_<2>{});
+  wait_vm<22>();
+  bar();
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a_lo[i][ks] = frag<AT>(smem + A_LO * HALF, wr * 64 + 16 * i, ks, lane);
+      b[0][i][ks] = frag<true>(smem + B_H0 * HALF, wc * 64 + 16 * i, ks, lane);
+    }
+  wait_vm<10>();
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+  bar();
+
+  // K-tile t in ring slot s0; s1, s2: those of t + 1 and t + 2.  DMA: 2 = both phases issue, 1 = only P0 does, 0 = none; WAIT: vmcnt at the end (-1: last)
+  auto ktile = [&](auto par_c, auto dma_c, auto wait_c, int t, int s0, int s1, int s2) __attribute__((always_inline)) {
+    constexpr int P = decltype(par_c)::value, DMA = decltype(dma_c)::value, WAIT = decltype(wait_c)::value;
+    constexpr bool NEXT = WAIT >= 0;
+    const unsigned so0 = (unsigned)(k0 + t + 2) * a_step, l0 = lds0 + s2;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int ks = q >> 3, i = (q >> 1) & 3, j = (q & 1) * 2;
+      if (DMA >= 1 && q % 3 == 0) {
+        const int n = q / 3, kind = n < 2 ? A_LO : A_HI, pc = n < 2 ? 2 + n : n - 2;
+        g4w_pair_dma(acc[i][j], acc[i][j + 1], a_lo[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], ra, so0, l0 + kind * HALF + pc * 4096);
+      } else {
+        g4w_pair(acc[i][j], acc[i][j + 1], a_lo[i][ks], b[P][j][ks], b[P][j + 1][ks]);
+      }
+      if (q < 8) a_hi[q & 3][q >> 2] = frag<AT>(smem + s0 + A_HI * HALF, wr * 64 + 16 * (q & 3), q >> 2, lane);
+      else if (NEXT && q < 12) b[P ^ 1][q & 3][0] = frag<true>(smem + s1 + B_H0 * HALF, wc * 64 + 16 * (q & 3), 0, lane);
+    }
+    const unsigned soa = (unsigned)(k0 + t + 3) * a_step, sob = (unsigned)(k0 + t + 3) * b_step, l1 = lds0 + s0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int ks = q >> 3, i = (q >> 1) & 3, j = (q & 1) * 2;
+      if (DMA == 2 && q % 3 == 0) {
+        const int n = q / 3, kind = n < 4 ? B_H0 : A_LO, pc = n & 3;
+        g4w_pair_dma(acc[4 + i][j], acc[4 + i][j + 1], a_hi[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], n < 4 ? rb : ra, n < 4 ? sob : soa,
+                     l1 + kind * HALF + pc * 4096);
+      } else {
+        g4w_pair(acc[4 + i][j], acc[4 + i][j + 1], a_hi[i][ks], b[P][j][ks], b[P][j + 1][ks]);
+      }
+      if (NEXT && q < 8) a_lo[q & 3][q >> 2] = frag<AT>(smem + s1 + A_LO * HALF, wr * 64 + 16 * (q & 3), q >> 2, lane);
+      else if (NEXT && q < 12) b[P ^ 1][q & 3][1] = frag<true>(smem + s1 + B_H0 * HALF, wc * 64 + 16 * (q & 3), 1, lane);
+    }
+    if constexpr (NEXT) {
+      wait_vm<NEXT ? WAIT : 0>();
+      __builtin_amdgcn_s_waitcnt(0xC07F);
+      bar();
+    }
+  };
+  int s0 = 0, s1 = SLOT, s2 = 2 * SLOT;
+  auto turn = [&]() __attribute__((always_inline)) {
+    const int s = s0;
+    s0 = s1, s1 = s2, s2 = s;
+  };
+  for (int t = 0; t < KT - 4; t += 2) {  // KT even, >= 4
+    ktile(K_<0>{}, K_<2>{}, K_<10>{}, t, s0, s1, s2);
+    turn();
+    ktile(K_<1>{}, K_<2>{}, K_<10>{}, t + 1, s0, s1, s2);
+    turn();
+  }
+  ktile(K_<0>{}, K_<2>{}, K_<10>{}, KT - 4, s0, s1, s2);
+  turn();
+  ktile(K_<1>{}, K_<1>{}, K_<4>{}, KT - 3, s0, s1, s2);
+  turn();
+  ktile(K_<0>{}, K_<0>{}, K_<0>{}, KT - 2, s0, s1, s2);
+  turn();
+  ktile(K_<1>{}, K_<0>{}, K_<-1>{}, KT - 1, s0, s1, s2);
+  fence_rows<4>(acc);
+
+  // lane holds C[wr * 128 + 16 i + (l & 15)][wc * 64 + 16 j + 4 (l >> 4) + r]
+  const int g = lane >> 4, i16 = lane & 15;
+  const long row0 = (long)tm * TM + wr * 128 + i16;
+  const int col0 = tn * TALL_N + wc * 64;
+  if (args.splits > 1 || OUT >= OUT_STORE_F32) {
+    const bool part = args.splits > 1;
+    const long ld = part ? args.N : args.ldc;
+    float* C = (part ? args.ws + (long)sp * args.M * args.N : static_cast<float*>(args.c)) + row0 * ld + col0 + 4 * g;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f32x4_t old[4];
+      const bool add = OUT == OUT_ADD_F32 && !part;
+      if (add) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) old[j] = *reinterpret_cast<const f32x4_t*>(C + 16 * i * ld + 16 * j);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t*>(C + 16 * i * ld + 16 * j) = add ? acc[i][j] + old[j] : acc[i][j];
+    }
+    return;
+  }
+  // bf16, 16 bytes to a lane: lanes of neighbouring groups swap halves of two column tiles
+  unsigned short* C = static_cast<unsigned short*>(args.c) + row0 * args.ldc + col0 + 16 * (g & 1) + 8 * (g >> 1);
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+#pragma unroll
+    for (int jp = 0; jp < 2; ++jp) {
+      unsigned short* p = C + 16 * i * args.ldc + 32 * jp;
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][2 * jp][e]), __float_as_uint(acc[i][2 * jp + 1][e]), false, false);
+        v[e] = __uint_as_float(r[0]);
+        v[4 + e] = __uint_as_float(r[1]);
+      }
+      if constexpr (OUT == OUT_ADD) {
+        float old[8];
+        load8(p, old);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += old[e];
+      }
+      store8(p, v);
+    }
+}
+
+// out (+)= the partial sums, added in the order of K; a thread's 8 columns of a row
+template <int OUT>
+__global__ __launch_bounds__(256) void gemm_tall_reduce(TallArgs args) {
+  const long e = ((long)blockIdx.x * 256 + threadIdx.x) * 8;  // M N is a multiple of 2048
+  const long row = e / args.N, col = e - row * args.N, MN = (long)args.M * args.N;
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const float* W = args.ws + e;
+#pragma unroll 4
+  for (int s = 0; s < args.splits; ++s) {
+    const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(W + s * MN), x1 = *reinterpret_cast<const f32x4_t*>(W + s * MN + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += x0[j], v[4 + j] += x1[j];
+  }
+  if constexpr (OUT >= OUT_STORE_F32) {
+    f32x4_t* p = reinterpret_cast<f32x4_t*>(static_cast<float*>(args.c) + row * args.ldc + col);
+    f32x4_t lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
+    if constexpr (OUT == OUT_ADD_F32) lo += p[0], hi += p[1];
+    p[0] = lo;
+    p[1] = hi;
+  } else {
+    unsigned short* p = static_cast<unsigned short*>(args.c) + row * args.ldc + col;
+    if constexpr (OUT == OUT_ADD) {
+      float old[8];
+      load8(p, old);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += old[j];
+    }
+    store8(p, v);
+  }
+}
+
+template <bool AT>
+void launch(const TallArgs& g, int out) {
+  const dim3 grid(g.tiles_m * g.tiles_n * g.splits), red((unsigned)((long)g.M * g.N / 2048));
+  auto go = [&](auto out_c) {
+    constexpr int OUT = decltype(out_c)::value;
+    hipLaunchKernelGGL((gemm_tall_kernel<AT, OUT>), grid, dim3(NT4), 0, stream(), g);
+    if (g.splits > 1) hipLaunchKernelGGL((gemm_tall_reduce<OUT>), red, dim3(256), 0, stream(), g);
+  };
+  switch (out) {
+    case OUT_STORE: go(K_<OUT_STORE>{}); break;
+    case OUT_ADD: go(K_<OUT_ADD>{}); break;
+    case OUT_STORE_F32: go(K_<OUT_STORE_F32>{}); break;
+    default: go(K_<OUT_ADD_F32>{}); break;
+  }
+}
+
+}  // namespace
+
+// K-ranges for this kernel where it is the faster one, else 0.  n_main whole tiles of 256 x 256 and n_tail in `splits` ranges each are gemm64's plan.  Both
+// times from the sizes, us: a round costs its K-tiles (0.72 here and 1.3 there for 64 of K, on a full chip) and a fixed part (4, 7: fill and store); partial sums
+// cost a launch (4) and their bytes, written and read, at 6 TB/s.  Ranges stay at four K-tiles and more, what the peeled loop takes.
+// Both sides measured, us: see above where these win; 192 tiles of 256 x 256 (4096 x 3072 x 768) 25.8 / 27.6 and 256 (4096 x 4096 x 2048) 53.0 / 62.4 there.
+int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits) {
+  const double cus = num_cus(), kt = K / TK;
+  auto rounds = [&](double items) { return std::ceil(items / cus); };
+  auto sums = [](double entries, int S) { return S > 1 ? 4.0 + entries * S * 8.0 / 6e6 : 0.0; };
+  double other = rounds(n_main) * (kt * 1.3 + 7.0);
+  if (n_tail > 0) other += rounds((double)n_tail * splits) * (kt / splits * 1.3 + 7.0) + sums((double)n_tail * TM * TN, splits);
+  int best = 0;
+  for (int S = 1; S <= 16 && K >= 4L * TK * S; ++S) {
+    const double part = 2.0 * std::ceil(kt / 2.0 / S);
+    const double us = rounds((double)(M / TM) * (N / TALL_N) * S) * (part * 0.72 + 4.0) + sums((double)M * N, S);
+    if (us < other) other = us, best = S;
+  }
+  return best;
+}
+
+// out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N and K of 128, K >= 256 splits.
+void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits) {
+  LLMCTL_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2 && a.is_cuda() && b.is_cuda() && out.is_cuda(), "gemm_tall: 2-D GPU operands");
+  const bool f32 = out.scalar_type() == at::kFloat;
+  LLMCTL_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && (f32 || out.scalar_type() == at::kBFloat16),
+               "gemm_tall: bf16 operands, bf16 or fp32 out");
+  const long M = at_ ? a.size(1) : a.size(0), K = at_ ? a.size(0) : a.size(1), N = b.size(1);
+  LLMCTL_CHECK(b.size(0) == K && out.size(0) == M && out.size(1) == N, "gemm_tall: shapes");
+  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && K % (2 * TK) == 0 && splits >= 1 && K >= 4 * TK * splits,
+               "gemm_tall: M in 256s, N and K in 128s, at least 256 of K to a split");
+  auto rows16 = [](const at::Tensor& t, int per) {
+    return t.stride(1) == 1 && t.stride(0) % per == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+  };
+  LLMCTL_CHECK(rows16(a, 8) && rows16(b, 8) && rows16(out, f32 ? 4 : 8), "gemm_tall: 16-byte aligned rows, unit column stride");
+  const long a_span = (at_ ? K : (long)TM) * a.stride(0) * 2, b_span = K * b.stride(0) * 2;
+  LLMCTL_CHECK(a_span < (1L << 31) && b_span < (1L << 31) && M * N / 2048 < (1L << 31), "gemm_tall: operand too large for 32-bit offsets");
+  const c10::DeviceGuard guard(a.device());
+  TallArgs g{bf_ptr(a), bf_ptr(b), out.data_ptr(), nullptr, (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K,
+             (int)(M / TM), (int)(N / TALL_N), (int)splits};
+  at::Tensor ws;
+  if (splits > 1) {
+    ws = at::empty({splits, M, N}, a.options().dtype(at::kFloat));
+    g.ws = ws.data_ptr<float>();
+  }
+  const int o = (f32 ? OUT_STORE_F32 : OUT_STORE) + (accumulate ? 1 : 0);
+  if (at_) launch<true>(g, o);
+  else launch<false>(g, o);
+}
+
+TORCH_LIBRARY_IMPL(llmctl, CUDA, m) { m.impl("gemm_tall", &gemm_tall); }
+
+}  // namespace llmctl

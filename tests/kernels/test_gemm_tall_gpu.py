@@ -1,0 +1,59 @@
+"""Backward products on 256 x 128 tiles: one tile and several, the shortest K range and uneven ones, each output form, rows wider than the matrix."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(at, M, N, K, pad):
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    shape = (K, M) if at else (M, K)
+    a = torch.randn(shape[0], shape[1] + pad, generator=g, device="cuda").bfloat16()[:, :shape[1]]
+    b = torch.randn(K, N + pad, generator=g, device="cuda").bfloat16()[:, :N]
+    return a, b
+
+
+def _bound(a, b, K, S):
+    """fp32 sums of K exact products in any order, and S partial sums: (K + S) 2^-24 of the sum of magnitudes"""
+    return (K + S) * 2.0**-24 * (a.abs() @ b.abs())
+
+
+@pytest.mark.parametrize("at,M,N,K,S,pad", [
+    (False, 256, 128, 256, 1, 0), (True, 256, 128, 256, 1, 8),        # one tile, the four peeled K-tiles alone
+    (False, 512, 384, 384, 1, 8), (True, 768, 256, 640, 1, 0),        # an odd number of pairs of K-tiles
+    (False, 1280, 128, 1152, 4, 0), (True, 256, 384, 1408, 5, 8),     # uneven ranges, tile rows that fill no group of four
+    (True, 768, 768, 8192, 12, 0), (False, 8192, 768, 768, 1, 0),
+])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("add", [False, True])
+def test_products(at, M, N, K, S, pad, f32, add):
+    from llmctl.ops._lib import native
+
+    a, b = _operands(at, M, N, K, pad)
+    full = torch.full((M, N + 8), 3.0, device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    out = full[:, :N]
+    old = out.double() if add else torch.zeros((), device="cuda", dtype=torch.float64)
+    if not add:
+        out.fill_(float("nan"))
+    native().gemm_tall(a, b, out, at, add, S)
+    A, B = (a.t() if at else a).double(), b.double()
+    ref, bound = A @ B + old, _bound(A, B, K, S + 1)
+    if not f32:  # one rounding of the fp32 result
+        bound = bound + 2.0**-8 * (ref.abs() + bound)
+    assert bool(((out.double() - ref).abs() <= bound + 2.0**-23 * ref.abs()).all())
+    assert bool((full[:, N:] == 3.0).all())
+
+
+@pytest.mark.parametrize("at,M,N,K", [(False, 8192, 768, 2304), (False, 2048, 768, 768), (True, 768, 3072, 1024), (True, 256, 256, 128),
+                                      (False, 512, 256, 128)])
+@pytest.mark.parametrize("odd_rows", [False, True])
+def test_gemm64_takes_either_tile(at, M, N, K, odd_rows):
+    """Whatever tile the plan takes, also for output rows of 8 bytes' alignment (those stay with the 256 x 256 tiles)."""
+    from llmctl.ops._lib import native
+
+    a, b = _operands(at, M, N, K, 0)
+    out = torch.full((M, N + 4), 3.0, device="cuda", dtype=torch.bfloat16)[:, :N] if odd_rows else torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    native().gemm64_ex(a, b, out, at, True, False, 304)
+    A, B = (a.t() if at else a).double(), b.double()
+    ref, bound = A @ B, _bound(A, B, K, 16)
+    assert bool(((out.double() - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
