@@ -337,12 +337,16 @@ class GradSink:
             s = cls._streams[device] = torch.cuda.Stream(device=device)
         return s
 
-    def attach(self, p: torch.nn.Parameter) -> None:
+    def attach(self, p: torch.nn.Parameter, writes: int = 1) -> None:
+        """``writes``: the gradients that one backward writes (2: an embedding that is the output projection too); the last of them
+        is what the callbacks are told of."""
         p._llmctl_grad_sink = self
+        p._llmctl_writes = p._llmctl_pending = writes
         p._llmctl_fresh = True
 
     def reset(self, p: torch.nn.Parameter) -> None:
         p._llmctl_fresh = True
+        p._llmctl_pending = p._llmctl_writes
 
     @staticmethod
     def _target(p: torch.nn.Parameter) -> torch.Tensor:
@@ -355,6 +359,10 @@ class GradSink:
 
     def _written(self, p: torch.nn.Parameter) -> None:
         p._llmctl_fresh = False
+        p._llmctl_pending -= 1
+        if p._llmctl_pending > 0:
+            return
+        p._llmctl_pending = p._llmctl_writes
         for cb in self.callbacks:
             cb(p)
 
@@ -457,6 +465,40 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -
     if not needs_grad:
         return forward_linear(x, w, b)
     return _Linear.apply(x, w, b)
+
+
+class _Embedding(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, ids, w):
+        from llmctl import ops
+
+        ctx.save_for_backward(ids)
+        ctx.wparam = w
+        return ops.embed_rows(ids, w)
+
+    @staticmethod
+    def backward(ctx, dy):
+        from llmctl import ops
+
+        (ids,) = ctx.saved_tensors
+        if ctx.needs_input_grad[1]:
+            w = ctx.wparam
+            sink: GradSink = w._llmctl_grad_sink
+            dy2 = dy.reshape(-1, dy.shape[-1])
+            g, add = sink.open(w)
+            if ops.embed_grad_ok(ids, dy2, g):
+                ops.embed_grad_(ids, dy2, g, add)
+                sink.close(w)
+            else:
+                sink.add(w, torch.ops.aten.embedding_dense_backward(dy2, ids, w.shape[0], -1, False))
+        return None, None
+
+
+def embedding(ids: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``w[ids]`` for ids ``[T]``; the gradient of a weight with a sink goes straight into its flat gradient."""
+    if torch.is_grad_enabled() and w.requires_grad and getattr(w, "_llmctl_grad_sink", None) is not None:
+        return _Embedding.apply(ids, w)
+    return F.embedding(ids, w)
 
 
 def data_grad(dy: torch.Tensor, w: torch.nn.Parameter) -> torch.Tensor:

@@ -25,7 +25,7 @@ import torch.nn.functional as F
 
 from llmctl import ops
 from llmctl.config.knobs import knobs
-from llmctl.exec.linear import data_grad, linear, swiglu_data_grad, weight_grad
+from llmctl.exec.linear import data_grad, embedding, linear, swiglu_data_grad, weight_grad
 from llmctl.parallel import async_tp
 from llmctl.parallel import context_parallel as cp
 from llmctl.parallel import tensor_parallel as tp
@@ -499,7 +499,7 @@ class DecoderLM(nn.Module):
         if pc.tp_size > 1:
             x = tp.vocab_parallel_embedding(ids, self.embed, self.vocab_start, pc.tp_group, pc.sequence_parallel)
         else:
-            x = F.embedding(ids, self.embed)
+            x = embedding(ids, self.embed)
         if self.pos_embed is not None:
             if positions is not None:  # explicit (e.g. per-document) positions
                 pos = self.pos_embed[positions.long()]

@@ -23,6 +23,8 @@ from .functional import (
     decode_norm_qkv_cache,
     decode_qkv_rope_cache,
     decode_up_swiglu,
+    embed_grad_,
+    embed_grad_ok,
     embed_rows,
     flash_attention,
     gelu,
@@ -52,6 +54,8 @@ from .functional import (
 __all__ = [
     "ref", "native_available", "adamw_step_", "add_layernorm", "add_rmsnorm", "clip_scale", "col_sum_", "cross_entropy", "decode_linear",
     "decode_attention_qkv", "decode_fused_ok", "decode_linear_add_rmsnorm", "decode_norm_linear", "decode_norm_qkv_cache", "decode_qkv_rope_cache", "decode_up_swiglu",
+    "embed_grad_",
+    "embed_grad_ok",
     "embed_rows",
     "flash_attention", "gelu", "kv_cache_write", "qkv_flash_attention", "qkv_split_cache", "l2norm_sq", "layernorm", "paged_attention_decode",
     "paged_prefill_attention", "prefill_work_list", "attn_merge_",

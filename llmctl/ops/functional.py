@@ -447,6 +447,24 @@ def col_sum_(x, out, add: bool):
         out.copy_(x.sum(0))
 
 
+EMBED_GRAD_TOKENS = 65536  # csrc/embed_grad.hip ranks the tokens by comparing all pairs
+
+
+def embed_grad_ok(ids, dy, g) -> bool:
+    """Whether ``embed_grad_`` (csrc/embed_grad.hip) takes these ids, rows and gradient."""
+    return (use_native(dy) and dy.dim() == 2 and dy.dtype == torch.bfloat16 and dy.stride(1) == 1 and dy.shape[1] % 8 == 0
+            and dy.stride(0) % 8 == 0 and dy.data_ptr() % 16 == 0 and 0 < dy.shape[0] <= EMBED_GRAD_TOKENS
+            and ids.dim() == 1 and ids.dtype == torch.int64 and ids.is_contiguous() and ids.is_cuda
+            and g.is_cuda and g.is_contiguous() and g.data_ptr() % 16 == 0 and g.dtype in (torch.bfloat16, torch.float32))
+
+
+def embed_grad_(ids, dy, g, add: bool):
+    """``g [V, H] (+)=`` the rows of ``dy [T, H]`` summed by their ids, in fp32 and in the same order every time: an embedding's gradient."""
+    if not add:
+        g.zero_()
+    native().embed_grad_(ids, dy, g, add)
+
+
 def l2norm_sq(t: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Sum of squares of ``t`` accumulated (fp32) into ``out`` (allocated if None)."""
     if out is None:

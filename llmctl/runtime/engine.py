@@ -260,7 +260,7 @@ class TrainingEngine:
             solo = ("embed", "lm_head") if (pp > 1 and mc.tie_word_embeddings) else ()
             self.flat = FlatParameters(named, bucket_numel=bucket_numel, align=align, solo=solo,
                                        grad_dtype=grad_dtype)
-            # kernel-written gradients (no AccumulateGrad pass); tied embeddings excluded
+            # kernel-written gradients (no AccumulateGrad pass)
             from llmctl.exec.linear import GradSink
 
             tied = mc.tie_word_embeddings
@@ -270,8 +270,11 @@ class TrainingEngine:
             leafs += ("attn_norm_w", "mlp_norm_w", "final_norm_w", "attn_norm_b", "mlp_norm_b", "final_norm_b")
             if pg.layout.tp == 1 and not mc.is_moe and not mc.gated_mlp:
                 leafs += ("bqkv", "bo", "b_up", "b_down")
+            # the embedding, where its rows are not shared out among ranks; tied, the output projection writes it too, and has to be here
+            if pg.layout.tp == 1 and not (tied and pp > 1):
+                leafs += ("embed",)
             self.grad_sink = GradSink()
-            self.flat.install_sinks(self.grad_sink, lambda n, p: n.split(".")[-1] in leafs)
+            self.flat.install_sinks(self.grad_sink, lambda n, p: 0 if n.split(".")[-1] not in leafs else 2 if tied and n == "embed" else 1)
         if pp > 1 and mc.tie_word_embeddings:
             from llmctl.parallel.pipeline import broadcast_tied_embedding
 

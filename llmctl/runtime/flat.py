@@ -168,10 +168,12 @@ class FlatParameters:
     def install_sinks(self, sink, predicate) -> int:
         """Attach a :class:`llmctl.exec.linear.GradSink` to every parameter for which
         ``predicate(name, p)`` holds; their gradients are then written (beta=0 first) by
-        the backward's kernels, so ``zero_grad`` skips them."""
-        self.sinked = [p for p in self.params if predicate(self.names[id(p)], p)]
+        the backward's kernels, so ``zero_grad`` skips them.  A predicate's number is how many
+        of them a backward writes."""
+        writes = {id(p): int(predicate(self.names[id(p)], p)) for p in self.params}
+        self.sinked = [p for p in self.params if writes[id(p)]]
         for p in self.sinked:
-            sink.attach(p)
+            sink.attach(p, writes[id(p)])
         self.sink = sink
         return len(self.sinked)
 
