@@ -227,6 +227,18 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         torch.mm(dy2.t(), x2, out=g)
 
 
+def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: torch.Tensor, add: bool) -> bool:
+    """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient; False: nothing done."""
+    M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
+    if not (_gemm64_ok(M, N, K, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32) and gb.dtype == g.dtype and gb.is_contiguous()
+            and g.stride(1) == 1 and g.stride(0) % 8 == 0 and g.data_ptr() % 16 == 0
+            and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3):
+        return False
+    from llmctl.ops._lib import native
+
+    return native().gemm64_wgrad_bias(dy2, x2, g, accumulate, gb, add)
+
+
 def side_chunks(M: int, N: int, K: int, T: int, F: int) -> int:
     """Chunks of 1024 elements per K-tile that ``gemm64_wgrad_swiglu``'s side job needs to cover
     ``T * F`` elements over the K-tiles of an ``[M, N] x K`` weight gradient (0: unsupported) —
@@ -382,6 +394,17 @@ class GradSink:
         wgrad_into(self._target(p), dy2, x2, accumulate=not p._llmctl_fresh)
         self._written(p)
 
+    def write_with_bias(self, p: torch.nn.Parameter, dy2: torch.Tensor, x2: torch.Tensor, b: torch.nn.Parameter) -> bool:
+        """``write`` with the bias ``b``'s gradient summed by the same kernel; False: it does not take them, nothing is written."""
+        if getattr(b, "_llmctl_grad_sink", None) is not self:
+            return False
+        gb, add = self.open(b)
+        if not wgrad_bias_into(self._target(p), dy2, x2, not p._llmctl_fresh, gb, add):
+            return False
+        self._written(p)
+        self.close(b)
+        return True
+
     def write_swiglu(self, p: torch.nn.Parameter, dy2: torch.Tensor, x2: torch.Tensor, dact: torch.Tensor,
                      gu: torch.Tensor) -> Optional[torch.Tensor]:
         """``write`` with the SwiGLU backward riding on the weight-gradient GEMM: returns
@@ -428,9 +451,12 @@ class _Linear(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1])
         x2 = x.reshape(-1, x.shape[-1])
         dw = None
+        bias = ctx.bparam is not None and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[1]:
             sink: Optional[GradSink] = getattr(ctx.wparam, "_llmctl_grad_sink", None)
-            if sink is not None:
+            if sink is not None and bias and sink.write_with_bias(ctx.wparam, dy2, x2, ctx.bparam):
+                bias = False
+            elif sink is not None:
                 sink.write(ctx.wparam, dy2, x2)  # weight grad first: lets its bucket's comm start earlier
             else:  # an ordinary gradient (AccumulateGrad adds it), still on the MFMA kernels when they fit
                 dw = torch.empty_like(w)
@@ -451,7 +477,7 @@ class _Linear(torch.autograd.Function):
                 dx = F.linear(dy, ctx.wt)
             else:
                 dx = dy.matmul(w)
-        db = bias_grad(ctx.bparam, dy2) if (ctx.bparam is not None and ctx.needs_input_grad[2]) else None
+        db = bias_grad(ctx.bparam, dy2) if bias else None
         return dx, dw, db
 
 

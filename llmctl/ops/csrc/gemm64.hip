@@ -1797,6 +1797,22 @@ void gemm64_ex(const at::Tensor& a, const at::Tensor& b, at::Tensor& out, bool a
   }
 }
 
+// g (+)= dy^T x and db (+)= the column sums of dy where the 256 x 128 tiles take the weight gradient (they carry the sums); false: nothing done, gemm64_ex and
+// col_sum_ are as fast or faster.  dy [T, M], x [T, N]; M, N in 256s, T in 128s, as gemm64_ex.
+bool gemm64_wgrad_bias(const at::Tensor& dy, const at::Tensor& x, at::Tensor g, bool accumulate, at::Tensor db, bool add) {
+  LLMCTL_CHECK(dy.dim() == 2 && x.dim() == 2 && dy.size(0) == x.size(0), "gemm64_wgrad_bias: dy [T, M], x [T, N]");
+  const long M = dy.size(1), N = x.size(1), K = dy.size(0);
+  if (!gemm64_supported(M, N, K) || N < 512) return false;
+  const c10::DeviceGuard dg(dy.device());
+  G64Args plan{};
+  plan.M = (int)M, plan.N = (int)N, plan.K = (int)K, plan.tiles_m = (int)(M / TM), plan.tiles_n = (int)(N / TN);
+  plan_split(plan, 0);
+  const int S = gemm_tall_splits(M, N, K, plan.n_main, (long)plan.tiles_m * plan.tiles_n - plan.n_main, plan.splits);
+  if (S == 0) return false;
+  gemm_tall(dy, x, g, true, accumulate, S, db, add);
+  return true;
+}
+
 // Down-projection data gradient fused with the SwiGLU backward:
 //   dAct = dy · W_down  (dy [M, H], W_down [H, F]; gemm64's dgrad layout, W read K-major)
 //   dgu[:, :F] = dAct * u * sig(g) * (1 + g (1 - sig(g))),  dgu[:, F:] = dAct * silu(g)
@@ -2126,6 +2142,7 @@ TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
   m.impl("gemm64_up_swiglu", &gemm64_up_swiglu);
   m.impl("gemm64_swiglu_fwd", &gemm64_swiglu_fwd);
   m.impl("gemm64_ex", &gemm64_ex);
+  m.impl("gemm64_wgrad_bias", &gemm64_wgrad_bias);
   m.impl("gemm64_swiglu_dgrad", &gemm64_swiglu_dgrad);
   m.impl("gemm64_wgrad_swiglu", &gemm64_wgrad_swiglu);
 }

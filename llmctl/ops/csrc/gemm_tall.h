@@ -4,5 +4,6 @@
 
 namespace llmctl {
 int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits);
-void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits);
+void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias = c10::nullopt,
+               bool bias_add = false);
 }  // namespace llmctl

@@ -31,7 +31,9 @@ struct TallArgs {
   const unsigned short* a;
   const unsigned short* b;
   void* c;
-  float* ws;  // [splits][M][N] fp32 partial sums (splits > 1)
+  float* ws;  // [splits][M][N] fp32 partial sums (splits > 1), then with a bias [splits][M]
+  void* bias;     // BIAS: [M], of c's type
+  int bias_add;
   long lda, ldb, ldc;
   int M, N, K;
   int tiles_m, tiles_n, splits;
@@ -46,7 +48,26 @@ __device__ __forceinline__ void fence_rows(f32x4_t (&acc)[8][4]) {
                  "+a"(acc[R + 3][1]), "+a"(acc[R + 3][2]), "+a"(acc[R + 3][3]));
 }
 
-template <bool AT, int OUT>
+// one MFMA; the two wait states are for operands that the compiler writes just ahead (a constant's copies: it does not look into the statement)
+__device__ __forceinline__ void mfma_acc(f32x4_t& c, const bf16x8_t& a, const bf16x8_t& b) {
+  asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %2, %1, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
+}
+
+template <int OUT>
+__device__ __forceinline__ void put1(void* out, int m, float v, int add) {
+  if constexpr (OUT >= OUT_STORE_F32) {
+    float* p = static_cast<float*>(out) + m;
+    *p = add ? *p + v : v;
+  } else {
+    unsigned short* p = static_cast<unsigned short*>(out) + m;
+    *p = f2bf(add ? bf2f(*p) + v : v);
+  }
+}
+
+// BIAS (weight gradients): dy's column sums, this product's row sums of A, ride along.  The waves of the first four tile columns take one of the tile's 16-row
+// blocks each, two more MFMAs against ones to a K-tile's 64 (a pass over dy and a launch to add its parts were 10 to 14 us a bias, 48 of them in a gpt2-125m step
+// of 8192 tokens: the step 12174 us, so 11860).  The block's fragments are read where its image is: of A_lo(t+1) in P1(t), of A_hi(t) in P0(t).
+template <bool AT, int OUT, bool BIAS>
 __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_tall_kernel(TallArgs args) {
   __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -92,6 +113,16 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   fence_rows<0>(acc);
   fence_rows<4>(acc);
+  const int blk = tn * 2 + wc;  // BIAS: of this tile's eight row blocks of a wave row
+  const bool sum_lo = BIAS && blk < 4, sum_hi = BIAS && blk >= 4 && blk < 8;
+  f32x4_t bacc = {0.f, 0.f, 0.f, 0.f};
+  bf16x8_t bf[2];
+  bf16x8_t ones = __builtin_bit_cast(bf16x8_t, s8_t{0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80});
+  if constexpr (BIAS) asm volatile("s_nop 7" : "+a"(bacc), "+v"(ones));  // (kept: not made anew for each use)
+  auto bias_frag = [&](const unsigned char* img) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) bf[ks] = frag<AT>(img, wr * 64 + 16 * (blk & 3), ks, lane);
+  };
 
   issue(K_<B_H0>{}, 0, 0, K_<4>{});
   issue(K_<A_LO>{}, 0, 0, K_<4>{});
@@ -110,6 +141,9 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       a_lo[i][ks] = frag<AT>(smem + A_LO * HALF, wr * 64 + 16 * i, ks, lane);
       b[0][i][ks] = frag<true>(smem + B_H0 * HALF, wc * 64 + 16 * i, ks, lane);
     }
+  if constexpr (BIAS) {
+    if (sum_lo) bias_frag(smem + A_LO * HALF);
+  }
   wait_vm<10>();
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
   bar();
@@ -130,6 +164,9 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       }
       if (q < 8) a_hi[q & 3][q >> 2] = frag<AT>(smem + s0 + A_HI * HALF, wr * 64 + 16 * (q & 3), q >> 2, lane);
       else if (NEXT && q < 12) b[P ^ 1][q & 3][0] = frag<true>(smem + s1 + B_H0 * HALF, wc * 64 + 16 * (q & 3), 0, lane);
+      if constexpr (BIAS) {
+        if (q == 12 && sum_hi) bias_frag(smem + s0 + A_HI * HALF);
+      }
     }
     const unsigned soa = (unsigned)(k0 + t + 3) * a_step, sob = (unsigned)(k0 + t + 3) * b_step, l1 = lds0 + s0;
 #pragma unroll
@@ -144,6 +181,10 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
       }
       if (NEXT && q < 8) a_lo[q & 3][q >> 2] = frag<AT>(smem + s1 + A_LO * HALF, wr * 64 + 16 * (q & 3), q >> 2, lane);
       else if (NEXT && q < 12) b[P ^ 1][q & 3][1] = frag<true>(smem + s1 + B_H0 * HALF, wc * 64 + 16 * (q & 3), 1, lane);
+      if constexpr (BIAS) {
+        if ((q == 4 || q == 8) && blk < 8) mfma_acc(bacc, bf[q / 4 - 1], ones);
+        if (NEXT && q == 12 && sum_lo) bias_frag(smem + s1 + A_LO * HALF);
+      }
     }
     if constexpr (NEXT) {
       wait_vm<NEXT ? WAIT : 0>();
@@ -175,6 +216,14 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const int g = lane >> 4, i16 = lane & 15;
   const long row0 = (long)tm * TM + wr * 128 + i16;
   const int col0 = tn * TALL_N + wc * 64;
+  if constexpr (BIAS) {
+    asm volatile("s_nop 7\n\ts_nop 7" : "+a"(bacc));
+    if (blk < 8 && g == 0) {  // bacc[r]: row l & 15 of the block, the same in every r and g
+      const int m = tm * TM + wr * 128 + 16 * blk + i16;
+      if (args.splits > 1) args.ws[((long)args.splits * args.N + sp) * args.M + m] = bacc[0];
+      else put1<OUT>(args.bias, m, bacc[0], args.bias_add);
+    }
+  }
   if (args.splits > 1 || OUT >= OUT_STORE_F32) {
     const bool part = args.splits > 1;
     const long ld = part ? args.N : args.ldc;
@@ -217,12 +266,19 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 }
 
 // out (+)= the partial sums, added in the order of K; a thread's 8 columns of a row
-template <int OUT>
+template <int OUT, bool BIAS>
 __global__ __launch_bounds__(256) void gemm_tall_reduce(TallArgs args) {
   const long e = ((long)blockIdx.x * 256 + threadIdx.x) * 8;  // M N is a multiple of 2048
   const long row = e / args.N, col = e - row * args.N, MN = (long)args.M * args.N;
   float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   const float* W = args.ws + e;
+  if (BIAS && e / 8 < args.M) {  // (N >= 512: threads enough)
+    const float* B = args.ws + args.splits * MN + e / 8;
+    float t = 0.f;
+#pragma unroll 4
+    for (int s = 0; s < args.splits; ++s) t += B[(long)s * args.M];
+    put1<OUT>(args.bias, (int)(e / 8), t, args.bias_add);
+  }
 #pragma unroll 4
   for (int s = 0; s < args.splits; ++s) {
     const f32x4_t x0 = *reinterpret_cast<const f32x4_t*>(W + s * MN), x1 = *reinterpret_cast<const f32x4_t*>(W + s * MN + 4);
@@ -252,8 +308,15 @@ void launch(const TallArgs& g, int out) {
   const dim3 grid(g.tiles_m * g.tiles_n * g.splits), red((unsigned)((long)g.M * g.N / 2048));
   auto go = [&](auto out_c) {
     constexpr int OUT = decltype(out_c)::value;
-    hipLaunchKernelGGL((gemm_tall_kernel<AT, OUT>), grid, dim3(NT4), 0, stream(), g);
-    if (g.splits > 1) hipLaunchKernelGGL((gemm_tall_reduce<OUT>), red, dim3(256), 0, stream(), g);
+    auto with = [&](auto bias_c) {
+      constexpr bool BIAS = decltype(bias_c)::value;
+      hipLaunchKernelGGL((gemm_tall_kernel<AT, OUT, BIAS>), grid, dim3(NT4), 0, stream(), g);
+      if (g.splits > 1) hipLaunchKernelGGL((gemm_tall_reduce<OUT, BIAS>), red, dim3(256), 0, stream(), g);
+    };
+    if constexpr (AT) {
+      if (g.bias != nullptr) return with(std::true_type{});
+    }
+    with(std::false_type{});
   };
   switch (out) {
     case OUT_STORE: go(K_<OUT_STORE>{}); break;
@@ -285,7 +348,9 @@ int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int split
 }
 
 // out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N and K of 128, K >= 256 splits.
-void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits) {
+// bias [M] (+)= the row sums of A, of out's type (at, N >= 512).
+void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias,
+               bool bias_add) {
   LLMCTL_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2 && a.is_cuda() && b.is_cuda() && out.is_cuda(), "gemm_tall: 2-D GPU operands");
   const bool f32 = out.scalar_type() == at::kFloat;
   LLMCTL_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && (f32 || out.scalar_type() == at::kBFloat16),
@@ -300,12 +365,15 @@ void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at
   LLMCTL_CHECK(rows16(a, 8) && rows16(b, 8) && rows16(out, f32 ? 4 : 8), "gemm_tall: 16-byte aligned rows, unit column stride");
   const long a_span = (at_ ? K : (long)TM) * a.stride(0) * 2, b_span = K * b.stride(0) * 2;
   LLMCTL_CHECK(a_span < (1L << 31) && b_span < (1L << 31) && M * N / 2048 < (1L << 31), "gemm_tall: operand too large for 32-bit offsets");
+  LLMCTL_CHECK(!bias.has_value() || (at_ && N >= 4 * TALL_N && bias->is_cuda() && bias->is_contiguous() && bias->numel() == M &&
+                                     bias->scalar_type() == out.scalar_type()),
+               "gemm_tall: a bias goes with a transposed A and 512 columns, [M] of out's type");
   const c10::DeviceGuard guard(a.device());
-  TallArgs g{bf_ptr(a), bf_ptr(b), out.data_ptr(), nullptr, (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K,
+  TallArgs g{bf_ptr(a), bf_ptr(b), out.data_ptr(), nullptr, bias.has_value() ? bias->data_ptr() : nullptr, bias_add, (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K,
              (int)(M / TM), (int)(N / TALL_N), (int)splits};
   at::Tensor ws;
   if (splits > 1) {
-    ws = at::empty({splits, M, N}, a.options().dtype(at::kFloat));
+    ws = at::empty({splits * M * (N + 1)}, a.options().dtype(at::kFloat));
     g.ws = ws.data_ptr<float>();
   }
   const int o = (f32 ? OUT_STORE_F32 : OUT_STORE) + (accumulate ? 1 : 0);

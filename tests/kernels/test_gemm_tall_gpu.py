@@ -57,3 +57,45 @@ def test_gemm64_takes_either_tile(at, M, N, K, odd_rows):
     A, B = (a.t() if at else a).double(), b.double()
     ref, bound = A @ B, _bound(A, B, K, 16)
     assert bool(((out.double() - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
+
+
+@pytest.mark.parametrize("M,N,K,S,pad", [(256, 512, 256, 1, 8), (512, 640, 640, 2, 0), (768, 3072, 8192, 3, 0), (2304, 768, 1152, 4, 8)])
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("add", [False, True])
+def test_column_sums_ride_along(M, N, K, S, pad, f32, add):
+    """The product as without them, the sums of dy's columns beside it."""
+    from llmctl.ops._lib import native
+
+    dy, x = _operands(True, M, N, K, pad)
+    dy = (dy.float() + 0.5).bfloat16()  # sums that do not cancel
+    dt = torch.float32 if f32 else torch.bfloat16
+    out, plain = torch.ones(M, N, device="cuda", dtype=dt), torch.ones(M, N, device="cuda", dtype=dt)
+    db = torch.linspace(-1, 1, M, device="cuda").to(dt)
+    ref = dy.double().sum(0) + (db.double() if add else 0.0)
+    bound = (K + S + 1) * 2.0**-24 * dy.double().abs().sum(0)
+    native().gemm_tall(dy, x, out, True, add, S, db, add)
+    native().gemm_tall(dy, x, plain, True, add, S)
+    assert torch.equal(out, plain)
+    err = (db.double() - ref).abs()
+    assert bool((err <= bound + (0 if f32 else 2.0**-8) * (ref.abs() + bound)).all())
+
+
+@pytest.mark.parametrize("tokens,out,inn", [(1024, 768, 3072), (2048, 2304, 768), (4096, 4096, 4096), (1000, 768, 768), (1024, 768, 256)])
+def test_linear_backward_with_sinks(tokens, out, inn):
+    """Both gradients land in their flat views whichever kernel takes the weight's, and each is told of once."""
+    from llmctl.exec.linear import GradSink, linear
+
+    torch.manual_seed(1)
+    w = torch.nn.Parameter((torch.randn(out, inn, device="cuda") * 0.02).bfloat16())
+    b = torch.nn.Parameter(torch.zeros(out, device="cuda", dtype=torch.bfloat16))
+    sink, told = GradSink(), []
+    sink.callbacks.append(lambda p: told.append(p))
+    for p in (w, b):
+        p.grad = torch.full_like(p, float("nan"))
+        sink.attach(p)
+    x, dy = torch.randn(tokens, inn, device="cuda").bfloat16(), torch.randn(tokens, out, device="cuda").bfloat16()
+    linear(x, w, b).backward(dy)
+    assert len(told) == 2 and {id(p) for p in told} == {id(w), id(b)}
+    linear(x, w, b).backward(dy)
+    for p, ref in ((w, dy.double().t() @ x.double()), (b, dy.double().sum(0))):
+        assert bool(((p.grad.double() - 2 * ref).abs() <= 2.0**-7 * 2 * ref.abs() + 1e-3 * ref.abs().max()).all())
