@@ -168,11 +168,11 @@ class DumazenLM(nn.Module):
         mult, eps, dt = self.cfg.residual_mult, self.cfg.layer_norm_eps, self.dtype
         x, h = hops.embed_f32(b.ids, self.embed)
         for i, layer in enumerate(self.layers):
-            y = layer.mixer.step(h, b, cache.layer(i))
+            y = layer.mixer.step(h, b, cache.layer(i), late=True)
             (y1, s1), (y2, s2) = y if isinstance(y, tuple) else ((y, 1.0), (None, 0.0))
             h = hops.norm_add_f32_(x, y1, s1, y2, s2, layer.norm1, mult, eps, True, dt)
             if layer.ff is not None:
-                h = hops.norm_add_f32_(x, layer.ff(h), 1.0, None, 0.0, layer.norm2, mult, eps, True, dt)
+                h = hops.norm_add_f32_(x, layer.ff(h, late=True), 1.0, None, 0.0, layer.norm2, mult, eps, True, dt)
             if trail is not None:
                 trail.append(x.clone())
         return x if rows is None else x.index_select(0, rows)

@@ -350,8 +350,9 @@ class GroupedAttention(nn.Module):
     def state_shapes(self):
         return [self.conv.state_shape()] if self.conv is not None else []
 
-    def step(self, h: torch.Tensor, b: StepBatch, cache, z: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """``z``: the input projection ``h W_qkv^T`` if the caller has made it (as columns of a wider product)."""
+    def step(self, h: torch.Tensor, b: StepBatch, cache, z: Optional[torch.Tensor] = None, late: bool = False) -> torch.Tensor:
+        """``z``: the input projection ``h W_qkv^T`` if the caller has made it (as columns of a wider product); ``late``: the result may come as
+        :func:`~llmctl.ops.hybrid.linear_parts` leaves it."""
         rows, states = cache if isinstance(cache, tuple) else (cache, ())
         T = h.shape[0]
         if z is None:
@@ -382,7 +383,7 @@ class GroupedAttention(nn.Module):
             outs.append(hops.latent_attention_decode(q[b.Tp:], rows, b.d_bt, b.d_ctx, self.window, self.sink, self.scale,
                                                      self.dv, max_ctx=b.d_max_ctx, **opt))
         o = outs[0] if len(outs) == 1 else torch.cat(outs)
-        return hops.linear(o.reshape(T, self.H * self.dv), self.w_o)
+        return (hops.linear_parts if late else hops.linear)(o.reshape(T, self.H * self.dv), self.w_o)
 
 
 class ClampedGLU(nn.Module):
@@ -575,14 +576,14 @@ class DenseFF(nn.Module):
         _init(self.w_up, 0.02)
         _init(self.w_down, 0.02)
 
-    def forward(self, h: torch.Tensor):
+    def forward(self, h: torch.Tensor, late: bool = False):
         if hops.rows_ok(h, self.w_up, self.b_up):  # the activation in the product's epilogue
             z = hops.rows_linear(h, self.w_up, self.b_up, self.act, self.ff)
             a = z[:, :self.ff]
         else:
             z = F.linear(h, self.w_up, self.b_up)
             a = hops.act_any(z[:, :self.ff], self.act)
-        y = hops.linear(a, self.w_down, self.b_down)
+        y = (hops.linear_parts if late else hops.linear)(a, self.w_down, self.b_down)
         return (y, z[:, self.ff:]) if self.side else y
 
 
@@ -791,7 +792,7 @@ class GatedDeltaRule(nn.Module):
 
     _norm_rows = GatedLinearAttention._norm_rows
 
-    def step(self, h: torch.Tensor, b: StepBatch, state, z: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def step(self, h: torch.Tensor, b: StepBatch, state, z: Optional[torch.Tensor] = None, late: bool = False) -> torch.Tensor:
         S, carried = _own_states(state)
         H, G, dv = self.H, self.G, self.dv
         if z is None:
@@ -800,7 +801,7 @@ class GatedDeltaRule(nn.Module):
         qk, v = hops.conv_silu_unit(z[:, :c], self.conv.tap_major(), None, carried, b, G, G, self.dk, self.dk ** -0.5, self.key_eps)
         y = hops.memory_scan(qk[:, :G], qk[:, G:], v.view(-1, H, dv), "delta", S, b, ga=z[:, g0:g0 + H], gb=z[:, g0 + H:g0 + 2 * H],
                              a_log=self.a_log, dt_bias=self.dt_bias, norm=(self._norm_rows(), z[:, c:g0], self.eps))
-        return hops.linear(y, self.w_o)
+        return (hops.linear_parts if late else hops.linear)(y, self.w_o)
 
 
 class Mamba2(nn.Module):
@@ -840,7 +841,7 @@ class Mamba2(nn.Module):
     def state_shapes(self):
         return [(self.H, self.N, self.dv), self.conv.state_shape()]
 
-    def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
+    def step(self, h: torch.Tensor, b: StepBatch, state, late: bool = False) -> torch.Tensor:
         S, carried = _own_states(state)
         T, n = h.shape[0], self.inner
         z = hops.odd_linear(h, self.w_in)
@@ -849,7 +850,8 @@ class Mamba2(nn.Module):
         B, C = (xbc[:, n + i * self.G * self.N:n + (i + 1) * self.G * self.N].unflatten(1, (self.G, self.N)) for i in range(2))
         o = hops.memory_scan(C, B, xbc[:, :n].unflatten(1, (self.H, self.dv)), "ssm", S, b, ga=z[:, c:c + self.H], a_log=self.a_log,
                              dt_bias=self.dt_bias, skip=self.skip)
-        return hops.linear(hops.gate_groupnorm(o.view(T, n), z[:, :n], self.norm, self.norm_groups, self.eps, h.dtype), self.w_o)
+        y = hops.gate_groupnorm(o.view(T, n), z[:, :n], self.norm, self.norm_groups, self.eps, h.dtype)
+        return (hops.linear_parts if late else hops.linear)(y, self.w_o)
 
 
 class Retention(nn.Module):
@@ -884,7 +886,7 @@ class Retention(nn.Module):
     def state_shapes(self):
         return [(self.H, self.dk, self.dv)]
 
-    def step(self, h: torch.Tensor, b: StepBatch, state) -> torch.Tensor:
+    def step(self, h: torch.Tensor, b: StepBatch, state, late: bool = False) -> torch.Tensor:
         S = _own_states(state)[0]
         H, dk, dv = self.H, self.dk, self.dv
         z = hops.odd_linear(h, self.w_in)
@@ -892,7 +894,7 @@ class Retention(nn.Module):
         v0, g0 = 2 * H * dk, 2 * H * dk + H * dv
         y = hops.memory_scan(qk[:, :H], qk[:, H:], z[:, v0:g0].unflatten(1, (H, dv)), "fixed", S, b, log_decay=self.log_decay,
                              norm=(None, z[:, g0:g0 + H * dv], self.eps))
-        return hops.linear(y, self.w_o)
+        return (hops.linear_parts if late else hops.linear)(y, self.w_o)
 
 
 class ParallelMixers(nn.Module):
@@ -934,11 +936,12 @@ class ParallelMixers(nn.Module):
             self._w_key = key
         return self._w
 
-    def step(self, h: torch.Tensor, b: StepBatch, cache):
+    def step(self, h: torch.Tensor, b: StepBatch, cache, late: bool = False):
+        kw = {"late": True} if late else {}
         rows, states = cache
         nl = len(self.left.state_shapes())
         w, bias, c0 = self._stacked()
         z = hops.odd_linear(h, w, bias)
-        yl = self.left.step(h, b, (rows, tuple(states[:nl])), z=z[:, :self.left.w_in.shape[0]])
-        yr = self.right.step(h, b, (rows, tuple(states[nl:])), z=z[:, c0:c0 + self.right.w_in.shape[0]])
+        yl = self.left.step(h, b, (rows, tuple(states[:nl])), z=z[:, :self.left.w_in.shape[0]], **kw)
+        yr = self.right.step(h, b, (rows, tuple(states[nl:])), z=z[:, c0:c0 + self.right.w_in.shape[0]], **kw)
         return (yl, self.left_scale), (yr, self.right_scale)

@@ -27,4 +27,23 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::opti
   return y;
 }
 
+// x w^T as fp32 sums over ``parts`` ranges of K, [parts or fewer, M, N], for norm_add_parts_f32_
+at::Tensor rows_parts(const at::Tensor& x, const at::Tensor& w, int64_t parts) {
+  HYB_CHECK(x.is_cuda() && w.is_cuda() && x.dim() == 2 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16,
+            "rows_parts: bf16 GPU matrices");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  HYB_CHECK(M <= 32 && w.size(1) == K && K % 8 == 0 && K > 0 && x.stride(1) == 1 && w.stride(1) == 1 && x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 &&
+                reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0,
+            "rows_parts: at most 32 rows, K a multiple of 8, rows aligned to 16 bytes");
+  HYB_CHECK(parts >= 1 && parts <= 16, "rows_parts: 1 .. 16 ranges");
+  c10::DeviceGuard guard(x.device());
+  const int64_t part = ((K + parts - 1) / parts + 31) / 32 * 32;
+  at::Tensor y = at::empty({(K + part - 1) / part, M, N}, x.options().dtype(at::kFloat));
+  if (M == 0 || N == 0) return y;
+  stream_linear::Args a{reinterpret_cast<const bf16_t*>(x.data_ptr()), (long)x.stride(0), reinterpret_cast<const bf16_t*>(w.data_ptr()), (long)w.stride(0),
+                        nullptr, y.data_ptr(), (int)M, (int)N, (int)K, 0, 0, 1};
+  stream_linear::launch_parts(a, (int)parts, cur_stream());
+  return y;
+}
+
 }  // namespace llmctl_hybrid

@@ -117,6 +117,59 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(float* __restrict__ x, con
   }
 }
 
+// norm_add_kernel for one or two results that are still fp32 sums over ranges of K (rows_parts) and, the first, without its bias: a thread's quads of all ranges
+// are in flight at once.  VQ quads a thread.
+template <int VQ>
+__global__ __launch_bounds__(NT) void norm_add_parts_kernel(float* __restrict__ x, const float* __restrict__ y1, int n1, const bf16_t* __restrict__ bias,
+                                                            float s1, const float* __restrict__ y2, int n2, float s2, const float* __restrict__ w,
+                                                            float mult, float plus, bf16_t* __restrict__ h, int W, int64_t TW, float eps) {
+  __shared__ float red[NW];
+  const int64_t row = blockIdx.x;
+  float4 a[VQ], xv[VQ], wv[VQ];
+  float q = 0.f;
+  auto add = [&](const float* y, int n, float scale) {
+    float4 p[VQ];
+#pragma unroll
+    for (int i = 0; i < VQ; ++i) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int s = 0; s < n; ++s)
+#pragma unroll
+      for (int i = 0; i < VQ; ++i) {
+        const float4 v = *reinterpret_cast<const float4*>(y + s * TW + row * W + min((int)(threadIdx.x + i * NT) * 4, W - 4));
+        p[i].x += v.x, p[i].y += v.y, p[i].z += v.z, p[i].w += v.w;
+      }
+#pragma unroll
+    for (int i = 0; i < VQ; ++i) a[i].x = fmaf(scale, p[i].x, a[i].x), a[i].y = fmaf(scale, p[i].y, a[i].y), a[i].z = fmaf(scale, p[i].z, a[i].z), a[i].w = fmaf(scale, p[i].w, a[i].w);
+  };
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
+    xv[i] = *reinterpret_cast<const float4*>(x + row * W + c);
+    wv[i] = *reinterpret_cast<const float4*>(w + c);
+    a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (bias != nullptr) {
+      const float4 b = ld4(bias + c);
+      a[i] = make_float4(s1 * b.x, s1 * b.y, s1 * b.z, s1 * b.w);
+    }
+  }
+  add(y1, n1, s1);
+  if (y2 != nullptr) add(y2, n2, s2);
+#pragma unroll
+  for (int i = 0; i < VQ; ++i)
+    if ((int)(threadIdx.x + i * NT) * 4 < W) q += a[i].x * a[i].x + a[i].y * a[i].y + a[i].z * a[i].z + a[i].w * a[i].w;
+  const float f = mult / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    if (c >= W) break;
+    const float4 o = make_float4(xv[i].x + a[i].x * f * (wv[i].x + plus), xv[i].y + a[i].y * f * (wv[i].y + plus), xv[i].z + a[i].z * f * (wv[i].z + plus),
+                                 xv[i].w + a[i].w * f * (wv[i].w + plus));
+    *reinterpret_cast<float4*>(x + row * W + c) = o;
+    const float v[4] = {o.x, o.y, o.z, o.w};
+    stn<bf16_t, 4>(h + row * W + c, v);
+  }
+}
+
 // one workgroup per (row, part)
 template <typename T, int N>
 __global__ __launch_bounds__(NT) void gate_groupnorm_kernel(const float* __restrict__ o, const T* __restrict__ z, int64_t z_st, const float* __restrict__ w,
@@ -269,6 +322,37 @@ at::Tensor norm_add_f32_(at::Tensor x, const at::Tensor& y1, double s1, const c1
     if (v4) go(norm_add_kernel<Tt, 4>);
     else go(norm_add_kernel<Tt, 1>);
   });
+  return h;
+}
+
+// norm_add_f32_ of results that are fp32 sums over ranges of K (rows_parts: [ranges, T, W]), y1 still without its bias; h is bf16
+at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const c10::optional<at::Tensor>& bias, double s1, const c10::optional<at::Tensor>& y2,
+                               double s2, const at::Tensor& w, double mult, double eps, bool one_plus) {
+  HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kFloat, "x: contiguous fp32 [T, W]");
+  const int64_t T = x.size(0), W = x.size(1);
+  auto parts = [&](const at::Tensor& t) {
+    return t.is_cuda() && t.dim() == 3 && t.is_contiguous() && t.scalar_type() == at::kFloat && t.size(0) >= 1 && t.size(1) == T && t.size(2) == W &&
+           reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+  };
+  HYB_CHECK(parts(y1) && (!y2.has_value() || parts(*y2)), "y: fp32 [ranges, T, W], x's rows");
+  HYB_CHECK(!bias.has_value() || (bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == W &&
+                                  reinterpret_cast<uintptr_t>(bias->data_ptr()) % 8 == 0),
+            "bias: bf16 [W]");
+  HYB_CHECK(f32w(w, W) && W % 4 == 0 && W <= 16 * NT && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
+            "w: fp32 [W]; W a multiple of 4, at most 4096");
+  c10::DeviceGuard guard(x.device());
+  at::Tensor h = at::empty({T, W}, x.options().dtype(at::kBFloat16));
+  if (T == 0 || W == 0) return h;
+  auto go = [&](auto kern) {
+    kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(x.data_ptr<float>(), y1.data_ptr<float>(), (int)y1.size(0),
+                                                     bias.has_value() ? reinterpret_cast<const bf16_t*>(bias->data_ptr()) : nullptr, (float)s1,
+                                                     y2.has_value() ? y2->data_ptr<float>() : nullptr, y2.has_value() ? (int)y2->size(0) : 0, (float)s2,
+                                                     w.data_ptr<float>(), (float)mult, one_plus ? 1.0f : 0.0f, reinterpret_cast<bf16_t*>(h.data_ptr()), (int)W, T * W, (float)eps);
+  };
+  if (W <= 4 * NT) go(norm_add_parts_kernel<1>);
+  else if (W <= 8 * NT) go(norm_add_parts_kernel<2>);
+  else go(norm_add_parts_kernel<4>);
   return h;
 }
 

@@ -35,6 +35,7 @@ struct Args {
   int act_cols;  // of the first that many columns
   int f32;  // y is fp32
   int rows = 0;  // outputs of a workgroup, at most 16 NT
+  int part = 0;  // > 0: blockIdx.y takes that much of K (a multiple of 32) and writes its own fp32 y [M, N]; no bias, no activation
 };
 
 __device__ __forceinline__ uint4 load_or_zero(const unsigned short* p, bool in) {
@@ -64,6 +65,13 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
   __shared__ acc_t red[NW][NT * MT][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, kg = lane >> 4;
+  if (g.part > 0) {
+    const int k0 = blockIdx.y * g.part;
+    g.x += k0;
+    g.w += k0;
+    g.K = min(g.part, g.K - k0);
+    g.y = static_cast<float*>(g.y) + (long)blockIdx.y * g.M * g.N;
+  }
   const int n0 = blockIdx.x * g.rows, n1 = min(n0 + g.rows, g.N);
   const unsigned short* wp[NT];
 #pragma unroll
@@ -148,7 +156,8 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
 template <int NT, int MT, int NW, int U>
 inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
   g.rows = rows;
-  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + rows - 1) / rows)), NW * 64, 0, st>>>(g);
+  const unsigned parts = g.part > 0 ? (unsigned)((g.K + g.part - 1) / g.part) : 1u;
+  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + rows - 1) / rows), parts), NW * 64, 0, st>>>(g);
 }
 
 // Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to
@@ -177,6 +186,25 @@ inline void launch(const Args& g, hipStream_t st) {
     go<3, 1, 4, 4>(g, st, rows);
   } else {
     go<4, 1, 4, 4>(g, st, rows);
+  }
+}
+
+// K in ``parts`` ranges, each its own fp32 [M, N], for a reader that adds them: one round of 256 workgroups of at most 64 rows
+inline void launch_parts(Args g, int parts, hipStream_t st) {
+  g.part = ((g.K + parts - 1) / parts + 31) / 32 * 32;
+  g.f32 = 1;
+  const int n = (g.K + g.part - 1) / g.part;
+  const int rows = ((g.N * n + 255) / 256 + 3) / 4 * 4;
+  if (g.M > 16) {
+    if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
+    else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);
+    else go<4, 2, 4, 4>(g, st, rows > 64 ? 64 : rows);
+  } else if (rows <= 16) {
+    go<1, 1, 4, 8>(g, st, rows);
+  } else if (rows <= 32) {
+    go<2, 1, 4, 8>(g, st, rows);
+  } else {
+    go<4, 1, 4, 4>(g, st, rows > 64 ? 64 : rows);
   }
 }
 

@@ -22,7 +22,7 @@ import torch
 from . import ref_hybrid as ref
 from ._lib import native_hybrid, use_native
 from .functional import odd_linear as wide_linear
-from .functional import stream_ok, wants_grad
+from .functional import stream_ok, stream_takes, wants_grad
 
 
 def layernorm_f32(x, w, b, eps: float, out_dtype):
@@ -520,6 +520,37 @@ def odd_linear(x, w, b=None):
     return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else wide_linear(x, w, b)
 
 
+class RowParts:
+    """A product of a few rows that is still fp32 sums ``[ranges, T, W]`` over ranges of K, and its bias: :func:`norm_add_f32_` adds them in its own
+    pass; :meth:`total` is the product as a tensor."""
+
+    def __init__(self, parts, bias):
+        self.parts, self.bias = parts, bias
+
+    def total(self):
+        y = self.parts.sum(0)
+        return (y if self.bias is None else y + self.bias.float()).to(torch.bfloat16)
+
+
+def row_ranges(M: int, N: int) -> int:
+    """Ranges of K for :class:`RowParts`, so that the weights of few outputs are streamed by all of the chip.  Product and residual norm in a graph, weights
+    from HBM, us, one launch of whole sums or the library's / here in 1, 2, 4, 8 ranges: 1 row 2048 x 8192 14.4 / 14.1, 12.5, 13.1, 13.7, 2048 x 2048 8.0 /
+    7.9, 7.5, 8.0, 8.6, 1024 x 4096 8.7 / 8.6, 7.7, 7.1, 7.9, 4096 x 4096 13.9 / 13.4, 14.4, 14.5, 14.3; 16 rows 2048 x 8192 16.9 / 18.6, 14.6, 13.9, 14.4,
+    2048 x 2048 9.4 / 9.2, 8.6, 8.6, 9.3, 1024 x 4096 11.1 / 10.8, 9.1, 8.0, 8.5, 1024 x 1024 6.6 / 6.5, 6.5, 6.1, 6.5, 4096 x 4096 17.1 / 15.3, 14.9, 15.2,
+    15.5; 32 rows 2048 x 8192 19.8 / 25.5, 18.4, 15.6, 15.7, 2048 x 2048 11.3 / 11.0, 9.7, 9.1, 11.0."""
+    if M <= 4:
+        return 4 if N <= 1024 else 2 if N <= 2048 else 1
+    return 4 if N <= 2048 or M > 16 else 2
+
+
+def linear_parts(x, w, b=None):
+    """:func:`linear` for a reader that takes :class:`RowParts` as well."""
+    M, N = x.shape[0], w.shape[0]
+    if M <= 32 and N % 4 == 0 and N <= 4096 and stream_takes(x, w, b) and (b is None or b.data_ptr() % 8 == 0):
+        return RowParts(native_hybrid().rows_parts(x, w, row_ranges(M, N)), b)
+    return linear(x, w, b)
+
+
 def linear_f32(x, w):
     """``x @ w^T`` with an fp32 result (inputs in their own dtype, fp32 accumulation)."""
     if x.dtype == torch.float32:
@@ -899,7 +930,10 @@ def gate_groupnorm(o, z, w, groups: int, eps: float, out_dtype):
 def norm_add_f32_(x, y1, s1: float, y2, s2: float, w, mult: float, eps: float, one_plus: bool, out_dtype):
     """The end of a sublayer whose only norm is on its result: ``y = s1 y1 (+ s2 y2)``, ``x += mult y / rms(y) (w + one_plus)``
     in place on the fp32 stream, and the next sublayer's input, x itself, in ``out_dtype``.  ``y [T, W]`` in the activation
-    dtype (row-strided views allowed)."""
+    dtype (row-strided views allowed), or :class:`RowParts`."""
+    if isinstance(y1, RowParts) and (y2 is None or (isinstance(y2, RowParts) and y2.bias is None)) and out_dtype == torch.bfloat16 and x.data_ptr() % 16 == 0:
+        return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus)
+    y1, y2 = (y.total() if isinstance(y, RowParts) else y for y in (y1, y2))
     if use_native(x):
         return native_hybrid().norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype == torch.bfloat16)
     return ref.norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype)
