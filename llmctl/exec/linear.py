@@ -196,6 +196,15 @@ def _gemm_ex_ok(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> bool:
     return dy2.stride(0) * K * 2 < 2**31 and x2.stride(0) * K * 2 < 2**31
 
 
+def _wgrad_whole(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> bool:
+    """Whether a weight whose rows are no multiple of 256 (a vocabulary) has its gradient made by gemm64 all the same: whole tiles, and a tile of their own for the
+    rows behind them.  us, library / so: 8192 tokens 50304 x 768 642 / 499, 8320 x 1024 173 / 134, 32136 x 4096 1935 / 1590, 4096 tokens 50304 x 768 345 / 272;
+    2048 tokens 182 / 176 (added to what is there 190 / 204), 1024 107 / 107, 512 64 / 72; 8192 tokens 5000 x 768 87 / 90."""
+    M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
+    return (M % 256 != 0 and M % 8 == 0 and M >= 8192 and K >= 3072 and _gemm64_ok(M // 256 * 256, N, K, g, dy2, x2) and K * dy2.stride(0) * 2 < 2**31
+            and K * x2.stride(0) * 2 < 2**31)
+
+
 def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool) -> None:
     """``g (+)= dy2^T @ x2``: the MFMA kernels read both K-major operands through
     ds_read_b64_tr_b16 (gemm64: +20-40 % over hipBLASLt on the GPT-7B shapes,
@@ -221,6 +230,15 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         from llmctl.ops._lib import native
 
         native().gemm_ex(dy2, x2, g, True, True, accumulate)
+    elif _wgrad_whole(g, dy2, x2):
+        from llmctl.ops._lib import native
+
+        whole = M // 256 * 256
+        native().gemm64_ex(dy2[:, :whole], x2, g[:whole], True, True, accumulate, gemm64_config("wgrad", whole, N, K))
+        last = torch.empty(256, N, dtype=torch.float32, device=g.device)  # a tile that ends at the last row
+        native().gemm64_ex(dy2[:, M - 256:], x2, last, True, True, False, gemm64_config("wgrad", 256, N, K))
+        rest = last[256 - (M - whole):]
+        g[whole:].add_(rest) if accumulate else g[whole:].copy_(rest)
     elif accumulate:
         g.addmm_(dy2.t(), x2)
     else:

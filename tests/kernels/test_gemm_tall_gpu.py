@@ -99,3 +99,22 @@ def test_linear_backward_with_sinks(tokens, out, inn):
     linear(x, w, b).backward(dy)
     for p, ref in ((w, dy.double().t() @ x.double()), (b, dy.double().sum(0))):
         assert bool(((p.grad.double() - 2 * ref).abs() <= 2.0**-7 * 2 * ref.abs() + 1e-3 * ref.abs().max()).all())
+
+
+@pytest.mark.parametrize("M,N,tokens", [(8200, 256, 3072), (8440, 512, 3200), (8320, 256, 3072)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_weight_gradient_of_a_vocabulary(M, N, tokens, f32):
+    """Rows that fill no whole tile: both parts of the gradient, stored and added to."""
+    from llmctl.exec.linear import _wgrad_whole, wgrad_into
+
+    dy, x = _operands(True, M, N, tokens, 0)
+    g = torch.full((M, N), float("nan"), device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    assert f32 or _wgrad_whole(g, dy, x)
+    A, B = dy.t().double(), x.double()
+    ref, bound = A @ B, _bound(A, B, tokens, 16)
+    wgrad_into(g, dy, x, False)
+    first = g.double()
+    # an fp32 gradient takes the library's product, rounded to bf16; each write of a bf16 one rounds once
+    assert bool(((first - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
+    wgrad_into(g, dy, x, True)
+    assert bool(((g.double() - first - ref).abs() <= bound + 2.0**-7 * (ref.abs() + first.abs() + bound)).all())
