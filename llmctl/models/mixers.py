@@ -430,7 +430,7 @@ class MLSTM(nn.Module):
         q, k = z[:, :H * dk].view(T, H, dk), z[:, H * dk:2 * H * dk].view(T, H, dk)
         v = z[:, 2 * H * dk:2 * H * dk + H * dv].view(T, H, dv)
         g = z[:, 2 * H * dk + H * dv:]
-        gates = F.linear(h.float(), self.w_if)  # fp32 [T, 2H]
+        gates = hops.linear_f32w(h, self.w_if, few=b.Tp == 0)  # fp32 [T, 2H]
         S, n, m = state
         key = ("mlstm_plan", H, dk, dv)
         if key not in b.scratch:

@@ -137,6 +137,7 @@ void memory_combine(at::Tensor S, const at::Tensor& slots, const at::Tensor& sta
 std::tuple<at::Tensor, at::Tensor> embed_f32(const at::Tensor& ids, const at::Tensor& table);
 at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const OptT& bias, double s1, const OptT& y2, double s2, const at::Tensor& w, double mult,
                                double eps, bool one_plus);
+at::Tensor rows_f32w(const at::Tensor& x, const at::Tensor& w);
 at::Tensor rows_parts(const at::Tensor& x, const at::Tensor& w, int64_t parts);
 at::Tensor norm_add_f32_(at::Tensor x, const at::Tensor& y1, double s1, const OptT& y2, double s2, const at::Tensor& w, double mult, double eps,
                          bool one_plus, bool out_bf16);
@@ -207,6 +208,7 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("memory_combine(Tensor(a!) S, Tensor slots, Tensor start, Tensor base, Tensor loc, Tensor dec, Tensor? trans, Tensor(b!) init) -> ()");
   m.def("embed_f32(Tensor ids, Tensor table) -> (Tensor, Tensor)");
   m.def("norm_add_parts_f32_(Tensor(a!) x, Tensor y1, Tensor? bias, float s1, Tensor? y2, float s2, Tensor w, float mult, float eps, bool one_plus) -> Tensor");
+  m.def("rows_f32w(Tensor x, Tensor w) -> Tensor");
   m.def("rows_parts(Tensor x, Tensor w, int parts) -> Tensor");
   m.def("norm_add_f32_(Tensor(a!) x, Tensor y1, float s1, Tensor? y2, float s2, Tensor w, float mult, float eps, bool one_plus, bool out_bf16) -> Tensor");
   m.def("gate_groupnorm(Tensor o, Tensor z, Tensor w, int groups, float eps, bool out_bf16) -> Tensor");
@@ -275,6 +277,7 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("memory_combine", &llmctl_hybrid::memory_combine);
   m.impl("embed_f32", &llmctl_hybrid::embed_f32);
   m.impl("norm_add_parts_f32_", &llmctl_hybrid::norm_add_parts_f32_);
+  m.impl("rows_f32w", &llmctl_hybrid::rows_f32w);
   m.impl("rows_parts", &llmctl_hybrid::rows_parts);
   m.impl("norm_add_f32_", &llmctl_hybrid::norm_add_f32_);
   m.impl("gate_groupnorm", &llmctl_hybrid::gate_groupnorm);

@@ -551,6 +551,14 @@ def linear_parts(x, w, b=None):
     return linear(x, w, b)
 
 
+def linear_f32w(x, w, few: bool):
+    """``x.float() @ w^T`` with fp32 weights, in fp32; ``few``: a step without prompts, whose at most 32 rows take one launch."""
+    if (few and use_native(x) and 1 <= x.shape[0] <= 32 and x.dtype == torch.bfloat16 and w.dtype == torch.float32 and w.is_contiguous() and x.stride(1) == 1
+            and x.shape[1] % 8 == 0 and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0 and not wants_grad(x, w)):
+        return native_hybrid().rows_f32w(x, w)
+    return torch.nn.functional.linear(x.float(), w)
+
+
 def linear_f32(x, w):
     """``x @ w^T`` with an fp32 result (inputs in their own dtype, fp32 accumulation)."""
     if x.dtype == torch.float32:

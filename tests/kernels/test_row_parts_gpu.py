@@ -52,3 +52,19 @@ def test_rule(M, N, K, parts):
     got = y.total() if parts else y
     ref = x.double() @ w.double().t() + b.double()
     assert bool(((got.double() - ref).abs() <= 2.0**-8 * ref.abs() + K * 2.0**-22 * 8).all())
+
+
+@pytest.mark.parametrize("T", [1, 4, 5, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(1, 8), (8, 2048), (32, 2056), (6, 4104)])
+def test_fp32_weights(T, N, K):
+    from llmctl.ops import hybrid as hops
+
+    g = torch.Generator(device="cuda").manual_seed(T * N + K)
+    x = torch.randn(T, K + 8, generator=g, device="cuda").bfloat16()[:, :K]
+    w = torch.randn(N, K, generator=g, device="cuda")
+    got = hops.linear_f32w(x, w, few=True)
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    err = (got.double() - ref).abs()
+    assert bool((err <= (K / 256 + 24) * 2.0**-24 * mag).all())  # a thread's chain of K / 256 and the sums over threads
+    lib = (torch.nn.functional.linear(x.float(), w).double() - ref).abs()
+    assert err.pow(2).mean() <= 4 * lib.pow(2).mean() + (2.0**-25 * mag).pow(2).mean()
