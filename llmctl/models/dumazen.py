@@ -147,6 +147,8 @@ class DumazenLM(nn.Module):
     def dtype(self):
         return self.embed.dtype
 
+    normed_step = True  # step takes ``final``
+
     def head_weight(self):
         return self.embed
 
@@ -162,23 +164,28 @@ class DumazenLM(nn.Module):
         return out
 
     # ------------------------------------------------------------------ serving step
-    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None):
+    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None, final: bool = False):
         """Run the step's packed tokens through all layers against the engine's cache (``cache.layer(i)``).  Returns the
-        fp32 residual stream of ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer."""
+        fp32 residual stream of ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer.  ``final`` (not with
+        ``rows`` or ``trail``): all rows :class:`~llmctl.ops.hybrid.Normed` instead, the final norm in the last residual update."""
         mult, eps, dt = self.cfg.residual_mult, self.cfg.layer_norm_eps, self.dtype
         x, h = hops.embed_f32(b.ids, self.embed)
+        if final and not self.layers:
+            return x
         for i, layer in enumerate(self.layers):
+            last = self.final_norm if final and i + 1 == len(self.layers) else None
             y = layer.mixer.step(h, b, cache.layer(i), late=True)
             (y1, s1), (y2, s2) = y if isinstance(y, tuple) else ((y, 1.0), (None, 0.0))
-            h = hops.norm_add_f32_(x, y1, s1, y2, s2, layer.norm1, mult, eps, True, dt)
+            h = hops.norm_add_f32_(x, y1, s1, y2, s2, layer.norm1, mult, eps, True, dt, last if layer.ff is None else None)
             if layer.ff is not None:
-                h = hops.norm_add_f32_(x, layer.ff(h, late=True), 1.0, None, 0.0, layer.norm2, mult, eps, True, dt)
+                h = hops.norm_add_f32_(x, layer.ff(h, late=True), 1.0, None, 0.0, layer.norm2, mult, eps, True, dt, last)
             if trail is not None:
                 trail.append(x.clone())
-        return x if rows is None else x.index_select(0, rows)
+        return hops.Normed(h) if final else x if rows is None else x.index_select(0, rows)
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
-        xn, _ = hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None, self.cfg.layer_norm_eps, True, self.dtype)
+        xn = x.h if isinstance(x, hops.Normed) else hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None,
+                                                                           self.cfg.layer_norm_eps, True, self.dtype)[0]
         return _mm_f32(xn, self.embed)
 
     # ------------------------------------------------------------------ checkpoint names

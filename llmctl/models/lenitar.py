@@ -147,14 +147,17 @@ class LenitarLM(nn.Module):
     def has_recurrent_state(self) -> bool:
         return any(l.mixer.cache_kind == "state" for l in self.layers)
 
+    normed_step = True  # step takes ``final``
+
     def head_weight(self):
         return self.lm_head
 
     # ------------------------------------------------------------------ serving step
-    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None):
+    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None, final: bool = False):
         """Run the step's packed tokens through all layers against the engine's cache (``cache.layer(i)``:
         the paged latent pool or the state pools of layer i).  Returns the fp32 residual stream of
-        ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer."""
+        ``rows`` (all rows if None) after the last layer; ``trail`` collects it after every layer.  ``final`` (not with
+        ``rows`` or ``trail``): all rows :class:`~llmctl.ops.hybrid.Normed` instead, the final norm in the last residual update."""
         cfg, eps, dt = self.cfg, self.cfg.layer_norm_eps, self.dtype
         n, T = len(self.layers), b.ids.shape[0]
         # decode steps: the norms find the rows' experts (a prompt's checks would cost the host more than its launch of a router)
@@ -167,6 +170,8 @@ class LenitarLM(nn.Module):
             if i + 1 < n and trail is None:
                 nxt = self.layers[i + 1]
                 h, routed = hops.add_layernorm_route_(x, y, z, nxt.norm_w, nxt.norm_b, eps, dt, routers[i + 1])
+            elif final:
+                return hops.Normed(hops.add_layernorm_f32_(x, y, z, self.final_norm_w, self.final_norm_b, eps, dt))
             else:
                 hops.residual_add_(x, y, z)
                 if trail is not None:
@@ -176,8 +181,8 @@ class LenitarLM(nn.Module):
         return x if rows is None else x.index_select(0, rows)
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
-        xn = hops.layernorm_f32(x.contiguous(), self.final_norm_w, self.final_norm_b, self.cfg.layer_norm_eps,
-                                self.dtype)
+        xn = x.h if isinstance(x, hops.Normed) else hops.layernorm_f32(x.contiguous(), self.final_norm_w, self.final_norm_b,
+                                                                       self.cfg.layer_norm_eps, self.dtype)
         return hops.linear(xn, self.lm_head)
 
     # ------------------------------------------------------------------ checkpoint names

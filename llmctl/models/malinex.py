@@ -188,6 +188,8 @@ class MalinexLM(nn.Module):
         """Positions the engine may ask for (rows of the learned position table)."""
         return self.pos.shape[0]
 
+    normed_step = True  # step takes ``final``
+
     def head_weight(self):
         return self.lm_head
 
@@ -201,19 +203,20 @@ class MalinexLM(nn.Module):
         return out
 
     # ------------------------------------------------------------------ serving step
-    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None):
+    def step(self, b: StepBatch, cache, rows: Optional[torch.Tensor] = None, trail: Optional[list] = None, final: bool = False):
         """Run the step's packed tokens through all layers against the engine's cache (``cache.layer(i)``:
         the rows or the state pools of layer i).  Returns the fp32 residual stream of ``rows`` (all rows
-        if None) after the last layer; ``trail`` collects it after every layer."""
+        if None) after the last layer; ``trail`` collects it after every layer.  ``final`` (not with ``rows`` or ``trail``): all rows
+        :class:`~llmctl.ops.hybrid.Normed` instead, the final norm in the last residual update."""
         eps, dt = self.cfg.layer_norm_eps, self.dtype
         n = len(self.order)
         if n == 0:
-            x, _ = hops.embed_rmsnorm_f32(b.ids, b.pos, self.embed, self.pos, self.final_norm, eps, dt)
-            return x if rows is None else x.index_select(0, rows)
+            x, h = hops.embed_rmsnorm_f32(b.ids, b.pos, self.embed, self.pos, self.final_norm, eps, dt)
+            return hops.Normed(h) if final else x if rows is None else x.index_select(0, rows)
         x, h = hops.embed_rmsnorm_f32(b.ids, b.pos, self.embed, self.pos, self.block(0).norm1, eps, dt)
         for i in range(n):
             layer = self.block(i)
-            nxt = self.block(i + 1).norm1 if i + 1 < n else None
+            nxt = self.block(i + 1).norm1 if i + 1 < n else self.final_norm if final else None
             y, r = layer.mixer.step(h, b, cache.layer(i))
             experts = layer.ff if isinstance(layer.ff, BiasedSoftmaxMoE) else None
             h, routed = hops.gated_norm_add_norm_route_(x, y, r, layer.norm1b, layer.norm2 if layer.ff is not None else nxt, eps, dt,
@@ -223,11 +226,11 @@ class MalinexLM(nn.Module):
                 h = hops.gated_norm_add_norm_f32_(x, y, r, layer.norm2b, nxt, eps, dt)
             if trail is not None:
                 trail.append(x.clone())
-        return x if rows is None else x.index_select(0, rows)
+        return hops.Normed(h) if final else x if rows is None else x.index_select(0, rows)
 
     def logits(self, x: torch.Tensor) -> torch.Tensor:
-        xn, _ = hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None, self.cfg.layer_norm_eps, False,
-                                       self.dtype)
+        xn = x.h if isinstance(x, hops.Normed) else hops.add_rmsnorm2_f32_(x.contiguous(), None, None, self.final_norm, None,
+                                                                           self.cfg.layer_norm_eps, False, self.dtype)[0]
         z = hops.linear_f32(xn, self.lm_head)
         return z if self.cfg.logit_scale == 1.0 else z * self.cfg.logit_scale
 

@@ -136,7 +136,7 @@ void memory_combine(at::Tensor S, const at::Tensor& slots, const at::Tensor& sta
                     const OptT& trans, at::Tensor init);
 std::tuple<at::Tensor, at::Tensor> embed_f32(const at::Tensor& ids, const at::Tensor& table);
 at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const OptT& bias, double s1, const OptT& y2, double s2, const at::Tensor& w, double mult,
-                               double eps, bool one_plus);
+                               double eps, bool one_plus, const OptT& w_next);
 at::Tensor rows_f32w(const at::Tensor& x, const at::Tensor& w);
 at::Tensor rows_parts(const at::Tensor& x, const at::Tensor& w, int64_t parts);
 at::Tensor norm_add_f32_(at::Tensor x, const at::Tensor& y1, double s1, const OptT& y2, double s2, const at::Tensor& w, double mult, double eps,
@@ -207,7 +207,7 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("memory_chunk_local(Tensor q, Tensor k, Tensor v, int kind, Tensor? ga, Tensor? gb, Tensor? a_log, Tensor? dt_bias, Tensor? log_decay, Tensor? skip, Tensor cu, Tensor(a!) loc, Tensor(b!) dec, Tensor(c!)? trans) -> ()");
   m.def("memory_combine(Tensor(a!) S, Tensor slots, Tensor start, Tensor base, Tensor loc, Tensor dec, Tensor? trans, Tensor(b!) init) -> ()");
   m.def("embed_f32(Tensor ids, Tensor table) -> (Tensor, Tensor)");
-  m.def("norm_add_parts_f32_(Tensor(a!) x, Tensor y1, Tensor? bias, float s1, Tensor? y2, float s2, Tensor w, float mult, float eps, bool one_plus) -> Tensor");
+  m.def("norm_add_parts_f32_(Tensor(a!) x, Tensor y1, Tensor? bias, float s1, Tensor? y2, float s2, Tensor w, float mult, float eps, bool one_plus, Tensor? w_next=None) -> Tensor");
   m.def("rows_f32w(Tensor x, Tensor w) -> Tensor");
   m.def("rows_parts(Tensor x, Tensor w, int parts) -> Tensor");
   m.def("norm_add_f32_(Tensor(a!) x, Tensor y1, float s1, Tensor? y2, float s2, Tensor w, float mult, float eps, bool one_plus, bool out_bf16) -> Tensor");

@@ -122,7 +122,8 @@ __global__ __launch_bounds__(NT) void norm_add_kernel(float* __restrict__ x, con
 template <int VQ>
 __global__ __launch_bounds__(NT) void norm_add_parts_kernel(float* __restrict__ x, const float* __restrict__ y1, int n1, const bf16_t* __restrict__ bias,
                                                             float s1, const float* __restrict__ y2, int n2, float s2, const float* __restrict__ w,
-                                                            float mult, float plus, bf16_t* __restrict__ h, int W, int64_t TW, float eps) {
+                                                            float mult, float plus, bf16_t* __restrict__ h, int W, int64_t TW, float eps,
+                                                            const float* __restrict__ wn) {
   __shared__ float red[NW];
   const int64_t row = blockIdx.x;
   float4 a[VQ], xv[VQ], wv[VQ];
@@ -165,7 +166,24 @@ __global__ __launch_bounds__(NT) void norm_add_parts_kernel(float* __restrict__ 
     const float4 o = make_float4(xv[i].x + a[i].x * f * (wv[i].x + plus), xv[i].y + a[i].y * f * (wv[i].y + plus), xv[i].z + a[i].z * f * (wv[i].z + plus),
                                  xv[i].w + a[i].w * f * (wv[i].w + plus));
     *reinterpret_cast<float4*>(x + row * W + c) = o;
+    a[i] = o;
+    if (wn != nullptr) continue;
     const float v[4] = {o.x, o.y, o.z, o.w};
+    stn<bf16_t, 4>(h + row * W + c, v);
+  }
+  if (wn == nullptr) return;
+  // h = x / rms(x) (wn + plus): the model's last norm
+  q = 0.f;
+#pragma unroll
+  for (int i = 0; i < VQ; ++i)
+    if ((int)(threadIdx.x + i * NT) * 4 < W) q += a[i].x * a[i].x + a[i].y * a[i].y + a[i].z * a[i].z + a[i].w * a[i].w;
+  const float fn = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+#pragma unroll
+  for (int i = 0; i < VQ; ++i) {
+    const int c = (int)(threadIdx.x + i * NT) * 4;
+    if (c >= W) break;
+    const float4 n = *reinterpret_cast<const float4*>(wn + c);
+    const float v[4] = {a[i].x * fn * (n.x + plus), a[i].y * fn * (n.y + plus), a[i].z * fn * (n.z + plus), a[i].w * fn * (n.w + plus)};
     stn<bf16_t, 4>(h + row * W + c, v);
   }
 }
@@ -327,7 +345,7 @@ at::Tensor norm_add_f32_(at::Tensor x, const at::Tensor& y1, double s1, const c1
 
 // norm_add_f32_ of results that are fp32 sums over ranges of K (rows_parts: [ranges, T, W]), y1 still without its bias; h is bf16
 at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const c10::optional<at::Tensor>& bias, double s1, const c10::optional<at::Tensor>& y2,
-                               double s2, const at::Tensor& w, double mult, double eps, bool one_plus) {
+                               double s2, const at::Tensor& w, double mult, double eps, bool one_plus, const c10::optional<at::Tensor>& w_next) {
   HYB_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() && x.scalar_type() == at::kFloat, "x: contiguous fp32 [T, W]");
   const int64_t T = x.size(0), W = x.size(1);
   auto parts = [&](const at::Tensor& t) {
@@ -341,6 +359,7 @@ at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const c10::op
   HYB_CHECK(f32w(w, W) && W % 4 == 0 && W <= 16 * NT && reinterpret_cast<uintptr_t>(w.data_ptr()) % 16 == 0 &&
                 reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0,
             "w: fp32 [W]; W a multiple of 4, at most 4096");
+  HYB_CHECK(!w_next.has_value() || (f32w(*w_next, W) && reinterpret_cast<uintptr_t>(w_next->data_ptr()) % 16 == 0), "w_next: fp32 [W]");
   c10::DeviceGuard guard(x.device());
   at::Tensor h = at::empty({T, W}, x.options().dtype(at::kBFloat16));
   if (T == 0 || W == 0) return h;
@@ -348,7 +367,8 @@ at::Tensor norm_add_parts_f32_(at::Tensor x, const at::Tensor& y1, const c10::op
     kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(x.data_ptr<float>(), y1.data_ptr<float>(), (int)y1.size(0),
                                                      bias.has_value() ? reinterpret_cast<const bf16_t*>(bias->data_ptr()) : nullptr, (float)s1,
                                                      y2.has_value() ? y2->data_ptr<float>() : nullptr, y2.has_value() ? (int)y2->size(0) : 0, (float)s2,
-                                                     w.data_ptr<float>(), (float)mult, one_plus ? 1.0f : 0.0f, reinterpret_cast<bf16_t*>(h.data_ptr()), (int)W, T * W, (float)eps);
+                                                     w.data_ptr<float>(), (float)mult, one_plus ? 1.0f : 0.0f, reinterpret_cast<bf16_t*>(h.data_ptr()), (int)W, T * W, (float)eps,
+                                                     w_next.has_value() ? w_next->data_ptr<float>() : nullptr);
   };
   if (W <= 4 * NT) go(norm_add_parts_kernel<1>);
   else if (W <= 8 * NT) go(norm_add_parts_kernel<2>);

@@ -520,6 +520,17 @@ def odd_linear(x, w, b=None):
     return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else wide_linear(x, w, b)
 
 
+class Normed:
+    """Rows that the final norm is already on, as a model's ``step(..., final=True)`` hands them to its ``logits``."""
+
+    def __init__(self, h):
+        self.h = h
+
+    @property
+    def shape(self):
+        return self.h.shape
+
+
 class RowParts:
     """A product of a few rows that is still fp32 sums ``[ranges, T, W]`` over ranges of K, and its bias: :func:`norm_add_f32_` adds them in its own
     pass; :meth:`total` is the product as a tensor."""
@@ -935,13 +946,17 @@ def gate_groupnorm(o, z, w, groups: int, eps: float, out_dtype):
     return ref.gate_groupnorm(o, z, w, groups, eps, out_dtype)
 
 
-def norm_add_f32_(x, y1, s1: float, y2, s2: float, w, mult: float, eps: float, one_plus: bool, out_dtype):
+def norm_add_f32_(x, y1, s1: float, y2, s2: float, w, mult: float, eps: float, one_plus: bool, out_dtype, w_next=None):
     """The end of a sublayer whose only norm is on its result: ``y = s1 y1 (+ s2 y2)``, ``x += mult y / rms(y) (w + one_plus)``
     in place on the fp32 stream, and the next sublayer's input, x itself, in ``out_dtype``.  ``y [T, W]`` in the activation
-    dtype (row-strided views allowed), or :class:`RowParts`."""
+    dtype (row-strided views allowed), or :class:`RowParts`.  ``w_next``: the RMS norm
+    of x by these weights instead (the same eps and ``one_plus``)."""
     if isinstance(y1, RowParts) and (y2 is None or (isinstance(y2, RowParts) and y2.bias is None)) and out_dtype == torch.bfloat16 and x.data_ptr() % 16 == 0:
-        return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus)
+        return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus, w_next)
     y1, y2 = (y.total() if isinstance(y, RowParts) else y for y in (y1, y2))
+    if w_next is not None:
+        norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype)
+        return add_rmsnorm2_f32_(x, None, None, w_next, None, eps, one_plus, out_dtype)[0]
     if use_native(x):
         return native_hybrid().norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype == torch.bfloat16)
     return ref.norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype)

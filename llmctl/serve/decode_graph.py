@@ -87,7 +87,7 @@ class DecodeGraph:
             g.capture_begin(pool=pool, capture_error_mode="thread_local")
             try:
                 self.batch.scratch.clear()
-                logits = model.logits(model.step(self.batch, cache))
+                logits = model.logits(model.step(self.batch, cache, **({"final": True} if getattr(model, "normed_step", False) else {})))
             except BaseException:
                 try:
                     g.capture_end()

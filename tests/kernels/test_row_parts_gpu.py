@@ -41,6 +41,25 @@ def test_norm_of_parts(T, W, n1, n2, bias):
     assert torch.equal(h, x.bfloat16())
 
 
+@pytest.mark.parametrize("T,W", [(1, 4), (7, 260), (16, 2048), (32, 4096)])
+@pytest.mark.parametrize("parts", [True, False])
+def test_norm_with_the_next(T, W, parts):
+    """The last residual update and the final norm in one pass: the same stream, and x's own norm."""
+    from llmctl.ops import hybrid as hops
+
+    g = torch.Generator(device="cuda").manual_seed(T + W)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, w, wn, y = rand(T, W), rand(W), rand(W), rand(3, T, W)
+    y = hops.RowParts(y, None) if parts else y[0].bfloat16()
+    x2 = x.clone()
+    hops.norm_add_f32_(x2, y, 0.5, None, 0.0, w, 0.5, 1e-6, True, torch.bfloat16)
+    h = hops.norm_add_f32_(x, y, 0.5, None, 0.0, w, 0.5, 1e-6, True, torch.bfloat16, wn)
+    assert torch.equal(x, x2)
+    xd = x.double()
+    want = xd / (xd.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * (wn.double() + 1.0)
+    assert bool(((h.double() - want).abs() <= (2.0**-8 + 1e-5) * want.abs() + 1e-30).all())
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(16, 2048, 8192, 4), (4, 2048, 2048, 2), (32, 4096, 512, 4), (33, 1024, 512, 0), (8, 4100, 512, 0), (8, 514, 512, 0)])
 def test_rule(M, N, K, parts):
     from llmctl.ops import hybrid as hops
