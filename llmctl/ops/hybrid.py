@@ -951,9 +951,10 @@ def norm_add_f32_(x, y1, s1: float, y2, s2: float, w, mult: float, eps: float, o
     in place on the fp32 stream, and the next sublayer's input, x itself, in ``out_dtype``.  ``y [T, W]`` in the activation
     dtype (row-strided views allowed), or :class:`RowParts`.  ``w_next``: the RMS norm
     of x by these weights instead (the same eps and ``one_plus``)."""
-    if isinstance(y1, RowParts) and (y2 is None or (isinstance(y2, RowParts) and y2.bias is None)) and out_dtype == torch.bfloat16 and x.data_ptr() % 16 == 0:
-        return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus, w_next)
-    y1, y2 = (y.total() if isinstance(y, RowParts) else y for y in (y1, y2))
+    if type(y1) is RowParts or type(y2) is RowParts:
+        if type(y1) is RowParts and (y2 is None or (type(y2) is RowParts and y2.bias is None)) and out_dtype == torch.bfloat16 and x.data_ptr() % 16 == 0:
+            return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus, w_next)
+        y1, y2 = (y.total() if type(y) is RowParts else y for y in (y1, y2))
     if w_next is not None:
         norm_add_f32_(x, y1, s1, y2, s2, w, mult, eps, one_plus, out_dtype)
         return add_rmsnorm2_f32_(x, None, None, w_next, None, eps, one_plus, out_dtype)[0]
