@@ -217,6 +217,8 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
             from llmctl.ops._lib import native
 
             native().gemm64_ex(dy2, x2, g, True, True, accumulate, gemm64_config("wgrad", M, N, K))
+        elif K % 128 and wgrad_bias_into(g, dy2, x2, accumulate, None, False):
+            pass
         elif accumulate:
             g.add_(dy2.t().matmul(x2))
         else:
@@ -226,6 +228,8 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         from llmctl.ops._lib import native
 
         native().gemm64_ex(dy2, x2, g, True, True, accumulate, gemm64_config("wgrad", M, N, K))
+    elif K % 128 and wgrad_bias_into(g, dy2, x2, accumulate, None, False):
+        pass
     elif _gemm_ex_ok(g, dy2, x2):
         from llmctl.ops._lib import native
 
@@ -245,10 +249,12 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         torch.mm(dy2.t(), x2, out=g)
 
 
-def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: torch.Tensor, add: bool) -> bool:
-    """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient; False: nothing done."""
+def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: Optional[torch.Tensor], add: bool) -> bool:
+    """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient, over any number of tokens from 256 on
+    (without ``gb`` where they are no multiple of 128); False: nothing done."""
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
-    if not (_gemm64_ok(M, N, K, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32) and gb.dtype == g.dtype and gb.is_contiguous()
+    if not (K >= 256 and _gemm64_ok(M, N, 128, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32)
+            and (gb is None or (gb.dtype == g.dtype and gb.is_contiguous()))
             and g.stride(1) == 1 and g.stride(0) % 8 == 0 and g.data_ptr() % 16 == 0
             and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3):
         return False

@@ -83,12 +83,37 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const int sp = item / tiles, wg = item - sp * tiles;
   const int grp = wg / (4 * args.tiles_n), gsz = min(4, args.tiles_m - grp * 4), inner = wg - grp * 4 * args.tiles_n;
   const int tm = grp * 4 + inner % gsz, tn = inner / gsz;
-  const int pairs = args.K / (2 * TK);
+  const int pairs = (args.K + 2 * TK - 1) / (2 * TK);  // AT: the last pair of K-tiles may be part full
   const int k0 = 2 * (int)((long)pairs * sp / args.splits), KT = 2 * (int)((long)pairs * (sp + 1) / args.splits) - k0;
 
   i32x4_t ra = make_rsrc(AT ? args.a + (long)tm * TM : args.a + (long)tm * TM * lda);
   i32x4_t rb = make_rsrc(args.b + (long)tn * TALL_N);
+  // AT: the last two K-tiles through buffers of their own that start with them and end with the last token's row, so that what is read past it is zero (a row
+  // past the end starts past the range: the rows do not overlap)
+  i32x4_t ta[2], tb[2];
+  if constexpr (AT) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int gk = 2 * pairs - 2 + i, rows = args.K - gk * TK;
+      ta[i] = make_rsrc_n(args.a + (long)gk * TK * lda + (long)tm * TM, rows > 0 ? (unsigned)(((long)(min(rows, TK) - 1) * lda + args.M - tm * TM) * 2) : 0u);
+      tb[i] = make_rsrc_n(args.b + (long)gk * TK * ldb + (long)tn * TALL_N, rows > 0 ? (unsigned)(((long)(min(rows, TK) - 1) * ldb + args.N - tn * TALL_N) * 2) : 0u);
+    }
+    asm volatile("s_nop 7" : "+s"(ta[0]), "+s"(ta[1]), "+s"(tb[0]), "+s"(tb[1]));
+  }
   asm volatile("s_nop 7" : "+s"(ra), "+s"(rb));  // lane-read scalars to the first DMA piece that uses them
+  // K-tile t of the item: its buffer and offset
+  auto src = [&](bool is_b, int t, unsigned step, unsigned& so) __attribute__((always_inline)) {
+    const int gk = k0 + t, i = gk - (2 * pairs - 2);
+    i32x4_t r = is_b ? rb : ra;
+    so = (unsigned)gk * step;
+    if constexpr (AT) {
+      if (i >= 0) {
+        r = is_b ? (i ? tb[1] : tb[0]) : (i ? ta[1] : ta[0]);
+        so = 0;
+      }
+    }
+    return r;
+  };
   const unsigned a_step = AT ? (unsigned)(TK * lda * 2) : (unsigned)(TK * 2), b_step = (unsigned)(TK * ldb * 2);
   unsigned vo[3][4];
 #pragma unroll
@@ -100,9 +125,10 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const unsigned lds0 = lds_addr(smem) + wave * 1024;
   auto issue = [&](auto kind_c, int t, int slot, auto n_c) __attribute__((always_inline)) {
     constexpr int kind = decltype(kind_c)::value, n = decltype(n_c)::value;
-    const unsigned so = (unsigned)(k0 + t) * (kind == B_H0 ? b_step : a_step);
+    unsigned so;
+    const i32x4_t r = src(kind == B_H0, t, kind == B_H0 ? b_step : a_step, so);
 #pragma unroll
-    for (int i = 0; i < n; ++i) bdma16(kind == B_H0 ? rb : ra, vo[kind][i], so, lds0 + slot + kind * HALF + i * 4096);
+    for (int i = 0; i < n; ++i) bdma16(r, vo[kind][i], so, lds0 + slot + kind * HALF + i * 4096);
   };
 
   f32x4_t acc[8][4];
@@ -152,13 +178,15 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto ktile = [&](auto par_c, auto dma_c, auto wait_c, int t, int s0, int s1, int s2) __attribute__((always_inline)) {
     constexpr int P = decltype(par_c)::value, DMA = decltype(dma_c)::value, WAIT = decltype(wait_c)::value;
     constexpr bool NEXT = WAIT >= 0;
-    const unsigned so0 = (unsigned)(k0 + t + 2) * a_step, l0 = lds0 + s2;
+    unsigned so0, soa, sob;
+    const i32x4_t ra0 = src(false, t + 2, a_step, so0);
+    const unsigned l0 = lds0 + s2;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int ks = q >> 3, i = (q >> 1) & 3, j = (q & 1) * 2;
       if (DMA >= 1 && q % 3 == 0) {
         const int n = q / 3, kind = n < 2 ? A_LO : A_HI, pc = n < 2 ? 2 + n : n - 2;
-        g4w_pair_dma(acc[i][j], acc[i][j + 1], a_lo[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], ra, so0, l0 + kind * HALF + pc * 4096);
+        g4w_pair_dma(acc[i][j], acc[i][j + 1], a_lo[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], ra0, so0, l0 + kind * HALF + pc * 4096);
       } else {
         g4w_pair(acc[i][j], acc[i][j + 1], a_lo[i][ks], b[P][j][ks], b[P][j + 1][ks]);
       }
@@ -168,13 +196,14 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
         if (q == 12 && sum_hi) bias_frag(smem + s0 + A_HI * HALF);
       }
     }
-    const unsigned soa = (unsigned)(k0 + t + 3) * a_step, sob = (unsigned)(k0 + t + 3) * b_step, l1 = lds0 + s0;
+    const i32x4_t ra1 = src(false, t + 3, a_step, soa), rb1 = src(true, t + 3, b_step, sob);
+    const unsigned l1 = lds0 + s0;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int ks = q >> 3, i = (q >> 1) & 3, j = (q & 1) * 2;
       if (DMA == 2 && q % 3 == 0) {
         const int n = q / 3, kind = n < 4 ? B_H0 : A_LO, pc = n & 3;
-        g4w_pair_dma(acc[4 + i][j], acc[4 + i][j + 1], a_hi[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], n < 4 ? rb : ra, n < 4 ? sob : soa,
+        g4w_pair_dma(acc[4 + i][j], acc[4 + i][j + 1], a_hi[i][ks], b[P][j][ks], b[P][j + 1][ks], vo[kind][pc], n < 4 ? rb1 : ra1, n < 4 ? sob : soa,
                      l1 + kind * HALF + pc * 4096);
       } else {
         g4w_pair(acc[4 + i][j], acc[4 + i][j + 1], a_hi[i][ks], b[P][j][ks], b[P][j + 1][ks]);
@@ -333,7 +362,7 @@ void launch(const TallArgs& g, int out) {
 // cost a launch (4) and their bytes, written and read, at 6 TB/s.  Ranges stay at four K-tiles and more, what the peeled loop takes.
 // Both sides measured, us: see above where these win; 192 tiles of 256 x 256 (4096 x 3072 x 768) 25.8 / 27.6 and 256 (4096 x 4096 x 2048) 53.0 / 62.4 there.
 int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits) {
-  const double cus = num_cus(), kt = K / TK;
+  const double cus = num_cus(), kt = (K + 2 * TK - 1) / (2 * TK) * 2;
   auto rounds = [&](double items) { return std::ceil(items / cus); };
   auto sums = [](double entries, int S) { return S > 1 ? 4.0 + entries * S * 8.0 / 6e6 : 0.0; };
   double other = rounds(n_main) * (kt * 1.3 + 7.0);
@@ -347,7 +376,8 @@ int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int split
   return best;
 }
 
-// out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N and K of 128, K >= 256 splits.
+// out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N of 128 and, not where at, K of 128; two pairs of
+// K-tiles, 256 of K, to a split.
 // bias [M] (+)= the row sums of A, of out's type (at, N >= 512).
 void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias,
                bool bias_add) {
@@ -357,8 +387,10 @@ void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at
                "gemm_tall: bf16 operands, bf16 or fp32 out");
   const long M = at_ ? a.size(1) : a.size(0), K = at_ ? a.size(0) : a.size(1), N = b.size(1);
   LLMCTL_CHECK(b.size(0) == K && out.size(0) == M && out.size(1) == N, "gemm_tall: shapes");
-  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && K % (2 * TK) == 0 && splits >= 1 && K >= 4 * TK * splits,
-               "gemm_tall: M in 256s, N and K in 128s, at least 256 of K to a split");
+  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && (at_ || K % (2 * TK) == 0) && splits >= 1 && K > 4 * TK * splits - 2 * TK &&
+                   (K + 2 * TK - 1) / (2 * TK) >= 2 * splits,
+               "gemm_tall: M in 256s, N (and K, but for a transposed A) in 128s, at least 256 of K to a split");
+  LLMCTL_CHECK(!at_ || K % (2 * TK) == 0 || (a.stride(0) >= M && b.stride(0) >= N), "gemm_tall: rows that do not overlap");
   auto rows16 = [](const at::Tensor& t, int per) {
     return t.stride(1) == 1 && t.stride(0) % per == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
   };

@@ -118,3 +118,44 @@ def test_weight_gradient_of_a_vocabulary(M, N, tokens, f32):
     assert bool(((first - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
     wgrad_into(g, dy, x, True)
     assert bool(((g.double() - first - ref).abs() <= bound + 2.0**-7 * (ref.abs() + first.abs() + bound)).all())
+
+
+@pytest.mark.parametrize("K,S", [(257, 1), (300, 1), (319, 1), (383, 1), (385, 2), (513, 2), (640, 2), (1000, 3), (3912, 4), (8191, 12)])
+@pytest.mark.parametrize("M,N,pad", [(256, 512, 0), (512, 640, 8)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_any_number_of_tokens(K, S, M, N, pad, bias):
+    """A weight gradient whose last K-tiles are part full: nothing of what lies behind the last token (NaN here) comes in."""
+    from llmctl.ops._lib import native
+
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    full = [torch.full((K + 160, n + pad), float("nan"), device="cuda", dtype=torch.bfloat16) for n in (M, N)]
+    dy, x = full[0][:K, :M], full[1][:K, :N]
+    for t in (dy, x):
+        t.copy_(torch.randn(t.shape, generator=g, device="cuda"))
+    out = torch.full((M, N), float("nan"), device="cuda")
+    db = torch.full((M,), float("nan"), device="cuda") if bias else None
+    native().gemm_tall(dy, x, out, True, False, S, db, False)
+    A, B = dy.t().double(), x.double()
+    assert bool(((out.double() - A @ B).abs() <= _bound(A, B, K, S)).all())
+    if bias:
+        assert bool(((db.double() - A.sum(1)).abs() <= (K + S) * 2.0**-24 * A.abs().sum(1)).all())
+
+
+@pytest.mark.parametrize("tokens,out,inn", [(3912, 768, 3072), (300, 2304, 768), (1111, 768, 256), (255, 768, 768), (2080, 4096, 4096)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_weight_gradients_of_odd_batches(tokens, out, inn, f32):
+    """Whichever kernel or library product takes them; each gradient stored once and added to once."""
+    from llmctl.exec.linear import GradSink, linear
+
+    torch.manual_seed(1)
+    w = torch.nn.Parameter((torch.randn(out, inn, device="cuda") * 0.02).bfloat16())
+    b = torch.nn.Parameter(torch.zeros(out, device="cuda", dtype=torch.bfloat16))
+    sink = GradSink()
+    for p in (w, b):
+        p.main_grad = torch.full(p.shape, float("nan"), device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+        sink.attach(p)
+    x, dy = torch.randn(tokens, inn, device="cuda").bfloat16(), torch.randn(tokens, out, device="cuda").bfloat16()
+    for _ in range(2):
+        linear(x, w, b).backward(dy)
+    for p, ref in ((w, dy.double().t() @ x.double()), (b, dy.double().sum(0))):
+        assert bool(((p.main_grad.double() - 2 * ref).abs() <= 2.0**-7 * 2 * ref.abs() + 1e-3 * ref.abs().max()).all())
