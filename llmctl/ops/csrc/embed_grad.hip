@@ -3,17 +3,18 @@
 // Bound: one pass over dy and the rows of g that it meets (8192 x 4096: 134 MB, 27 us at a copy's rate).  Three launches, no atomics, the same bits every time:
 //   order  the tokens ranked by (id, position): ids in LDS, every wave counts for two tokens the ids below and the equal ones before and in all.  T^2 compares,
 //          four a lane and read; 65536 tokens are the most that is taken here; a radix sort is five launches.
-//   rows   a wave per 16 sorted tokens and 512 columns, all loads in flight; a run of one id inside the 16 is final, a run across an edge leaves a partial row
-//   edges  the wave whose 16 a crossing run starts in adds the partial rows in order
+//   rows   a wave per 8 sorted tokens and 512 columns, all loads in flight; a run of one id inside the 8 is final, a run across an edge leaves a partial row
+//   edges  the wave whose 8 a crossing run starts in adds the partial rows in order
 // so a token that fills half the batch is summed by as many waves as any other half.
 // Measured on one MI355X, us, against the library's (sort, segments, scatter into a dense gradient that is then added), ids drawn evenly / all the same:
-// 8192 x 768 into 50304 rows 40.6 / 72.7 (141.7 / 331), 8192 x 4096 into 32000 74.5 / 105 (465 / 554), 24576 x 4096 283 / 406 (943 / 1176), 65536 x 4096
-// 1098 / 1545 (1492 / 3219).
+// 8192 x 768 into 50304 rows 29.4 / 109 (141 / 329), 8192 x 4096 into 32000 49.7 / 200 (468 / 555), 24576 x 4096 230 / 434 (947 / 1179), 65536 x 4096
+// 1011 / 1939 (1495 / 3232), 256 x 64 into 256 12.5 / 12.5 (18.5 / 26).  16 tokens a wave: 40.8, 75, 283, 1091, 17.3, and less only where most tokens are the
+// same (72, 104, 406, 1538, 16): a wave adds to the rows of its ids one after the other.
 #include "common.h"
 
 namespace llmctl {
 namespace {
-constexpr int RUN = 16, ORDER_IDS = 16384, ORDER_WAVES = 16;
+constexpr int RUN = 8, ORDER_IDS = 16384, ORDER_WAVES = 16;
 
 struct EmbedGradArgs {
   const int64_t* ids;

@@ -15,7 +15,7 @@ def _ids(kind, T, V, g):
     return torch.randint(0, V, (T,), generator=g, device="cuda")
 
 
-@pytest.mark.parametrize("T,H,V", [(1, 8, 3), (15, 8, 40), (16, 512, 5), (17, 520, 5), (33, 768, 64), (300, 64, 7), (2048, 768, 1000), (16385, 16, 300)])
+@pytest.mark.parametrize("T,H,V", [(1, 8, 3), (15, 8, 40), (16, 512, 5), (17, 520, 5), (33, 768, 64), (300, 64, 7), (8, 8, 3), (9, 512, 4), (2048, 768, 1000), (16385, 16, 300)])
 @pytest.mark.parametrize("kind", ["same", "distinct", "skewed", "any"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("add", [False, True])
