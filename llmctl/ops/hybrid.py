@@ -952,7 +952,8 @@ def norm_add_f32_(x, y1, s1: float, y2, s2: float, w, mult: float, eps: float, o
     dtype (row-strided views allowed), or :class:`RowParts`.  ``w_next``: the RMS norm
     of x by these weights instead (the same eps and ``one_plus``)."""
     if type(y1) is RowParts or type(y2) is RowParts:
-        if type(y1) is RowParts and (y2 is None or (type(y2) is RowParts and y2.bias is None)) and out_dtype == torch.bfloat16 and x.data_ptr() % 16 == 0:
+        if (type(y1) is RowParts and (y2 is None or (type(y2) is RowParts and y2.bias is None)) and out_dtype == torch.bfloat16
+                and (x.data_ptr() | w.data_ptr() | (0 if w_next is None else w_next.data_ptr())) % 16 == 0):
             return native_hybrid().norm_add_parts_f32_(x, y1.parts, y1.bias, s1, None if y2 is None else y2.parts, s2, w, mult, eps, one_plus, w_next)
         y1, y2 = (y.total() if type(y) is RowParts else y for y in (y1, y2))
     if w_next is not None:

@@ -87,3 +87,21 @@ def test_fp32_weights(T, N, K):
     assert bool((err <= (K / 256 + 24) * 2.0**-24 * mag).all())  # a thread's chain of K / 256 and the sums over threads
     lib = (torch.nn.functional.linear(x.float(), w).double() - ref).abs()
     assert err.pow(2).mean() <= 4 * lib.pow(2).mean() + (2.0**-25 * mag).pow(2).mean()
+
+
+@pytest.mark.parametrize("off", ["w", "w_next", "x"])
+def test_norm_vectors_off_16_bytes(off):
+    """A norm vector or stream that is an offset view takes the general form, with the same stream."""
+    from llmctl.ops import hybrid as hops
+
+    T, W = 7, 260
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda n, name: torch.randn(n + 1, generator=g, device="cuda")[1 if name == off else 0:][:n]
+    x, w, wn = rand(T * W, "x").view(T, W), rand(W, "w"), rand(W, "w_next")
+    y = torch.randn(3, T, W, generator=g, device="cuda")
+    yb = y.sum(0).bfloat16().double()  # (the general form's product is rounded)
+    want = x.double() + 0.5 * yb / (yb.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * (w.double() + 1.0)
+    h = hops.norm_add_f32_(x, hops.RowParts(y, None), 1.0, None, 0.0, w, 0.5, 1e-6, True, torch.bfloat16, wn)
+    assert bool(((x.double() - want).abs() <= 1e-5 * (x.double().abs() + want.abs() + 1.0)).all())  # an fp32 norm
+    hw = want / (want.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * (wn.double() + 1.0)
+    assert bool(((h.double() - hw).abs() <= (2.0**-8 + 1e-5) * hw.abs() + 1e-5).all())
