@@ -138,7 +138,7 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
     }
     if (g.f32) {
       float* y = static_cast<float*>(g.y) + o;
-      if (left == 4 && (o & 3) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
+      if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
       else
         for (int j = 0; j < left; ++j) y[j] = v[j];
     } else {
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
       unsigned short h[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) h[j] = __bfloat16_as_ushort(__float2bfloat16(v[j]));
-      if (left == 4 && (o & 3) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
+      if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
       else
         for (int j = 0; j < left; ++j) y[j] = h[j];
     }

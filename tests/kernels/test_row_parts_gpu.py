@@ -20,6 +20,21 @@ def test_parts_add_up(M, N, K, parts):
     assert bool(((p.double().sum(0) - ref).abs() <= K * 2.0**-24 * mag).all())  # fp32 sums of exact products
 
 
+@pytest.mark.parametrize("M,N", [(1, 6), (3, 6), (5, 10), (7, 513), (17, 1), (32, 4095)])
+def test_ranges_that_start_between_quads(M, N):
+    """Ranges of M * N sums that are no multiple of four: the second one and later start off 16 bytes, where nothing is stored in quads."""
+    from llmctl.ops.hybrid import native_hybrid
+
+    K = 1000
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+    x, w = torch.randn(M, K, generator=g, device="cuda").bfloat16(), torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    p = native_hybrid().rows_parts(x, w, 4)
+    part = (K // 4 + 31) // 32 * 32
+    for i, got in enumerate(p):
+        xi, wi = x[:, i * part:(i + 1) * part].double(), w[:, i * part:(i + 1) * part].double()
+        assert bool(((got.double() - xi @ wi.t()).abs() <= part * 2.0**-24 * (xi.abs() @ wi.abs().t())).all())
+
+
 @pytest.mark.parametrize("T", [1, 7, 32])
 @pytest.mark.parametrize("W", [4, 260, 1024, 2048, 4096])
 @pytest.mark.parametrize("n1,n2,bias", [(1, 0, False), (4, 0, True), (3, 2, False), (16, 1, True)])
