@@ -536,10 +536,13 @@ class _Embedding(torch.autograd.Function):
             sink: GradSink = w._llmctl_grad_sink
             dy2 = dy.reshape(-1, dy.shape[-1])
             g, add = sink.open(w)
-            if ops.embed_grad_ok(ids, dy2, g):
+            ok = ops.embed_grad_ok(ids, dy2, g)
+            if ok and ops.embed_grad_pays(dy2.shape[0], dy2.shape[1], g.shape[0]):
                 ops.embed_grad_(ids, dy2, g, add)
                 sink.close(w)
             else:
+                if ok and (add or g.dtype == torch.float32):  # (the sums in fp32 up to the flat gradient, as the kernel holds them)
+                    dy2 = dy2.float()
                 sink.add(w, torch.ops.aten.embedding_dense_backward(dy2, ids, w.shape[0], -1, False))
         return None, None
 

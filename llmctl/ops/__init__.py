@@ -25,6 +25,7 @@ from .functional import (
     decode_up_swiglu,
     embed_grad_,
     embed_grad_ok,
+    embed_grad_pays,
     embed_rows,
     flash_attention,
     gelu,
@@ -56,6 +57,7 @@ __all__ = [
     "decode_attention_qkv", "decode_fused_ok", "decode_linear_add_rmsnorm", "decode_norm_linear", "decode_norm_qkv_cache", "decode_qkv_rope_cache", "decode_up_swiglu",
     "embed_grad_",
     "embed_grad_ok",
+    "embed_grad_pays",
     "embed_rows",
     "flash_attention", "gelu", "kv_cache_write", "qkv_flash_attention", "qkv_split_cache", "l2norm_sq", "layernorm", "paged_attention_decode",
     "paged_prefill_attention", "prefill_work_list", "attn_merge_",

@@ -450,6 +450,15 @@ def col_sum_(x, out, add: bool):
 EMBED_GRAD_TOKENS = 65536  # csrc/embed_grad.hip ranks the tokens by comparing all pairs
 
 
+def embed_grad_pays(T: int, H: int, V: int) -> bool:
+    """Is ``embed_grad_`` faster than the library's dense gradient and what adds it?  Ranking all pairs grows with the square of the tokens, the library's sort
+    and passes with the tokens, their rows and the table's (in us, on the right; a small table's rows repeat and stay in cache).  us, library / here, ids drawn
+    evenly: 16384 tokens 32000 x 64 79 / 64, 256 x 64 72 / 63; 24576 32000 x 64 92 / 120, x 256 124 / 125, x 4096 980 / 248; 32768 32000 x 512 187 / 208, x 1024
+    314 / 221; 50000 50304 x 1024 474 / 531, x 2048 927 / 612; 65536 32000 x 64 106 / 724, x 2048 826 / 865.  Ids as often as in text (1 / rank): 24576 32000 x 64
+    144 / 141, 32768 x 512 219 / 239, x 1024 283 / 248, 65536 x 64 253 / 779; all the same 65536 x 64 1725 / 1337."""
+    return T <= EMBED_GRAD_TOKENS and 1.65e-7 * T * T <= 25 + 2.2e-3 * T + 2.9e-6 * min(T, 8 * V) * H + 1.4e-6 * V * H
+
+
 def embed_grad_ok(ids, dy, g) -> bool:
     """Whether ``embed_grad_`` (csrc/embed_grad.hip) takes these ids, rows and gradient."""
     return (use_native(dy) and dy.dim() == 2 and dy.dtype == torch.bfloat16 and dy.stride(1) == 1 and dy.shape[1] % 8 == 0

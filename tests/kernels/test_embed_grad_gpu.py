@@ -70,3 +70,34 @@ def test_sink(tied):
     assert w.grad is flat
     # tied: x's gradient is rounded to bf16 once before the rows are summed; each write rounds the flat gradient once more
     assert (flat.double() - ref).abs().max() <= 6 * 2.0**-8 * ref.abs().max()
+
+
+@pytest.mark.parametrize("T,H,V", [(20000, 8, 256), (24576, 64, 300)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens", ["few", "all"])
+def test_many_tokens_of_narrow_rows(T, H, V, dtype, tokens, monkeypatch):
+    """The library's sums past the rule's line: two backwards, held in fp32 up to the flat gradient as the kernel holds them."""
+    from llmctl import ops
+    from llmctl.exec.linear import GradSink, embedding
+
+    assert not ops.embed_grad_pays(T, H, V) or T == 20000
+    monkeypatch.setattr(ops, "embed_grad_pays", lambda *a: False)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    w = torch.nn.Parameter(torch.randn(V, H, generator=g, device="cuda").bfloat16())
+    flat = torch.full((V, H), float("nan"), device="cuda", dtype=dtype)
+    sink = GradSink()
+    sink.attach(w)
+    if dtype == torch.float32:
+        w.main_grad = flat
+    else:
+        w.grad = flat
+    ref, mag, err = torch.zeros(V, H, device="cuda", dtype=torch.float64), torch.zeros(V, H, device="cuda", dtype=torch.float64), 0.0
+    for _ in range(2):
+        ids = torch.randint(0, V if tokens == "all" else 3, (T,), generator=g, device="cuda")
+        dy = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+        embedding(ids, w).backward(dy)
+        ref.index_add_(0, ids, dy.double())
+        mag.index_add_(0, ids, dy.double().abs())
+        # fp32 sums, and for a bf16 gradient the rounding of each write of it
+        err = err + (T + 1) * 2.0**-24 * mag + (2.0**-8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
+    assert bool(((flat.double() - ref).abs() <= err * (1 + 2.0**-7) + 1e-30).all())
