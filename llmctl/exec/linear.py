@@ -23,6 +23,7 @@ step.  The down projection's data gradient can carry the SwiGLU backward in its 
 
 from __future__ import annotations
 
+import functools
 from typing import Callable, List, Optional, Tuple
 
 import torch
@@ -249,6 +250,15 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         torch.mm(dy2.t(), x2, out=g)
 
 
+@functools.lru_cache(maxsize=4096)
+def _bias_rides(M: int, N: int, K: int, bias: bool) -> bool:
+    """Whether the 256 x 128 tiles take a weight gradient of these sizes (``gemm64_wgrad_splits``).  Kept by size: a call that was refused cost the host 5 us, and a
+    backward that is bound by its launches two of them a layer (300 tokens, 8192 x 2048 with a bias 43.5 us, so 31)."""
+    from llmctl.ops._lib import native
+
+    return native().gemm64_wgrad_splits(M, N, K, bias) > 0
+
+
 def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: Optional[torch.Tensor], add: bool) -> bool:
     """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient, over any number of tokens from 256 on
     (without ``gb`` where they are no multiple of 128); False: nothing done."""
@@ -256,7 +266,8 @@ def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumu
     if not (K >= 256 and _gemm64_ok(M, N, 128, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32)
             and (gb is None or (gb.dtype == g.dtype and gb.is_contiguous()))
             and g.stride(1) == 1 and g.stride(0) % 8 == 0 and g.data_ptr() % 16 == 0
-            and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3):
+            and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3
+            and _bias_rides(M, N, K, gb is not None)):
         return False
     from llmctl.ops._lib import native
 

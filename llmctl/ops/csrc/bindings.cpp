@@ -12,6 +12,7 @@ int64_t car_sig_words();
 int64_t car_error(int64_t sig_ptr);
 void set_knob(const std::string& name, int64_t value);  // knobs.cpp
 void clear_knobs();
+int64_t gemm64_wgrad_splits(int64_t M, int64_t N, int64_t K, bool bias);
 }  // namespace llmctl
 
 TORCH_LIBRARY(llmctl, m) {
@@ -77,6 +78,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("car_ipc_close(int ptr) -> ()", &llmctl::car_ipc_close);
   m.def("car_sig_words() -> int", &llmctl::car_sig_words);
   m.def("car_error(int sig_ptr) -> int", &llmctl::car_error);
+  m.def("gemm64_wgrad_splits(int M, int N, int K, bool bias) -> int", &llmctl::gemm64_wgrad_splits);
   m.def("set_knob(str name, int value) -> ()", &llmctl::set_knob);
   m.def("clear_knobs() -> ()", &llmctl::clear_knobs);
   m.def("gemm_ex(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, int variant=-1) -> ()");

@@ -2,7 +2,7 @@
 //
 // Bound: one pass over dy and the rows of g that it meets (8192 x 4096: 134 MB, 27 us at a copy's rate).  Three launches, no atomics, the same bits every time:
 //   order  the tokens ranked by (id, position): ids in LDS, every wave counts for two tokens the ids below and the equal ones before and in all.  T^2 compares,
-//          four a lane and read; 65536 tokens are the most that is taken here; a radix sort is five launches.
+//          four a lane and read; 65536 tokens are the most that is taken here, and of narrow rows fewer pay (embed_grad_pays); a radix sort is five launches.
 //   rows   a wave per 8 sorted tokens and 512 columns, all loads in flight; a run of one id inside the 8 is final, a run across an edge leaves a partial row
 //   edges  the wave whose 8 a crossing run starts in adds the partial rows in order
 // so a token that fills half the batch is summed by as many waves as any other half.

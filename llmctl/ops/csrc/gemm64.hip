@@ -1797,20 +1797,25 @@ void gemm64_ex(const at::Tensor& a, const at::Tensor& b, at::Tensor& out, bool a
   }
 }
 
+// K-ranges in which the 256 x 128 tiles take a weight gradient dy^T x (dy [K, M], x [K, N]) and, with ``bias``, dy's column sums; 0: not by these sizes.  M, N in
+// 256s; K any number from 256 on, without a bias no multiple of 128 (those are gemm64_ex's).
+int64_t gemm64_wgrad_splits(int64_t M, int64_t N, int64_t K, bool bias) {
+  if (M <= 0 || N <= 0 || M % TM != 0 || N % TN != 0 || K < 4 * TK || (bias ? N < 512 : K % (2 * TK) == 0)) return 0;
+  G64Args plan{};
+  plan.M = (int)M, plan.N = (int)N, plan.K = (int)((K + 2 * TK - 1) / (2 * TK) * (2 * TK)), plan.tiles_m = (int)(M / TM), plan.tiles_n = (int)(N / TN);
+  plan_split(plan, 0);
+  return gemm_tall_splits(M, N, K, plan.n_main, (long)plan.tiles_m * plan.tiles_n - plan.n_main, plan.splits);
+}
+
 // g (+)= dy^T x and db (+)= the column sums of dy where the 256 x 128 tiles take the weight gradient (they carry the sums); false: nothing done, gemm64_ex and
-// col_sum_ are as fast or faster.  dy [T, M], x [T, N]; M, N in 256s; T any number from 256 on, without db no multiple of 128 (those are gemm64_ex's).
+// col_sum_ are as fast or faster.  dy [T, M], x [T, N]; sizes: gemm64_wgrad_splits, which the caller asks first and keeps by size.
 // gpt2-125m, 2 x 1956 tokens: the library's products 49 us a weight gradient and 9 a bias, 30.5 together; the step 9786 us of kernels, so 8498.
 bool gemm64_wgrad_bias(const at::Tensor& dy, const at::Tensor& x, at::Tensor g, bool accumulate, const c10::optional<at::Tensor>& db, bool add) {
   LLMCTL_CHECK(dy.dim() == 2 && x.dim() == 2 && dy.size(0) == x.size(0), "gemm64_wgrad_bias: dy [T, M], x [T, N]");
   const long M = dy.size(1), N = x.size(1), K = dy.size(0);
-  const bool whole = K % (2 * TK) == 0;
-  if (M <= 0 || N <= 0 || M % TM != 0 || N % TN != 0 || K < 4 * TK || (db.has_value() ? N < 512 : whole)) return false;
-  if (!whole && (dy.stride(0) < M || x.stride(0) < N)) return false;
+  if (K % (2 * TK) != 0 && (dy.stride(0) < M || x.stride(0) < N)) return false;
   const c10::DeviceGuard dg(dy.device());
-  G64Args plan{};
-  plan.M = (int)M, plan.N = (int)N, plan.K = (int)((K + 2 * TK - 1) / (2 * TK) * (2 * TK)), plan.tiles_m = (int)(M / TM), plan.tiles_n = (int)(N / TN);
-  plan_split(plan, 0);
-  const int S = gemm_tall_splits(M, N, K, plan.n_main, (long)plan.tiles_m * plan.tiles_n - plan.n_main, plan.splits);
+  const int64_t S = gemm64_wgrad_splits(M, N, K, db.has_value());
   if (S == 0) return false;
   gemm_tall(dy, x, g, true, accumulate, S, db, add);
   return true;

@@ -159,3 +159,28 @@ def test_weight_gradients_of_odd_batches(tokens, out, inn, f32):
         linear(x, w, b).backward(dy)
     for p, ref in ((w, dy.double().t() @ x.double()), (b, dy.double().sum(0))):
         assert bool(((p.main_grad.double() - 2 * ref).abs() <= 2.0**-7 * 2 * ref.abs() + 1e-3 * ref.abs().max()).all())
+
+
+def test_refusals_are_kept_by_size(monkeypatch):
+    """Sizes that the 256 x 128 tiles leave to others are asked about once, not in every backward."""
+    import importlib
+
+    from llmctl.ops._lib import native
+
+    L = importlib.import_module("llmctl.exec.linear")
+    L._bias_rides.cache_clear()
+    K, M, N = 300, 6144, 2048
+    assert native().gemm64_wgrad_splits(M, N, K, True) == 0
+    calls = []
+
+    class Counting:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(native(), name)
+
+    monkeypatch.setattr("llmctl.ops._lib.native", lambda: Counting())
+    dy, x = torch.randn(K, M, device="cuda").bfloat16(), torch.randn(K, N, device="cuda").bfloat16()
+    g, gb = torch.empty(M, N, device="cuda", dtype=torch.bfloat16), torch.empty(M, device="cuda", dtype=torch.bfloat16)
+    for _ in range(3):
+        assert not L.wgrad_bias_into(g, dy, x, False, gb, False)
+    assert calls == ["gemm64_wgrad_splits"]
