@@ -358,20 +358,28 @@ void launch(const TallArgs& g, int out) {
 }  // namespace
 
 // K-ranges for this kernel where it is the faster one, else 0.  n_main whole tiles of 256 x 256 and n_tail in `splits` ranges each are gemm64's plan.  Both
-// times from the sizes, us: a round costs its K-tiles (0.72 here and 1.3 there for 64 of K, on a full chip) and a fixed part (4, 7: fill and store); partial sums
-// cost a launch (4) and their bytes, written and read, at 6 TB/s.  Ranges stay at four K-tiles and more, what the peeled loop takes.
-// Both sides measured, us: see above where these win; 192 tiles of 256 x 256 (4096 x 3072 x 768) 25.8 / 27.6 and 256 (4096 x 4096 x 2048) 53.0 / 62.4 there.
+// times from the sizes, us: a round costs its K-tiles and a fixed part (fill and store), a K-tile of 64 more the fuller the chip is (0.74 here on an empty one, 0.80
+// on a full one; 0.92 and 1.28 there); partial sums cost a launch and their bytes, written and read.  Ranges stay at four K-tiles and more, what the peeled loop
+// takes.  Constants fitted to 540 sizes, both layouts, 256 to 24576 rows, operands from HBM (profiles/backward_tiles.txt): the choice is within 0.5 % of the faster one
+// on average; by it these tiles take 13 % less time than 256 x 256 ones everywhere, and in 5 sizes 3 to 7 % more (12288 x 2048 x 1536 71.9, here 77.2).  The margin
+// keeps long single rounds of less than the chip on the others, which their last K-tiles' loads hold up here (2560 x 2560 weight gradients over 16384 rows 191 there,
+// here 250; 5120 x 1280 over 6144 80 and 97).
 int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits) {
   const double cus = num_cus(), kt = (K + 2 * TK - 1) / (2 * TK) * 2;
-  auto rounds = [&](double items) { return std::ceil(items / cus); };
-  auto sums = [](double entries, int S) { return S > 1 ? 4.0 + entries * S * 8.0 / 6e6 : 0.0; };
-  double other = rounds(n_main) * (kt * 1.3 + 7.0);
-  if (n_tail > 0) other += rounds((double)n_tail * splits) * (kt / splits * 1.3 + 7.0) + sums((double)n_tail * TM * TN, splits);
+  auto rounds = [&](double items, double k, double empty, double full, double fixed) {
+    const double whole = std::floor(items / cus), rest = items - whole * cus;
+    return whole * (k * (empty + full) + fixed) + (rest > 0 ? k * (empty + full * rest / cus) + fixed : 0.0);
+  };
+  auto other = [&](double items, double k) { return rounds(items, k, 0.92, 0.36, 10.4); };
+  double limit = other((double)n_main, kt);
+  if (n_tail > 0) limit += other((double)n_tail * splits, kt / splits);
+  if (n_tail > 0 && splits > 1) limit += 8.2 + (double)n_tail * TM * TN * splits * 8.0 / 14.7e6;
+  limit *= 0.972;
   int best = 0;
   for (int S = 1; S <= 16 && K >= 4L * TK * S; ++S) {
-    const double part = 2.0 * std::ceil(kt / 2.0 / S);
-    const double us = rounds((double)(M / TM) * (N / TALL_N) * S) * (part * 0.72 + 4.0) + sums((double)M * N, S);
-    if (us < other) other = us, best = S;
+    const double us = rounds((double)(M / TM) * (N / TALL_N) * S, 2.0 * std::ceil(kt / 2.0 / S), 0.743, 0.06, 5.4) +
+                      (S > 1 ? 5.8 + (double)M * N * S * 8.0 / 9.6e6 : 0.0);
+    if (us < limit) limit = us, best = S;
   }
   return best;
 }

@@ -184,3 +184,12 @@ def test_refusals_are_kept_by_size(monkeypatch):
     for _ in range(3):
         assert not L.wgrad_bias_into(g, dy, x, False, gb, False)
     assert calls == ["gemm64_wgrad_splits"]
+
+
+@pytest.mark.parametrize("M,N,K,ranges", [(2560, 2560, 16384, 0), (5120, 1280, 6144, 0), (6144, 2048, 16384, 0), (3072, 1024, 12288, 0), (1536, 2048, 8192, 0), (768, 3072, 8192, 3),
+                                          (2304, 768, 8192, 4), (2048, 2048, 2048, 1), (1024, 4096, 6144, 2), (4096, 4096, 8192, 0)])
+def test_sizes_of_the_rule(M, N, K, ranges):
+    """Weight gradients on both sides of the line (``profiles/backward_tiles.txt``)."""
+    from llmctl.ops._lib import native
+
+    assert native().gemm64_wgrad_splits(M, N, K, True) == ranges
