@@ -263,11 +263,12 @@ def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumu
     """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient, over any number of tokens from 256 on
     (without ``gb`` where they are no multiple of 128); False: nothing done."""
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
-    if not (K >= 256 and _gemm64_ok(M, N, 128, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32)
+    if M % 256 or N % 256 or K < 256 or not dy2.is_cuda or not _bias_rides(M, N, K, gb is not None):  # (most refusals end here)
+        return False
+    if not (_gemm64_ok(M, N, 128, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32)
             and (gb is None or (gb.dtype == g.dtype and gb.is_contiguous()))
             and g.stride(1) == 1 and g.stride(0) % 8 == 0 and g.data_ptr() % 16 == 0
-            and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3
-            and _bias_rides(M, N, K, gb is not None)):
+            and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31 and gemm64_config("wgrad", M, N, K) // 100 == 3):
         return False
     from llmctl.ops._lib import native
 
