@@ -136,6 +136,12 @@ def dgrad64_rows(tokens: int, w: torch.Tensor) -> int:
     return rows
 
 
+def _tied(w: torch.Tensor) -> bool:
+    """A weight that is the embedding and the output projection.  It keeps no W^T copy: its data gradient runs on gemm64 whatever the tokens, us, W^T copy made
+    and read / gemm64: 50304 x 768 16640 tokens 1510 / 1271, 20480 1529 / 1098, 50304 x 1024 20480 1630 / 1447, 32000 x 2048 20480 2511 / 1736."""
+    return getattr(w, "_llmctl_writes", 1) > 1
+
+
 def weight_t_ok(tokens: int, w: torch.Tensor) -> bool:
     """Does the data gradient of a sinked ``w`` for ``tokens`` rows go through a W^T copy?  Where it does not run on gemm64, and
     (knob dgrad64 = auto, unless its sink was made to keep copies) the layout's gain on the product covers the copy: weights of 2^24
@@ -143,7 +149,7 @@ def weight_t_ok(tokens: int, w: torch.Tensor) -> bool:
     8.51, 4096 16.2 / 16.0, 8192 26.4 / 26.7, 16384 47.1 / 48.2; gpt2-125m (weights of at most 2^21.2 entries) 1024 tokens 12.2 /
     8.8, 8192 13.2 / 12.9, 32768 37.5 / 37.1."""
     sink = getattr(w, "_llmctl_grad_sink", None)
-    if sink is None or dgrad64_shape_ok(tokens, w):
+    if sink is None or _tied(w) or dgrad64_shape_ok(tokens, w):
         return False
     if sink.always_transpose or knobs().dgrad64 != "auto":
         return True
@@ -499,9 +505,9 @@ class _Linear(torch.autograd.Function):
                 wgrad_into(dw, dy2, x2, accumulate=False)
         dx = None
         if ctx.needs_input_grad[0]:
-            # an unsinked weight keeps no W^T copy, so its alternative is hipBLASLt's slower "NN"
+            # an unsinked or tied weight keeps no W^T copy, so its alternative is hipBLASLt's slower "NN"
             # layout: gemm64 (W read K-major) whenever the shape fits, unless knob dgrad64 is off
-            free = getattr(ctx.wparam, "_llmctl_grad_sink", None) is None and knobs().dgrad64 != "off"
+            free = (getattr(ctx.wparam, "_llmctl_grad_sink", None) is None or _tied(ctx.wparam)) and knobs().dgrad64 != "off"
             if dgrad64_ok(dy2, w) or (free and dy2.is_cuda and dy2.dtype == torch.bfloat16 and _rows_ok(dy2)
                                       and _gemm64_ok(dy2.shape[0], w.shape[1], w.shape[0], w)
                                       and w.shape[0] * w.stride(0) * 2 < 2**31):

@@ -28,3 +28,25 @@ def test_data_gradient_routes(T, inn, out, route):
     want = dy.float() @ w.detach().float()
     # one rounding to bf16 over fp32 sums of ``out`` terms
     assert ((x.grad.float() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * out ** 0.5).all()
+
+
+@pytest.mark.parametrize("T,inn,out,gemm64", [(16384, 256, 128, True), (16640, 256, 128, True), (16640, 4096, 4096, True), (16700, 4096, 4096, False), (16640, 4096, 4104, False)])
+def test_a_tied_weight_keeps_no_copy(T, inn, out, gemm64, monkeypatch):
+    """The embedding that is the output projection too: gemm64 beyond 16384 rows as well, else W as it is."""
+    import importlib
+
+    from llmctl.config.knobs import override
+
+    L = importlib.import_module("llmctl.exec.linear")
+    rows, whole = [], L.dgrad64
+    monkeypatch.setattr(L, "dgrad64", lambda dy, w, r=None: rows.append(r) or whole(dy, w, r))
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    with override(dgrad64="auto"):
+        x, w, dy = r(T, inn).requires_grad_(), torch.nn.Parameter(r(out, inn)), r(T, out)
+        w.grad = torch.zeros_like(w)
+        L.GradSink().attach(w, 2)
+        L.linear(x, w).backward(dy)
+    assert getattr(w, "_llmctl_wt", None) is None and rows == ([None] if gemm64 else [])
+    want = dy.float() @ w.detach().float()
+    assert ((x.grad.float() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * out ** 0.5).all()
