@@ -250,7 +250,10 @@ class InferenceEngine:
             self.model.step(batch, self.kv_cache, rows=rows_d)
             return torch.empty(0, self.cfg.vocab_size, device=d, dtype=self.dtype)
         every = len(rows) == len(ids) and list(rows) == list(range(len(ids)))  # (a decode step reads all of its rows)
-        x = self.model.step(batch, self.kv_cache, rows=None if every else rows_d, trail=trail)
+        if every and trail is None and Tp == 0 and getattr(self.model, "normed_step", False):
+            x = self.model.step(batch, self.kv_cache, final=True)  # (as it is recorded: the same bits)
+        else:
+            x = self.model.step(batch, self.kv_cache, rows=None if every else rows_d, trail=trail)
         return self.model.logits(x)
 
     def _weights_key(self):

@@ -316,3 +316,70 @@ def test_the_upload_of_a_step_does_not_wait():
     assert not done.query()
     for g, w in zip(got, want):
         assert g.shape == w.shape and torch.equal(g.cpu(), torch.from_numpy(w))
+
+
+def _cache_tensors(e):
+    out = []
+    for i in range(len(e.kv_cache._layers)):
+        v = e.kv_cache.layer(i)
+        for w in v if isinstance(v, tuple) else (v,):
+            out += list(w) if isinstance(w, tuple) else [w]
+    return out
+
+
+@pytest.mark.parametrize("name,cut", [("lenitar-w128-l4", None), ("malinex-w128-l4-h4-g2-e4-s1", None), ("malinex-w128-l3-h4-g2", None), ("dumazen-w128-l4-h4-g2", None),
+                                      ("dumazen-w128-l4-h4-g2", "ff"), ("dumazen-w128-l4-h4-g2", "layers"), ("malinex-w128-l3-h4-g2", "layers")])
+def test_a_step_gives_the_same_bits_captured_or_not(name, cut):
+    """One decode step from the same caches, eager, captured, and eager with the final norm as a pass of its own; a last layer without a feed-forward part, and
+    no layers at all."""
+    from llmctl.serve.decode_graph import DecodeGraph
+    from llmctl.serve.scheduler import PrefillChunk
+
+    e = _engine(name, False, torch.bfloat16)
+    if cut == "ff":
+        e.model.layers[-1].ff = None
+    elif cut == "layers":
+        if hasattr(e.model, "order"):
+            e.model.order = []
+        else:
+            e.model.layers = torch.nn.ModuleList()
+    gen = torch.Generator().manual_seed(2)
+    seqs = []
+    for n in (63, 40, 17):  # the longest context becomes 64, which the captured step's bound is too
+        ids = torch.randint(0, 500, (n,), generator=gen).tolist()
+        s = e.open_sequence(ids)
+        e.prefill([PrefillChunk(s, 0, n)])
+        e.scheduler.computed(s, n)
+        e.scheduler.extend(s, [n])
+        s._decode_slot = int(e.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+        seqs.append(s)
+    plan = e.decode_plan(seqs)
+    assert max(plan["ctx"]) == 64
+    live = _cache_tensors(e)
+    saved = [t.clone() for t in live]
+
+    def restore():
+        with torch.inference_mode():
+            for t, v in zip(live, saved):
+                t.copy_(v)
+
+    with torch.inference_mode():
+        eager = e.decode_exec(plan).clone()
+        restore()
+        g = DecodeGraph(3, e.max_blocks_per_seq, 64, e.device)
+        g.capture(e.model, e.kv_cache, torch.cuda.graph_pool_handle())
+        run = lambda: g.run({"ids": plan["ids"], "slots": plan["slots"], "pos": plan["positions"], "ctx": plan["ctx"], "start": plan["positions"], "state": plan["state"],
+                             "bt": plan["bt"]})
+        captured = run()
+        for _ in range(2):  # (a replay after others, from the same caches)
+            restore()
+            assert torch.equal(run(), captured)
+        restore()
+        e.model.normed_step = False  # the final norm of its own, in the form that prompts take
+        apart = e.decode_exec(plan)
+        assert torch.equal(eager, captured)
+        # the same norm in another order of its sum: its bf16 results may round the other way
+        a, b = eager.float(), apart.float()
+        assert ((a - b).norm(dim=1) <= 2.0**-7 * b.norm(dim=1)).all()
+    g.release()
+    e.close()
