@@ -328,7 +328,7 @@ def _cache_tensors(e):
 
 
 @pytest.mark.parametrize("name,cut", [("lenitar-w128-l4", None), ("malinex-w128-l4-h4-g2-e4-s1", None), ("malinex-w128-l3-h4-g2", None), ("dumazen-w128-l4-h4-g2", None),
-                                      ("dumazen-w128-l4-h4-g2", "ff"), ("dumazen-w128-l4-h4-g2", "layers"), ("malinex-w128-l3-h4-g2", "layers")])
+                                      ("malinex-w2048-l3-h16-g4", None), ("dumazen-w2048-l3-h16-g4", None), ("dumazen-w128-l4-h4-g2", "ff"), ("dumazen-w128-l4-h4-g2", "layers"), ("malinex-w128-l3-h4-g2", "layers")])
 def test_a_step_gives_the_same_bits_captured_or_not(name, cut):
     """One decode step from the same caches, eager, captured, and eager with the final norm as a pass of its own; a last layer without a feed-forward part, and
     no layers at all."""
