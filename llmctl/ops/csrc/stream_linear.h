@@ -160,17 +160,28 @@ inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
   kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + rows - 1) / rows), parts), NW * 64, 0, st>>>(g);
 }
 
-// Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to
-// nothing, and from 6144 outputs on smaller workgroups in more rounds hide the latency better (one row, K 2048, one round / rounds of at most 16
-// weight rows: N 8192 9.9 / 8.5 us, N 12288 13.0 / 12.0; from K 3072 on the other way: N 9248 x 4096 17.7 / 18.3, so rounds of 32 there).  The
-// waves and so the order of a sum depend on M, N and K alone, not on who owns an output (8 waves of 4 steps instead of 4 of 8: N 2048 6.00 /
-// 6.06 us, N 4096 7.16 / 7.26, not worth other results).
+// Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to nothing, and
+// from 6144 outputs on smaller workgroups in more rounds hide the latency better (one row, one round / rounds of at most 16 weight rows: 8192 x 2048 9.9 / 8.5 us,
+// 12288 x 2048 13.0 / 12.0, 8192 x 2304 11.3 / 9.9; four rows from K 3072 on the other way: 9248 x 4096 17.7 / 18.3, so rounds of 32 there).  Half as many rows where those
+// of W lie a multiple of 8192 entries apart and crowd the same channels (16384 x 8192: four rows of x 64.8 / 53.9, five 72.9 / 57.6), and for more than 12288 short
+// ones (five rows 15360 x 1024 9.7 / 8.9).  Below K 512 a workgroup of its own for a few outputs costs more than idle CUs: whole tiles (768 x 256
+// 3.3 / 2.9).  The waves and so the order of a sum depend on M, N and K alone, not on who owns an output (8 waves of 4 steps instead of 4 of 8: N 2048 6.00 / 6.06
+// us, N 4096 7.16 / 7.26, not worth other results).
 inline void launch(const Args& g, hipStream_t st) {
   const bool few = g.M <= 4 && g.N >= 6144;
-  const int tall = !few ? 64 : g.N > 16384 || g.K <= 2048 ? 16 : 32;         // rows of a workgroup at most
-  const int rounds = (g.N + 256 * tall - 1) / (256 * tall);                  // of 256 workgroups
-  int rows = (g.N + 256 * rounds - 1) / (256 * rounds);
-  if (g.N > 16384) rows = few ? 16 : (rows + 3) / 4 * 4;  // (whole quads are stored at once)
+  int rows;
+  if (g.K < 512) {
+    rows = few || g.N < 5120 ? 16 : g.M > 16 || g.N < 24576 ? 32 : 64;
+  } else {
+    int tall = !few ? 64 : g.N > 16384 || g.K <= 2048 || (g.M <= 3 && g.N <= 8192 && g.K <= 3072) ? 16 : 32;  // rows of a workgroup at most
+    if (g.M <= 16 && g.N <= 16384) {
+      if (g.K % 8192 == 0 && g.N > (few ? 8192 : 12288)) tall /= 2;
+      else if (!few && g.K <= 1024 && g.N > 12288) tall = 32;
+    }
+    const int rounds = (g.N + 256 * tall - 1) / (256 * tall);  // of 256 workgroups
+    rows = (g.N + 256 * rounds - 1) / (256 * rounds);
+    if (g.N > 16384) rows = few ? 16 : (rows + 3) / 4 * 4;  // (whole quads are stored at once)
+  }
   if (g.M > 16) {
     if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
     else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);

@@ -585,17 +585,26 @@ def stream_ok(x, w, b=None) -> bool:
 def stream_pays(M: int, N: int, K: int) -> bool:
     """Is the weight stream faster than the library's product?  In a graph, weights from HBM, us, library / here, beside each line.  (The
     library splits K over the chip at some sizes and not at others: 16 rows 4096 x 8192 15.0, 4096 x 11008 37.)"""
-    if M > 16:  # a fragment of x more for every one of W: 32 rows 4240 x 2048 12.2 / 9.7, 12288 x 2048 15.7 / 15.5, 14336 x 1024 21.5 / 10.8, but 14336 x 2048
-        # 16.7 / 17.2, 6144 x 3072 13.1 / 14.2, 50304 x 768 20.7 / 25.2; 152064 x 3072 295 / 202; 24 rows 4096 x 4096 13.6 / 13.1
-        return K <= (2048 if N <= 12288 else 1024 if N <= 32000 else 0) or (N >= 102400 and K <= 4096) or (M <= 24 and N <= 4096 and K <= 4096)
+    if M > 16:  # a fragment of x more for every one of W: 32 rows 4240 x 2048 12.2 / 9.7, 12288 x 1024 12.4 / 9.4, 16384 x 512 8.8 / 7.2, but 12288 x 256 5.3 / 5.8,
+        # 28672 x 768 13.9 / 15.7, 6144 x 3072 13.1 / 14.2, 50304 x 768 20.7 / 25.2, 102400 x 256 17.6 / 18.4; 24 rows 4096 x 4096 13.6 / 13.1, 12288 x 2048 15.8 / 15.0
+        if N > 40960:  # where the last of the library's rounds of 256-wide tiles leaves CUs idle: 32 rows 152064 x 3072 295 / 202, 128256 x 2304 110 / 131
+            return N >= 102400 and (512 if M > 24 else 0) <= K <= 4096 and 0 < -(-N // 256) % 256 <= 192
+        if N > 8192:
+            return 512 <= K <= (2048 if N <= 12288 and M <= 24 else 1024) and (N <= 24576 or 31744 <= N <= 32000)
+        return K <= 2048 or (M <= 24 and N <= 4096 and K <= 4096)
     if K > 4096 and K % 8192 == 0:  # rows of W that lie a multiple of 8192 entries apart crowd the same channels: 8 rows 2048 x 8192 13.0 / 12.4, 6144 x 8192
-        # 23.7 / 25.6, 16384 x 16384 101 / 129; 4 rows 32000 x 8192 111 / 94; 16 rows 2048 x 8192 13.6 / 15.4
-        return (M <= 8 and N <= (4096 if K == 8192 else 2304)) or (M <= 4 and K == 8192 and N >= 20480)
-    if K > 4096 and M > 8:  # a workgroup reads all of x for its few rows of W: 16 rows 3648 x 6144 13.2 / 14.8, 2304 x 5120 12.3 / 11.7, 12288 x 10240 58 / 51, 32000 x
-        # 6144 86 / 77, 50304 x 12288 220 / 237
-        return 4096 < N <= 40960 or (N <= 2304 and K < 6144)
-    if K > 4096:  # 8 rows 2048 x 6144 11.2 / 10.1, 4096 x 12288 23.0 / 24.5, 12288 x 12288 61 / 57, 50304 x 5120 94 / 102
-        return M <= 4 or ((N <= 40960 or N >= 61440) and not (K % 4096 == 0 and K < 16384 and 2304 < N <= 4096))
+        # 23.7 / 25.6, 16384 x 16384 101 / 129; 4 rows 12288 x 8192 48 / 51, 16384 x 8192 63 / 55, 32000 x 8192 111 / 94; 16 rows 2048 x 8192 13.6 / 15.4
+        return (M <= 8 and N <= (4096 if K == 8192 else 2304)) or (M <= 5 and K == 8192 and 16384 <= N <= 40960)
+    if K > 4096 and M > 8:  # a workgroup reads all of x for its few rows of W: 16 rows 3648 x 6144 13.2 / 14.8, 1024 x 5120 7.5 / 9.3, 6144 x 7168 19.8 / 22.5, 12288 x 10240
+        # 58 / 51, 32000 x 6144 86 / 77, 50304 x 12288 220 / 237; 14 rows 1024 x 5120 12.5 / 8.2; 12 rows 6144 x 7168 19.8 / 21.2
+        if 24576 < N <= 30720 and 10240 < K < 12288:
+            return False
+        return (8192 if M > 12 and K <= 10240 else 4096) < N <= 40960 or (N <= 2304 and K < 6144 and (M <= 14 or N > 1024))
+    if K > 4096:  # 8 rows 2048 x 6144 11.2 / 10.1, 4096 x 12288 23.0 / 24.5, 3072 x 14336 20.2 / 23.8, 12288 x 12288 61 / 57, 50304 x 5120 94 / 102; 4 rows 50304 x 11008 195 / 234, 24576 x
+        # 20480 176 / 201
+        if 40960 < N < 61440 or (M <= 4 and 24576 < N <= 30720 and 10240 <= K <= 12288) or (K > 16384 and N >= 18432):
+            return False
+        return M <= 4 or not (K % 2048 == 0 and 12288 <= K < 16384 and 2304 < N <= (4096 if K == 12288 else 3840))
     # 16 rows 2048 x 2048 11.1 / 6.1, 8256 x 2048 14.2 / 11.0, 32000 x 2048 35 / 30, 50304 x 768 20.0 / 21.8, 50304 x 3072 62 / 68, 102400 x 2048 147 / 86, 65024 x 3072
     # 76 / 81, 152064 x 3072 295 / 183; 4 rows 50304 x 768 19.7 / 19.3
     return M <= 4 or N <= 40960 or N >= 61440
@@ -605,13 +614,17 @@ def stream_pays(M: int, N: int, K: int) -> bool:
 def decode_form(M: int, N: int, K: int) -> str:
     """The form of :func:`decode_linear` by size: ``stream``, ``skinny`` (``csrc/skinny_gemm.hip``) or ``library``.  Beside
     :func:`stream_pays`, us in a graph, stream / skinny:"""
-    # short rows: 1 row 2304 x 768 3.63 / 3.32, 8192 x 768 5.66 / 5.30; 16 rows 768 x 512 3.48 / 3.07, 5152 x 512 4.51 / 4.08, but 2304 x 768 4.10 / 4.06 and 768 x 768
-    # 3.88 / 3.97; 24 rows 4096 x 768 4.87 / 4.57
-    if K < (768 if 4 < M <= 16 and N < 3072 else 1024) and N <= (16384 if M <= 4 else 5152 if M <= 16 else 4096):
+    # short rows: 1 row 2304 x 768 3.63 / 3.32, 8192 x 768 5.66 / 5.30; 16 rows 768 x 512 3.48 / 3.07, 512 x 768 3.8 / 3.4, but 2304 x 768 4.10 / 4.06 and 768 x 768 3.88 / 3.97; 24
+    # rows 4096 x 768 4.87 / 4.57.  (More than 4096 outputs that are a multiple of 64 take skinny's other tiles: 16 rows 5120 x 512 4.6 / 6.8, but 5152 x 512 4.5 / 4.1.)
+    if K < (768 if 4 < M <= 16 and 512 < N < 3072 else 1024) and N <= (16384 if M <= 4 else 5152 if M <= 16 and N % 64 else 4096):
         return "skinny"
-    # few long rows, of which skinny splits K over the chip: 8 rows 1024 x 12288 15.0 / 13.3, 16 rows 768 x 10240 15.5 / 13.6, 12 rows 2048 x 28672 42.6 / 37.1,
-    # 16 rows 2048 x 14336 24.7 / 21.5
-    if 4 < M <= 16 and K > (8192 if N <= 1024 else 12288) and N <= (2048 if M >= 8 else 1024):
+    if M <= 4 and 2304 <= N <= 4096 and K <= 1280:  # 4 rows 3072 x 1280 4.9 / 4.7, 3648 x 1280 5.1 / 4.7
+        return "skinny"
+    if 4 < M <= 16 and N % 64 and 8192 < N <= 10240 and K < (1024 if M <= 8 else 512):  # 8 rows 9248 x 256 4.4 / 3.6, x 896 7.3 / 6.8; 16 rows x 384 5.5 / 4.5
+        return "skinny"
+    # few long rows, of which skinny splits K over the chip: 8 rows 1024 x 12288 15.0 / 13.3, 1280 x 11008 14.8 / 13.4, 16 rows 768 x 10240 15.5 / 13.6, 1536 x 10240 17.5 / 14.9,
+    # 12 rows 2048 x 28672 42.6 / 37.1, 16 rows 2048 x 14336 24.7 / 21.5
+    if 4 < M <= 16 and K > (8192 if N <= (1024 if M < 8 else 1280 if M < 12 else 1536) else 12288) and N <= (2048 if M >= 8 else 1024):
         return "skinny"
     # (the library's own times jump here: 12 rows 2048 x 11008 35.8, stream 18.2; 2048 x 10240 13.1 and 13.1)
     return "stream" if stream_pays(M, N, K) or (M <= 16 and N <= 4096 and K % 8192) else "library"

@@ -9,3 +9,19 @@ from llmctl.ops import functional as F
                                         (65536, 4096, 32000, True), (65537, 4096, 32000, False)])
 def test_embedding_gradients(T, H, V, pays):
     assert F.embed_grad_pays(T, H, V) == pays
+
+
+@pytest.mark.parametrize("M,N,K,stream", [(32, 12288, 256, False), (32, 12288, 512, True), (32, 12288, 1280, False), (24, 12288, 2048, True), (17, 28672, 768, False), (24, 32000, 1024, True),
+                                          (32, 128256, 2304, False), (32, 152064, 3072, True), (32, 102400, 256, False), (17, 102400, 256, True), (16, 1024, 5120, False),
+                                          (14, 1024, 5120, True), (16, 6144, 7168, False), (16, 6912, 11008, True), (12, 29696, 11008, False), (4, 16384, 8192, True), (5, 16384, 8192, True),
+                                          (4, 12288, 8192, False), (8, 3072, 14336, False), (8, 4096, 14336, True), (4, 50304, 11008, False), (4, 24576, 20480, False), (4, 29696, 11008, False),
+                                          (1, 2048, 2048, True)])
+def test_weight_streams(M, N, K, stream):
+    assert F.stream_pays(M, N, K) == stream
+
+
+@pytest.mark.parametrize("M,N,K,form", [(16, 5120, 512, "stream"), (16, 5152, 512, "skinny"), (8, 4608, 256, "stream"), (8, 512, 768, "skinny"), (8, 768, 768, "stream"), (16, 1536, 10240, "skinny"),
+                                        (8, 1280, 11008, "skinny"), (8, 1536, 11008, "stream"), (16, 9248, 384, "skinny"), (16, 9248, 512, "stream"), (8, 9248, 896, "skinny"),
+                                        (4, 3648, 1280, "skinny"), (4, 2048, 1280, "stream"), (5, 16384, 8192, "stream"), (16, 2048, 14336, "skinny"), (1, 2304, 768, "skinny")])
+def test_forms_of_a_few_rows(M, N, K, form):
+    assert F.decode_form(M, N, K) == form
