@@ -17,6 +17,8 @@ residual stream are fp32 inside every kernel whatever the activation dtype (bf16
 
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import ref_hybrid as ref
@@ -554,10 +556,18 @@ def row_ranges(M: int, N: int) -> int:
     return 4 if N <= 2048 or M > 16 else 2
 
 
+@functools.lru_cache(maxsize=4096)
+def parts_pay(M: int, N: int, K: int) -> bool:
+    """Are partial sums, added by the residual norm, faster than the whole product?  Product and norm in a graph, weights from HBM, us, whole / parts: 16 rows 2048 x 512 7.1 / 6.8,
+    1024 x 4096 11.1 / 6.8, 4096 x 11008 40 / 25, but 2048 x 256 5.9 / 6.3 and 1536 x 256 (5 rows) 5.6 / 6.3; 32 rows 4096 x 2048 12.9 / 11.5, 4096 x 1024 10.3 / 11.0, 2560 x 512 8.2 / 8.8;
+    8 rows 4096 x 16384 37.3 / 39.9."""
+    return M <= 32 and N % 4 == 0 and N <= 4096 and K >= 512 and not (M > 16 and N > 2048 and K < 2048) and not (4 < M <= 16 and N > 3072 and K >= 16384)
+
+
 def linear_parts(x, w, b=None):
     """:func:`linear` for a reader that takes :class:`RowParts` as well."""
     M, N = x.shape[0], w.shape[0]
-    if M <= 32 and N % 4 == 0 and N <= 4096 and stream_takes(x, w, b) and (b is None or b.data_ptr() % 8 == 0):
+    if parts_pay(M, N, x.shape[1]) and stream_takes(x, w, b) and (b is None or b.data_ptr() % 8 == 0):
         return RowParts(native_hybrid().rows_parts(x, w, row_ranges(M, N)), b)
     return linear(x, w, b)
 

@@ -75,7 +75,8 @@ def test_norm_with_the_next(T, W, parts):
     assert bool(((h.double() - want).abs() <= (2.0**-8 + 1e-5) * want.abs() + 1e-30).all())
 
 
-@pytest.mark.parametrize("M,N,K,parts", [(16, 2048, 8192, 4), (4, 2048, 2048, 2), (32, 4096, 512, 4), (33, 1024, 512, 0), (8, 4100, 512, 0), (8, 514, 512, 0)])
+# (32 rows 4096 x 512: whole 8.9 us with the norm, in four ranges 9.8)
+@pytest.mark.parametrize("M,N,K,parts", [(16, 2048, 8192, 4), (4, 2048, 2048, 2), (32, 4096, 512, 0), (32, 4096, 2048, 4), (33, 1024, 512, 0), (8, 4100, 512, 0), (8, 514, 512, 0)])
 def test_rule(M, N, K, parts):
     from llmctl.ops import hybrid as hops
 

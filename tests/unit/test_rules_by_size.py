@@ -2,6 +2,7 @@
 import pytest
 
 from llmctl.ops import functional as F
+from llmctl.ops import hybrid as H
 
 
 @pytest.mark.parametrize("T,H,V,pays", [(8192, 64, 256, True), (16384, 64, 256, True), (24576, 64, 32000, False), (24576, 4096, 32000, True), (32768, 128, 50304, False),
@@ -25,3 +26,9 @@ def test_weight_streams(M, N, K, stream):
                                         (4, 3648, 1280, "skinny"), (4, 2048, 1280, "stream"), (5, 16384, 8192, "stream"), (16, 2048, 14336, "skinny"), (1, 2304, 768, "skinny")])
 def test_forms_of_a_few_rows(M, N, K, form):
     assert F.decode_form(M, N, K) == form
+
+
+@pytest.mark.parametrize("M,N,K,pays", [(16, 2048, 512, True), (16, 2048, 256, False), (32, 4096, 2048, True), (32, 4096, 1024, False), (32, 2048, 1024, True), (8, 4096, 16384, False),
+                                        (17, 4096, 16384, True), (4, 4096, 16384, True), (33, 2048, 2048, False), (16, 4100, 2048, False)])
+def test_partial_sums(M, N, K, pays):
+    assert H.parts_pay(M, N, K) == pays
