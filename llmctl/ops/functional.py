@@ -753,23 +753,39 @@ def _gemm64_fwd_takes(x, w, b=None) -> bool:
 
 
 def odd_linear(x, w, b=None):
-    """``x @ w^T (+ b)`` for layers whose outputs fill no whole tiles of 256: the in-house kernel where the library's products lose to it, else the
-    library's.  From 9 * 2^20 outputs on, us, library / here: K 2048 2300 x 4240 44.8 / 40.6, 3379 x 4240 64.5 / 49.2, 3379 x 9248 132 / 114, 4090 x 12008
-    201 / 145, 2911 x 8256 93 / 87; K 1024 2911 x 4240 42 / 28; K 4096 2300 x 4240 74 / 70; below: 1331 x 4240 29 / 39, 1800 x 5152 44 / 42.  (Outputs in
-    whole tiles: 3379 x 6144 73 / 86, 3379 x 8192 88 / 95.)"""
-    N = w.shape[0]
-    if N % 256 and N % 8 == 0 and x.shape[0] * N >= 9 << 20 and x.shape[1] >= 1024 and _gemm64_fwd_takes(x, w, b):
+    """``x @ w^T (+ b)`` for layers whose outputs fill no whole tiles of 256: the in-house kernel where the library's products lose to it (:func:`odd_pays`), else the
+    library's."""
+    if odd_pays(x.shape[0], w.shape[0], x.shape[1]) and _gemm64_fwd_takes(x, w, b):
         return native().gemm64_fwd(x, w, b)
     return torch.nn.functional.linear(x, w, b)
+
+
+@functools.lru_cache(maxsize=4096)
+def odd_pays(T: int, N: int, K: int) -> bool:
+    """Rule of :func:`odd_linear`: from 9 * 2^20 outputs on, unless the tiles of 256 x 256 leave the second round of 256, or with a long K the only one, short.  us, library / here: K 2048
+    3379 x 4240 64.5 / 49.2, 3379 x 9248 132 / 114, 4090 x 12008 201 / 145, 2911 x 8256 93 / 87; K 1024 2911 x 4240 42 / 28; below: 1331 x 4240 29 / 39, 1800 x 5152 44 / 42; 1.2
+    to 1.5 rounds: K 1024 6000 x 3208 50.8 / 55.5, K 3072 1800 x 10504 105 / 114, K 2048 1800 x 12008 86 / 92, 3379 x 6200 83 / 88; less than one: K 4096 1000 x 10504 78 / 85, 1331 x 8256 79 / 87.  (Outputs in
+    whole tiles: 3379 x 6144 73 / 86, 3379 x 8192 88 / 95.)"""
+    tiles = -(-T // 256) * -(-N // 256)
+    return N % 256 != 0 and N % 8 == 0 and K >= 1024 and T * N >= 9 << 20 and not 307 < tiles < 384 and not (tiles < 200 and K >= 4096)
+
+
+@functools.lru_cache(maxsize=4096)
+def ragged_swiglu_pays(T: int, F: int) -> bool:
+    """Does the gated kernel take a projection to 2 F outputs of a number of tokens that is no multiple of 256?  From 11 * 2^20 entries on, unless a third of its tile rows is
+    empty or its tiles of 256 x 128 pairs make about one and a half rounds of 256.  us, library and SwiGLU pass / here: 4096 -> 2 x 11008 500 tokens 93 / 85, 700 144 /
+    118, 1331 308 / 210, 2911 503 / 394, 4095 680 / 528; 4096 -> 2 x 8192 700 86 / 84, 2911 296 / 288, but 1331 160 / 181, 1500 168 / 177; 2048 -> 2 x 4096 1500 50 / 46, but 1023 40 /
+    43; 8192 -> 2 x 28672 300 312 / 347."""
+    rows = -(-T // 256)
+    return F % 128 == 0 and 2 * T * F >= 11 << 20 and 3 * T >= 2 * 256 * rows and not 346 <= rows * (F // 128) <= 410
 
 
 def up_swiglu(x, w, b=None):
     """``silu(gate) * up`` of the gate/up projection ``x @ w^T (+ b)`` (w = [W_gate; W_up]).
     Serving prefill: tokens a multiple of 256 run the gemm64 kernel with the SwiGLU in its
     epilogue (``gemm64_swiglu_fwd``: gate and matching up rows in one output tile, only the
-    [T, F] activation stored — no gu tensor, no SwiGLU pass), and so do other numbers of tokens from 11 * 2^20 entries of the projection on (us,
-    library and SwiGLU pass / here: 4096 -> 2 x 11008 500 tokens 93 / 85, 700 144 / 118, 1331 308 / 210, 2911 503 / 394, 4095 680 / 528; 4096 -> 2 x 8192 700
-    86 / 84, 1331 159 / 172, 2911 296 / 288; 2048 -> 2 x 4096 1500 50 / 46, but 1023 40 / 43).  Knob ``prefill_swiglu`` off disables (A/B)."""
+    [T, F] activation stored — no gu tensor, no SwiGLU pass), and so do other numbers of tokens where that pays (:func:`ragged_swiglu_pays`).  Knob ``prefill_swiglu``
+    off disables (A/B)."""
     x2 = x.reshape(-1, x.shape[-1])
     T, F = x2.shape[0], w.shape[0] // 2
     if (b is None and knobs().prefill_swiglu and use_native(x) and T % 256 == 0
@@ -780,7 +796,7 @@ def up_swiglu(x, w, b=None):
 
         act = native().gemm64_swiglu_fwd(x2, w, gemm64_config("fwd", T, 2 * F, x2.shape[1]) % 1000)
         return act.view(*x.shape[:-1], F)
-    if b is None and knobs().prefill_swiglu and F % 128 == 0 and w.shape[0] % 2 == 0 and T * w.shape[0] >= 11 << 20 and _gemm64_fwd_takes(x2, w):
+    if b is None and knobs().prefill_swiglu and w.shape[0] % 2 == 0 and ragged_swiglu_pays(T, F) and _gemm64_fwd_takes(x2, w):
         return native().gemm64_fwd(x2, w, None, True).view(*x.shape[:-1], F)
     from llmctl.exec.linear import forward_linear
 

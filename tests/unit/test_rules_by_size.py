@@ -32,3 +32,15 @@ def test_forms_of_a_few_rows(M, N, K, form):
                                         (17, 4096, 16384, True), (4, 4096, 16384, True), (33, 2048, 2048, False), (16, 4100, 2048, False)])
 def test_partial_sums(M, N, K, pays):
     assert H.parts_pay(M, N, K) == pays
+
+
+@pytest.mark.parametrize("T,N,K,pays", [(2300, 4240, 2048, True), (2300, 4240, 4096, False), (1331, 8256, 4096, False), (1331, 8256, 2048, True), (1800, 10504, 3072, False), (3379, 6200, 2048, False),
+                                        (4090, 12008, 2048, True), (1331, 4240, 2048, False), (3379, 6144, 2048, False), (3379, 4240, 1000, False)])
+def test_odd_products(T, N, K, pays):
+    assert F.odd_pays(T, N, K) == pays
+
+
+@pytest.mark.parametrize("T,F_,pays", [(1331, 11008, True), (1331, 8192, False), (2911, 8192, True), (300, 28672, False), (500, 11008, False), (700, 11008, True), (1500, 4096, True), (1023, 4096, False),
+                                       (1331, 8200, False)])
+def test_gated_products(T, F_, pays):
+    assert F.ragged_swiglu_pays(T, F_) == pays
