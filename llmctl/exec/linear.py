@@ -205,11 +205,17 @@ def _gemm_ex_ok(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> bool:
 
 def _wgrad_whole(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor) -> bool:
     """Whether a weight whose rows are no multiple of 256 (a vocabulary) has its gradient made by gemm64 all the same: whole tiles, and a tile of their own for the
-    rows behind them.  us, library / so: 8192 tokens 50304 x 768 642 / 499, 8320 x 1024 173 / 134, 32136 x 4096 1935 / 1590, 4096 tokens 50304 x 768 345 / 272;
-    2048 tokens 182 / 176 (added to what is there 190 / 204), 1024 107 / 107, 512 64 / 72; 8192 tokens 5000 x 768 87 / 90."""
+    rows behind them (``_whole_pays``)."""
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
-    return (M % 256 != 0 and M % 8 == 0 and M >= 8192 and K >= 3072 and _gemm64_ok(M // 256 * 256, N, K, g, dy2, x2) and K * dy2.stride(0) * 2 < 2**31
+    return (M % 256 != 0 and M % 8 == 0 and _whole_pays(M, N, K) and _gemm64_ok(M // 256 * 256, N, K, g, dy2, x2) and K * dy2.stride(0) * 2 < 2**31
             and K * x2.stride(0) * 2 < 2**31)
+
+
+def _whole_pays(M: int, N: int, K: int) -> bool:
+    """The second product and its copies are 16 us and more, so products from about 100 us on.  us, library / so: 8192 tokens 50304 x 768 642 / 499, 32136 x 4096 1935 / 1590; 3072
+    tokens 50304 x 768 268 / 220, x 512 190 / 160, 8200 x 2048 127 / 102, but 12008 x 512 53 / 59, 32136 x 256 60 / 66, 32136 x 768 153 / 160; 6144 tokens 8200 x 768 91 / 102, 50304 x 256
+    198 / 166; 2048 tokens 50304 x 768 204 / 204, 1024 107 / 107; 8192 tokens 5000 x 768 87 / 90, 40008 x 256 183 / 222."""
+    return M >= 8192 and K >= 3072 and M * N * K >= (65e9 if M >= 40000 or N >= 2048 else 90e9) and (N >= 512 or M >= 49152)
 
 
 def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool) -> None:
@@ -245,11 +251,12 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
         from llmctl.ops._lib import native
 
         whole = M // 256 * 256
-        native().gemm64_ex(dy2[:, :whole], x2, g[:whole], True, True, accumulate, gemm64_config("wgrad", whole, N, K))
         last = torch.empty(256, N, dtype=torch.float32, device=g.device)  # a tile that ends at the last row
-        native().gemm64_ex(dy2[:, M - 256:], x2, last, True, True, False, gemm64_config("wgrad", 256, N, K))
-        rest = last[256 - (M - whole):]
-        g[whole:].add_(rest) if accumulate else g[whole:].copy_(rest)
+        if accumulate:  # (the library's add of fp32 rows to bf16 ones takes 47 us, the two copies 3 each)
+            last.copy_(g[M - 256:])
+        native().gemm64_ex(dy2[:, :whole], x2, g[:whole], True, True, accumulate, gemm64_config("wgrad", whole, N, K))
+        native().gemm64_ex(dy2[:, M - 256:], x2, last, True, True, accumulate, gemm64_config("wgrad", 256, N, K))
+        g[whole:].copy_(last[256 - (M - whole):])
     elif accumulate:
         g.addmm_(dy2.t(), x2)
     else:

@@ -103,10 +103,13 @@ def test_linear_backward_with_sinks(tokens, out, inn):
 
 @pytest.mark.parametrize("M,N,tokens", [(8200, 256, 3072), (8440, 512, 3200), (8320, 256, 3072)])
 @pytest.mark.parametrize("f32", [False, True])
-def test_weight_gradient_of_a_vocabulary(M, N, tokens, f32):
+def test_weight_gradient_of_a_vocabulary(M, N, tokens, f32, monkeypatch):
     """Rows that fill no whole tile: both parts of the gradient, stored and added to."""
+    import importlib
+
     from llmctl.exec.linear import _wgrad_whole, wgrad_into
 
+    monkeypatch.setattr(importlib.import_module("llmctl.exec.linear"), "_whole_pays", lambda *a: True)  # (the rule takes larger ones)
     dy, x = _operands(True, M, N, tokens, 0)
     g = torch.full((M, N), float("nan"), device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
     assert f32 or _wgrad_whole(g, dy, x)
@@ -118,6 +121,25 @@ def test_weight_gradient_of_a_vocabulary(M, N, tokens, f32):
     assert bool(((first - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
     wgrad_into(g, dy, x, True)
     assert bool(((g.double() - first - ref).abs() <= bound + 2.0**-7 * (ref.abs() + first.abs() + bound)).all())
+
+
+def test_adding_a_vocabularys_gradient_stays_off_mixed_adds():
+    """Rows behind the whole tiles are added in fp32 by the product itself, not by an elementwise add of two types."""
+    from torch.profiler import ProfilerActivity, profile
+
+    from llmctl.exec.linear import _wgrad_whole, wgrad_into
+
+    M, N, tokens = 8200, 2048, 4096
+    dy, x = _operands(True, M, N, tokens, 0)
+    g = torch.randn(M, N, device="cuda").bfloat16()
+    assert _wgrad_whole(g, dy, x)
+    before = g.double()
+    with profile(activities=[ProfilerActivity.CPU]) as prof:
+        wgrad_into(g, dy, x, True)
+    assert "aten::add_" not in {e.key for e in prof.key_averages()}
+    A, B = dy.t().double(), x.double()
+    ref, bound = A @ B, _bound(A, B, tokens, 16)
+    assert bool(((g.double() - before - ref).abs() <= bound + 2.0**-8 * (ref.abs() + before.abs() + bound)).all())
 
 
 @pytest.mark.parametrize("K,S", [(257, 1), (300, 1), (319, 1), (383, 1), (385, 2), (513, 2), (640, 2), (1000, 3), (3912, 4), (8191, 12)])

@@ -1,4 +1,6 @@
 """Rules by size: the forms that measuring found faster, on both sides of the lines."""
+import importlib
+
 import pytest
 
 from llmctl.ops import functional as F
@@ -44,3 +46,9 @@ def test_odd_products(T, N, K, pays):
                                        (1331, 8200, False)])
 def test_gated_products(T, F_, pays):
     assert F.ragged_swiglu_pays(T, F_) == pays
+
+
+@pytest.mark.parametrize("M,N,K,pays", [(50304, 768, 8192, True), (50304, 512, 3072, True), (50304, 768, 2048, False), (50304, 256, 6144, True), (40008, 256, 8192, False), (12008, 512, 3072, False),
+                                        (32136, 768, 3072, False), (8200, 2048, 4096, True), (8200, 768, 6144, False), (5000, 4096, 16384, False)])
+def test_weight_gradients_of_a_vocabulary(M, N, K, pays):
+    assert importlib.import_module("llmctl.exec.linear")._whole_pays(M, N, K) == pays
