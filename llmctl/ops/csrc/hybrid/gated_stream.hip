@@ -117,9 +117,9 @@ __global__ __launch_bounds__(NT) void gated_norm_add_norm_quads_kernel(float* __
   if constexpr (ROUTE) route.row<NW, VQ>(g, row, W);
 }
 
-// A thread's first KEEP columns are all asked for before the first is used (one after another 16 rows of 2048 took 9.7 us, so 4.9; 2911 rows 24.9 and
-// 18.3).  The columns stay with their threads, and so the order of the sum, on which near ties of the first layer's experts hang.
-template <typename T>
+// A thread's first COLS columns are all asked for before the first is used (one after another 16 rows of 2048 took 9.7 us, so 4.9; 2911 rows 24.9 and
+// 18.3; four for rows of up to 1024: 2048 rows of 768 5.6 us with eight, so 5.2).  The columns stay with their threads, and so the order of the sum, on which near ties of the first layer's experts hang.
+template <typename T, int COLS>
 __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pos,
                                                            const T* __restrict__ table, const T* __restrict__ ptable, const float* __restrict__ w,
                                                            float* __restrict__ x, T* __restrict__ h, int W, float eps) {
@@ -127,9 +127,9 @@ __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __rest
   const int64_t row = blockIdx.x;
   const T* e = table + ids[row] * (int64_t)W;
   const T* p = ptable + (int64_t)pos[row] * W;
-  float v[KEEP], pv[KEEP], wv[KEEP];
+  float v[COLS], pv[COLS], wv[COLS];
 #pragma unroll
-  for (int i = 0; i < KEEP; ++i) {
+  for (int i = 0; i < COLS; ++i) {
     const int c = min((int)(threadIdx.x + i * NT), W - 1);
     v[i] = ldf(e + c);
     pv[i] = ldf(p + c);
@@ -137,25 +137,25 @@ __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __rest
   }
   float q = 0.f;
 #pragma unroll
-  for (int i = 0; i < KEEP; ++i) {
+  for (int i = 0; i < COLS; ++i) {
     const int c = threadIdx.x + i * NT;
     if (c >= W) break;
     v[i] += pv[i];
     x[row * W + c] = v[i];
     q += v[i] * v[i];
   }
-  for (int c = threadIdx.x + KEEP * NT; c < W; c += NT) {
+  for (int c = threadIdx.x + COLS * NT; c < W; c += NT) {
     const float u = ldf(e + c) + ldf(p + c);
     x[row * W + c] = u;
     q += u * u;
   }
   const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
 #pragma unroll
-  for (int i = 0; i < KEEP; ++i) {
+  for (int i = 0; i < COLS; ++i) {
     const int c = threadIdx.x + i * NT;
     if (c < W) stf(h + row * W + c, v[i] * rstd * wv[i]);
   }
-  for (int c = threadIdx.x + KEEP * NT; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
+  for (int c = threadIdx.x + COLS * NT; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
 }
 
 template <int KIND>
@@ -465,9 +465,12 @@ std::tuple<at::Tensor, at::Tensor> embed_rmsnorm_f32(const at::Tensor& ids, cons
   if (T == 0) return {x, h};
   dispatch_act(table, [&](auto* tag) {
     using Tt = std::remove_pointer_t<decltype(tag)>;
-    embed_rmsnorm_kernel<Tt><<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), (const Tt*)table.data_ptr(),
-                                                                        (const Tt*)pos_table.data_ptr(), w.data_ptr<float>(), x.data_ptr<float>(),
-                                                                        (Tt*)h.data_ptr(), (int)W, (float)eps);
+    auto go = [&](auto kern) {
+      kern<<<dim3((unsigned)T), NT, 0, cur_stream()>>>(ids.data_ptr<int64_t>(), pos.data_ptr<int>(), (const Tt*)table.data_ptr(), (const Tt*)pos_table.data_ptr(),
+                                                       w.data_ptr<float>(), x.data_ptr<float>(), (Tt*)h.data_ptr(), (int)W, (float)eps);
+    };
+    if (W <= 4 * NT) go(embed_rmsnorm_kernel<Tt, 4>);
+    else go(embed_rmsnorm_kernel<Tt, KEEP>);
   });
   return {x, h};
 }

@@ -542,7 +542,8 @@ at::Tensor sigmoid_gate_mul(const at::Tensor& o, const at::Tensor& g) {
     const T *op = (const T*)o.data_ptr(), *gp = (const T*)g.data_ptr();
     const int W = (int)o.size(1), per = (int)(o.size(1) / g.size(1));
     auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    if (W % N == 0 && at16(op) && at16(y.data_ptr()) && (per % N == 0 || (per == 1 && at16(gp) && g.stride(0) % N == 0)))
+    // (up to 2^17 elements a thread each covers the latency better: 16 rows of 4096 1.94 us, in sixteen-byte pieces 2.14)
+    if (n > 1 << 17 && W % N == 0 && at16(op) && at16(y.data_ptr()) && (per % N == 0 || (per == 1 && at16(gp) && g.stride(0) % N == 0)))
       gate_mul_vec_kernel<T><<<dim3((unsigned)((n / N + 255) / 256)), 256, 0, cur_stream()>>>(op, gp, g.stride(0), (T*)y.data_ptr(), o.size(0), W, per);
     else
       gate_mul_kernel<T, T><<<dim3((unsigned)((n + 255) / 256)), 256, 0, cur_stream()>>>(op, gp, g.stride(0), (T*)y.data_ptr(), o.size(0), W, per);

@@ -49,3 +49,11 @@ def test_gates(T, W, per, dtype, off):
     want = (o.double() * torch.sigmoid(gate.double().repeat_interleave(per, 1)))
     # expf, an fp32 division and a product: a few ulp, then one rounding
     assert ((got.double() - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,W,per", [(64, 2048, 1), (65, 2048, 1), (257, 1032, 1), (700, 256, 128), (1400, 96, 8), (1400, 96, 4), (4000, 36, 12), (4500, 30, 1)])
+@pytest.mark.parametrize("off", [0, 2, 8])
+def test_gates_of_many_rows(T, W, per, dtype, off):
+    """Sixteen bytes a thread, past 2^17 elements."""
+    test_gates(T, W, per, dtype, off)
