@@ -715,6 +715,7 @@ __device__ __forceinline__ void g2p_fence(f32x4_t (&acc)[8][8]) {
 template <int EPI, bool RS = false, bool RAG = false>
 __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)[8][8], int tm, int tn, int wr, int wc,
                                              int lane, int sp, int u, const float* rsl = nullptr) {
+  static_assert(!RAG || (!RS && (EPI == EPI_STORE || EPI == EPI_SWIGLU_FWD)), "rows and columns past the end: plain and gated stores alone");
   constexpr bool PAIRED_B = EPI == EPI_UP_SWIGLU || EPI == EPI_SWIGLU_FWD;
   const int g = lane >> 4, i16 = lane & 15;
   // RS: the lane's row 16 i + i16 of the wave's 128 is scaled by rs[row], read per row block from
@@ -885,8 +886,7 @@ __device__ __forceinline__ void g4w_epilogue(const G64Args& args, f32x4_t (&acc)
     auto in = [&](int jp) __attribute__((always_inline)) { return !RAG || (row_in && tn * TN + wc * 128 + cs + 32 * jp < args.N); };
     if constexpr (EPI == EPI_ACC) {
 #pragma unroll
-      for (int jp = 0; jp < 4; ++jp)
-        old[jp] = in(jp) ? *reinterpret_cast<const uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp) : make_uint4(0, 0, 0, 0);
+      for (int jp = 0; jp < 4; ++jp) old[jp] = *reinterpret_cast<const uint4*>(Cb + (long)(16 * i) * args.ldc + 32 * jp);
     }
 #pragma unroll
     for (int jp = 0; jp < 4; ++jp) {
@@ -1425,7 +1425,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   auto rs_issue = [&]() __attribute__((always_inline)) {
     if constexpr (RS) {
       if (wave == 0)
-        bdma16(RAG ? make_rsrc_n(args.rs + (long)c_tm * TM, (unsigned)(min(args.M - c_tm * TM, TM) * 4)) : make_rsrc(args.rs + (long)c_tm * TM), (unsigned)(tid & 63) * 16u, 0u,
+        bdma16(make_rsrc(args.rs + (long)c_tm * TM), (unsigned)(tid & 63) * 16u, 0u,
                lds_addr(smem) + 2 * BUF + (it & 1) * 1024);
     }
   };

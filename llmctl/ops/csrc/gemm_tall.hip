@@ -385,7 +385,7 @@ int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int split
 }
 
 // out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N of 128 and, not where at, K of 128; two pairs of
-// K-tiles, 256 of K, to a split.
+// K-tiles to a split, 256 of K, of which the last one of a transposed A has more than 128.
 // bias [M] (+)= the row sums of A, of out's type (at, N >= 512).
 void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias,
                bool bias_add) {
@@ -395,9 +395,8 @@ void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at
                "gemm_tall: bf16 operands, bf16 or fp32 out");
   const long M = at_ ? a.size(1) : a.size(0), K = at_ ? a.size(0) : a.size(1), N = b.size(1);
   LLMCTL_CHECK(b.size(0) == K && out.size(0) == M && out.size(1) == N, "gemm_tall: shapes");
-  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && (at_ || K % (2 * TK) == 0) && splits >= 1 && K > 4 * TK * splits - 2 * TK &&
-                   (K + 2 * TK - 1) / (2 * TK) >= 2 * splits,
-               "gemm_tall: M in 256s, N (and K, but for a transposed A) in 128s, at least 256 of K to a split");
+  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && (at_ || K % (2 * TK) == 0) && splits >= 1 && (K + 2 * TK - 1) / (2 * TK) >= 2 * splits,
+               "gemm_tall: M in 256s, N (and K, but for a transposed A) in 128s, two pairs of K-tiles of 64 to a split, the last of them part full at most");
   LLMCTL_CHECK(!at_ || K % (2 * TK) == 0 || (a.stride(0) >= M && b.stride(0) >= N), "gemm_tall: rows that do not overlap");
   auto rows16 = [](const at::Tensor& t, int per) {
     return t.stride(1) == 1 && t.stride(0) % per == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;

@@ -3,13 +3,13 @@
 // The bound is the weight stream and, below some 20 MB of weights, the latency of one round trip to HBM plus the launch
 // (3.5 us in a graph).  Measured beside the library's product (one MI355X, weights from HBM, 16 rows, us):
 //   N x K        768 x 768  768 x 3072  2048 x 2048  2048 x 4096  4240 x 2048  8256 x 2048  9248 x 2048  10496 x 2048  32000 x 2048
-//   library          5.2         9.1        11.0         14.8         12.1         13.9         15.9         15.0          35
-//   whole tiles      4.0         7.7         6.5         10.0         10.5         15.0         15.5         15.0          29
-//   here             3.9         6.6         6.1          9.0          7.8         10.8         11.6         12.6          29
+//   library          5.1         9.3         8.4         14.8         12.2         14.2         14.5         15.1          34
+//   whole tiles      4.1         8.0         6.3         10.2         10.4         15.0         15.5         16.0          29
+//   here             4.0         6.7         5.8          9.1          7.9         11.1         11.8         12.7          30
 // A workgroup owns whole outputs (no partial sums between workgroups) and draws some 30 GB/s, so all 256 CUs must have the same number of them:
 // it owns N / 256 outputs (or an even part, see launch), whatever that is, and the MFMA tiles' other rows repeat its last one (``whole tiles``:
 // 16 or 32 outputs each, which left CUs idle below 4096 outputs and made two uneven rounds above 8192).  With K beyond 4096 a
-// workgroup's own read of x weighs as much as its weights: 2048 x 8192 takes 15 us against the library's 13.6, which splits K over the
+// workgroup's own read of x weighs as much as its weights: 2048 x 8192 takes 16 us against the library's 13.7, which splits K over the
 // chip.  The callers' rules (llmctl/ops/functional.py: stream_pays, decode_form) leave such shapes.
 #pragma once
 
