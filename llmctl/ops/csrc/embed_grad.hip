@@ -8,7 +8,8 @@
 // so a token that fills half the batch is summed by as many waves as any other half.
 // Measured on one MI355X, us, against the library's (sort, segments, scatter into a dense gradient that is then added), ids drawn evenly / all the same:
 // 8192 x 768 into 50304 rows 29.4 / 109 (141 / 329), 8192 x 4096 into 32000 49.7 / 200 (468 / 555), 24576 x 4096 230 / 434 (947 / 1179), 65536 x 4096
-// 1011 / 1939 (1495 / 3232), 256 x 64 into 256 12.5 / 12.5 (18.5 / 26).  16 tokens a wave: 40.8, 75, 283, 1091, 17.3, and less only where most tokens are the
+// 1011 / 1939 (1495 / 3232), 256 x 64 into 256 12.5 / 12.5 (18.5 / 26); ids drawn as 1 / rank, 8192 x 768 into 50304 47 (152),
+// 8192 x 4096 into 32000 103 (451).  16 tokens a wave: 40.8, 75, 283, 1091, 17.3, and less only where most tokens are the
 // same (72, 104, 406, 1538, 16): a wave adds to the rows of its ids one after the other.
 #include "common.h"
 

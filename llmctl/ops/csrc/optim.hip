@@ -111,8 +111,8 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const T* __restrict__ x, lon
 
 // The end of the clip norm, one thread: norm = sqrt(nsq) / divisor, the factor min(1, max_norm / (norm + 1e-6)) / divisor (1 / divisor
 // without clipping), NaN where the norm is not finite, and the count of such steps.  As tensor operations these were 16 launches of one
-// element each between the norm and the update that waits for it: a step of the 2-layer test model, whose host time is the
-// bound, 1772 -> 1608 us.  Same operations in the same order, so the same bits (a division by the divisor is a product with its
+// element each between the norm and the update that waits for it, 79 us of host time and 26 in a captured graph; this kernel 8 and
+// 4.6.  Same operations in the same order, so the same bits (a division by the divisor is a product with its
 // rounded reciprocal there too).
 __global__ void clip_scale_kernel(const float* __restrict__ nsq, const int* __restrict__ skipped, float inv_div, float max_norm,
                                   float* __restrict__ norm, float* __restrict__ coef, int* __restrict__ skipped_out) {

@@ -34,7 +34,9 @@ def layernorm_f32(x, w, b, eps: float, out_dtype):
     return ref.layernorm_f32(x, w, b, eps, out_dtype)
 
 
-ROUTED_ROWS = 64  # steps of at most so many rows are routed by the kernels that norm them: a row reads all of the router's weight
+ROUTED_ROWS = 64  # steps of at most so many rows are routed by the kernels that norm them: a row reads all of the router's weight.
+# 64 rows of width 2048, the norm and a routing launch against one kernel, us: 8 experts 13 / 6.6, 32 23 / 11, 128 63 / 28; of 126 sizes (4 to 128
+# experts, width 1024 to 4096, 1 to 64 rows) none is slower in one.
 
 
 def embed_layernorm_f32(ids, table, scale: float, w, b, eps: float):
