@@ -50,6 +50,7 @@ class PerfKnobs:
     fused_rope_attn: bool = True   # RoPE folded into the attention kernels' Q/K loads
     moe_pad: bool = True           # MoE expert rows padded to multiples of 256 (gemm64 expert GEMMs)
     overlap_optimizer: bool = False  # ZeRO-0: per-bucket AdamW under the backward (measured neutral)
+    step_graph: bool = True        # small steps: forward and backward replayed from one HIP graph (llmctl/runtime/step_graph.py)
     gemm_tuning: bool = True       # hipBLASLt TunableOp solutions (configs/gemm_tuning/*.csv)
     # ---- attention kernels (native: flash_attn_fwd.hip / flash_attn_bwd.hip)
     fa_split: int = -1             # forward causal K/V split: -1 auto, 0 off, 1 on

@@ -28,6 +28,7 @@ from llmctl.parallel.groups import ProcessGroups, build_process_groups
 from llmctl.runtime.faults import FaultInjector
 from llmctl.runtime.flat import FlatParameters
 from llmctl.runtime.optimizer import FlatAdamW, LRSchedule
+from llmctl.runtime.step_graph import StepGraphs
 from llmctl.utils.env import dist_env
 from llmctl.utils.seed import set_seed
 
@@ -137,6 +138,7 @@ class TrainingEngine:
         self.epoch = 0
         self.consumed_samples = 0
         self.metrics_hooks: List = []
+        self.step_graphs = StepGraphs()
         self._build()
         self.faults = FaultInjector(self.rank, c.output_dir)
 
@@ -407,7 +409,9 @@ class TrainingEngine:
 
         use(self.knobs)
         self.model.train()
-        c = self.config
+        loss = self.step_graphs.run(self, batches)
+        if loss is not None:
+            return self._apply(batches, loss)
         # with the side-stream update the previous step may still be reading the gradients:
         # zero them only once the first forward has waited for every bucket (its pre-hooks)
         late_zero = self.optimizer.overlap_update
@@ -449,6 +453,17 @@ class TrainingEngine:
             self.esync.finish()
         if self.pipeline is not None:
             self.pipeline.sync_tied_grads()
+        return self._apply(batches, loss)
+
+    def _gradients(self, x, y, denom: float) -> torch.Tensor:
+        """What a step of one micro-batch on one GPU does before the optimizer (``step_graph`` records it)."""
+        self.flat.zero_grad()
+        loss = self._forward_backward(x, y, denom)
+        self.sync.finish()
+        return loss
+
+    def _apply(self, batches, loss) -> Dict[str, torch.Tensor]:
+        """The optimizer's part of ``train_step``."""
         lr = self.scheduler(self.global_step)  # 0-based index of the step being applied (HF)
         self.global_step += 1
         if self.eopt is not None:

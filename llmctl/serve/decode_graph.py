@@ -145,6 +145,11 @@ class GraphTable:
     def __len__(self) -> int:
         return self._graphs
 
+    def due(self, shape: Tuple[int, int]) -> bool:
+        """Whether the next step of ``shape`` may be replayed or recorded."""
+        e = self._shapes.get(shape, 0)
+        return e is not None and (not isinstance(e, int) or e >= WARM_STEPS)
+
     def step(self, shape: Tuple[int, int], record: Callable[[Tuple[int, int]], Optional[DecodeGraph]]) -> Optional[DecodeGraph]:
         """The graph that runs the next step of ``shape``; None: it runs eagerly.  ``record(shape)``: its graph, or None where it
         cannot be recorded."""

@@ -1,0 +1,89 @@
+"""Replayed training steps (``llmctl.runtime.step_graph``) against eager ones, and the steps that must not be replayed."""
+
+import dataclasses
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def engine(model="tiny", layers=2, knob=True, tokens=(2, 128), **kw):
+    from llmctl.models import get_model_config
+    from llmctl.runtime.engine import TrainingConfig, TrainingEngine
+
+    cfg = dataclasses.replace(get_model_config(model), layers=layers)
+    return TrainingEngine(TrainingConfig(model_name_or_path=model, batch_size=tokens[0], seq_len=tokens[1], device="cuda", log_level="warning",
+                                         learning_rate=1e-3, max_steps=50, seed=3, perf_knobs={"step_graph": knob}, **kw), cfg)
+
+
+def batch(eng, g, b, s):
+    t = torch.randint(0, eng.model_config.vocab_size, (b, s + 1), generator=g).to("cuda")
+    return t[:, :-1], t[:, 1:]  # (rows of another tensor, as a loader's are)
+
+
+@pytest.mark.parametrize("model,layers,sizes", [("tiny", 2, [(2, 128)]), ("tiny", 2, [(1, 65), (3, 100), (8, 512)]), ("gpt2-125m", 2, [(2, 64), (1, 333)])])
+def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes):
+    """Losses, norms, gradients and states over many steps of alternating shapes, other work on the device between them.  Both sides run the same
+    kernels; what differs from run to run is the order of the clip norm's atomics (and a library product's partial sums), which moves the weights by
+    rounding: the bound is four times the spread of two eager runs, or rounding of bf16 weights (2^-9) where they happen to agree."""
+    def run(knob):
+        eng, g, out = engine(model, layers, knob), torch.Generator().manual_seed(1), []
+        for step in range(5):
+            for b, s in sizes:
+                r = eng.train_step([batch(eng, g, b, s)])
+                keep = torch.full((1 << 20,), float(step), device="cuda")  # memory that a stale pointer would hit
+                out += [r["loss"], r["grad_norm"], keep.sum() * 0]
+        torch.cuda.synchronize()
+        assert len(eng.step_graphs.table) == (len(sizes) if knob else 0)
+        return torch.stack([o.float().reshape(()) for o in out]), eng.flat.grad.float(), eng.optimizer.master, eng.optimizer.exp_avg
+
+    a, b, c = run(True), run(False), run(False)
+    for x, y, z in zip(a, b, c):
+        assert torch.isfinite(x).all()
+        assert (x - y).norm() <= max(4 * (y - z).norm().item(), 2.0 ** -9 * y.norm().item())
+
+
+def test_what_listens_is_heard(native_lib):
+    """Hooks, modes and faults see every step; parameters that change storage or stop training are not replayed into."""
+    eng, g = engine(), torch.Generator().manual_seed(2)
+    step = lambda: eng.train_step([batch(eng, g, 2, 128)])  # noqa: E731
+    for _ in range(4):  # (the first one builds the rotary tables)
+        step()
+    assert len(eng.step_graphs.table) == 1
+    seen = []
+    h = eng.model.layers[0].register_forward_hook(lambda *a: seen.append(1))
+    step(), step()
+    assert len(seen) == 2
+    h.remove()
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t, lambda t: t):
+        step()
+    assert packed
+    p = eng.model.layers[0].wo
+    p.requires_grad_(False)
+    for _ in range(4):
+        step()
+    assert float(p.grad.abs().max()) == 0  # not trained, whatever was recorded before
+    p.requires_grad_(True)
+    w = eng.model.layers[1].attn_norm_w
+    before = eng.flat.grad.clone()
+    with torch.no_grad():
+        w.data = torch.zeros_like(w)  # another storage: the model reads this one
+    for _ in range(4):
+        step()
+    wq = eng.model.layers[1].wqkv
+    assert float(wq.grad.abs().max()) == 0 and not torch.equal(before, eng.flat.grad)
+    p.grad = None
+    step()
+    assert p.grad is not None and p.grad.data_ptr() == eng.flat.grad.data_ptr() + 2 * eng.flat.offsets[id(p)]
+
+
+def test_long_steps_stay_eager(native_lib):
+    from llmctl.runtime.step_graph import pays
+
+    assert pays(3_000_000, 256, 2) and pays(124_000_000, 1024, 12) and not pays(124_000_000, 8192, 12) and not pays(6_700_000_000, 64, 32)
+    eng, g = engine("gpt2-125m", 1), torch.Generator().manual_seed(3)
+    for _ in range(4):
+        eng.train_step([batch(eng, g, 8, 1024)])
+    assert len(eng.step_graphs.table) == 0
