@@ -64,6 +64,7 @@ class PerfKnobs:
     cp_zigzag: bool = True         # load-balanced (zig-zag) causal ring attention
     # ---- serving (llmctl/serve, llmctl/ops/functional.py; native: paged_attn.hip, skinny_gemm.hip)
     decode_fused: bool = True      # decode projections with fused epilogues
+    decode_layers: bool = True     # a few rows of a small GPT-2 style model: all layers of a step in one launch
     decode_splits: int = 0         # paged-attention context splits (0: auto)
     decode_v3: int = 1             # skinny decode GEMM v3 schedule
     skinny_gemm: str = "auto"      # decode-size GEMMs: auto (weight stream, skinny kernel or library by size) | all (skinny) | off

@@ -18,7 +18,7 @@ from .functional import (
     decode_fused_ok,
     decode_linear,
     decode_linear_fp8,
-    decode_linear_add_rmsnorm,
+    decode_layers, decode_layers_ok, decode_layers_workspace, decode_linear_add_rmsnorm,
     decode_norm_linear,
     decode_norm_qkv_cache,
     decode_qkv_rope_cache,

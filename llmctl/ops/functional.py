@@ -696,6 +696,29 @@ def decode_norm_qkv_cache(x, res, nw, nb, eps: float, w, b, nq: int, nkv: int, k
     return qkv_split_cache(decode_linear(xn, w, b), nq, nkv, k_cache, v_cache, slots)[0], r
 
 
+def decode_layers_ok(hidden: int, heads: int, kv_heads: int, ffn: int, layers: int, rows: int, cache) -> bool:
+    """Does ``csrc/decode_layers.hip`` run a whole decode step of this size in one launch (LayerNorm, biases, GELU and learned positions are the caller's to
+    know), and does it pay?  Up to four rows, where the launches are most of a step: gpt2-125m, us a step, a launch per product / this: one row at context 129
+    367 / 200, 2000 425 / 251, two rows 382 / 237, four 425 / 332 (a row more costs 45, beside launches 20); four layers of 256, one row 122 / 77, of 1024, four
+    rows 175 / 161."""
+    return (knobs().decode_layers and use_native(cache) and cache.dtype == torch.bfloat16 and cache.is_contiguous() and 1 <= rows <= 4 and 1 <= layers <= 32
+            and hidden % 256 == 0 and 256 <= hidden <= 1024 and heads == kv_heads and heads * 64 == hidden and ffn == 4 * hidden
+            and torch.cuda.get_device_properties(cache.device).multi_processor_count >= 128)
+
+
+def decode_layers_workspace(hidden: int, device) -> torch.Tensor:
+    """The words that a model's steps exchange (``decode_layers``): one per engine, whose steps follow one another."""
+    return torch.zeros(native().decode_layers_words(hidden), dtype=torch.int64, device=device)
+
+
+def decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps: float, workspace, workgroups: int = 128,
+                  gate_us: int = 200):
+    """The final norm's rows of a decode step: embedding, all layers with their paged cache, final norm.  ``weights``: per layer the attention norm (weight,
+    bias), QKV, output projection, MLP norm, up and down (weight and bias each), then the final norm; ``k_cache`` / ``v_cache``: all layers' ``[L, blocks,
+    block, heads, 64]``.  ``workgroups``: fewer than 128 each do the work of several; ``gate_us``: the step begins without those that do not run by then."""
+    return native().decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps, workspace, workgroups, gate_us)
+
+
 def _dequant(w, w_scale, dtype):
     """bf16 image of an fp8 (e4m3fn) weight with fp32 row scales (fallback paths)."""
     return w if w_scale is None else (w.float() * w_scale.float().unsqueeze(1)).to(dtype)
@@ -887,5 +910,5 @@ __all__ = [
     "gelu", "cross_entropy", "adamw_step_", "clip_scale", "embed_rows", "l2norm_sq", "kv_cache_write", "qkv_split_cache", "paged_attention_decode",
     "sample", "decode_linear", "decode_linear_fp8", "decode_fused_ok", "decode_qkv_rope_cache", "decode_up_swiglu", "decode_attention_qkv", "up_swiglu",
     "decode_linear_add_rmsnorm", "rope_qkv_cache", "paged_prefill_attention", "prefill_work_list", "attn_merge_",
-    "rms_rstd", "rowscale_ok", "linear_rowscale", "up_swiglu_rowscale", "linear_acc_",
+    "rms_rstd", "rowscale_ok", "decode_layers_ok", "decode_layers", "decode_layers_workspace", "linear_rowscale", "up_swiglu_rowscale", "linear_acc_",
 ]

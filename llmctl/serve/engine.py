@@ -139,6 +139,7 @@ class InferenceEngine:
         self.rope = self.model.rope_tables(self.max_model_len, self.device)
         # MoE routing sizes the expert segments on the host: decode runs eagerly
         self.use_graphs = use_graphs and self.device.type == "cuda" and not cfg.is_moe
+        self._layers_ws = None  # _step_workspace
         self._graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, Dict[str, torch.Tensor]]] = {}
         # sampling uniforms come from the host (one H2D copy with the step's other inputs), so
         # in-graph sampling and the eager path draw the same stream
@@ -649,9 +650,32 @@ class InferenceEngine:
                 and all(l.attn_norm_b is None and l.mlp_norm_b is None for l in m.layers)
                 and self.knobs.decode_fused)
 
+    def _step_workspace(self, n: int) -> Optional[torch.Tensor]:
+        """The workspace of ``ops.decode_layers`` where the whole step of ``n`` rows runs in one launch."""
+        cfg, m = self.cfg, self.model
+        if not (self.tp == 1 and self.rope is None and m.pos_embed is not None and m.final_norm_b is not None and not cfg.gated_mlp and not cfg.is_moe
+                and all(p is not None and p.dtype == torch.bfloat16 and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in self._step_weights())
+                and ops.decode_layers_ok(cfg.hidden, cfg.heads, cfg.kv_heads, cfg.ffn, len(m.layers), n, self.kv_cache.k)):
+            return None
+        if self._layers_ws is None and not torch.cuda.is_current_stream_capturing():
+            self._layers_ws = ops.decode_layers_workspace(cfg.hidden, self.device)
+        return self._layers_ws
+
+    def _step_weights(self) -> List[torch.Tensor]:
+        m, out = self.model, []
+        for l in m.layers:
+            out += [l.attn_norm_w, l.attn_norm_b, l.wqkv, l.bqkv, l.wo, l.bo, l.mlp_norm_w, l.mlp_norm_b, l.w_up, l.b_up, l.w_down, l.b_down]
+        return out + [m.final_norm_w, m.final_norm_b]
+
     def _decode_body(self, ids, positions, slots, block_tables, ctx_lens) -> torch.Tensor:
         if self._fused_decode():
             return self._decode_body_fused(ids, positions, slots, block_tables, ctx_lens)
+        ws = self._step_workspace(ids.shape[0])
+        if ws is not None:
+            m = self.model
+            xn = ops.decode_layers(ids, positions, slots, block_tables, ctx_lens, m.embed, m.pos_embed, self._step_weights(), self.kv_cache.k,
+                                   self.kv_cache.v, self.cfg.layer_norm_eps, ws)
+            return self._gather_vocab(ops.decode_linear(xn, m.head_weight()))
         x = self._embed(ids, positions)
         res = None
         kc, vc = self.kv_cache.k, self.kv_cache.v
@@ -835,7 +859,7 @@ class InferenceEngine:
             torch.cuda.synchronize(self.device)
         self.kv_cache = None
         self._w8 = self._w8_head = None
-        self._nf = None
+        self._nf = self._layers_ws = None
         self.rope = None
         if self.device.type == "cuda":
             torch.cuda.empty_cache()

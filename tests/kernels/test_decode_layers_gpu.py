@@ -1,0 +1,130 @@
+"""A whole decode step in one launch (``csrc/decode_layers.hip``) against plain torch in float64, and against itself with other numbers of workgroups."""
+
+import math
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+V, BLOCK = 64, 16
+
+
+def make(H, L, ctx, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s, k=1.0: (torch.randn(*s, generator=g) * k).to(torch.bfloat16).cuda()  # noqa: E731
+    B, mb = len(ctx), max(ctx) // BLOCK + 2
+    w = []
+    for _ in range(L):
+        w += [1 + r(H, k=0.1), r(H, k=0.1), r(3 * H, H, k=0.05), r(3 * H, k=0.1), r(H, H, k=0.03), r(H, k=0.1),
+              1 + r(H, k=0.1), r(H, k=0.1), r(4 * H, H, k=0.03), r(4 * H, k=0.1), r(H, 4 * H, k=0.02), r(H, k=0.1)]
+    w += [1 + r(H, k=0.1), r(H, k=0.1)]
+    blocks = B * mb + 1
+    bt = (1 + torch.randperm(B * mb, generator=g)).view(B, mb).int().cuda()
+    k, v = r(L, blocks, BLOCK, H // 64, 64), r(L, blocks, BLOCK, H // 64, 64)
+    pos = torch.tensor([c - 1 for c in ctx], dtype=torch.int32).cuda()
+    slots = torch.tensor([int(bt[b, (c - 1) // BLOCK]) * BLOCK + (c - 1) % BLOCK for b, c in enumerate(ctx)]).cuda()
+    return dict(ids=torch.randint(0, V, (B,), generator=g).cuda(), positions=pos, slots=slots, block_tables=bt,
+                ctx_lens=torch.tensor(ctx, dtype=torch.int32).cuda(), table=r(V, H), pos_table=r(max(ctx), H), weights=w, k_cache=k, v_cache=v, eps=1e-5)
+
+
+def plain(a):
+    """The same in float64, K and V of the step's tokens rounded as the cache holds them; returns (rows, keys, values)."""
+    w, H = [t.double() for t in a["weights"]], a["table"].shape[1]
+    L, heads, ks, vs = (len(w) - 2) // 12, a["table"].shape[1] // 64, [], []
+    x = a["table"].double()[a["ids"]] + a["pos_table"].double()[a["positions"].long()]
+    for l in range(L):
+        n1w, n1b, wqkv, bqkv, wo, bo, n2w, n2b, wu, bu, wd, bd = w[12 * l:12 * l + 12]
+        q, k, v = (F.layer_norm(x, (H,), n1w, n1b, a["eps"]) @ wqkv.t() + bqkv).view(-1, 3, heads, 64).unbind(1)
+        k, v, o = k.bfloat16().double(), v.bfloat16().double(), []
+        ks.append(k), vs.append(v)
+        for b, c in enumerate(a["ctx_lens"].tolist()):
+            rows = (a["block_tables"][b].long()[:, None] * BLOCK + torch.arange(BLOCK, device="cuda")).reshape(-1)[:c - 1]
+            kk = torch.cat([a["k_cache"][l].view(-1, heads, 64)[rows].double(), k[b:b + 1]])
+            vv = torch.cat([a["v_cache"][l].view(-1, heads, 64)[rows].double(), v[b:b + 1]])
+            o.append(torch.einsum("ht,thd->hd", torch.softmax(torch.einsum("hd,thd->ht", q[b], kk) / 8, -1), vv).reshape(-1))
+        x = x + torch.stack(o) @ wo.t() + bo
+        x = x + F.gelu(F.layer_norm(x, (H,), n2w, n2b, a["eps"]) @ wu.t() + bu, approximate="tanh") @ wd.t() + bd
+    return F.layer_norm(x, (H,), w[-2], w[-1], a["eps"]), torch.stack(ks), torch.stack(vs)
+
+
+def run(a, ws, **kw):
+    from llmctl import ops
+
+    b = dict(a, k_cache=a["k_cache"].clone(), v_cache=a["v_cache"].clone())
+    out = ops.decode_layers(b["ids"], b["positions"], b["slots"], b["block_tables"], b["ctx_lens"], b["table"], b["pos_table"], b["weights"], b["k_cache"],
+                            b["v_cache"], b["eps"], ws, **kw)
+    return out, b["k_cache"], b["v_cache"]
+
+
+# one row without a past, spans of 256 keys and one more, several spans' sums, rows of different lengths in groups of two and three, every width
+@pytest.mark.parametrize("H,L,ctx", [(256, 2, [1]), (256, 1, [4001]), (768, 3, [129]), (768, 2, [257]), (768, 2, [258]), (768, 2, [2000, 1]), (512, 2, [17, 600, 1025]),
+                                     (1024, 2, [5, 300, 1, 16]), (256, 2, [513, 512, 2, 33])])
+def test_step_matches_float64(native_lib, H, L, ctx):
+    """Against float64.  What is rounded: K, V, the MLP's activations (bf16, 2^-9 each) and the result (2^-9); every layer's come on top of the former ones'."""
+    from llmctl import ops
+
+    a = make(H, L, ctx)
+    ws = ops.decode_layers_workspace(H, "cuda")
+    want, ks, vs = plain(a)
+    first = None
+    for step in range(3):  # (the workspace carries its count on)
+        out, k, v = run(a, ws)
+        torch.cuda.synchronize()
+        assert (out.double() - want).norm() <= (1 + L) * 2.0 ** -8 * want.norm()
+        rows = a["slots"].long()
+        for got, new, old in ((k, ks, a["k_cache"]), (v, vs, a["v_cache"])):
+            flat = got.view(L, -1, H // 64, 64)
+            assert (flat[:, rows].double() - new).norm() <= L * 2.0 ** -8 * new.norm()
+            keep = torch.ones(flat.shape[1], dtype=torch.bool, device="cuda")
+            keep[rows] = False
+            assert torch.equal(flat[:, keep], old.view(L, -1, H // 64, 64)[:, keep])  # nothing else is written
+        first = first if first is not None else (out, k, v)
+        assert all(torch.equal(x, y) for x, y in zip(first, (out, k, v)))
+
+
+@pytest.mark.parametrize("workgroups,gate_us", [(1, 200), (7, 200), (127, 200), (128, 0), (128, 1)])
+@pytest.mark.parametrize("ctx", [[300], [40, 1, 700]])
+def test_any_number_of_workgroups(native_lib, workgroups, gate_us, ctx):
+    """Shares that go round, and a gate that closes before all are there, give the same bits; so does a graph, replayed beside other work."""
+    from llmctl import ops
+
+    a = make(256, 2, ctx, seed=1)
+    ws = ops.decode_layers_workspace(256, "cuda")
+    want = run(a, ws)
+    for _ in range(4):
+        got = run(a, ws, workgroups=workgroups, gate_us=gate_us)
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(want, got))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        got = run(a, ws, workgroups=workgroups, gate_us=gate_us)
+    for _ in range(4):
+        got[0].zero_()
+        g.replay()
+        assert torch.equal(got[0], want[0])
+        run(a, ws)
+
+
+def test_rows_without_a_slot_are_not_cached(native_lib):
+    from llmctl import ops
+
+    a = make(256, 1, [20, 1], seed=2)
+    a["slots"] = torch.tensor([int(a["slots"][0]), -1], device="cuda")
+    _, k, _ = run(a, ops.decode_layers_workspace(256, "cuda"))
+    assert int((k != a["k_cache"]).any(-1).any(-1).sum()) == 1
+
+
+def test_what_it_does_not_take(native_lib):
+    from llmctl import ops
+
+    cache = torch.zeros(1, 1, 1, 1, 64, dtype=torch.bfloat16, device="cuda")
+    ok = lambda *a, c=cache: ops.decode_layers_ok(*a, c)  # noqa: E731
+    assert ok(768, 12, 12, 3072, 12, 4) and not ok(768, 12, 12, 3072, 12, 5) and not ok(768, 12, 4, 3072, 12, 1) and not ok(768, 6, 6, 3072, 12, 1)
+    assert not ok(1280, 20, 20, 5120, 12, 1) and not ok(768, 12, 12, 2048, 12, 1) and not ok(768, 12, 12, 3072, 33, 1)
+    a = make(256, 1, [3])
+    with pytest.raises(RuntimeError):
+        run(dict(a, weights=a["weights"][:-1]), ops.decode_layers_workspace(256, "cuda"))
+    with pytest.raises(RuntimeError):
+        run(a, ops.decode_layers_workspace(512, "cuda"))
+    assert math.isfinite(float(run(a, ops.decode_layers_workspace(256, "cuda"))[0].float().sum()))
