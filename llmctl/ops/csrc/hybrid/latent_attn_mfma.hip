@@ -13,6 +13,11 @@
 //   * Q fragments stay in registers for the whole key loop; softmax is lane-local (query on the lane),
 //     exp2 domain, deferred rescale; the sink starts the running maximum and the denominator;
 //   * the key loop runs only over the tiles that the rows' windows touch.
+// Bound: at one wave a SIMD (keys wider than 128) the chain of a tile, fill requests, scores, softmax, values; the MFMAs are a fifth of it.  What a tile's chain held beside
+// them, us a layer, 2048 tokens x 16 heads, keys of 192, window 1024 (three layers 206 us, so 143): a block-table entry used right where it was loaded (the wave that looked the
+// slots up waited for HBM in every tile), a slot lookup in LDS per DMA piece, score fragments read just ahead of their MFMAs, a branch per masked element.  The other forms: 16 heads
+// over 4 kv groups, sigmoid weights, five portions of 2911 tokens 126 us, so 76; keys of 128, window 1024, 2048 + 1331 tokens 68.5, so 55.7.  With the blocks of a head on one XCD,
+// whose L2 then holds its keys, alone: 126, so 113.
 // Value columns beyond 256 go to further workgroups (blockIdx.z), which recompute the scores.
 // Shapes it takes: R and rank multiples of 8, R <= 640; anything else runs the generic kernels.
 #include "attn_common.h"
@@ -48,6 +53,7 @@ struct LArgs {
   float cap_log2, cap_inv2;     // CAP forms: x (log2 domain) = cap_log2 * tanh(s * scale); cap_inv2 = 2 log2(e) scale / cap
   // SPLIT forms: the key range of a decode row is spread over blockIdx.x (few sequences would otherwise leave the chip idle): each split
   // writes its unnormalised fp32 output and (running maximum, denominator) here, and row_merge joins them
+  int xcd;  // prompt forms: the heads (a multiple of eight) are shared out to the XCDs
   int nsplit;
   float* ws_o;   // [rows, nsplit, rk]
   float* ws_ml;  // [rows, nsplit, 2]
@@ -61,9 +67,9 @@ struct LArgs {
 // Keys and values up to 128 wide: two workgroups per CU (64.5 KB of images each; held to 256 registers, one's softmax runs beside the
 // other's products).  16 heads over 4 kv groups, portions of 2048 and 1331 tokens: 156 us at one per CU (200 + 96 registers),
 // 100 so.  Wider keys stay at one: 192-wide keys took 108 us against 99, with one set of images instead of two 107.
-template <int NCB, int NDB, bool ROT, bool SIG = false, bool CAP = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
-  constexpr int NKS = NCB * 8;
+template <int NKS, int NDB, bool ROT, bool SIG = false, bool CAP = false, bool SPLIT = false>
+__global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
+  constexpr int NCB = (NKS + 7) / 8;
   constexpr int NTB = (NDB + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // the tile images: one set, or two (the fill of tile t + 1 then runs beside the products of tile t)
@@ -74,16 +80,22 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, hh = lane >> 5;
-  const int n = blockIdx.y;
-  const int hg = blockIdx.z / a.nvt, v0 = (blockIdx.z % a.nvt) * (NDB * 32);
+  // workgroups go round the XCDs in order; the blocks of a head, and the heads of a kv group, read the same keys, so they are dealt to one XCD and its L2
+  unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+  if (!SPLIT && a.xcd) {
+    const unsigned slice = gridDim.x * gridDim.y, l = bx + gridDim.x * by + slice * bz, v = (l & 7) * (gridDim.z / 8 * slice) + (l >> 3);
+    bz = v / slice, by = (v - bz * slice) / gridDim.x, bx = v - bz * slice - by * gridDim.x;
+  }
+  const int n = by;
+  const int hg = bz / a.nvt, v0 = (bz % a.nvt) * (NDB * 32);
   const int P = a.H / a.G;                       // query heads per kv group
   const int grp = hg / a.hpg, hsub = (hg % a.hpg) * a.HB;  // this workgroup's kv group, its first head inside it
   const int q_begin = SPLIT ? n : a.cu[n];
   const int qlen = SPLIT ? 1 : a.cu[n + 1] - q_begin;
   const int HB = a.HB, TB = 128 / HB;
   // prompt portions: the last query blocks of a sequence see the most keys; they are dispatched first
-  const int split = SPLIT ? blockIdx.x : 0;
-  const int tok0 = SPLIT ? 0 : (int)(gridDim.x - 1 - blockIdx.x) * TB;
+  const int split = SPLIT ? bx : 0;
+  const int tok0 = SPLIT ? 0 : (int)(gridDim.x - 1 - bx) * TB;
   if (tok0 >= qlen) return;
   const int ctx = a.ctx[n];
   const int pos0 = ctx - qlen;
@@ -168,35 +180,39 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   // to LDS (no registers, all pieces of the tile in flight at once); the images' swizzles are applied
   // to the source chunk.  Keys past the context and columns past the row read a valid neighbour instead
   // (finite data): such keys are masked below and such columns meet zero Q entries or are never stored.
+  // A wave's rows of an image are 16 apart, so their swizzle is one number and the four slots serve all images.
+  const int frow = wave_u * 4 + (lane >> 4), fch = lane & 15;
+  int fcol[NCB + NTB];
+#pragma unroll
+  for (int img = 0; img < NCB + NTB; ++img) {
+    const int col = img < NCB ? a.koff + (img * 16 + (fch ^ swz_row<128>(frow))) * 8 : ((v0 / 128 + (img - NCB)) * 16 + (fch ^ swz_tr<128>(frow))) * 8;
+    fcol[img] = min(col, a.rs - 8);
+  }
   auto fill = [&](int sbuf, int ibuf) {
-#pragma unroll 4
-    for (int g = wave_u; g < 16 * (NCB + NTB); g += 4) {
-      const int img = g >> 4, rg = g & 15;
-      const int krow = rg * 4 + (lane >> 4), chp = lane & 15;
-      const long slot = slot_lds[sbuf * LKB + krow];
-      int col;
-      if (img < NCB) {
-        col = a.koff + (img * 16 + (chp ^ swz_row<128>(krow))) * 8;
-      } else {
-        col = ((v0 / 128 + (img - NCB)) * 16 + (chp ^ swz_tr<128>(krow))) * 8;
-      }
-      col = min(col, a.rs - 8);
-      dma16(a.cache + (slot * a.G + grp) * a.rs + col, lds_base + (unsigned)(ibuf * BUFB + img * LIMG + rg * 1024));
+    int slot[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) slot[j] = slot_lds[sbuf * LKB + 16 * j + frow];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const unsigned short* base = a.cache + ((long)slot[j] * a.G + grp) * a.rs;
+#pragma unroll
+      for (int img = 0; img < NCB + NTB; ++img) dma16(base + fcol[img], lds_base + (unsigned)(ibuf * BUFB + img * LIMG + (wave_u + 4 * j) * 1024));
     }
   };
   // double-buffered form: the slots of tile t + 2 are requested BEFORE the fill of tile t + 1 is issued and
   // stored to LDS at the top of the next iteration, so that no wave waits on its own fill in between (a
   // wave's memory operations complete in order)
-  auto slot_of = [&](int t) {
+  int pend = 0, pend_in = 0;  // the block, as the table holds it (an operation on it here would wait for it), and the place in the block
+  auto ask_slot = [&](int t) {
     const int key = min(t * LKB + tid, ctx - 1);
-    return btn[key / a.bs] * a.bs + key % a.bs;
+    pend = btn[key / a.bs];
+    pend_in = key % a.bs;
   };
-  int pend = 0;
   if (t_lo < t_hi) load_slots(tile_of(t_lo), 0);
   if constexpr (DB) {
     if (t_lo < t_hi) {
       __syncthreads();
-      if (t_lo + 1 < t_hi && tid < LKB) pend = slot_of(tile_of(t_lo + 1));
+      if (t_lo + 1 < t_hi && tid < LKB) ask_slot(tile_of(t_lo + 1));
       fill(0, 0);
     }
   }
@@ -207,10 +223,10 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
     if constexpr (DB) {
       // tile t was requested one iteration ago.  After the barrier every wave's pieces of it have landed,
       // every wave is done with tile t - 1 (its images may be overwritten) and the slots of t + 1 are visible
-      if (t + 1 < t_hi && tid < LKB) slot_lds[(sbuf ^ 1) * LKB + tid] = pend;
+      if (t + 1 < t_hi && tid < LKB) slot_lds[(sbuf ^ 1) * LKB + tid] = pend * a.bs + pend_in;
       vm_wait<0>();
       __syncthreads();
-      if (t + 2 < t_hi && tid < LKB) pend = slot_of(tile_of(t + 2));
+      if (t + 2 < t_hi && tid < LKB) ask_slot(tile_of(t + 2));
       if (t + 1 < t_hi) fill(sbuf ^ 1, sbuf ^ 1);
     } else {
       __syncthreads();
@@ -224,15 +240,33 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
 
     f32x16 s[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[kb][i] = 0.f;
+    // the next k-steps' fragments are read while the ones before them are multiplied (left to itself the compiler reads each just ahead of its use)
+    constexpr int KST = NKS >= 32 ? 1 : 2;  // (the widest keys have no registers for more)
+    bf16x8_t kf[2][KST][2];
+    auto read_k = [&](int k0, bf16x8_t (&f)[KST][2]) {
 #pragma unroll
-      for (int ks = 0; ks < NKS; ++ks) {
-        const bf16x8_t kf = lds_read_b128(Ks + (ks >> 3) * LIMG + kb * 32 * LROWB, k_row + (k_x ^ (((2 * ks) & 15) << 4)));
-        s[kb] = mfma32(kf, qf[ks], s[kb]);
-      }
+      for (int i = 0; i < KST; ++i)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+          f[i][kb] = lds_read_b128(Ks + ((k0 + i) >> 3) * LIMG + kb * 32 * LROWB, k_row + (k_x ^ (((2 * (k0 + i)) & 15) << 4)));
+    };
+    read_k(0, kf[0]);
+#pragma unroll
+    for (int k0 = 0; k0 < NKS; k0 += KST) {
+      if (k0 + KST < NKS) read_k(k0 + KST, kf[(k0 / KST + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < KST; ++i)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] = mfma32(kf[(k0 / KST) & 1][i][kb], qf[k0 + i], s[kb]);
+      __builtin_amdgcn_sched_barrier(0);
     }
+    auto hidden = [&](int key) {  // (no branches: 32 of them per tile and lane)
+      return !valid | (key > my_pos) | ((key < my_lo) & ((key >= a.keep) | (key < my_c0))) | (key >= ctx);
+    };
     bf16x8_t pb[2][2];
     if constexpr (SIG) {
       // x (log2 domain) = s * scale - a log2(1 + b (i - j)) + bias; weight = 1 / (1 + 2^-x); hidden keys weigh 0
@@ -245,7 +279,7 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
           const float dist = (float)max(my_pos - key, 0);
           const float x = s[kb][i] * my_scale - pen_a * __log2f(1.0f + pen_b * dist) + sig_b2;
           const float w = __builtin_amdgcn_rcpf(1.0f + fast_exp2(-x));
-          p[i] = (!valid || key > my_pos || (key < my_lo && (key >= a.keep || key < my_c0)) || key >= ctx) ? 0.f : w;
+          p[i] = hidden(key) ? 0.f : w;
         }
         pb[kb][0] = to_bf16x8(p);
         pb[kb][1] = to_bf16x8(p + 8);
@@ -273,12 +307,12 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
             if constexpr (CAP) x = a.cap_log2 * (1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + fast_exp2(s[kb][i] * a.cap_inv2)));
             else x = s[kb][i] * my_scale;
             const int key = kv0 + kb * 32 + acc_row(i, hh);
-            if (!valid || key > my_pos || (key < my_lo && (key >= a.keep || key < my_c0)) || key >= ctx) x = -INFINITY;
+            x = hidden(key) ? -INFINITY : x;
             s[kb][i] = x;
             mx = fmaxf(mx, x);
           }
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      mx = xor32_max(mx);
       const bool grow = __builtin_amdgcn_ballot_w64(mx > m_i + kRescaleTh) != 0;
       const float m_raw = grow ? fmaxf(m_i, mx) : m_i;
       const float m_new = m_raw == -INFINITY ? 0.f : m_raw;  // nothing seen yet (a later split, all keys masked)
@@ -294,7 +328,7 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
         pb[kb][0] = to_bf16x8(p);
         pb[kb][1] = to_bf16x8(p + 8);
       }
-      rs += __shfl_xor(rs, 32);
+      rs = xor32_add(rs);
       if (grow) {
         const float alpha = fast_exp2(m_i - m_new);
         l_i *= alpha;
@@ -360,17 +394,18 @@ __global__ __launch_bounds__(256, NCB == 1 && NDB <= 4 ? 2 : 1) void latent_attn
   }
 }
 
-template <int NCB, bool SPLIT, bool ROT, bool SIG = false, bool CAP = false>
+template <int NKS, bool SPLIT, bool ROT, bool SIG = false, bool CAP = false>
 void launch_ncb(const LArgs& a, int ndb, dim3 grid, hipStream_t st) {
   auto go = [&](auto kern, int NDBv) {
+    constexpr int NCB = (NKS + 7) / 8;
     const size_t one = (size_t)(NCB + (NDBv + 3) / 4) * LIMG;
     const size_t lds = (2 * one + 1024 <= 160 * 1024 ? 2 * one : one) + 2 * LKB * sizeof(int);
     HYB_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess, "LDS size");
     kern<<<grid, 256, lds, st>>>(a);
   };
-  if (ndb == 2) go(latent_attn_mfma_kernel<NCB, 2, ROT, SIG, CAP, SPLIT>, 2);
-  else if (ndb == 4) go(latent_attn_mfma_kernel<NCB, 4, ROT, SIG, CAP, SPLIT>, 4);
-  else go(latent_attn_mfma_kernel<NCB, 8, ROT, SIG, CAP, SPLIT>, 8);
+  if (ndb == 2) go(latent_attn_mfma_kernel<NKS, 2, ROT, SIG, CAP, SPLIT>, 2);
+  else if (ndb == 4) go(latent_attn_mfma_kernel<NKS, 4, ROT, SIG, CAP, SPLIT>, 4);
+  else go(latent_attn_mfma_kernel<NKS, 8, ROT, SIG, CAP, SPLIT>, 8);
 }
 
 template <bool SPLIT>
@@ -378,21 +413,24 @@ void launch_form(const LArgs& a, int ncb, int ndb, dim3 grid, const RowAttnOpts&
   hipStream_t st = cur_stream();
   if (x.softcap > 0.0) {  // built for keys up to 256 wide, plain softmax form (the caller checks)
     HYB_CHECK(x.hscale == nullptr && ncb <= 2, "capped scores: no per-head factor, keys up to 256 wide");
-    if (ncb == 1) launch_ncb<1, SPLIT, false, false, true>(a, ndb, grid, st);
-    else launch_ncb<2, SPLIT, false, false, true>(a, ndb, grid, st);
+    if (ncb == 1) launch_ncb<8, SPLIT, false, false, true>(a, ndb, grid, st);
+    else launch_ncb<16, SPLIT, false, false, true>(a, ndb, grid, st);
   } else if (x.sig_bias != nullptr) {  // built for keys up to 256 wide (latent_attn_mfma_ok)
-    if (ncb == 1) launch_ncb<1, SPLIT, false, true>(a, ndb, grid, st);
-    else launch_ncb<2, SPLIT, false, true>(a, ndb, grid, st);
+    if (ncb == 1) launch_ncb<8, SPLIT, false, true>(a, ndb, grid, st);
+    else launch_ncb<16, SPLIT, false, true>(a, ndb, grid, st);
   } else if (x.ofreq != nullptr) {
-    if (ncb == 1) launch_ncb<1, SPLIT, true>(a, ndb, grid, st);
-    else launch_ncb<2, SPLIT, true>(a, ndb, grid, st);
+    if (ncb == 1) launch_ncb<8, SPLIT, true>(a, ndb, grid, st);
+    else launch_ncb<16, SPLIT, true>(a, ndb, grid, st);
   } else {
     switch (ncb) {
-      case 1: launch_ncb<1, SPLIT, false>(a, ndb, grid, st); break;
-      case 2: launch_ncb<2, SPLIT, false>(a, ndb, grid, st); break;
-      case 3: launch_ncb<3, SPLIT, false>(a, ndb, grid, st); break;
-      case 4: launch_ncb<4, SPLIT, false>(a, ndb, grid, st); break;
-      default: launch_ncb<5, SPLIT, false>(a, ndb, grid, st); break;
+      case 1: launch_ncb<8, SPLIT, false>(a, ndb, grid, st); break;
+      case 2:
+        if (!SPLIT && a.R <= 192) launch_ncb<12, false, false>(a, ndb, grid, st);
+        else launch_ncb<16, SPLIT, false>(a, ndb, grid, st);
+        break;
+      case 3: launch_ncb<24, SPLIT, false>(a, ndb, grid, st); break;
+      case 4: launch_ncb<32, SPLIT, false>(a, ndb, grid, st); break;
+      default: launch_ncb<40, SPLIT, false>(a, ndb, grid, st); break;
     }
   }
 }
@@ -441,7 +479,8 @@ void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::T
   const Cut c(qa.size(2), rk, qa.size(1) / x.groups, max_q < 64);
   const int TB = 128 / c.HB, z = (int)x.groups * c.hpg * c.nvt;
   HYB_CHECK(ns <= 65535 && z <= 65535, "grid too large");
-  const LArgs a = make_args(qa, cache, bt, cu.data_ptr<int>(), ctx, window, sink, scale, rk, out, x, c);
+  LArgs a = make_args(qa, cache, bt, cu.data_ptr<int>(), ctx, window, sink, scale, rk, out, x, c);
+  a.xcd = z % 8 == 0 ? 1 : 0;
   launch_form<false>(a, c.ncb, c.ndb, dim3((unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)z), x);
 }
 
