@@ -12,6 +12,7 @@ int64_t car_sig_words();
 int64_t car_error(int64_t sig_ptr);
 void set_knob(const std::string& name, int64_t value);  // knobs.cpp
 void clear_knobs();
+int64_t graph_memsets(int64_t graph);
 int64_t gemm64_wgrad_splits(int64_t M, int64_t N, int64_t K, bool bias);
 int64_t decode_layers_words(int64_t hidden);
 }  // namespace llmctl
@@ -84,6 +85,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("gemm64_wgrad_splits(int M, int N, int K, bool bias) -> int", &llmctl::gemm64_wgrad_splits);
   m.def("set_knob(str name, int value) -> ()", &llmctl::set_knob);
   m.def("clear_knobs() -> ()", &llmctl::clear_knobs);
+  m.def("graph_memsets(int graph) -> int", &llmctl::graph_memsets);
   m.def("gemm_ex(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, int variant=-1) -> ()");
   m.def("hbm_copy(Tensor src, Tensor(a!) dst) -> ()");
   m.def("gemm64_ex(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, int config=4) -> ()");

@@ -30,8 +30,6 @@
 // delta = rowsum(dO * O) is computed by the dQ kernel (its dO rows are in registers) and read by
 // the dK/dV kernel launched after it.
 #include <cstdlib>
-#include <map>
-#include <mutex>
 
 #include "attn_common.h"
 
@@ -1426,19 +1424,8 @@ int dkv_mode() {
   return (m >= 0 && m <= 2) ? (int)m : 2;
 }
 
-// the persistent dK/dV kernel's per-XCD item counters: one buffer per (device, stream), zeroed
-// before every launch on that stream.  Launches on one stream are ordered, so they may share a
-// buffer; two streams (or threads launching on them) never do.  The map is mutex-guarded.
-int* dkv_queue(hipStream_t s) {
-  static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, int*> bufs;
-  int dev = 0;
-  LLMCTL_HIP_CHECK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lk(mu);
-  int*& q = bufs[{dev, s}];
-  if (q == nullptr) LLMCTL_HIP_CHECK(hipMalloc(&q, 64 * sizeof(int)));
-  return q;
-}
+// the persistent dK/dV kernel's per-XCD item counters start at zero (a kernel: a recorded memset has given wrong counters on replays)
+__global__ void dkv_queue_zero(int* q) { q[threadIdx.x] = 0; }
 
 // dkv_impl: -1 = default (knob dkv), 0 = unpipelined kernel, 1 = pipelined where built
 template <int HD, bool CAUSAL, bool DOC>
@@ -1457,8 +1444,9 @@ void launch_bwd(const BwdArgs& a, hipStream_t s, bool do_dq, bool do_dkv, int dk
       }
       if constexpr (!DOC) {  // persistent form: S % 128 (>= 2 tiles per item)
         if (a.S % KV_KB == 0 && (dkv_impl == 3 || dkv_impl == 4 || (dkv_impl < 0 && dkv_mode() == 2))) {
-          int* wq = dkv_queue(s);
-          LLMCTL_HIP_CHECK(hipMemsetAsync(wq, 0, 8 * sizeof(int), s));
+          at::Tensor queue = at::empty({8}, at::TensorOptions().dtype(at::kInt).device(at::kCUDA, at::hip::current_device()));
+          int* wq = queue.data_ptr<int>();
+          hipLaunchKernelGGL(dkv_queue_zero, dim3(1), dim3(8), 0, s, wq);
           int nwg = std::min<long>((long)num_cus(), (long)a.B * a.Hkv * nkb);
           // per-XCD queues (B*Hkv % 8 == 0) are drained by blocks with blockIdx & 7 == queue:
           // fewer than 8 workgroups would leave queues without a consumer

@@ -90,7 +90,9 @@ class StepGraph:
 
     def capture(self, engine, denom: float, stream, pool) -> None:
         """Record.  Nothing runs, so a failure (raised) leaves the gradients as they were."""
-        g = torch.cuda.CUDAGraph()
+        from llmctl.ops._lib import native
+
+        g = torch.cuda.CUDAGraph(keep_graph=True)
         with graph_capture_gc_guard(collect=False), torch.cuda.stream(stream):
             # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
             g.capture_begin(pool=pool, capture_error_mode="thread_local")
@@ -104,6 +106,11 @@ class StepGraph:
                 g.reset()
                 raise
             g.capture_end()
+        if native().graph_memsets(g.raw_cuda_graph()):  # (a library's sum over many blocks clears its counters so)
+            del loss
+            g.reset()
+            raise RuntimeError("the step records a memset")
+        g.instantiate()
         self.graph, self.loss = g, loss
 
     def run(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:

@@ -8,11 +8,11 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def engine(model="tiny", layers=2, knob=True, tokens=(2, 128), **kw):
+def engine(model="tiny", layers=2, knob=True, tokens=(2, 128), heads=None, **kw):
     from llmctl.models import get_model_config
     from llmctl.runtime.engine import TrainingConfig, TrainingEngine
 
-    cfg = dataclasses.replace(get_model_config(model), layers=layers)
+    cfg = dataclasses.replace(get_model_config(model), layers=layers, **({} if heads is None else dict(heads=heads, kv_heads=heads)))
     return TrainingEngine(TrainingConfig(model_name_or_path=model, batch_size=tokens[0], seq_len=tokens[1], device="cuda", log_level="warning",
                                          learning_rate=1e-3, max_steps=50, seed=3, perf_knobs={"step_graph": knob}, **kw), cfg)
 
@@ -22,20 +22,23 @@ def batch(eng, g, b, s):
     return t[:, :-1], t[:, 1:]  # (rows of another tensor, as a loader's are)
 
 
-@pytest.mark.parametrize("model,layers,sizes", [("tiny", 2, [(2, 128)]), ("tiny", 2, [(1, 65), (3, 100), (8, 512)]), ("gpt2-125m", 2, [(2, 64), (1, 333)])])
-def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes):
+# (the last two: heads of 128, whose dK/dV kernel counts its items in memory, and a loss over 16384 tokens, which the library sums with a memset: such steps stay eager)
+@pytest.mark.parametrize("model,layers,sizes,heads,recorded", [
+    ("tiny", 2, [(2, 128)], None, 1), ("tiny", 2, [(1, 65), (3, 100), (8, 512)], None, 3), ("gpt2-125m", 2, [(2, 64), (1, 333)], None, 2),
+    ("tiny", 2, [(2, 128), (5, 256)], 2, 2), ("tiny", 1, [(32, 512)], None, None)])
+def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes, heads, recorded):
     """Losses, norms, gradients and states over many steps of alternating shapes, other work on the device between them.  Both sides run the same
     kernels; what differs from run to run is the order of the clip norm's atomics (and a library product's partial sums), which moves the weights by
     rounding: the bound is four times the spread of two eager runs, or rounding of bf16 weights (2^-9) where they happen to agree."""
     def run(knob):
-        eng, g, out = engine(model, layers, knob), torch.Generator().manual_seed(1), []
+        eng, g, out = engine(model, layers, knob, heads=heads), torch.Generator().manual_seed(1), []
         for step in range(5):
             for b, s in sizes:
                 r = eng.train_step([batch(eng, g, b, s)])
                 keep = torch.full((1 << 20,), float(step), device="cuda")  # memory that a stale pointer would hit
                 out += [r["loss"], r["grad_norm"], keep.sum() * 0]
         torch.cuda.synchronize()
-        assert len(eng.step_graphs.table) == (len(sizes) if knob else 0)
+        assert recorded is None or len(eng.step_graphs.table) == (recorded if knob else 0)
         return torch.stack([o.float().reshape(()) for o in out]), eng.flat.grad.float(), eng.optimizer.master, eng.optimizer.exp_avg
 
     a, b, c = run(True), run(False), run(False)
@@ -77,6 +80,19 @@ def test_what_listens_is_heard(native_lib):
     p.grad = None
     step()
     assert p.grad is not None and p.grad.data_ptr() == eng.flat.grad.data_ptr() + 2 * eng.flat.offsets[id(p)]
+
+
+def test_memsets_of_a_recording_are_counted(native_lib):
+    x = torch.ones(1 << 22, device="cuda")
+    for f, n in ((lambda: x.mul_(1.0), 0), (lambda: x.sum(), None)):
+        f()
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            out = f()
+        found = native_lib.graph_memsets(g.raw_cuda_graph())
+        assert found == n if n is not None else found >= 0
+        del out
+        g.reset()
 
 
 def test_long_steps_stay_eager(native_lib):
