@@ -82,6 +82,7 @@ struct BwdArgs {
   // dS = p dP', no per-element subtract or LSE scaling)
   float* rck_w;
   long rc_n;
+  int together;  // heads_together
   // diagnostic timeline (fa_bwd_ablate abl 6 only): per workgroup 8 x u64, see the pipelined kernel
   unsigned long long* stamps = nullptr;
 };
@@ -198,10 +199,11 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkv_kernel(BwdArgs a) {
   if (BH % 8) {
     bh = blockIdx.x % BH;
     kblk = blockIdx.x / BH;  // small kblk = most query tiles under causal: dispatched first
-  } else {  // XCD-aware: XCD x walks kv-heads [x*BH/8, (x+1)*BH/8), a head's key blocks back to back
+  } else {  // XCD-aware: XCD x walks kv-heads [x*BH/8, (x+1)*BH/8)
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    bh = x * (BH >> 3) + j / nkb;
-    kblk = j % nkb;
+    if (CAUSAL) causal_block(j, nkb, BH >> 3, a.together, bh, kblk);
+    else bh = j / nkb, kblk = j % nkb;
+    bh += x * (BH >> 3);
   }
   const int b = bh / a.Hkv, hk = bh % a.Hkv;
   const int group = a.Hq / a.Hkv;
@@ -594,8 +596,9 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkv_pipe_kernel(BwdArgs a) {
     kblk = blockIdx.x / BH;
   } else {
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    bh = x * (BH >> 3) + j / nkb;
-    kblk = j % nkb;
+    if (CAUSAL) causal_block(j, nkb, BH >> 3, a.together, bh, kblk);
+    else bh = j / nkb, kblk = j % nkb;
+    bh += x * (BH >> 3);
   }
   const int b = bh / a.Hkv, hk = bh % a.Hkv;
   const int group = a.Hq / a.Hkv;
@@ -922,7 +925,9 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkv_persist_kernel(BwdArgs a, i
   // twice during one compute item (one variable lost the first of the two: a skipped item)
   int pend0 = -1, pend1 = -1, npend = 0;
   auto iss_begin = [&](int item) __attribute__((always_inline)) {
-    const int bh = bh_base + item / nkb, kb = item % nkb;
+    int bh, kb;
+    causal_block(item, nkb, per_xcd ? BH / 8 : BH, a.together, bh, kb);
+    bh += bh_base;
     const int bb = bh / a.Hkv, hkk = bh % a.Hkv;
     iq_start = kb * KV_KB;
     iq0 = iq_start;
@@ -969,7 +974,9 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkv_persist_kernel(BwdArgs a, i
 
   bf16x8_t kf[NKS], vf[NKS];
   auto load_kv = [&](int item) __attribute__((always_inline)) {
-    const int bh = bh_base + item / nkb, kb = item % nkb;
+    int bh, kb;
+    causal_block(item, nkb, per_xcd ? BH / 8 : BH, a.together, bh, kb);
+    bh += bh_base;
     const int bb = bh / a.Hkv, hkk = bh % a.Hkv;
     const int key = kb * KV_KB + wave * 32 + r;
     const unsigned short* Kp = a.k + bb * a.k_sb + hkk * a.k_sh + (long)key * a.k_ss + 8 * hh;
@@ -1012,7 +1019,9 @@ __global__ __launch_bounds__(256, 1) void fa_bwd_dkv_persist_kernel(BwdArgs a, i
   for (;;) {  // ---- items
     stamp(0);
     stamp(3);
-    const int bh = bh_base + cur / nkb, kb = cur % nkb;
+    int bh, kb;
+    causal_block(cur, nkb, per_xcd ? BH / 8 : BH, a.together, bh, kb);
+    bh += bh_base;
     const int b = bh / a.Hkv, hk = bh % a.Hkv;
     const int k0 = kb * KV_KB;
     const int wkey0 = k0 + wave * 32;
@@ -1224,10 +1233,11 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dq_kernel(BwdArgs a) {
   if (BH % 8) {
     bh = blockIdx.x % BH;
     qi = blockIdx.x / BH;
-  } else {  // XCD-aware: XCD x walks heads [x*BH/8, (x+1)*BH/8), a head's q-blocks back to back
+  } else {  // XCD-aware: XCD x walks heads [x*BH/8, (x+1)*BH/8)
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    bh = x * (BH >> 3) + j / nqb;
-    qi = j % nqb;
+    if (CAUSAL) causal_block(j, nqb, BH >> 3, a.together, bh, qi);
+    else bh = j / nqb, qi = j % nqb;
+    bh += x * (BH >> 3);
   }
   const int qblk = nqb - 1 - qi;  // heaviest first
   const int b = bh / a.Hq, hq = bh % a.Hq;
@@ -1429,7 +1439,8 @@ __global__ void dkv_queue_zero(int* q) { q[threadIdx.x] = 0; }
 
 // dkv_impl: -1 = default (knob dkv), 0 = unpipelined kernel, 1 = pipelined where built
 template <int HD, bool CAUSAL, bool DOC>
-void launch_bwd(const BwdArgs& a, hipStream_t s, bool do_dq, bool do_dkv, int dkv_impl) {
+void launch_bwd(BwdArgs a, hipStream_t s, bool do_dq, bool do_dkv, int dkv_impl) {
+  a.together = heads_together(a.S, HD);
   if (do_dq) {
     const int nqb = (a.S + DQ_QB - 1) / DQ_QB;
     hipLaunchKernelGGL((fa_bwd_dq_kernel<HD, CAUSAL, DOC>), dim3((unsigned)(a.B * a.Hq * nqb)), dim3(256), 0, s, a);

@@ -21,9 +21,8 @@
 //     plain one — round 1's per-element divergent branches cost ~30 % of the loop's issue slots
 //     (profiles/attn_fwd_isa_r2.txt);
 //   * causal: tiles wholly above a wave's diagonal are skipped; dispatch is XCD-aware: each XCD
-//     (workgroup i -> XCD i % 8) walks a contiguous range of heads with a head's q-blocks back
-//     to back, heaviest first, so the few heads resident per XCD keep their K/V in its L2
-//     (the head-major order kept ~48 heads = 48 MB of K/V live per 4 MB L2);
+//     (workgroup i -> XCD i % 8) walks a contiguous range of heads in groups whose K/V its L2
+//     holds, a group's q-blocks heaviest first (causal_block);
 //   * packed sequences (optional ``doc_start[B,S]``: position where each token's document
 //     begins, non-decreasing): key j is visible to query i iff doc_start[i] <= j <= i; the
 //     K/V loop starts at the block's first document start, so the work is sum(doc_len^2);
@@ -59,6 +58,7 @@ struct FwdArgs {
   const int* doc;    // [B, S] document start per token, or nullptr
   unsigned short* o_part;  // SPLIT: [2, B, S, Hq, HD] bf16 normalised partial outputs
   float* lse_part;   // SPLIT: [2, B, Hq, S] natural-log partial LSEs
+  int together;      // heads_together
   int prio;          // raise the wave priority over its MFMA phases (A/B knob fa_prio)
 };
 
@@ -86,12 +86,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fa_fwd_kernel(FwdArgs a) {
     bh = blockIdx.x % BH;
     rest = blockIdx.x / BH;
   } else {
-    // XCD-aware order: workgroup i runs on XCD i % 8; XCD x walks the heads
-    // [x*BH/8, (x+1)*BH/8) one after another, all q-blocks of a head back to back (heaviest
-    // first), so the K/V stream of the ~4 heads resident on an XCD stays in its 4 MB L2
+    // XCD-aware order: workgroup i runs on XCD i % 8; XCD x walks the heads [x*BH/8, (x+1)*BH/8)
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    bh = x * (BH >> 3) + j / nqb;
-    rest = j % nqb;
+    if (CAUSAL) causal_block(j, nqb, BH >> 3, a.together, bh, rest);
+    else bh = j / nqb, rest = j % nqb;
+    bh += x * (BH >> 3);
   }
   const int part = SPLIT ? rest & 1 : 0;
   const int qblk = nqb - 1 - (SPLIT ? rest >> 1 : rest);  // heaviest (largest causal span) first
@@ -467,6 +466,7 @@ std::tuple<at::Tensor, at::Tensor> flash_attn_fwd(const at::Tensor& q, const at:
             q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
             v.stride(0), v.stride(1), v.stride(2), o.stride(0), o.stride(1), o.stride(2),
             (float)(scale * 1.4426950408889634), nullptr, nullptr, nullptr, 0};
+  a.together = heads_together(S, D);
   a.prio = knob("fa_prio", 1) != 0 ? 1 : 0;  // default on: 2-3 % at B12 S2048 (0: off, A/B)
   // workgroup shape: knob fa_nw = 8 -> 8 waves (256 rows) with a 3-slot ring, one workgroup per
   // CU; default 4 waves (128 rows) with a 2-slot ring, two per CU (A/B knob, tools/attn_bench.py)
