@@ -382,20 +382,26 @@ class BiasedSoftmaxMoE(nn.Module):
                 return hops.glu_act(u, "silu", scale)
             return hops.act_any(u, self.act, scale)
 
-        z = ys = None
-        if self.w_sup is not None:
+        z = ys = ride = None
+        down = self._down_list()
+        if self.shared_ff and T <= 32 and hops.shared_rides(x, self.w_sup, self.b_sup, self.sup_rows, self.w_sdown, self.act) and (
+                routed or (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1])
+                           and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router))):
+            ride = (self.w_sup, self.b_sup, self.sup_rows, self.w_sdown, self.shared_gate)
+        elif self.w_sup is not None:
             fused = self.act != "swiglu" and hops.rows_ok(x, self.w_sup, self.b_sup)  # the activation in the product's epilogue
             z = (hops.rows_linear(x, self.w_sup, self.b_sup, self.act, self.sup_rows) if fused
                  else hops.linear(x, self.w_sup, self.b_sup))
             if self.shared_ff:
                 u = z[:, :self.sup_rows]
                 ys = hops.linear(u if fused else act(u), self.w_sdown)
-        gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate else None
-        down = self._down_list()
-        if routed or (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
+        gate = z[:, self.sup_rows:self.sup_rows + 1] if self.shared_gate and z is not None else None
+        if ride is not None or routed or (hops.experts_pay(T, self.top, self.E, self.up_rows, x.shape[1]) and not hops.wants_grad(ys, gate)
                       and hops.experts_ok(x, self.w_up, down, self.E + self.identity, self.top, self.w_router)):
             out = hops.routed_experts(x, self.w_router, self.bias, self.top, self.groups, self.keep, True, self.renorm, self.w_up, down,
-                                      self.act, ys, gate, **({"late": late, "routed": routed} if late else {}))
+                                      self.act, ys, gate, **({"late": late, "routed": routed} if late else {}), **({"ride": ride} if ride else {}))
+            if ride is not None:
+                out, z = out
             return (out, z[:, self.sup_rows + (1 if self.shared_gate else 0):]) if self.side else out
         topi, topw = hops.bias_topk_router(torch.nn.functional.linear(x.float(), self.w_router), self.bias, self.top,
                                            self.groups, self.keep, self.renorm)

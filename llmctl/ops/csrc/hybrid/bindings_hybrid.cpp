@@ -57,6 +57,10 @@ at::Tensor rows_linear(const at::Tensor& x, const at::Tensor& w, const c10::opti
 std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t top,
                                              int64_t groups, int64_t keep, bool softmax, bool renorm);
 at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act);
+std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_expert_rows_shared(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up,
+                                                                      at::TensorList down, int64_t act, const at::Tensor& w_sup,
+                                                                      const c10::optional<at::Tensor>& b_sup, int64_t act_cols, const at::Tensor& w_sdown);
+bool moe_shared_rides(int64_t M, int64_t N, int64_t K, int64_t ff);
 at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
                        const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate);
 at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
@@ -181,6 +185,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("rows_linear(Tensor x, Tensor w, Tensor? bias, int act, int act_cols, bool f32) -> Tensor");
   m.def("moe_route(Tensor x, Tensor w, Tensor? bias, int top, int groups, int keep, bool softmax, bool renorm) -> (Tensor, Tensor)");
   m.def("moe_expert_rows(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act) -> Tensor");
+  m.def("moe_expert_rows_shared(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor w_sup, Tensor? b_sup, int act_cols, Tensor w_sdown) -> (Tensor, Tensor, Tensor)");
+  m.def("moe_shared_rides(int M, int N, int K, int ff) -> bool", &llmctl_hybrid::moe_shared_rides);
   m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
   m.def("moe_sum(Tensor y, Tensor idx, Tensor wgt, Tensor x, Tensor? shared, Tensor? gate, int experts) -> Tensor");
   m.def("add_experts_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? w, Tensor? bias, float eps, Tensor y, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts, Tensor? router=None, Tensor? rbias=None, int top=0, int groups=1, int keep=1, bool softmax=False, bool renorm=False) -> Tensor[]");
@@ -243,6 +249,7 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("rows_linear", &llmctl_hybrid::rows_linear);
   m.impl("moe_route", &llmctl_hybrid::moe_route);
   m.impl("moe_expert_rows", &llmctl_hybrid::moe_expert_rows);
+  m.impl("moe_expert_rows_shared", &llmctl_hybrid::moe_expert_rows_shared);
   m.impl("moe_experts", &llmctl_hybrid::moe_experts);
   m.impl("moe_sum", &llmctl_hybrid::moe_sum);
   m.impl("add_experts_layernorm_f32_", &llmctl_hybrid::add_experts_layernorm_f32_);

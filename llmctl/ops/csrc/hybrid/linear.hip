@@ -1,6 +1,6 @@
 // Projections of a few rows (decode steps): see ../stream_linear.h.
 #include "hybrid_common.h"
-#include "stream_linear.h"
+#include "stream_linear_launch.h"
 
 namespace llmctl_hybrid {
 

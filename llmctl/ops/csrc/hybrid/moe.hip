@@ -35,6 +35,7 @@
 // last round of tiles.  A layer of 2048 tokens took 700 us before (sort, per-expert GEMMs, copies), 16 tokens 350 us.
 #include "expert_rows.h"
 #include "router_rows.h"
+#include "stream_linear.h"
 
 namespace llmctl_hybrid {
 namespace {
@@ -349,16 +350,28 @@ struct SmallArgs {
   long ldw;
   void* out;  // UP: bf16 [N, cols]; DOWN: fp32 [N, cols]
   const int* idx;
-  int N, K, cols, top, act;
+  int N, K, cols, top, act, E;
+  stream_linear::Args side;  // SIDE: the shared expert's product of the same rows, its workgroups behind the experts' in blockIdx.y
+  int side_groups;
 };
 
-template <int MT, int MODE>
+// SIDE: a shared expert's projection of the step's rows (form <1, MT, 4, 8> of stream_linear.h, so the bits are those of a launch of its own) rides along: it is
+// as long as its launch and one round trip, and the experts' workgroups leave bandwidth over.  16 rows of width 2048, 8 experts of 1024 and a shared one of 1024: the
+// four launches 6.9 + 4.6 + 9.8 + 10.6 us a layer, the two 13.4 + 12.4; a step of three layers 299 us, so 282.
+template <int MT, int MODE, bool SIDE>
 __global__ __launch_bounds__(256) void moe_small_kernel(SmallArgs g) {
   constexpr int NM = MODE == UP_GLU ? 2 : 1;
   constexpr int U = MT >= 4 ? 4 : 8;  // K steps in flight (16 took 27 + 18 us where 8 took 26 + 14)
   __shared__ int list[SMALL_ROWS];
   __shared__ int count;
   __shared__ facc red[4][MT * NM][64];
+  if constexpr (SIDE) {
+    if ((int)blockIdx.y >= g.E) {
+      const int i = ((int)blockIdx.y - g.E) * (int)gridDim.x + (int)blockIdx.x;
+      if (i < g.side_groups) stream_linear::workgroup<1, MT, 4, 8>(g.side, (unsigned)i, 0, reinterpret_cast<stream_linear::acc_t(*)[MT][64]>(red));
+      return;
+    }
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int e = blockIdx.y, n0 = blockIdx.x * 16;
   const int r = lane & 15, kg = lane >> 4;
@@ -384,7 +397,7 @@ __global__ __launch_bounds__(256) void moe_small_kernel(SmallArgs g) {
     }
   };
   // with two copies per expert or more nearly every expert runs: its first weights are on their way while the rows are found
-  const bool early = g.N >= 2 * (int)gridDim.y;
+  const bool early = g.N >= 2 * g.E;
   if (early) fetch_w(s0);
   if (wave == 0) {
     int c = 0;
@@ -556,7 +569,19 @@ std::tuple<at::Tensor, at::Tensor> moe_route(const at::Tensor& x, const at::Tens
 
 // Results of the chosen experts of every row of x, [T * top, W] by entry: fp32 for few tokens, else bf16.  ``act``: 0 relu^2, 1 silu-gated
 // (up weights hold [gate ; up]), 2 gelu.  idx >= the number of experts: an expert that gives its input, whose entries are not written.
-at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act) {
+namespace {
+// A shared expert's two products beside the experts': z = act(x w_up^T + bias) on its first act_cols columns, y = z[:, :act_cols] w_down^T.
+struct SharedExpert {
+  const at::Tensor *up, *bias, *down;
+  int64_t act_cols;
+  at::Tensor z, y;
+};
+bool side_rides(int64_t M, int64_t N, int64_t K) {
+  const stream_linear::Form f = stream_linear::form_of((int)M, (int)N, (int)K);
+  return M <= 32 && f.nt == 1 && f.nw == 4 && f.u == 8;
+}
+
+at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act, SharedExpert* sh) {
   int64_t E, R, W, E2, W2, ff;
   long ldu, ldd;
   const ExpertPtrs pu = expert_ptrs(up, E, R, W, ldu, "up"), pd = expert_ptrs(down, E2, W2, ff, ldd, "down");
@@ -576,14 +601,37 @@ at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at:
   const bf16_t* xp = reinterpret_cast<const bf16_t*>(x.data_ptr());
   bf16_t* ap = reinterpret_cast<bf16_t*>(a.data_ptr());
   if (small) {
-    SmallArgs u{xp, (long)x.stride(0), pu, ldu, ap, idx.data_ptr<int>(), (int)N, (int)W, (int)ff, (int)top, (int)act};
-    SmallArgs d{ap, (long)ff, pd, ldd, y.data_ptr(), idx.data_ptr<int>(), (int)N, (int)ff, (int)W, (int)top, (int)act};
-    const dim3 gu((unsigned)((ff + 15) / 16), (unsigned)E), gd((unsigned)((W + 15) / 16), (unsigned)E);
+    SmallArgs u{xp, (long)x.stride(0), pu, ldu, ap, idx.data_ptr<int>(), (int)N, (int)W, (int)ff, (int)top, (int)act, (int)E, {}, 0};
+    SmallArgs d{ap, (long)ff, pd, ldd, y.data_ptr(), idx.data_ptr<int>(), (int)N, (int)ff, (int)W, (int)top, (int)act, (int)E, {}, 0};
+    dim3 gu((unsigned)((ff + 15) / 16), (unsigned)E), gd((unsigned)((W + 15) / 16), (unsigned)E);
+    if (sh != nullptr) {
+      const int64_t C = sh->up->size(0);
+      sh->z = at::empty({T, C}, x.options());
+      sh->y = at::empty({T, W}, x.options());
+      auto ptr = [](const at::Tensor& t) { return reinterpret_cast<const bf16_t*>(t.data_ptr()); };
+      u.side = stream_linear::Args{xp, (long)x.stride(0), ptr(*sh->up), (long)sh->up->stride(0), sh->bias != nullptr ? ptr(*sh->bias) : nullptr, sh->z.data_ptr(),
+                                   (int)T, (int)C, (int)W, act == 0 ? 3 : 1, (int)sh->act_cols, 0};
+      d.side = stream_linear::Args{ptr(sh->z), (long)C, ptr(*sh->down), (long)sh->down->stride(0), nullptr, sh->y.data_ptr(), (int)T, (int)W, (int)sh->act_cols, 0, 0, 0};
+      auto ride = [](SmallArgs& g, dim3& grid) {
+        g.side.rows = stream_linear::form_of(g.side.M, g.side.N, g.side.K).rows;
+        g.side_groups = (g.side.N + g.side.rows - 1) / g.side.rows;
+        grid.y += ((unsigned)g.side_groups + grid.x - 1) / grid.x;
+      };
+      ride(u, gu);
+      ride(d, gd);
+    }
     auto go = [&](auto mt) {
       constexpr int MT = decltype(mt)::value;
-      if (act == 1) moe_small_kernel<MT, UP_GLU><<<gu, 256, 0, st>>>(u);
-      else moe_small_kernel<MT, UP_PLAIN><<<gu, 256, 0, st>>>(u);
-      moe_small_kernel<MT, DOWN><<<gd, 256, 0, st>>>(d);
+      if constexpr (MT <= 2) {
+        if (sh != nullptr) {
+          moe_small_kernel<MT, UP_PLAIN, true><<<gu, 256, 0, st>>>(u);
+          moe_small_kernel<MT, DOWN, true><<<gd, 256, 0, st>>>(d);
+          return;
+        }
+      }
+      if (act == 1) moe_small_kernel<MT, UP_GLU, false><<<gu, 256, 0, st>>>(u);
+      else moe_small_kernel<MT, UP_PLAIN, false><<<gu, 256, 0, st>>>(u);
+      moe_small_kernel<MT, DOWN, false><<<gd, 256, 0, st>>>(d);
     };
     if (T <= 16) go(std::integral_constant<int, 1>{});
     else if (T <= 32) go(std::integral_constant<int, 2>{});
@@ -611,6 +659,33 @@ at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at:
     }
   }
   return y;
+}
+
+}  // namespace
+
+at::Tensor moe_expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act) {
+  return expert_rows(x, idx, wgt, up, down, act, nullptr);
+}
+
+// Whether moe_expert_rows_shared takes a shared expert of these sizes: M rows of width K to N columns, the first ff of them back to K.
+bool moe_shared_rides(int64_t M, int64_t N, int64_t K, int64_t ff) { return M >= 1 && M <= 32 && ff >= 8 && ff <= N && side_rides(M, N, K) && side_rides(M, K, ff); }
+
+// moe_expert_rows of at most 32 rows, and a shared expert's products in the same launches: (experts' rows, act(x w_sup^T + bias) with the activation on
+// the first act_cols columns, those columns' product with w_sdown).  act: 0 relu^2, 2 gelu.
+std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_expert_rows_shared(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up,
+                                                                      at::TensorList down, int64_t act, const at::Tensor& w_sup,
+                                                                      const c10::optional<at::Tensor>& b_sup, int64_t act_cols, const at::Tensor& w_sdown) {
+  HYB_CHECK(x.dim() == 2 && w_sup.dim() == 2 && w_sdown.dim() == 2 && (act == 0 || act == 2), "shared expert: matrices, relu^2 or gelu");
+  const int64_t M = x.size(0), K = x.size(1), N = w_sup.size(0);
+  HYB_CHECK(moe_shared_rides(M, N, K, act_cols) && act_cols % 8 == 0 && N % 8 == 0, "shared expert: sizes (moe_shared_rides)");
+  for (const at::Tensor* w : {&w_sup, &w_sdown})
+    HYB_CHECK(w->is_cuda() && w->scalar_type() == at::kBFloat16 && rows16(*w), "shared expert: bf16 weights, aligned rows");
+  HYB_CHECK(w_sup.size(1) == K && w_sdown.size(0) == K && w_sdown.size(1) == act_cols, "shared expert: weights fit each other");
+  if (b_sup.has_value())
+    HYB_CHECK(b_sup->is_cuda() && b_sup->scalar_type() == at::kBFloat16 && b_sup->is_contiguous() && b_sup->numel() == N, "shared expert: bias bf16 [N]");
+  SharedExpert sh{&w_sup, b_sup.has_value() ? &*b_sup : nullptr, &w_sdown, act_cols, {}, {}};
+  const at::Tensor y = expert_rows(x, idx, wgt, up, down, act, &sh);
+  return {y, sh.z, sh.y};
 }
 
 ExpertRows expert_rows_of(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x,

@@ -60,19 +60,19 @@ __device__ __forceinline__ float activate(int act, float v) {
 // A workgroup of NW waves owns ``rows`` weight rows, at most 16 NT; the waves split K.  A lane streams 16 bytes of its weight row per 32-deep step,
 // U steps in flight before the first MFMA; the weight fragment is the MFMA row operand, so a lane ends up with four
 // neighbouring outputs of one token.  K is a multiple of 8 (the last step is filled up with zeros), N any.
+// Workgroup (bx, by); red: LDS for the waves' sums.
 template <int NT, int MT, int NW, int U>
-__global__ __launch_bounds__(NW * 64) void kernel(Args g) {
-  __shared__ acc_t red[NW][NT * MT][64];
+__device__ __forceinline__ void workgroup(Args g, unsigned bx, unsigned by, acc_t (*red)[NT * MT][64]) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, kg = lane >> 4;
   if (g.part > 0) {
-    const int k0 = blockIdx.y * g.part;
+    const int k0 = by * g.part;
     g.x += k0;
     g.w += k0;
     g.K = min(g.part, g.K - k0);
-    g.y = static_cast<float*>(g.y) + (long)blockIdx.y * g.M * g.N;
+    g.y = static_cast<float*>(g.y) + (long)by * g.M * g.N;
   }
-  const int n0 = blockIdx.x * g.rows, n1 = min(n0 + g.rows, g.N);
+  const int n0 = bx * g.rows, n1 = min(n0 + g.rows, g.N);
   const unsigned short* wp[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) wp[n] = g.w + (long)min(n0 + n * 16 + r, n1 - 1) * g.ldw + 8 * kg;
@@ -140,7 +140,9 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
       float* y = static_cast<float*>(g.y) + o;
       if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
       else
-        for (int j = 0; j < left; ++j) y[j] = v[j];
+#pragma unroll  // (a loop of ``left`` turns would index the values by a register: through LDS, 8256 x 2048 24 us for 11.5)
+        for (int j = 0; j < 4; ++j)
+          if (j < left) y[j] = v[j];
     } else {
       unsigned short* y = static_cast<unsigned short*>(g.y) + o;
       unsigned short h[4];
@@ -148,16 +150,11 @@ __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
       for (int j = 0; j < 4; ++j) h[j] = __bfloat16_as_ushort(__float2bfloat16(v[j]));
       if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
       else
-        for (int j = 0; j < left; ++j) y[j] = h[j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < left) y[j] = h[j];
     }
   }
-}
-
-template <int NT, int MT, int NW, int U>
-inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
-  g.rows = rows;
-  const unsigned parts = g.part > 0 ? (unsigned)((g.K + g.part - 1) / g.part) : 1u;
-  kernel<NT, MT, NW, U><<<dim3((unsigned)((g.N + rows - 1) / rows), parts), NW * 64, 0, st>>>(g);
 }
 
 // Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to nothing, and
@@ -167,56 +164,29 @@ inline void go(Args g, hipStream_t st, int rows = 16 * NT) {
 // ones (five rows 15360 x 1024 9.7 / 8.9).  Below K 512 a workgroup of its own for a few outputs costs more than idle CUs: whole tiles (768 x 256
 // 3.3 / 2.9).  The waves and so the order of a sum depend on M, N and K alone, not on who owns an output (8 waves of 4 steps instead of 4 of 8: N 2048 6.00 / 6.06
 // us, N 4096 7.16 / 7.26, not worth other results).
-inline void launch(const Args& g, hipStream_t st) {
-  const bool few = g.M <= 4 && g.N >= 6144;
+struct Form {
+  int nt, mt, nw, u, rows;
+};
+inline Form form_of(int M, int N, int K) {
+  const bool few = M <= 4 && N >= 6144;
   int rows;
-  if (g.K < 512) {
-    rows = few || g.N < 5120 ? 16 : g.M > 16 || g.N < 24576 ? 32 : 64;
+  if (K < 512) {
+    rows = few || N < 5120 ? 16 : M > 16 || N < 24576 ? 32 : 64;
   } else {
-    int tall = !few ? 64 : g.N > 16384 || g.K <= 2048 || (g.M <= 3 && g.N <= 8192 && g.K <= 3072) ? 16 : 32;  // rows of a workgroup at most
-    if (g.M <= 16 && g.N <= 16384) {
-      if (g.K % 8192 == 0 && g.N > (few ? 8192 : 12288)) tall /= 2;
-      else if (!few && g.K <= 1024 && g.N > 12288) tall = 32;
+    int tall = !few ? 64 : N > 16384 || K <= 2048 || (M <= 3 && N <= 8192 && K <= 3072) ? 16 : 32;  // rows of a workgroup at most
+    if (M <= 16 && N <= 16384) {
+      if (K % 8192 == 0 && N > (few ? 8192 : 12288)) tall /= 2;
+      else if (!few && K <= 1024 && N > 12288) tall = 32;
     }
-    const int rounds = (g.N + 256 * tall - 1) / (256 * tall);  // of 256 workgroups
-    rows = (g.N + 256 * rounds - 1) / (256 * rounds);
-    if (g.N > 16384) rows = few ? 16 : (rows + 3) / 4 * 4;  // (whole quads are stored at once)
+    const int rounds = (N + 256 * tall - 1) / (256 * tall);  // of 256 workgroups
+    rows = (N + 256 * rounds - 1) / (256 * rounds);
+    if (N > 16384) rows = few ? 16 : (rows + 3) / 4 * 4;  // (whole quads are stored at once)
   }
-  if (g.M > 16) {
-    if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
-    else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);
-    else if (rows <= 48) go<3, 2, 4, 4>(g, st, rows);
-    else go<4, 2, 4, 4>(g, st, rows);
-  } else if (rows <= 16) {
-    if (few) go<1, 1, 2, 8>(g, st, rows);
-    else go<1, 1, 4, 8>(g, st, rows);
-  } else if (rows <= 32) {
-    if (few) go<2, 1, 4, 4>(g, st, rows);
-    else go<2, 1, 4, 8>(g, st, rows);
-  } else if (rows <= 48) {
-    go<3, 1, 4, 4>(g, st, rows);
-  } else {
-    go<4, 1, 4, 4>(g, st, rows);
-  }
-}
-
-// K in ``parts`` ranges, each its own fp32 [M, N], for a reader that adds them: one round of 256 workgroups of at most 64 rows
-inline void launch_parts(Args g, int parts, hipStream_t st) {
-  g.part = ((g.K + parts - 1) / parts + 31) / 32 * 32;
-  g.f32 = 1;
-  const int n = (g.K + g.part - 1) / g.part;
-  const int rows = ((g.N * n + 255) / 256 + 3) / 4 * 4;
-  if (g.M > 16) {
-    if (rows <= 16) go<1, 2, 4, 8>(g, st, rows);
-    else if (rows <= 32) go<2, 2, 4, 4>(g, st, rows);
-    else go<4, 2, 4, 4>(g, st, rows > 64 ? 64 : rows);
-  } else if (rows <= 16) {
-    go<1, 1, 4, 8>(g, st, rows);
-  } else if (rows <= 32) {
-    go<2, 1, 4, 8>(g, st, rows);
-  } else {
-    go<4, 1, 4, 4>(g, st, rows > 64 ? 64 : rows);
-  }
+  const int nt = rows <= 16 ? 1 : rows <= 32 ? 2 : rows <= 48 ? 3 : 4;
+  if (M > 16) return {nt, 2, 4, nt == 1 ? 8 : 4, rows};
+  if (nt == 1) return {1, 1, few ? 2 : 4, 8, rows};
+  if (nt == 2) return {2, 1, 4, few ? 4 : 8, rows};
+  return {nt, 1, 4, 4, rows};
 }
 
 }  // namespace stream_linear

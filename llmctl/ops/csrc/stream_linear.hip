@@ -1,6 +1,6 @@
 // Projections of a few rows with their bias and activation in the same launch: see stream_linear.h.
 #include "common.h"
-#include "stream_linear.h"
+#include "stream_linear_launch.h"
 
 namespace llmctl {
 

@@ -24,7 +24,7 @@ import torch
 from . import ref_hybrid as ref
 from ._lib import native_hybrid, use_native
 from .functional import odd_linear as wide_linear
-from .functional import stream_ok, stream_takes, wants_grad
+from .functional import stream_ok, stream_pays, stream_takes, wants_grad
 
 
 def layernorm_f32(x, w, b, eps: float, out_dtype):
@@ -639,20 +639,42 @@ def experts_pay(T: int, top: int, E: int, rows: int, width: int) -> bool:
     return size < 7 << 23 or T * top // E * size < 7 << 34
 
 
+@functools.lru_cache(maxsize=4096)
+def _shared_rides(M: int, N: int, K: int, ff: int) -> bool:
+    return stream_pays(M, N, K) and stream_pays(M, K, ff) and native_hybrid().moe_shared_rides(M, N, K, ff)
+
+
+def shared_rides(x, w_sup, b_sup, cols: int, w_sdown, act: str) -> bool:
+    """Does a shared expert of these few rows (``act(x w_sup^T + b_sup)`` on its first ``cols`` columns, their product with ``w_sdown``) go into the
+    launches of :func:`routed_experts`?  Where :func:`rows_linear` would take both products in the one form that fits beside an expert's workgroup:
+    the sums and their order are the same."""
+    N, K = w_sup.shape
+    return (act in ("relu2", "gelu") and x.shape[0] <= 32 and (N | cols) & 7 == 0 and x.dim() == 2 and stream_takes(x, w_sup, b_sup)
+            and stream_takes(x, w_sdown) and _shared_rides(x.shape[0], N, K, cols))
+
+
 def routed_experts(x, w_router, bias, top: int, groups: int, keep: int, softmax: bool, renorm: bool, up, down, act: str, shared=None,
-                   gate=None, late: bool = False, routed=None):
+                   gate=None, late: bool = False, routed=None, ride=None):
     """``sum_k w_k expert_k(x_t)`` over the chosen experts of every row of ``x [T, W]`` (bf16) -> fp32 ``[T, W]``, all on the device:
     router (fp32 scores of the fp32 ``w_router [E, W]``; ``softmax``: :func:`bias_topk_router`'s choice, else
     :func:`group_topk_router`'s), copies grouped by expert, grouped products, weighted sum.  ``act``: ``relu2`` / ``gelu`` / ``swiglu``
     (``up`` holds ``[gate ; up]``).  Router outputs beyond the experts are experts that give their input.  ``shared [T, W]`` (times
     ``sigmoid(gate [T, 1])`` if given) is added.  ``late``: an :class:`ExpertSum` instead of the sum; ``routed``: the
-    choice and its weights, where the rows' norm has made them.  Operands: :func:`experts_ok`."""
+    choice and its weights, where the rows' norm has made them.  Operands: :func:`experts_ok`.  ``ride`` = ``(w_sup, b_sup, cols, w_sdown,
+    gated)``: the shared expert is computed here (:func:`shared_rides`; ``gated``: column ``cols`` of its first product is the gate) and the
+    result is ``(sum, first product)``."""
     nat = native_hybrid()
     idx, wgt = routed or nat.moe_route(x, w_router, bias, top, groups, keep, softmax, renorm)
     ups = expert_list(up)
-    rows = nat.moe_expert_rows(x, idx, wgt, ups, expert_list(down), _EXPERT_ACTS[act])
+    if ride is None:
+        rows = nat.moe_expert_rows(x, idx, wgt, ups, expert_list(down), _EXPERT_ACTS[act])
+    else:
+        w_sup, b_sup, cols, w_sdown, gated = ride
+        rows, z, shared = nat.moe_expert_rows_shared(x, idx, wgt, ups, expert_list(down), _EXPERT_ACTS[act], w_sup, b_sup, cols, w_sdown)
+        gate = z[:, cols:cols + 1] if gated else None
     out = ExpertSum(rows, idx, wgt, x, shared, gate, ups[0].shape[0] if ups[0].dim() == 3 else len(ups))
-    return out if late else out.total()
+    out = out if late else out.total()
+    return out if ride is None else (out, z)
 
 
 def act_any(x, kind: str, scale=None):
