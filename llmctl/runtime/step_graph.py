@@ -87,15 +87,26 @@ class StepGraph:
     def __init__(self, x: torch.Tensor, y: torch.Tensor):
         self.x, self.y = torch.empty_like(x, memory_format=torch.contiguous_format), torch.empty_like(y, memory_format=torch.contiguous_format)
         self.graph = self.loss = None
+        self.served = False  # the generator's tensors belong to graphs that were recorded in inference mode
+
+    def _begin(self, pool):
+        # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
+        for self.served in (False, True):
+            g = torch.cuda.CUDAGraph(keep_graph=True)
+            try:
+                with torch.inference_mode(self.served):  # (a graph writes the generator's seed as it begins and as it is replayed)
+                    g.capture_begin(pool=pool, capture_error_mode="thread_local")
+                return g
+            except RuntimeError as e:
+                if self.served or "nference" not in str(e):
+                    raise
 
     def capture(self, engine, denom: float, stream, pool) -> None:
         """Record.  Nothing runs, so a failure (raised) leaves the gradients as they were."""
         from llmctl.ops._lib import native
 
-        g = torch.cuda.CUDAGraph(keep_graph=True)
         with graph_capture_gc_guard(collect=False), torch.cuda.stream(stream):
-            # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
-            g.capture_begin(pool=pool, capture_error_mode="thread_local")
+            g = self._begin(pool)
             try:
                 loss = engine._gradients(self.x, self.y, denom)
             except BaseException:
@@ -116,7 +127,8 @@ class StepGraph:
     def run(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
         self.x.copy_(x)
         self.y.copy_(y)
-        self.graph.replay()
+        with torch.inference_mode(self.served):
+            self.graph.replay()
         return self.loss.clone()  # (the next replay writes the graph's own)
 
     def release(self) -> None:

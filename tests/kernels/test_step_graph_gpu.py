@@ -47,6 +47,21 @@ def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes, heads
         assert (x - y).norm() <= max(4 * (y - z).norm().item(), 2.0 ** -9 * y.norm().item())
 
 
+def test_recorded_beside_a_serving_graph(native_lib):
+    """A graph recorded in inference mode that is still there owns the generator's tensors: they are not written outside that mode."""
+    served = torch.cuda.CUDAGraph()
+    t = torch.zeros(8, device="cuda")
+    with torch.inference_mode():
+        t.add_(1)
+        with torch.cuda.graph(served):
+            t.add_(1)
+    eng, g = engine(), torch.Generator().manual_seed(4)
+    for _ in range(5):
+        assert torch.isfinite(eng.train_step([batch(eng, g, 2, 128)])["loss"])
+        served.replay()
+    assert len(eng.step_graphs.table) == 1
+
+
 def test_what_listens_is_heard(native_lib):
     """Hooks, modes and faults see every step; parameters that change storage or stop training are not replayed into."""
     eng, g = engine(), torch.Generator().manual_seed(2)
