@@ -107,6 +107,92 @@ def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] =
     return F.linear(x, w, b)
 
 
+@functools.lru_cache(maxsize=4096)
+def small_pays(layout: str, M: int, N: int, K: int, bias: bool = False) -> bool:
+    """Is ``gemm_small`` (csrc/gemm_small.hip) the fastest form of this product of a training step?  ``fwd``: M tokens, N outputs; ``dgrad``: K
+    outputs, N inputs; ``wgrad``: M outputs, N inputs, K tokens, ``bias``: and the bias's gradient, which else takes two launches more below 256
+    tokens.  Where the tiles of 32 are about one round of the chip; beyond that each operand is read too often.  us in a graph, the next best / here:
+    fwd 1024 tokens 512 x 256 5.8 / 5.5, 768 x 256 5.9 / 6.3; 200 768 x 768 7.5 / 6.1, 384 7.7 / 8.8; 64 768 x 3072 10.1 / 13.5; 512 1024 x 512 7.8 / 7.0;
+    dgrad 128 tokens 768 x 3072 10.1 / 8.2, 200 9.1 / 10.7, 512 768 x 768 12.9 / 8.4, 640 8.1 / 8.4; beyond K 1024 the 256-row tiles are what is left behind:
+    256 1408 x 256 12.8 / 8.0, 2304 x 768 16.2 / 11.1, 128 1536 x 512 8.2 / 8.7, 48 3072 x 768 9.1 / 11.7;
+    wgrad 4096 tokens 768 x 256 18.5 / 15.1, 1408 x 256 27.6 / 25.7, 1024 768 x 768 16.9 / 10.9, 128 2304 x 768 11.3 / 10.3, 256 9.2 / 10.7, 48 7.2 / 9.4;
+    with a bias 200 2304 x 768 13.5 / 10.5, 128 3072 x 768 15.9 / 14.2."""
+    w = -(-M // 32) * -(-N // 32)
+    if layout == "fwd":
+        return (w <= 256 and K <= 1024) or (w <= 512 and K <= 512)
+    if layout == "dgrad":
+        return (w <= 256 or (w <= 384 and K <= 1024) or (w <= 704 and K <= 256)) and (K <= 1024 or (K <= 3072 and M % 256 == 0))
+    return ((w <= 384 and K <= 4096) or (w <= 1024 and K <= 1024) or (w <= 1792 and 64 <= K <= 128)
+            or (bias and w <= 2304 and 64 <= K < 256))
+
+
+def _small_ok(layout: str, M: int, N: int, K: int, out_cols: Tuple[torch.Tensor, ...], *ts: torch.Tensor, bias: bool = False) -> bool:
+    """``small_pays``, and ``gemm_small`` takes the bf16 operands ``ts`` (``out_cols``: an output that is there already, bf16 or fp32).  Tensors of
+    a transform (vmap) and a backward that is differentiated itself stay with the library; so do sizes with a tuned gemm64 config."""
+    if not (M and K and small_pays(layout, M, N, K, bias)) or N % 8 or (layout == "wgrad" and M % 8) or (layout != "wgrad" and K % 8):
+        return False
+    if not _gemm64_enabled() or layout in GEMM64_CONFIGS or (layout, M, N, K) in GEMM64_SHAPE_CONFIGS:
+        return False
+    for t in ts + out_cols:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dim() != 2 or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                or torch._C._functorch.is_legacy_batchedtensor(t) or t.stride(0) < t.shape[1]):
+            return False
+    if any(t.dtype is not torch.bfloat16 for t in ts) or any(t.dtype not in (torch.bfloat16, torch.float32) for t in out_cols):
+        return False
+    from llmctl.ops._lib import use_native
+
+    return use_native(ts[0]) and _rows_ok(*ts, *out_cols)
+
+
+def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``x @ w^T (+ b)`` for the forward of an autograd function, on ``gemm_small`` where it takes it; else None."""
+    N, K = w.shape
+    M = x.numel() // K if K and x.shape[-1] == K else 0
+    if not M or not small_pays("fwd", M, N, K) or knobs().fwd64 == "off" or torch.is_autocast_enabled("cuda"):
+        return None
+    if type(x) is not torch.Tensor or torch._C._functorch.is_legacy_batchedtensor(x) or not x.is_contiguous():
+        return None
+    x2 = x.detach().view(M, K)
+    if not _small_ok("fwd", M, N, K, (), x2, w) or not (b is None or (b.dtype is torch.bfloat16 and b.is_cuda and b.is_contiguous() and b.shape == (N,)
+                                                                     and b.data_ptr() % 8 == 0)):
+        return None
+    from llmctl.ops._lib import native
+
+    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    native().gemm_small(x2, w, y, False, False, False, b)
+    return y.view(*x.shape[:-1], N)
+
+
+def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``dy2 @ w`` on ``gemm_small`` (into ``out``) where it takes it; else None.  Weights whose sink was made to keep W^T copies stay with them."""
+    M, (O, I) = dy2.shape[0], w.shape
+    if dy2.dim() != 2 or dy2.shape[1] != O or not small_pays("dgrad", M, I, O) or knobs().dgrad64 != "auto" or torch.is_grad_enabled():
+        return None
+    sink = getattr(w, "_llmctl_grad_sink", None)
+    if (sink is not None and sink.always_transpose) or not _small_ok("dgrad", M, I, O, () if out is None else (out,), dy2, w):
+        return None
+    from llmctl.ops._lib import native
+
+    dx = torch.empty(M, I, dtype=dy2.dtype, device=dy2.device) if out is None else out
+    native().gemm_small(dy2, w, dx, False, True, False)
+    return dx
+
+
+def small_wgrad(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: Optional[torch.Tensor] = None, add: bool = False) -> bool:
+    """``g (+)= dy2^T x2`` (and ``gb (+)= dy2.sum(0)``) on ``gemm_small`` where it takes them; False: nothing done."""
+    M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
+    if not small_pays("wgrad", M, N, K, gb is not None) or not knobs().wgrad_kernel or torch.is_grad_enabled():
+        return False
+    if not _small_ok("wgrad", M, N, K, (g,), dy2, x2, bias=gb is not None):
+        return False
+    if gb is not None and not (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == M):
+        return False
+    from llmctl.ops._lib import native
+
+    native().gemm_small(dy2, x2, g, True, True, accumulate, None, gb, add)
+    return True
+
+
 def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     """Will ``dx = dy W`` for ``tokens`` rows run on gemm64?  (Decided at forward time: the
     weight's W^T copy is only kept for layers whose data gradient cannot.)  ``fused``: the
@@ -224,6 +310,8 @@ def wgrad_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate:
     profiles/gemm64_variants_r2.jsonl; the 32-deep gemm_ex where K is not a multiple of 128);
     other shapes go to hipBLASLt."""
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
+    if small_wgrad(g, dy2, x2, accumulate):
+        return
     if g.dtype == torch.float32:  # fp32 main gradient: accumulate without a bf16 rounding
         if (_gemm64_ok(M, N, K, dy2, x2) and g.is_cuda and g.stride(1) == 1 and g.stride(0) % 4 == 0
                 and g.data_ptr() % 16 == 0 and K * dy2.stride(0) * 2 < 2**31 and K * x2.stride(0) * 2 < 2**31):
@@ -276,6 +364,8 @@ def wgrad_bias_into(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumu
     """``g (+)= dy2^T x2`` and ``gb (+)= dy2.sum(0)`` in one kernel where the 256 x 128 tiles take the weight gradient, over any number of tokens from 256 on
     (without ``gb`` where they are no multiple of 128); False: nothing done."""
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
+    if gb is not None and small_wgrad(g, dy2, x2, accumulate, gb, add):
+        return True
     if M % 256 or N % 256 or K < 256 or not dy2.is_cuda or not _bias_rides(M, N, K, gb is not None):  # (most refusals end here)
         return False
     if not (_gemm64_ok(M, N, 128, dy2, x2) and g.is_cuda and g.dtype in (torch.bfloat16, torch.float32)
@@ -492,7 +582,8 @@ class _Linear(torch.autograd.Function):
         ctx.wt = None
         if ctx.needs_input_grad[0] and weight_t_ok(x.numel() // x.shape[-1], w):
             ctx.wt = sink.weight_t(w)
-        return forward_linear(x, w, b)
+        y = small_linear(x, w, b)
+        return forward_linear(x, w, b) if y is None else y
 
     @staticmethod
     def backward(ctx, dy):
@@ -515,7 +606,10 @@ class _Linear(torch.autograd.Function):
             # an unsinked or tied weight keeps no W^T copy, so its alternative is hipBLASLt's slower "NN"
             # layout: gemm64 (W read K-major) whenever the shape fits, unless knob dgrad64 is off
             free = (getattr(ctx.wparam, "_llmctl_grad_sink", None) is None or _tied(ctx.wparam)) and knobs().dgrad64 != "off"
-            if dgrad64_ok(dy2, w) or (free and dy2.is_cuda and dy2.dtype == torch.bfloat16 and _rows_ok(dy2)
+            dx = small_dgrad(dy2, w) if ctx.wt is None else None
+            if dx is not None:
+                dx = dx.view(*dy.shape[:-1], w.shape[1])
+            elif dgrad64_ok(dy2, w) or (free and dy2.is_cuda and dy2.dtype == torch.bfloat16 and _rows_ok(dy2)
                                       and _gemm64_ok(dy2.shape[0], w.shape[1], w.shape[0], w)
                                       and w.shape[0] * w.stride(0) * 2 < 2**31):
                 dx = dgrad64(dy2, w).view(*dy.shape[:-1], w.shape[1])
@@ -583,6 +677,9 @@ def data_grad(dy: torch.Tensor, w: torch.nn.Parameter) -> torch.Tensor:
     """``dy @ w`` for hand-written backward passes: gemm64 when the shape fits, else through
     the weight's transposed copy when its sink keeps one."""
     dy2 = dy.reshape(-1, dy.shape[-1])
+    dx = small_dgrad(dy2, w)
+    if dx is not None:
+        return dx.view(*dy.shape[:-1], w.shape[1])
     if dgrad64_ok(dy2, w):
         return dgrad64(dy2, w).view(*dy.shape[:-1], w.shape[1])
     if dgrad64_part(dy2, w):
@@ -596,6 +693,8 @@ def data_grad(dy: torch.Tensor, w: torch.nn.Parameter) -> torch.Tensor:
 
 def data_grad_into(dy2: torch.Tensor, w: torch.nn.Parameter, out: torch.Tensor) -> None:
     """``out = dy2 @ w`` into a preallocated (row-slice) output: gemm64 writes it directly."""
+    if small_dgrad(dy2, w, out) is not None:
+        return
     if dgrad64_ok(dy2, w) and _rows_ok(out):
         from llmctl.ops._lib import native
 

@@ -84,12 +84,13 @@ class _SwiGLUDown(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, gu, w_down, recompute=False):
-        from llmctl.exec.linear import wgrad_swiglu_ok
+        from llmctl.exec.linear import small_linear, wgrad_swiglu_ok
         from llmctl.ops._lib import native, use_native
         from llmctl.ops import ref
 
         act = native().swiglu_fwd(gu) if use_native(gu) else ref.swiglu_fwd(gu)
-        out = F.linear(act, w_down)
+        out = small_linear(act, w_down)
+        out = F.linear(act, w_down) if out is None else out
         T = gu.numel() // gu.shape[-1]
         ctx.side = gu.requires_grad and wgrad_swiglu_ok(w_down, T, w_down.shape[1])
         if ctx.side:

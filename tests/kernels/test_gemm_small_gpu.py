@@ -1,0 +1,114 @@
+"""Products of few entries (csrc/gemm_small.hip) against 64 bits, and the training linear on them."""
+
+import importlib
+
+import pytest
+import torch
+
+from llmctl.ops._lib import native
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+L = importlib.import_module("llmctl.exec.linear")
+
+
+def _rows(R, C, pad, dtype=torch.bfloat16):
+    """[R, C] inside a larger tensor that is NaN around it."""
+    t = torch.full((R + 1, C + pad), float("nan"), device="cuda", dtype=dtype)
+    t[:R, :C] = torch.randn(R, C, device="cuda").to(dtype)
+    return t[:R, :C]
+
+
+def _check(got, want, mag, K):
+    # the output's rounding, and K + 8 fp32 additions of products that are exact
+    half = 2.0 ** -8 if got.dtype == torch.bfloat16 else 2.0 ** -23
+    assert ((got.double() - want).abs() <= half * want.abs() + (K + 16) * 2.0 ** -24 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("layout, M, N, K", [
+    ("fwd", 1, 8, 8), ("fwd", 33, 40, 72), ("fwd", 64, 64, 256), ("fwd", 100, 712, 704), ("fwd", 31, 32, 1024),
+    ("dgrad", 1, 8, 8), ("dgrad", 33, 40, 72), ("dgrad", 65, 256, 1408), ("dgrad", 100, 712, 1016), ("dgrad", 256, 24, 3072),
+    ("wgrad", 8, 8, 1), ("wgrad", 40, 72, 33), ("wgrad", 264, 256, 100), ("wgrad", 64, 32, 4096), ("wgrad", 768, 768, 71), ("wgrad", 1032, 568, 129)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_product_against_64_bits(layout, M, N, K, dtype):
+    torch.manual_seed(M + N + K)
+    at, bt = layout == "wgrad", layout != "fwd"
+    a = _rows(*((K, M) if at else (M, K)), 8)
+    b = _rows(*((K, N) if bt else (N, K)), 16)
+    ad, bd = (a.t() if at else a).double(), (b if bt else b.t()).double()
+    want, mag = ad @ bd, ad.abs() @ bd.abs()
+    out = _rows(M, N, 8, dtype)
+    keep = out.double()
+    native().gemm_small(a, b, out, at, bt, False)
+    _check(out, want, mag, K)
+    out.copy_(keep)
+    if at:
+        sums = torch.randn(M, device="cuda").to(dtype)
+        before = sums.double()
+        native().gemm_small(a, b, out, True, True, True, None, sums, True)
+        _check(sums, before + ad.sum(1), before.abs() + ad.abs().sum(1), K)
+        native().gemm_small(a, b, out, True, True, False, None, sums, False)
+        _check(sums, ad.sum(1), ad.abs().sum(1), K)
+    else:
+        bias = torch.randn(N, device="cuda").bfloat16()
+        native().gemm_small(a, b, out, at, bt, True, bias)
+        _check(out, want + keep + bias.double(), mag + keep.abs() + bias.double().abs(), K)
+
+
+@pytest.mark.parametrize("T, O, I, bias", [(96, 256, 704, False), (256, 768, 256, True), (130, 2304, 768, True), (200, 64, 64, True)])
+def test_training_linear(T, O, I, bias, monkeypatch):
+    """Sinked gradients, stored and added to, and ordinary ones: as 64 bits give them, on ``gemm_small``."""
+    torch.manual_seed(T)
+    x = torch.randn(2, T // 2, I, device="cuda").bfloat16().requires_grad_()
+    w = torch.nn.Parameter((torch.randn(O, I, device="cuda") * I ** -0.5).bfloat16())
+    b = torch.nn.Parameter(torch.randn(O, device="cuda").bfloat16()) if bias else None
+    dy = torch.randn(2, T // 2, O, device="cuda").bfloat16()
+    assert L.small_pays("wgrad", O, I, T, bias)
+    xd, wd, dyd = (t.detach().double() for t in (x, w, dy))
+    y = L.linear(x, w, b)
+    want = xd @ wd.t() + (b.detach().double() if bias else 0)
+    _check(y, want, xd.abs() @ wd.abs().t() + 4, I)
+    y.backward(dy)
+    _check(x.grad, dyd @ wd, dyd.abs() @ wd.abs(), O)
+    d2, x2 = dyd.flatten(0, 1), xd.flatten(0, 1)
+    _check(w.grad, d2.t() @ x2, d2.abs().t() @ x2.abs(), T)
+    sink = L.GradSink()
+    for p in (w, b):
+        if p is not None:
+            p.grad = torch.full_like(p, float("nan"))  # the first write stores
+            sink.attach(p)
+    for n in (1, 2):
+        x.grad = None
+        L.linear(x, w, b).backward(dy)
+        want, mag = n * (d2.t() @ x2), 3 * n * (d2.abs().t() @ x2.abs())
+        assert ((w.grad.double() - want).abs() <= n * 2.0 ** -8 * want.abs() + 2.0 ** -8 * (n - 1) * want.abs() + (T + 16) * 2.0 ** -24 * mag).all()
+        if bias:
+            want, mag = n * d2.sum(0), 3 * n * d2.abs().sum(0)
+            assert ((b.grad.double() - want).abs() <= 2 * n * 2.0 ** -8 * want.abs() + (T + 16) * 2.0 ** -24 * mag).all()
+
+
+def test_second_gradients_and_autocast_stay_with_the_library():
+    x = torch.randn(64, 64, device="cuda").bfloat16().requires_grad_()
+    w = torch.randn(64, 64, device="cuda").bfloat16()
+    y = L.linear(x, w)
+    dy = torch.randn_like(y).requires_grad_()
+    (dx,) = torch.autograd.grad(y, x, dy, create_graph=True)
+    (back,) = torch.autograd.grad(dx.float().sum(), dy)
+    assert torch.allclose(back.float(), w.float().sum(1).expand_as(back), atol=0.5)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert L.linear(x.detach(), w).dtype == torch.float16
+
+
+@pytest.mark.parametrize("bad", ["odd columns", "rows that are not aligned", "shapes", "type"])
+def test_refused_on_the_host(bad):
+    a, b = torch.randn(16, 64, device="cuda").bfloat16(), torch.randn(32, 64, device="cuda").bfloat16()
+    out = torch.empty(16, 32, device="cuda").bfloat16()
+    if bad == "odd columns":
+        b, out = b[:30], out[:, :30]
+    elif bad == "rows that are not aligned":
+        a = torch.randn(16, 68, device="cuda").bfloat16()[:, 4:]
+    elif bad == "shapes":
+        out = out[:8]
+    else:
+        a = a.float()
+    with pytest.raises(RuntimeError, match="gemm_small"):
+        native().gemm_small(a, b, out, False, False, False)
