@@ -90,10 +90,13 @@ def fwd64_pick(M: int, N: int, K: int) -> bool:
     return (N >= 16384 and M <= 8192) or (M <= 2048 and (N >= 8192 or K >= 8192))
 
 
-def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``x @ w^T (+ b)``: gemm64 for the shapes ``fwd64_pick`` selects, hipBLASLt otherwise."""
+def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, layout: str = "eager") -> torch.Tensor:
+    """``x @ w^T (+ b)``: small products on gemm_small (``small_pays``), gemm64 for the shapes ``fwd64_pick`` selects, hipBLASLt otherwise."""
     N, K = w.shape
     M = x.numel() // K if x.shape[-1] == K else 0
+    y = small_linear(x, w, b, layout) if w.is_cuda else None
+    if y is not None:
+        return y
     if M and fwd64_pick(M, N, K) and x.dtype == torch.bfloat16:
         x2 = x.reshape(M, K)
         if _gemm64_ok(M, N, K, x2, w) and 256 * x2.stride(0) * 2 < 2**31 and 256 * w.stride(0) * 2 < 2**31:
@@ -116,8 +119,12 @@ def small_pays(layout: str, M: int, N: int, K: int, bias: bool = False) -> bool:
     dgrad 128 tokens 768 x 3072 10.1 / 8.2, 200 9.1 / 10.7, 512 768 x 768 12.9 / 8.4, 640 8.1 / 8.4; beyond K 1024 the 256-row tiles are what is left behind:
     256 1408 x 256 12.8 / 8.0, 2304 x 768 16.2 / 11.1, 128 1536 x 512 8.2 / 8.7, 48 3072 x 768 9.1 / 11.7;
     wgrad 4096 tokens 768 x 256 18.5 / 15.1, 1408 x 256 27.6 / 25.7, 1024 768 x 768 16.9 / 10.9, 128 2304 x 768 11.3 / 10.3, 256 9.2 / 10.7, 48 7.2 / 9.4;
-    with a bias 200 2304 x 768 13.5 / 10.5, 128 3072 x 768 15.9 / 14.2."""
+    with a bias 200 2304 x 768 13.5 / 10.5, 128 3072 x 768 15.9 / 14.2.
+    ``eager``: the forward of a prompt, whose launches the host feeds one by one: a library product takes it 20 us, this 9, so every product of at most
+    some 16 us (gpt2-125m, a prompt of 100 tokens 2130 / 1400, of 300 2140 / 1400, of 800 2205 / 2035; the tiny model, 470 504 / 396)."""
     w = -(-M // 32) * -(-N // 32)
+    if layout == "eager":
+        return M > 32 and (K * -(-w // 256) <= 3072 if w <= 512 else K * -(-w // 1024) <= 1536)
     if layout == "fwd":
         return (w <= 256 and K <= 1024) or (w <= 512 and K <= 512)
     if layout == "dgrad":
@@ -126,41 +133,49 @@ def small_pays(layout: str, M: int, N: int, K: int, bias: bool = False) -> bool:
             or (bias and w <= 2304 and 64 <= K < 256))
 
 
-def _small_ok(layout: str, M: int, N: int, K: int, out_cols: Tuple[torch.Tensor, ...], *ts: torch.Tensor, bias: bool = False) -> bool:
-    """``small_pays``, and ``gemm_small`` takes the bf16 operands ``ts`` (``out_cols``: an output that is there already, bf16 or fp32).  Tensors of
-    a transform (vmap) and a backward that is differentiated itself stay with the library; so do sizes with a tuned gemm64 config."""
-    if not (M and K and small_pays(layout, M, N, K, bias)) or N % 8 or (layout == "wgrad" and M % 8) or (layout != "wgrad" and K % 8):
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+_is_wrapped, _is_legacy_batched = torch._C._functorch.is_functorch_wrapped_tensor, torch._C._functorch.is_legacy_batchedtensor
+
+
+def _small_operand(t: torch.Tensor, dtypes=(torch.bfloat16,)) -> bool:
+    """A matrix of aligned rows that ``gemm_small`` reads, and no tensor of a transform (vmap)."""
+    if type(t) not in _PLAIN or not t.is_cuda or t.dtype not in dtypes or t.dim() != 2 or _is_wrapped(t) or _is_legacy_batched(t):
         return False
-    if not _gemm64_enabled() or layout in GEMM64_CONFIGS or (layout, M, N, K) in GEMM64_SHAPE_CONFIGS:
-        return False
-    for t in ts + out_cols:
-        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda or t.dim() != 2 or torch._C._functorch.is_functorch_wrapped_tensor(t)
-                or torch._C._functorch.is_legacy_batchedtensor(t) or t.stride(0) < t.shape[1]):
-            return False
-    if any(t.dtype is not torch.bfloat16 for t in ts) or any(t.dtype not in (torch.bfloat16, torch.float32) for t in out_cols):
-        return False
+    st = t.stride()
+    return st[1] == 1 and st[0] & 7 == 0 and st[0] >= t.shape[1] and t.data_ptr() & 15 == 0
+
+
+def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
+    """``gemm_small`` takes operands of these sizes; sizes with a tuned gemm64 config stay with that."""
     from llmctl.ops._lib import use_native
 
-    return use_native(ts[0]) and _rows_ok(*ts, *out_cols)
+    return (M > 0 and K > 0 and N & 7 == 0 and ((M if layout == "wgrad" else K) & 7) == 0 and _gemm64_enabled()
+            and not (layout in GEMM64_CONFIGS or (layout, M, N, K) in GEMM64_SHAPE_CONFIGS)
+            and all(map(_small_operand, ts)) and use_native(ts[0]))
 
 
-def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``x @ w^T (+ b)`` for the forward of an autograd function, on ``gemm_small`` where it takes it; else None."""
+def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, layout: str = "fwd", act: int = 0) -> Optional[torch.Tensor]:
+    """``act(x @ w^T (+ b))`` on ``gemm_small`` where it takes it and no gradient is wanted of it (the forward of an autograd function, serving); else
+    None.  ``layout``: the rule of ``small_pays``; ``act``: as in csrc/stream_linear.h (0: none)."""
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    if not M or not small_pays("fwd", M, N, K) or knobs().fwd64 == "off" or torch.is_autocast_enabled("cuda"):
+    if not M or not small_pays(layout, M, N, K) or knobs().fwd64 == "off":
         return None
-    if type(x) is not torch.Tensor or torch._C._functorch.is_legacy_batchedtensor(x) or not x.is_contiguous():
+    if layout == "eager" and torch.cuda.is_current_stream_capturing() and not small_pays("fwd", M, N, K):
         return None
-    x2 = x.detach().view(M, K)
-    if not _small_ok("fwd", M, N, K, (), x2, w) or not (b is None or (b.dtype is torch.bfloat16 and b.is_cuda and b.is_contiguous() and b.shape == (N,)
-                                                                     and b.data_ptr() % 8 == 0)):
+    if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not x.is_contiguous() or torch.is_autocast_enabled("cuda")
+            or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
+            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
+        return None
+    x2 = x if x.dim() == 2 else x.view(M, K)
+    if not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (b.dtype is torch.bfloat16 and b.is_cuda and b.is_contiguous()
+                                                                  and b.shape == (N,) and b.data_ptr() & 7 == 0)):
         return None
     from llmctl.ops._lib import native
 
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
-    native().gemm_small(x2, w, y, False, False, False, b)
-    return y.view(*x.shape[:-1], N)
+    native().gemm_small(x2, w, y, False, False, False, b, None, False, act)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
 def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
@@ -169,7 +184,7 @@ def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] 
     if dy2.dim() != 2 or dy2.shape[1] != O or not small_pays("dgrad", M, I, O) or knobs().dgrad64 != "auto" or torch.is_grad_enabled():
         return None
     sink = getattr(w, "_llmctl_grad_sink", None)
-    if (sink is not None and sink.always_transpose) or not _small_ok("dgrad", M, I, O, () if out is None else (out,), dy2, w):
+    if (sink is not None and sink.always_transpose) or not _small_ok("dgrad", M, I, O, dy2, w, *(() if out is None else (out,))):
         return None
     from llmctl.ops._lib import native
 
@@ -183,7 +198,7 @@ def small_wgrad(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
     if not small_pays("wgrad", M, N, K, gb is not None) or not knobs().wgrad_kernel or torch.is_grad_enabled():
         return False
-    if not _small_ok("wgrad", M, N, K, (g,), dy2, x2, bias=gb is not None):
+    if not _small_ok("wgrad", M, N, K, dy2, x2) or not _small_operand(g, (torch.bfloat16, torch.float32)):
         return False
     if gb is not None and not (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == M):
         return False
@@ -582,8 +597,7 @@ class _Linear(torch.autograd.Function):
         ctx.wt = None
         if ctx.needs_input_grad[0] and weight_t_ok(x.numel() // x.shape[-1], w):
             ctx.wt = sink.weight_t(w)
-        y = small_linear(x, w, b)
-        return forward_linear(x, w, b) if y is None else y
+        return forward_linear(x, w, b, "fwd")
 
     @staticmethod
     def backward(ctx, dy):

@@ -215,7 +215,7 @@ class _UpSwiGLUDown(torch.autograd.Function):
         x2 = x.reshape(-1, x.shape[-1])
         T = x2.shape[0]
         gu, act = native().gemm64_up_swiglu(x2, w_up, gemm64_config("fwd", T, w_up.shape[0], x2.shape[1]) % 1000)
-        out = forward_linear(act, w_down)
+        out = forward_linear(act, w_down, layout="fwd")
         if ctx.needs_input_grad[0]:
             _prep_weight_t(w_up, T)
         # the SwiGLU backward as the down projection wgrad's side job (swiglu_bwd = side), as

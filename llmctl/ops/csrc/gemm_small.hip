@@ -15,6 +15,7 @@
 // The error against 64 bits is that of the output's rounding, as before.
 #include "common.h"
 #include "attn_common.h"
+#include "stream_linear.h"
 
 namespace llmctl {
 using namespace attn;
@@ -29,7 +30,7 @@ struct SmallGemm {
   const unsigned short* bias;  // not TA: nullptr or [N], added to every row
   void* sums;                  // TA: nullptr or [M] (+)= the sums of A over K, of c's type
   long lda, ldb, ldc;
-  int M, N, K, f32, add, add_sums, tiles_n;
+  int M, N, K, f32, add, add_sums, tiles_n, act;  // act (not TA): as in stream_linear.h, of the sum and the bias
 };
 
 __device__ __forceinline__ uint4 zero_or(const unsigned short* p, bool in) {
@@ -182,6 +183,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_small_kernel(SmallGemm g) {
       v[0] += __uint_as_float(x.x << 16), v[1] += __uint_as_float(x.x & 0xffff0000u);
       v[2] += __uint_as_float(x.y << 16), v[3] += __uint_as_float(x.y & 0xffff0000u);
     }
+    if (!TA && g.act != 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = stream_linear::activate(g.act, v[j]);
+    }
     if (g.f32) {
       f32x4_t* o = reinterpret_cast<f32x4_t*>(static_cast<float*>(g.c) + (long)row * g.ldc + col);
       *o = g.add ? *o + v : v;
@@ -213,15 +218,16 @@ __global__ __launch_bounds__(64 * NW) void gemm_small_kernel(SmallGemm g) {
 
 }  // namespace
 
-// out [M, N] (+)= A B^T (A [M, K], B [N, K]), A B (bt: B [K, N]) or A^T B (at and bt: A [K, M]); out bf16 or fp32.  N a multiple of 8, M where at, K where an operand
+// out [M, N] (+)= act(A B^T + bias) (A [M, K], B [N, K]), A B (bt: B [K, N]) or A^T B (at and bt: A [K, M]); out bf16 or fp32.  N a multiple of 8, M where at, K where an operand
 // runs along it; aligned rows.  bias bf16 [N] (not at); sums [M] (+)= the sums of A over K (at), of out's type.
 void gemm_small(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool bt, bool accumulate, const c10::optional<at::Tensor>& bias,
-                const c10::optional<at::Tensor>& sums, bool add_sums) {
+                const c10::optional<at::Tensor>& sums, bool add_sums, int64_t act) {
   LLMCTL_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2 && a.is_cuda() && b.is_cuda() && out.is_cuda(), "gemm_small: 2-D GPU operands");
   const bool f32 = out.scalar_type() == at::kFloat;
   LLMCTL_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && (f32 || out.scalar_type() == at::kBFloat16),
                "gemm_small: bf16 operands, bf16 or fp32 out");
-  LLMCTL_CHECK(!at_ || bt, "gemm_small: a transposed A goes with a transposed B");
+  LLMCTL_CHECK((!at_ || bt) && act >= 0 && act <= 3 && (act == 0 || (!at_ && !accumulate)),
+               "gemm_small: a transposed A goes with a transposed B, an activation (0 .. 3) with neither of A transposed and a sum");
   const long M = at_ ? a.size(1) : a.size(0), K = at_ ? a.size(0) : a.size(1), N = bt ? b.size(1) : b.size(0);
   LLMCTL_CHECK((bt ? b.size(0) : b.size(1)) == K && out.size(0) == M && out.size(1) == N, "gemm_small: shapes");
   LLMCTL_CHECK(N % 8 == 0 && (!at_ || M % 8 == 0) && (at_ || K % 8 == 0) && M < (1l << 24) && N < (1l << 24) && K < (1l << 24), "gemm_small: sizes in 8s");
@@ -238,13 +244,14 @@ void gemm_small(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool a
   if (M == 0 || N == 0) return;
   c10::DeviceGuard guard(a.device());
   auto ptr = [](const at::Tensor& t) { return reinterpret_cast<const unsigned short*>(t.data_ptr()); };
-  // Tiles of 32; a weight gradient of many reads its operands half as often in tiles of 64 (64 tokens 768 x 768 5.6 / 5.2 us, 2304 x 768 11.3 / 9.4; 512 x 256 3.8 / 5.1)
-  const long tile = at_ && (M + 31) / 32 * ((N + 31) / 32) > 512 ? 64 : 32;
+  // Tiles of 32; where they are many, tiles of 64 read the operands half as often (weight gradients of 64 tokens 768 x 768 5.6 / 5.2 us, 2304 x 768 11.3 / 9.4, 512 x
+  // 256 3.8 / 5.1; forward 640 tokens 2304 x 768 20.1 / 15.4, 768 x 768 8.8 / 9.7)
+  const long tile = (at_ || !bt) && (M + 31) / 32 * ((N + 31) / 32) > 512 ? 64 : 32;
   const int tiles_n = (int)((N + tile - 1) / tile);
   const long tiles = (M + tile - 1) / tile * tiles_n;
   LLMCTL_CHECK(tiles < (1l << 31), "gemm_small: too many tiles");
   SmallGemm g{ptr(a), ptr(b), out.data_ptr(), bias.has_value() ? ptr(*bias) : nullptr, sums.has_value() ? sums->data_ptr() : nullptr,
-              (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K, f32, accumulate, add_sums, tiles_n};
+              (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K, f32, accumulate, add_sums, tiles_n, (int)act};
   const dim3 grid((unsigned)tiles);
   const hipStream_t st = stream();
   if (at_) {
@@ -254,7 +261,8 @@ void gemm_small(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool a
     if (K >= 1024) gemm_small_kernel<false, true, 2, 4, 8><<<grid, 512, 0, st>>>(g);
     else gemm_small_kernel<false, true, 2, 4, 4><<<grid, 256, 0, st>>>(g);
   } else {
-    gemm_small_kernel<false, false, 2, 4, 4><<<grid, 256, 0, st>>>(g);
+    if (tile == 64) gemm_small_kernel<false, false, 4, 2, 4><<<grid, 256, 0, st>>>(g);
+    else gemm_small_kernel<false, false, 2, 4, 4><<<grid, 256, 0, st>>>(g);
   }
 }
 

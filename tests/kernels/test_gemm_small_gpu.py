@@ -112,3 +112,27 @@ def test_refused_on_the_host(bad):
         a = a.float()
     with pytest.raises(RuntimeError, match="gemm_small"):
         native().gemm_small(a, b, out, False, False, False)
+
+
+@pytest.mark.parametrize("M, N, K, act", [(33, 40, 72, None), (100, 2304, 768, None), (100, 3072, 768, "gelu"), (640, 2304, 768, "gelu"), (700, 712, 256, None)])
+def test_a_prompts_products(M, N, K, act, monkeypatch):
+    """Serving's products of more rows than a decode step's: one launch, activation included, against 64 bits."""
+    from llmctl import ops
+
+    torch.manual_seed(M)
+    x, w = torch.randn(M, K, device="cuda").bfloat16(), (torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16()
+    b = torch.randn(N, device="cuda").bfloat16()
+    assert L.small_pays("eager", M, N, K)
+    calls, small = [], L.small_linear
+    monkeypatch.setattr(L, "small_linear", lambda *a: calls.append(small(*a)) or calls[-1])
+    with torch.inference_mode():
+        got = ops.decode_linear(x, w, b, act=act)
+    assert calls and calls[0] is got
+    want = x.double() @ w.double().t() + b.double()
+    mag = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    if act is None:
+        _check(got, want, mag, K)
+        return
+    want = 0.5 * want * (1 + torch.tanh(0.7978845608028654 * (want + 0.044715 * want ** 3)))
+    # a gelu's slope is at most 1.13; its own fp32 steps: a few roundings of values up to |x| (1 + tanh)
+    assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1.13 * (K + 16) * 2.0 ** -24 * mag + 2.0 ** -20 * mag).all()
