@@ -208,6 +208,36 @@ def small_wgrad(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate
     return True
 
 
+def small_back(dy2: torch.Tensor, p: torch.nn.Parameter, w: torch.Tensor, x2: torch.Tensor,
+               b: Optional[torch.nn.Parameter] = None) -> Optional[torch.Tensor]:
+    """Both gradients of a sinked ``p`` (``w``: its values) and of its bias in one launch of ``gemm_small``'s tiles, where they take the two products and the weight's
+    are no more than a round or two: the weight's (and bias's) into the sink, ``dy2 @ w`` returned; None: nothing done.  256 tokens, a step of the tiny model 306 us in two launches a
+    layer's product, so 279."""
+    sink: Optional[GradSink] = getattr(p, "_llmctl_grad_sink", None)
+    T, (O, I) = dy2.shape[0], w.shape
+    if (sink is None or sink.always_transpose or dy2.dim() != 2 or dy2.shape[1] != O or x2.shape != (T, I) or -(-O // 32) * -(-I // 32) > 512
+            or not small_pays("dgrad", T, I, O) or not small_pays("wgrad", O, I, T) or torch.is_grad_enabled()
+            or knobs().dgrad64 != "auto" or not knobs().wgrad_kernel):
+        return None
+    gb, add = None, False
+    if b is not None:
+        if getattr(b, "_llmctl_grad_sink", None) is not sink:
+            return None
+        gb, add = sink.open(b)
+    g, more = sink.open(p)
+    if (not _small_ok("dgrad", T, I, O, dy2, w) or not _small_ok("wgrad", O, I, T, x2) or not _small_operand(g, (torch.bfloat16, torch.float32))
+            or not (gb is None or (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == O))):
+        return None
+    from llmctl.ops._lib import native
+
+    dx = torch.empty(T, I, dtype=dy2.dtype, device=dy2.device)
+    native().gemm_small_back(dy2, w, dx, x2, g, more, gb, add)
+    sink.close(p)
+    if b is not None:
+        sink.close(b)
+    return dx
+
+
 def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     """Will ``dx = dy W`` for ``tokens`` rows run on gemm64?  (Decided at forward time: the
     weight's W^T copy is only kept for layers whose data gradient cannot.)  ``fused``: the
@@ -606,6 +636,10 @@ class _Linear(torch.autograd.Function):
         x2 = x.reshape(-1, x.shape[-1])
         dw = None
         bias = ctx.bparam is not None and ctx.needs_input_grad[2]
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[1] and ctx.wt is None:
+            dx = small_back(dy2, ctx.wparam, w, x2, ctx.bparam if bias else None)
+            if dx is not None:
+                return dx.view(*dy.shape[:-1], w.shape[1]), None, None
         if ctx.needs_input_grad[1]:
             sink: Optional[GradSink] = getattr(ctx.wparam, "_llmctl_grad_sink", None)
             if sink is not None and bias and sink.write_with_bias(ctx.wparam, dy2, x2, ctx.bparam):

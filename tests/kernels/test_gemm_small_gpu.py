@@ -76,9 +76,13 @@ def test_training_linear(T, O, I, bias, monkeypatch):
         if p is not None:
             p.grad = torch.full_like(p, float("nan"))  # the first write stores
             sink.attach(p)
+    calls, back = [], L.small_back
+    monkeypatch.setattr(L, "small_back", lambda *a: calls.append(back(*a)) or calls[-1])
     for n in (1, 2):
         x.grad = None
         L.linear(x, w, b).backward(dy)
+        assert (calls[-1] is not None) == (O * I < 1024 * 513)  # both products in one launch
+        _check(x.grad, dyd @ wd, dyd.abs() @ wd.abs(), O)
         want, mag = n * (d2.t() @ x2), 3 * n * (d2.abs().t() @ x2.abs())
         assert ((w.grad.double() - want).abs() <= n * 2.0 ** -8 * want.abs() + 2.0 ** -8 * (n - 1) * want.abs() + (T + 16) * 2.0 ** -24 * mag).all()
         if bias:
