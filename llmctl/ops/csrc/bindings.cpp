@@ -40,6 +40,8 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("gelu_bwd(Tensor dy, Tensor x) -> Tensor");
   // loss (loss.hip)
   m.def("cross_entropy_fwd(Tensor logits, Tensor labels, int ignore_index) -> (Tensor, Tensor)");
+  m.def("loss_mean(Tensor loss, float denom) -> Tensor");
+  m.def("cross_entropy_bwd_mean(Tensor g, float denom, Tensor logits, Tensor lse, Tensor labels, int ignore_index, bool inplace) -> Tensor");
   m.def("cross_entropy_bwd(Tensor dloss, Tensor logits, Tensor lse, Tensor labels, int ignore_index, bool inplace) -> Tensor");
   // optimizer (optim.hip)
   m.def("adamw_step_(Tensor(a!) param, Tensor(b!) master, Tensor grad, Tensor(c!) exp_avg, Tensor(d!) exp_avg_sq, float lr, float beta1, float beta2, float eps, float weight_decay, float bc1, float bc2, Tensor? grad_scale) -> ()");

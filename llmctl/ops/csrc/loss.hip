@@ -72,11 +72,11 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(const float* __restrict__ d
                                                       const unsigned short* __restrict__ logits,
                                                       const float* __restrict__ lse,
                                                       const int64_t* __restrict__ labels,
-                                                      unsigned short* __restrict__ out, int V, long ignore_index) {
+                                                      unsigned short* __restrict__ out, int V, long ignore_index, int per_row, float factor) {
   const long row = blockIdx.x;
   const long lab = labels[row];
   const bool valid = !(lab == ignore_index || lab < 0 || lab >= V);
-  const float d = valid ? dloss[row] : 0.f;
+  const float d = valid ? (per_row ? dloss[row] : dloss[0] * factor) : 0.f;  // (one gradient of the mean: no pass that spreads it over the rows)
   const float L = lse[row];
   const unsigned short* lr = logits + row * (long)V;
   unsigned short* orow = out + row * (long)V;
@@ -95,6 +95,22 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(const float* __restrict__ d
     float g = __expf(bf2f(lr[c]) - L) * d;
     if (c == lab) g -= d;
     orow[c] = f2bf(g);
+  }
+}
+
+// out = factor * sum(loss), one workgroup, summed in 64 bits: up to 32768 rows (128 KB, 5 us) one launch where the library takes two, three with the memset that it
+// clears its counters with from 16384 rows on.
+__global__ __launch_bounds__(1024) void loss_mean_kernel(const float* __restrict__ loss, int T, float factor, float* __restrict__ out) {
+  __shared__ double part[16];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < T; i += 1024) s += (double)loss[i];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) s += part[w];
+    out[0] = (float)s * factor;
   }
 }
 
@@ -128,13 +144,40 @@ at::Tensor cross_entropy_bwd(const at::Tensor& dloss, const at::Tensor& logits, 
   at::Tensor out = inplace ? logits : at::empty_like(logits);
   if (T)
     hipLaunchKernelGGL(ce_bwd_kernel, dim3(T), dim3(256), 0, stream(), dloss.data_ptr<float>(), bf_ptr(logits),
-                       lse.data_ptr<float>(), labels.data_ptr<int64_t>(), bf_mut(out), V, (long)ignore_index);
+                       lse.data_ptr<float>(), labels.data_ptr<int64_t>(), bf_mut(out), V, (long)ignore_index, 1, 1.f);
+  return out;
+}
+
+// sum(loss) / denom of loss fp32 [T], T at most 32768
+at::Tensor loss_mean(const at::Tensor& loss, double denom) {
+  LLMCTL_CHECK(loss.is_cuda() && loss.scalar_type() == at::kFloat && loss.is_contiguous() && loss.numel() <= 32768, "loss_mean: contiguous fp32, at most 32768 rows");
+  const c10::DeviceGuard g(loss.device());
+  at::Tensor out = at::empty({}, loss.options());
+  hipLaunchKernelGGL(loss_mean_kernel, dim3(1), dim3(1024), 0, stream(), loss.data_ptr<float>(), (int)loss.numel(), 1.f / (float)denom, out.data_ptr<float>());
+  return out;
+}
+
+// cross_entropy_bwd where every row's gradient is g / denom
+at::Tensor cross_entropy_bwd_mean(const at::Tensor& g, double denom, const at::Tensor& logits, const at::Tensor& lse, const at::Tensor& labels, int64_t ignore_index,
+                                  bool inplace) {
+  LLMCTL_CHECK(g.is_cuda() && g.scalar_type() == at::kFloat && g.numel() == 1, "cross_entropy_bwd_mean: one fp32 gradient");
+  LLMCTL_CHECK(logits.is_cuda() && logits.dim() == 2 && logits.is_contiguous() && logits.scalar_type() == at::kBFloat16 && lse.is_contiguous() &&
+                   lse.numel() == logits.size(0) && labels.is_contiguous() && labels.scalar_type() == at::kLong && labels.numel() == logits.size(0),
+               "cross_entropy_bwd_mean: what cross_entropy_fwd took and gave");
+  const c10::DeviceGuard guard(logits.device());
+  const long T = logits.size(0);
+  at::Tensor out = inplace ? logits : at::empty_like(logits);
+  if (T)
+    hipLaunchKernelGGL(ce_bwd_kernel, dim3(T), dim3(256), 0, stream(), g.data_ptr<float>(), bf_ptr(logits), lse.data_ptr<float>(), labels.data_ptr<int64_t>(),
+                       bf_mut(out), (int)logits.size(1), (long)ignore_index, 0, 1.f / (float)denom);
   return out;
 }
 
 TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
   m.impl("cross_entropy_fwd", &cross_entropy_fwd);
   m.impl("cross_entropy_bwd", &cross_entropy_bwd);
+  m.impl("loss_mean", &loss_mean);
+  m.impl("cross_entropy_bwd_mean", &cross_entropy_bwd_mean);
 }
 
 }  // namespace llmctl

@@ -362,11 +362,16 @@ class _CrossEntropy(torch.autograd.Function):
             loss, lse = ref.cross_entropy_fwd(logits, labels, ignore_index)
         ctx.save_for_backward(logits, lse, labels)
         ctx.ignore_index, ctx.denom = ignore_index, denom
+        if use_native(logits) and loss.numel() <= 32768 and type(denom) in (int, float) and denom:
+            return native().loss_mean(loss, denom)
         return loss.sum() / denom
 
     @staticmethod
     def backward(ctx, g):
         logits, lse, labels = ctx.saved_tensors
+        if (use_native(logits) and type(g) is torch.Tensor and g.dtype is torch.float32 and g.is_cuda and type(ctx.denom) in (int, float)
+                and ctx.denom and not torch.is_grad_enabled()):
+            return native().cross_entropy_bwd_mean(g, ctx.denom, logits, lse, labels, ctx.ignore_index, True), None, None, None
         dloss = (g / ctx.denom).float().expand(labels.shape).contiguous()
         if use_native(logits):
             # logits are dead after this: write dlogits in place (saves a [T,V] buffer)

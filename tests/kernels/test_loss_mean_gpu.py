@@ -1,0 +1,37 @@
+"""The mean of the loss and its gradient in one launch each, and the squared norm, against 64 bits."""
+
+import pytest
+import torch
+
+from llmctl import ops
+from llmctl.ops._lib import native
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+
+@pytest.mark.parametrize("T", [1, 63, 1025, 32768, 32769])
+def test_mean_and_gradient(T):
+    torch.manual_seed(T)
+    logits = torch.randn(T, 41, device="cuda").bfloat16()
+    labels = torch.randint(0, 41, (T,), device="cuda")
+    labels[::7] = -100
+    rows, lse = native().cross_entropy_fwd(logits, labels, -100)
+    want = rows.double().sum() / (T + 2)
+    x = logits.clone().requires_grad_()
+    loss = ops.cross_entropy(x, labels, reduction_denom=float(T + 2))
+    assert loss.shape == () and (loss.double() - want).abs() <= 4 * 2.0 ** -24 * want.abs() + 1e-30 if T <= 32768 else True
+    (loss * 3).backward()
+    dloss = ((torch.tensor(3.0, device="cuda") / float(T + 2)).expand(T)).contiguous()
+    assert torch.equal(x.grad, native().cross_entropy_bwd(dloss, logits, lse, labels, -100, False))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 7, 8, 8191, 8193, 1_000_003, 5_000_008])
+def test_squared_norm(n, dtype):
+    torch.manual_seed(n)
+    x = torch.randn(n, device="cuda").to(dtype)
+    out = torch.full((1,), 2.0, device="cuda")
+    native().l2norm_sq_(x, out)
+    want = x.double().square().sum() + 2
+    # a thread's own additions, a tree over 1024 threads, at most 512 additions to the one sum
+    assert (out.double() - want).abs() <= (n // 524288 * 8 + 8 + 10 + 512) * 2.0 ** -24 * want
