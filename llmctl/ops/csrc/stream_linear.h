@@ -60,101 +60,10 @@ __device__ __forceinline__ float activate(int act, float v) {
 // A workgroup of NW waves owns ``rows`` weight rows, at most 16 NT; the waves split K.  A lane streams 16 bytes of its weight row per 32-deep step,
 // U steps in flight before the first MFMA; the weight fragment is the MFMA row operand, so a lane ends up with four
 // neighbouring outputs of one token.  K is a multiple of 8 (the last step is filled up with zeros), N any.
-// Workgroup (bx, by); red: LDS for the waves' sums.
+// Workgroup (bx, by) of a launch that does other things too; red: LDS for the waves' sums.
 template <int NT, int MT, int NW, int U>
 __device__ __forceinline__ void workgroup(Args g, unsigned bx, unsigned by, acc_t (*red)[NT * MT][64]) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r = lane & 15, kg = lane >> 4;
-  if (g.part > 0) {
-    const int k0 = by * g.part;
-    g.x += k0;
-    g.w += k0;
-    g.K = min(g.part, g.K - k0);
-    g.y = static_cast<float*>(g.y) + (long)by * g.M * g.N;
-  }
-  const int n0 = bx * g.rows, n1 = min(n0 + g.rows, g.N);
-  const unsigned short* wp[NT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n) wp[n] = g.w + (long)min(n0 + n * 16 + r, n1 - 1) * g.ldw + 8 * kg;
-  const unsigned short* xp[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) xp[m] = g.x + (long)min(m * 16 + r, g.M - 1) * g.ldx + 8 * kg;
-  acc_t acc[NT][MT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[n][m] = acc_t{0.f, 0.f, 0.f, 0.f};
-  const int steps = (g.K + 31) / 32, per = (steps + NW - 1) / NW;
-  const int s0 = wave * per, s1 = min(s0 + per, steps), whole = min(s1, g.K / 32);
-  for (int s = s0; s < s1; s += U) {
-    uint4 wv[U][NT], xv[U][MT];
-    if (s + U <= whole) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int n = 0; n < NT; ++n) wv[u][n] = *reinterpret_cast<const uint4*>(wp[n] + (s + u) * 32);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) xv[u][m] = *reinterpret_cast<const uint4*>(xp[m] + (s + u) * 32);
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const bool in = s + u < s1 && (s + u) * 32 + 8 * kg < g.K;
-#pragma unroll
-        for (int n = 0; n < NT; ++n) wv[u][n] = load_or_zero(wp[n] + (s + u) * 32, in);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) xv[u][m] = load_or_zero(xp[m] + (s + u) * 32, in);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // the whole batch in flight before the first MFMA
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(frag_t, wv[u][n]), __builtin_bit_cast(frag_t, xv[u][m]),
-                                                              acc[n][m], 0, 0, 0);
-  }
-#pragma unroll
-  for (int n = 0; n < NT; ++n)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) red[wave][n * MT + m][lane] = acc[n][m];
-  __syncthreads();
-  for (int i = tid; i < NT * MT * 64; i += NW * 64) {
-    const int t = i >> 6, l = i & 63, row = (t % MT) * 16 + (l & 15), c = n0 + (t / MT) * 16 + 4 * (l >> 4);
-    if (row >= g.M || c >= n1) continue;
-    acc_t s = red[0][t][l];
-#pragma unroll
-    for (int v = 1; v < NW; ++v) s += red[v][t][l];
-    const long o = (long)row * g.N + c;
-    const int left = min(4, n1 - c);
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float b = g.bias != nullptr && j < left ? __uint_as_float((unsigned)g.bias[c + j] << 16) : 0.f;
-      v[j] = activate(c + j < g.act_cols ? g.act : 0, s[j] + b);
-    }
-    if (g.f32) {
-      float* y = static_cast<float*>(g.y) + o;
-      if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) *reinterpret_cast<float4*>(y) = make_float4(v[0], v[1], v[2], v[3]);
-      else
-#pragma unroll  // (a loop of ``left`` turns would index the values by a register: through LDS, 8256 x 2048 24 us for 11.5)
-        for (int j = 0; j < 4; ++j)
-          if (j < left) y[j] = v[j];
-    } else {
-      unsigned short* y = static_cast<unsigned short*>(g.y) + o;
-      unsigned short h[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) h[j] = __bfloat16_as_ushort(__float2bfloat16(v[j]));
-      if (left == 4 && (reinterpret_cast<uintptr_t>(y) & 7) == 0) *reinterpret_cast<uint2*>(y) = make_uint2(h[0] | ((unsigned)h[1] << 16), h[2] | ((unsigned)h[3] << 16));
-      else
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (j < left) y[j] = h[j];
-    }
-  }
+#include "stream_linear_body.inc"
 }
 
 // Weight rows per workgroup: one round of 256 workgroups where they own at most 64 rows each, else even rounds.  Up to four rows of x cost next to nothing, and

@@ -7,7 +7,8 @@ namespace stream_linear {
 template <int NT, int MT, int NW, int U>
 __global__ __launch_bounds__(NW * 64) void kernel(Args g) {
   __shared__ acc_t red[NW][NT * MT][64];
-  workgroup<NT, MT, NW, U>(g, blockIdx.x, blockIdx.y, red);
+  const auto &bx = blockIdx.x, &by = blockIdx.y;
+#include "stream_linear_body.inc"
 }
 
 template <int NT, int MT, int NW, int U>
