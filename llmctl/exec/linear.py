@@ -94,9 +94,10 @@ def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] =
     """``x @ w^T (+ b)``: small products on gemm_small (``small_pays``), gemm64 for the shapes ``fwd64_pick`` selects, hipBLASLt otherwise."""
     N, K = w.shape
     M = x.numel() // K if x.shape[-1] == K else 0
-    y = small_linear(x, w, b, layout) if w.is_cuda else None
-    if y is not None:
-        return y
+    if M > 32 or layout != "eager":
+        y = small_linear(x, w, b, layout)
+        if y is not None:
+            return y
     if M and fwd64_pick(M, N, K) and x.dtype == torch.bfloat16:
         x2 = x.reshape(M, K)
         if _gemm64_ok(M, N, K, x2, w) and 256 * x2.stride(0) * 2 < 2**31 and 256 * w.stride(0) * 2 < 2**31:
@@ -159,7 +160,7 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
     None.  ``layout``: the rule of ``small_pays``; ``act``: as in csrc/stream_linear.h (0: none)."""
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    if not M or not small_pays(layout, M, N, K) or knobs().fwd64 == "off":
+    if not M or not small_pays(layout, M, N, K) or not w.is_cuda or knobs().fwd64 == "off":
         return None
     if layout == "eager" and torch.cuda.is_current_stream_capturing() and not small_pays("fwd", M, N, K):
         return None

@@ -663,7 +663,7 @@ def decode_linear(x, w, b=None, act: Optional[str] = None):
         form = "stream"  # (the activation pass takes multiples of 8)
     if y is None and form == "stream" and x.dim() == 2 and stream_takes(x, w, b):
         return native().stream_linear(x, w, b, _ROW_ACTS[act])
-    if y is None and act == "gelu":
+    if y is None and act == "gelu" and M > 32:
         y = small_linear(x, w, b, "eager", _ROW_ACTS[act])
         if y is not None:
             return y
