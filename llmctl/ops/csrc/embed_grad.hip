@@ -1,6 +1,7 @@
 // Gradient of an embedding table: g[v] (+)= the sum of dy's rows whose token is v.
 //
-// Bound: one pass over dy and the rows of g that it meets (8192 x 4096: 134 MB, 27 us at a copy's rate).  Three launches, no atomics, the same bits every time:
+// Bound: one pass over dy and the rows of g that it meets (8192 x 4096: 134 MB, 27 us at a copy's rate).  Three launches (one for few tokens), no atomics, the same bits
+// every time:
 //   order  the tokens ranked by (id, position): ids in LDS, every wave counts for two tokens the ids below and the equal ones before and in all.  T^2 compares,
 //          four a lane and read; 65536 tokens are the most that is taken here, and of narrow rows fewer pay (embed_grad_pays); a radix sort is five launches.
 //   rows   a wave per 8 sorted tokens and 512 columns, all loads in flight; a run of one id inside the 8 is final, a run across an edge leaves a partial row
@@ -8,13 +9,15 @@
 // so a token that fills half the batch is summed by as many waves as any other half.
 // Measured on one MI355X, us, against the library's (sort, segments, scatter into a dense gradient that is then added), ids drawn evenly / all the same:
 // 8192 x 768 into 50304 rows 29.4 / 109 (141 / 329), 8192 x 4096 into 32000 49.7 / 200 (468 / 555), 24576 x 4096 230 / 434 (947 / 1179), 65536 x 4096
-// 1011 / 1939 (1495 / 3232), 256 x 64 into 256 12.5 / 12.5 (18.5 / 26); ids drawn as 1 / rank, 8192 x 768 into 50304 47 (152),
+// 1011 / 1939 (1495 / 3232), 256 x 256 into 512 3.8 / 7.5 (256 x 64 18.5 / 26); ids drawn as 1 / rank, 8192 x 768 into 50304 47 (152),
 // 8192 x 4096 into 32000 103 (451).  16 tokens a wave: 40.8, 75, 283, 1091, 17.3, and less only where most tokens are the
 // same (72, 104, 406, 1538, 16): a wave adds to the rows of its ids one after the other.
 #include "common.h"
 
 namespace llmctl {
 namespace {
+constexpr int FEW_IDS = 384;  // tokens of one launch: 256 tokens 50304 x 768, ids drawn evenly / half of them the same / all, 11.1 / 12.9 / 12.0 us in three, so 3.8 / 6.0 / 8.3; 512 of 4096 11.7 / 14.8 / 16.5, so
+// 10.3 / 11.9 / 17.8
 constexpr int RUN = 8, ORDER_IDS = 16384, ORDER_WAVES = 16;
 
 struct EmbedGradArgs {
@@ -152,6 +155,61 @@ __global__ __launch_bounds__(256) void embed_edges_kernel(EmbedGradArgs a) {
   for (int i = k + 1; i <= k1; ++i) take(2L * i, false);
   put_row<G>(a, id, c, v);
 }
+// Few tokens, one launch: a workgroup per token and 512 columns, ids in LDS; that of an id's first token sums its rows, every wave a quarter of the places, up to
+// sixteen rows in flight, in eights (as the three launches do).
+template <typename G>
+__global__ __launch_bounds__(256) void embed_few_kernel(EmbedGradArgs a) {
+  __shared__ int s[FEW_IDS];
+  __shared__ __attribute__((aligned(16))) float part[3][64][8];
+  const int T = a.T, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t = blockIdx.x;
+  for (int i = threadIdx.x; i < T; i += 256) s[i] = (int)a.ids[i];
+  __syncthreads();
+  const int id = s[t], c = (blockIdx.y * 64 + lane) * 8, cl = min(c, a.H - 8);
+  for (int b = 0; b < t; b += 64)
+    if (__ballot(b + lane < t && s[min(b + lane, T - 1)] == id)) return;  // (all waves of the workgroup)
+  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int b = 64 * wave; b < T; b += 256) {
+    unsigned long long m = __ballot(b + lane >= t && b + lane < T && s[min(b + lane, T - 1)] == id);
+    while (m) {
+      uint4 row[16];
+      int n = 0;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        row[i] = make_uint4(0, 0, 0, 0);
+        if (m) {
+          row[i] = *reinterpret_cast<const uint4*>(a.dy + (long)(b + __builtin_ctzll(m)) * a.dy_ld + cl);
+          m &= m - 1;
+          ++n;
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (8 * h >= n) break;
+        float w[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 8 * h; i < 8 * h + 8; ++i) {
+          if (i >= n) break;
+          const unsigned u[4] = {row[i].x, row[i].y, row[i].z, row[i].w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[2 * j] += bf2f(u[j] & 0xffff), w[2 * j + 1] += bf2f(u[j] >> 16);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] += w[j];
+      }
+    }
+  }
+  if (wave > 0) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) part[wave - 1][lane][j] = v[j];
+  }
+  __syncthreads();
+  if (wave > 0 || c >= a.H) return;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += part[k][lane][j];
+  put_row<G>(a, id, c, v);
+}
 }  // namespace
 
 // g [V, H] (+)= the rows of dy [T, H] by their ids; without add, g's other rows are left as they are (the caller zeroes them)
@@ -167,6 +225,14 @@ void embed_grad_(const at::Tensor& ids, const at::Tensor& dy, at::Tensor g, bool
   LLMCTL_CHECK(H % 8 == 0 && T <= 65536, "embed_grad: H in 8s, at most 65536 tokens");
   if (T == 0 || H == 0) return;
   const c10::DeviceGuard guard(dy.device());
+  if (T <= FEW_IDS) {
+    const EmbedGradArgs a{ids.data_ptr<int64_t>(), bf_ptr(dy), g.data_ptr(), nullptr, nullptr, nullptr, nullptr, (long)dy.stride(0), (long)g.size(0), (int)T, (int)H,
+                          add};
+    const dim3 few((unsigned)T, (unsigned)((H / 8 + 63) / 64));
+    if (g.scalar_type() == at::kFloat) hipLaunchKernelGGL(embed_few_kernel<float>, few, dim3(256), 0, stream(), a);
+    else hipLaunchKernelGGL(embed_few_kernel<unsigned short>, few, dim3(256), 0, stream(), a);
+    return;
+  }
   const int chunks = (int)((T + RUN - 1) / RUN);
   auto order = at::empty({3, T}, ids.options().dtype(at::kInt));
   auto part = at::empty({chunks, 2, H}, dy.options().dtype(at::kFloat));

@@ -101,3 +101,24 @@ def test_many_tokens_of_narrow_rows(T, H, V, dtype, tokens, monkeypatch):
         # fp32 sums, and for a bf16 gradient the rounding of each write of it
         err = err + (T + 1) * 2.0**-24 * mag + (2.0**-8 * ref.abs() if dtype == torch.bfloat16 else 0.0)
     assert bool(((flat.double() - ref).abs() <= err * (1 + 2.0**-7) + 1e-30).all())
+
+
+@pytest.mark.parametrize("T", [2, 63, 64, 65, 255, 257, 384, 385])
+@pytest.mark.parametrize("kind", ["same", "distinct", "skewed"])
+@pytest.mark.parametrize("H", [8, 520])
+def test_few_tokens(T, kind, H):
+    """The one launch of few tokens and the three of more: places at the edges of a wave's 64 and of the line between them."""
+    from llmctl import ops
+
+    V = 700
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    ids = _ids(kind, T, V, g)
+    dy = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    out = torch.randn(V, H, generator=g, device="cuda")
+    ref = out.double()
+    mag = ref.abs()
+    ref.index_add_(0, ids, dy.double())
+    mag.index_add_(0, ids, dy.double().abs())
+    ops.embed_grad_(ids, dy, out, True)
+    n = torch.bincount(ids, minlength=V).max().item()
+    assert bool(((out.double() - ref).abs() <= (n + 1) * 2.0 ** -24 * mag).all())
