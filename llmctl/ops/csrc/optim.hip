@@ -86,29 +86,37 @@ __global__ __launch_bounds__(256) void adamw_kernel(unsigned short* __restrict__
 }
 
 // Bound: the read (5 TB/s), and for a small model the adds to one address, some 10 ns each: 1024 threads to one of them, at most 512.  us, 256 threads and 2048 / so:
-// 1.7 million bf16 entries 14.6 / 6.8, 10 million 31.4 / 12.2, 124 million 80.5 / 70.2, with the events around them.
+// 1.7 million bf16 entries 14.6 / 7.0, 10 million 31.4 / 12.3, 124 million 80.5 / 71.1, with the events around them.  Off 64 bits by 3.7e-7 at 550 million (2.6e-6 with
+// 32-bit sums).
 template <typename T>
 __global__ __launch_bounds__(1024) void sumsq_kernel(const T* __restrict__ x, long n, float* __restrict__ out) {
-  __shared__ float sm[16];
-  float s = 0.f;
+  __shared__ double sm[16];
+  double s = 0.0;  // (of eights in 32 bits: a thread of a large model adds a thousand squares)
   const long n8 = n >> 3;
   const long stride = (long)gridDim.x * 1024;
   for (long i = (long)blockIdx.x * 1024 + threadIdx.x; i < n8; i += stride) {
-    float v[8];
+    float v[8], q = 0.f;
     load_grad8<T>(x + i * 8, v);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += v[j] * v[j];
+    for (int j = 0; j < 8; ++j) q += v[j] * v[j];
+    s += (double)q;
   }
   if (blockIdx.x == 0) {
     for (long o = n8 * 8 + threadIdx.x; o < n; o += 1024) {
       float v;
       if constexpr (sizeof(T) == 2) v = bf2f(((const unsigned short*)x)[o]);
       else v = ((const float*)x)[o];
-      s += v * v;
+      s += (double)(v * v);
     }
   }
-  const float r = block_sum<16>(s, sm);
-  if (threadIdx.x == 0) atomicAdd(out, r);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) s += sm[w];
+    atomicAdd(out, (float)s);
+  }
 }
 
 // The end of the clip norm, one thread: norm = sqrt(nsq) / divisor, the factor min(1, max_norm / (norm + 1e-6)) / divisor (1 / divisor
