@@ -160,7 +160,7 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
     None.  ``layout``: the rule of ``small_pays``; ``act``: as in csrc/stream_linear.h (0: none)."""
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    if not M or not small_pays(layout, M, N, K) or not w.is_cuda or knobs().fwd64 == "off":
+    if not M or not small_pays(layout, M, N, K) or not w.is_cuda or knobs().fwd64 != "auto":
         return None
     if layout == "eager" and torch.cuda.is_current_stream_capturing() and not small_pays("fwd", M, N, K):
         return None
