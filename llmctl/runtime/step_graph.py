@@ -3,8 +3,8 @@
 A step of a small model is bound by the host: every launch passes through an autograd function, its checks and the
 dispatcher, 15 to 20 us each, while the kernels take 3 to 10.  The recording holds ``zero_grad``, the model's forward and backward
 and ``settle_grads``; the clip norm and AdamW, whose step count and learning rate are launch arguments, stay outside and run as
-ever.  Whole steps, one MI355X, us, eager / replayed: tiny (2 layers) 256 tokens 1528 / 426, 4096 tokens 1711 / 685; gpt2-125m (12
-layers) 128 tokens 8072 / 3615, 1024 7137 / 4816, 2048 7352 / 5863.
+ever.  Whole steps, one MI355X, us, eager / replayed: tiny (2 layers) 256 tokens 1333 / 263, 4096 tokens 1742 / 628; gpt2-125m (12
+layers) 128 tokens 7925 / 3165, 1024 7944 / 4700, 2048 8088 / 5793.
 
 A replay runs no Python, so whatever a step's Python could see or change is compared with what was recorded before every
 replay (:func:`fingerprint`), and a step that anything listens to (hooks, dispatch modes, anomaly mode, faults to inject) runs eagerly."""
@@ -20,7 +20,7 @@ from llmctl.utils.env import graph_capture_gc_guard
 
 # What a recording is worth, from the sizes: host seconds of an eager step against seconds of its kernels (the products, and weights, gradients and
 # optimizer states through HBM).  Where the kernels take longer than the host a replay gains nothing and would keep its activations for
-# itself: gpt2-125m eager / replayed, us, 4096 tokens 7972 / 7879, 8192 11679 / 11692; one GPT-7B layer 64 tokens 4017 / 3991.
+# itself: gpt2-125m eager / replayed, us, 4096 tokens 8180 / 8188, 8192 11399 / 11395; one GPT-7B layer 64 tokens 4017 / 3991.
 HOST_STEP, HOST_LAYER = 0.5e-3, 0.55e-3
 PRODUCT_RATE, BYTES_PER_PARAMETER, COPY_RATE = 0.45e15, 40, 4.5e12
 
