@@ -7,7 +7,9 @@
 //
 // Operands travel as 8-byte words {value, tag}, written and polled with relaxed agent-scope accesses, which pass the XCDs' L2s by: a word that carries its own
 // tag needs no flag, no barrier and no fence (an agent fence writes an L2 back: a grid barrier with fences measured 20 us, with a counter of relaxed accesses
-// 4.3, such words 1.5 us for 512 among 64 workgroups, 2.2 among 128).  The tag is the layer, counted on over all steps; the count lives in the workspace.
+// 4.3, such words 1.5 us for 512 among 64 workgroups, 2.2 among 128).  The tag is the layer, counted on over all steps (32 bits, of the MLP's words the low 16); the
+// count lives in the workspace.  Words of rows and spans that a step does not have get its last tag all the same, so that none is older than the step before, whose
+// tags no layer of this one has, and the count may wrap.
 // Layer: qkv -> heads (a workgroup per head, row and span of keys) -> output projection -> up -> down, five such exchanges.  A word's place is used once a
 // layer.  Nobody writes it again before all have read it: between two writes of any place every workgroup takes part in the down projection's exchange, which
 // every workgroup waits for, and each sends its part of that after it has read what the layer sent before.
@@ -603,6 +605,20 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         r.load(w.wd, v * NO, wave, lane);
         down_of(r, bf2f(global(w.bd)[v * NO + tid % NO]), v);
       }
+    }
+    // ---- the words that this step has not written (nobody waits for them)
+    {
+      const unsigned last = base + g.L;
+      auto age = [&](u64* p, int from, int to, u64 v) __attribute__((always_inline)) {
+        for (int i = from + me * THREADS + tid; i < to; i += N * THREADS) put_word(p + i, v);
+      };
+      const u64 v = (u64)last << 32;
+      age(pq, g.B * 3 * H, MAX_ROWS * 3 * H, v);
+      age(pa, g.B * H, MAX_ROWS * H, v);
+      age(px, g.B * H, MAX_ROWS * H, v);
+      age(py, g.B * H, MAX_ROWS * H, v);
+      age(ph, g.B * PARTS * WF, MAX_ROWS * PARTS * WF, (u64)(last & 0xffffu) << 48);
+      age(ps, splits > 1 ? items * (D + 2) : 0, PARTS * (D + 2), v);
     }
     // ---- the final norm: row b by whoever holds share b
     for (int v = me; v < g.B; v += N) {

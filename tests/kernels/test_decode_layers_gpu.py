@@ -128,3 +128,45 @@ def test_what_it_does_not_take(native_lib):
     with pytest.raises(RuntimeError):
         run(a, ops.decode_layers_workspace(512, "cuda"))
     assert math.isfinite(float(run(a, ops.decode_layers_workspace(256, "cuda"))[0].float().sum()))
+
+
+def _count(ws, base):
+    """The layers that a workspace has counted (second word, low half; the high one is zero between steps)."""
+    ws[1] = base
+
+
+def _fits(a, got):
+    want, ks, _ = plain(a)
+    assert float((got[0].double() - want).norm()) <= (1 + len(ks)) * 2.0 ** -8 * float(want.norm())
+    new = run(a, torch.zeros_like(a["ws"]))  # a workspace that has seen no step
+    assert all(torch.equal(x, y) for x, y in zip(got, new))
+
+
+@pytest.mark.parametrize("L", [2, 3, 5])
+@pytest.mark.parametrize("bits", [16, 32])
+def test_words_that_narrower_steps_left_are_not_taken(native_lib, L, bits):
+    """Two rows, then so many steps of one row (counted, not run, but for the last) that the next first layer's count ends in the bits of a word that the second row
+    left; then two rows of other tokens."""
+    from llmctl import ops
+
+    two, one, other = (make(256, L, ctx, seed=s) for s, ctx in ((1, [40, 30]), (2, [21]), (3, [33, 600])))
+    for last in range(1, L + 1):  # whichever layer's word it were
+        two["ws"] = one["ws"] = other["ws"] = ws = ops.decode_layers_workspace(256, "cuda")
+        run(two, ws)
+        _count(ws, ((1 << bits) + last - 1 - L) & 0xffffffff)
+        _fits(one, run(one, ws))
+        _fits(other, run(other, ws))
+
+
+@pytest.mark.parametrize("start", [0, 65536 - 14, (1 << 32) - 14])
+def test_rows_and_spans_come_and_go_on_one_workspace(native_lib, start):
+    """Steps of 4, 1, 2 .. rows, one span of keys and several, the count past 16 and past 32 bits on the way."""
+    from llmctl import ops
+
+    ws = ops.decode_layers_workspace(256, "cuda")
+    steps = [dict(make(256, 3, ctx, seed=i), ws=ws) for i, ctx in enumerate(([20, 3, 700, 1], [1500], [9, 40], [5], [2000, 300, 7, 64], [11, 800]))]
+    for turn in range(2):
+        for i, a in enumerate(steps):
+            if turn and not i:
+                _count(ws, start)
+            _fits(a, run(a, ws))
