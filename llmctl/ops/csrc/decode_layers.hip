@@ -436,14 +436,15 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
             s[u] = score(k, t0 + (u * WAVES + wave) * 8 + tg < k1);
             mn = fmaxf(mn, s[u]);
           }
-          const float keep = mn == -INFINITY ? 1.f : exp2f(m - mn);
+          const float top_s = mn == -INFINITY ? 0.f : mn;  // (scores that are not numbers are no maximum, and come through the exponentials)
+          const float keep = exp2f(m - top_s);
           m = mn;
           sum *= keep;
 #pragma unroll
           for (int j = 0; j < 8; ++j) o[j] *= keep;
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            const float e = mn == -INFINITY ? 0.f : exp2f(s[u] - mn);
+            const float e = exp2f(s[u] - top_s);
             float v[8];
             load8(reinterpret_cast<const bf16*>(&vv[u]), v);
             sum += e;
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) kn[j] = qkv[1][sub * 8 + j];
         const float sn = score(kn, own), mw = lanes_max(fmaxf(m, sn));
-        const float keep = mw == -INFINITY ? 0.f : exp2f(m - mw), en = mw == -INFINITY ? 0.f : exp2f(sn - mw);
+        const float top_w = mw == -INFINITY ? 0.f : mw, keep = exp2f(m - top_w), en = exp2f(sn - top_w);
         sum = groups_sum(sum * keep + en);
 #pragma unroll
         for (int j = 0; j < 8; ++j) o[j] = groups_sum(o[j] * keep + en * qkv[2][sub * 8 + j]);

@@ -170,3 +170,15 @@ def test_rows_and_spans_come_and_go_on_one_workspace(native_lib, start):
             if turn and not i:
                 _count(ws, start)
             _fits(a, run(a, ws))
+
+
+@pytest.mark.parametrize("ctx,bad", [([20], range(19)), ([700, 5], range(0, 8)), ([300], [270])])
+def test_keys_that_are_not_numbers_come_through(native_lib, ctx, bad):
+    """A key row of NaN makes its head's scores NaN: the row's result shows it, whichever lanes read it, and the other row's does not."""
+    from llmctl import ops
+
+    a = make(256, 1, ctx)
+    for t in bad:
+        a["k_cache"][0, int(a["block_tables"][0, t // BLOCK]), t % BLOCK] = float("nan")
+    out = run(a, ops.decode_layers_workspace(256, "cuda"))[0]
+    assert bool(torch.isnan(out[0]).all()) and bool(torch.isfinite(out[1:]).all())
