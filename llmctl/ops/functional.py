@@ -711,6 +711,7 @@ def decode_layers_ok(hidden: int, heads: int, kv_heads: int, ffn: int, layers: i
     367 / 200, 2000 425 / 251, two rows 382 / 237, four 425 / 332 (a row more costs 45, beside launches 20); four layers of 256, one row 122 / 77, of 1024, four
     rows 175 / 161."""
     return (knobs().decode_layers and use_native(cache) and cache.dtype == torch.bfloat16 and cache.is_contiguous() and 1 <= rows <= 4 and 1 <= layers <= 32
+            and cache.dim() == 5 and cache.shape[-1] == 64 and cache.data_ptr() % 16 == 0 and cache[0].numel() < 1 << 35
             and hidden % 256 == 0 and 256 <= hidden <= 1024 and heads == kv_heads and heads * 64 == hidden and ffn == 4 * hidden
             and torch.cuda.get_device_properties(cache.device).multi_processor_count >= 128)
 

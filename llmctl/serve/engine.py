@@ -654,7 +654,8 @@ class InferenceEngine:
         """The workspace of ``ops.decode_layers`` where the whole step of ``n`` rows runs in one launch."""
         cfg, m = self.cfg, self.model
         if not (self.tp == 1 and self.rope is None and m.pos_embed is not None and m.final_norm_b is not None and not cfg.gated_mlp and not cfg.is_moe
-                and all(p is not None and p.dtype == torch.bfloat16 and p.is_contiguous() and p.data_ptr() % 16 == 0 for p in self._step_weights())
+                and all(p is not None and p.dtype == torch.bfloat16 and p.is_contiguous() and p.data_ptr() % 16 == 0
+                        for p in (m.embed, m.pos_embed, *self._step_weights()))
                 and ops.decode_layers_ok(cfg.hidden, cfg.heads, cfg.kv_heads, cfg.ffn, len(m.layers), n, self.kv_cache.k)):
             return None
         if self._layers_ws is None and not torch.cuda.is_current_stream_capturing():

@@ -1,5 +1,6 @@
 """A whole decode step in one launch (``csrc/decode_layers.hip``) against plain torch in float64, and against itself with other numbers of workgroups."""
 
+import json
 import math
 
 import pytest
@@ -182,3 +183,61 @@ def test_keys_that_are_not_numbers_come_through(native_lib, ctx, bad):
         a["k_cache"][0, int(a["block_tables"][0, t // BLOCK]), t % BLOCK] = float("nan")
     out = run(a, ops.decode_layers_workspace(256, "cuda"))[0]
     assert bool(torch.isnan(out[0]).all()) and bool(torch.isfinite(out[1:]).all())
+
+
+def engine(tmp_path, knob=True, graphs=True, **kw):
+    from llmctl.serve.engine import InferenceEngine
+
+    f = tmp_path / "model.json"
+    f.write_text(json.dumps({"name": "narrow", "arch": "decoder-only", "layers": 3, "hidden": 256, "ffn": 1024, "heads": 4, "vocab_size": 512, "norm": "layernorm",
+                             "activation": "gelu", "position": "learned", "max_position_embeddings": 512, **kw}))
+    return InferenceEngine(str(f), device="cuda", max_batch_size=4, num_kv_blocks=128, block_size=BLOCK, max_model_len=512, use_graphs=graphs, seed=5,
+                           perf_knobs={"decode_layers": knob})
+
+
+def steps(eng, prompts, n=4, change=None):
+    """The logits of a prompt's last token and of n decode steps of fixed tokens, the sequences' caches made by the engine."""
+    from llmctl.serve.scheduler import PrefillChunk
+
+    seqs = [eng.open_sequence(p) for p in prompts]
+    out = [eng.prefill([PrefillChunk(s, 0, len(s.prompt_ids)) for s in seqs]).float().clone()]
+    if change is not None:
+        change(eng)
+    for i in range(n):
+        for s in seqs:
+            s.output_ids.append(7 * i + len(s.prompt_ids))
+            s._decode_slot = eng.kv.append_token(s.seq_id)
+        out.append(eng.decode(seqs).float().clone())
+    return out
+
+
+def off_16_bytes(t):
+    u = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)[4:].view(t.shape)
+    return torch.nn.Parameter(u.copy_(t.detach()), requires_grad=False)
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("what", ["as it is", "wider heads", "narrower heads", "embedding off 16 bytes", "positions off 16 bytes"])
+def test_engine_takes_what_it_took(native_lib, tmp_path, graphs, what):
+    """Through the engine's own rule: a model that fits gives the chain's logits to rounding, one that does not (heads that are not hidden / heads wide, tables that the
+    kernel cannot read in 16 bytes) runs the chain, bit for bit."""
+    kw = {"wider heads": dict(head_dim=128), "narrower heads": dict(head_dim=64, hidden=512, ffn=2048)}.get(what, {})
+
+    def change(eng):
+        if what == "embedding off 16 bytes":
+            eng.model.embed = off_16_bytes(eng.model.embed)
+        elif what == "positions off 16 bytes":
+            eng.model.pos_embed = off_16_bytes(eng.model.pos_embed)
+
+    outs, taken = [], []
+    for knob in (True, False):
+        eng = engine(tmp_path, knob, graphs, **kw)
+        outs.append(steps(eng, [list(range(3, 40)), list(range(5, 9))], change=change))
+        taken.append(eng._step_workspace(2) is not None)
+        eng.close()
+    assert taken == [what == "as it is", False]
+    for x, y in zip(*outs):
+        if taken[0]:
+            assert float((x - y).norm()) <= 3 * 2.0 ** -7 * float(y.norm())  # the chain rounds its rows between launches, three layers of them
+        else:
+            assert torch.equal(x, y)
