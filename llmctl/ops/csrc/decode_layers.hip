@@ -262,11 +262,11 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
   const unsigned base = peek(&ctl->base);
   if (tid == 0) {
     int n = 0;
-    if (!(ticket & CLOSED)) {
+    if (!(ticket & CLOSED) && (ticket & 0xffffu) < gridDim.x) {
       const long t0 = wall_clock64();
       unsigned seen = peek(&ctl->gate);
       for (;;) {
-        const unsigned count = seen & 0xffffu;
+        const unsigned count = min(seen & 0xffffu, gridDim.x);  // (no more shares than there are, whoever else took numbers here)
         if (seen & CLOSED) n = (seen >> 16) & 0xff;
         else if (count == gridDim.x) n = (int)count;
         if (n != 0) break;

@@ -717,7 +717,7 @@ def decode_layers_ok(hidden: int, heads: int, kv_heads: int, ffn: int, layers: i
 
 
 def decode_layers_workspace(hidden: int, device) -> torch.Tensor:
-    """The words that a model's steps exchange (``decode_layers``): one per engine, whose steps follow one another."""
+    """The words that the workgroups of a step exchange (``decode_layers``), for steps that follow one another: a graph's, or one eager step's."""
     return torch.zeros(native().decode_layers_words(hidden), dtype=torch.int64, device=device)
 
 

@@ -139,7 +139,6 @@ class InferenceEngine:
         self.rope = self.model.rope_tables(self.max_model_len, self.device)
         # MoE routing sizes the expert segments on the host: decode runs eagerly
         self.use_graphs = use_graphs and self.device.type == "cuda" and not cfg.is_moe
-        self._layers_ws = None  # _step_workspace
         self._graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, Dict[str, torch.Tensor]]] = {}
         # sampling uniforms come from the host (one H2D copy with the step's other inputs), so
         # in-graph sampling and the eager path draw the same stream
@@ -650,17 +649,13 @@ class InferenceEngine:
                 and all(l.attn_norm_b is None and l.mlp_norm_b is None for l in m.layers)
                 and self.knobs.decode_fused)
 
-    def _step_workspace(self, n: int) -> Optional[torch.Tensor]:
-        """The workspace of ``ops.decode_layers`` where the whole step of ``n`` rows runs in one launch."""
+    def _one_launch(self, n: int) -> bool:
+        """Does ``ops.decode_layers`` run the whole step of ``n`` rows?"""
         cfg, m = self.cfg, self.model
-        if not (self.tp == 1 and self.rope is None and m.pos_embed is not None and m.final_norm_b is not None and not cfg.gated_mlp and not cfg.is_moe
+        return (self.tp == 1 and self.rope is None and m.pos_embed is not None and m.final_norm_b is not None and not cfg.gated_mlp and not cfg.is_moe
                 and all(p is not None and p.dtype == torch.bfloat16 and p.is_contiguous() and p.data_ptr() % 16 == 0
                         for p in (m.embed, m.pos_embed, *self._step_weights()))
-                and ops.decode_layers_ok(cfg.hidden, cfg.heads, cfg.kv_heads, cfg.ffn, len(m.layers), n, self.kv_cache.k)):
-            return None
-        if self._layers_ws is None and not torch.cuda.is_current_stream_capturing():
-            self._layers_ws = ops.decode_layers_workspace(cfg.hidden, self.device)
-        return self._layers_ws
+                and ops.decode_layers_ok(cfg.hidden, cfg.heads, cfg.kv_heads, cfg.ffn, len(m.layers), n, self.kv_cache.k))
 
     def _step_weights(self) -> List[torch.Tensor]:
         m, out = self.model, []
@@ -668,11 +663,12 @@ class InferenceEngine:
             out += [l.attn_norm_w, l.attn_norm_b, l.wqkv, l.bqkv, l.wo, l.bo, l.mlp_norm_w, l.mlp_norm_b, l.w_up, l.b_up, l.w_down, l.b_down]
         return out + [m.final_norm_w, m.final_norm_b]
 
-    def _decode_body(self, ids, positions, slots, block_tables, ctx_lens) -> torch.Tensor:
+    def _decode_body(self, ids, positions, slots, block_tables, ctx_lens, workspace=None) -> torch.Tensor:
+        """``workspace``: of ``ops.decode_layers``, a graph's own.  An eager step takes a new one: two may run on two streams."""
         if self._fused_decode():
             return self._decode_body_fused(ids, positions, slots, block_tables, ctx_lens)
-        ws = self._step_workspace(ids.shape[0])
-        if ws is not None:
+        if self._one_launch(ids.shape[0]) and (workspace is not None or not torch.cuda.is_current_stream_capturing()):
+            ws = ops.decode_layers_workspace(self.cfg.hidden, self.device) if workspace is None else workspace
             m = self.model
             xn = ops.decode_layers(ids, positions, slots, block_tables, ctx_lens, m.embed, m.pos_embed, self._step_weights(), self.kv_cache.k,
                                    self.kv_cache.v, self.cfg.layer_norm_eps, ws)
@@ -799,6 +795,7 @@ class InferenceEngine:
         bufs = dict(zip(self._STAGED, packed_views(buf, offs, arrays)))
         bufs["u"] = bufs["u"].view(torch.float32)
         bufs.update(inputs=buf, ids_end=offs[1], stage=stage, turn=0,
+                    workspace=ops.decode_layers_workspace(self.cfg.hidden, d) if self._one_launch(nb) else None,
                     # in-graph sampling: per-row parameters (rewritten when the batch's change)
                     temp=torch.zeros(nb, dtype=torch.float32, device=d), topk=torch.zeros(nb, dtype=torch.int32, device=d),
                     topp=torch.ones(nb, dtype=torch.float32, device=d))
@@ -812,7 +809,7 @@ class InferenceEngine:
         """Decode step + sampling; the sampled ids also become the next step's input ids (the
         asynchronous path launches step N + 1 without reading step N's tokens first)."""
         bufs["logits"] = self._decode_body(bufs["ids"], bufs["positions"], bufs["slots"], bufs["block_tables"],
-                                           bufs["ctx_lens"])
+                                           bufs["ctx_lens"], bufs["workspace"])
         bufs["toks"] = ops.sample(bufs["logits"].contiguous(), bufs["temp"], bufs["topk"], bufs["topp"], bufs["u"])
         bufs["ids"].copy_(bufs["toks"])
 
@@ -860,7 +857,7 @@ class InferenceEngine:
             torch.cuda.synchronize(self.device)
         self.kv_cache = None
         self._w8 = self._w8_head = None
-        self._nf = self._layers_ws = None
+        self._nf = None
         self.rope = None
         if self.device.type == "cuda":
             torch.cuda.empty_cache()

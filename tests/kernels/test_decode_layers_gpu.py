@@ -233,7 +233,7 @@ def test_engine_takes_what_it_took(native_lib, tmp_path, graphs, what):
     for knob in (True, False):
         eng = engine(tmp_path, knob, graphs, **kw)
         outs.append(steps(eng, [list(range(3, 40)), list(range(5, 9))], change=change))
-        taken.append(eng._step_workspace(2) is not None)
+        taken.append(eng._one_launch(2))
         eng.close()
     assert taken == [what == "as it is", False]
     for x, y in zip(*outs):
@@ -241,3 +241,27 @@ def test_engine_takes_what_it_took(native_lib, tmp_path, graphs, what):
             assert float((x - y).norm()) <= 3 * 2.0 ** -7 * float(y.norm())  # the chain rounds its rows between launches, three layers of them
         else:
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+def test_steps_on_two_streams(native_lib, tmp_path, graphs):
+    """Eager steps of one engine, or its graphs of one row and of two, on two streams at a time: each has words of its own."""
+    eng = engine(tmp_path, graphs=graphs)
+    steps(eng, [[1, 2]], n=0)
+    seqs = [eng.open_sequence(list(range(2, n))) for n in (30, 50, 400)]
+    with torch.inference_mode():
+        eng.kv_cache.k.normal_(), eng.kv_cache.v.normal_()
+    for s in seqs:
+        s._decode_slot = int(eng.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+    parts = (seqs[:1], seqs[1:])
+    want = [eng.decode(p).clone() for p in parts]
+    streams = [torch.cuda.Stream() for _ in parts]
+    torch.cuda.synchronize()
+    for _ in range(20):
+        got = []
+        for s, p in zip(streams, parts):
+            with torch.cuda.stream(s):
+                got.append(eng.decode(p).clone())
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
+    eng.close()
