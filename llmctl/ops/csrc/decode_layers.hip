@@ -16,6 +16,11 @@
 //
 // A workgroup waits only for workgroups that run: each takes a number at the start; the step begins when all have one or, after the gate's time, with those that
 // have (any number works: the 128 shares go round); later ones find the gate closed and leave.  So no launch beside it, however long, can stop it for good.
+// The gate's time is what fewer workgroups cost: as much for every round of shares beyond the first as that round takes, so a step beside another stream's kernels
+// takes at most about twice what the best choice would have (after a fixed 200 us some went through with one workgroup).  gpt2-125m, context 129, us a step by
+// workgroups: 128 164, 127 208, 64 247, 32 361, 16 587, 7 1234, 1 7671; four rows 253 .. 17614.  Beside causal attention of 4 x 4096 tokens, 32 heads (670 us a
+// launch), us a step, median and longest of 540: 688, 1050; after 200 us 671, 10926; the chain of launches 1539, 1709.  Beside products of 8192 930 (the chain 23400),
+// of 2048 278 (555), copies 428 (871).
 // Waits are bounded all the same (SPINS): a step that overran would end with NaN.
 //
 // fp32 throughout but for weights, cache rows, the MLP's activations (three to a word, rounded as between two launches) and the normed result; the sums of a
@@ -67,7 +72,7 @@ struct StepArgs {
   u64* ws;
   long rows, prows, layer_stride;  // of the tables; elements of a layer's cache
   float eps, scale;
-  int L, B, heads, block, max_blocks, gate_ticks;  // (of the 100 MHz clock)
+  int L, B, heads, block, max_blocks, gate_ticks;  // a round's, of the 100 MHz clock
 };
 
 template <int CTRL>
@@ -270,7 +275,8 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         if (seen & CLOSED) n = (seen >> 16) & 0xff;
         else if (count == gridDim.x) n = (int)count;
         if (n != 0) break;
-        if (wall_clock64() - t0 >= g.gate_ticks) {
+        // (rounds that these would take, less the one that all take; a second at the most)
+        if (wall_clock64() - t0 >= min((long)g.gate_ticks * ((PARTS + (int)count - 1) / (int)count - 1), 100000000l)) {
           unsigned want = seen;
           if (__hip_atomic_compare_exchange_strong(&ctl->gate, &want, seen | CLOSED | (count << 16), __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT))
@@ -675,7 +681,7 @@ at::Tensor decode_layers(const at::Tensor& ids, const at::Tensor& positions, con
   LLMCTL_CHECK(table.dim() == 2 && H % 256 == 0 && H >= 256 && H <= 1024 && B >= 1 && B <= MAX_ROWS && L >= 1 && L <= MAX_LAYERS && (int64_t)w.size() == 12 * L + 2,
                "decode_layers: up to 4 rows, 32 layers of 256 to 1024 columns");
   LLMCTL_CHECK(workgroups >= 1 && workgroups <= PARTS, "decode_layers: 1 to 128 workgroups");
-  LLMCTL_CHECK(gate_us >= 0 && gate_us <= 1000000, "decode_layers: the gate's time");
+  LLMCTL_CHECK(gate_us >= 0 && gate_us <= 1000000, "decode_layers: the gate's time for a round");
   auto ints = [&](const at::Tensor& t, at::ScalarType type, int64_t n) {
     return t.is_cuda() && t.is_contiguous() && t.scalar_type() == type && t.numel() == n;
   };

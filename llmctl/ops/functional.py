@@ -722,10 +722,13 @@ def decode_layers_workspace(hidden: int, device) -> torch.Tensor:
 
 
 def decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps: float, workspace, workgroups: int = 128,
-                  gate_us: int = 200):
+                  gate_us: Optional[int] = None):
     """The final norm's rows of a decode step: embedding, all layers with their paged cache, final norm.  ``weights``: per layer the attention norm (weight,
     bias), QKV, output projection, MLP norm, up and down (weight and bias each), then the final norm; ``k_cache`` / ``v_cache``: all layers' ``[L, blocks,
-    block, heads, 64]``.  ``workgroups``: fewer than 128 each do the work of several; ``gate_us``: the step begins without those that do not run by then."""
+    block, heads, 64]``.  ``workgroups``: fewer than 128 each do the work of several; ``gate_us``: how long it waits for those that do not run yet, for every round of
+    shares that the others would take beyond the first (None: about as long as that round, 5 us a layer and 2.5 a further row)."""
+    if gate_us is None:
+        gate_us = 5 * (len(weights) // 12) * (ids.shape[0] + 1) // 2
     return native().decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps, workspace, workgroups, gate_us)
 
 
