@@ -96,7 +96,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const T* __restrict__ logit
           B = wb[w];
           I = wi[w];
         }
-      out[row] = I;
+      out[row] = I < V ? I : 0;  // (a row without a number has no largest one: as below, a token that the next step can look up)
     }
     return;
   }

@@ -882,6 +882,17 @@ def test_sampling_greedy_ties_and_odd_vocab(native_lib, V):
     assert torch.equal(got, exp)
 
 
+@pytest.mark.parametrize("V", [32000, 1003])
+@pytest.mark.parametrize("temp", [0.0, 1.0])
+def test_sampling_a_row_without_numbers_stays_in_the_vocabulary(native_lib, V, temp):
+    """The sampled ids are the next step's input before the host has seen them: whatever the logits, an embedding has a row for them."""
+    logits = torch.full((2, V), float("nan"), device=DEV, dtype=torch.bfloat16)
+    logits[1] = -float("inf")
+    one = torch.ones(2, device=DEV)
+    got = native_lib.sample(logits, one * temp, torch.zeros(2, dtype=torch.int32, device=DEV), one, one / 2)
+    assert 0 <= int(got.min()) and int(got.max()) < V
+
+
 @pytest.mark.parametrize("with_pos", [False, True])
 def test_rope_flash_attention_inplace_matches(native_lib, with_pos):
     """In-place RoPE (rope_qk_inplace_: q / k heads of qkv rotated in place, attention on strided
