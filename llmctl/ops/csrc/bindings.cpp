@@ -60,7 +60,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("paged_attention_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor context_lens, float scale) -> Tensor");
   m.def("norm_linear(Tensor x, Tensor? res, Tensor nw, Tensor nb, float eps, Tensor w, Tensor? bias, int act) -> (Tensor, Tensor)");
   m.def("norm_qkv_cache(Tensor x, Tensor? res, Tensor nw, Tensor nb, float eps, Tensor w, Tensor? bias, int nq, int nkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slots) -> (Tensor, Tensor)");
-  m.def("decode_layers(Tensor ids, Tensor positions, Tensor slots, Tensor block_tables, Tensor ctx, Tensor table, Tensor ptable, Tensor[] w, Tensor(a!) k, Tensor(b!) v, float eps, Tensor(c!) workspace, int workgroups, int gate_us) -> Tensor");
+  m.def("decode_layers(Tensor ids, Tensor positions, Tensor slots, Tensor block_tables, Tensor ctx, Tensor table, Tensor ptable, Tensor[] w, Tensor(a!) k, Tensor(b!) v, float eps, Tensor(c!) workspace, int workgroups, int gate_us, Tensor(d!)? lost=None, int spins=2097152) -> Tensor");
   m.def("decode_layers_words(int hidden) -> int", &llmctl::decode_layers_words);
   m.def("stream_linear(Tensor x, Tensor w, Tensor? bias, int act) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w, Tensor? bias) -> Tensor");

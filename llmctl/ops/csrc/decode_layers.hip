@@ -21,7 +21,7 @@
 // workgroups: 128 164, 127 208, 64 247, 32 361, 16 587, 7 1234, 1 7671; four rows 253 .. 17614.  Beside causal attention of 4 x 4096 tokens, 32 heads (670 us a
 // launch), us a step, median and longest of 540: 688, 1050; after 200 us 671, 10926; the chain of launches 1539, 1709.  Beside products of 8192 930 (the chain 23400),
 // of 2048 278 (555), copies 428 (871).
-// Waits are bounded all the same (SPINS): a step that overran would end with NaN.
+// Waits are bounded all the same: a step that overran ends with NaN rows and sets a word of the host's.
 //
 // fp32 throughout but for weights, cache rows, the MLP's activations (three to a word, rounded as between two launches) and the normed result; the sums of a
 // product run over 64 lanes, then pairwise, whatever the number of workgroups.
@@ -38,7 +38,6 @@ namespace {
 constexpr int PARTS = 128, WAVES = 8, THREADS = WAVES * 64, MAX_LAYERS = 32, MAX_ROWS = 4, R = 4;  // R: MLP width over hidden
 constexpr int D = 64, U = 4;  // head size; cache tokens that a lane has in flight
 constexpr int SPAN = U * WAVES * 8;                    // keys of a workgroup, where there are workgroups to share them out to
-constexpr int SPINS = 1 << 21;
 constexpr unsigned CLOSED = 1u << 30;
 
 using u64 = unsigned long long;
@@ -59,7 +58,11 @@ struct LayerW {
 };
 
 struct Control {  // the workspace starts with this, zero before the first step
-  unsigned gate, left, base, late;
+  unsigned gate, left, base, late;  // left: workgroups that are through, and above bit 16 those that saw the step lost
+};
+struct Wait {
+  Control* ctl;
+  int spins;  // tries of a wait
 };
 
 struct StepArgs {
@@ -68,8 +71,9 @@ struct StepArgs {
   bf16 *kc, *vc, *out;
   const int64_t *ids, *slots;
   const int *pos, *bt, *ctx;
-  Control* ctl;
+  Wait wait;
   u64* ws;
+  unsigned* lost;  // nullptr or the host's word that a lost step sets
   long rows, prows, layer_stride;  // of the tables; elements of a layer's cache
   float eps, scale;
   int L, B, heads, block, max_blocks, gate_ticks;  // a round's, of the 100 MHz clock
@@ -113,23 +117,23 @@ __device__ __forceinline__ float groups_sum(float v) {
 __device__ __forceinline__ void put_word(u64* p, u64 v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void send(u64* p, float v, unsigned tag) { put_word(p, ((u64)tag << 32) | __float_as_uint(v)); }
 __device__ __forceinline__ unsigned peek(const unsigned* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// whether to stop waiting: after SPINS tries of anybody's, the step is lost
-__device__ __forceinline__ bool give_up(int n, Control* ctl) {
-  if ((n & 4095) != 0) return false;
-  if (n >= SPINS) __hip_atomic_store(&ctl->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return n >= SPINS || peek(&ctl->late) != 0;
+// whether to stop waiting: after so many tries of anybody's, the step is lost
+__device__ __forceinline__ bool give_up(int n, Wait w) {
+  if ((n & 4095) != 0 && n < w.spins) return false;
+  if (n >= w.spins) __hip_atomic_store(&w.ctl->late, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return n >= w.spins || peek(&w.ctl->late) != 0;
 }
 __device__ __forceinline__ u64 word(const u64* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ __forceinline__ float take(const u64* p, unsigned tag, Control* ctl) {
+__device__ __forceinline__ float take(const u64* p, unsigned tag, Wait wait) {
   for (int n = 1;; ++n) {
     const u64 v = word(p);
     if ((unsigned)(v >> 32) == tag) return __uint_as_float((unsigned)v);
-    if (give_up(n, ctl)) return __uint_as_float(0x7fc00000u);
+    if (give_up(n, wait)) return __uint_as_float(0x7fc00000u);
   }
 }
 // count words, eight of a thread's in flight; put(i, word) for each.  BITS: of the tag, at the top
 template <int BITS, typename Put>
-__device__ __forceinline__ void gather(const u64* src, int count, unsigned tag, Control* ctl, Put put) {
+__device__ __forceinline__ void gather(const u64* src, int count, unsigned tag, Wait wait, Put put) {
   constexpr int W = 8;
   for (int i0 = threadIdx.x; i0 < count; i0 += W * THREADS) {
     u64 v[W];
@@ -143,7 +147,7 @@ __device__ __forceinline__ void gather(const u64* src, int count, unsigned tag, 
 #pragma unroll
       for (int j = 0; j < W; ++j)
         if ((miss >> j & 1) && (unsigned)(v[j] >> (64 - BITS)) == (tag & (unsigned)((1ull << BITS) - 1))) miss &= ~(1u << j);
-      if (miss != 0 && give_up(n, ctl)) {
+      if (miss != 0 && give_up(n, wait)) {
 #pragma unroll
         for (int j = 0; j < W; ++j)
           if (miss >> j & 1) v[j] = 0x7fc07fc07fc07fc0ull;
@@ -156,8 +160,8 @@ __device__ __forceinline__ void gather(const u64* src, int count, unsigned tag, 
   }
 }
 // fp32 words into LDS
-__device__ __forceinline__ void gather_f32(float* dst, const u64* src, int count, unsigned tag, Control* ctl) {
-  gather<32>(src, count, tag, ctl, [&](int i, u64 v) { dst[i] = __uint_as_float((unsigned)v); });
+__device__ __forceinline__ void gather_f32(float* dst, const u64* src, int count, unsigned tag, Wait wait) {
+  gather<32>(src, count, tag, wait, [&](int i, u64 v) { dst[i] = __uint_as_float((unsigned)v); });
 }
 
 __device__ __forceinline__ void widen(b4 v, float (&o)[4]) {
@@ -260,7 +264,8 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
   __shared__ LayerW layers[MAX_LAYERS];  // (read from the arguments, a layer's line of them is fetched when the layer starts)
   __shared__ int who[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  Control* ctl = g.ctl;
+  const Wait wait = g.wait;
+  Control* ctl = wait.ctl;
   // ---- the gate
   unsigned ticket = 0;
   if (tid == 0) ticket = __hip_atomic_fetch_add(&ctl->gate, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -315,6 +320,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
   u64* const py = ph + (long)MAX_ROWS * F;
   u64* const ps = py + (long)MAX_ROWS * H;
 
+  bool late = false;  // a wait of this workgroup, or one that it has heard of, ran out (thread 0's)
   if (N != 0) {
     Rows<KC, UQ> wq;
     Rows<KC, UO> wo;
@@ -371,7 +377,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
       const unsigned tag = base + l + 1;
       // ---- qkv
       if (l > 0) {
-        gather_f32(xs[0], py, g.B * H, tag - 1, ctl);
+        gather_f32(xs[0], py, g.B * H, tag - 1, wait);
         __syncthreads();
       }
       auto qkv_of = [&](const Rows<KC, UQ>& r, float bias, int v) __attribute__((always_inline)) {
@@ -406,7 +412,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         }
         if (tid < 3 * D) {
           const int which = tid >> 6, d = tid & 63;
-          float t = take(pq + (long)b * 3 * H + which * H + h * D + d, tag, ctl);
+          float t = take(pq + (long)b * 3 * H + which * H + h * D + d, tag, wait);
           if (which != 0) {  // as the cache holds it
             const bf16 r = f2bf(t);
             t = bf2f(r);
@@ -499,7 +505,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         for (int it = me; it < items; it += N) {
           if (it % splits) continue;  // the first span's workgroup adds them
           float* buf = &hs[0][0];
-          gather_f32(buf, ps + (long)it * (D + 2), splits * (D + 2), tag, ctl);
+          gather_f32(buf, ps + (long)it * (D + 2), splits * (D + 2), tag, wait);
           __syncthreads();
           if (tid < D) {
             float M = -INFINITY, S = 0.f, O = 0.f;
@@ -515,7 +521,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         }
       }
       // ---- output projection
-      gather_f32(as[0], pa, g.B * H, tag, ctl);
+      gather_f32(as[0], pa, g.B * H, tag, wait);
       __syncthreads();
       auto out_of = [&](const Rows<KC, UO>& r, float bias, int v) __attribute__((always_inline)) {
 #pragma unroll ROWS == 1 ? 1 : 2
@@ -537,7 +543,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         out_of(r, bias_of(w.bo, v * NO, NO), v);
       }
       // ---- up
-      gather_f32(xs[0], px, g.B * H, tag, ctl);
+      gather_f32(xs[0], px, g.B * H, tag, wait);
       __syncthreads();
       auto up_of = [&](const Rows<KC, UF>& r, float bias, int share) __attribute__((always_inline)) {
 #pragma unroll ROWS == 1 ? 1 : 2
@@ -567,7 +573,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
         up_of(r, bias_of(w.bu, v * NF, NF), v);
       }
       // ---- down
-      gather<16>(ph, g.B * PARTS * WF, tag, ctl, [&](int i, u64 v) {
+      gather<16>(ph, g.B * PARTS * WF, tag, wait, [&](int i, u64 v) {
         const int b = i / (PARTS * WF), k = i - b * PARTS * WF, o = k % WF * 3;
         float* dst = hs[b] + k / WF * NF + o;
 #pragma unroll
@@ -615,6 +621,7 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
     }
     // ---- the words that this step has not written (nobody waits for them)
     {
+      late = peek(&ctl->late) != 0;
       const unsigned last = base + g.L;
       auto age = [&](u64* p, int from, int to, u64 v) __attribute__((always_inline)) {
         for (int i = from + me * THREADS + tid; i < to; i += N * THREADS) put_word(p + i, v);
@@ -629,14 +636,14 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
     }
     // ---- the final norm: row b by whoever holds share b
     for (int v = me; v < g.B; v += N) {
-      gather_f32(as[v], py + (long)v * H, H, base + g.L, ctl);
+      gather_f32(as[v], py + (long)v * H, H, base + g.L, wait);
       __syncthreads();
       if (wave == 0) {
         norm_of(g.nw, g.nb);
         float x[KC][4];
         read_row(as[v], lane, x);
         layernorm(x, nw, nb, g.eps);
-        const bool late = peek(&ctl->late) != 0;
+        late |= peek(&ctl->late) != 0;
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
           bf16 o[4];
@@ -649,7 +656,11 @@ __global__ __launch_bounds__(THREADS, 1) void decode_layers_kernel(StepArgs g) {
   }
   // ---- the last one out readies the workspace for the next step
   __syncthreads();
-  if (tid == 0 && __hip_atomic_fetch_add(&ctl->left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+  if (tid != 0) return;
+  const unsigned out = 1u + (late ? 1u << 16 : 0u);
+  const unsigned left = out + __hip_atomic_fetch_add(&ctl->left, out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((left & 0xffffu) == gridDim.x) {
+    if (left >> 16 && g.lost != nullptr) __hip_atomic_store(g.lost, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     auto put = [](unsigned* p, unsigned v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     put(&ctl->base, base + g.L);
     put(&ctl->late, 0u);
@@ -673,15 +684,18 @@ int64_t decode_layers_words(int64_t hidden) {  // 8-byte words of a workspace
 
 // The final norm's rows [B, H] of a decode step: ``w`` holds per layer the attention norm (weight, bias), QKV, output projection, MLP norm, up and
 // down (weight, bias each), then the final norm.  k, v: the cache [L, blocks, block, heads, 64]; workspace: int64 [decode_layers_words], zero
-// before its first step and used by one step at a time.
+// before its first step and used by one step at a time.  lost: pinned host memory, set to 1 by a step whose waits ran out (``spins`` tries), whose rows are NaN.
 at::Tensor decode_layers(const at::Tensor& ids, const at::Tensor& positions, const at::Tensor& slots, const at::Tensor& block_tables,
                          const at::Tensor& ctx, const at::Tensor& table, const at::Tensor& ptable, at::TensorList w, at::Tensor k, at::Tensor v,
-                         double eps, at::Tensor workspace, int64_t workgroups, int64_t gate_us) {
+                         double eps, at::Tensor workspace, int64_t workgroups, int64_t gate_us, const c10::optional<at::Tensor>& lost, int64_t spins) {
   const int64_t B = ids.numel(), H = table.size(1), L = ((int64_t)w.size() - 2) / 12, heads = H / D;
   LLMCTL_CHECK(table.dim() == 2 && H % 256 == 0 && H >= 256 && H <= 1024 && B >= 1 && B <= MAX_ROWS && L >= 1 && L <= MAX_LAYERS && (int64_t)w.size() == 12 * L + 2,
                "decode_layers: up to 4 rows, 32 layers of 256 to 1024 columns");
   LLMCTL_CHECK(workgroups >= 1 && workgroups <= PARTS, "decode_layers: 1 to 128 workgroups");
   LLMCTL_CHECK(gate_us >= 0 && gate_us <= 1000000, "decode_layers: the gate's time for a round");
+  LLMCTL_CHECK(spins >= 1 && spins <= (1 << 21), "decode_layers: 1 to 2^21 tries of a wait");
+  LLMCTL_CHECK(!lost.has_value() || (lost->device().is_cpu() && lost->is_pinned() && lost->scalar_type() == at::kInt && lost->numel() == 1),
+               "decode_layers: lost: one int32 of pinned memory");
   auto ints = [&](const at::Tensor& t, at::ScalarType type, int64_t n) {
     return t.is_cuda() && t.is_contiguous() && t.scalar_type() == type && t.numel() == n;
   };
@@ -709,7 +723,12 @@ at::Tensor decode_layers(const at::Tensor& ids, const at::Tensor& positions, con
   a.kc = bf_mut(k), a.vc = bf_mut(v), a.out = bf_mut(out);
   a.ids = ids.data_ptr<int64_t>(), a.slots = slots.data_ptr<int64_t>();
   a.pos = positions.data_ptr<int32_t>(), a.bt = block_tables.data_ptr<int32_t>(), a.ctx = ctx.data_ptr<int32_t>();
-  a.ctl = reinterpret_cast<Control*>(workspace.data_ptr<int64_t>());
+  a.wait = Wait{reinterpret_cast<Control*>(workspace.data_ptr<int64_t>()), (int)spins};
+  if (lost.has_value()) {
+    void* p = nullptr;
+    LLMCTL_HIP_CHECK(hipHostGetDevicePointer(&p, lost->data_ptr<int32_t>(), 0));
+    a.lost = static_cast<unsigned*>(p);
+  }
   a.ws = reinterpret_cast<u64*>(workspace.data_ptr<int64_t>()) + sizeof(Control) / 8;
   a.rows = table.size(0), a.prows = ptable.size(0), a.layer_stride = k.numel() / L;
   a.eps = (float)eps, a.scale = 0.125f;

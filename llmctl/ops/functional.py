@@ -722,14 +722,16 @@ def decode_layers_workspace(hidden: int, device) -> torch.Tensor:
 
 
 def decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps: float, workspace, workgroups: int = 128,
-                  gate_us: Optional[int] = None):
+                  gate_us: Optional[int] = None, lost: Optional[torch.Tensor] = None, spins: int = 1 << 21):
     """The final norm's rows of a decode step: embedding, all layers with their paged cache, final norm.  ``weights``: per layer the attention norm (weight,
     bias), QKV, output projection, MLP norm, up and down (weight and bias each), then the final norm; ``k_cache`` / ``v_cache``: all layers' ``[L, blocks,
     block, heads, 64]``.  ``workgroups``: fewer than 128 each do the work of several; ``gate_us``: how long it waits for those that do not run yet, for every round of
-    shares that the others would take beyond the first (None: about as long as that round, 5 us a layer and 2.5 a further row)."""
+    shares that the others would take beyond the first (None: about as long as that round, 5 us a layer and 2.5 a further row).  ``lost``: an int32 of pinned host memory
+    that becomes 1 when a workgroup's wait for the others runs out (``spins`` tries, seconds); the rows are NaN then and the cache rows void."""
     if gate_us is None:
         gate_us = 5 * (len(weights) // 12) * (ids.shape[0] + 1) // 2
-    return native().decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps, workspace, workgroups, gate_us)
+    return native().decode_layers(ids, positions, slots, block_tables, ctx_lens, table, pos_table, weights, k_cache, v_cache, eps, workspace, workgroups, gate_us,
+                                  lost, spins)
 
 
 def _dequant(w, w_scale, dtype):

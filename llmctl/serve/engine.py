@@ -48,6 +48,8 @@ log = logging.getLogger("llmctl.serve")
 
 
 class InferenceEngine:
+    _lost = _lost_host = None  # (a family with layers of its own has no such steps)
+
     def __init__(self, model_path: str = "tiny", device: str = "auto", dtype=torch.bfloat16, max_batch_size: int = 8,
                  max_batch_tokens: int = 8192, max_model_len: Optional[int] = None, kv_cache_fraction: float = 0.85,
                  block_size: int = 16, num_kv_blocks: Optional[int] = None, scheduler: str = "dynamic",
@@ -139,6 +141,8 @@ class InferenceEngine:
         self.rope = self.model.rope_tables(self.max_model_len, self.device)
         # MoE routing sizes the expert segments on the host: decode runs eagerly
         self.use_graphs = use_graphs and self.device.type == "cuda" and not cfg.is_moe
+        self._lost = torch.zeros(1, dtype=torch.int32, pin_memory=True) if self.device.type == "cuda" else None  # _raise_if_lost
+        self._lost_host = None if self._lost is None else self._lost.numpy()
         self._graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, Dict[str, torch.Tensor]]] = {}
         # sampling uniforms come from the host (one H2D copy with the step's other inputs), so
         # in-graph sampling and the eager path draw the same stream
@@ -649,6 +653,12 @@ class InferenceEngine:
                 and all(l.attn_norm_b is None and l.mlp_norm_b is None for l in m.layers)
                 and self.knobs.decode_fused)
 
+    def _raise_if_lost(self) -> None:
+        """A step in one launch whose workgroups waited too long for one another (``ops.decode_layers``): told by the host's word that it set."""
+        if self._lost is not None and self._lost_host[0]:
+            self._lost_host[0] = 0
+            raise RuntimeError("a decode step was lost (its workgroups waited too long for one another): its logits, tokens and cache rows are void")
+
     def _one_launch(self, n: int) -> bool:
         """Does ``ops.decode_layers`` run the whole step of ``n`` rows?"""
         cfg, m = self.cfg, self.model
@@ -671,7 +681,7 @@ class InferenceEngine:
             ws = ops.decode_layers_workspace(self.cfg.hidden, self.device) if workspace is None else workspace
             m = self.model
             xn = ops.decode_layers(ids, positions, slots, block_tables, ctx_lens, m.embed, m.pos_embed, self._step_weights(), self.kv_cache.k,
-                                   self.kv_cache.v, self.cfg.layer_norm_eps, ws)
+                                   self.kv_cache.v, self.cfg.layer_norm_eps, ws, lost=self._lost)
             return self._gather_vocab(ops.decode_linear(xn, m.head_weight()))
         x = self._embed(ids, positions)
         res = None
@@ -885,6 +895,7 @@ class InferenceEngine:
         use_knobs(self.knobs)
         if self.hybrid:
             return self._hybrid_decode(plan)
+        self._raise_if_lost()
         ids, positions, slots, ctx, bt = plan["ids"], plan["positions"], plan["slots"], plan["ctx"], plan["bt"]
         n = len(ids)
         self.stats["decode_tokens"] += n
@@ -992,6 +1003,7 @@ class InferenceEngine:
         ``decode_s`` plan; returns the device tensor of sampled ids (graph: the static ``toks``
         buffer, all bucket rows)."""
         use_knobs(self.knobs)
+        self._raise_if_lost()
         cont = bool(plan["cont"])
         if self.use_graphs:
             _, b = self._stage_and_replay(plan, cont)
@@ -1025,6 +1037,7 @@ class InferenceEngine:
         """Read an in-flight step's tokens (the one host sync of the pipeline) and append them."""
         if p["event"] is not None:
             p["event"].synchronize()
+        self._raise_if_lost()
         toks = p["host"][: p["n"]].tolist()
         produced = 0
         for seq, tok in zip(p["seqs"], toks):
@@ -1069,7 +1082,9 @@ class InferenceEngine:
 
     # ------------------------------------------------------------------ sampling
     def sample(self, logits: torch.Tensor, seqs: List[Sequence]) -> List[int]:
-        return self._sample_rows(logits, seqs).tolist()
+        toks = self._sample_rows(logits, seqs).tolist()
+        self._raise_if_lost()
+        return toks
 
     def _sample_rows(self, logits: torch.Tensor, seqs: List[Sequence]) -> torch.Tensor:
         """Sampled token ids (device tensor) of the rows of ``logits``, one uniform per row from

@@ -290,3 +290,48 @@ def test_steps_beside_a_full_chip(native_lib):
             took.append(ev[0].elapsed_time(ev[1]))
         side.synchronize()
     assert max(took) < 2.5, sorted(took)[-5:]
+
+
+def test_a_lost_step_is_told(native_lib, tmp_path, monkeypatch):
+    """A step whose waits run out (of one try here) ends with NaN rows and sets the host's word; the workspace serves the next one.  Through an engine: whoever asks for
+    its tokens, or for the next step, is told, once."""
+    import functools
+
+    from llmctl import ops
+    from llmctl.serve.scheduler import SamplingParams
+
+    a, ws, lost = make(256, 2, [40, 9]), ops.decode_layers_workspace(256, "cuda"), torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    want = run(a, ws, lost=lost)
+    torch.cuda.synchronize()
+    assert int(lost) == 0
+    out = run(a, ws, lost=lost, spins=1)[0]
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(out).all()) and int(lost) == 1
+    lost.zero_()
+    got = run(a, ws, lost=lost)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(got, want)) and int(lost) == 0
+    with pytest.raises(RuntimeError):
+        run(a, ws, lost=torch.zeros(1, dtype=torch.int32))  # not pinned: no kernel could write it
+
+    eng = engine(tmp_path, graphs=False)
+    steps(eng, [[1, 2, 3]], n=2)
+    seq = eng.open_sequence([5, 6, 7])
+    seq._decode_slot = int(eng.kv.slots(seq.seq_id, 2, 1)[0])
+    whole, short = ops.decode_layers, functools.partial(ops.decode_layers, spins=1)
+    for ask in (lambda x: eng.sample(x, [seq]), lambda x: (torch.cuda.synchronize(), eng.decode([seq]))):
+        monkeypatch.setattr(ops, "decode_layers", short)
+        logits = eng.decode([seq])
+        monkeypatch.setattr(ops, "decode_layers", whole)
+        with pytest.raises(RuntimeError, match="lost"):
+            ask(logits)
+        assert bool(torch.isfinite(eng.decode([seq])).all())
+    eng.scheduler.finish(seq, "stop")
+    eng.add_request([4, 5, 6], SamplingParams(max_tokens=8, temperature=0.0))
+    monkeypatch.setattr(ops, "decode_layers", short)
+    with pytest.raises(RuntimeError, match="lost"):  # the step after it is under way by then, with its tokens
+        for _ in range(4):
+            eng.step()
+    monkeypatch.setattr(ops, "decode_layers", whole)
+    torch.cuda.synchronize()
+    eng.close()
