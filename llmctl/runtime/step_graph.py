@@ -67,12 +67,16 @@ def fingerprint(engine) -> Optional[Tuple]:
     ps = [p for d in mods for p in d._parameters.values() if p is not None]
     if any(p._backward_hooks for p in ps):
         return None
+    sinked = [getattr(p, "_llmctl_grad_sink", None) is sink for p in ps]
+    for p, written in zip(ps, sinked):  # the engine's own hook and no other
+        if [*(p._post_accumulate_grad_hooks or {}).values()] != ([] if written else [sync._on_grad]):
+            return None
     at, size, grads = flat.grad.data_ptr(), flat.grad.element_size(), [p.grad for p in flat.params]
     if any(g is None or g.data_ptr() != at + size * flat.offsets[id(p)] for p, g in zip(flat.params, grads)):
         return None  # (``zero_grad`` puts the views back)
     ropes = [t for v in m._rope_cache.values() for t in v]
     return (list(map(id, mods)), list(map(id, ps)), list(map(id, ropes)), list(map(torch.Tensor.data_ptr, ps)),
-            [(p.requires_grad, p._llmctl_writes if getattr(p, "_llmctl_grad_sink", None) is sink else 0, len(p._post_accumulate_grad_hooks or ())) for p in ps],
+            [(p.requires_grad, p._llmctl_writes if written else 0) for p, written in zip(ps, sinked)],
             at, dict(vars(m.cfg)), dict(vars(m.pc)), engine.knobs,
             dict(GEMM64_CONFIGS), dict(GEMM64_SHAPE_CONFIGS), torch.are_deterministic_algorithms_enabled(), (mods, ps, ropes))
 

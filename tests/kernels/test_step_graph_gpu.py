@@ -97,6 +97,32 @@ def test_what_listens_is_heard(native_lib):
     assert p.grad is not None and p.grad.data_ptr() == eng.flat.grad.data_ptr() + 2 * eng.flat.offsets[id(p)]
 
 
+def test_gradient_hooks_are_heard(native_lib):
+    """Post-accumulate hooks: a user's that is there from the first step on (on a weight whose gradient a product writes, on a vector), and one in the place of the engine's own."""
+    eng, g, seen = engine(), torch.Generator().manual_seed(5), []
+    l = eng.model.layers[0]
+    hooks = [p.register_post_accumulate_grad_hook(lambda p: seen.append(1)) for p in (l.wo, l.attn_norm_w)]
+    step = lambda: eng.train_step([batch(eng, g, 2, 128)])  # noqa: E731
+    for n in range(1, 6):
+        step()
+        assert len(seen) == 2 * n
+    assert len(eng.step_graphs.table) == 0
+    for h in hooks:
+        h.remove()
+    for _ in range(4):
+        step()
+    assert len(eng.step_graphs.table) == 1 and len(seen) == 10
+    eng, seen = engine("gpt2-125m", 2), []
+    for _ in range(4):
+        step()
+    assert len(eng.step_graphs.table) == 1
+    p = next(p for p in eng.flat.params if p._post_accumulate_grad_hooks)
+    p._post_accumulate_grad_hooks.clear()
+    p.register_post_accumulate_grad_hook(lambda p: (seen.append(1), eng.sync._on_grad(p)) and None)
+    step(), step()
+    assert len(seen) == 2
+
+
 def test_memsets_of_a_recording_are_counted(native_lib):
     x = torch.ones(1 << 22, device="cuda")
     for f, n in ((lambda: x.mul_(1.0), 0), (lambda: x.sum(), None)):
