@@ -39,6 +39,28 @@ def _watched() -> bool:
             or not C._autograd._saved_tensors_hooks_is_enabled() or torch.cuda.is_current_stream_capturing())
 
 
+_STEP = ("_gradients", "_forward_backward", "_packing")  # the engine's methods in a recording
+
+
+def _own_code(engine) -> bool:
+    """Nobody has put code of their own, by a subclass or on an object, in the place of what a recording runs once."""
+    from llmctl.comms.overlap import GradSyncEngine
+    from llmctl.exec.linear import GradSink
+    from llmctl.runtime.engine import TrainingEngine
+    from llmctl.runtime.flat import FlatParameters
+
+    return (all(getattr(type(engine), n) is getattr(TrainingEngine, n) and n not in vars(engine) for n in _STEP)
+            and all(type(o) is t and not any(map(callable, vars(o).values()))
+                    for o, t in ((engine.sync, GradSyncEngine), (engine.flat, FlatParameters), (engine.grad_sink, GradSink))))
+
+
+def _values(v):
+    """A copy of a configuration's values that later changes inside it do not reach."""
+    if isinstance(v, dict):
+        return {k: _values(x) for k, x in v.items()}
+    return [_values(x) for x in v] if isinstance(v, (list, tuple)) else v
+
+
 def fingerprint(engine) -> Optional[Tuple]:
     """What the recorded calls of a step depend on besides its batch; None: this step must run eagerly."""
     from torch.nn.modules import module as nnm
@@ -51,7 +73,7 @@ def fingerprint(engine) -> Optional[Tuple]:
     if (engine.env.world_size > 1 or engine.eflat is not None or engine.pipeline is not None or engine.faults
             or c.pack_sequences or opt.overlap_update or opt._pending or flat.main_grads or sync is None or not sync.enabled
             or type(m) is not DecoderLM or m.cfg.is_moe or m.pc.activation_checkpoint != "none"
-            or any(n in vars(engine) for n in ("_forward_backward", "_packing", "_gradients")) or not use_native(flat.data)
+            or not _own_code(engine) or not use_native(flat.data)
             or torch.cuda.current_device() != engine.device.index
             or nnm._global_forward_hooks or nnm._global_forward_pre_hooks or nnm._global_backward_hooks or nnm._global_backward_pre_hooks or _watched()):
         return None
@@ -77,7 +99,7 @@ def fingerprint(engine) -> Optional[Tuple]:
     ropes = [t for v in m._rope_cache.values() for t in v]
     return (list(map(id, mods)), list(map(id, ps)), list(map(id, ropes)), list(map(torch.Tensor.data_ptr, ps)),
             [(p.requires_grad, p._llmctl_writes if written else 0) for p, written in zip(ps, sinked)],
-            at, dict(vars(m.cfg)), dict(vars(m.pc)), engine.knobs,
+            at, _values(vars(m.cfg)), dict(vars(m.pc)), engine.knobs,
             dict(GEMM64_CONFIGS), dict(GEMM64_SHAPE_CONFIGS), torch.are_deterministic_algorithms_enabled(), (mods, ps, ropes))
 
 

@@ -8,12 +8,12 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def engine(model="tiny", layers=2, knob=True, tokens=(2, 128), heads=None, **kw):
+def engine(model="tiny", layers=2, knob=True, tokens=(2, 128), heads=None, cls=None, **kw):
     from llmctl.models import get_model_config
     from llmctl.runtime.engine import TrainingConfig, TrainingEngine
 
     cfg = dataclasses.replace(get_model_config(model), layers=layers, **({} if heads is None else dict(heads=heads, kv_heads=heads)))
-    return TrainingEngine(TrainingConfig(model_name_or_path=model, batch_size=tokens[0], seq_len=tokens[1], device="cuda", log_level="warning",
+    return (cls or TrainingEngine)(TrainingConfig(model_name_or_path=model, batch_size=tokens[0], seq_len=tokens[1], device="cuda", log_level="warning",
                                          learning_rate=1e-3, max_steps=50, seed=3, perf_knobs={"step_graph": knob}, **kw), cfg)
 
 
@@ -121,6 +121,37 @@ def test_gradient_hooks_are_heard(native_lib):
     p.register_post_accumulate_grad_hook(lambda p: (seen.append(1), eng.sync._on_grad(p)) and None)
     step(), step()
     assert len(seen) == 2
+
+
+def test_steps_of_a_subclass_run_its_own_code(native_lib):
+    """What an engine of another class, or its configuration, changes from step to step is not frozen in a recording."""
+    from llmctl.runtime.engine import TrainingEngine
+    from llmctl.runtime.step_graph import fingerprint, same
+
+    class Weighted(TrainingEngine):
+        calls = 0
+
+        def _forward_backward(self, *a, **kw):
+            self.calls += 1
+            return super()._forward_backward(*a, **kw)
+
+    class Named(TrainingEngine):  # overrides nothing that a step runs
+        def evaluate(self, batches):
+            return 0.0
+
+    for cls, calls, recorded in ((Weighted, 5, 0), (Named, None, 1)):
+        eng, g = engine(cls=cls), torch.Generator().manual_seed(6)
+        for _ in range(5):
+            eng.train_step([batch(eng, g, 2, 128)])
+        assert len(eng.step_graphs.table) == recorded and getattr(eng, "calls", None) == calls
+    before = fingerprint(eng)
+    assert same(before, fingerprint(eng))
+    for d, k in ((eng.model.cfg.rope, "base"), (eng.model.cfg.attention, "scale")):
+        old = dict(d)
+        d[k] = 123.0
+        assert not same(before, fingerprint(eng))
+        d.clear(), d.update(old)
+    assert same(before, fingerprint(eng))
 
 
 def test_memsets_of_a_recording_are_counted(native_lib):
