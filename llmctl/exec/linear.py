@@ -146,6 +146,12 @@ def _small_operand(t: torch.Tensor, dtypes=(torch.bfloat16,)) -> bool:
     return st[1] == 1 and st[0] & 7 == 0 and st[0] >= t.shape[1] and t.data_ptr() & 15 == 0
 
 
+def _small_bias(b: torch.Tensor, N: int) -> bool:
+    """The same of a bias."""
+    return (type(b) in _PLAIN and b.is_cuda and b.dtype is torch.bfloat16 and not _is_wrapped(b) and not _is_legacy_batched(b) and b.shape == (N,)
+            and b.is_contiguous() and b.data_ptr() & 7 == 0)
+
+
 def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
     """``gemm_small`` takes operands of these sizes; sizes with a tuned gemm64 config stay with that."""
     from llmctl.ops._lib import use_native
@@ -169,8 +175,7 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
             or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
         return None
     x2 = x if x.dim() == 2 else x.view(M, K)
-    if not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (b.dtype is torch.bfloat16 and b.is_cuda and b.is_contiguous()
-                                                                  and b.shape == (N,) and b.data_ptr() & 7 == 0)):
+    if not _small_ok("fwd", M, N, K, x2, w) or not (b is None or _small_bias(b, N)):
         return None
     from llmctl.ops._lib import native
 

@@ -140,3 +140,18 @@ def test_a_prompts_products(M, N, K, act, monkeypatch):
     want = 0.5 * want * (1 + torch.tanh(0.7978845608028654 * (want + 0.044715 * want ** 3)))
     # a gelu's slope is at most 1.13; its own fp32 steps: a few roundings of values up to |x| (1 + tanh)
     assert ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1.13 * (K + 16) * 2.0 ** -24 * mag + 2.0 ** -20 * mag).all()
+
+
+def test_a_transformed_bias_stays_with_the_library():
+    """A bias that vmap runs over, old or new, or of a class of its own: as the library takes them."""
+    x, w, b = (torch.randn(*s, device="cuda").bfloat16() for s in ((64, 256), (256, 256), (3, 256)))
+
+    class Own(torch.Tensor):
+        pass
+
+    with torch.no_grad():
+        assert L.small_linear(x, w, b[0], "eager") is not None
+        for over in (torch.vmap, torch._vmap_internals._vmap):
+            assert torch.equal(over(lambda r: L.forward_linear(x, w, r))(b), over(lambda r: torch.nn.functional.linear(x, w, r))(b))
+        got = L.forward_linear(x, w, b[0].as_subclass(Own))
+        assert type(got) is Own and torch.equal(got.as_subclass(torch.Tensor), torch.nn.functional.linear(x, w, b[0]))
