@@ -138,6 +138,12 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _is_wrapped, _is_legacy_batched = torch._C._functorch.is_functorch_wrapped_tensor, torch._C._functorch.is_legacy_batchedtensor
 
 
+def _calls_are_seen() -> bool:
+    """Something in this thread traces, counts or replaces the library's calls (which take symbolic sizes, and other ones when a trace is run)."""
+    C = torch._C
+    return C._len_torch_dispatch_stack() > 0 or C._len_torch_function_stack() > 0 or C._get_tracing_state() is not None
+
+
 def _small_operand(t: torch.Tensor, dtypes=(torch.bfloat16,)) -> bool:
     """A matrix of aligned rows that ``gemm_small`` reads, and no tensor of a transform (vmap)."""
     if type(t) not in _PLAIN or not t.is_cuda or t.dtype not in dtypes or t.dim() != 2 or _is_wrapped(t) or _is_legacy_batched(t):
@@ -164,6 +170,8 @@ def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
 def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, layout: str = "fwd", act: int = 0) -> Optional[torch.Tensor]:
     """``act(x @ w^T (+ b))`` on ``gemm_small`` where it takes it and no gradient is wanted of it (the forward of an autograd function, serving); else
     None.  ``layout``: the rule of ``small_pays``; ``act``: as in csrc/stream_linear.h (0: none)."""
+    if _calls_are_seen():
+        return None
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
     if not M or not small_pays(layout, M, N, K) or not w.is_cuda or knobs().fwd64 != "auto":
@@ -186,6 +194,8 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
 
 def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``dy2 @ w`` on ``gemm_small`` (into ``out``) where it takes it; else None.  Weights whose sink was made to keep W^T copies stay with them."""
+    if _calls_are_seen():
+        return None
     M, (O, I) = dy2.shape[0], w.shape
     if dy2.dim() != 2 or dy2.shape[1] != O or not small_pays("dgrad", M, I, O) or knobs().dgrad64 != "auto" or torch.is_grad_enabled():
         return None
@@ -201,6 +211,8 @@ def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] 
 
 def small_wgrad(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate: bool, gb: Optional[torch.Tensor] = None, add: bool = False) -> bool:
     """``g (+)= dy2^T x2`` (and ``gb (+)= dy2.sum(0)``) on ``gemm_small`` where it takes them; False: nothing done."""
+    if _calls_are_seen():
+        return False
     M, N, K = dy2.shape[1], x2.shape[1], dy2.shape[0]
     if not small_pays("wgrad", M, N, K, gb is not None) or not knobs().wgrad_kernel or torch.is_grad_enabled():
         return False
@@ -221,7 +233,7 @@ def small_back(dy2: torch.Tensor, p: torch.nn.Parameter, w: torch.Tensor, x2: to
     layer's product, so 279."""
     sink: Optional[GradSink] = getattr(p, "_llmctl_grad_sink", None)
     T, (O, I) = dy2.shape[0], w.shape
-    if (sink is None or sink.always_transpose or dy2.dim() != 2 or dy2.shape[1] != O or x2.shape != (T, I) or -(-O // 32) * -(-I // 32) > 512
+    if (sink is None or _calls_are_seen() or sink.always_transpose or dy2.dim() != 2 or dy2.shape[1] != O or x2.shape != (T, I) or -(-O // 32) * -(-I // 32) > 512
             or not small_pays("dgrad", T, I, O) or not small_pays("wgrad", O, I, T) or torch.is_grad_enabled()
             or knobs().dgrad64 != "auto" or not knobs().wgrad_kernel):
         return None

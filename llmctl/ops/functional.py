@@ -362,7 +362,7 @@ class _CrossEntropy(torch.autograd.Function):
             loss, lse = ref.cross_entropy_fwd(logits, labels, ignore_index)
         ctx.save_for_backward(logits, lse, labels)
         ctx.ignore_index, ctx.denom = ignore_index, denom
-        if use_native(logits) and loss.numel() <= 32768 and type(denom) in (int, float) and denom:
+        if use_native(logits) and type(denom) in (int, float) and denom and not torch.jit.is_tracing() and loss.numel() <= 32768:
             return native().loss_mean(loss, denom)
         return loss.sum() / denom
 

@@ -155,3 +155,43 @@ def test_a_transformed_bias_stays_with_the_library():
             assert torch.equal(over(lambda r: L.forward_linear(x, w, r))(b), over(lambda r: torch.nn.functional.linear(x, w, r))(b))
         got = L.forward_linear(x, w, b[0].as_subclass(Own))
         assert type(got) is Own and torch.equal(got.as_subclass(torch.Tensor), torch.nn.functional.linear(x, w, b[0]))
+
+
+def test_traced_and_counted_products_stay_with_the_library():
+    """Modes that see the library's calls, and traces, which are run with other sizes, see the products as they ever did, forward and backward."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    x, w, b = (torch.randn(*s, device="cuda").bfloat16() for s in ((65, 256), (256, 256), (256,)))  # (of 65 tokens the library had all three products)
+    longer = torch.randn(101, 256, device="cuda").bfloat16()
+    assert L.small_linear(x, w, b, "eager") is not None
+
+    def step(x):
+        x, v = x.detach().requires_grad_(), w.detach().requires_grad_()
+        return torch.autograd.grad(L.linear(x, v, b), (x, v), torch.ones(x.shape[0], 256, device="cuda", dtype=x.dtype))
+
+    with torch.no_grad():
+        for traced in (make_fx(lambda x: L.forward_linear(x, w, b), tracing_mode="symbolic", _allow_non_fake_inputs=True)(x),
+                       make_fx(lambda x: L.forward_linear(x, w, b))(x), torch.jit.trace(lambda x: L.forward_linear(x, w, b), x, check_trace=False)):
+            assert torch.equal(traced(longer), torch.nn.functional.linear(longer, w, b))
+
+    def back(x):
+        x = x.detach().requires_grad_()
+        return torch.autograd.grad(L.linear(x, w, b).sum(), x)[0]
+
+    traced = make_fx(back, tracing_mode="symbolic", _allow_non_fake_inputs=True)(x)
+    got, want = traced(longer).float(), back(longer).float()
+    assert float((got - want).norm()) <= 2.0 ** -7 * float(want.norm())  # each rounds its sums to bf16 once
+    with FlopCounterMode(display=False) as count:
+        step(x)
+    assert count.get_total_flops() == 3 * 2 * 65 * 256 * 256
+
+
+def test_a_traced_loss_takes_other_lengths():
+    from llmctl import ops
+
+    short, long = (torch.randn(T, 64, device="cuda").bfloat16() for T in (32, 32769))
+    traced = torch.jit.trace(lambda x, y: ops.cross_entropy(x, y, reduction_denom=16.0), (short, torch.zeros(32, dtype=torch.int64, device="cuda")), check_trace=False)
+    y = torch.zeros(32769, dtype=torch.int64, device="cuda")
+    want = float(torch.nn.functional.cross_entropy(long.double(), y, reduction="sum")) / 16
+    assert abs(float(traced(long, y)) - want) <= 64 * 2.0 ** -24 * want
