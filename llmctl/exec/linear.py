@@ -162,7 +162,7 @@ def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
     """``gemm_small`` takes operands of these sizes; sizes with a tuned gemm64 config stay with that."""
     from llmctl.ops._lib import use_native
 
-    return (M > 0 and K > 0 and N & 7 == 0 and ((M if layout == "wgrad" else K) & 7) == 0 and _gemm64_enabled()
+    return (M > 0 and N > 0 and K > 0 and N & 7 == 0 and ((M if layout == "wgrad" else K) & 7) == 0 and _gemm64_enabled()
             and not (layout in GEMM64_CONFIGS or (layout, M, N, K) in GEMM64_SHAPE_CONFIGS)
             and all(map(_small_operand, ts)) and use_native(ts[0]))
 

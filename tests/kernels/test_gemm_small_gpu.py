@@ -195,3 +195,14 @@ def test_a_traced_loss_takes_other_lengths():
     y = torch.zeros(32769, dtype=torch.int64, device="cuda")
     want = float(torch.nn.functional.cross_entropy(long.double(), y, reduction="sum")) / 16
     assert abs(float(traced(long, y)) - want) <= 64 * 2.0 ** -24 * want
+
+
+@pytest.mark.parametrize("shape", [(64, 64), (2, 40, 64)])
+def test_no_outputs(shape):
+    """A weight without rows: an empty result, as from the library."""
+    from llmctl import ops
+
+    x, w, b = (torch.randn(*s, device="cuda").bfloat16() for s in (shape, (0, 64), (0,)))
+    with torch.no_grad():
+        assert L.forward_linear(x, w, b).shape == (*shape[:-1], 0)
+        assert ops.decode_linear(x, w, b).shape == (*shape[:-1], 0)
