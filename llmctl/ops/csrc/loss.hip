@@ -98,9 +98,9 @@ __global__ __launch_bounds__(256) void ce_bwd_kernel(const float* __restrict__ d
   }
 }
 
-// out = factor * sum(loss), one workgroup, summed in 64 bits: up to 32768 rows (128 KB, 5 us) one launch where the library takes two, three with the memset that it
+// out = sum(loss) / denom, one workgroup, summed in 64 bits: up to 32768 rows (128 KB, 5 us) one launch where the library takes two, three with the memset that it
 // clears its counters with from 16384 rows on.
-__global__ __launch_bounds__(1024) void loss_mean_kernel(const float* __restrict__ loss, int T, float factor, float* __restrict__ out) {
+__global__ __launch_bounds__(1024) void loss_mean_kernel(const float* __restrict__ loss, int T, double denom, float* __restrict__ out) {
   __shared__ double part[16];
   double s = 0.0;
   for (int i = threadIdx.x; i < T; i += 1024) s += (double)loss[i];
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(1024) void loss_mean_kernel(const float* __restrict
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 16; ++w) s += part[w];
-    out[0] = (float)s * factor;
+    out[0] = (float)(s / denom);
   }
 }
 
@@ -153,7 +153,7 @@ at::Tensor loss_mean(const at::Tensor& loss, double denom) {
   LLMCTL_CHECK(loss.is_cuda() && loss.scalar_type() == at::kFloat && loss.is_contiguous() && loss.numel() <= 32768, "loss_mean: contiguous fp32, at most 32768 rows");
   const c10::DeviceGuard g(loss.device());
   at::Tensor out = at::empty({}, loss.options());
-  hipLaunchKernelGGL(loss_mean_kernel, dim3(1), dim3(1024), 0, stream(), loss.data_ptr<float>(), (int)loss.numel(), 1.f / (float)denom, out.data_ptr<float>());
+  hipLaunchKernelGGL(loss_mean_kernel, dim3(1), dim3(1024), 0, stream(), loss.data_ptr<float>(), (int)loss.numel(), denom, out.data_ptr<float>());
   return out;
 }
 

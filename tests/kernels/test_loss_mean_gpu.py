@@ -35,3 +35,11 @@ def test_squared_norm(n, dtype):
     want = x.double().square().sum() + 2
     # a thread's own additions, a tree over 1024 threads, at most 512 additions to the one sum
     assert (out.double() - want).abs() <= (n // 524288 * 8 + 8 + 10 + 512) * 2.0 ** -24 * want
+
+
+@pytest.mark.parametrize("denom", [3, 1e38, 1e39])
+def test_any_denominator(denom):
+    """The quotient is rounded once, whether or not the denominator is a 32-bit number."""
+    logits, labels = torch.randn(64, 41, device="cuda").bfloat16(), torch.zeros(64, dtype=torch.int64, device="cuda")
+    want = native().cross_entropy_fwd(logits, labels, -100)[0].double().sum() / denom
+    assert abs(float(ops.cross_entropy(logits, labels, reduction_denom=denom)) - float(want)) <= 2.0 ** -24 * float(want)
