@@ -30,6 +30,7 @@ import torch
 import torch.nn.functional as F
 
 from llmctl.config.knobs import knobs
+from llmctl.ops._lib import native, use_native  # (once: an import in a function is 0.5 us a call)
 
 
 # gemm64_ex config: knob gemm64_config (see gemm64_config below).  A tuning cache
@@ -138,10 +139,13 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _is_wrapped, _is_legacy_batched = torch._C._functorch.is_functorch_wrapped_tensor, torch._C._functorch.is_legacy_batchedtensor
 
 
+_modes, _function_modes, _tracing = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._is_tracing
+_any_autocast, _forward_ad = torch._C._is_any_autocast_enabled, torch.autograd.forward_ad
+
+
 def _calls_are_seen() -> bool:
-    """Something in this thread traces, counts or replaces the library's calls (which take symbolic sizes, and other ones when a trace is run)."""
-    C = torch._C
-    return C._len_torch_dispatch_stack() > 0 or C._len_torch_function_stack() > 0 or C._get_tracing_state() is not None
+    """Something in this thread traces, counts or replaces the library's calls (which take symbolic sizes, and other ones when a trace is run).  0.3 us."""
+    return _modes() or _function_modes() or _tracing()
 
 
 def _small_operand(t: torch.Tensor, dtypes=(torch.bfloat16,)) -> bool:
@@ -160,8 +164,6 @@ def _small_bias(b: torch.Tensor, N: int) -> bool:
 
 def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
     """``gemm_small`` takes operands of these sizes; sizes with a tuned gemm64 config stay with that."""
-    from llmctl.ops._lib import use_native
-
     return (M > 0 and N > 0 and K > 0 and N & 7 == 0 and ((M if layout == "wgrad" else K) & 7) == 0 and _gemm64_enabled()
             and not (layout in GEMM64_CONFIGS or (layout, M, N, K) in GEMM64_SHAPE_CONFIGS)
             and all(map(_small_operand, ts)) and use_native(ts[0]))
@@ -170,23 +172,19 @@ def _small_ok(layout: str, M: int, N: int, K: int, *ts: torch.Tensor) -> bool:
 def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, layout: str = "fwd", act: int = 0) -> Optional[torch.Tensor]:
     """``act(x @ w^T (+ b))`` on ``gemm_small`` where it takes it and no gradient is wanted of it (the forward of an autograd function, serving); else
     None.  ``layout``: the rule of ``small_pays``; ``act``: as in csrc/stream_linear.h (0: none)."""
-    if _calls_are_seen():
-        return None
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    if not M or not small_pays(layout, M, N, K) or not w.is_cuda or knobs().fwd64 != "auto":
+    if not M or type(M * N) is not int or not small_pays(layout, M, N, K) or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
+        return None  # (symbolic and traced sizes are no ints)
+    if layout == "eager" and not small_pays("fwd", M, N, K) and torch.cuda.is_current_stream_capturing():
         return None
-    if layout == "eager" and torch.cuda.is_current_stream_capturing() and not small_pays("fwd", M, N, K):
-        return None
-    if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not x.is_contiguous() or torch.is_autocast_enabled("cuda")
+    if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not x.is_contiguous() or _any_autocast()
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
-            or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
+            or _forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
         return None
     x2 = x if x.dim() == 2 else x.view(M, K)
     if not _small_ok("fwd", M, N, K, x2, w) or not (b is None or _small_bias(b, N)):
         return None
-    from llmctl.ops._lib import native
-
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     native().gemm_small(x2, w, y, False, False, False, b, None, False, act)
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
@@ -202,8 +200,6 @@ def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] 
     sink = getattr(w, "_llmctl_grad_sink", None)
     if (sink is not None and sink.always_transpose) or not _small_ok("dgrad", M, I, O, dy2, w, *(() if out is None else (out,))):
         return None
-    from llmctl.ops._lib import native
-
     dx = torch.empty(M, I, dtype=dy2.dtype, device=dy2.device) if out is None else out
     native().gemm_small(dy2, w, dx, False, True, False)
     return dx
@@ -220,8 +216,6 @@ def small_wgrad(g: torch.Tensor, dy2: torch.Tensor, x2: torch.Tensor, accumulate
         return False
     if gb is not None and not (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == M):
         return False
-    from llmctl.ops._lib import native
-
     native().gemm_small(dy2, x2, g, True, True, accumulate, None, gb, add)
     return True
 
@@ -246,8 +240,6 @@ def small_back(dy2: torch.Tensor, p: torch.nn.Parameter, w: torch.Tensor, x2: to
     if (not _small_ok("dgrad", T, I, O, dy2, w) or not _small_ok("wgrad", O, I, T, x2) or not _small_operand(g, (torch.bfloat16, torch.float32))
             or not (gb is None or (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == O))):
         return None
-    from llmctl.ops._lib import native
-
     dx = torch.empty(T, I, dtype=dy2.dtype, device=dy2.device)
     native().gemm_small_back(dy2, w, dx, x2, g, more, gb, add)
     sink.close(p)
