@@ -1,5 +1,6 @@
 """Replayed training steps (``llmctl.runtime.step_graph``) against eager ones, and the steps that must not be replayed."""
 
+import ctypes
 import dataclasses
 
 import pytest
@@ -22,14 +23,17 @@ def batch(eng, g, b, s):
     return t[:, :-1], t[:, 1:]  # (rows of another tensor, as a loader's are)
 
 
-# (the last two: heads of 128, whose dK/dV kernel counts its items in memory, and a loss over 16384 tokens, which the library sums with a memset: such steps stay eager)
+# (the last three: heads of 128, whose dK/dV kernel clears its counters with a launch of its own; a loss over 16384 tokens, one launch too; and one over more than 32768,
+# which the library sums with a memset, so that its steps stay eager)
 @pytest.mark.parametrize("model,layers,sizes,heads,recorded", [
     ("tiny", 2, [(2, 128)], None, 1), ("tiny", 2, [(1, 65), (3, 100), (8, 512)], None, 3), ("gpt2-125m", 2, [(2, 64), (1, 333)], None, 2),
-    ("tiny", 2, [(2, 128), (5, 256)], 2, 2), ("tiny", 1, [(32, 512)], None, None)])
+    ("tiny", 2, [(2, 128), (5, 256)], 2, 2), ("tiny", 1, [(32, 512)], None, 1), ("tiny", 1, [(65, 512)], None, 0)])
 def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes, heads, recorded):
     """Losses, norms, gradients and states over many steps of alternating shapes, other work on the device between them.  Both sides run the same
     kernels; what differs from run to run is the order of the clip norm's atomics (and a library product's partial sums), which moves the weights by
     rounding: the bound is four times the spread of two eager runs, or rounding of bf16 weights (2^-9) where they happen to agree."""
+    from llmctl.runtime.step_graph import pays
+
     def run(knob):
         eng, g, out = engine(model, layers, knob, heads=heads), torch.Generator().manual_seed(1), []
         for step in range(5):
@@ -38,7 +42,8 @@ def test_replayed_steps_match_eager_ones(native_lib, model, layers, sizes, heads
                 keep = torch.full((1 << 20,), float(step), device="cuda")  # memory that a stale pointer would hit
                 out += [r["loss"], r["grad_norm"], keep.sum() * 0]
         torch.cuda.synchronize()
-        assert recorded is None or len(eng.step_graphs.table) == (recorded if knob else 0)
+        assert len(eng.step_graphs.table) == (recorded if knob else 0)
+        assert all(pays(eng.flat.numel, b * s, layers) for b, s in sizes)  # (none is left eager for its length)
         return torch.stack([o.float().reshape(()) for o in out]), eng.flat.grad.float(), eng.optimizer.master, eng.optimizer.exp_avg
 
     a, b, c = run(True), run(False), run(False)
@@ -154,17 +159,27 @@ def test_steps_of_a_subclass_run_its_own_code(native_lib):
     assert same(before, fingerprint(eng))
 
 
-def test_memsets_of_a_recording_are_counted(native_lib):
-    x = torch.ones(1 << 22, device="cuda")
-    for f, n in ((lambda: x.mul_(1.0), 0), (lambda: x.sum(), None)):
-        f()
-        g = torch.cuda.CUDAGraph(keep_graph=True)
-        with torch.cuda.graph(g):
-            out = f()
-        found = native_lib.graph_memsets(g.raw_cuda_graph())
-        assert found == n if n is not None else found >= 0
-        del out
-        g.reset()
+class _Memset(ctypes.Structure):  # hipMemsetParams
+    _fields_ = [("dst", ctypes.c_void_p), ("elementSize", ctypes.c_uint), ("height", ctypes.c_size_t), ("pitch", ctypes.c_size_t), ("value", ctypes.c_uint),
+                ("width", ctypes.c_size_t)]
+
+
+@pytest.mark.parametrize("memsets", [0, 1, 3])
+def test_memsets_of_a_graph_are_counted(native_lib, memsets):
+    """In a graph that was put together by hand and is never run, and in a recording that has none."""
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    x, graph, node = torch.ones(256, device="cuda"), ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipGraphCreate(ctypes.byref(graph), 0) == 0
+    for _ in range(memsets):
+        assert hip.hipGraphAddMemsetNode(ctypes.byref(node), graph, None, ctypes.c_size_t(0), ctypes.byref(_Memset(x.data_ptr(), 4, 1, 4 * x.numel(), 0, x.numel()))) == 0
+    assert hip.hipGraphAddEmptyNode(ctypes.byref(node), graph, None, ctypes.c_size_t(0)) == 0
+    assert native_lib.graph_memsets(graph.value) == memsets
+    assert hip.hipGraphDestroy(graph) == 0
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        x.mul_(1.0)
+    assert native_lib.graph_memsets(g.raw_cuda_graph()) == 0
+    g.reset()
 
 
 def test_long_steps_stay_eager(native_lib):
