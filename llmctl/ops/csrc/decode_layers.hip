@@ -29,7 +29,7 @@
 // What it took (one row, gpt2-125m, context 129, whole step; five launches a layer 369 us): 64 workgroups of 1024 threads 369 us, registers spilt; 512 threads and
 // the pointers in LDS 282; global, not flat, loads 270; no load under a condition (its use waits for all loads) 254; the next weights asked for after a
 // product's results are sent 234; 128 workgroups 219; asking again only for missing words 214; three activations to a word 206.  Now, us, launches / this: one row
-// context 129 367 / 200, 700 399 / 232, 2000 425 / 251; two rows 382 / 237; three 419 / 310; four 425 / 332.  Of a layer's 13 us half is the words' way.
+// context 129 381 / 203, 700 406 / 233, 2000 432 / 252; at 129 two rows 396 / 239, three 418 / 294, four 420 / 297.  Of a layer's 13 us half is the words' way.
 #include "common.h"
 
 namespace llmctl {

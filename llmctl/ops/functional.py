@@ -708,8 +708,7 @@ def decode_norm_qkv_cache(x, res, nw, nb, eps: float, w, b, nq: int, nkv: int, k
 def decode_layers_ok(hidden: int, heads: int, kv_heads: int, ffn: int, layers: int, rows: int, cache) -> bool:
     """Does ``csrc/decode_layers.hip`` run a whole decode step of this size in one launch (LayerNorm, biases, GELU and learned positions are the caller's to
     know), and does it pay?  Up to four rows, where the launches are most of a step: gpt2-125m, us a step, a launch per product / this: one row at context 129
-    367 / 200, 2000 425 / 251, two rows 382 / 237, four 425 / 332 (a row more costs 45, beside launches 20); four layers of 256, one row 122 / 77, of 1024, four
-    rows 175 / 161."""
+    381 / 203, 2000 432 / 252, at 129 two rows 396 / 239, four 420 / 297; four layers of 256, one row 127 / 78, of 1024, four rows 171 / 153."""
     return (knobs().decode_layers and use_native(cache) and cache.dtype == torch.bfloat16 and cache.is_contiguous() and 1 <= rows <= 4 and 1 <= layers <= 32
             and cache.dim() == 5 and cache.shape[-1] == 64 and cache.data_ptr() % 16 == 0 and cache[0].numel() < 1 << 35
             and hidden % 256 == 0 and 256 <= hidden <= 1024 and heads == kv_heads and heads * 64 == hidden and ffn == 4 * hidden

@@ -3,8 +3,8 @@
 A step of a small model is bound by the host: every launch passes through an autograd function, its checks and the
 dispatcher, 15 to 20 us each, while the kernels take 3 to 10.  The recording holds ``zero_grad``, the model's forward and backward
 and ``settle_grads``; the clip norm and AdamW, whose step count and learning rate are launch arguments, stay outside and run as
-ever.  Whole steps, one MI355X, us, eager / replayed: tiny (2 layers) 256 tokens 1333 / 263, 4096 tokens 1742 / 628; gpt2-125m (12
-layers) 128 tokens 7925 / 3165, 1024 7944 / 4700, 2048 8088 / 5793.
+ever.  Whole steps, one MI355X, us, eager / replayed: tiny (2 layers) 256 tokens 940 / 262, 4096 tokens 1335 / 627; gpt2-125m (12
+layers) 128 tokens 5852 / 3210, 1024 5888 / 4699, 2048 7594 / 5745 (eager steps are the host's and differ from one to another: 1333, 1742, 7925, 7944, 8088).
 
 A replay runs no Python, so whatever a step's Python could see or change is compared with what was recorded before every
 replay (:func:`fingerprint`), and a step that anything listens to (hooks, dispatch modes, anomaly mode, faults to inject) runs eagerly."""
