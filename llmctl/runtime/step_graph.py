@@ -113,53 +113,38 @@ class StepGraph:
     def __init__(self, x: torch.Tensor, y: torch.Tensor):
         self.x, self.y = torch.empty_like(x, memory_format=torch.contiguous_format), torch.empty_like(y, memory_format=torch.contiguous_format)
         self.graph = self.loss = None
-        self.served = False  # the generator's tensors belong to graphs that were recorded in inference mode
-
-    def _begin(self, pool):
-        # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
-        for self.served in (False, True):
-            g = torch.cuda.CUDAGraph(keep_graph=True)
-            try:
-                with torch.inference_mode(self.served):  # (a graph writes the generator's seed as it begins and as it is replayed)
-                    g.capture_begin(pool=pool, capture_error_mode="thread_local")
-                return g
-            except RuntimeError as e:
-                if self.served or "nference" not in str(e):
-                    raise
 
     def capture(self, engine, denom: float, stream, pool) -> None:
         """Record.  Nothing runs, so a failure (raised) leaves the gradients as they were."""
         from llmctl.ops._lib import native
 
+        lib, g = native(), torch.classes.llmctl.StepCapture(*pool)
         with graph_capture_gc_guard(collect=False), torch.cuda.stream(stream):
-            g = self._begin(pool)
+            g.begin()
             try:
                 loss = engine._gradients(self.x, self.y, denom)
             except BaseException:
-                try:
-                    g.capture_end()
-                except RuntimeError:
-                    pass  # (the first error is the one to tell)
-                g.reset()
+                g.release()
                 raise
-            g.capture_end()
-        if native().graph_memsets(g.raw_cuda_graph()):  # (a library's sum over many blocks clears its counters so)
-            del loss
-            g.reset()
-            raise RuntimeError("the step records a memset")
-        g.instantiate()
+            try:
+                g.end()
+                if lib.graph_memsets(g.graph()):  # (a library's sum over many blocks clears its counters so)
+                    raise RuntimeError("the step records a memset")
+                g.instantiate()
+            except RuntimeError:
+                del loss
+                g.release()
+                raise
         self.graph, self.loss = g, loss
 
     def run(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
         self.x.copy_(x)
         self.y.copy_(y)
-        with torch.inference_mode(self.served):
-            self.graph.replay()
+        self.graph.replay()
         return self.loss.clone()  # (the next replay writes the graph's own)
 
     def release(self) -> None:
-        torch.cuda.synchronize(self.x.device)  # its last replay, on whatever stream
-        self.graph.reset()
+        self.graph.release()  # (waits for its last replay, on whatever stream)
         self.graph = self.loss = None
 
 

@@ -2,6 +2,7 @@
 
 import ctypes
 import dataclasses
+import threading
 
 import pytest
 import torch
@@ -64,6 +65,60 @@ def test_recorded_beside_a_serving_graph(native_lib):
     for _ in range(5):
         assert torch.isfinite(eng.train_step([batch(eng, g, 2, 128)])["loss"])
         served.replay()
+    assert len(eng.step_graphs.table) == 1
+
+
+def test_other_threads_draw_while_a_step_is_recorded(native_lib, monkeypatch):
+    """A step draws no random numbers: a thread that does, on its own stream, is not kept from it by a recording, and its numbers are those of the seed."""
+    from llmctl.runtime.flat import FlatParameters
+
+    zero_grad, drawn, failed = FlatParameters.zero_grad, [], []
+
+    def draw():
+        try:
+            drawn.append(torch.randn(64, device="cuda"))
+        except RuntimeError as e:
+            failed.append(e)
+
+    def beside(self):
+        if torch.cuda.is_current_stream_capturing():
+            t = threading.Thread(target=draw)
+            t.start(), t.join()
+        return zero_grad(self)
+
+    monkeypatch.setattr(FlatParameters, "zero_grad", beside)
+    eng, g = engine(), torch.Generator().manual_seed(7)
+    torch.cuda.manual_seed(11)
+    want = [torch.randn(64, device="cuda") for _ in range(2)]
+    torch.cuda.manual_seed(11)
+    for _ in range(5):
+        eng.train_step([batch(eng, g, 2, 128)])
+    assert len(eng.step_graphs.table) == 1 and not failed and len(drawn) == 1
+    draw()
+    assert all(torch.equal(x, y) for x, y in zip(want, drawn))
+
+
+def test_a_recording_that_fails(native_lib, monkeypatch):
+    """Its steps stay eager; other shapes are recorded, and given back with the engine."""
+    from llmctl.runtime.flat import FlatParameters
+
+    zero_grad, fail = FlatParameters.zero_grad, [True]
+
+    def broken(self):
+        zero_grad(self)
+        if fail and torch.cuda.is_current_stream_capturing():
+            fail.clear()
+            raise RuntimeError("no")
+
+    monkeypatch.setattr(FlatParameters, "zero_grad", broken)
+    eng, g = engine(), torch.Generator().manual_seed(8)
+    for b in (2, 3):
+        for _ in range(4):
+            assert torch.isfinite(eng.train_step([batch(eng, g, b, 128)])["loss"])
+        assert len(eng.step_graphs.table) == b - 2
+    eng.step_graphs.table.clear()
+    for _ in range(4):
+        assert torch.isfinite(eng.train_step([batch(eng, g, 2, 128)])["loss"])
     assert len(eng.step_graphs.table) == 1
 
 
