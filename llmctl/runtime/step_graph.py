@@ -11,7 +11,8 @@ replay (:func:`fingerprint`), and a step that anything listens to (hooks, dispat
 
 from __future__ import annotations
 
-from typing import List, Optional, Tuple
+import weakref
+from typing import Dict, List, Optional, Tuple
 
 import torch
 
@@ -148,11 +149,24 @@ class StepGraph:
         self.graph = self.loss = None
 
 
+# streams of engines that are gone, by device: the library keeps two workspaces for good per stream that its products are recorded on (160 MB), and the graphs
+# of engines that live side by side may not share one
+_idle: Dict[torch.device, List["torch.cuda.Stream"]] = {}
+
+
 class StepGraphs:
     """The recorded steps of one engine: a stream and a memory pool of its own (the graphs run one after the other, as the steps do)."""
 
     def __init__(self):
         self.table, self.seen, self.stream, self.pool = GraphTable(), None, None, None
+
+    def _take_stream(self, device: torch.device) -> None:
+        idle = _idle.setdefault(device, [])
+        try:
+            self.stream = idle.pop()
+        except IndexError:
+            self.stream = torch.cuda.Stream(device=device)
+        weakref.finalize(self, idle.append, self.stream).atexit = False
 
     def run(self, engine, batches: List[Tuple[torch.Tensor, torch.Tensor]]) -> Optional[torch.Tensor]:
         """The loss of a replayed step, its gradients in the flat buffer; None: run it eagerly."""
@@ -183,7 +197,7 @@ class StepGraphs:
         if not len(self.table):  # (a pool ends with its last graph)
             self.pool = torch.cuda.graph_pool_handle()
         if self.stream is None:
-            self.stream = torch.cuda.Stream(device=engine.device)
+            self._take_stream(engine.device)
         try:
             g = StepGraph(x, y)
             g.capture(engine, denom, self.stream, self.pool)

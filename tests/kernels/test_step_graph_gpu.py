@@ -2,6 +2,7 @@
 
 import ctypes
 import dataclasses
+import gc
 import threading
 
 import pytest
@@ -120,6 +121,28 @@ def test_a_recording_that_fails(native_lib, monkeypatch):
     for _ in range(4):
         assert torch.isfinite(eng.train_step([batch(eng, g, 2, 128)])["loss"])
     assert len(eng.step_graphs.table) == 1
+
+
+def test_streams_of_engines_that_are_gone_are_used_again(native_lib):
+    """Engines that live side by side record on streams of their own (the library's workspaces go by stream); the next one takes that of one that is gone."""
+    def recorded():
+        eng, g = engine(), torch.Generator().manual_seed(9)
+        for _ in range(4):
+            eng.train_step([batch(eng, g, 2, 128)])
+        assert len(eng.step_graphs.table) == 1
+        return eng, eng.step_graphs.stream.cuda_stream
+
+    gc.collect()
+    a, on_a = recorded()
+    b, on_b = recorded()
+    assert on_a != on_b
+    del a
+    gc.collect()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    c, on_c = recorded()
+    assert on_c == on_a
+    assert torch.cuda.memory_allocated() - before < 64 << 20  # an engine of this model, and no further workspaces
 
 
 def test_what_listens_is_heard(native_lib):
