@@ -248,6 +248,41 @@ def small_back(dy2: torch.Tensor, p: torch.nn.Parameter, w: torch.Tensor, x2: to
     return dx
 
 
+@functools.lru_cache(maxsize=4096)
+def _back_splits(T: int, O: int, I: int, bias: bool) -> int:
+    """The rule of ``gemm_tall_back`` (csrc/gemm_tall.hip), by size: ranges of the weight gradient, 0: two launches are as fast."""
+    return native().gemm64_back_splits(T, O, I, bias)
+
+
+def tall_back(dy2: torch.Tensor, p: torch.nn.Parameter, w: torch.Tensor, x2: torch.Tensor,
+              b: Optional[torch.nn.Parameter] = None) -> Optional[torch.Tensor]:
+    """:func:`small_back` on the 256 x 128 tiles (``gemm_tall_back``): both gradients of a sinked ``p`` in one launch where that takes less time than two; None: nothing
+    done.  Steps of gpt2-125m, us: 8192 tokens 11450, so 11240; 3912 8360 / 7830; 1920 5750 / 5130; 1326 4880 /
+    4440 (the data gradient was the library's there)."""
+    sink: Optional[GradSink] = getattr(p, "_llmctl_grad_sink", None)
+    T, (O, I) = dy2.shape[0], w.shape
+    if (sink is None or O & 255 or I & 255 or T < 256 or T > DGRAD64_TOKENS or not w.is_cuda or _calls_are_seen() or sink.always_transpose or dy2.dim() != 2
+            or dy2.shape[1] != O or x2.shape != (T, I) or not _back_splits(T, O, I, b is not None) or torch.is_grad_enabled() or knobs().dgrad64 != "auto"
+            or not knobs().wgrad_kernel or gemm64_config("wgrad", O, I, T) // 100 != 3 or gemm64_config("dgrad", T, I, O) // 100 != 3):
+        return None
+    gb, add = None, False
+    if b is not None:
+        if getattr(b, "_llmctl_grad_sink", None) is not sink:
+            return None
+        gb, add = sink.open(b)
+    g, more = sink.open(p)
+    if (not _small_ok("dgrad", T, I, O, dy2, w) or not _small_ok("wgrad", O, I, T, x2) or not _small_operand(g, (torch.bfloat16, torch.float32))
+            or not (gb is None or (gb.dtype == g.dtype and gb.is_contiguous() and gb.is_cuda and gb.numel() == O))
+            or max(T * dy2.stride(0), T * x2.stride(0), O * w.stride(0)) >= 1 << 30):
+        return None
+    dx = torch.empty(T, I, dtype=dy2.dtype, device=dy2.device)
+    native().gemm_tall_back(dy2, w, dx, x2, g, more, _back_splits(T, O, I, b is not None), gb, add)
+    sink.close(p)
+    if b is not None:
+        sink.close(b)
+    return dx
+
+
 def dgrad64_shape_ok(tokens: int, w: torch.Tensor, fused: bool = False) -> bool:
     """Will ``dx = dy W`` for ``tokens`` rows run on gemm64?  (Decided at forward time: the
     weight's W^T copy is only kept for layers whose data gradient cannot.)  ``fused``: the
@@ -648,6 +683,8 @@ class _Linear(torch.autograd.Function):
         bias = ctx.bparam is not None and ctx.needs_input_grad[2]
         if ctx.needs_input_grad[0] and ctx.needs_input_grad[1] and ctx.wt is None:
             dx = small_back(dy2, ctx.wparam, w, x2, ctx.bparam if bias else None)
+            if dx is None:
+                dx = tall_back(dy2, ctx.wparam, w, x2, ctx.bparam if bias else None)
             if dx is not None:
                 return dx.view(*dy.shape[:-1], w.shape[1]), None, None
         if ctx.needs_input_grad[1]:

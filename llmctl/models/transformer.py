@@ -105,7 +105,7 @@ class _SwiGLUDown(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
-        from llmctl.exec.linear import small_back
+        from llmctl.exec.linear import small_back, tall_back
         from llmctl.ops._lib import native, use_native
         from llmctl.ops import ref
 
@@ -127,7 +127,11 @@ class _SwiGLUDown(torch.autograd.Function):
 
             dw = weight_grad(ctx.wparam, dout2, act2)
             return (native().swiglu_bwd(dact, gu) if use_native(gu) else ref.swiglu_bwd(dact, gu)), dw, None
-        dact = small_back(dout2, ctx.wparam, ctx.wparam, act2) if use_native(gu) and ctx.needs_input_grad[0] and ctx.needs_input_grad[1] else None
+        dact = None
+        if use_native(gu) and ctx.needs_input_grad[0] and ctx.needs_input_grad[1]:
+            dact = small_back(dout2, ctx.wparam, ctx.wparam, act2)
+            if dact is None:
+                dact = tall_back(dout2, ctx.wparam, ctx.wparam, act2)
         if dact is not None:
             return native().swiglu_bwd(dact.view(act.shape), gu), None, None
         dw = weight_grad(ctx.wparam, dout2, act2)

@@ -14,6 +14,7 @@ void set_knob(const std::string& name, int64_t value);  // knobs.cpp
 void clear_knobs();
 int64_t graph_memsets(int64_t graph);
 int64_t gemm64_wgrad_splits(int64_t M, int64_t N, int64_t K, bool bias);
+int64_t gemm64_back_splits(int64_t T, int64_t O, int64_t I, bool bias);
 int64_t decode_layers_words(int64_t hidden);
 }  // namespace llmctl
 
@@ -85,6 +86,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("car_sig_words() -> int", &llmctl::car_sig_words);
   m.def("car_error(int sig_ptr) -> int", &llmctl::car_error);
   m.def("gemm64_wgrad_splits(int M, int N, int K, bool bias) -> int", &llmctl::gemm64_wgrad_splits);
+  m.def("gemm64_back_splits(int T, int O, int I, bool bias) -> int", &llmctl::gemm64_back_splits);
   m.def("set_knob(str name, int value) -> ()", &llmctl::set_knob);
   m.def("clear_knobs() -> ()", &llmctl::clear_knobs);
   m.def("graph_memsets(int graph) -> int", &llmctl::graph_memsets);
@@ -102,6 +104,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("gemm_tall(Tensor a, Tensor b, Tensor(a!) out, bool at, bool accumulate, int splits, Tensor(b!)? bias=None, bool bias_add=False) -> ()");
   m.def("gemm_small(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, Tensor? bias=None, Tensor(b!)? sums=None, bool add_sums=False, int act=0) -> ()");
   m.def("gemm_small_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, Tensor(c!)? sums=None, bool add_sums=False) -> ()");
+  m.def("gemm_tall_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, int splits, Tensor(c!)? db=None, bool add=False) -> ()");
   m.def("gemm64_wgrad_bias(Tensor dy, Tensor x, Tensor(a!) g, bool accumulate, Tensor(b!)? db, bool add) -> bool");
   m.def("embed_grad_(Tensor ids, Tensor dy, Tensor(a!) g, bool add) -> ()");
   m.def("transpose_(Tensor src, Tensor(a!) dst) -> ()");

@@ -1807,6 +1807,20 @@ int64_t gemm64_wgrad_splits(int64_t M, int64_t N, int64_t K, bool bias) {
   return gemm_tall_splits(M, N, K, plan.n_main, (long)plan.tiles_m * plan.tiles_n - plan.n_main, plan.splits);
 }
 
+// Ranges of the weight gradient in which gemm_tall_back takes a layer's two gradients (T tokens, O outputs, I inputs); 0: two launches are as fast.
+int64_t gemm64_back_splits(int64_t T, int64_t O, int64_t I, bool bias) {
+  if (T <= 0 || O <= 0 || I <= 0 || O % TM != 0 || I % TN != 0) return 0;
+  auto us = [](long M, long N, long K) {
+    G64Args plan{};
+    plan.M = (int)M, plan.N = (int)N, plan.K = (int)((K + 2 * TK - 1) / (2 * TK) * (2 * TK)), plan.tiles_m = (int)((M + TM - 1) / TM), plan.tiles_n = (int)(N / TN);
+    plan_split(plan, 0);
+    double t = 0.0;
+    gemm_tall_splits((M + TM - 1) / TM * TM, N, K, plan.n_main, (long)plan.tiles_m * plan.tiles_n - plan.n_main, plan.splits, &t);
+    return t;
+  };
+  return gemm_tall_back_splits(T, O, I, bias, us(T, I, O) + us(O, I, T));
+}
+
 // g (+)= dy^T x and db (+)= the column sums of dy where the 256 x 128 tiles take the weight gradient (they carry the sums); false: nothing done, gemm64_ex and
 // col_sum_ are as fast or faster.  dy [T, M], x [T, N]; sizes: gemm64_wgrad_splits, which the caller asks first and keeps by size.
 // gpt2-125m, 2 x 1956 tokens: the library's products 49 us a weight gradient and 9 a bias, 30.5 together; the step 9786 us of kernels, so 8498.

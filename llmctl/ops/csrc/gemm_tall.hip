@@ -20,6 +20,9 @@
 #include "gemm_tall.h"
 #include "gemm64_tiles.h"
 
+#include <functional>
+#include <queue>
+
 namespace llmctl {
 using namespace attn;
 namespace {
@@ -67,9 +70,9 @@ __device__ __forceinline__ void put1(void* out, int m, float v, int add) {
 // BIAS (weight gradients): dy's column sums, this product's row sums of A, ride along.  The waves of the first four tile columns take one of the tile's 16-row
 // blocks each, two more MFMAs against ones to a K-tile's 64 (a pass over dy and a launch to add its parts were 10 to 14 us a bias, 48 of them in a gpt2-125m step
 // of 8192 tokens: the step 12174 us, so 11860).  The block's fragments are read where its image is: of A_lo(t+1) in P1(t), of A_hi(t) in P0(t).
+// Not AT: rows past the last are read as zeros or not at all, and not stored.
 template <bool AT, int OUT, bool BIAS>
-__global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_tall_kernel(TallArgs args) {
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
+__device__ __forceinline__ void tall_workgroup(const TallArgs& args, int block, unsigned char* smem) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wr = wave >> 1, wc = wave & 1;
@@ -77,8 +80,8 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 
   // item: split outermost, then groups of four tile rows, row innermost; each XCD takes a contiguous run of them, so its L2 holds the panels that it shares
   const int n_items = args.tiles_m * args.tiles_n * args.splits;
-  const int q8 = n_items / 8, r8 = n_items % 8, x = blockIdx.x % 8;
-  const int item = (x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8) + blockIdx.x / 8;
+  const int q8 = n_items / 8, r8 = n_items % 8, x = block % 8;
+  const int item = (x < r8 ? x * (q8 + 1) : r8 * (q8 + 1) + (x - r8) * q8) + block / 8;
   const int tiles = args.tiles_m * args.tiles_n;
   const int sp = item / tiles, wg = item - sp * tiles;
   const int grp = wg / (4 * args.tiles_n), gsz = min(4, args.tiles_m - grp * 4), inner = wg - grp * 4 * args.tiles_n;
@@ -86,7 +89,8 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   const int pairs = (args.K + 2 * TK - 1) / (2 * TK);  // AT: the last pair of K-tiles may be part full
   const int k0 = 2 * (int)((long)pairs * sp / args.splits), KT = 2 * (int)((long)pairs * (sp + 1) / args.splits) - k0;
 
-  i32x4_t ra = make_rsrc(AT ? args.a + (long)tm * TM : args.a + (long)tm * TM * lda);
+  i32x4_t ra = AT ? make_rsrc(args.a + (long)tm * TM)
+                  : make_rsrc_n(args.a + (long)tm * TM * lda, (unsigned)min(((long)(min(args.M - tm * TM, TM) - 1) * lda + args.K) * 2, 0x7fffffffL));
   i32x4_t rb = make_rsrc(args.b + (long)tn * TALL_N);
   // AT: the last two K-tiles through buffers of their own that start with them and end with the last token's row, so that what is read past it is zero (a row
   // past the end starts past the range: the rows do not overlap)
@@ -272,6 +276,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
   }
   // bf16, 16 bytes to a lane: lanes of neighbouring groups swap halves of two column tiles
   unsigned short* C = static_cast<unsigned short*>(args.c) + row0 * args.ldc + col0 + 16 * (g & 1) + 8 * (g >> 1);
+  const int rows = AT ? TM : args.M - (tm * TM + wr * 128 + i16);  // (the lanes that swap hold one row)
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -290,8 +295,24 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += old[e];
       }
-      store8(p, v);
+      if (16 * i < rows) store8(p, v);
     }
+}
+
+template <bool AT, int OUT, bool BIAS>
+__global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_tall_kernel(TallArgs args) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
+  tall_workgroup<AT, OUT, BIAS>(args, (int)blockIdx.x, smem);
+}
+
+// A layer's two gradients in one launch: the longer items first, n_first of them, and the others on the CUs that have none or are done.
+template <int OUT, bool BIAS>
+__global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_tall_back_kernel(TallArgs data, TallArgs weight, int n_first, bool data_first) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
+  const bool first = (int)blockIdx.x < n_first;
+  const int block = (int)blockIdx.x - (first ? 0 : n_first);
+  if (first == data_first) tall_workgroup<false, OUT_STORE, false>(data, block, smem);
+  else tall_workgroup<true, OUT, BIAS>(weight, block, smem);
 }
 
 // out (+)= the partial sums, added in the order of K; a thread's 8 columns of a row
@@ -357,6 +378,25 @@ void launch(const TallArgs& g, int out) {
 
 }  // namespace
 
+namespace {
+// us of `items` workgroups, one to a CU at a time, of k K-tiles each: `empty` + `full` times the share of the chip that is filled a K-tile, `fixed` a workgroup
+double rounds_us(double items, double k, double empty, double full, double fixed) {
+  const double cus = num_cus(), whole = std::floor(items / cus), rest = items - whole * cus;
+  return whole * (k * (empty + full) + fixed) + (rest > 0 ? k * (empty + full * rest / cus) + fixed : 0.0);
+}
+double pairs_of(long K) { return (double)((K + 2 * TK - 1) / (2 * TK)); }
+double split_k(double pairs, int S) { return 2.0 * std::ceil(pairs / S); }
+constexpr double TALL_EMPTY = 0.743, TALL_FULL = 0.06, TALL_FIXED = 5.4;
+double reduce_us(long M, long N, int S) { return S > 1 ? 5.8 + (double)M * N * S * 8.0 / 9.6e6 : 0.0; }
+double wide_us(long K, long n_main, long n_tail, int splits) {  // gemm64's 256 x 256 tiles
+  const double kt = 2.0 * pairs_of(K);
+  double us = rounds_us((double)n_main, kt, 0.92, 0.36, 10.4);
+  if (n_tail > 0) us += rounds_us((double)n_tail * splits, kt / splits, 0.92, 0.36, 10.4);
+  if (n_tail > 0 && splits > 1) us += 8.2 + (double)n_tail * TM * TN * splits * 8.0 / 14.7e6;
+  return us;
+}
+}  // namespace
+
 // K-ranges for this kernel where it is the faster one, else 0.  n_main whole tiles of 256 x 256 and n_tail in `splits` ranges each are gemm64's plan.  Both
 // times from the sizes, us: a round costs its K-tiles and a fixed part (fill and store), a K-tile of 64 more the fuller the chip is (0.74 here on an empty one, 0.80
 // on a full one; 0.92 and 1.28 there); partial sums cost a launch and their bytes, written and read.  Ranges stay at four K-tiles and more, what the peeled loop
@@ -364,40 +404,69 @@ void launch(const TallArgs& g, int out) {
 // on average; by it these tiles take 13 % less time than 256 x 256 ones everywhere, and in 5 sizes 3 to 7 % more (12288 x 2048 x 1536 71.9, here 77.2).  The margin
 // keeps long single rounds of less than the chip on the others, which their last K-tiles' loads hold up here (2560 x 2560 weight gradients over 16384 rows 191 there,
 // here 250; 5120 x 1280 over 6144 80 and 97).
-int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits) {
-  const double cus = num_cus(), kt = (K + 2 * TK - 1) / (2 * TK) * 2;
-  auto rounds = [&](double items, double k, double empty, double full, double fixed) {
-    const double whole = std::floor(items / cus), rest = items - whole * cus;
-    return whole * (k * (empty + full) + fixed) + (rest > 0 ? k * (empty + full * rest / cus) + fixed : 0.0);
-  };
-  auto other = [&](double items, double k) { return rounds(items, k, 0.92, 0.36, 10.4); };
-  double limit = other((double)n_main, kt);
-  if (n_tail > 0) limit += other((double)n_tail * splits, kt / splits);
-  if (n_tail > 0 && splits > 1) limit += 8.2 + (double)n_tail * TM * TN * splits * 8.0 / 14.7e6;
+// us_of: the faster one's time.
+int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int splits, double* us_of) {
+  double limit = wide_us(K, n_main, n_tail, splits);
+  if (us_of != nullptr) *us_of = limit;
   limit *= 0.972;
   int best = 0;
   for (int S = 1; S <= 16 && K >= 4L * TK * S; ++S) {
-    const double us = rounds((double)(M / TM) * (N / TALL_N) * S, 2.0 * std::ceil(kt / 2.0 / S), 0.743, 0.06, 5.4) +
-                      (S > 1 ? 5.8 + (double)M * N * S * 8.0 / 9.6e6 : 0.0);
+    const double us = rounds_us((double)(M / TM) * (N / TALL_N) * S, split_k(pairs_of(K), S), TALL_EMPTY, TALL_FULL, TALL_FIXED) + reduce_us(M, N, S);
+    if (us < limit) limit = us, best = S;
+  }
+  if (us_of != nullptr && best > 0) *us_of = limit;
+  return best;
+}
+
+// K-ranges of the weight gradient where a layer's two gradients, dy w and dy^T x of T tokens, O outputs and I inputs, take less time in one launch
+// (gemm_tall_back) than in two, of either kind of tiles; else 0.  The second launch's workgroups start on the CUs that the first ones leave idle: 8192 tokens of
+// a 768 x 3072 layer are 192 and 216 workgroups, 64 and 40 CUs idle.  two_us is the time of the two by the model above (data gradients whose tokens are no
+// multiple of 256 go to the library, which takes as long as these tiles), and the one launch's the end of a list of workgroups, longest first, dealt out to the CUs.
+// Constants fitted to 330 sizes (256 to 9216 tokens, 256 to 6144 outputs, 256 to 4096 inputs; profiles/backward_pairs.txt): what the rule picks takes 23 % less time
+// than two launches on average and 2 % more than the best choice; in one size 11 % more than two (7168 x 3072 x 768 85.7, so 94.9), in one 2 %.
+// us, two launches / one: 8192 tokens 768 x 768 40.2 / 34.0, 2304 x 768 76.3 / 70.0, 3072 x 768 99.4 / 87.7, 768 x 3072 106.8 / 97.7; 1326 tokens 768 x 3072 37.4 /
+// 24.0; but 8192 x 4096 x 4096 373 / 436, where 256 x 256 tiles fill the chip.
+constexpr double BACK_TILE = 0.76, BACK_FIXED = 4.0, BACK_MARGIN = 1.05;
+int64_t gemm_tall_back_splits(int64_t T, int64_t O, int64_t I, bool bias, double two_us) {
+  if (T < 4 * TK || O <= 0 || I <= 0 || O % TM != 0 || I % TN != 0 || (bias && I < 4 * TALL_N)) return 0;
+  const long nd = (T + TM - 1) / TM * (I / TALL_N), tiles = O / TM * (I / TALL_N);
+  if (nd + tiles > 8L * num_cus()) return 0;  // (rounds enough to fill the last one's gap)
+  const double d_us = O / TK * BACK_TILE + BACK_FIXED;
+  double limit = two_us * BACK_MARGIN;
+  int64_t best = 0;
+  for (int S = 1; S <= 16 && T >= 4L * TK * S; ++S) {
+    const double w_us = split_k(pairs_of(T), S) * BACK_TILE + BACK_FIXED;
+    std::priority_queue<double, std::vector<double>, std::greater<double>> cus(std::greater<double>(), std::vector<double>(num_cus(), 0.0));
+    double end = 0.0;
+    auto deal = [&](long n, double us) {
+      for (long i = 0; i < n; ++i) {
+        const double t = cus.top() + us;
+        cus.pop();
+        cus.push(t);
+        end = std::max(end, t);
+      }
+    };
+    if (d_us >= w_us) deal(nd, d_us), deal(tiles * S, w_us);
+    else deal(tiles * S, w_us), deal(nd, d_us);
+    const double us = end + (S > 1 ? 4.5 + (double)O * I * S * 8.0 / 7.0e6 : 0.0);
     if (us < limit) limit = us, best = S;
   }
   return best;
 }
 
-// out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N of 128 and, not where at, K of 128; two pairs of
-// K-tiles to a split, 256 of K, of which the last one of a transposed A has more than 128.
-// bias [M] (+)= the row sums of A, of out's type (at, N >= 512).
-void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias,
-               bool bias_add) {
+namespace {
+// the operands of one product; ragged: rows of A (not transposed) that fill no whole tile
+TallArgs tall_args(const at::Tensor& a, const at::Tensor& b, const at::Tensor& out, bool at_, int64_t splits, const c10::optional<at::Tensor>& bias, bool bias_add, bool ragged) {
   LLMCTL_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2 && a.is_cuda() && b.is_cuda() && out.is_cuda(), "gemm_tall: 2-D GPU operands");
   const bool f32 = out.scalar_type() == at::kFloat;
   LLMCTL_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && (f32 || out.scalar_type() == at::kBFloat16),
                "gemm_tall: bf16 operands, bf16 or fp32 out");
   const long M = at_ ? a.size(1) : a.size(0), K = at_ ? a.size(0) : a.size(1), N = b.size(1);
   LLMCTL_CHECK(b.size(0) == K && out.size(0) == M && out.size(1) == N, "gemm_tall: shapes");
-  LLMCTL_CHECK(M > 0 && N > 0 && M % TM == 0 && N % TALL_N == 0 && (at_ || K % (2 * TK) == 0) && splits >= 1 && (K + 2 * TK - 1) / (2 * TK) >= 2 * splits,
+  LLMCTL_CHECK(M > 0 && N > 0 && (M % TM == 0 || ragged) && N % TALL_N == 0 && (at_ || K % (2 * TK) == 0) && splits >= 1 && (K + 2 * TK - 1) / (2 * TK) >= 2 * splits,
                "gemm_tall: M in 256s, N (and K, but for a transposed A) in 128s, two pairs of K-tiles of 64 to a split, the last of them part full at most");
   LLMCTL_CHECK(!at_ || K % (2 * TK) == 0 || (a.stride(0) >= M && b.stride(0) >= N), "gemm_tall: rows that do not overlap");
+  LLMCTL_CHECK(at_ || M % TM == 0 || a.stride(0) >= K, "gemm_tall: rows that do not overlap");
   auto rows16 = [](const at::Tensor& t, int per) {
     return t.stride(1) == 1 && t.stride(0) % per == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
   };
@@ -407,19 +476,62 @@ void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at
   LLMCTL_CHECK(!bias.has_value() || (at_ && N >= 4 * TALL_N && bias->is_cuda() && bias->is_contiguous() && bias->numel() == M &&
                                      bias->scalar_type() == out.scalar_type()),
                "gemm_tall: a bias goes with a transposed A and 512 columns, [M] of out's type");
+  return TallArgs{bf_ptr(a), bf_ptr(b), out.data_ptr(), nullptr, bias.has_value() ? bias->data_ptr() : nullptr, bias_add, (long)a.stride(0), (long)b.stride(0),
+                  (long)out.stride(0), (int)M, (int)N, (int)K, (int)((M + TM - 1) / TM), (int)(N / TALL_N), (int)splits};
+}
+// room for the partial sums of more than one range
+at::Tensor tall_room(TallArgs& g, const at::Tensor& a) {
+  if (g.splits <= 1) return {};
+  at::Tensor ws = at::empty({(long)g.splits * g.M * (g.N + 1)}, a.options().dtype(at::kFloat));
+  g.ws = ws.data_ptr<float>();
+  return ws;
+}
+}  // namespace
+
+// out [M, N] (+)= A B with B [K, N] and A [M, K], or [K, M] where at; out bf16 or fp32.  M a multiple of 256, N of 128 and, not where at, K of 128; two pairs of
+// K-tiles to a split, 256 of K, of which the last one of a transposed A has more than 128.
+// bias [M] (+)= the row sums of A, of out's type (at, N >= 512).
+void gemm_tall(const at::Tensor& a, const at::Tensor& b, at::Tensor out, bool at_, bool accumulate, int64_t splits, const c10::optional<at::Tensor>& bias,
+               bool bias_add) {
+  TallArgs g = tall_args(a, b, out, at_, splits, bias, bias_add, false);
   const c10::DeviceGuard guard(a.device());
-  TallArgs g{bf_ptr(a), bf_ptr(b), out.data_ptr(), nullptr, bias.has_value() ? bias->data_ptr() : nullptr, bias_add, (long)a.stride(0), (long)b.stride(0), (long)out.stride(0), (int)M, (int)N, (int)K,
-             (int)(M / TM), (int)(N / TALL_N), (int)splits};
-  at::Tensor ws;
-  if (splits > 1) {
-    ws = at::empty({splits * M * (N + 1)}, a.options().dtype(at::kFloat));
-    g.ws = ws.data_ptr<float>();
-  }
-  const int o = (f32 ? OUT_STORE_F32 : OUT_STORE) + (accumulate ? 1 : 0);
+  const at::Tensor ws = tall_room(g, a);
+  const int o = (out.scalar_type() == at::kFloat ? OUT_STORE_F32 : OUT_STORE) + (accumulate ? 1 : 0);
   if (at_) launch<true>(g, o);
   else launch<false>(g, o);
 }
 
-TORCH_LIBRARY_IMPL(llmctl, CUDA, m) { m.impl("gemm_tall", &gemm_tall); }
+// A layer's two gradients in one launch: dx = dy w of any number of rows, g (+)= dy^T x in `splits` ranges of the tokens and, where given, db (+)= dy's column
+// sums.  dy [T, O], w [O, I], x [T, I]; O in 256s, I in 128s (with db from 512 on), T >= 256 a split.
+void gemm_tall_back(const at::Tensor& dy, const at::Tensor& w, at::Tensor dx, const at::Tensor& x, at::Tensor g, bool accumulate, int64_t splits,
+                    const c10::optional<at::Tensor>& db, bool add) {
+  LLMCTL_CHECK(dx.scalar_type() == at::kBFloat16, "gemm_tall_back: dx bf16");
+  const TallArgs d = tall_args(dy, w, dx, false, 1, c10::nullopt, false, true);
+  TallArgs v = tall_args(dy, x, g, true, splits, db, add, false);
+  const c10::DeviceGuard guard(dy.device());
+  const at::Tensor ws = tall_room(v, dy);
+  const int nd = d.tiles_m * d.tiles_n, nv = v.tiles_m * v.tiles_n * v.splits;
+  const bool d_first = d.K / TK >= 2 * (((v.K + 2 * TK - 1) / (2 * TK) + v.splits - 1) / v.splits);
+  auto go = [&](auto out_c) {
+    constexpr int OUT = decltype(out_c)::value;
+    auto with = [&](auto bias_c) {
+      constexpr bool BIAS = decltype(bias_c)::value;
+      hipLaunchKernelGGL((gemm_tall_back_kernel<OUT, BIAS>), dim3(nd + nv), dim3(NT4), 0, stream(), d, v, d_first ? nd : nv, d_first);
+      if (v.splits > 1) hipLaunchKernelGGL((gemm_tall_reduce<OUT, BIAS>), dim3((unsigned)((long)v.M * v.N / 2048)), dim3(256), 0, stream(), v);
+    };
+    if (v.bias != nullptr) with(std::true_type{});
+    else with(std::false_type{});
+  };
+  const bool f32 = g.scalar_type() == at::kFloat;
+  if (f32 && accumulate) go(K_<OUT_ADD_F32>{});
+  else if (f32) go(K_<OUT_STORE_F32>{});
+  else if (accumulate) go(K_<OUT_ADD>{});
+  else go(K_<OUT_STORE>{});
+}
+
+TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
+  m.impl("gemm_tall", &gemm_tall);
+  m.impl("gemm_tall_back", &gemm_tall_back);
+}
 
 }  // namespace llmctl

@@ -215,3 +215,54 @@ def test_sizes_of_the_rule(M, N, K, ranges):
     from llmctl.ops._lib import native
 
     assert native().gemm64_wgrad_splits(M, N, K, True) == ranges
+
+
+@pytest.mark.parametrize("T,O,I,S,pad", [(256, 256, 128, 1, 0), (257, 256, 640, 1, 8), (511, 512, 512, 1, 0), (640, 768, 512, 2, 8), (1000, 256, 768, 3, 0),
+                                         (1326, 2304, 768, 1, 0), (8192, 768, 512, 5, 0)])  # data gradients' last rows, either kind of workgroup first
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("add", [False, True])
+@pytest.mark.parametrize("bias", [False, True])
+def test_both_gradients_in_one_launch(T, O, I, S, pad, f32, add, bias):
+    from llmctl.ops._lib import native
+
+    if bias and I < 512:
+        pytest.skip("column sums ride from 512 inputs on")
+    g = torch.Generator(device="cuda").manual_seed(T + O + I)
+    rows = lambda n, c: torch.randn(n, c + pad, generator=g, device="cuda").bfloat16()[:, :c]
+    dy, w, x = rows(T, O), rows(O, I), rows(T, I)
+    dt = torch.float32 if f32 else torch.bfloat16
+    dx = torch.full((T + 2, I), 3.0, device="cuda", dtype=torch.bfloat16)
+    gw, gb = (torch.full(s, 2.0 if add else float("nan"), device="cuda", dtype=dt) for s in ((O, I), (O,)))
+    native().gemm_tall_back(dy, w, dx[:T], x, gw, add, S, gb if bias else None, add)
+    D, W, X = dy.double(), w.double(), x.double()
+    old = 2.0 if add else 0.0
+    for out, ref, mag, n, half in ((dx[:T], D @ W, D.abs() @ W.abs(), O, True), (gw, D.t() @ X + old, D.t().abs() @ X.abs(), T, not f32),
+                                   *([(gb, D.sum(0) + old, D.abs().sum(0), T, not f32)] if bias else [])):
+        bound = (n + S + 1) * 2.0**-24 * mag + 2.0**-23 * ref.abs()
+        if half:  # one rounding of the fp32 result
+            bound = bound + 2.0**-8 * (ref.abs() + bound)
+        assert bool(((out.double() - ref).abs() <= bound).all())
+    assert bool((dx[T:] == 3.0).all())
+
+
+@pytest.mark.parametrize("tokens,out,inn,bias", [(8192, 768, 768, True), (1326, 2304, 768, True), (640, 768, 3072, False)])
+def test_layers_take_the_one_launch(tokens, out, inn, bias, monkeypatch):
+    import importlib
+
+    L = importlib.import_module("llmctl.exec.linear")
+    calls, back = [], L.tall_back
+    monkeypatch.setattr(L, "tall_back", lambda *a: calls.append(back(*a)) or calls[-1])
+    sink = L.GradSink()
+    w = torch.nn.Parameter(torch.randn(out, inn, device="cuda", dtype=torch.bfloat16) * 0.05)
+    b = torch.nn.Parameter(torch.zeros(out, device="cuda", dtype=torch.bfloat16)) if bias else None
+    for p in (w, b) if bias else (w,):
+        p.grad = torch.full_like(p, float("nan"))
+        sink.attach(p)
+    x = torch.randn(tokens, inn, device="cuda", dtype=torch.bfloat16).requires_grad_()
+    dy = torch.randn(tokens, out, device="cuda", dtype=torch.bfloat16)
+    L.linear(x, w, b).backward(dy)
+    assert len(calls) == 1 and calls[0] is not None
+    D = dy.double()
+    pairs = [(x.grad, D @ w.detach().double()), (w.grad, D.t() @ x.detach().double())] + ([(b.grad, D.sum(0))] if bias else [])
+    for got, ref in pairs:  # bf16 of fp32 sums: 2^-9 an entry at most, 0.0017 of the norm
+        assert float((got.double() - ref).norm() / ref.norm()) < 2.0**-9
