@@ -158,11 +158,13 @@ __global__ __launch_bounds__(NT) void embed_rmsnorm_kernel(const int64_t* __rest
   for (int c = threadIdx.x + COLS * NT; c < W; c += NT) stf(h + row * W + c, x[row * W + c] * rstd * w[c]);  // the thread's own stores
 }
 
-template <int KIND>
+template <typename T, int KIND>
 __device__ __forceinline__ float act_one(float v) {
   if constexpr (KIND == 0) {
     const float r = fmaxf(v, 0.f);
     return r * r;
+  } else if constexpr (sizeof(T) == 2) {
+    return gelu_erf16(v);
   } else {
     return 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
   }
@@ -174,23 +176,22 @@ __global__ void act_kernel(const T* __restrict__ x, int64_t x_st, const float* _
   if (i >= rows * F) return;
   const int64_t r = i / F;
   const int c = (int)(i - r * F);
-  stf(y + i, act_one<KIND>(ldf(x + r * x_st + c)) * (scale != nullptr ? scale[r] : 1.0f));
+  stf(y + i, act_one<T, KIND>(ldf(x + r * x_st + c)) * (scale != nullptr ? scale[r] : 1.0f));
 }
 
-template <typename T, int KIND>
-__global__ void act_vec_kernel(const T* __restrict__ x, int64_t x_st, const float* __restrict__ scale, T* __restrict__ y, int64_t rows, int F) {
+// I: unsigned where the rows' quads or octets count to less than 2^32.  3379 x 8192 (bf16, erf GELU): ACT_US
+template <typename T, int KIND, typename I>
+__global__ __launch_bounds__(256) void act_vec_kernel(const T* __restrict__ x, int64_t x_st, const float* __restrict__ scale, T* __restrict__ y, I n, I per) {
   constexpr int N = Vec16<T>::N;
-  const int per = F / N;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * per) return;
-  const int64_t r = i / per;
-  const int c = (int)(i - r * per) * N;
+  const I i = (I)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const I r = i / per, c = i - r * per;
   float v[N];
-  Vec16<T>::load(x + r * x_st + c, v);
+  Vec16<T>::load(x + (int64_t)r * x_st + (int64_t)c * N, v);
   const float f = scale != nullptr ? scale[r] : 1.0f;
 #pragma unroll
-  for (int k = 0; k < N; ++k) v[k] = act_one<KIND>(v[k]) * f;
-  Vec16<T>::store(y + r * F + c, v);
+  for (int k = 0; k < N; ++k) v[k] = act_one<T, KIND>(v[k]) * f;
+  Vec16<T>::store(y + (int64_t)i * N, v);
 }
 
 // The tanh GELU 0.5 z (1 + tanh(y)) is z sigmoid(2 y), y = sqrt(2 / pi) (z + 0.044715 z^3).
@@ -493,8 +494,14 @@ at::Tensor act_any(const at::Tensor& x, int64_t kind, const c10::optional<at::Te
     const int64_t nv = vec ? n / Vec16<T>::N : n;
     const dim3 grid((unsigned)((nv + 255) / 256));
     if (vec) {
-      if (kind == 0) act_vec_kernel<T, 0><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), rows, F);
-      else act_vec_kernel<T, 1><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), rows, F);
+      auto go = [&](auto i) {
+        using I = decltype(i);
+        const I per = (I)(F / Vec16<T>::N);
+        if (kind == 0) act_vec_kernel<T, 0, I><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), (I)nv, per);
+        else act_vec_kernel<T, 1, I><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), (I)nv, per);
+      };
+      if (nv <= 0xffffff00L) go(0u);
+      else go((uint64_t)0);
     } else {
       if (kind == 0) act_kernel<T, 0><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), rows, F);
       else act_kernel<T, 1><<<grid, 256, 0, st>>>((const T*)x.data_ptr(), x.stride(0), sp, (T*)y.data_ptr(), rows, F);

@@ -8,8 +8,9 @@
 //
 //   * moe_route_kernel: 16 tokens per workgroup, logits on the fp32 matrix cores, scores and choice in the same kernel: no
 //     logits tensor, no fp32 copy of the rows.  Steps of up to 64 tokens whose norm is at hand are routed there (router_rows.h).
-//   * moe_group_kernel: one workgroup per expert scans the choices twice (histogram, then ballot prefix): a stable counting
-//     sort, and the list of row tiles that the grouped product walks.
+//   * moe_group_kernel: one workgroup per expert counts the choices and places its own: a stable counting sort, and the list of row
+//     tiles that the grouped product walks.
+//   * moe_wide_kernel (moe_wide.h): tiles of up to 288 x 128, K in 128s from 256 on.
 //   * moe_tile_kernel: BM x BN tiles of one expert's rows, K in 64-deep steps through LDS, the global loads of the next step
 //     (64-wide tiles: the next three) in registers under the MFMAs of this one.  16-byte chunks are swizzled by the row, so a wave's fragment
 //     reads touch every bank slot equally.  The weight fragment is the MFMA row operand: a lane ends up with four neighbouring
@@ -22,17 +23,15 @@
 //   * moe_combine_kernel: out_t = sum_k w_tk y_tk (+ w x_t for experts without weights) (+ the shared expert), fp32; where the
 //     result goes straight into the residual stream and a norm, their kernel sums instead (expert_rows.h).
 //
-// A row tile has 128 rows when the experts get 96 or more on average, else 64 (and 64 columns): below that the grid
-// of 128 x 128 tiles does not fill the chip and the K loop of every workgroup is a chain of load latencies.  The large tile
-// keeps one LDS buffer (32 KB) so that three workgroups fit a CU: 4096 copies make 1.1 rounds of two per CU but one of three
-// (2048 tokens: up 62 us against 81 with two buffers); the small one keeps three steps in flight (37 -> 30 us at 65 tokens).
+// Other widths, and experts that get less than 96 rows on average (48 where tiles of 64 x 64 would make more than a round of the chip, below), have tiles of 128 x 128 (96
+// rows and more) or 64 x 64: with few tiles the K loop of every workgroup is a chain of load latencies.  The large tile
+// keeps one LDS buffer (32 KB) so that three workgroups fit a CU; the small one keeps three steps in flight (37 -> 30 us at 65 tokens).
 //
 // Measured, one MI355X, width 2048, 8 gated experts of 1024, top 2 (up / down; weights from HBM):
 //   tokens      16          32         64        128        256        512       1024       2048       4096
-//   us       26 / 14     27 / 14    30 / 16    31 / 16    36 / 18    46 / 25    48 / 28    62 / 36    97 / 55   (4096: 710 / 620 TFLOP/s)
-//   router      9           9         10         10         10         10         10         10         12
-// up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from 2048 the LDS reads of 64 x 64 wave tiles and the
-// last round of tiles.  A layer of 2048 tokens took 700 us before (sort, per-expert GEMMs, copies), 16 tokens 350 us.
+//   us       26 / 14     27 / 14    30 / 16    21 / 11    23 / 13    27 / 15    32 / 20    37 / 24    65 / 39
+// up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from there on what a CU can have in flight (moe_wide.h).  On tiles of 128 x 128, 512 tokens took
+// 38 / 22, 1024 39 / 22, 2048 62 / 36, 4096 97 / 55; 2911 tokens through 8 experts without gates 51 / 46, so 33 / 36.
 #include "expert_rows.h"
 #include "router_rows.h"
 #include "stream_linear.h"
@@ -60,7 +59,7 @@ __device__ __forceinline__ float expert_act(int act, float u, float g) {
     const float r = fmaxf(u, 0.f);
     return r * r;
   }
-  return 0.5f * u * (1.0f + erff(u * 0.70710678118654752440f));
+  return gelu_erf16(u);
 }
 
 // The tiled form rounds the first projection's results to the activation's type before the activation, as a product and an
@@ -142,60 +141,94 @@ __global__ __launch_bounds__(ROUTE_WAVES * 64) void moe_route_kernel(const bf16_
 }
 
 // ------------------------------------------------------------------------------------------------ grouping
+// Row tiles of n rows: of BM each, or (WIDE_ROWS, moe_wide.h) of 256 but the last one, which has 33 to 288.
+constexpr int WIDE_ROWS = 288, WIDE_HALF = 128;
+__device__ __forceinline__ int row_tiles(int n, int BM) { return BM != WIDE_ROWS ? (n + BM - 1) / BM : n <= BM ? n > 0 : (n - 33) / 256 + 1; }
+__device__ __forceinline__ bool half_tile(int n, int BM) {  // the last one has at most 128 rows
+  return BM == WIDE_ROWS && n > 0 && n - 256 * (row_tiles(n, BM) - 1) <= WIDE_HALF;
+}
+
 // Workgroup e: where expert e's copies start, which they are (in token order), and its row tiles.  ``tiles``: [0] = their
-// number, then (expert, first sorted row, rows) each.  Entries of experts without weights (>= E) are left out.
+// number without the half ones, [1] = that of the half ones (WIDE_ROWS), then (expert, first sorted row, rows) each, the half ones last.  Entries of experts without
+// weights (>= E) are left out.
+// A thread takes `per` neighbouring copies, so that one pass over them and one scan over the workgroup place them all; a pass for the counts and rounds of 1024 with two
+// barriers each took, us, so: 2048 tokens, 8 experts, top 2 6.5 / 4.7, 3565 9.6 / 5.5; 2031
+// tokens, 32 experts, top 4 10.9 / 7.4.
+constexpr int GROUP_KEEP = 16;  // copies a thread keeps in registers between the two passes
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int N, int E, int BM, int* __restrict__ perm,
                                                          int* __restrict__ tiles) {
   __shared__ int hist[MAX_EXPERTS];
-  __shared__ int wsum[17];
+  __shared__ int wsum[16];
   __shared__ int base[2];
   const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid < MAX_EXPERTS) hist[tid] = 0;
-  __syncthreads();
-  for (int i = tid; i < N; i += 1024) {
-    const int v = idx[i];
-    if (v < E) atomicAdd(&hist[v], 1);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    int at = 0, tile = 0;
-    for (int j = 0; j < e; ++j) {
-      at += hist[j];
-      tile += (hist[j] + BM - 1) / BM;
-    }
-    const int n = hist[e], nt = (n + BM - 1) / BM;
-    for (int k = 0; k < nt; ++k) {
-      int* d = tiles + 1 + 3 * (tile + k);
-      d[0] = e;
-      d[1] = at + k * BM;
-      d[2] = min(BM, n - k * BM);
-    }
-    if (e == E - 1) tiles[0] = tile + nt;
-    base[0] = at;
-  }
-  __syncthreads();
-  int at = base[0];
-  for (int i0 = 0; i0 < N; i0 += 1024) {
-    const int i = i0 + tid;
-    const bool mine = i < N && idx[i] == e;
-    const unsigned long long m = __ballot(mine);
-    if (lane == 0) wsum[wave] = __popcll(m);
-    __syncthreads();
-    int before = 0, all = 0;
+  const int per = (N + 1023) / 1024, i0 = tid * per, n_i = max(0, min(per, N - i0));
+  int v[GROUP_KEEP], mine = 0;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int c = wsum[v];
-      before += v < wave ? c : 0;
-      all += c;
-    }
-    if (mine) perm[at + before + __popcll(m & ((1ull << lane) - 1ull))] = i;
-    at += all;
-    __syncthreads();
+  for (int k = 0; k < GROUP_KEEP; ++k) {
+    v[k] = -1;
+    if (k < per && k < n_i) v[k] = idx[i0 + k];
   }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < GROUP_KEEP; ++k) {
+    if (k >= per) break;
+    mine += v[k] == e;
+    if (v[k] >= 0 && v[k] < E) atomicAdd(&hist[v[k]], 1);
+  }
+  for (int k = GROUP_KEEP; k < n_i; ++k) {
+    const int x = idx[i0 + k];
+    mine += x == e;
+    if (x < E) atomicAdd(&hist[x], 1);
+  }
+  int before = 0, all = 0;  // copies of e ahead of this thread's, and in all, within the wave: bit by bit of their numbers
+  for (int b = 0; per >> b != 0; ++b) {
+    const unsigned long long m = __ballot(mine >> b & 1);
+    before += __popcll(m & ((1ull << lane) - 1ull)) << b;
+    all += __popcll(m) << b;
+  }
+  if (lane == 0) wsum[wave] = all;
+  __syncthreads();
+  if (wave == 0) {
+    int at = 0, tile = 0, half = 0, whole = 0;  // before this expert: rows, tiles, half tiles; whole tiles of all
+#pragma unroll
+    for (int j = lane; j < MAX_EXPERTS; j += 64) {
+      if (j >= E) continue;
+      const int n = row_tiles(hist[j], BM), h = half_tile(hist[j], BM);
+      whole += n - h;
+      if (j < e) at += hist[j], tile += n - h, half += h;
+    }
+    for (int o = 32; o > 0; o >>= 1)
+      if (E > o) at += __shfl_xor(at, o, 64), tile += __shfl_xor(tile, o, 64), half += __shfl_xor(half, o, 64), whole += __shfl_xor(whole, o, 64);
+    at = __builtin_amdgcn_readfirstlane(at), tile = __builtin_amdgcn_readfirstlane(tile);
+    half = __builtin_amdgcn_readfirstlane(half), whole = __builtin_amdgcn_readfirstlane(whole);
+    const int n = hist[e], nt = row_tiles(n, BM), h = half_tile(n, BM), step = BM == WIDE_ROWS ? 256 : BM;
+    for (int k = lane; k < nt; k += 64) {
+      int* d = tiles + 2 + 3 * (h && k == nt - 1 ? whole + half : tile + k);
+      d[0] = e;
+      d[1] = at + k * step;
+      d[2] = k < nt - 1 ? step : n - k * step;
+    }
+    if (lane == 0) {
+      if (e == E - 1) tiles[0] = whole, tiles[1] = half + h;
+      base[0] = at;
+    }
+  }
+  __syncthreads();
+  int at = base[0] + before;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) at += w < wave ? wsum[w] : 0;
+#pragma unroll
+  for (int k = 0; k < GROUP_KEEP; ++k) {
+    if (k >= per) break;
+    if (v[k] == e) perm[at++] = i0 + k;
+  }
+  for (int k = GROUP_KEEP; k < n_i; ++k)
+    if (idx[i0 + k] == e) perm[at++] = i0 + k;
 }
 
 // ------------------------------------------------------------------------------------------------ tiles
-enum { UP_GLU = 0, UP_PLAIN = 1, DOWN = 2 };
+enum { UP_GLU = 0, UP_PLAIN = 1, DOWN = 2, UP_GELU = 3 };  // UP_GELU: moe_wide.h
 // Row tiles that walk the columns together: an XCD's neighbouring workgroups then share weights as well as rows.  One at a time, every row tile read its
 // expert's weights from the memory side again.  Whole layer, us, one / eight at a time (2, 4, 16 and 32 lie between): 8 gated experts of 4096 x 8192, top 2,
 // 2048 tokens 1476 / 1136, 16384 tokens 11072 / 7517; 2048 x 4096 at 2048 340 / 325, 16384 2138 / 1979; 2048 x 1024 at 2048 118 / 119.
@@ -210,6 +243,7 @@ struct TileArgs {
   const int* perm;
   const int* tiles;
   int K, cols, top, act, ntile;  // cols: ff (UP) or width (DOWN); ntile: column tiles
+  int max_tiles;                 // of rows (room in tiles)
 };
 
 template <int BM, int BN, int MODE, int PF, int NB, int OCC>
@@ -227,7 +261,7 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
   const int tile = xcd * q8 + min(xcd, r8) + (id >> 3);
   const int first = tile / (BAND * g.ntile) * BAND, in = tile - first * g.ntile, high = min(BAND, g.tiles[0] - first);
   const int nt = in / high, mt = first + in - nt * high;
-  const int e = g.tiles[1 + 3 * mt], row0 = g.tiles[2 + 3 * mt], rows = g.tiles[3 + 3 * mt];
+  const int e = g.tiles[2 + 3 * mt], row0 = g.tiles[3 + 3 * mt], rows = g.tiles[4 + 3 * mt];
   const bf16_t* __restrict__ w = g.w.p[e];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
@@ -341,6 +375,13 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
     }
   }
 }
+
+}  // namespace
+}  // namespace llmctl_hybrid
+#include "moe_wide.h"
+namespace llmctl_hybrid {
+namespace {
+static_assert(WIDE_ROWS == wide::ROWS, "row tiles");
 
 // ------------------------------------------------------------------------------------------------ few tokens
 struct SmallArgs {
@@ -637,18 +678,29 @@ at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Ten
     else if (T <= 32) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 4>{});
   } else {
-    const bool wide = N >= 96 * E;
-    const int BM = wide ? 128 : 64, BN = BM;
-    const int64_t mt = (N + BM - 1) / BM + E;  // no more row tiles than this
-    at::Tensor ints = at::empty({N + 1 + 3 * mt}, idx.options());
+    // tiles of up to 288 rows (moe_wide.h) where the experts get 96 rows on average, or 48 and tiles of 64 x 64 make more than a round of the chip; else, and for
+    // widths in no 128s, of 128 or 64
+    const bool wide = (N >= 96 * E || (N >= 48 * E && (N / 64 + E / 2) * (W / 64) >= 400)) && W % 128 == 0 && ff % 128 == 0 && W >= 256 && ff >= 256 && T * x.stride(0) < ((int64_t)1 << 30) && N * ff < ((int64_t)1 << 30) &&
+                      R * ldu < ((int64_t)1 << 30) && W * ldd < ((int64_t)1 << 30);
+    const int BM = wide ? WIDE_ROWS : N >= 96 * E ? 128 : 64, BN = wide ? wide::COLS : BM;
+    const int64_t mt = wide ? N / 256 + E : (N + BM - 1) / BM + E;  // no more row tiles than this
+    at::Tensor ints = at::empty({N + 2 + 3 * mt}, idx.options());
     int* perm = ints.data_ptr<int>();
     int* tiles = perm + N;
     moe_group_kernel<<<dim3((unsigned)E), 1024, 0, st>>>(idx.data_ptr<int>(), (int)N, (int)E, BM, perm, tiles);
-    const int cu = act == 1 ? BN / 2 : BN;
-    TileArgs u{xp, (long)x.stride(0), pu, ldu, ap, perm, tiles, (int)W, (int)ff, (int)top, (int)act, (int)((ff + cu - 1) / cu)};
-    TileArgs d{ap, (long)ff, pd, ldd, reinterpret_cast<bf16_t*>(y.data_ptr()), perm, tiles, (int)ff, (int)W, (int)top, (int)act, (int)((W + BN - 1) / BN)};
+    const int64_t cu = act == 1 ? BN / 2 : BN;
+    TileArgs u{xp, (long)x.stride(0), pu, ldu, ap, perm, tiles, (int)W, (int)ff, (int)top, (int)act, (int)((ff + cu - 1) / cu), (int)mt};
+    TileArgs d{ap, (long)ff, pd, ldd, reinterpret_cast<bf16_t*>(y.data_ptr()), perm, tiles, (int)ff, (int)W, (int)top, (int)act, (int)((W + BN - 1) / BN), (int)mt};
+    if (wide) {  // (16 more: what the two runs of an XCD are rounded up by)
+      const dim3 gu((unsigned)(mt * u.ntile + 16)), gd((unsigned)(mt * d.ntile + 16));
+      if (act == 1) moe_wide_kernel<UP_GLU><<<gu, 256, 0, st>>>(u);
+      else if (act == 0) moe_wide_kernel<UP_PLAIN><<<gu, 256, 0, st>>>(u);
+      else moe_wide_kernel<UP_GELU><<<gu, 256, 0, st>>>(u);
+      moe_wide_kernel<DOWN><<<gd, 256, 0, st>>>(d);
+      return y;
+    }
     const dim3 gu((unsigned)(mt * u.ntile)), gd((unsigned)(mt * d.ntile));
-    if (wide) {
+    if (BM == 128) {
       if (act == 1) moe_tile_kernel<128, 128, UP_GLU, 1, 1, 3><<<gu, 256, 0, st>>>(u);
       else moe_tile_kernel<128, 128, UP_PLAIN, 1, 1, 3><<<gu, 256, 0, st>>>(u);
       moe_tile_kernel<128, 128, DOWN, 1, 1, 3><<<gd, 256, 0, st>>>(d);

@@ -59,6 +59,29 @@ def test_experts_against_float64(T, W, ff, E, top, act):
     assert torch.equal(got, again)  # a list of expert weights is the same product, and no atomics: bit for bit
 
 
+@pytest.mark.parametrize("act", ["swiglu", "relu2", "gelu"])
+@pytest.mark.parametrize("W,ff,top", [(256, 256, 1), (384, 640, 1), (1024, 256, 2)])
+@pytest.mark.parametrize("counts", [[1, 33, 128, 129, 0, 256, 257], [288, 289, 127, 544, 0, 545, 32], [0, 0, 0, 0, 0, 0, 2305]])
+def test_wide_tiles_at_their_edges(counts, W, ff, top, act):
+    """Rows that just fill a half tile, a tile, a tile and its ninth block, and one more; widths of the shortest K range and of uneven ones; copies of no expert between."""
+    from llmctl.ops import hybrid as hops
+
+    E = len(counts)
+    chosen = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)] + [torch.full((40,), E)])
+    chosen = chosen[torch.randperm(len(chosen), generator=torch.Generator().manual_seed(W))]
+    T = -(-len(chosen) // top)
+    idx = torch.full((T * top,), E, dtype=torch.int32)
+    idx[:len(chosen)] = chosen.int()
+    idx = idx.view(T, top).cuda()
+    x, _, up, down = _case(T, W, ff, E, act, seed=sum(counts))
+    d3 = down.view(W, E, ff).transpose(0, 1)
+    w = torch.rand(T, top, device="cuda")
+    got = hops.native_hybrid().moe_experts(x, idx, w, [up], [d3], hops._EXPERT_ACTS[act])
+    want = _plain(x, idx.long(), w, up, d3, act, E)
+    # as above, row by row: a wrong row would not show in the norm of all
+    assert bool(((got.double() - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1) + 1e-12).all())
+
+
 @pytest.mark.parametrize("T", [5, 64, 65, 700])
 def test_one_expert_takes_all_and_experts_without_weights(T):
     from llmctl.ops import hybrid as hops
