@@ -92,11 +92,13 @@ def fwd64_pick(M: int, N: int, K: int) -> bool:
 
 
 def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, layout: str = "eager") -> torch.Tensor:
-    """``x @ w^T (+ b)``: small products on gemm_small (``small_pays``), gemm64 for the shapes ``fwd64_pick`` selects, hipBLASLt otherwise."""
+    """``x @ w^T (+ b)``: small products on gemm_small (``small_pays``), those of one to a few rounds of tiles on gemm_rows (``rows_form``), gemm64 for the shapes ``fwd64_pick`` selects, hipBLASLt otherwise."""
     N, K = w.shape
     M = x.numel() // K if x.shape[-1] == K else 0
     if M > 32 or layout != "eager":
         y = small_linear(x, w, b, layout)
+        if y is None:
+            y = rows_linear(x, w, b)
         if y is not None:
             return y
     if M and fwd64_pick(M, N, K) and x.dtype == torch.bfloat16:
@@ -187,6 +189,54 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
         return None
     y = torch.empty(M, N, dtype=x.dtype, device=x.device)
     native().gemm_small(x2, w, y, False, False, False, b, None, False, act)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
+
+
+_CUS = 256  # of an MI355X
+
+
+def _rounds_us(items: int, ktiles: float, empty: float, full: float, fixed: float) -> float:
+    """Workgroups of one to a CU: a round's K-tiles at ``empty`` us and ``full`` more on a full chip, and a fixed part."""
+    whole, rest = divmod(items, _CUS)
+    return whole * (ktiles * (empty + full) + fixed) + (ktiles * (empty + full * rest / _CUS) + fixed if rest else 0.0)
+
+
+@functools.lru_cache(maxsize=8192)
+def rows_form(M: int, N: int, K: int) -> int:
+    """The tiles of ``gemm_rows`` (csrc/gemm_rows.hip: 1 = 256 rows, 2 = 128) that multiply M rows of width K to N outputs faster than the library, or 0.  Times by a
+    model of either's workgroups and of the library's products, us: 12 and 1300 TFLOP/s, small ones 6 and 550; constants fitted to 245 sizes, 33 to 4096 rows, 256 to
+    12288 outputs, K 256 to 8192, operands from HBM (``profiles/prompt_products.txt``).  The rule takes 81 of them, in 20 % less time; one of these takes 4 % more.
+    us, library / here: 2048 x 2048 x 2048 25.8 / 17.8, 2048 x 3712 x 2048 35.5 / 29.0, 2911 x 2048 x 1024 23.2 / 16.8, 1128 x 3584 x 1664 21.4 / 15.5, 769 x 2816 x 256
+    9.4 / 6.4; left to the library: 1.1 rounds, 2911 x 3072 x 2048 36.8 / 46.0; few tiles and a long K, 551 x 1472 x 1024
+    9.2 / 9.6, 93 x 256 x 4608 12.8 / 24.6; large products, 3379 x 8192 x 2048 94 / 109."""
+    if M <= 32 or N <= 0 or N & 7 or K & 127 or K < 256:
+        return 0
+    cols, kt = -(-N // 128), K / 64
+    tall = _rounds_us((1 if M <= 288 else (M - 33) // 256 + 1) * cols, kt, 0.47, 0.36, 5.0)
+    half = _rounds_us(-(-M // 128) * cols, kt, 0.28, 0.18, 4.0)
+    gflop = 2e-9 * M * N * K
+    if min(tall, half) >= (0.95 if K <= 2304 else 0.85) * min(12.0 + gflop / 1.3, 6.0 + gflop / 0.55):  # (GPT-7B's, 900 x 4096 x 4096, 39 / 34, took its prompt 1 % longer)
+        return 0
+    return 1 if tall <= half else 2
+
+
+def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``x @ w^T (+ b)`` on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
+    None.  A library product takes the host 24 us, this 9: Lenitar's prompt of 2048 tokens, sixteen of them,
+    1198 us, so 1127 (kernels 1190 / 1106); gpt2-125m's of 700 and 300 tokens 2195 / 1870."""
+    N, K = w.shape
+    M = x.numel() // K if K and x.shape[-1] == K else 0
+    if not M or type(M * N) is not int or not rows_form(M, N, K) or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
+        return None  # (symbolic and traced sizes are no ints)
+    if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not (x.dim() == 2 or x.is_contiguous()) or _any_autocast()
+            or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
+            or _forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
+        return None
+    x2 = x if x.dim() == 2 else x.view(M, K)
+    if (not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (_small_bias(b, N) and b.data_ptr() & 15 == 0))
+            or 512 * x2.stride(0) >= 1 << 30 or 512 * w.stride(0) >= 1 << 30):
+        return None
+    y = native().gemm_rows(x2, w, b, rows_form(M, N, K))
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 

@@ -191,7 +191,7 @@ class LatentAttention(nn.Module):
     def _attend_expanded(self, q: torch.Tensor, b: StepBatch, lat: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
         """``lat``: the step's cache rows [latent | rotary key]; ``rows [T, H, dv + dn + dr]``, which hold the rotary key already."""
         T, H, dn, dr, dv = q.shape[0], self.H, self.dn, self.dr, self.dv
-        rows[:, :, :dv + dn] = F.linear(lat[:, :self.rk], self._w_uvk()).view(T, H, dv + dn)  # per head [v | k | shared rotary key]
+        rows[:, :, :dv + dn] = hops.linear(lat[:, :self.rk], self._w_uvk()).view(T, H, dv + dn)  # per head [v | k | shared rotary key]
         if self.qr:  # (a product of its own)
             qa = hops.rotary_tail_(q, b.pos, self.inv_freq, self.rot_dims, dn, self.interleaved, self.rot_amp)
         else:
@@ -581,7 +581,7 @@ class DenseFF(nn.Module):
             z = hops.rows_linear(h, self.w_up, self.b_up, self.act, self.ff)
             a = z[:, :self.ff]
         else:
-            z = F.linear(h, self.w_up, self.b_up)
+            z = hops.linear(h, self.w_up, self.b_up)
             a = hops.act_any(z[:, :self.ff], self.act)
         y = (hops.linear_parts if late else hops.linear)(a, self.w_down, self.b_down)
         return (y, z[:, self.ff:]) if self.side else y

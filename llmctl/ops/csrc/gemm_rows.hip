@@ -1,0 +1,117 @@
+// Products of a prompt's rows, y = act(x w^T (+ bias)) in bf16, on the tiles of wide_tiles.h: any number of rows, outputs in 8s, K in 128s from 256 on.
+//
+// Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, gemm_rows_form says.
+#include "wide_tiles.h"
+
+namespace llmctl {
+namespace {
+using namespace wide;
+
+struct RowsArgs {
+  const unsigned short* a;
+  const unsigned short* b;
+  const unsigned short* bias;
+  unsigned short* c;
+  long lda, ldb;
+  int M, N, K;
+  int tiles_m, tiles_n;
+};
+constexpr int BAND = 4;  // tile rows that walk the columns together
+
+template <bool HALVES>
+__global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_rows_kernel(RowsArgs g) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[3 * SLOT];
+  static_assert(4 * SLOT_H <= 3 * SLOT, "LDS");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave >> 1, wc = wave & 1;
+  // a run of neighbouring tiles to each XCD
+  const int n = g.tiles_m * g.tiles_n, q8 = n >> 3, r8 = n & 7, xcd = blockIdx.x & 7, tile = xcd * q8 + min(xcd, r8) + ((int)blockIdx.x >> 3);
+  const int first = tile / (BAND * g.tiles_n) * BAND, in = tile - first * g.tiles_n, high = min(BAND, g.tiles_m - first);
+  const int tn = in / high, tm = first + in - tn * high;
+  const int row0 = tm * (HALVES ? 128 : 256), rows = HALVES ? min(128, g.M - row0) : tm == g.tiles_m - 1 ? g.M - row0 : 256, col0 = tn * COLS;
+  // DMA offsets: piece i of an image holds its rows 32 i + tid / 8, chunk tid % 8 of a K-tile's eight at its swizzled place; rows past the end are the last one's
+  unsigned va[9], vb[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int ir = 32 * i + (tid >> 3);
+    vb[i] = (unsigned)min(ir, g.N - 1 - col0) * (unsigned)(g.ldb * 2) + (unsigned)(((tid & 7) ^ swr(ir)) << 4);
+  }
+  const Tile t{g.a + (long)row0 * g.lda, g.b + (long)col0 * g.ldb, g.K};
+  first_b<HALVES ? 2 : 3>(t, vb, smem, HALVES ? SLOT_H : SLOT, HALVES ? HALF : B_H0 * HALF);
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    const int ir = 32 * (i & 3) + (tid >> 3);
+    const int r = i == 8 ? 256 + (tid >> 3) : HALVES ? ir : i < 4 ? tile_pos<A_LO>(ir) : tile_pos<A_HI>(ir);
+    va[i] = (unsigned)min(r, rows - 1) * (unsigned)(g.lda * 2) + (unsigned)(((tid & 7) ^ swr(i == 8 ? tid >> 3 : ir)) << 4);
+  }
+  // lane holds [16 i + (l & 15)][16 j + 4 (l >> 4) + r] of its wave's part; 16 bytes to a lane: lanes of neighbouring groups swap halves of two column tiles
+  const int kg = lane >> 4, i16 = lane & 15, c0 = col0 + wc * 64 + 16 * (kg & 1) + 8 * (kg >> 1);
+  auto out = [&](auto mb_c) __attribute__((always_inline)) {
+    constexpr int MB = decltype(mb_c)::value;
+    f32x4_t acc[9][4];
+    if constexpr (MB == 4) run_half(t, va, vb, smem, acc);
+    else run<MB>(t, va, vb, smem, acc);
+    float bias[2][8];
+#pragma unroll
+    for (int jp = 0; jp < 2; ++jp) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bias[jp][e] = 0.f;
+      if (g.bias != nullptr && c0 + 32 * jp < g.N) load8(g.bias + c0 + 32 * jp, bias[jp]);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int r = i == 8 ? 256 + wr * 16 + i16 : wr * (HALVES ? 64 : 128) + 16 * i + i16;
+#pragma unroll
+      for (int jp = 0; jp < 2; ++jp) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[i][2 * jp][e]), __float_as_uint(acc[i][2 * jp + 1][e]), false, false);
+          v[e] = __uint_as_float(s[0]);
+          v[4 + e] = __uint_as_float(s[1]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += bias[jp][e];
+        if (r < rows && c0 + 32 * jp < g.N) store8(g.c + (long)(row0 + r) * g.N + c0 + 32 * jp, v);
+      }
+    }
+  };
+  if constexpr (HALVES) {
+    out(K_<4>{});
+  } else {
+    if (rows <= 256) out(K_<8>{});
+    else out(K_<9>{});
+  }
+}
+
+int row_tiles(int64_t M) { return M <= ROWS ? 1 : (int)((M - 33) / 256 + 1); }
+}  // namespace
+
+// y [M, N] = x w^T (+ bias); form: 1 = tiles of 256 rows, 2 = of 128
+at::Tensor gemm_rows(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t form) {
+  LLMCTL_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_cuda() && w.is_cuda() && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.stride(1) == 1 &&
+                   w.stride(1) == 1,
+               "gemm_rows: bf16 GPU x [M, K] and w [N, K] with unit inner strides");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  LLMCTL_CHECK(w.size(1) == K && K % 128 == 0 && K >= 256 && N % 8 == 0 && (form == 1 || form == 2), "gemm_rows: K in 128s from 256 on, N in 8s, form 1 or 2");
+  LLMCTL_CHECK(x.stride(0) % 8 == 0 && w.stride(0) % 8 == 0 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 && (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0,
+               "gemm_rows: 16-byte aligned rows");
+  const bool has_bias = bias.has_value() && bias->defined();
+  if (has_bias)
+    LLMCTL_CHECK(bias->is_cuda() && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N && (reinterpret_cast<uintptr_t>(bias->data_ptr()) & 15) == 0,
+                 "gemm_rows: bias bf16 [N], aligned to 16 bytes");
+  LLMCTL_CHECK(ROWS * x.stride(0) < (1L << 30) && COLS * w.stride(0) < (1L << 30) && x.stride(0) >= 0 && w.stride(0) >= 0 && M < (1L << 31) && N < (1L << 31),
+               "gemm_rows: operand too large for 32-bit offsets");
+  const c10::DeviceGuard guard(x.device());
+  at::Tensor y = at::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return y;
+  RowsArgs g{bf_ptr(x), bf_ptr(w), has_bias ? bf_ptr(*bias) : nullptr, reinterpret_cast<unsigned short*>(y.data_ptr()), (long)x.stride(0), (long)w.stride(0),
+             (int)M, (int)N, (int)K, form == 1 ? row_tiles(M) : (int)((M + 127) / 128), (int)((N + COLS - 1) / COLS)};
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
+  if (form == 1) gemm_rows_kernel<false><<<grid, NT4, 0, stream()>>>(g);
+  else gemm_rows_kernel<true><<<grid, NT4, 0, stream()>>>(g);
+  return y;
+}
+
+TORCH_LIBRARY_IMPL(llmctl, CUDA, m) { m.impl("gemm_rows", &gemm_rows); }
+
+}  // namespace llmctl

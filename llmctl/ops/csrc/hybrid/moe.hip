@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
 #include "moe_wide.h"
 namespace llmctl_hybrid {
 namespace {
-static_assert(WIDE_ROWS == wide::ROWS, "row tiles");
+static_assert(WIDE_ROWS == llmctl::wide::ROWS, "row tiles");
 
 // ------------------------------------------------------------------------------------------------ few tokens
 struct SmallArgs {
@@ -682,7 +682,7 @@ at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Ten
     // widths in no 128s, of 128 or 64
     const bool wide = (N >= 96 * E || (N >= 48 * E && (N / 64 + E / 2) * (W / 64) >= 400)) && W % 128 == 0 && ff % 128 == 0 && W >= 256 && ff >= 256 && T * x.stride(0) < ((int64_t)1 << 30) && N * ff < ((int64_t)1 << 30) &&
                       R * ldu < ((int64_t)1 << 30) && W * ldd < ((int64_t)1 << 30);
-    const int BM = wide ? WIDE_ROWS : N >= 96 * E ? 128 : 64, BN = wide ? wide::COLS : BM;
+    const int BM = wide ? WIDE_ROWS : N >= 96 * E ? 128 : 64, BN = wide ? llmctl::wide::COLS : BM;
     const int64_t mt = wide ? N / 256 + E : (N + BM - 1) / BM + E;  // no more row tiles than this
     at::Tensor ints = at::empty({N + 2 + 3 * mt}, idx.options());
     int* perm = ints.data_ptr<int>();

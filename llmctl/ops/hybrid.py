@@ -513,15 +513,27 @@ def rows_linear(x, w, b=None, act=None, act_cols=None, f32: bool = False):
     return native_hybrid().rows_linear(x, w, b, _ROW_ACTS[act], w.shape[0] if act_cols is None else act_cols, f32)
 
 
+_prompt_linear = None  # exec.linear's rows_linear (which imports this package: at the first call)
+
+
+def _library_linear(x, w, b, other):
+    global _prompt_linear
+    if _prompt_linear is None:
+        from llmctl.exec.linear import rows_linear as _prompt_linear
+    y = _prompt_linear(x, w, b)
+    return other(x, w, b) if y is None else y
+
+
 def linear(x, w, b=None):
-    """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), others are the library's product."""
-    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else torch.nn.functional.linear(x, w, b)
+    """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), prompts run on the tiles of ``csrc/gemm_rows.hip`` where these are faster than the
+    library's product (:func:`llmctl.exec.linear.rows_form`)."""
+    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else _library_linear(x, w, b, torch.nn.functional.linear)
 
 
 def odd_linear(x, w, b=None):
-    """:func:`linear` where the outputs may fill no whole tiles and no expert choice hangs on the order of the sums: prompts take
+    """:func:`linear` where the outputs may fill no whole tiles and no expert choice hangs on the order of the sums: large prompts take
     :func:`llmctl.ops.functional.odd_linear`'s form."""
-    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else wide_linear(x, w, b)
+    return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else _library_linear(x, w, b, wide_linear)
 
 
 class Normed:

@@ -1,0 +1,50 @@
+"""Prompt products on tiles of up to 288 rows x 128: rows that just fill a tile and one more, the shortest K and odd numbers of pairs of K-tiles, outputs that fill no tile, rows wider
+than the matrix, a bias; and the route that takes them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 33, 128, 129, 256, 288, 289, 544, 545, 1000])
+@pytest.mark.parametrize("N,K,pad", [(8, 256, 0), (128, 384, 8), (264, 640, 0), (1000, 2048, 8)])
+@pytest.mark.parametrize("form", [1, 2])
+def test_products(M, N, K, pad, form):
+    from llmctl.ops._lib import native
+
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    rows = lambda n: torch.randn(n, K + pad, generator=g, device="cuda").bfloat16()[:, :K]
+    x, w = rows(M), rows(N)
+    b = torch.randn(N, generator=g, device="cuda").bfloat16() if pad else None
+    got = native().gemm_rows(x, w, b, form)
+    X, W = x.double(), w.double()
+    ref, mag = X @ W.t(), X.abs() @ W.abs().t()
+    if b is not None:
+        ref, mag = ref + b.double(), mag + b.double().abs()
+    bound = (K + 1) * 2.0**-24 * mag  # fp32 sums of K exact products in any order; then one rounding
+    assert bool(((got.double() - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
+
+
+def test_route():
+    """Sizes of the rule run on these tiles, inside autograd too; other callers keep the library: a wanted gradient outside of it, autocast, batched rows of a transform."""
+    import importlib
+
+    L = importlib.import_module("llmctl.exec.linear")
+    assert L.rows_form(2048, 2048, 2048) == 2 and L.rows_form(2911, 2048, 1024) == 1
+    assert not any(L.rows_form(*s) for s in ((32, 2048, 2048), (2048, 2044, 2048), (2048, 2048, 2000), (2048, 2048, 128), (93, 256, 4608), (3379, 8192, 2048), (0, 256, 256)))
+    x, w = (torch.randn(n, 1024, device="cuda", dtype=torch.bfloat16) for n in (1500, 2048))
+    b = torch.randn(2048, device="cuda", dtype=torch.bfloat16)
+    ref = x.double() @ w.double().t() + b.double()
+    for y in (L.rows_linear(x, w, b), L.rows_linear(x.view(3, 500, 1024), w, b).view(1500, 2048)):
+        assert float((y.double() - ref).norm() / ref.norm()) < 2.0**-9
+    p = w.clone().requires_grad_()
+    assert L.rows_linear(x, p, b) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert L.rows_linear(x, w, b) is None
+    assert L.rows_linear(x[:, 1:], w[:, 1:]) is None and L.rows_linear(x.t().contiguous().t(), w) is None and L.rows_linear(x.float(), w.float()) is None
+    y = torch.vmap(lambda t: L.forward_linear(t, w, b))(x.view(3, 500, 1024))
+    assert float((y.reshape(1500, 2048).double() - ref).norm() / ref.norm()) < 2.0**-8
+    xg = x.clone().requires_grad_()
+    y = L.linear(xg, p, b)
+    y.sum().backward()
+    assert float((y.double() - ref).norm() / ref.norm()) < 2.0**-9 and xg.grad is not None and p.grad is not None
