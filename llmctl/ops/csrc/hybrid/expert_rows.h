@@ -29,6 +29,13 @@ template <typename Y, int NT, int VQ>
 __device__ __forceinline__ void expert_sum_quads(const ExpertRows& m, int64_t r, int W, float4 (&s)[VQ]) {
 #pragma unroll
   for (int i = 0; i < VQ; ++i) s[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 sv[VQ];
+  float gate = 0.f;
+  if (m.shared != nullptr) {  // (asked for with the rest, used last)
+    if (m.gate != nullptr) gate = ldf(m.gate + r * m.ld_gate);
+#pragma unroll
+    for (int i = 0; i < VQ; ++i) sv[i] = ld4(m.shared + r * m.ld_shared + min((int)(threadIdx.x + i * NT) * 4, W - 4));
+  }
   for (int k0 = 0; k0 < m.top; k0 += 2) {
     float4 v[2][VQ];
     int id[2];
@@ -53,11 +60,10 @@ __device__ __forceinline__ void expert_sum_quads(const ExpertRows& m, int64_t r,
     }
   }
   if (m.shared != nullptr) {
-    const float g = m.gate != nullptr ? 1.0f / (1.0f + expf(-ldf(m.gate + r * m.ld_gate))) : 1.0f;
+    const float g = m.gate != nullptr ? 1.0f / (1.0f + expf(-gate)) : 1.0f;
 #pragma unroll
     for (int i = 0; i < VQ; ++i) {
-      const float4 v = ld4(m.shared + r * m.ld_shared + min((int)(threadIdx.x + i * NT) * 4, W - 4));
-      s[i].x = fmaf(g, v.x, s[i].x), s[i].y = fmaf(g, v.y, s[i].y), s[i].z = fmaf(g, v.z, s[i].z), s[i].w = fmaf(g, v.w, s[i].w);
+      s[i].x = fmaf(g, sv[i].x, s[i].x), s[i].y = fmaf(g, sv[i].y, s[i].y), s[i].z = fmaf(g, sv[i].z, s[i].z), s[i].w = fmaf(g, sv[i].w, s[i].w);
     }
   }
 }

@@ -124,41 +124,53 @@ __global__ __launch_bounds__(NT) void norm_add_parts_kernel(float* __restrict__ 
                                                             float s1, const float* __restrict__ y2, int n2, float s2, const float* __restrict__ w,
                                                             float mult, float plus, bf16_t* __restrict__ h, int W, int64_t TW, float eps,
                                                             const float* __restrict__ wn) {
-  __shared__ float red[NW];
+  __shared__ float red[2][NW];
+  constexpr int B = VQ == 4 ? 4 : 8;  // ranges asked for at once
   const int64_t row = blockIdx.x;
-  float4 a[VQ], xv[VQ], wv[VQ];
-  float q = 0.f;
-  auto add = [&](const float* y, int n, float scale) {
-    float4 p[VQ];
+  float4 a[VQ], xv[VQ], wv[VQ], nv[VQ], r1[B][VQ], r2[B][VQ];
+  auto load = [&](const float* y, int n, int s0, float4 (&p)[B][VQ]) {
 #pragma unroll
-    for (int i = 0; i < VQ; ++i) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 4
-    for (int s = 0; s < n; ++s)
+    for (int s = 0; s < B; ++s)
 #pragma unroll
-      for (int i = 0; i < VQ; ++i) {
-        const float4 v = *reinterpret_cast<const float4*>(y + s * TW + row * W + min((int)(threadIdx.x + i * NT) * 4, W - 4));
-        p[i].x += v.x, p[i].y += v.y, p[i].z += v.z, p[i].w += v.w;
-      }
-#pragma unroll
-    for (int i = 0; i < VQ; ++i) a[i].x = fmaf(scale, p[i].x, a[i].x), a[i].y = fmaf(scale, p[i].y, a[i].y), a[i].z = fmaf(scale, p[i].z, a[i].z), a[i].w = fmaf(scale, p[i].w, a[i].w);
+      for (int i = 0; i < VQ; ++i)
+        if (s0 + s < n) p[s][i] = *reinterpret_cast<const float4*>(y + (s0 + s) * TW + row * W + min((int)(threadIdx.x + i * NT) * 4, W - 4));
   };
+  load(y1, n1, 0, r1);
+  if (y2 != nullptr) load(y2, n2, 0, r2);
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = min((int)(threadIdx.x + i * NT) * 4, W - 4);
     xv[i] = *reinterpret_cast<const float4*>(x + row * W + c);
     wv[i] = *reinterpret_cast<const float4*>(w + c);
+    nv[i] = *reinterpret_cast<const float4*>((wn != nullptr ? wn : w) + c);
     a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (bias != nullptr) {
       const float4 b = ld4(bias + c);
       a[i] = make_float4(s1 * b.x, s1 * b.y, s1 * b.z, s1 * b.w);
     }
   }
-  add(y1, n1, s1);
-  if (y2 != nullptr) add(y2, n2, s2);
+  auto add = [&](const float* y, int n, float scale, float4 (&r)[B][VQ]) {
+    float4 p[VQ];
+#pragma unroll
+    for (int i = 0; i < VQ; ++i) p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < n; s0 += B) {
+      if (s0 > 0) load(y, n, s0, r);
+#pragma unroll
+      for (int s = 0; s < B; ++s)
+#pragma unroll
+        for (int i = 0; i < VQ; ++i)
+          if (s0 + s < n) p[i].x += r[s][i].x, p[i].y += r[s][i].y, p[i].z += r[s][i].z, p[i].w += r[s][i].w;
+    }
+#pragma unroll
+    for (int i = 0; i < VQ; ++i) a[i].x = fmaf(scale, p[i].x, a[i].x), a[i].y = fmaf(scale, p[i].y, a[i].y), a[i].z = fmaf(scale, p[i].z, a[i].z), a[i].w = fmaf(scale, p[i].w, a[i].w);
+  };
+  add(y1, n1, s1, r1);
+  if (y2 != nullptr) add(y2, n2, s2, r2);
+  float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i)
     if ((int)(threadIdx.x + i * NT) * 4 < W) q += a[i].x * a[i].x + a[i].y * a[i].y + a[i].z * a[i].z + a[i].w * a[i].w;
-  const float f = mult / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+  const float f = mult / sqrtf(block_sum<NW, true>(q, red[0]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
@@ -177,12 +189,12 @@ __global__ __launch_bounds__(NT) void norm_add_parts_kernel(float* __restrict__ 
 #pragma unroll
   for (int i = 0; i < VQ; ++i)
     if ((int)(threadIdx.x + i * NT) * 4 < W) q += a[i].x * a[i].x + a[i].y * a[i].y + a[i].z * a[i].z + a[i].w * a[i].w;
-  const float fn = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+  const float fn = 1.0f / sqrtf(block_sum<NW, true>(q, red[1]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
     if (c >= W) break;
-    const float4 n = *reinterpret_cast<const float4*>(wn + c);
+    const float4 n = nv[i];
     const float v[4] = {a[i].x * fn * (n.x + plus), a[i].y * fn * (n.y + plus), a[i].z * fn * (n.z + plus), a[i].w * fn * (n.w + plus)};
     stn<bf16_t, 4>(h + row * W + c, v);
   }

@@ -3,6 +3,8 @@
 
 #include "hybrid_common.h"
 
+#include <type_traits>
+
 namespace llmctl_hybrid {
 
 constexpr int MAX_ROUTED = 128;  // router outputs
@@ -17,16 +19,14 @@ RouterChoice router_choice(const at::Tensor& w, int64_t W, const c10::optional<a
 
 // Over the wave, or (not ``wide``) over its first 16 lanes, where alone the result then is.
 __device__ __forceinline__ float wave_max_of(float v, bool wide) {
-  if (wide) v = fmaxf(v, __shfl_xor(v, 32, 64)), v = fmaxf(v, __shfl_xor(v, 16, 64));
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  if (wide) return wave_max(v);
+  v = fmaxf(v, row_ror<8>(v)), v = fmaxf(v, row_ror<4>(v)), v = fmaxf(v, row_ror<2>(v));
+  return fmaxf(v, row_ror<1>(v));
 }
 __device__ __forceinline__ float wave_sum_of(float v, bool wide) {
-  if (wide) v += __shfl_xor(v, 32, 64), v += __shfl_xor(v, 16, 64);
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  if (wide) return wave_sum(v);
+  v += row_ror<8>(v), v += row_ror<4>(v), v += row_ror<2>(v);
+  return v + row_ror<1>(v);
 }
 
 // The lowest index of the largest of up to 128 values, two per lane (indices lane and lane + 64), among those with ``in``; the
@@ -108,20 +108,28 @@ __device__ __forceinline__ void choose_experts(float* lg, int lane, const Router
   }
 }
 
-// Logits of one row under the fp32 router weight w [E, W], and the choice; a workgroup of NW waves holds the row (as it rounds to bf16) in
-// quads threadIdx.x + i * 64 * NW.  ``part`` [NW][8] and ``lg`` [MAX_ROUTED] in LDS.  For steps of few rows: a row reads all of the
-// weight, from L2, and the row's kernel is on the chip anyway (a launch of its own: 10 us for 16 rows; here 4).
+// The router weight's rows e0 .. e0 + 7, as a workgroup of NW waves multiplies them: quads threadIdx.x + i * 64 * NW.
 template <int NW, int VQ>
-__device__ __forceinline__ void route_row(const float* __restrict__ w, const RouterChoice& c, const float4 (&h)[VQ], int W, float (*part)[8], float* lg,
-                                          int* __restrict__ idx, float* __restrict__ wgt) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int e0 = 0; e0 < c.E; e0 += 8) {
-    float4 wv[8][VQ];
+struct RouterRows {
+  float4 v[8][VQ];
+  __device__ __forceinline__ void load(const float* __restrict__ w, int E, int W, int e0) {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int i = 0; i < VQ; ++i) wv[j][i] = ld4(w + (int64_t)min(e0 + j, c.E - 1) * W + min((tid + i * 64 * NW) * 4, W - 4));
-    __builtin_amdgcn_sched_barrier(0);  // all in flight
+      for (int i = 0; i < VQ; ++i) v[j][i] = ld4(w + (int64_t)min(e0 + j, E - 1) * W + min(((int)threadIdx.x + i * 64 * NW) * 4, W - 4));
+  }
+};
+
+// Logits of one row under the fp32 router weight w [E, W], and the choice; a workgroup of NW waves holds the row (as it rounds to bf16) in
+// quads threadIdx.x + i * 64 * NW.  ``wv``: the first eight rows of the weight, asked for with the row itself.  ``part`` [NW][8] and
+// ``lg`` [MAX_ROUTED] in LDS.  For steps of few rows: a row reads all of the weight, from L2, and the row's kernel is on the chip anyway
+// (a launch of its own: 10 us for 16 rows; here 2).
+template <int NW, int VQ>
+__device__ __forceinline__ void route_row(const float* __restrict__ w, const RouterChoice& c, const float4 (&h)[VQ], RouterRows<NW, VQ>& wv, int W, float (*part)[8],
+                                          float* lg, int* __restrict__ idx, float* __restrict__ wgt) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int e0 = 0; e0 < c.E; e0 += 8) {
+    if (e0 > 0) wv.load(w, c.E, W, e0);
     float a[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -129,21 +137,26 @@ __device__ __forceinline__ void route_row(const float* __restrict__ w, const Rou
 #pragma unroll
       for (int i = 0; i < VQ; ++i)
         if ((tid + i * 64 * NW) * 4 < W)
-          a[j] = fmaf(h[i].x, wv[j][i].x, fmaf(h[i].y, wv[j][i].y, fmaf(h[i].z, wv[j][i].z, fmaf(h[i].w, wv[j][i].w, a[j]))));
+          a[j] = fmaf(h[i].x, wv.v[j][i].x, fmaf(h[i].y, wv.v[j][i].y, fmaf(h[i].z, wv.v[j][i].z, fmaf(h[i].w, wv.v[j][i].w, a[j]))));
     }
-    // eight sums over the wave: every exchange halves what a lane keeps, so lane 8 v ends with sum v
+    // eight sums over the wave: every exchange, with the lanes 32, 16 and 8 away, halves what a lane keeps, so lane 8 v ends with sum v
 #pragma unroll
-    for (int n = 4; n >= 1; n >>= 1) {
-      const bool high = (lane & (8 * n)) != 0;
-#pragma unroll
-      for (int j = 0; j < n; ++j) {
-        const float give = high ? a[j] : a[j + n], own = high ? a[j + n] : a[j];
-        a[j] = own + __shfl_xor(give, 8 * n, 64);
-      }
+    for (int j = 0; j < 4; ++j) {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[j]), __float_as_uint(a[j + 4]), false, false);
+      a[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
 #pragma unroll
-    for (int o = 4; o > 0; o >>= 1) a[0] += __shfl_xor(a[0], o, 64);
-    if ((lane & 7) == 0) part[wave][lane >> 3] = a[0];
+    for (int j = 0; j < 2; ++j) {
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[j]), __float_as_uint(a[j + 2]), false, false);
+      a[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    const bool high = (lane & 8) != 0;
+    float t = (high ? a[1] : a[0]) + row_ror<8>(high ? a[0] : a[1]);
+    auto dpp = [](float v, auto ctrl) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, 0xf, 0xf, true)); };
+    t += dpp(dpp(t, std::integral_constant<int, 0x1b>{}), std::integral_constant<int, 0x141>{});  // quads and then eights mirrored: the lane 4 away
+    t += dpp(t, std::integral_constant<int, 0x4e>{});
+    t += dpp(t, std::integral_constant<int, 0xb1>{});
+    if ((lane & 7) == 0) part[wave][lane >> 3] = t;
     __syncthreads();
     if (tid < 8 && e0 + tid < c.E) {
       float s = part[0][tid];
@@ -164,12 +177,12 @@ struct RouteOut {
   float* wgt;
 
   template <int NW, int VQ>
-  __device__ __forceinline__ void row(float4 (&h)[VQ], int64_t r, int W) const {
+  __device__ __forceinline__ void row(float4 (&h)[VQ], RouterRows<NW, VQ>& wv, int64_t r, int W) const {
     __shared__ float part[NW][8], lg[MAX_ROUTED];
     auto bf = [](float v) { return __bfloat162float(__float2bfloat16(v)); };
 #pragma unroll
     for (int i = 0; i < VQ; ++i) h[i] = make_float4(bf(h[i].x), bf(h[i].y), bf(h[i].z), bf(h[i].w));
-    route_row<NW, VQ>(w, c, h, W, part, lg, idx + r * c.top, wgt + r * c.top);
+    route_row<NW, VQ>(w, c, h, wv, W, part, lg, idx + r * c.top, wgt + r * c.top);
   }
 };
 

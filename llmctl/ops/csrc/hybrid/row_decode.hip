@@ -260,7 +260,15 @@ __global__ __launch_bounds__(WAVES * 64, NK > 18 ? 1 : 2) void row_decode_kernel
 __global__ __launch_bounds__(128) void row_merge_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, unsigned short* __restrict__ out,
                                                         int nsplit, int rk, const float* __restrict__ ofreq, const int* __restrict__ ctx, int H) {
   __shared__ float fac[64];
+  constexpr int B = 8;  // splits asked for at once, the first of them before their factors are there
   const long row = blockIdx.x;
+  float4 x[B];
+  auto load = [&](int s0, int c) {
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (s0 + u < nsplit && c < rk) x[u] = *reinterpret_cast<const float4*>(ws_o + (row * nsplit + s0 + u) * rk + c);
+  };
+  load(0, threadIdx.x * 4);
   if (threadIdx.x < 64) {
     const int s = threadIdx.x;
     const float m = s < nsplit ? ws_ml[(row * nsplit + s) * 2] : -INFINITY, l = s < nsplit ? ws_ml[(row * nsplit + s) * 2 + 1] : 0.f;
@@ -272,11 +280,14 @@ __global__ __launch_bounds__(128) void row_merge_kernel(const float* __restrict_
   __syncthreads();
   for (int c = threadIdx.x * 4; c < rk; c += 512) {
     float v[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int s = 0; s < nsplit; ++s) {  // (a split that saw nothing wrote zeros)
-      const float f = fac[s];
-      const float4 x = *reinterpret_cast<const float4*>(ws_o + (row * nsplit + s) * rk + c);
-      v[0] = fmaf(x.x, f, v[0]), v[1] = fmaf(x.y, f, v[1]), v[2] = fmaf(x.z, f, v[2]), v[3] = fmaf(x.w, f, v[3]);
+    for (int s0 = 0; s0 < nsplit; s0 += B) {  // (a split that saw nothing wrote zeros)
+      if (s0 > 0 || c >= 512) load(s0, c);
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        if (s0 + u >= nsplit) break;
+        const float f = fac[s0 + u];
+        v[0] = fmaf(x[u].x, f, v[0]), v[1] = fmaf(x[u].y, f, v[1]), v[2] = fmaf(x[u].z, f, v[2]), v[3] = fmaf(x[u].w, f, v[3]);
+      }
     }
     if (ofreq != nullptr) turn_back(v, ofreq, (float)(ctx[row / H] - 1), c);
     store4(out + row * rk + c, v);

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
                                                                  const float* __restrict__ b, const float* __restrict__ w,
                                                                  const float* __restrict__ bias, T* __restrict__ h, int W, float eps,
                                                                  ExpertRows m, RouteOut route) {
-  __shared__ float red[NW];
+  __shared__ float red[2][NW];
   const int64_t r = blockIdx.x;
   float4 v[VQ], av[VQ], bv[VQ], wv[VQ], cv[VQ];
 #pragma unroll
@@ -60,6 +60,8 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
     if constexpr (std::is_void_v<Y>) bv[i] = b != nullptr ? ld4(b + r * W + c) : make_float4(0.f, 0.f, 0.f, 0.f);
     if (h != nullptr) wv[i] = ld4(w + c), cv[i] = ld4(bias + c);
   }
+  RouterRows<NW, VQ> rw;
+  if constexpr (ROUTE) rw.load(route.w, route.c.E, W, 0);
   if constexpr (!std::is_void_v<Y>) expert_sum_quads<Y, NT, VQ>(m, r, W, bv);
   float s = 0.f;
 #pragma unroll
@@ -73,14 +75,14 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
     }
   }
   if (h == nullptr) return;
-  const float mean = block_sum<NW>(s, red) / (float)W;
+  const float mean = block_sum<NW, true>(s, red[0]) / (float)W;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     v[i].x -= mean, v[i].y -= mean, v[i].z -= mean, v[i].w -= mean;
     if ((int)(threadIdx.x + i * NT) * 4 < W) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
   }
-  const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+  const float rstd = 1.0f / sqrtf(block_sum<NW, true>(q, red[1]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(NT) void add_layernorm_quads_kernel(float* __restri
                        v[i].w * rstd * wv[i].w + cv[i].w);
     if (c < W) st4(h + r * W + c, v[i]);
   }
-  if constexpr (ROUTE) route.row<NW, VQ>(v, r, W);
+  if constexpr (ROUTE) route.row<NW, VQ>(v, rw, r, W);
 }
 
 // The first of a step: x = table[id] * scale, h = LayerNorm(x) * w + bias; the product in fp32, as a cast and a multiplication give it.  One
@@ -97,7 +99,7 @@ template <typename T, int VQ, bool ROUTE>
 __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t* __restrict__ ids, const T* __restrict__ table, int64_t rows,
                                                                    float scale, const float* __restrict__ w, const float* __restrict__ bias,
                                                                    float* __restrict__ x, T* __restrict__ h, int W, float eps, RouteOut route) {
-  __shared__ float red[NW];
+  __shared__ float red[2][NW];
   const int64_t r = blockIdx.x, id = ids[r];
   CUDA_KERNEL_ASSERT(id >= 0 && id < rows);
   float4 v[VQ], wv[VQ], cv[VQ];
@@ -108,6 +110,8 @@ __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t
     wv[i] = ld4(w + c);
     cv[i] = ld4(bias + c);
   }
+  RouterRows<NW, VQ> rw;
+  if constexpr (ROUTE) rw.load(route.w, route.c.E, W, 0);
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
@@ -118,14 +122,14 @@ __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t
       s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
   }
-  const float mean = block_sum<NW>(s, red) / (float)W;
+  const float mean = block_sum<NW, true>(s, red[0]) / (float)W;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     v[i].x -= mean, v[i].y -= mean, v[i].z -= mean, v[i].w -= mean;
     if ((int)(threadIdx.x + i * NT) * 4 < W) q += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
   }
-  const float rstd = 1.0f / sqrtf(block_sum<NW>(q, red) / (float)W + eps);
+  const float rstd = 1.0f / sqrtf(block_sum<NW, true>(q, red[1]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < VQ; ++i) {
     const int c = (int)(threadIdx.x + i * NT) * 4;
@@ -133,7 +137,7 @@ __global__ __launch_bounds__(NT) void embed_layernorm_quads_kernel(const int64_t
                        v[i].w * rstd * wv[i].w + cv[i].w);
     if (c < W) st4(h + r * W + c, v[i]);
   }
-  if constexpr (ROUTE) route.row<NW, VQ>(v, r, W);
+  if constexpr (ROUTE) route.row<NW, VQ>(v, rw, r, W);
 }
 
 // Rows that the quads do not take: x alone, its LayerNorm by add_layernorm_kernel.
