@@ -430,8 +430,10 @@ class MLSTM(nn.Module):
         q, k = z[:, :H * dk].view(T, H, dk), z[:, H * dk:2 * H * dk].view(T, H, dk)
         v = z[:, 2 * H * dk:2 * H * dk + H * dv].view(T, H, dv)
         g = z[:, 2 * H * dk + H * dv:]
-        gates = hops.linear_f32w(h, self.w_if, few=b.Tp == 0)  # fp32 [T, 2H]
         S, n, m = state
+        if hops.state_decode_ok(z, S, b, dv):
+            return hops.linear(hops.mlstm_decode(q, k, v, h, self.w_if, self.b_i, self.b_f, self.cap, 1.0 / math.sqrt(dk), S, n, m, b, self.norm, g, self.eps), self.w_o)
+        gates = hops.linear_f32w(h, self.w_if, few=b.Tp == 0)  # fp32 [T, 2H]
         key = ("mlstm_plan", H, dk, dv)
         if key not in b.scratch:
             b.scratch[key] = hops.mlstm_chunk_plan(b.cu_host, h.device, H, dk, dv) if h.is_cuda else None
@@ -490,7 +492,11 @@ class GatedLinearAttention(nn.Module):
         q, k = z[:, :a].unflatten(1, (H, dk)), z[:, a:c].unflatten(1, (H, dk))
         v = z[:, c:e].unflatten(1, (H, dv))
         g = z[:, e:e + H * dv]
-        decay = _mm_f32(z[:, e + H * dv:self.cols], self.w_a2)  # fp32 [T, H * dk]
+        low = z[:, e + H * dv:self.cols]
+        if hops.state_decode_ok(z, state[0], b, dv) and low.dtype == self.w_a2.dtype and self.w_a2.is_contiguous():
+            y = hops.linear(hops.gla_decode(q, k, v, low, self.w_a2, self.b_a2, self.tau, dk ** -0.5, state[0], b, self._norm_rows(), g, self.eps), self.w_o)
+            return (y, z[:, self.cols:]) if self.side else y
+        decay = _mm_f32(low, self.w_a2)  # fp32 [T, H * dk]
         key = ("gla_plan", H, dk, dv)
         if key not in b.scratch:
             b.scratch[key] = hops.gla_plan(b.cu_host, h.device, H, dk, dv) if h.is_cuda else None

@@ -95,6 +95,11 @@ at::Tensor act_any(const at::Tensor& x, int64_t kind, const c10::optional<at::Te
 at::Tensor qk_fullnorm_prep(const at::Tensor& z, int64_t H, int64_t G, int64_t dk, int64_t dv, const at::Tensor& q_norm, const at::Tensor& k_norm,
                             double eps, const at::Tensor& pos, double temp_coef, int64_t temp_every, at::Tensor cache, const at::Tensor& slots,
                             const c10::optional<at::Tensor>& freq, int64_t rot, bool interleaved, double amp);
+at::Tensor gla_decode(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& a, const at::Tensor& w, const at::Tensor& b, double tau,
+                      double qscale, at::Tensor S, const at::Tensor& slots, const at::Tensor& start, const at::Tensor& hn_w, const at::Tensor& hn_g, double eps);
+at::Tensor mlstm_decode(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const c10::optional<at::Tensor>& raw, const at::Tensor& h, const at::Tensor& w,
+                        const at::Tensor& b_i, const at::Tensor& b_f, double cap, double qscale, at::Tensor S, at::Tensor n, at::Tensor m, const at::Tensor& slots,
+                        const at::Tensor& start, const at::Tensor& hn_w, const at::Tensor& hn_g, double eps);
 at::Tensor gla_scan(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& z, const at::Tensor& z_bias,
                     double tau, double qscale, at::Tensor S, const at::Tensor& slots, const at::Tensor& cu, const at::Tensor& start,
                     const c10::optional<at::Tensor>& logd, bool write_out, bool write_state);
@@ -194,6 +199,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("gated_norm_add_experts_f32_(Tensor(a!) x, Tensor r, Tensor w_post, Tensor? w_next, float eps, Tensor ye, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts) -> Tensor");
   m.def("act_any(Tensor x, int kind, Tensor? scale=None) -> Tensor");
   m.def("qk_fullnorm_prep(Tensor z, int H, int G, int dk, int dv, Tensor q_norm, Tensor k_norm, float eps, Tensor pos, float temp_coef, int temp_every, Tensor(a!) cache, Tensor slots, Tensor? freq=None, int rot=0, bool interleaved=False, float amp=1.0) -> Tensor");
+  m.def("gla_decode(Tensor q, Tensor k, Tensor v, Tensor a, Tensor w, Tensor b, float tau, float qscale, Tensor(a!) S, Tensor slots, Tensor start, Tensor hn_w, Tensor hn_g, float eps) -> Tensor");
+  m.def("mlstm_decode(Tensor q, Tensor k, Tensor v, Tensor? raw, Tensor h, Tensor w, Tensor b_i, Tensor b_f, float cap, float qscale, Tensor(a!) S, Tensor(b!) n, Tensor(c!) m, Tensor slots, Tensor start, Tensor hn_w, Tensor hn_g, float eps) -> Tensor");
   m.def("gla_scan(Tensor q, Tensor k, Tensor v, Tensor z, Tensor z_bias, float tau, float qscale, Tensor(a!) S, Tensor slots, Tensor cu, Tensor start, Tensor(b!)? logd=None, bool write_out=True, bool write_state=True) -> Tensor");
   m.def("latent_q_rows(Tensor q, Tensor w_uk, Tensor pos, Tensor inv_freq, int rot_dims, bool interleaved, float amp) -> Tensor");
   m.def("latent_out_rows(Tensor o, Tensor w, Tensor? gate=None) -> Tensor");
@@ -257,6 +264,8 @@ TORCH_LIBRARY_IMPL(llmctl_hybrid, CUDA, m) {
   m.impl("gated_norm_add_experts_f32_", &llmctl_hybrid::gated_norm_add_experts_f32_);
   m.impl("act_any", &llmctl_hybrid::act_any);
   m.impl("qk_fullnorm_prep", &llmctl_hybrid::qk_fullnorm_prep);
+  m.impl("gla_decode", &llmctl_hybrid::gla_decode);
+  m.impl("mlstm_decode", &llmctl_hybrid::mlstm_decode);
   m.impl("gla_scan", &llmctl_hybrid::gla_scan);
   m.impl("latent_q_rows", &llmctl_hybrid::latent_q_rows);
   m.impl("latent_out_rows", &llmctl_hybrid::latent_out_rows);

@@ -433,6 +433,29 @@ def gla_chunk_plan(cu_host, device, least: int = 4 * GLA_CHUNK):
             torch.ones(P, dtype=torch.int32, device=device), P)
 
 
+def state_decode_ok(z, S, b, dv: int) -> bool:
+    """Whether a step's rows are one decoded token each that :func:`gla_decode` and :func:`mlstm_decode` take and are faster for: bf16 projections ``z`` on a GPU, heads of
+    at most 128 values in quads and keys of at most 128 channels, or 256 for up to 64 sequences (times in ``csrc/hybrid/state_decode.hip``)."""
+    T = z.shape[0]
+    return (b.Tp == 0 and T == b.state.numel() > 0 and use_native(z) and z.dtype == torch.bfloat16 and z.stride(1) == 1 and dv % 4 == 0 and dv <= 128
+            and S.shape[2] <= (128 if T > 64 else 256) and S.dtype == torch.float32 and S.is_contiguous() and S.data_ptr() % 16 == 0 and not wants_grad(z))
+
+
+def gla_decode(q, k, v, a, w, z_bias, tau: float, qscale: float, S, b, norm, g, eps: float):
+    """:func:`headnorm_gate` (silu) of :func:`gla_scan` with the decay logits ``linear_f32(a, w)``, in one launch, where :func:`state_decode_ok`."""
+    return native_hybrid().gla_decode(q, k, v, a, w, z_bias, tau, qscale, S, b.state, b.start, norm, g, eps)
+
+
+def mlstm_decode(q, k, v, h, w_if, b_i, b_f, cap: float, qscale: float, S, n, m, b, norm, g, eps: float):
+    """:func:`headnorm_gate` of :func:`mlstm_scan` with the gates ``linear_f32w(h, w_if)``, in one launch, where :func:`state_decode_ok`; rows in no quads have the gates'
+    product before it."""
+    raw = None
+    if not (h.dtype == torch.bfloat16 and w_if.is_contiguous() and h.stride(1) == 1 and h.shape[1] % 4 == 0 and h.stride(0) % 4 == 0 and h.data_ptr() % 8 == 0
+            and w_if.data_ptr() % 16 == 0):
+        raw = linear_f32w(h, w_if, few=True)
+    return native_hybrid().mlstm_decode(q, k, v, raw, h, w_if, b_i, b_f, cap, qscale, S, n, m, b.state, b.start, norm, g, eps)
+
+
 def gla_scan(q, k, v, z, z_bias, tau: float, qscale: float, S, state_slots, cu, start, cu_host=None, plan=None):
     """Gated linear attention over the step's tokens: per head a memory ``S [dk, dv]`` with a decay per
     key channel, ``a_t = sigmoid(z_t + z_bias)^(1/tau)`` (computed as ``exp(log_sigmoid / tau)`` in fp32),
