@@ -220,8 +220,8 @@ def rows_form(M: int, N: int, K: int) -> int:
     return 1 if tall <= half else 2
 
 
-def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``x @ w^T (+ b)`` on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
+def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """``x @ w^T (+ b)`` (into ``out`` ``[M, groups, N / groups]``, whose rows and groups may lie apart) on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
     None.  A library product takes the host 24 us, this 9: Lenitar's prompt of 2048 tokens, sixteen of them,
     1198 us, so 1127 (kernels 1190 / 1106); gpt2-125m's of 700 and 300 tokens 2195 / 1870."""
     N, K = w.shape
@@ -236,6 +236,12 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
     if (not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (_small_bias(b, N) and b.data_ptr() & 15 == 0))
             or 512 * x2.stride(0) >= 1 << 30 or 512 * w.stride(0) >= 1 << 30):
         return None
+    if out is not None:
+        if not (type(out) is torch.Tensor and out.dtype is torch.bfloat16 and out.shape[2] & 7 == 0 and out.stride(2) == 1 and out.stride(0) & 7 == 0
+                and out.stride(1) & 7 == 0 and out.data_ptr() & 15 == 0):
+            return None
+        native().gemm_rows_into(x2, w, b, rows_form(M, N, K), out)
+        return out
     y = native().gemm_rows(x2, w, b, rows_form(M, N, K))
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 

@@ -188,10 +188,10 @@ class LatentAttention(nn.Module):
             self._uvt, self._uvt_key = self.w_uv.detach().transpose(1, 2).contiguous(), key
         return self._uvt
 
-    def _attend_expanded(self, q: torch.Tensor, b: StepBatch, lat: torch.Tensor, rows: torch.Tensor) -> torch.Tensor:
+    def _attend_expanded(self, q: torch.Tensor, b: StepBatch, lat: torch.Tensor, rows: torch.Tensor, gate: Optional[torch.Tensor]) -> torch.Tensor:
         """``lat``: the step's cache rows [latent | rotary key]; ``rows [T, H, dv + dn + dr]``, which hold the rotary key already."""
         T, H, dn, dr, dv = q.shape[0], self.H, self.dn, self.dr, self.dv
-        rows[:, :, :dv + dn] = hops.linear(lat[:, :self.rk], self._w_uvk()).view(T, H, dv + dn)  # per head [v | k | shared rotary key]
+        hops.linear_into(lat[:, :self.rk], self._w_uvk(), rows[:, :, :dv + dn])  # per head [v | k | shared rotary key]
         if self.qr:  # (a product of its own)
             qa = hops.rotary_tail_(q, b.pos, self.inv_freq, self.rot_dims, dn, self.interleaved, self.rot_amp)
         else:
@@ -200,7 +200,7 @@ class LatentAttention(nn.Module):
         if "own_rows" not in b.scratch:
             b.scratch["own_rows"] = (b.p_cu[:-1, None] + torch.arange(b.max_q, device=q.device, dtype=torch.int32)[None, :]).clamp_(max=T - 1).contiguous()
         o = hops.latent_attention_prefill(qa, rows.view(T, 1, -1), b.scratch["own_rows"], b.p_cu, b.p_ctx, self.window, self.sink,
-                                          self.scale, dv, b.max_q, groups=H, koff=dv)
+                                          self.scale, dv, b.max_q, groups=H, koff=dv, gate=gate)
         return o.reshape(T, H * dv)
 
     def step(self, h: torch.Tensor, b: StepBatch, cache) -> torch.Tensor:
@@ -224,10 +224,7 @@ class LatentAttention(nn.Module):
                 lat = cache.view(-1, self.rk + self.dr).index_select(0, b.slots)  # the rows just written
                 rows[:, :, dv + dn:] = lat[:, None, self.rk:]
         if rows is not None:
-            o = self._attend_expanded(q, b, lat, rows)
-            if self.has_gate:
-                o = hops.sigmoid_gate_mul(o, z[:, c:])
-            return hops.linear(o, self.w_o)
+            return hops.linear(self._attend_expanded(q, b, lat, rows, z[:, c:] if self.has_gate else None), self.w_o)
         qa = hops.latent_queries(q, self.w_uk, b.pos, self.inv_freq, self.rot_dims, self.interleaved, self.rot_amp)
         outs = []
         if b.Tp:
@@ -554,16 +551,15 @@ class SigmoidAttention(nn.Module):
         q = hops.qk_fullnorm_prep(z, H, G, dk, dv, self.q_norm, self.k_norm, self.eps, b.pos, self.temp_coef,
                                   self.temp_every, rows, b.slots)
         opt = dict(groups=G, koff=dv, sig_bias=self.bias, dist_a=self.dist_a, dist_b=self.dist_b)
-        outs = []
+        outs, gate = [], z[:, self.cols - H:self.cols]
         if b.Tp:
             outs.append(hops.latent_attention_prefill(q[:b.Tp], rows, b.p_bt, b.p_cu, b.p_ctx, self.window, None,
-                                                      self.scale, dv, b.max_q, **opt))
+                                                      self.scale, dv, b.max_q, gate=gate[:b.Tp], **opt))
         if T > b.Tp:
             outs.append(hops.latent_attention_decode(q[b.Tp:], rows, b.d_bt, b.d_ctx, self.window, None, self.scale, dv,
-                                                     max_ctx=b.d_max_ctx, **opt))
+                                                     max_ctx=b.d_max_ctx, gate=gate[b.Tp:], **opt))
         o = outs[0] if len(outs) == 1 else torch.cat(outs)
-        g0 = self.cols - H
-        y = hops.linear(hops.sigmoid_gate_mul(o.reshape(T, H * dv), z[:, g0:self.cols]), self.w_o)
+        y = hops.linear(o.reshape(T, H * dv), self.w_o)
         return (y, z[:, self.cols:]) if self.side else y
 
 

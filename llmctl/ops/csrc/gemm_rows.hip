@@ -1,5 +1,6 @@
 // Products of a prompt's rows, y = act(x w^T (+ bias)) in bf16, on the tiles of wide_tiles.h: any number of rows, outputs in 8s, K in 128s from 256 on.
 //
+// y's columns may lie in groups apart (a latent prompt's keys and values beside a shared rotary key: the copy into place took 9.4 us for 2048 tokens of 16 heads).
 // Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, gemm_rows_form says.
 #include "wide_tiles.h"
 
@@ -15,6 +16,8 @@ struct RowsArgs {
   long lda, ldb;
   int M, N, K;
   int tiles_m, tiles_n;
+  long ldc;
+  int gw, gstep;  // y's columns lie in groups of gw (8s), gstep apart
 };
 constexpr int BAND = 4;  // tile rows that walk the columns together
 
@@ -51,8 +54,11 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
     if constexpr (MB == 4) run_half(t, va, vb, smem, acc);
     else run<MB>(t, va, vb, smem, acc);
     float bias[2][8];
+    int at[2];  // where in a row of y the lane's columns are
 #pragma unroll
     for (int jp = 0; jp < 2; ++jp) {
+      const int c = c0 + 32 * jp, grp = g.gw < g.N ? c / g.gw : 0;
+      at[jp] = c + grp * (g.gstep - g.gw);
 #pragma unroll
       for (int e = 0; e < 8; ++e) bias[jp][e] = 0.f;
       if (g.bias != nullptr && c0 + 32 * jp < g.N) load8(g.bias + c0 + 32 * jp, bias[jp]);
@@ -71,7 +77,7 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += bias[jp][e];
-        if (r < rows && c0 + 32 * jp < g.N) store8(g.c + (long)(row0 + r) * g.N + c0 + 32 * jp, v);
+        if (r < rows && c0 + 32 * jp < g.N) store8(g.c + (long)(row0 + r) * g.ldc + at[jp], v);
       }
     }
   };
@@ -84,10 +90,9 @@ __global__ __launch_bounds__(NT4, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 }
 
 int row_tiles(int64_t M) { return M <= ROWS ? 1 : (int)((M - 33) / 256 + 1); }
-}  // namespace
 
-// y [M, N] = x w^T (+ bias); form: 1 = tiles of 256 rows, 2 = of 128
-at::Tensor gemm_rows(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t form) {
+// y [M, N], or [M, groups, N / groups] whose rows and groups may lie apart; undefined: made here
+void rows_product(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t form, at::Tensor& y) {
   LLMCTL_CHECK(x.dim() == 2 && w.dim() == 2 && x.is_cuda() && w.is_cuda() && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && x.stride(1) == 1 &&
                    w.stride(1) == 1,
                "gemm_rows: bf16 GPU x [M, K] and w [N, K] with unit inner strides");
@@ -101,17 +106,38 @@ at::Tensor gemm_rows(const at::Tensor& x, const at::Tensor& w, const c10::option
                  "gemm_rows: bias bf16 [N], aligned to 16 bytes");
   LLMCTL_CHECK(ROWS * x.stride(0) < (1L << 30) && COLS * w.stride(0) < (1L << 30) && x.stride(0) >= 0 && w.stride(0) >= 0 && M < (1L << 31) && N < (1L << 31),
                "gemm_rows: operand too large for 32-bit offsets");
+  const bool into = y.defined();
+  if (into)
+    LLMCTL_CHECK(y.is_cuda() && y.scalar_type() == at::kBFloat16 && y.dim() == 3 && y.size(0) == M && y.size(1) * y.size(2) == N && y.size(2) % 8 == 0 &&
+                     (y.size(2) <= 1 || y.stride(2) == 1) && y.stride(0) % 8 == 0 && y.stride(1) % 8 == 0 && y.stride(1) >= y.size(2) &&
+                     y.stride(0) >= y.size(1) * y.stride(1) - (y.stride(1) - y.size(2)) && y.size(1) * y.stride(1) < (1L << 31) &&
+                     (reinterpret_cast<uintptr_t>(y.data_ptr()) & 15) == 0,
+                 "gemm_rows: out bf16 [M, groups, N / groups], rows and groups apart, in 8s");
   const c10::DeviceGuard guard(x.device());
-  at::Tensor y = at::empty({M, N}, x.options());
-  if (M == 0 || N == 0) return y;
+  if (!into) y = at::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return;
   RowsArgs g{bf_ptr(x), bf_ptr(w), has_bias ? bf_ptr(*bias) : nullptr, reinterpret_cast<unsigned short*>(y.data_ptr()), (long)x.stride(0), (long)w.stride(0),
-             (int)M, (int)N, (int)K, form == 1 ? row_tiles(M) : (int)((M + 127) / 128), (int)((N + COLS - 1) / COLS)};
+             (int)M, (int)N, (int)K, form == 1 ? row_tiles(M) : (int)((M + 127) / 128), (int)((N + COLS - 1) / COLS), into ? (long)y.stride(0) : (long)N,
+             into ? (int)y.size(2) : (int)N, into ? (int)y.stride(1) : (int)N};
   const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
   if (form == 1) gemm_rows_kernel<false><<<grid, NT4, 0, stream()>>>(g);
   else gemm_rows_kernel<true><<<grid, NT4, 0, stream()>>>(g);
+}
+}  // namespace
+
+// x w^T (+ bias); form: 1 = tiles of 256 rows, 2 = of 128
+at::Tensor gemm_rows(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t form) {
+  at::Tensor y;
+  rows_product(x, w, bias, form, y);
   return y;
 }
+void gemm_rows_into(const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias, int64_t form, at::Tensor out) {
+  rows_product(x, w, bias, form, out);
+}
 
-TORCH_LIBRARY_IMPL(llmctl, CUDA, m) { m.impl("gemm_rows", &gemm_rows); }
+TORCH_LIBRARY_IMPL(llmctl, CUDA, m) {
+  m.impl("gemm_rows", &gemm_rows);
+  m.impl("gemm_rows_into", &gemm_rows_into);
+}
 
 }  // namespace llmctl

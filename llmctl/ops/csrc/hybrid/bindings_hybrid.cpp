@@ -27,12 +27,12 @@ at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, co
                                int64_t max_q, bool mfma, int64_t groups, int64_t koff, int64_t chunk,
                                const c10::optional<at::Tensor>& hscale, const c10::optional<at::Tensor>& ofreq,
                                const c10::optional<at::Tensor>& sig_bias, const c10::optional<at::Tensor>& dist_a,
-                               const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first);
+                               const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first, const c10::optional<at::Tensor>& gate);
 at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx,
                               int64_t window, const c10::optional<at::Tensor>& sink, double scale, int64_t rk, bool mfma, int64_t groups,
                               int64_t koff, int64_t chunk, const c10::optional<at::Tensor>& hscale, const c10::optional<at::Tensor>& ofreq,
                               int64_t max_ctx, const c10::optional<at::Tensor>& sig_bias, const c10::optional<at::Tensor>& dist_a,
-                              const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first);
+                              const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first, const c10::optional<at::Tensor>& gate);
 std::tuple<at::Tensor, at::Tensor> add_rmsnorm2_f32_(at::Tensor x, const c10::optional<at::Tensor>& a, const c10::optional<at::Tensor>& b,
                                                      const at::Tensor& w1, const c10::optional<at::Tensor>& w2, double eps, bool one_plus,
                                                      bool out_bf16);
@@ -167,8 +167,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("latent_prep(Tensor z, int nq, Tensor q_w, Tensor kv_w, int dr, float eps, Tensor pos, Tensor inv_freq, int rot_dims, Tensor(a!) cache, Tensor slots, bool interleaved, float amp, Tensor(b!)? rows, int kcol) -> (Tensor, Tensor)");
   m.def("rotary_tail_(Tensor(a!) q, Tensor pos, Tensor inv_freq, int rot_dims, int dn, bool interleaved, float amp) -> ()");
   m.def("latent_q_assemble(Tensor q_lat, Tensor q, Tensor pos, Tensor inv_freq, int rot_dims, int dn, bool interleaved=False, float amp=1.0) -> Tensor");
-  m.def("latent_attn_prefill(Tensor qa, Tensor cache, Tensor bt, Tensor cu, Tensor ctx, int window, Tensor? sink, float scale, int rk, int max_q, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0) -> Tensor");
-  m.def("latent_attn_decode(Tensor qa, Tensor cache, Tensor bt, Tensor ctx, int window, Tensor? sink, float scale, int rk, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, int max_ctx=0, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0) -> Tensor");
+  m.def("latent_attn_prefill(Tensor qa, Tensor cache, Tensor bt, Tensor cu, Tensor ctx, int window, Tensor? sink, float scale, int rk, int max_q, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0, Tensor? gate=None) -> Tensor");
+  m.def("latent_attn_decode(Tensor qa, Tensor cache, Tensor bt, Tensor ctx, int window, Tensor? sink, float scale, int rk, bool mfma=True, int groups=1, int koff=0, int chunk=1073741824, Tensor? hscale=None, Tensor? ofreq=None, int max_ctx=0, Tensor? sig_bias=None, Tensor? dist_a=None, Tensor? dist_b=None, float softcap=0.0, int keep_first=0, Tensor? gate=None) -> Tensor");
   m.def("add_rmsnorm2_f32_(Tensor(a!) x, Tensor? a, Tensor? b, Tensor w1, Tensor? w2, float eps, bool one_plus, bool out_bf16) -> (Tensor, Tensor)");
   m.def("residual_add_act_(Tensor(a!) x, Tensor a, Tensor? b) -> ()");
   m.def("clamped_glu(Tensor gu, float limit, float alpha) -> Tensor");

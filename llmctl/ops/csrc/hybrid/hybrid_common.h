@@ -169,7 +169,15 @@ struct RowAttnOpts {
   const float* sig_bias = nullptr;    // [H]: no softmax; a visible key weighs sigmoid(score + sig_bias), nothing is normalised
   double softcap = 0.0;               // c > 0: the scaled score becomes c tanh(score / c)
   int64_t keep_first = 0;             // the window does not hide the keys at positions below this
+  const bf16_t* gate = nullptr;       // the output (bf16) times sigmoid(gate): a row's gate_per neighbouring columns share one
+  int64_t gate_st = 0;
+  int gate_per = 1;
 };
+
+// an output as its own rounding to bf16 leaves it, times the sigmoid of a gate; the hardware's exponential and reciprocal are good to an ulp
+__device__ __forceinline__ float gated(float v, float g) {
+  return __bfloat162float(__float2bfloat16(v)) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
+}
 
 // How a launch over decode rows is cut: its workgroups before a row's keys are split, the splits, and the 64-key steps of a row at most
 struct DecodeCut {

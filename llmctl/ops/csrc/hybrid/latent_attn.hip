@@ -405,7 +405,7 @@ void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::T
 bool decode_tiles_pay(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t window, const RowAttnOpts& x, int64_t most);
 void latent_attn_mfma_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
                              double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x);
-void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
+bool row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
                 double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x);
 
 // ------------------------------------------------------------------------------------------ host
@@ -543,6 +543,23 @@ static RowAttnOpts row_opts(const at::Tensor& qa, const at::Tensor& cache, int64
   return x;
 }
 
+at::Tensor sigmoid_gate_mul(const at::Tensor& o, const at::Tensor& g);  // stream.hip
+
+// A gate of the output ([rows, H * rk] or [rows, H]): the matrix-core kernels apply a bf16 one (of a column each: in quads) as they store (true), after the others it is a pass of its own.
+static bool take_gate(RowAttnOpts& x, const c10::optional<at::Tensor>& gate, const at::Tensor& qa, int64_t rk) {
+  if (!gate.has_value()) return false;
+  check_rows(*gate, "gate");
+  const int64_t H = qa.size(1);
+  HYB_CHECK(gate->size(0) == qa.size(0) && (gate->size(1) == H * rk || gate->size(1) == H), "gate: [rows, H * rk] or [rows, H]");
+  if (gate->scalar_type() != at::kBFloat16 || qa.scalar_type() != at::kBFloat16) return false;
+  if (gate->size(1) != H && (rk % 4 != 0 || !quads_ok(reinterpret_cast<const bf16_t*>(gate->data_ptr()), gate->stride(0), 4))) return false;
+  x.gate = reinterpret_cast<const bf16_t*>(gate->data_ptr()), x.gate_st = gate->stride(0), x.gate_per = gate->size(1) == H ? (int)rk : 1;
+  return true;
+}
+static at::Tensor gate_after(const at::Tensor& out, const c10::optional<at::Tensor>& gate) {
+  return gate.has_value() ? sigmoid_gate_mul(out.view({out.size(0), -1}), *gate).view(out.sizes()) : out;
+}
+
 static GenArgs gen_args(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, const float* sink,
                         int64_t window, double scale, int64_t rk, const RowAttnOpts& x) {
   GenArgs g;
@@ -576,7 +593,8 @@ at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, co
                                int64_t max_q, bool mfma, int64_t groups, int64_t koff, int64_t chunk,
                                const c10::optional<at::Tensor>& hscale, const c10::optional<at::Tensor>& ofreq,
                                const c10::optional<at::Tensor>& sig_bias, const c10::optional<at::Tensor>& dist_a,
-                               const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first) {
+                               const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first,
+                               const c10::optional<at::Tensor>& gate) {
   HYB_CHECK(qa.is_cuda() && qa.is_contiguous() && qa.dim() == 3, "qa: contiguous [T, H, R]");
   const int64_t T = qa.size(0), H = qa.size(1), R = qa.size(2);
   check_cache(cache, qa, cache.size(2));
@@ -588,14 +606,15 @@ at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, co
   HYB_CHECK(window >= 1 && max_q >= 1, "window >= 1, max_q >= 1");
   window = std::min<int64_t>(window, (int64_t)1 << 30);
   const float* sink_p;
-  const RowAttnOpts x = row_opts(qa, cache, rk, sink, groups, koff, chunk, hscale, ofreq, 0, &sink_p, sig_bias, dist_a, dist_b, softcap, keep_first);
+  RowAttnOpts x = row_opts(qa, cache, rk, sink, groups, koff, chunk, hscale, ofreq, 0, &sink_p, sig_bias, dist_a, dist_b, softcap, keep_first);
   HYB_CHECK((size_t)R * 64 * sizeof(float) <= 160 * 1024, "key too wide for the query tile in LDS");
+  const bool stored = take_gate(x, gate, qa, rk);
   c10::DeviceGuard guard(qa.device());
   at::Tensor out = at::empty({T, H, rk}, qa.options());
   if (T == 0 || ns == 0) return out;
   if (mfma && mfma_cap_ok(x, R) && (x.dist_a == nullptr || x.sig_bias != nullptr) && latent_attn_mfma_ok(qa, rk, cache.size(2) / groups, koff, x.ofreq != nullptr || x.sig_bias != nullptr)) {
     latent_attn_mfma(qa, cache, bt, cu, ctx, window, sink_p, scale, rk, max_q, out, x);
-    return out;
+    return stored ? out : gate_after(out, gate);
   }
   const int VT = rk <= 32 ? 32 : (rk <= 64 ? 64 : 128);
   const int nvt = (int)((rk + VT - 1) / VT);
@@ -619,14 +638,15 @@ at::Tensor latent_attn_prefill(const at::Tensor& qa, const at::Tensor& cache, co
       else launch(latent_attn_prefill_kernel<Tt, 128, false>);
     }
   });
-  return out;
+  return gate_after(out, gate);
 }
 
 at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx,
                               int64_t window, const c10::optional<at::Tensor>& sink, double scale, int64_t rk, bool mfma, int64_t groups,
                               int64_t koff, int64_t chunk, const c10::optional<at::Tensor>& hscale, const c10::optional<at::Tensor>& ofreq,
                               int64_t max_ctx, const c10::optional<at::Tensor>& sig_bias, const c10::optional<at::Tensor>& dist_a,
-                              const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first) {
+                              const c10::optional<at::Tensor>& dist_b, double softcap, int64_t keep_first,
+                              const c10::optional<at::Tensor>& gate) {
   HYB_CHECK(qa.is_cuda() && qa.is_contiguous() && qa.dim() == 3, "qa: contiguous [n, H, R]");
   const int64_t ns = qa.size(0), H = qa.size(1), R = qa.size(2);
   check_cache(cache, qa, cache.size(2));
@@ -636,14 +656,15 @@ at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, con
   HYB_CHECK(window >= 1, "window >= 1");
   window = std::min<int64_t>(window, (int64_t)1 << 30);
   const float* sink_p;
-  const RowAttnOpts x = row_opts(qa, cache, rk, sink, groups, koff, chunk, hscale, ofreq, max_ctx, &sink_p, sig_bias, dist_a, dist_b, softcap, keep_first);
+  RowAttnOpts x = row_opts(qa, cache, rk, sink, groups, koff, chunk, hscale, ofreq, max_ctx, &sink_p, sig_bias, dist_a, dist_b, softcap, keep_first);
+  bool stored = take_gate(x, gate, qa, rk);
   c10::DeviceGuard guard(qa.device());
   at::Tensor out = at::empty({ns, H, rk}, qa.options());
   if (ns == 0) return out;
   if (mfma && mfma_cap_ok(x, R) && (x.dist_a == nullptr || x.sig_bias != nullptr) && latent_attn_mfma_ok(qa, rk, cache.size(2) / groups, koff, x.ofreq != nullptr || x.sig_bias != nullptr)) {
     if (decode_tiles_pay(ns, H, R, rk, window, x, bt.size(1) * cache.size(1))) latent_attn_mfma_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
-    else row_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
-    return out;
+    else stored &= row_decode(qa, cache, bt, ctx, window, sink_p, scale, rk, out, x);
+    return stored ? out : gate_after(out, gate);
   }
   HYB_CHECK(rk <= 512, "generic decode kernel: value width <= 512");
   const int64_t Rp = R + (R & 1);  // keeps the int64 array 8-byte aligned
@@ -662,7 +683,7 @@ at::Tensor latent_attn_decode(const at::Tensor& qa, const at::Tensor& cache, con
       else launch(latent_attn_decode_kernel<Tt, 8, false>);
     }
   });
-  return out;
+  return gate_after(out, gate);
 }
 
 }  // namespace llmctl_hybrid

@@ -55,6 +55,9 @@ struct LArgs {
   // writes its unnormalised fp32 output and (running maximum, denominator) here, and row_merge joins them
   int xcd;  // prompt forms: the heads (a multiple of eight) are shared out to the XCDs
   int nsplit;
+  const unsigned short* gate;  // nullptr, or RowAttnOpts::gate
+  long gate_st;
+  int gate_per;
   float* ws_o;   // [rows, nsplit, rk]
   float* ws_ml;  // [rows, nsplit, 2]
 };
@@ -368,29 +371,54 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
   } else if (valid) {
     const float inv = 1.f / l_i;
     unsigned short* Op = a.out + ((long)(q_begin + my_tok) * a.H + my_head) * a.rk;
+    // A copy for either, not a branch in each of its stores: a launch without a gate reads no more code than before.  2048 tokens x 16 heads of 128 columns, a gate each:
+    // 49.7 us and a pass of 8.8 for the gate, so 53.5 (with a gate loaded where it is used 59.9).
+    auto store = [&](auto gated_c) __attribute__((always_inline)) {
+      constexpr bool GATED = decltype(gated_c)::value;
+      // a lane's gates lie in its own row, 8 bytes at a time: all on their way before the first is used
+      const bf16_t* Gp = a.gate + (long)(q_begin + my_tok) * a.gate_st;
+      const bool each = a.gate_per == 1;
+      float4 gt[GATED ? NDB : 1][4];
+      if constexpr (GATED) {
+        const float one = each ? 0.f : ldf(Gp + my_head);
 #pragma unroll
-    for (int d = 0; d < NDB; ++d)
+        for (int d = 0; d < NDB; ++d)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int col = v0 + d * 32 + 8 * g + 4 * hh;
-        if (col < a.rk) {
-          if constexpr (ROT) {  // turn the neighbour pairs (col, col + 1), (col + 2, col + 3) back
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-              float sn, cs;
-              sincosf((float)my_pos * a.ofreq[(col + j) >> 1], &sn, &cs);
-              const float u = o[d][4 * g + j], w = o[d][4 * g + j + 1];
-              o[d][4 * g + j] = u * cs + w * sn;
-              o[d][4 * g + j + 1] = w * cs - u * sn;
-            }
+          for (int g = 0; g < 4; ++g) {
+            const int col = v0 + d * 32 + 8 * g + 4 * hh;
+            gt[d][g] = each ? ld4(Gp + (long)my_head * a.rk + min(col, a.rk - 4)) : make_float4(one, one, one, one);
           }
-          unsigned short w4[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w4[j] = __bfloat16_as_ushort(__float2bfloat16(o[d][4 * g + j] * inv));
-          *reinterpret_cast<uint2*>(Op + col) =
-              make_uint2((unsigned)w4[0] | ((unsigned)w4[1] << 16), (unsigned)w4[2] | ((unsigned)w4[3] << 16));
-        }
       }
+#pragma unroll
+      for (int d = 0; d < NDB; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int col = v0 + d * 32 + 8 * g + 4 * hh;
+          if (col < a.rk) {
+            if constexpr (ROT) {  // turn the neighbour pairs (col, col + 1), (col + 2, col + 3) back
+#pragma unroll
+              for (int j = 0; j < 4; j += 2) {
+                float sn, cs;
+                sincosf((float)my_pos * a.ofreq[(col + j) >> 1], &sn, &cs);
+                const float u = o[d][4 * g + j], w = o[d][4 * g + j + 1];
+                o[d][4 * g + j] = u * cs + w * sn;
+                o[d][4 * g + j + 1] = w * cs - u * sn;
+              }
+            }
+            unsigned short w4[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              float v = o[d][4 * g + j] * inv;
+              if constexpr (GATED) v = gated(v, (&gt[d][g].x)[j]);
+              w4[j] = __bfloat16_as_ushort(__float2bfloat16(v));
+            }
+            *reinterpret_cast<uint2*>(Op + col) =
+                make_uint2((unsigned)w4[0] | ((unsigned)w4[1] << 16), (unsigned)w4[2] | ((unsigned)w4[3] << 16));
+          }
+        }
+    };
+    if (a.gate != nullptr) store(std::true_type{});
+    else store(std::false_type{});
   }
 }
 
@@ -461,6 +489,7 @@ LArgs make_args(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor&
   a.scale_log2 = (float)(scale * 1.4426950408889634), a.cap_log2 = (float)(x.softcap * 1.4426950408889634);
   a.cap_inv2 = x.softcap > 0.0 ? (float)(2.0 * 1.4426950408889634 * scale / x.softcap) : 0.f;
   a.nsplit = 1;
+  a.gate = x.gate, a.gate_st = x.gate_st, a.gate_per = x.gate_per;
   return a;
 }
 }  // namespace
@@ -484,7 +513,7 @@ void latent_attn_mfma(const at::Tensor& qa, const at::Tensor& cache, const at::T
   launch_form<false>(a, c.ncb, c.ndb, dim3((unsigned)((max_q + TB - 1) / TB), (unsigned)ns, (unsigned)z), x);
 }
 
-void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const float* ofreq);  // row_decode.hip
+void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const RowAttnOpts& x);  // row_decode.hip
 
 // The decode form's cut: the visible key tiles are split over workgroups until the launch has a few hundred of them.  ``images``: 128-column
 // images of a tile's keys and values in LDS.
@@ -514,7 +543,7 @@ void latent_attn_mfma_decode(const at::Tensor& qa, const at::Tensor& cache, cons
     a.ws_o = ws_o.data_ptr<float>(), a.ws_ml = ws_ml.data_ptr<float>();
   }
   launch_form<true>(a, c.ncb, c.ndb, dim3((unsigned)a.nsplit, (unsigned)ns, (unsigned)z), x);
-  if (a.nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x.ofreq);
+  if (a.nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x);
 }
 
 }  // namespace llmctl_hybrid

@@ -66,6 +66,12 @@ __device__ __forceinline__ void turn_back(float (&v)[4], const float* ofreq, flo
   }
 }
 
+__device__ __forceinline__ void gate4(float (&v)[4], const bf16_t* row, int per, int head, int rk, int c) {
+  const float4 g = per == 1 ? ld4(row + (long)head * rk + c) : make_float4(ldf(row + head), 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = gated(v[j], per == 1 ? (&g.x)[j] : g.x);
+}
+
 __device__ __forceinline__ void store4(unsigned short* p, const float (&v)[4]) {
   unsigned short h[4];
 #pragma unroll
@@ -258,7 +264,8 @@ __global__ __launch_bounds__(WAVES * 64, NK > 18 ? 1 : 2) void row_decode_kernel
 // out[row] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M = max_s m_s (splits that saw nothing: m = -inf, l = 0).  One workgroup
 // per row: the splits' factors once (a lane each), then four columns a thread.
 __global__ __launch_bounds__(128) void row_merge_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, unsigned short* __restrict__ out,
-                                                        int nsplit, int rk, const float* __restrict__ ofreq, const int* __restrict__ ctx, int H) {
+                                                        int nsplit, int rk, const float* __restrict__ ofreq, const int* __restrict__ ctx, int H, const bf16_t* __restrict__ gate,
+                                                        long gate_st, int gate_per) {
   __shared__ float fac[64];
   constexpr int B = 8;  // splits asked for at once, the first of them before their factors are there
   const long row = blockIdx.x;
@@ -290,16 +297,17 @@ __global__ __launch_bounds__(128) void row_merge_kernel(const float* __restrict_
       }
     }
     if (ofreq != nullptr) turn_back(v, ofreq, (float)(ctx[row / H] - 1), c);
+    if (gate != nullptr) gate4(v, gate + row / H * gate_st, gate_per, (int)(row % H), rk, c);
     store4(out + row * rk + c, v);
   }
 }
 }  // namespace
 
 // Joins the splits of decode rows: ws_o [ns H, nsplit, rk], ws_ml [ns H, nsplit, 2] -> out [ns, H, rk]; at most 64 splits
-void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const float* ofreq) {
+void row_merge(const at::Tensor& ws_o, const at::Tensor& ws_ml, at::Tensor& out, const at::Tensor& ctx, const RowAttnOpts& x) {
   row_merge_kernel<<<dim3((unsigned)ws_o.size(0)), 128, 0, cur_stream()>>>(ws_o.data_ptr<float>(), ws_ml.data_ptr<float>(),
-                                                                         reinterpret_cast<unsigned short*>(out.data_ptr()), (int)ws_o.size(1), (int)ws_o.size(2), ofreq,
-                                                                         ctx.data_ptr<int>(), (int)out.size(1));
+                                                                         reinterpret_cast<unsigned short*>(out.data_ptr()), (int)ws_o.size(1), (int)ws_o.size(2), x.ofreq,
+                                                                         ctx.data_ptr<int>(), (int)out.size(1), x.gate, (long)x.gate_st, x.gate_per);
 }
 
 namespace {
@@ -340,8 +348,9 @@ bool decode_tiles_pay(int64_t ns, int64_t H, int64_t R, int64_t rk, int64_t wind
   return row > tile;
 }
 
-// Keys up to 640 wide; keys, values, sub-rows and the key offset in multiples of 8 (latent_attn_mfma_ok).
-void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
+// Keys up to 640 wide; keys, values, sub-rows and the key offset in multiples of 8 (latent_attn_mfma_ok).  True: the gate, if any, is in the output (the merge applies it;
+// rows of one split are left to a pass of its own: the widest form has no registers for it).
+bool row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor& bt, const at::Tensor& ctx, int64_t window, const float* sink,
                 double scale, int64_t rk, at::Tensor& out, const RowAttnOpts& x) {
   const int64_t ns = qa.size(0), H = qa.size(1), R = qa.size(2), G = x.groups, P = H / G, rs = cache.size(2) / G;
   const int htiles = (int)((P + 15) / 16);
@@ -375,7 +384,8 @@ void row_decode(const at::Tensor& qa, const at::Tensor& cache, const at::Tensor&
   else if (nv == 16) go(row_decode_kernel<8, 16>, 16);
   else if (R <= 576) go(row_decode_kernel<18, 32>, 32);
   else go(row_decode_kernel<20, 32>, 32);
-  if (nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x.ofreq);
+  if (nsplit > 1) row_merge(ws_o, ws_ml, out, ctx, x);
+  return nsplit > 1;
 }
 
 }  // namespace llmctl_hybrid

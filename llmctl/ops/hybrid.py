@@ -154,7 +154,7 @@ NO_LIMIT = 1 << 30  # a window or chunk that never masks
 
 def latent_attention_prefill(qa, cache, bt, cu, ctx, window: int, sink, scale: float, rk: int, max_q: int,
                              mfma: bool = True, groups: int = 1, koff: int = 0, chunk: int = NO_LIMIT, hscale=None,
-                             ofreq=None, sig_bias=None, dist_a=None, dist_b=None, softcap: float = 0.0, keep_first: int = 0):
+                             ofreq=None, sig_bias=None, dist_a=None, dist_b=None, softcap: float = 0.0, keep_first: int = 0, gate=None):
     """Prompt portions: sequence n's query rows ``[cu[n], cu[n+1])`` end at position ``ctx[n]-1``;
     ``max_q``: the longest portion (sizes the launch).  bf16 shapes that fit run on the matrix cores
     (``mfma=False`` forces the generic fp32-SIMT kernel, which also serves fp32).
@@ -169,26 +169,29 @@ def latent_attention_prefill(qa, cache, bt, cu, ctx, window: int, sink, scale: f
     ``sig_bias`` (fp32 [H]): the weights are not a softmax; a visible key weighs ``sigmoid(score + sig_bias)``
     and nothing is normalised over the keys (no sink then).  ``softcap`` c > 0: the scaled score becomes
     ``c tanh(score / c)`` before masks and softmax; ``keep_first`` n > 0: the window does not hide the keys at
-    positions below n (nothing is renumbered: such keys are addressed by their own positions)."""
+    positions below n (nothing is renumbered: such keys are addressed by their own positions).  ``gate`` (``[T, H * rk]`` or ``[T, H]``): the output
+    is that of :func:`sigmoid_gate_mul` (in the matrix-core kernels as they store it)."""
     if use_native(qa):
         return native_hybrid().latent_attn_prefill(qa, cache, bt, cu, ctx, window, sink, scale, rk, max_q, mfma, groups,
-                                                   koff, chunk, hscale, ofreq, sig_bias, dist_a, dist_b, softcap, keep_first)
-    return ref.latent_attention(qa, cache, bt, cu, ctx, window, sink, scale, rk, groups, koff, chunk, hscale, ofreq,
-                                sig_bias, dist_a, dist_b, softcap, keep_first)
+                                                   koff, chunk, hscale, ofreq, sig_bias, dist_a, dist_b, softcap, keep_first, gate)
+    o = ref.latent_attention(qa, cache, bt, cu, ctx, window, sink, scale, rk, groups, koff, chunk, hscale, ofreq,
+                             sig_bias, dist_a, dist_b, softcap, keep_first)
+    return o if gate is None else sigmoid_gate_mul(o.flatten(1), gate).view(o.shape)
 
 
 def latent_attention_decode(qa, cache, bt, ctx, window: int, sink, scale: float, rk: int, mfma: bool = True,
                             groups: int = 1, koff: int = 0, chunk: int = NO_LIMIT, hscale=None, ofreq=None,
                             max_ctx: int = 0, sig_bias=None, dist_a=None, dist_b=None, softcap: float = 0.0,
-                            keep_first: int = 0):
+                            keep_first: int = 0, gate=None):
     """One query row per sequence, at position ``ctx[n] - 1`` (options as in the prefill form;
     ``max_ctx``: the longest context if the host knows it, it sizes the split of the keys)."""
     if use_native(qa):
         return native_hybrid().latent_attn_decode(qa, cache, bt, ctx, window, sink, scale, rk, mfma, groups, koff, chunk,
-                                                  hscale, ofreq, max_ctx, sig_bias, dist_a, dist_b, softcap, keep_first)
+                                                  hscale, ofreq, max_ctx, sig_bias, dist_a, dist_b, softcap, keep_first, gate)
     cu = torch.arange(qa.shape[0] + 1, dtype=torch.int32)
-    return ref.latent_attention(qa, cache, bt, cu, ctx, window, sink, scale, rk, groups, koff, chunk, hscale, ofreq,
-                                sig_bias, dist_a, dist_b, softcap, keep_first)
+    o = ref.latent_attention(qa, cache, bt, cu, ctx, window, sink, scale, rk, groups, koff, chunk, hscale, ofreq,
+                             sig_bias, dist_a, dist_b, softcap, keep_first)
+    return o if gate is None else sigmoid_gate_mul(o.flatten(1), gate).view(o.shape)
 
 
 def add_rmsnorm2_f32_(x, a, b, w1, w2, eps: float, one_plus: bool, out_dtype):
@@ -551,6 +554,15 @@ def linear(x, w, b=None):
     """``x @ w^T (+ b)``: steps of a few rows stream the weight (:func:`rows_linear`), prompts run on the tiles of ``csrc/gemm_rows.hip`` where these are faster than the
     library's product (:func:`llmctl.exec.linear.rows_form`)."""
     return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else _library_linear(x, w, b, torch.nn.functional.linear)
+
+
+def linear_into(x, w, out) -> None:
+    """``out [T, groups, n] = x @ w^T``, a view whose rows and groups may lie apart."""
+    global _prompt_linear
+    if _prompt_linear is None:
+        from llmctl.exec.linear import rows_linear as _prompt_linear
+    if x.shape[0] <= 32 or _prompt_linear(x, w, None, out) is None:
+        out.copy_(linear(x, w).view(out.shape))
 
 
 def odd_linear(x, w, b=None):

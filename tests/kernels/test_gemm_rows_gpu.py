@@ -48,3 +48,27 @@ def test_route():
     y = L.linear(xg, p, b)
     y.sum().backward()
     assert float((y.double() - ref).norm() / ref.norm()) < 2.0**-9 and xg.grad is not None and p.grad is not None
+
+
+@pytest.mark.parametrize("M,K", [(33, 256), (129, 384), (545, 640)])
+@pytest.mark.parametrize("groups,n,gap", [(1, 264, 8), (3, 88, 16), (33, 8, 8), (16, 256, 64)])
+@pytest.mark.parametrize("form", [1, 2])
+def test_into_groups_that_lie_apart(M, K, groups, n, gap, form):
+    from llmctl.ops._lib import native
+
+    g = torch.Generator(device="cuda").manual_seed(M + groups)
+    x, w = (torch.randn(r, K, generator=g, device="cuda").bfloat16() for r in (M, groups * n))
+    y = torch.full((M + 1, groups, n + gap), 7.0, device="cuda", dtype=torch.bfloat16)
+    native().gemm_rows_into(x, w, None, form, y[:M, :, :n])
+    assert torch.equal(y[:M, :, :n].reshape(M, -1), native().gemm_rows(x, w, None, form))
+    assert bool((y[:, :, n:] == 7).all()) and bool((y[M] == 7).all())
+
+
+def test_linear_into_takes_any_rows():
+    from llmctl.ops import hybrid as hops
+
+    for T, dtype in ((1, torch.bfloat16), (20, torch.bfloat16), (300, torch.bfloat16), (40, torch.float32)):
+        x, w = torch.randn(T, 512, device="cuda", dtype=dtype), torch.randn(4 * 64, 512, device="cuda", dtype=dtype)
+        y = torch.zeros(T, 4, 72, device="cuda", dtype=dtype)
+        hops.linear_into(x, w, y[:, :, :64])
+        assert torch.equal(y[:, :, :64].reshape(T, 256), hops.linear(x, w)) and not y[:, :, 64:].any()
