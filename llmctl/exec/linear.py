@@ -98,7 +98,7 @@ def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] =
     if M > 32 or layout != "eager":
         y = small_linear(x, w, b, layout)
         if y is None:
-            y = rows_linear(x, w, b)
+            y = rows_linear(x, w, b, None, 0, layout == "eager")
         if y is not None:
             return y
     if M and fwd64_pick(M, N, K) and x.dtype == torch.bfloat16:
@@ -201,33 +201,73 @@ def _rounds_us(items: int, ktiles: float, empty: float, full: float, fixed: floa
     return whole * (ktiles * (empty + full) + fixed) + (ktiles * (empty + full * rest / _CUS) + fixed if rest else 0.0)
 
 
+def _tile_rows(M: int, form: int) -> int:
+    return -(-M // 128) if form == 2 else 1 if M <= 288 else (M - 33) // 256 + 1
+
+
 @functools.lru_cache(maxsize=8192)
-def rows_form(M: int, N: int, K: int) -> int:
-    """The tiles of ``gemm_rows`` (csrc/gemm_rows.hip: 1 = 256 rows, 2 = 128) that multiply M rows of width K to N outputs faster than the library, or 0.  Times by a
-    model of either's workgroups and of the library's products, us: 12 and 1300 TFLOP/s, small ones 6 and 550; constants fitted to 245 sizes, 33 to 4096 rows, 256 to
-    12288 outputs, K 256 to 8192, operands from HBM (``profiles/prompt_products.txt``).  The rule takes 81 of them, in 20 % less time; one of these takes 4 % more.
+def rows_form(M: int, N: int, K: int, act: bool = False, eager: bool = False) -> int:
+    """How ``gemm_rows`` (csrc/gemm_rows.hip) multiplies M rows of width K to N outputs where that is faster than the library: tiles (1 = 256 rows, 2 = 128) + 4 (ranges of K - 1);
+    else 0.  ``act``: an activation follows, which costs the library's product a pass; ``eager``: launches that the host feeds one by one.
+    From 1024 rows on, one range of K: a model of either's workgroups and of the library's products, us: 12 and 1300 TFLOP/s, small ones 6 and 550; constants fitted to 245 sizes, 33
+    to 4096 rows, 256 to 12288 outputs, K 256 to 8192, operands from HBM (``profiles/prompt_products.txt``).  The rule takes 81 of them, in 20 % less time; one of these takes 4 % more.
     us, library / here: 2048 x 2048 x 2048 25.8 / 17.8, 2048 x 3712 x 2048 35.5 / 29.0, 2911 x 2048 x 1024 23.2 / 16.8, 1128 x 3584 x 1664 21.4 / 15.5, 769 x 2816 x 256
-    9.4 / 6.4; left to the library: 1.1 rounds, 2911 x 3072 x 2048 36.8 / 46.0; few tiles and a long K, 551 x 1472 x 1024
-    9.2 / 9.6, 93 x 256 x 4608 12.8 / 24.6; large products, 3379 x 8192 x 2048 94 / 109."""
+    9.4 / 6.4; left to the library: 1.1 rounds, 2911 x 3072 x 2048 36.8 / 46.0; large products, 3379 x 8192 x 2048 94 / 109.
+    Up to 1024 rows: :func:`_few_rows_form`."""
     if M <= 32 or N <= 0 or N & 7 or K & 127 or K < 256:
         return 0
+    code = _few_rows_form(M, N, K, act, eager) if M <= 1024 else 0
+    if code:
+        return code
     cols, kt = -(-N // 128), K / 64
-    tall = _rounds_us((1 if M <= 288 else (M - 33) // 256 + 1) * cols, kt, 0.47, 0.36, 5.0)
-    half = _rounds_us(-(-M // 128) * cols, kt, 0.28, 0.18, 4.0)
+    tall = _rounds_us(_tile_rows(M, 1) * cols, kt, 0.47, 0.36, 5.0 + act * _ACT_TILE[1])
+    half = _rounds_us(_tile_rows(M, 2) * cols, kt, 0.28, 0.18, 4.0 + act * _ACT_TILE[2])
     gflop = 2e-9 * M * N * K
-    if min(tall, half) >= (0.95 if K <= 2304 else 0.85) * min(12.0 + gflop / 1.3, 6.0 + gflop / 0.55):  # (GPT-7B's, 900 x 4096 x 4096, 39 / 34, took its prompt 1 % longer)
+    if min(tall, half) >= (0.95 if K <= 2304 else 0.85) * min(12.0 + gflop / 1.3, 6.0 + gflop / 0.55) + act * _act_us(M, N):  # (GPT-7B's, 900 x 4096 x 4096, 39 / 34, took its prompt 1 % longer)
         return 0
     return 1 if tall <= half else 2
 
 
-def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-    """``x @ w^T (+ b)`` (into ``out`` ``[M, groups, N / groups]``, whose rows and groups may lie apart) on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
-    None.  A library product takes the host 24 us, this 9: Lenitar's prompt of 2048 tokens, sixteen of them,
+_ACT_TILE = {1: 4.7, 2: 2.4}  # GELUs of a tile in its epilogue, us: nothing else runs on its CU meanwhile
+
+
+def _act_us(M: int, N: int) -> float:
+    return 3.0 + 1e-6 * M * N  # an activation pass of its own, us
+
+
+def _few_rows_form(M: int, N: int, K: int, act: bool, eager: bool) -> int:
+    """:func:`rows_form` of a short prompt.  Its tiles are few, so K is cut into ranges of 256 at least; and an eager step is the host's: a library product takes the host 24 us, this 9 (13
+    with the pass that adds the ranges), so a product of at most 22 us
+    and 4 Mi outputs may take a few us longer there.  Both models fitted to 280 sizes, 40 to 2000 rows
+    (``profiles/short_prompt_products.txt``).
+    us, library / here: 128 x 4096 x 11008 79 / 46, 200 59 / 52, 64 x 2048 x 8192 26 / 19, 600 49 / 38, 256 x 8256 x 2048 31 / 26; for the host's sake 256 x 2048 x 2048 11.3 / 15.0, 128 x 2048 x
+    4096 12.8 / 17.2; left to the library 128 x 12288 x 4096 45 / 53, 450 x 22016 x 4096 98 / 129.  Prompts, us a step: dumazen width 2048 100 tokens 1387, so 1101, 450 1331 / 1211;
+    lenitar 300 982 / 843; malinex 200 948 / 807; GPT-7B layers 200 923 / 883; with the GELU in it gpt2-125m 600 1844 / 1548."""
+    cols, stream = -(-N // 128), 4.0 + N * K * 2e-6 / 2.2
+    best, code = 1e9, 0
+    for splits in (1, 2, 3, 4, 6, 8, 12, 16):
+        if splits > 1 and (splits > K // 256 or splits * cols * _tile_rows(M, 1) > 512):
+            break
+        kt, add = K / 64 / splits, 0.0 if splits == 1 else 4.1 + splits * M * N * 4e-6 / 2.36
+        for form, (empty, full, fixed) in ((1, (0.73, 0.38, 2.5)), (2, (0.52, 0.20, 1.7))):
+            t = _rounds_us(splits * cols * _tile_rows(M, form), kt, empty, full, fixed + (act * _ACT_TILE[form] if splits == 1 else 0.0)) + add
+            if t < best:
+                best, code = t, form + 4 * (splits - 1)
+    best, gflop, mb = max(best, stream), 2e-9 * M * N * K, N * K * 2e-6
+    library = (6.1 + 0.237 * mb + 0.8 * gflop + 0.585 * gflop ** 0.5 + 0.545 * mb ** 0.5) * (1.25 if K >= 8192 else 1.0) + act * _act_us(M, N)
+    return code if best < (0.92 if mb <= 64 or K >= 8192 else 0.8) * library or (eager and M * N <= 4 << 20 and best <= min(library + 7.0, 22.0)) else 0
+
+
+def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, act: int = 0,
+                eager: bool = True) -> Optional[torch.Tensor]:
+    """``act(x @ w^T (+ b))`` (into ``out`` ``[M, groups, N / groups]``, whose rows and groups may lie apart) on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
+    None.  ``act``: 0 none, 1 erf GELU, 2 tanh GELU (without ``out``).  A library product takes the host 24 us, this 9: Lenitar's prompt of 2048 tokens, sixteen of them,
     1198 us, so 1127 (kernels 1190 / 1106); gpt2-125m's of 700 and 300 tokens 2195 / 1870."""
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    if not M or type(M * N) is not int or not rows_form(M, N, K) or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
-        return None  # (symbolic and traced sizes are no ints)
+    code = rows_form(M, N, K, act != 0, eager) if M and type(M * N) is int else 0  # (symbolic and traced sizes are no ints)
+    if not code or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
+        return None
     if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not (x.dim() == 2 or x.is_contiguous()) or _any_autocast()
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
             or _forward_ad._current_level >= 0 or torch.compiler.is_compiling()):
@@ -236,13 +276,17 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
     if (not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (_small_bias(b, N) and b.data_ptr() & 15 == 0))
             or 512 * x2.stride(0) >= 1 << 30 or 512 * w.stride(0) >= 1 << 30):
         return None
+    if eager and M <= 1024 and torch.cuda.is_current_stream_capturing():
+        code = rows_form(M, N, K, act != 0)
+        if not code:
+            return None
     if out is not None:
         if not (type(out) is torch.Tensor and out.dtype is torch.bfloat16 and out.shape[2] & 7 == 0 and out.stride(2) == 1 and out.stride(0) & 7 == 0
                 and out.stride(1) & 7 == 0 and out.data_ptr() & 15 == 0):
             return None
-        native().gemm_rows_into(x2, w, b, rows_form(M, N, K), out)
+        native().gemm_rows_into(x2, w, b, code & 3, out, (code >> 2) + 1)
         return out
-    y = native().gemm_rows(x2, w, b, rows_form(M, N, K))
+    y = native().gemm_rows(x2, w, b, code & 3, (code >> 2) + 1, act)
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 

@@ -582,6 +582,8 @@ class DenseFF(nn.Module):
         if hops.rows_ok(h, self.w_up, self.b_up):  # the activation in the product's epilogue
             z = hops.rows_linear(h, self.w_up, self.b_up, self.act, self.ff)
             a = z[:, :self.ff]
+        elif self.act == "gelu" and not self.side:
+            a = hops.linear_gelu(h, self.w_up, self.b_up)
         else:
             z = hops.linear(h, self.w_up, self.b_up)
             a = hops.act_any(z[:, :self.ff], self.act)

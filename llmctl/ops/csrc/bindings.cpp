@@ -104,8 +104,8 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("gemm_tall(Tensor a, Tensor b, Tensor(a!) out, bool at, bool accumulate, int splits, Tensor(b!)? bias=None, bool bias_add=False) -> ()");
   m.def("gemm_small(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, Tensor? bias=None, Tensor(b!)? sums=None, bool add_sums=False, int act=0) -> ()");
   m.def("gemm_small_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, Tensor(c!)? sums=None, bool add_sums=False) -> ()");
-  m.def("gemm_rows(Tensor x, Tensor w, Tensor? bias, int form) -> Tensor");
-  m.def("gemm_rows_into(Tensor x, Tensor w, Tensor? bias, int form, Tensor(a!) out) -> ()");
+  m.def("gemm_rows(Tensor x, Tensor w, Tensor? bias, int form, int splits=1, int act=0) -> Tensor");
+  m.def("gemm_rows_into(Tensor x, Tensor w, Tensor? bias, int form, Tensor(a!) out, int splits=1) -> ()");
   m.def("gemm_tall_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, int splits, Tensor(c!)? db=None, bool add=False) -> ()");
   m.def("gemm64_wgrad_bias(Tensor dy, Tensor x, Tensor(a!) g, bool accumulate, Tensor(b!)? db, bool add) -> bool");
   m.def("embed_grad_(Tensor ids, Tensor dy, Tensor(a!) g, bool add) -> ()");

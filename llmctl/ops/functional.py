@@ -640,7 +640,7 @@ def decode_linear(x, w, b=None, act: Optional[str] = None):
     (``decode_form``): a stream of the weight with bias and activation in the same launch (``csrc/stream_linear.h``),
     ``csrc/skinny_gemm.hip``, or the library.  A tuned configuration or knob ``skinny_gemm`` = ``all`` picks
     ``csrc/skinny_gemm.hip``, ``off`` the library.  Other inputs: the library and an activation pass."""
-    from llmctl.exec.linear import forward_linear, small_linear
+    from llmctl.exec.linear import forward_linear, rows_linear, small_linear
 
     mode = knobs().skinny_gemm
     (M, K), N = x.shape if x.dim() == 2 else (0, 0), w.shape[0]
@@ -665,6 +665,8 @@ def decode_linear(x, w, b=None, act: Optional[str] = None):
         return native().stream_linear(x, w, b, _ROW_ACTS[act])
     if y is None and act == "gelu" and M > 32:
         y = small_linear(x, w, b, "eager", _ROW_ACTS[act])
+        if y is None:
+            y = rows_linear(x, w, b, None, _ROW_ACTS[act])
         if y is not None:
             return y
     if y is None:

@@ -556,6 +556,17 @@ def linear(x, w, b=None):
     return rows_linear(x, w, b) if x.shape[0] <= 32 and rows_ok(x, w, b) else _library_linear(x, w, b, torch.nn.functional.linear)
 
 
+def linear_gelu(x, w, b=None):
+    """The erf GELU of :func:`linear`: in the product's epilogue where the tiles take it."""
+    y = None
+    if x.shape[0] > 32:
+        global _prompt_linear
+        if _prompt_linear is None:
+            from llmctl.exec.linear import rows_linear as _prompt_linear
+        y = _prompt_linear(x, w, b, None, 1)
+    return act_any(linear(x, w, b), "gelu") if y is None else y
+
+
 def linear_into(x, w, out) -> None:
     """``out [T, groups, n] = x @ w^T``, a view whose rows and groups may lie apart."""
     global _prompt_linear

@@ -25,13 +25,41 @@ def test_products(M, N, K, pad, form):
     assert bool(((got.double() - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
 
 
+@pytest.mark.parametrize("M", [1, 33, 128, 129, 288, 289, 700])
+@pytest.mark.parametrize("N,K,splits", [(8, 512, 2), (264, 896, 3), (1000, 2048, 8), (136, 4224, 16)])
+@pytest.mark.parametrize("form,act", [(1, 0), (2, 0), (1, 1), (2, 2)])
+def test_ranges_of_k_and_activations(M, N, K, splits, form, act):
+    """Ranges of 256 on, of unlike length too; erf and tanh GELU of the sum, in the tiles' epilogue and in the pass that adds the ranges."""
+    from llmctl.ops._lib import native
+
+    g = torch.Generator(device="cuda").manual_seed(M + 3 * N + 7 * K)
+    x, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+    b = torch.randn(N, generator=g, device="cuda").bfloat16()
+    X = x.double()
+    w = (w.float() * 2.0 ** -round(K.bit_length() / 2)).bfloat16()  # (an exact scale: sums near 1, where the GELUs bend)
+    W = w.double()
+    ref, mag = X @ W.t() + b.double(), X.abs() @ W.abs().t() + b.double().abs()
+    bound = (K + splits + 1) * 2.0**-24 * mag  # fp32 sums of exact products
+    if act:
+        # both GELUs' slopes stay below 1.13; 3e-7 |sum| for the fp32 forms (erf: 2.3e-7)
+        bound = 1.13 * bound + 2.0**-20 * ref.abs()
+        ref = torch.nn.functional.gelu(ref, approximate="tanh" if act == 2 else "none")
+    for n in (1, splits):
+        got = native().gemm_rows(x, w, b, form, n, act)
+        assert bool(((got.double() - ref).abs() <= bound + 2.0**-8 * (ref.abs() + bound)).all())
+    y = torch.full((M + 1, N // 8, 16), 7.0, device="cuda", dtype=torch.bfloat16)
+    native().gemm_rows_into(x, w, b, form, y[:M, :, :8], splits)
+    assert torch.equal(y[:M, :, :8].reshape(M, N), native().gemm_rows(x, w, b, form, splits)) and bool((y[:, :, 8:] == 7).all()) and bool((y[M] == 7).all())
+
+
 def test_route():
     """Sizes of the rule run on these tiles, inside autograd too; other callers keep the library: a wanted gradient outside of it, autocast, batched rows of a transform."""
     import importlib
 
     L = importlib.import_module("llmctl.exec.linear")
     assert L.rows_form(2048, 2048, 2048) == 2 and L.rows_form(2911, 2048, 1024) == 1
-    assert not any(L.rows_form(*s) for s in ((32, 2048, 2048), (2048, 2044, 2048), (2048, 2048, 2000), (2048, 2048, 128), (93, 256, 4608), (3379, 8192, 2048), (0, 256, 256)))
+    assert not any(L.rows_form(*s) for s in ((32, 2048, 2048), (2048, 2044, 2048), (2048, 2048, 2000), (2048, 2048, 128), (3379, 8192, 2048), (900, 12288, 4096), (0, 256, 256)))
+    assert L.rows_form(128, 4096, 11008) >> 2 and L.rows_form(200, 2048, 2048, False, True) >> 2 and not L.rows_form(200, 2048, 2048)  # (the host's gain alone)
     x, w = (torch.randn(n, 1024, device="cuda", dtype=torch.bfloat16) for n in (1500, 2048))
     b = torch.randn(2048, device="cuda", dtype=torch.bfloat16)
     ref = x.double() @ w.double().t() + b.double()
