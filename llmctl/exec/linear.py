@@ -290,6 +290,32 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
+@functools.lru_cache(maxsize=1024)
+def _prompt_form(M: int, N: int, K: int, act: bool) -> Optional[int]:
+    """The route of an eager prompt's product through ``ops.functional.decode_linear`` as csrc/dense_prompt.cpp names it; None: another one."""
+    if N & 7 or K & 7:
+        return None
+    if small_pays("eager", M, N, K):
+        return -1
+    code = rows_form(M, N, K, act, True)
+    if not code and act:
+        code = rows_form(M, N, K, False, True)
+        code = code and code + (1 << 20)
+    return None if not code and fwd64_pick(M, N, K) else code
+
+
+def prompt_forms(x: torch.Tensor, sizes) -> Optional[List[int]]:
+    """The routes of the products ``(N, K, activation)`` of one eager prompt's rows ``x [M, .]``, where nothing that those routes look at asks for others; else None."""
+    M, kn = x.shape[0], knobs()
+    if (type(x) is not torch.Tensor or M <= 32 or type(M) is not int or not x.is_cuda or x.dtype is not torch.bfloat16 or _calls_are_seen() or _any_autocast()
+            or _is_legacy_batched(x) or _is_wrapped(x) or torch.is_grad_enabled() or _forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+            or kn.fwd64 != "auto" or kn.skinny_gemm != "auto" or not _gemm64_enabled() or GEMM64_CONFIGS or GEMM64_SHAPE_CONFIGS or not use_native(x)
+            or torch.cuda.is_current_stream_capturing()):
+        return None
+    forms = [_prompt_form(M, *s) for s in sizes]
+    return None if None in forms else forms
+
+
 def small_dgrad(dy2: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """``dy2 @ w`` on ``gemm_small`` (into ``out``) where it takes it; else None.  Weights whose sink was made to keep W^T copies stay with them."""
     if _calls_are_seen():

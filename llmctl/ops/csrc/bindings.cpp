@@ -104,6 +104,7 @@ TORCH_LIBRARY(llmctl, m) {
   m.def("gemm_tall(Tensor a, Tensor b, Tensor(a!) out, bool at, bool accumulate, int splits, Tensor(b!)? bias=None, bool bias_add=False) -> ()");
   m.def("gemm_small(Tensor a, Tensor b, Tensor(a!) out, bool at, bool bt, bool accumulate, Tensor? bias=None, Tensor(b!)? sums=None, bool add_sums=False, int act=0) -> ()");
   m.def("gemm_small_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, Tensor(c!)? sums=None, bool add_sums=False) -> ()");
+  m.def("dense_prompt_layers(Tensor x, Tensor[] params, int[] forms, int nq, int nkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor slots, Tensor? doc, float eps) -> Tensor[]");
   m.def("gemm_rows(Tensor x, Tensor w, Tensor? bias, int form, int splits=1, int act=0) -> Tensor");
   m.def("gemm_rows_into(Tensor x, Tensor w, Tensor? bias, int form, Tensor(a!) out, int splits=1) -> ()");
   m.def("gemm_tall_back(Tensor dy, Tensor w, Tensor(a!) dx, Tensor x, Tensor(b!) g, bool accumulate, int splits, Tensor(c!)? db=None, bool add=False) -> ()");

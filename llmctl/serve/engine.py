@@ -35,7 +35,10 @@ import torch.nn.functional as F
 from llmctl import ops
 from llmctl.config.knobs import use as use_knobs
 from llmctl.io.artifact import load_model
+from llmctl.exec.linear import prompt_forms
 from llmctl.models import DecoderLM
+from llmctl.models.transformer import DecoderLayer
+from llmctl.ops._lib import native
 from llmctl.utils.env import graph_capture_gc_guard
 
 from .block_manager import PagedKVCache, make_kv_manager
@@ -45,6 +48,10 @@ from .scheduler import ContinuousBatchScheduler, PrefillChunk, SamplingParams, S
 from .tokenizer import load_tokenizer
 
 log = logging.getLogger("llmctl.serve")
+
+# csrc/dense_prompt.cpp's order; and what its call stands for, unless an engine has its own
+_LAYER_PARAMS = ("attn_norm_w", "attn_norm_b", "wqkv", "bqkv", "wo", "bo", "mlp_norm_w", "mlp_norm_b", "w_up", "b_up", "w_down", "b_down")
+_LOOP = frozenset(("_norm", "_qkv", "_row_linear", "_mlp", "_reduce"))
 
 
 class InferenceEngine:
@@ -556,7 +563,10 @@ class InferenceEngine:
             return self._gather_vocab(ops.decode_linear(xn, self.model.head_weight()))
         res = None
         kc, vc = self.kv_cache.k, self.kv_cache.v
-        for li, layer in enumerate(self.model.layers):
+        done = self._prompt_layers(x, slots, doc) if fa else ()
+        if done:
+            x, res = done
+        for li, layer in enumerate(() if done else self.model.layers):
             xn, res = self._norm(layer, x, res, "attn")
             q, k, v = self._qkv(layer, xn, pos, self.max_model_len, kc[li], vc[li], slots)
             if fa:
@@ -572,6 +582,25 @@ class InferenceEngine:
         if not plan["last"]:
             return torch.empty(0, self.cfg.vocab_size, device=d, dtype=x.dtype)
         return self._final(x.index_select(0, last), res.index_select(0, last))
+
+    def _prompt_layers(self, x, slots, doc):
+        """The layers of fresh prompts from one native call (csrc/dense_prompt.cpp), for models with LayerNorms, biases and an ungated GELU: the launches of the loop
+        in ``prefill_exec``, fed faster.  Returns (the last layer's output, the residual stream), or () where the loop has to run."""
+        cfg = self.cfg
+        if (type(self) is not InferenceEngine or self.tp != 1 or cfg.norm != "layernorm" or cfg.gated_mlp or cfg.is_moe or self.rope is not None or ops.functional.SKINNY_CONFIGS
+                or not _LOOP.isdisjoint(self.__dict__)):
+            return ()
+        layers = self.model.layers
+        params = [layer._parameters.get(n) for layer in layers for n in _LAYER_PARAMS]
+        if any(type(t) is not torch.nn.Parameter for t in params) or any(type(layer) is not DecoderLayer for layer in layers):
+            return ()
+        wqkv, wo, w_up, w_down = (params[i].shape for i in (2, 4, 8, 10))
+        if not len(wqkv) == len(wo) == len(w_up) == len(w_down) == 2:
+            return ()
+        forms = prompt_forms(x, ((*wqkv, False), (*wo, False), (*w_up, True), (*w_down, False)))
+        if forms is None:
+            return ()
+        return native().dense_prompt_layers(x, params, forms, layers[0].nq, layers[0].nkv, self.kv_cache.k, self.kv_cache.v, slots, doc, cfg.layer_norm_eps)
 
     # ------------------------------------------------------------------ mixed prefill + decode
     def mixed_plan(self, chunks: List[PrefillChunk], seqs: List[Sequence]) -> Dict:
