@@ -484,7 +484,7 @@ class GatedLinearAttention(nn.Module):
         if isinstance(state, tuple) and len(state) == 2 and isinstance(state[1], tuple):  # (rows, states)
             state = state[1]
         T, H, dk, dv = h.shape[0], self.H, self.dk, self.dv
-        z = hops.linear(h, self.w_in, self.b_in)
+        z = hops.odd_linear(h, self.w_in, self.b_in)
         a, c, e = H * dk, 2 * H * dk, 2 * H * dk + H * dv
         q, k = z[:, :a].unflatten(1, (H, dk)), z[:, a:c].unflatten(1, (H, dk))
         v = z[:, c:e].unflatten(1, (H, dv))
@@ -547,7 +547,7 @@ class SigmoidAttention(nn.Module):
     def step(self, h: torch.Tensor, b: StepBatch, cache):
         rows = cache[0] if isinstance(cache, tuple) else cache
         T, H, G, dk, dv = h.shape[0], self.H, self.G, self.dk, self.dv
-        z = hops.linear(h, self.w_in, self.b_in)
+        z = hops.odd_linear(h, self.w_in, self.b_in)
         q = hops.qk_fullnorm_prep(z, H, G, dk, dv, self.q_norm, self.k_norm, self.eps, b.pos, self.temp_coef,
                                   self.temp_every, rows, b.slots)
         opt = dict(groups=G, koff=dv, sig_bias=self.bias, dist_a=self.dist_a, dist_b=self.dist_b)
