@@ -70,8 +70,16 @@ struct LArgs {
 // Keys and values up to 128 wide: two workgroups per CU (64.5 KB of images each; held to 256 registers, one's softmax runs beside the
 // other's products).  16 heads over 4 kv groups, portions of 2048 and 1331 tokens: 156 us at one per CU (200 + 96 registers),
 // 100 so.  Wider keys stay at one: 192-wide keys took 108 us against 99, with one set of images instead of two 107.
+// Prompts with keys of 129 to 256 columns: one workgroup's images fill a CU, so it has eight waves there, two on the same 32 query rows: the first takes the first 32 keys of
+// every tile, the other the rest, each with a maximum, denominator and output of its own, which meet in LDS at the end: one's
+// softmax runs beside the other's products.  2048 tokens x 16 heads, keys of 192, window 1024: 52.5 us, so 43.4.  (Wider keys or values have no registers for it; of keys up to 128
+// two workgroups of four waves share a CU.)
+constexpr bool two_key_groups(int nks, int ndb, bool split) { return !split && nks > 8 && nks <= 16 && ndb <= 4; }
+
 template <int NKS, int NDB, bool ROT, bool SIG = false, bool CAP = false, bool SPLIT = false>
-__global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
+__global__ __launch_bounds__(two_key_groups(NKS, NDB, SPLIT) ? 512 : 256, (NKS <= 8 && NDB <= 4) || two_key_groups(NKS, NDB, SPLIT) ? 2 : 1) void latent_attn_mfma_kernel(LArgs a) {
+  constexpr bool KG2 = two_key_groups(NKS, NDB, SPLIT);
+  constexpr int KBN = KG2 ? 1 : 2, NW = KG2 ? 8 : 4;  // blocks of 32 keys that a wave takes of a tile; waves
   constexpr int NCB = (NKS + 7) / 8;
   constexpr int NTB = (NDB + 3) / 4;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -81,7 +89,8 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
   constexpr bool DB = 2 * BUFB + 1024 <= 160 * 1024;
 
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = KG2 ? (tid >> 6) & 3 : tid >> 6;
+  const int kgrp = KG2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
   const int r = lane & 31, hh = lane >> 5;
   // workgroups go round the XCDs in order; the blocks of a head, and the heads of a kv group, read the same keys, so they are dealt to one XCD and its L2
   unsigned bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
@@ -126,7 +135,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
   float m_i = -INFINITY, l_i = 0.f;
-  if (a.sink != nullptr && split == 0) {  // the sink: one unit of mass at its own logit, counted by the first split
+  if (a.sink != nullptr && split == 0 && kgrp == 0) {  // the sink: one unit of mass at its own logit, counted by the first split
     m_i = a.sink[headc] * kLog2e;
     l_i = 1.0f;
   }
@@ -134,7 +143,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
   float pen_a = 0.f, pen_b = 0.f, sig_b2 = 0.f;
   if constexpr (SIG) {
     m_i = 0.f;
-    l_i = split == 0 ? 1.f : 0.f;
+    l_i = split == 0 && kgrp == 0 ? 1.f : 0.f;
     if (a.dist_a != nullptr) pen_a = a.dist_a[headc], pen_b = a.dist_b[headc];
     sig_b2 = a.sig_bias[headc] * kLog2e;
   }
@@ -169,7 +178,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
   // K fragment of k-step ks, rows kb * 32 + r: chunk (2 ks + hh) ^ (r & 15) = (2 ks) ^ (hh ^ (r & 15))
   const int k_row = r * LROWB, k_x = (hh ^ (r & 15)) << 4;
 
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned lds_base = lds_addr(smem);
   // cache slots of a tile's 64 keys, looked up in the block table one tile ahead (double-buffered)
   int* slot_lds = reinterpret_cast<int*>(smem + (DB ? 2 : 1) * BUFB);
@@ -183,7 +192,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
   // to LDS (no registers, all pieces of the tile in flight at once); the images' swizzles are applied
   // to the source chunk.  Keys past the context and columns past the row read a valid neighbour instead
   // (finite data): such keys are masked below and such columns meet zero Q entries or are never stored.
-  // A wave's rows of an image are 16 apart, so their swizzle is one number and the four slots serve all images.
+  // A wave's rows of an image are 16 (32) apart, so their swizzle is one number and its slots serve all images.
   const int frow = wave_u * 4 + (lane >> 4), fch = lane & 15;
   int fcol[NCB + NTB];
 #pragma unroll
@@ -192,14 +201,14 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
     fcol[img] = min(col, a.rs - 8);
   }
   auto fill = [&](int sbuf, int ibuf) {
-    int slot[4];
+    int slot[16 / NW];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) slot[j] = slot_lds[sbuf * LKB + 16 * j + frow];
+    for (int j = 0; j < 16 / NW; ++j) slot[j] = slot_lds[sbuf * LKB + 4 * NW * j + frow];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 16 / NW; ++j) {
       const unsigned short* base = a.cache + ((long)slot[j] * a.G + grp) * a.rs;
 #pragma unroll
-      for (int img = 0; img < NCB + NTB; ++img) dma16(base + fcol[img], lds_base + (unsigned)(ibuf * BUFB + img * LIMG + (wave_u + 4 * j) * 1024));
+      for (int img = 0; img < NCB + NTB; ++img) dma16(base + fcol[img], lds_base + (unsigned)(ibuf * BUFB + img * LIMG + (wave_u + NW * j) * 1024));
     }
   };
   // double-buffered form: the slots of tile t + 2 are requested BEFORE the fill of tile t + 1 is issued and
@@ -238,22 +247,23 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
       vm_wait<0>();
       __syncthreads();
     }
-    const int kv0 = tile_of(t) * LKB;
-    if (!wave_live || kv0 > w_last || (kv0 + LKB - 1 < w_lo && kv0 >= a.keep)) continue;
+    const int kv0 = tile_of(t) * LKB + kgrp * 32;  // the wave's first key of the tile
+    if (!wave_live || kv0 > w_last || (kv0 + KBN * 32 - 1 < w_lo && kv0 >= a.keep)) continue;
+    Ks += kgrp * 32 * LROWB, Vs += kgrp * 32 * LROWB;
 
-    f32x16 s[2];
+    f32x16 s[KBN];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KBN; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[kb][i] = 0.f;
     // the next k-steps' fragments are read while the ones before them are multiplied (left to itself the compiler reads each just ahead of its use)
     constexpr int KST = NKS >= 32 ? 1 : 2;  // (the widest keys have no registers for more)
-    bf16x8_t kf[2][KST][2];
-    auto read_k = [&](int k0, bf16x8_t (&f)[KST][2]) {
+    bf16x8_t kf[2][KST][KBN];
+    auto read_k = [&](int k0, bf16x8_t (&f)[KST][KBN]) {
 #pragma unroll
       for (int i = 0; i < KST; ++i)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < KBN; ++kb)
           f[i][kb] = lds_read_b128(Ks + ((k0 + i) >> 3) * LIMG + kb * 32 * LROWB, k_row + (k_x ^ (((2 * (k0 + i)) & 15) << 4)));
     };
     read_k(0, kf[0]);
@@ -264,17 +274,17 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
 #pragma unroll
       for (int i = 0; i < KST; ++i)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) s[kb] = mfma32(kf[(k0 / KST) & 1][i][kb], qf[k0 + i], s[kb]);
+        for (int kb = 0; kb < KBN; ++kb) s[kb] = mfma32(kf[(k0 / KST) & 1][i][kb], qf[k0 + i], s[kb]);
       __builtin_amdgcn_sched_barrier(0);
     }
     auto hidden = [&](int key) {  // (no branches: 32 of them per tile and lane)
       return !valid | (key > my_pos) | ((key < my_lo) & ((key >= a.keep) | (key < my_c0))) | (key >= ctx);
     };
-    bf16x8_t pb[2][2];
+    bf16x8_t pb[KBN][2];
     if constexpr (SIG) {
       // x (log2 domain) = s * scale - a log2(1 + b (i - j)) + bias; weight = 1 / (1 + 2^-x); hidden keys weigh 0
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+      for (int kb = 0; kb < KBN; ++kb) {
         float p[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -289,11 +299,11 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
       }
     } else {
       float mx = -INFINITY;
-      if (kv0 + LKB - 1 <= w_first && kv0 >= w_lo_last && kv0 + LKB - 1 < ctx) {
-        // every key of the tile is visible to every row of this wave: no mask (rows past the portion's end
+      if (kv0 + KBN * 32 - 1 <= w_first && kv0 >= w_lo_last && kv0 + KBN * 32 - 1 < ctx) {
+        // every key is visible to every row of this wave: no mask (rows past the portion's end
         // carry finite scores of a repeated row and are never stored)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < KBN; ++kb)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             if constexpr (CAP) s[kb][i] = a.cap_log2 * (1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + fast_exp2(s[kb][i] * a.cap_inv2)));
@@ -303,7 +313,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
         if (!valid) mx = -INFINITY;  // such a row must not trigger the wave's rescale
       } else {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+        for (int kb = 0; kb < KBN; ++kb)
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             float x;
@@ -321,7 +331,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
       const float m_new = m_raw == -INFINITY ? 0.f : m_raw;  // nothing seen yet (a later split, all keys masked)
       float rs = 0.f;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+      for (int kb = 0; kb < KBN; ++kb) {
         float p[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -344,7 +354,7 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
       m_i = m_raw;
     }
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KBN; ++kb)
 #pragma unroll
       for (int st = 0; st < 2; ++st)
 #pragma unroll
@@ -352,6 +362,31 @@ __global__ __launch_bounds__(256, NKS <= 8 && NDB <= 4 ? 2 : 1) void latent_attn
           const bf16x8_t vf = tr_frag_at<128>(Vs + (d >> 2) * LIMG, kb * 32 + 16 * st, tr_lo[d & 3], tr_hi[d & 3]);
           o[d] = mfma32(vf, pb[kb][st], o[d]);
         }
+  }
+
+  if constexpr (KG2) {  // the second group's results into the first's, through the images (all of whose fills have landed)
+    static_assert(4 * 64 * (NDB * 16 + 2) * 4 <= (DB ? 2 : 1) * BUFB, "LDS");
+    float* xs = reinterpret_cast<float*>(smem) + wave * 64 * (NDB * 16 + 2) + lane;
+    __syncthreads();
+    if (kgrp == 1) {
+#pragma unroll
+      for (int d = 0; d < NDB; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) xs[64 * (d * 16 + i)] = o[d][i];
+      xs[64 * NDB * 16] = m_i;
+      xs[64 * (NDB * 16 + 1)] = l_i;
+    }
+    __syncthreads();
+    if (kgrp == 1) return;
+    const float m_o = xs[64 * NDB * 16], l_o = xs[64 * (NDB * 16 + 1)];
+    const float m_both = fmaxf(m_i, m_o), m_ref = m_both == -INFINITY ? 0.f : m_both;
+    const float f_i = SIG ? 1.f : fast_exp2(m_i - m_ref), f_o = SIG ? 1.f : fast_exp2(m_o - m_ref);
+    l_i = l_i * f_i + l_o * f_o;
+    m_i = m_both;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[d][i] = o[d][i] * f_i + xs[64 * (d * 16 + i)] * f_o;
   }
 
   if (SPLIT && valid && a.nsplit > 1) {
@@ -429,7 +464,7 @@ void launch_ncb(const LArgs& a, int ndb, dim3 grid, hipStream_t st) {
     const size_t one = (size_t)(NCB + (NDBv + 3) / 4) * LIMG;
     const size_t lds = (2 * one + 1024 <= 160 * 1024 ? 2 * one : one) + 2 * LKB * sizeof(int);
     HYB_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess, "LDS size");
-    kern<<<grid, 256, lds, st>>>(a);
+    kern<<<grid, two_key_groups(NKS, NDBv, SPLIT) ? 512 : 256, lds, st>>>(a);
   };
   if (ndb == 2) go(latent_attn_mfma_kernel<NKS, 2, ROT, SIG, CAP, SPLIT>, 2);
   else if (ndb == 4) go(latent_attn_mfma_kernel<NKS, 4, ROT, SIG, CAP, SPLIT>, 4);
