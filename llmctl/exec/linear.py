@@ -192,6 +192,21 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
+def small_linear_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]:
+    """``x @ w^T`` of a prompt's rows with an fp32 result on ``gemm_small``, by the rules of :func:`small_linear`'s ``eager`` form, up to 2 Mi outputs;
+    else None.  Decay logits of gated linear attention (K 64), us, library / here: 200 x 1024 1.8 / 1.7, 2000 x 512 2.6 / 4.1, 2911 x 1024 4.8 / 9.1; a library product takes the host 24 us, this
+    9: malinex width 2048, 200 tokens 797 / 753, width 1024, 3800 tokens 964 / 924; 2911 tokens of width 2048 1375 / 1381, so left."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or type(x.shape[0]) is not int or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
+        return None
+    M, (N, K) = x.shape[0], w.shape
+    if (M * N > 2 << 20 or not small_pays("eager", M, N, K) or torch.cuda.is_current_stream_capturing() or _any_autocast() or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+            or _forward_ad._current_level >= 0 or torch.compiler.is_compiling() or not _small_ok("fwd", M, N, K, x, w)):
+        return None
+    y = torch.empty(M, N, dtype=torch.float32, device=x.device)
+    native().gemm_small(x, w, y, False, False, False)
+    return y
+
+
 _CUS = 256  # of an MI355X
 
 

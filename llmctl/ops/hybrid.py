@@ -646,6 +646,12 @@ def linear_f32(x, w):
         return torch.nn.functional.linear(x, w)
     if rows_ok(x, w):
         return rows_linear(x, w, f32=True)
+    if x.shape[0] > 32:  # a prompt's small products (the library's take the host 24 us, these 9)
+        from llmctl.exec.linear import small_linear_f32
+
+        y = small_linear_f32(x, w)
+        if y is not None:
+            return y
     if wants_grad(x, w):  # (the library's product with another output type has no derivative)
         return torch.nn.functional.linear(x, w).float()
     try:

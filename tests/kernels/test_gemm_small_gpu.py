@@ -206,3 +206,22 @@ def test_no_outputs(shape):
     with torch.no_grad():
         assert L.forward_linear(x, w, b).shape == (*shape[:-1], 0)
         assert ops.decode_linear(x, w, b).shape == (*shape[:-1], 0)
+
+
+@pytest.mark.parametrize("M,N,K,own", [(33, 8, 8, True), (200, 1024, 64, True), (2048, 1024, 72, True), (2049, 1024, 64, False), (40, 32000, 64, True), (64, 512, 68, False), (64, 8192, 2048, False)])
+def test_prompts_with_fp32_results(M, N, K, own):
+    """Rows cut from wider ones; sums of K exact products in fp32, in any order."""
+    from llmctl.exec.linear import small_linear_f32
+    from llmctl.ops import hybrid as hops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = torch.randn(M, K + 24, generator=g, device="cuda").bfloat16()[:, 8:8 + K], torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    X, W = x.double(), w.double()
+    y = small_linear_f32(x, w)
+    assert (y is not None) == (own and K % 8 == 0)
+    for got in (y, hops.linear_f32(x, w)):
+        assert got is None or (got.dtype == torch.float32 and bool(((got.double() - X @ W.t()).abs() <= K * 2.0**-23 * (X.abs() @ W.abs().t())).all()))
+    p = w.clone().requires_grad_()
+    assert small_linear_f32(x, p) is None and small_linear_f32(x.float(), w.float()) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert small_linear_f32(x, w) is None
