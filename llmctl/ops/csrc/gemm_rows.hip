@@ -3,7 +3,7 @@
 // A few hundred rows are 16 to 128 tiles, and a tile's K-tiles from HBM take a workgroup 0.5 to 0.8 us each whatever the others do (the lines that one CU can have on
 // their way): such products are cut into ranges of K, one workgroup each, whose fp32 sums gemm_rows_sum adds in the order of K.
 // us, one range / the best: 128 x 4096 x 11008 124 / 46 (2 TB/s), 200 x 2048 x 2048 19.0 / 13.7 (the adding pass and its launch are 6 of them), 200 x 2048 x 8192 68.7 / 22.9.
-// GELUs in the epilogue: 4.7 us a tile of 256 rows, which nothing overlaps, so large products leave them to a pass (3379 x 8192: 27 us).
+// GELUs in the epilogue: 3.9 us a tile of 256 rows, which nothing overlaps, so large products leave them to a pass (3379 x 8192: 27 us).
 //
 // y's columns may lie in groups apart (a latent prompt's keys and values beside a shared rotary key: the copy into place took 9.4 us for 2048 tokens of 16 heads).
 // Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, gemm_rows_form says.
@@ -32,7 +32,7 @@ constexpr int BAND = 4;  // tile rows that walk the columns together
 // ACT as in stream_linear.h (1 erf GELU, 2 tanh GELU), of the fp32 sum and the bias
 template <int ACT>
 __device__ __forceinline__ float act_of(float v) {
-  if constexpr (ACT == 1) return gelu_erf16(v);
+  if constexpr (ACT == 1) return gelu_erf(v);
   if constexpr (ACT == 2) return v / (1.0f + __expf(-1.5957691216057308f * (v + 0.044715f * v * v * v)));  // v sigmoid(2 z) = 0.5 v (1 + tanh z)
   return v;
 }

@@ -26,7 +26,7 @@ __device__ __forceinline__ float ldf(const bf16_t* p) { return __uint_as_float((
 __device__ __forceinline__ void stf(float* p, float v) { *p = v; }
 __device__ __forceinline__ void stf(bf16_t* p, float v) { *p = __bfloat16_as_ushort(__float2bfloat16(v)); }
 
-using llmctl::gelu_erf16;
+using llmctl::gelu_erf;
 
 // 16-byte accesses: 8 bf16 or 4 fp32 consecutive elements <-> floats (the pointer must be 16-byte aligned)
 template <typename T>

@@ -59,7 +59,7 @@ __device__ __forceinline__ float expert_act(int act, float u, float g) {
     const float r = fmaxf(u, 0.f);
     return r * r;
   }
-  return gelu_erf16(u);
+  return gelu_erf(u);
 }
 
 // The tiled form rounds the first projection's results to the activation's type before the activation, as a product and an
