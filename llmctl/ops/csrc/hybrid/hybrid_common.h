@@ -159,10 +159,9 @@ struct RowAttnOpts {
   int gate_per = 1;
 };
 
-// an output as its own rounding to bf16 leaves it, times the sigmoid of a gate; the hardware's exponential and reciprocal are good to an ulp
-__device__ __forceinline__ float gated(float v, float g) {
-  return __bfloat162float(__float2bfloat16(v)) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g));
-}
+// an output as its own rounding to bf16 leaves it, times the sigmoid of a gate, in the arithmetic of gate_mul_kernel (2 to a rounded multiple of g and the hardware's reciprocal are up to
+// 63 * 2^-24 off at g = -80)
+__device__ __forceinline__ float gated(float v, float g) { return __bfloat162float(__float2bfloat16(v)) * (1.0f / (1.0f + expf(-g))); }
 
 // How a launch over decode rows is cut: its workgroups before a row's keys are split, the splits, and the 64-key steps of a row at most
 struct DecodeCut {

@@ -407,7 +407,8 @@ __global__ __launch_bounds__(two_key_groups(NKS, NDB, SPLIT) ? 512 : 256, (NKS <
     const float inv = 1.f / l_i;
     unsigned short* Op = a.out + ((long)(q_begin + my_tok) * a.H + my_head) * a.rk;
     // A copy for either, not a branch in each of its stores: a launch without a gate reads no more code than before.  2048 tokens x 16 heads of 128 columns, a gate each:
-    // 49.7 us and a pass of 8.8 for the gate, so 53.5 (with a gate loaded where it is used 59.9).
+    // 53.3 us and a pass of 8.5 for the gate, so 58.9; 600 tokens 21.0 and 4.0, so 27.2 (the sigmoids' code is read once, from memory), but a launch less for the host: lenitar, 700 tokens
+    // 939 us with the pass, so 915.
     auto store = [&](auto gated_c) __attribute__((always_inline)) {
       constexpr bool GATED = decltype(gated_c)::value;
       // a lane's gates lie in its own row, 8 bytes at a time: all on their way before the first is used

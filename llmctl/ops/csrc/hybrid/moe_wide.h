@@ -12,9 +12,6 @@
 
 namespace llmctl_hybrid {
 namespace {
-// silu(g) u; the hardware's exponential and reciprocal are good to an ulp, a result is rounded to 8 bits
-__device__ __forceinline__ float silu_mul(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)) * u; }
-
 // (The activation is a parameter: with a branch on it in the 144 places of an epilogue the instructions came from memory, 10 us a launch.)
 template <int MODE>
 __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) void moe_wide_kernel(TileArgs g) {
@@ -102,7 +99,7 @@ __global__ __launch_bounds__(256, 1) __attribute__((amdgpu_waves_per_eu(1, 1))) 
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) x[j][q] = silu_mul(bf16_of(a[j][q]), bf16_of(a[j + 2][q]));
+        for (int q = 0; q < 4; ++q) x[j][q] = expert_act(1, bf16_of(a[j + 2][q]), bf16_of(a[j][q]));
       put(x[0], x[1], c0 + wc * 32);
     } else {
 #pragma unroll

@@ -75,3 +75,30 @@ def test_gelu_of_experts():
     many, few = _experts(x, "gelu")
     assert torch.equal(many, few)
     _check_gelu(x, many)
+
+
+def test_silu_of_experts():
+    x = _numbers()
+    many, few = _experts(torch.where(x.abs() < 2.0**63, x, torch.zeros_like(x)), "swiglu")  # (their squares are finite)
+    assert torch.equal(many, few)
+
+
+@pytest.mark.parametrize("each", [True, False])
+def test_gates_of_attention(each):
+    """Every number as a gate: what the pass after the attention gives, prompts and decode rows whose splits a merge joins."""
+    from llmctl.ops import hybrid as hops
+
+    H, R, T = 2, 128, N
+    g = torch.Generator(device="cuda").manual_seed(0)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    cache, bt = r(T * 8, 16, R), torch.arange(T * 8, device="cuda", dtype=torch.int32).view(T, 8)
+    gate = _numbers() if each else _numbers()[:, :H]
+    for col in range(0, 1 if each else N, H):
+        if not each:
+            gate = _numbers()[:, col:col + H]
+        qa, one = r(T, H, R), torch.full((T,), 128, device="cuda", dtype=torch.int32)
+        cu = torch.tensor([0, T // 2, T], device="cuda", dtype=torch.int32)
+        calls = [lambda **kw: hops.latent_attention_decode(qa, cache, bt, one, hops.NO_LIMIT, None, 0.1, R, max_ctx=128, **kw),
+                 lambda **kw: hops.latent_attention_prefill(qa, cache, bt[:2], cu, one[:2], hops.NO_LIMIT, None, 0.1, R, T // 2, **kw)]
+        for call in calls:
+            assert torch.equal(call(gate=gate).reshape(T, -1), hops.sigmoid_gate_mul(call().reshape(T, -1), gate))
