@@ -224,26 +224,26 @@ def _tile_rows(M: int, form: int) -> int:
 def rows_form(M: int, N: int, K: int, act: bool = False, eager: bool = False) -> int:
     """How ``gemm_rows`` (csrc/gemm_rows.hip) multiplies M rows of width K to N outputs where that is faster than the library: tiles (1 = 256 rows, 2 = 128) + 4 (ranges of K - 1);
     else 0.  ``act``: an activation follows, which costs the library's product a pass; ``eager``: launches that the host feeds one by one.
-    From 1024 rows on, one range of K: a model of either's workgroups and of the library's products, us: 12 and 1300 TFLOP/s, small ones 6 and 550; constants fitted to 245 sizes, 33
-    to 4096 rows, 256 to 12288 outputs, K 256 to 8192, operands from HBM (``profiles/prompt_products.txt``).  The rule takes 81 of them, in 20 % less time; one of these takes 4 % more.
-    us, library / here: 2048 x 2048 x 2048 25.8 / 17.8, 2048 x 3712 x 2048 35.5 / 29.0, 2911 x 2048 x 1024 23.2 / 16.8, 1128 x 3584 x 1664 21.4 / 15.5, 769 x 2816 x 256
-    9.4 / 6.4; left to the library: 1.1 rounds, 2911 x 3072 x 2048 36.8 / 46.0; large products, 3379 x 8192 x 2048 94 / 109.
-    Up to 1024 rows: :func:`_few_rows_form`."""
+    Up to 1024 rows: :func:`_few_rows_form`, and nothing else.  Beyond, one range of K: a model of either's workgroups and of the library's products, us: 12 and 1300 TFLOP/s, small ones 6 and 550,
+    fitted to kernel times with operands from HBM (``profiles/prompt_products.txt``, to 4096 rows, 256 to 12288 outputs, K 256 to 8192).  Of its 73 sizes of more than 1024
+    rows the rule takes 31, in 21 % less time; one of these takes longer, 1049 x 256 x 256 5.3 / 5.6.  In ``profiles/short_prompt_products.txt`` (42 such sizes) 19, in 8 % less; four take longer,
+    1300 x 3072 x 1024 15.4 / 18.1, the others up to 0.7 us.
+    us, library / here: 2048 x 2048 x 2048 25.8 / 17.8, 2048 x 3712 x 2048 35.5 / 29.0, 2911 x 2048 x 1024 23.2 / 16.8, 1128 x 3584 x 1664 21.4 / 15.5; left to the library: 1.1 rounds,
+    2911 x 3072 x 2048 36.8 / 46.0; large products, 3379 x 8192 x 2048 94 / 109."""
     if M <= 32 or N <= 0 or N & 7 or K & 127 or K < 256:
         return 0
-    code = _few_rows_form(M, N, K, act, eager) if M <= 1024 else 0
-    if code:
-        return code
+    if M <= 1024:
+        return _few_rows_form(M, N, K, act, eager)
     cols, kt = -(-N // 128), K / 64
     tall = _rounds_us(_tile_rows(M, 1) * cols, kt, 0.47, 0.36, 5.0 + act * _ACT_TILE[1])
     half = _rounds_us(_tile_rows(M, 2) * cols, kt, 0.28, 0.18, 4.0 + act * _ACT_TILE[2])
     gflop = 2e-9 * M * N * K
-    if min(tall, half) >= (0.95 if K <= 2304 else 0.85) * min(12.0 + gflop / 1.3, 6.0 + gflop / 0.55) + act * _act_us(M, N):  # (GPT-7B's, 900 x 4096 x 4096, 39 / 34, took its prompt 1 % longer)
+    if min(tall, half) >= (0.95 if K <= 2304 else 0.85) * min(12.0 + gflop / 1.3, 6.0 + gflop / 0.55) + act * _act_us(M, N):
         return 0
     return 1 if tall <= half else 2
 
 
-_ACT_TILE = {1: 4.7, 2: 2.4}  # GELUs of a tile in its epilogue, us: nothing else runs on its CU meanwhile
+_ACT_TILE = {1: 3.9, 2: 2.1}  # GELUs of a tile in its epilogue, us: nothing else runs on its CU meanwhile
 
 
 def _act_us(M: int, N: int) -> float:
@@ -251,26 +251,32 @@ def _act_us(M: int, N: int) -> float:
 
 
 def _few_rows_form(M: int, N: int, K: int, act: bool, eager: bool) -> int:
-    """:func:`rows_form` of a short prompt.  Its tiles are few, so K is cut into ranges of 256 at least; and an eager step is the host's: a library product takes the host 24 us, this 9 (13
-    with the pass that adds the ranges), so a product of at most 22 us
-    and 4 Mi outputs may take a few us longer there.  Both models fitted to 280 sizes, 40 to 2000 rows
-    (``profiles/short_prompt_products.txt``).
-    us, library / here: 128 x 4096 x 11008 79 / 46, 200 59 / 52, 64 x 2048 x 8192 26 / 19, 600 49 / 38, 256 x 8256 x 2048 31 / 26; for the host's sake 256 x 2048 x 2048 11.3 / 15.0, 128 x 2048 x
-    4096 12.8 / 17.2; left to the library 128 x 12288 x 4096 45 / 53, 450 x 22016 x 4096 98 / 129.  Prompts, us a step: dumazen width 2048 100 tokens 1387, so 1101, 450 1331 / 1211;
-    lenitar 300 982 / 843; malinex 200 948 / 807; GPT-7B layers 200 923 / 883; with the GELU in it gpt2-125m 600 1844 / 1548."""
-    cols, stream = -(-N // 128), 4.0 + N * K * 2e-6 / 2.2
+    """:func:`rows_form` of up to 1024 rows.  Their tiles are few, so K is cut into ranges of 256 at least.  The model of these launches is a fit to their times at 1211 sizes
+    (12 % off in the root mean square), the library's a lower bound, for its own times jump by a half from one size to the next (256 x 6144 x 2048 27.4, 288 rows 18.8): a pick is to be
+    faster wherever they fall (``profiles/few_rows_products.txt``, ``short_prompt_products.txt`` and ``prompt_products.txt``).  334 of the sizes are taken, in 19 % less time; six of these take longer,
+    291 x 256 x 8192 14.2 / 15.3 the longest of its own.
+    ``eager``: a step's launches are the host's time, and a library product takes it 24 us, this 9 (13 with the pass that adds the ranges): of up to 6 Mi outputs and 36 us also what may take
+    the chip a few us longer, 7 and a quarter of the library's lower bound by the model, 6.3 at most of the sizes timed (200 x 6144 x 2048 16.7 / 23.0; all 1000 that are taken, in 10 % less).
+    us, library / here: 600 x 2048 x 8192 47 / 36, 128 x 4096 x 11008 79 / 46; left to the library 900 x 2048 x 2048 16.3 / 20.3, 288 x 32000 x 2048 68 / 81, 128 x 12288 x 4096 45 / 53; for the
+    host's sake 256 x 2048 x 2048 11.3 / 14.9.  Prompts, us a step, with every product the library's / here: dumazen width 2048 100 tokens 1387 / 1118, 450 1331 / 1110, 900 tokens
+    1440 / 1380; lenitar 300 982 / 880; malinex 200 948 / 809."""
+    cols, stream = -(-N // 128), 4.0 + N * K * 2e-6 / 2.1
     best, code = 1e9, 0
     for splits in (1, 2, 3, 4, 6, 8, 12, 16):
         if splits > 1 and (splits > K // 256 or splits * cols * _tile_rows(M, 1) > 512):
             break
-        kt, add = K / 64 / splits, 0.0 if splits == 1 else 4.1 + splits * M * N * 4e-6 / 2.36
-        for form, (empty, full, fixed) in ((1, (0.73, 0.38, 2.5)), (2, (0.52, 0.20, 1.7))):
+        kt, add = K / 64 / splits, 0.0 if splits == 1 else 4.6 + splits * M * N * 4e-6 / 2.94
+        for form, (empty, full, fixed) in ((1, (0.626, 0.39, 4.9)), (2, (0.448, 0.237, 3.85))):
             t = _rounds_us(splits * cols * _tile_rows(M, form), kt, empty, full, fixed + (act * _ACT_TILE[form] if splits == 1 else 0.0)) + add
             if t < best:
                 best, code = t, form + 4 * (splits - 1)
-    best, gflop, mb = max(best, stream), 2e-9 * M * N * K, N * K * 2e-6
-    library = (6.1 + 0.237 * mb + 0.8 * gflop + 0.585 * gflop ** 0.5 + 0.545 * mb ** 0.5) * (1.25 if K >= 8192 else 1.0) + act * _act_us(M, N)
-    return code if best < (0.92 if mb <= 64 or K >= 8192 else 0.8) * library or (eager and M * N <= 4 << 20 and best <= min(library + 7.0, 22.0)) else 0
+    best, gflop = max(best, stream), 2e-9 * M * N * K
+    if K < 8192:
+        library = 7.7 + 0.1 * N * K * 2e-6 + 0.96 * gflop
+    else:  # (few tiles and long chains there too: it leaves the chip idle until some 40 GFLOP)
+        library = min(13.5 + 2.9 * gflop, 60.0 + 0.85 * gflop)
+    library += act * _act_us(M, N)
+    return code if best < library or (eager and M * N <= 6 << 20 and best <= min(1.25 * library + 7.0, 36.0)) else 0
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, act: int = 0,

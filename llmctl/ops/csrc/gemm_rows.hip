@@ -6,7 +6,7 @@
 // GELUs in the epilogue: 3.9 us a tile of 256 rows, which nothing overlaps, so large products leave them to a pass (3379 x 8192: 27 us).
 //
 // y's columns may lie in groups apart (a latent prompt's keys and values beside a shared rotary key: the copy into place took 9.4 us for 2048 tokens of 16 heads).
-// Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, gemm_rows_form says.
+// Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, rows_form of exec/linear.py says.
 #include "gelu_erf.h"
 #include "wide_tiles.h"
 

@@ -121,7 +121,7 @@ def _fwd_into(w, b):
             if b is not None:
                 out += b
         else:
-            out.copy_(forward_linear(xc, w, b))
+            out.copy_(forward_linear(xc, w, b, "fwd"))
     return mm
 
 
@@ -187,7 +187,7 @@ class _RowSP(torch.autograd.Function):
 
         ctx.save_for_backward(x, w)
         ctx.wparam, ctx.group = w, group
-        return _matmul_rs(x.contiguous(), group, lambda xc: forward_linear(xc, w))
+        return _matmul_rs(x.contiguous(), group, lambda xc: forward_linear(xc, w, layout="fwd"))
 
     @staticmethod
     def backward(ctx, dy):

@@ -1,0 +1,62 @@
+"""The rule of the prompt products' tiles against the times that its figures are from: up to 1024 rows nothing that it takes is much slower than the library's product, whichever the
+file, and what it takes for the host's sake costs the chip a few us."""
+import importlib
+import re
+from pathlib import Path
+
+import pytest
+
+L = importlib.import_module("llmctl.exec.linear")
+PROFILES = Path(__file__).resolve().parents[2] / "profiles"
+
+
+def _times():
+    """(rows, outputs, K, library's us, {(tiles, ranges of K): us})"""
+    for name in ("few_rows_products.txt", "short_prompt_products.txt"):
+        for line in (PROFILES / name).read_text().splitlines():
+            if m := re.match(r"(\d+) (\d+) (\d+) \| ([\d.]+) \| \S+ \| (.*)$", line):
+                yield *map(int, m.groups()[:3]), float(m[4]), {(int(a), int(b)): float(t) for a, b, t in re.findall(r"(\d):(\d+) ([\d.]+)", m[5])}
+    for line in (PROFILES / "prompt_products.txt").read_text().splitlines():
+        if m := re.match(r"(\d+) (\d+) (\d+) \| ([\d.]+) \| ([\d.]+) ([\d.]+) \|", line):
+            yield *map(int, m.groups()[:3]), float(m[4]), {(1, 1): float(m[5]), (2, 1): float(m[6])}
+
+
+def _picks(eager):
+    for M, N, K, library, own in _times():
+        code = L.rows_form(M, N, K, False, eager)
+        form = code & 3, (code >> 2) + 1
+        if M <= 1024 and code and form in own:
+            yield M, N, K, library, own[form]
+
+
+def test_picks_are_faster():
+    picks = list(_picks(False))
+    assert len(picks) >= 300 and all(own <= 1.08 * library for *_, library, own in picks)
+    assert sum(own > library for *_, library, own in picks) <= 6
+    assert sum(own for *_, own in picks) < 0.83 * sum(library for *_, library, _ in picks)
+
+
+def test_what_the_host_saves_costs_the_chip_little():
+    picks = list(_picks(True))
+    assert len(picks) >= 900 and all(own <= library + 6.4 for *_, library, own in picks)
+    assert sum(own for *_, own in picks) < 0.92 * sum(library for *_, library, _ in picks)
+
+
+@pytest.mark.parametrize("M,N,K", [(900, 2048, 2048), (450, 3712, 2048), (350, 5136, 2048), (288, 6144, 2048), (288, 5136, 2048), (288, 32000, 2048), (100, 4096, 4096), (200, 8192, 2048)])
+def test_the_librarys(M, N, K):
+    """(288 x 32000 x 2048 is more than the host's sake allows)"""
+    assert L.rows_form(M, N, K) == 0 and (N < 32000 or L.rows_form(M, N, K, False, True) == 0)
+
+
+def test_training_under_tensor_parallelism_does_not_ask_for_the_hosts_sake(monkeypatch):
+    import torch
+
+    tp = importlib.import_module("llmctl.parallel.async_tp")
+    asked, own = [], L.forward_linear
+    monkeypatch.setattr(L, "forward_linear", lambda x, w, b=None, layout="eager": asked.append(layout) or own(x, w, b, layout))
+    monkeypatch.setattr(tp, "_matmul_rs", lambda x, group, mm: mm(x))
+    x, w = torch.randn(4, 16), torch.randn(8, 16)
+    out = torch.zeros(4, 12)[:, :8]
+    tp._fwd_into(w, None)(x, out)
+    y = tp._RowSP.apply(x, w, None)
+    assert torch.equal(out, y) and torch.allclose(y, x @ w.t(), atol=1e-5) and len(asked) == 2 and "eager" not in asked
