@@ -61,8 +61,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_expert_rows_shared(const at::
                                                                       at::TensorList down, int64_t act, const at::Tensor& w_sup,
                                                                       const c10::optional<at::Tensor>& b_sup, int64_t act_cols, const at::Tensor& w_sdown);
 bool moe_shared_rides(int64_t M, int64_t N, int64_t K, int64_t ff);
+bool moe_wide_pays(int64_t N, int64_t E, int64_t W, int64_t ff, bool glu);
 at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
-                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate);
+                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t form);
 at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor& wgt, const at::Tensor& x, const c10::optional<at::Tensor>& shared,
                    const c10::optional<at::Tensor>& gate, int64_t experts);
 std::vector<at::Tensor> add_experts_layernorm_f32_(at::Tensor x, const at::Tensor& a, const c10::optional<at::Tensor>& w, const c10::optional<at::Tensor>& bias,
@@ -192,7 +193,8 @@ TORCH_LIBRARY(llmctl_hybrid, m) {
   m.def("moe_expert_rows(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act) -> Tensor");
   m.def("moe_expert_rows_shared(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor w_sup, Tensor? b_sup, int act_cols, Tensor w_sdown) -> (Tensor, Tensor, Tensor)");
   m.def("moe_shared_rides(int M, int N, int K, int ff) -> bool", &llmctl_hybrid::moe_shared_rides);
-  m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None) -> Tensor");
+  m.def("moe_wide_pays(int N, int E, int W, int ff, bool glu) -> bool", &llmctl_hybrid::moe_wide_pays);
+  m.def("moe_experts(Tensor x, Tensor idx, Tensor wgt, Tensor[] up, Tensor[] down, int act, Tensor? shared=None, Tensor? gate=None, int form=0) -> Tensor");
   m.def("moe_sum(Tensor y, Tensor idx, Tensor wgt, Tensor x, Tensor? shared, Tensor? gate, int experts) -> Tensor");
   m.def("add_experts_layernorm_f32_(Tensor(a!) x, Tensor a, Tensor? w, Tensor? bias, float eps, Tensor y, Tensor idx, Tensor wgt, Tensor xin, Tensor? shared, Tensor? gate, int experts, Tensor? router=None, Tensor? rbias=None, int top=0, int groups=1, int keep=1, bool softmax=False, bool renorm=False) -> Tensor[]");
   m.def("gated_norm_add_norm_route_(Tensor(a!) x, Tensor y, Tensor r, Tensor w_post, Tensor w_next, float eps, Tensor router, Tensor? rbias, int top, int groups, int keep, bool softmax, bool renorm) -> Tensor[]");

@@ -23,8 +23,8 @@
 //   * moe_combine_kernel: out_t = sum_k w_tk y_tk (+ w x_t for experts without weights) (+ the shared expert), fp32; where the
 //     result goes straight into the residual stream and a norm, their kernel sums instead (expert_rows.h).
 //
-// Other widths, and experts that get less than 96 rows on average (48 where tiles of 64 x 64 would make more than a round of the chip, below), have tiles of 128 x 128 (96
-// rows and more) or 64 x 64: with few tiles the K loop of every workgroup is a chain of load latencies.  The large tile
+// Other widths, and sizes that moe_wide_pays leaves, have tiles of 128 x 128 (96
+// rows an expert and more) or 64 x 64: with few tiles the K loop of every workgroup is a chain of load latencies.  The large tile
 // keeps one LDS buffer (32 KB) so that three workgroups fit a CU; the small one keeps three steps in flight (37 -> 30 us at 65 tokens).
 //
 // Measured, one MI355X, width 2048, 8 gated experts of 1024, top 2 (up / down; weights from HBM):
@@ -143,8 +143,8 @@ __global__ __launch_bounds__(ROUTE_WAVES * 64) void moe_route_kernel(const bf16_
 // ------------------------------------------------------------------------------------------------ grouping
 // Row tiles of n rows: of BM each, or (WIDE_ROWS, moe_wide.h) of 256 but the last one, which has 33 to 288.
 constexpr int WIDE_ROWS = 288, WIDE_HALF = 128;
-__device__ __forceinline__ int row_tiles(int n, int BM) { return BM != WIDE_ROWS ? (n + BM - 1) / BM : n <= BM ? n > 0 : (n - 33) / 256 + 1; }
-__device__ __forceinline__ bool half_tile(int n, int BM) {  // the last one has at most 128 rows
+__host__ __device__ __forceinline__ int row_tiles(int n, int BM) { return BM != WIDE_ROWS ? (n + BM - 1) / BM : n <= BM ? n > 0 : (n - 33) / 256 + 1; }
+__host__ __device__ __forceinline__ bool half_tile(int n, int BM) {  // the last one has at most 128 rows
   return BM == WIDE_ROWS && n > 0 && n - 256 * (row_tiles(n, BM) - 1) <= WIDE_HALF;
 }
 
@@ -380,6 +380,32 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
 }  // namespace llmctl_hybrid
 #include "moe_wide.h"
 namespace llmctl_hybrid {
+// Whether N copies for E experts run on tiles of up to 288 x 128 (moe_wide.h) rather than on tiles of 128 x 128 or, below 96 rows an expert, 64 x 64: both products' rounds, in
+// units of a K-step of 64 of a round of 128 x 128 tiles (three to a CU).  The experts' rows are taken as random choices spread them.  A round of 256 full tiles counts 0.24 a K-step and
+// 8.5, one of half tiles, behind them, 0.377 and 2.15; 64 x 64 tiles 0.875 a K-step, four to a CU and no whole rounds.  The constants are fitted to the comparison, not to the
+// times, at 1803 sizes (66 to 4096 tokens, widths 512 to 4096, 4 to 64 experts of 256 to 2048, top 1 to 6: profiles/expert_tiles.txt): 737 are taken, in 13 % less time, 27 of them
+// are slower, by 6 % at most (383 tokens of width 512, 8 gated experts of 2048, top 6: 75 / 80 us); 93 % of what the better choice everywhere would give.  By rows per expert alone
+// 94 sizes were more than 5 % slower: 2612 tokens of width 1024, 32 gated experts of 512, top 4 86 / 94, 377 of width 2048, 8 of 256 40 / 51.
+bool moe_wide_pays(int64_t N, int64_t E, int64_t W, int64_t ff, bool glu) {
+  if (E < 1 || N < 48 * E || N > INT32_MAX || W % 128 != 0 || ff % 128 != 0 || W < 256 || ff < 256) return false;
+  const int B = N >= 96 * E ? 128 : 64;
+  const double mean = (double)N / E, dev = std::sqrt(mean * (1.0 - 1.0 / E));
+  double full = 0.0, half = 0.0, other = 0.0;  // row tiles
+  for (const auto& [z, p] : {std::pair{-1.22, 0.3}, {0.0, 0.4}, {1.22, 0.3}}) {
+    const int n = (int)std::nearbyint(mean + z * dev), h = half_tile(n, WIDE_ROWS);
+    full += E * p * (row_tiles(n, WIDE_ROWS) - h), half += E * p * h, other += E * p * row_tiles(std::max(n, 1), B);
+  }
+  double wide = 0.0, narrow = 0.0;
+  for (const auto& [cols, K] : {std::pair{glu ? 2 * ff : ff, W}, {W, ff}}) {
+    const double steps = (double)K / 64, nt = (double)cols / 128, cf = 0.24 * steps + 8.5, ch = 0.377 * steps + 2.15;
+    const double span = std::ceil(full * nt / 256 - 0.04) * cf, left = half * nt * ch / 256 - 0.85 * std::max(0.0, span - full * nt * cf / 256);
+    wide += span + (left > 0.0 ? std::ceil(left / ch - 0.04) * ch : 0.0);
+    const double items = other * std::ceil((double)cols / B);
+    narrow += steps * (B == 128 ? std::max(1.0, std::ceil(items / 768 - 0.1)) : 0.875 * items / 1024);
+  }
+  return wide < narrow;
+}
+
 namespace {
 static_assert(WIDE_ROWS == llmctl::wide::ROWS, "row tiles");
 
@@ -622,7 +648,8 @@ bool side_rides(int64_t M, int64_t N, int64_t K) {
   return M <= 32 && f.nt == 1 && f.nw == 4 && f.u == 8;
 }
 
-at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act, SharedExpert* sh) {
+at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act, SharedExpert* sh,
+                       int64_t form = 0) {
   int64_t E, R, W, E2, W2, ff;
   long ldu, ldd;
   const ExpertPtrs pu = expert_ptrs(up, E, R, W, ldu, "up"), pd = expert_ptrs(down, E2, W2, ff, ldd, "down");
@@ -678,10 +705,8 @@ at::Tensor expert_rows(const at::Tensor& x, const at::Tensor& idx, const at::Ten
     else if (T <= 32) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 4>{});
   } else {
-    // tiles of up to 288 rows (moe_wide.h) where the experts get 96 rows on average, or 48 and tiles of 64 x 64 make more than a round of the chip; else, and for
-    // widths in no 128s, of 128 or 64
-    const bool wide = (N >= 96 * E || (N >= 48 * E && (N / 64 + E / 2) * (W / 64) >= 400)) && W % 128 == 0 && ff % 128 == 0 && W >= 256 && ff >= 256 && T * x.stride(0) < ((int64_t)1 << 30) && N * ff < ((int64_t)1 << 30) &&
-                      R * ldu < ((int64_t)1 << 30) && W * ldd < ((int64_t)1 << 30);
+    const bool wide = form != 1 && (moe_wide_pays(N, E, W, ff, act == 1) || (form == 2 && W % 128 == 0 && ff % 128 == 0 && W >= 256 && ff >= 256)) && T * x.stride(0) < ((int64_t)1 << 30) && N * ff < ((int64_t)1 << 30) && R * ldu < ((int64_t)1 << 30) &&
+                      W * ldd < ((int64_t)1 << 30);
     const int BM = wide ? WIDE_ROWS : N >= 96 * E ? 128 : 64, BN = wide ? llmctl::wide::COLS : BM;
     const int64_t mt = wide ? N / 256 + E : (N + BM - 1) / BM + E;  // no more row tiles than this
     at::Tensor ints = at::empty({N + 2 + 3 * mt}, idx.options());
@@ -778,9 +803,10 @@ at::Tensor moe_sum(const at::Tensor& y, const at::Tensor& idx, const at::Tensor&
   return out;
 }
 
+// form (tests, sweeps): 0 the faster tiles (moe_wide_pays), 1 those of 64 or 128 rows, 2 those of moe_wide.h where they take the widths
 at::Tensor moe_experts(const at::Tensor& x, const at::Tensor& idx, const at::Tensor& wgt, at::TensorList up, at::TensorList down, int64_t act,
-                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate) {
-  const at::Tensor y = moe_expert_rows(x, idx, wgt, up, down, act);
+                       const c10::optional<at::Tensor>& shared, const c10::optional<at::Tensor>& gate, int64_t form) {
+  const at::Tensor y = expert_rows(x, idx, wgt, up, down, act, nullptr, form);
   return moe_sum(y, idx, wgt, x, shared, gate, up.size() == 1 && up[0].dim() == 3 ? up[0].size(0) : (int64_t)up.size());
 }
 

@@ -6,7 +6,7 @@
 // most 128 rows are dealt out last, to the CUs that are done first.
 // us, tiles of 128 x 128 / these: width 2048, 8 experts of 1024, up (gated) and down, 459 tokens 36.5, 21.7 / 25.4, 15.0, 1021 46.9, 27.0 / 34.8, 20.3, 3035 83, 47 / 66, 39;
 // without gates 3011 tokens 49, 46 / 33, 36; width 4096, 8 of 1408, gated, 1511 tokens 118, 65 / 100, 54; 32 experts, width 1024, 1699 tokens 32, 29 / 26, 24, but gated
-// 2612 tokens, a third of whose tiles start a new round, 70, 39 / 78, 39.
+// 2612 tokens, a third of whose tiles start a new round, 70, 39 / 78, 39 (which moe_wide_pays leaves to the others).
 #pragma once
 #include "wide_tiles.h"
 

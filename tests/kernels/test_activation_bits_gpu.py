@@ -60,27 +60,27 @@ def test_gelu_of_fp32_sums():
 
 
 def _experts(x, act):
-    """Rows of many and of few, whose kernel takes the first projection's sums as they are: here exact bf16 numbers."""
+    """Rows of many on either kind of tiles, and of few, whose kernel takes the first projection's sums as they are: here exact bf16 numbers."""
     from llmctl.ops import hybrid as hops
 
     one = _eye()
     up = torch.cat([one, one])[None] if act == "swiglu" else one[None]
     nat, idx, w = hops.native_hybrid(), torch.zeros(N, 1, device="cuda", dtype=torch.int32), torch.ones(N, 1, device="cuda")
-    call = lambda a, b: nat.moe_experts(x[a:b], idx[a:b], w[a:b], [up], [one[None]], hops._EXPERT_ACTS[act]).bfloat16()
-    return call(0, N), torch.cat([call(i, i + 64) for i in range(0, N, 64)])
+    call = lambda a, b, form: nat.moe_experts(x[a:b], idx[a:b], w[a:b], [up], [one[None]], hops._EXPERT_ACTS[act], None, None, form).bfloat16()
+    return [call(0, N, 1), call(0, N, 2)], torch.cat([call(i, i + 64, 0) for i in range(0, N, 64)])
 
 
 def test_gelu_of_experts():
     x = _numbers()
     many, few = _experts(x, "gelu")
-    assert torch.equal(many, few)
-    _check_gelu(x, many)
+    assert all(torch.equal(y, few) for y in many)
+    _check_gelu(x, few)
 
 
 def test_silu_of_experts():
     x = _numbers()
     many, few = _experts(torch.where(x.abs() < 2.0**63, x, torch.zeros_like(x)), "swiglu")  # (their squares are finite)
-    assert torch.equal(many, few)
+    assert all(torch.equal(y, few) for y in many)
 
 
 @pytest.mark.parametrize("each", [True, False])

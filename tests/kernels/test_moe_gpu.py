@@ -76,10 +76,30 @@ def test_wide_tiles_at_their_edges(counts, W, ff, top, act):
     x, _, up, down = _case(T, W, ff, E, act, seed=sum(counts))
     d3 = down.view(W, E, ff).transpose(0, 1)
     w = torch.rand(T, top, device="cuda")
-    got = hops.native_hybrid().moe_experts(x, idx, w, [up], [d3], hops._EXPERT_ACTS[act])
     want = _plain(x, idx.long(), w, up, d3, act, E)
-    # as above, row by row: a wrong row would not show in the norm of all
-    assert bool(((got.double() - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1) + 1e-12).all())
+    for form in (0, 2):  # (which the rule takes, and these tiles)
+        got = hops.native_hybrid().moe_experts(x, idx, w, [up], [d3], hops._EXPERT_ACTS[act], None, None, form)
+        # as above, row by row: a wrong row would not show in the norm of all
+        assert bool(((got.double() - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1) + 1e-12).all())
+
+
+def test_tiles_that_pay():
+    """The rule of the wide tiles against the times that its figures are from."""
+    import re
+    from pathlib import Path
+
+    from llmctl.ops import hybrid as hops
+
+    pays = hops.native_hybrid().moe_wide_pays
+    picks = []
+    for line in (Path(__file__).resolve().parents[2] / "profiles" / "expert_tiles.txt").read_text().splitlines():
+        if m := re.match(r"(\d+) (\d+) (\d+) (\d+) (\d+) (\w+) \| ([\d.]+) \| ([\d.]+)$", line):
+            T, W, ff, E, top = map(int, m.groups()[:5])
+            if pays(T * top, E, W, ff, m[6] == "swiglu"):
+                picks.append((float(m[7]), float(m[8])))
+    assert len(picks) >= 700 and all(wide <= 1.07 * other for other, wide in picks) and sum(wide > other for other, wide in picks) <= 30
+    assert sum(wide for _, wide in picks) < 0.88 * sum(other for other, _ in picks)
+    assert not any(pays(N, E, W, ff, True) for N, E, W, ff in ((0, 8, 2048, 1024), (383, 8, 2048, 1024), (4096, 8, 2048, 1000), (4096, 8, 2040, 1024), (4096, 8, 128, 1024), (4096, 0, 2048, 1024)))
 
 
 @pytest.mark.parametrize("T", [5, 64, 65, 700])
