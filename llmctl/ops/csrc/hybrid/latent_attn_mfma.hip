@@ -411,19 +411,20 @@ __global__ __launch_bounds__(two_key_groups(NKS, NDB, SPLIT) ? 512 : 256, (NKS <
     // 939 us with the pass, so 915.
     auto store = [&](auto gated_c) __attribute__((always_inline)) {
       constexpr bool GATED = decltype(gated_c)::value;
-      // a lane's gates lie in its own row, 8 bytes at a time: all on their way before the first is used
+      // a lane's gates lie in its own row, 8 bytes at a time: all on their way before the first is used, but for the widest turned values, whose loop stays one (an array that it
+      // indexes would lie in scratch memory: 1088 bytes a lane for 576, in launches without a gate too)
+      constexpr bool AHEAD = !(ROT && NDB > 4);
       const bf16_t* Gp = a.gate + (long)(q_begin + my_tok) * a.gate_st;
       const bool each = a.gate_per == 1;
-      float4 gt[GATED ? NDB : 1][4];
-      if constexpr (GATED) {
-        const float one = each ? 0.f : ldf(Gp + my_head);
+      float one = 0.f;
+      if constexpr (GATED) one = each ? 0.f : ldf(Gp + my_head);
+      auto gates = [&](int col) { return each ? ld4(Gp + (long)my_head * a.rk + min(col, a.rk - 4)) : make_float4(one, one, one, one); };
+      float4 gt[GATED && AHEAD ? NDB : 1][4];
+      if constexpr (GATED && AHEAD) {
 #pragma unroll
         for (int d = 0; d < NDB; ++d)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int col = v0 + d * 32 + 8 * g + 4 * hh;
-            gt[d][g] = each ? ld4(Gp + (long)my_head * a.rk + min(col, a.rk - 4)) : make_float4(one, one, one, one);
-          }
+          for (int g = 0; g < 4; ++g) gt[d][g] = gates(v0 + d * 32 + 8 * g + 4 * hh);
       }
 #pragma unroll
       for (int d = 0; d < NDB; ++d)
@@ -442,10 +443,15 @@ __global__ __launch_bounds__(two_key_groups(NKS, NDB, SPLIT) ? 512 : 256, (NKS <
               }
             }
             unsigned short w4[4];
+            float4 gv;
+            if constexpr (GATED) {
+              if constexpr (AHEAD) gv = gt[d][g];
+              else gv = gates(col);
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
               float v = o[d][4 * g + j] * inv;
-              if constexpr (GATED) v = gated(v, (&gt[d][g].x)[j]);
+              if constexpr (GATED) v = gated(v, (&gv.x)[j]);
               w4[j] = __bfloat16_as_ushort(__float2bfloat16(v));
             }
             *reinterpret_cast<uint2*>(Op + col) =
