@@ -422,11 +422,12 @@ int gemm_tall_splits(long M, long N, long K, long n_main, long n_tail, int split
 // (gemm_tall_back) than in two, of either kind of tiles; else 0.  The second launch's workgroups start on the CUs that the first ones leave idle: 8192 tokens of
 // a 768 x 3072 layer are 192 and 216 workgroups, 64 and 40 CUs idle.  two_us is the time of the two by the model above (data gradients whose tokens are no
 // multiple of 256 go to the library, which takes as long as these tiles), and the one launch's the end of a list of workgroups, longest first, dealt out to the CUs.
-// Constants fitted to 330 sizes (256 to 9216 tokens, 256 to 6144 outputs, 256 to 4096 inputs; profiles/backward_pairs.txt): what the rule picks takes 23 % less time
-// than two launches on average and 2 % more than the best choice; in one size 11 % more than two (7168 x 3072 x 768 85.7, so 94.9), in one 2 %.
+// Constants fitted to 330 sizes (256 to 9216 tokens, 256 to 6144 outputs, 256 to 4096 inputs; profiles/backward_pairs.txt): what the rule picks takes 21 % less time
+// than two launches on average and 1 % more than the best choice; in one of 257 sizes 2 % more than two (3328 x 5120 x 1024 90.3, so 91.8).  More ranges have to save 2 %: by less than
+// that 7168 x 3072 x 768 went into six, 94.9, where two launches are 85.7 and four ranges 80.2.
 // us, two launches / one: 8192 tokens 768 x 768 40.2 / 34.0, 2304 x 768 76.3 / 70.0, 3072 x 768 99.4 / 87.7, 768 x 3072 106.8 / 97.7; 1326 tokens 768 x 3072 37.4 /
 // 24.0; but 8192 x 4096 x 4096 373 / 436, where 256 x 256 tiles fill the chip.
-constexpr double BACK_TILE = 0.76, BACK_FIXED = 4.0, BACK_MARGIN = 1.05;
+constexpr double BACK_TILE = 0.76, BACK_FIXED = 4.0, BACK_MARGIN = 1.05, BACK_MORE = 0.98;
 int64_t gemm_tall_back_splits(int64_t T, int64_t O, int64_t I, bool bias, double two_us) {
   if (T < 4 * TK || O <= 0 || I <= 0 || O % TM != 0 || I % TN != 0 || (bias && I < 4 * TALL_N)) return 0;
   const long nd = (T + TM - 1) / TM * (I / TALL_N), tiles = O / TM * (I / TALL_N);
@@ -449,7 +450,7 @@ int64_t gemm_tall_back_splits(int64_t T, int64_t O, int64_t I, bool bias, double
     if (d_us >= w_us) deal(nd, d_us), deal(tiles * S, w_us);
     else deal(tiles * S, w_us), deal(nd, d_us);
     const double us = end + (S > 1 ? 4.5 + (double)O * I * S * 8.0 / 7.0e6 : 0.0);
-    if (us < limit) limit = us, best = S;
+    if (us < limit * (best == 0 ? 1.0 : BACK_MORE)) limit = us, best = S;
   }
   return best;
 }

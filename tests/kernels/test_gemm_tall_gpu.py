@@ -266,3 +266,22 @@ def test_layers_take_the_one_launch(tokens, out, inn, bias, monkeypatch):
     pairs = [(x.grad, D @ w.detach().double()), (w.grad, D.t() @ x.detach().double())] + ([(b.grad, D.sum(0))] if bias else [])
     for got, ref in pairs:  # bf16 of fp32 sums: 2^-9 an entry at most, 0.0017 of the norm
         assert float((got.double() - ref).norm() / ref.norm()) < 2.0**-9
+
+
+def test_the_one_launch_is_taken_where_it_is_faster():
+    """The rule against the times that its figures are from."""
+    import re
+    from pathlib import Path
+
+    from llmctl.ops._lib import native
+
+    picks = []
+    for line in (Path(__file__).resolve().parents[2] / "profiles" / "backward_pairs.txt").read_text().splitlines():
+        if m := re.match(r"(\d+) (\d+) (\d+) (\d) \| ([\d.]+) \| (.*)$", line):
+            T, O, I, bias = map(int, m.groups()[:4])
+            one = {int(s): float(t) for s, t in re.findall(r"(\d+):([\d.]+)", m[6])}
+            ranges = native().gemm64_back_splits(T, O, I, bool(bias))
+            if ranges in one:
+                picks.append((float(m[5]), one[ranges]))
+    assert len(picks) >= 250 and all(one <= 1.02 * two for two, one in picks)
+    assert sum(one for _, one in picks) < 0.8 * sum(two for two, _ in picks)
