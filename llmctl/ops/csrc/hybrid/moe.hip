@@ -153,7 +153,8 @@ __host__ __device__ __forceinline__ bool half_tile(int n, int BM) {  // the last
 // weights (>= E) are left out.
 // A thread takes `per` neighbouring copies, so that one pass over them and one scan over the workgroup place them all; a pass for the counts and rounds of 1024 with two
 // barriers each took, us, so: 2048 tokens, 8 experts, top 2 6.5 / 4.7, 3565 9.6 / 5.5; 2031
-// tokens, 32 experts, top 4 10.9 / 7.4.
+// tokens, 32 experts, top 4 10.9 / 7.4; 16384 copies, 8 experts 18.0 / 13.8, 32768 34.0 / 29.6, 65536 63.8 / 65.3, 131072 127 / 136.  (In chunks of 16384, with copies beyond the first
+// read twice as well: 20000 copies 13.3, so 25.2.)
 constexpr int GROUP_KEEP = 16;  // copies a thread keeps in registers between the two passes
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int N, int E, int BM, int* __restrict__ perm,
                                                          int* __restrict__ tiles) {

@@ -83,6 +83,26 @@ def test_wide_tiles_at_their_edges(counts, W, ff, top, act):
         assert bool(((got.double() - want).norm(dim=1) <= 2.0 ** -7 * want.norm(dim=1) + 1e-12).all())
 
 
+@pytest.mark.parametrize("T,top,E", [(8192, 2, 8), (8193, 2, 8), (9000, 2, 9), (16385, 1, 3), (11000, 3, 40), (20000, 2, 8)])
+@pytest.mark.parametrize("form", [1, 2])
+def test_copies_of_more_than_a_chunk(T, top, E, form):
+    """16384 copies are placed at a time, and the wide tiles' lanes hold 64 row tiles; unlike shares, an expert that nobody chose and copies of none between."""
+    from llmctl.ops import hybrid as hops
+
+    W = ff = 256
+    x, _, up, down = _case(T, W, ff, E, "relu2", seed=T)
+    d3 = down.view(W, E, ff).transpose(0, 1)
+    g = torch.Generator().manual_seed(T)
+    share = torch.rand(E + 1, generator=g) + 0.05
+    share[E // 2] = 0.0
+    idx = torch.multinomial(share.expand(T, -1), top, generator=g).int().cuda()
+    w = torch.rand(T, top, generator=g).cuda()
+    got = hops.native_hybrid().moe_experts(x, idx, w, [up], [d3], 0, None, None, form)
+    want = _plain(x, idx.long(), w, up, d3, "relu2", E)
+    # roundings to bf16 (2^-8 at most) of the first product, which the square doubles, of the activation and of the result, whose rows can hang on a few large activations
+    assert bool(((got.double() - want).norm(dim=1) <= 2.0 ** -6 * want.norm(dim=1) + 1e-12).all())
+
+
 def test_tiles_that_pay():
     """The rule of the wide tiles against the times that its figures are from."""
     import re
