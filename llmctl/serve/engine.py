@@ -49,9 +49,8 @@ from .tokenizer import load_tokenizer
 
 log = logging.getLogger("llmctl.serve")
 
-# csrc/dense_prompt.cpp's order; and what its call stands for, unless an engine has its own
+# csrc/dense_prompt.cpp's order
 _LAYER_PARAMS = ("attn_norm_w", "attn_norm_b", "wqkv", "bqkv", "wo", "bo", "mlp_norm_w", "mlp_norm_b", "w_up", "b_up", "w_down", "b_down")
-_LOOP = frozenset(("_norm", "_qkv", "_row_linear", "_mlp", "_reduce"))
 
 
 class InferenceEngine:
@@ -588,7 +587,8 @@ class InferenceEngine:
         in ``prefill_exec``, fed faster.  Returns (the last layer's output, the residual stream), or () where the loop has to run."""
         cfg = self.cfg
         if (type(self) is not InferenceEngine or self.tp != 1 or cfg.norm != "layernorm" or cfg.gated_mlp or cfg.is_moe or self.rope is not None or ops.functional.SKINNY_CONFIGS
-                or not _LOOP.isdisjoint(self.__dict__)):
+                or any(n in self.__dict__ or InferenceEngine.__dict__[n] is not f for n, f in _LOOP_METHODS.items())
+                or any(getattr(ops, n) is not f for n, f in _LOOP_OPS.items())):
             return ()
         layers = self.model.layers
         params = [layer._parameters.get(n) for layer in layers for n in _LAYER_PARAMS]
@@ -1228,3 +1228,8 @@ class InferenceEngine:
         while any(s.status != "finished" for s in seqs):
             self.step()
         return seqs
+
+
+# what a prompt's native call stands for (_prompt_layers): taken only while they are these
+_LOOP_METHODS = {n: InferenceEngine.__dict__[n] for n in ("_norm", "_qkv", "_row_linear", "_mlp", "_reduce")}
+_LOOP_OPS = {n: getattr(ops, n) for n in ("layernorm", "add_layernorm", "decode_linear", "qkv_split_cache", "flash_attention")}

@@ -1,4 +1,4 @@
-"""A prompt's layers from one native call: the same bits as the engine's loop over its layers, at sizes on every route of the products; and who keeps the loop."""
+"""A prompt's layers from one native call: the same bits as the engine's loop over its layers, on every route of the products; and who keeps the loop."""
 import dataclasses
 import json
 
@@ -48,6 +48,36 @@ def test_same_bits_as_the_loop(tmp_path, lens, kw):
     eng._prompt_layers = lambda *a: ()
     for a, b in zip(got, _step(eng, lens)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kw,lens,route", [({}, (100,), "small"), ({}, (1000,), "tiles"), ({}, (1000, 900, 850), "library"),
+                                           (dict(hidden=2048, heads=16, kv_heads=16, ffn=7680), (614,), "apart")])
+def test_routes_of_the_gelu(tmp_path, kw, lens, route):
+    """The up projection on gemm_small, on the prompt tiles, as the library's product with a pass for the GELU, and on the tiles with a pass (where the epilogue costs more than it)."""
+    from llmctl.exec.linear import prompt_forms
+
+    eng = _engine(tmp_path, **kw)
+    x = torch.empty(sum(lens), eng.cfg.hidden, device="cuda", dtype=torch.bfloat16)
+    with torch.inference_mode():
+        form, = prompt_forms(x, ((eng.cfg.ffn, eng.cfg.hidden, True),))
+    assert route == ("small" if form < 0 else "library" if form == 0 else "apart" if form >= 1 << 20 else "tiles")
+    test_same_bits_as_the_loop(tmp_path, lens, kw)
+
+
+def test_patched_methods_and_ops_keep_the_loop(tmp_path, monkeypatch):
+    from llmctl import ops
+    from llmctl.serve.engine import InferenceEngine
+
+    eng = _engine(tmp_path)
+    run = lambda: eng._prompt_layers(torch.randn(64, 768, device="cuda", dtype=torch.bfloat16), torch.full((64,), -1, device="cuda"), None)
+    with torch.inference_mode():
+        assert len(run()) == 2
+        for where, name in ((InferenceEngine, "_mlp"), (InferenceEngine, "_norm"), (ops, "flash_attention"), (ops, "decode_linear")):
+            own = getattr(where, name)
+            with monkeypatch.context() as m:
+                m.setattr(where, name, lambda *a, **k: own(*a, **k))
+                assert not run()
+        assert len(run()) == 2
 
 
 def test_others_keep_the_loop(tmp_path):
