@@ -284,6 +284,8 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
     """``act(x @ w^T (+ b))`` (into ``out`` ``[M, groups, N / groups]``, whose rows and groups may lie apart) on ``gemm_rows`` where it takes it, pays (:func:`rows_form`) and no gradient is wanted of it (the forward of an autograd function, serving); else
     None.  ``act``: 0 none, 1 erf GELU, 2 tanh GELU (without ``out``).  A library product takes the host 24 us, this 9: Lenitar's prompt of 2048 tokens, sixteen of them,
     1198 us, so 1127 (kernels 1190 / 1106); gpt2-125m's of 700 and 300 tokens 2195 / 1870."""
+    if w.dim() != 2:  # (a vector: the library's)
+        return None
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
     code = rows_form(M, N, K, act != 0, eager) if M and type(M * N) is int else 0  # (symbolic and traced sizes are no ints)

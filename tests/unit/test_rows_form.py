@@ -60,3 +60,13 @@ def test_training_under_tensor_parallelism_does_not_ask_for_the_hosts_sake(monke
     tp._fwd_into(w, None)(x, out)
     y = tp._RowSP.apply(x, w, None)
     assert torch.equal(out, y) and torch.allclose(y, x @ w.t(), atol=1e-5) and len(asked) == 2 and "eager" not in asked
+
+
+def test_a_vector_is_a_weight_too():
+    import torch
+
+    from llmctl.ops import hybrid as hops
+
+    x, w = torch.randn(40, 16), torch.randn(16)
+    for f in (hops.linear, hops.odd_linear):
+        assert torch.equal(f(x, w), torch.nn.functional.linear(x, w))
