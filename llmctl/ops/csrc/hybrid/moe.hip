@@ -27,11 +27,11 @@
 // rows an expert and more) or 64 x 64: with few tiles the K loop of every workgroup is a chain of load latencies.  The large tile
 // keeps one LDS buffer (32 KB) so that three workgroups fit a CU; the small one keeps three steps in flight (37 -> 30 us at 65 tokens).
 //
-// Measured, one MI355X, width 2048, 8 gated experts of 1024, top 2 (up / down; weights from HBM):
+// Measured, one MI355X, width 2048, 8 gated experts of 1024, top 2 (up / down, kernel times; all caches written over before each layer):
 //   tokens      16          32         64        128        256        512       1024       2048       4096
-//   us       26 / 14     27 / 14    30 / 16    21 / 11    23 / 13    27 / 15    32 / 20    37 / 24    65 / 39
-// up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from there on what a CU can have in flight (moe_wide.h).  On tiles of 128 x 128, 512 tokens took
-// 38 / 22, 1024 39 / 22, 2048 62 / 36, 4096 97 / 55; 2911 tokens through 8 experts without gates 51 / 46, so 33 / 36.
+//   us       27 / 15     27 / 15    29 / 17    32 / 16    37 / 19    42 / 21    50 / 25    50 / 25    97 / 49
+// up to 64 tokens the bound is the weight stream (67 + 34 MB: 2.5 TB/s), from there on what a CU can have in flight (moe_wide.h).  On tiles of 128 x 128, 512 tokens take
+// 47 / 26, 1024 55 / 30, 2048 67 / 39, 4096 98 / 59.
 #include "expert_rows.h"
 #include "router_rows.h"
 #include "stream_linear.h"
@@ -382,11 +382,12 @@ __global__ __launch_bounds__(256, OCC) void moe_tile_kernel(TileArgs g) {
 #include "moe_wide.h"
 namespace llmctl_hybrid {
 // Whether N copies for E experts run on tiles of up to 288 x 128 (moe_wide.h) rather than on tiles of 128 x 128 or, below 96 rows an expert, 64 x 64: both products' rounds, in
-// units of a K-step of 64 of a round of 128 x 128 tiles (three to a CU).  The experts' rows are taken as random choices spread them.  A round of 256 full tiles counts 0.24 a K-step and
-// 8.5, one of half tiles, behind them, 0.377 and 2.15; 64 x 64 tiles 0.875 a K-step, four to a CU and no whole rounds.  The constants are fitted to the comparison, not to the
-// times, at 1803 sizes (66 to 4096 tokens, widths 512 to 4096, 4 to 64 experts of 256 to 2048, top 1 to 6: profiles/expert_tiles.txt): 737 are taken, in 13 % less time, 27 of them
-// are slower, by 6 % at most (383 tokens of width 512, 8 gated experts of 2048, top 6: 75 / 80 us); 93 % of what the better choice everywhere would give.  By rows per expert alone
-// 94 sizes were more than 5 % slower: 2612 tokens of width 1024, 32 gated experts of 512, top 4 86 / 94, 377 of width 2048, 8 of 256 40 / 51.
+// units of a K-step of 64 of a round of 128 x 128 tiles (three to a CU; the fuller the chip is, the longer: 0.32).  The experts' rows are taken as random choices spread them.
+// A round of 256 full tiles counts 0.42 a K-step and 3.3, one of half tiles, behind them, 0.24 and 2.8, gates 7.3 more (half of it in a half tile); 64 x 64 tiles 1.04 a K-step, four to a CU and no whole
+// rounds.  The constants are fitted to the comparison, not to the times, at 1803 sizes (66 to 4096 tokens, widths 512 to 4096, 4 to 64 experts of 256 to 2048, top 1 to 6:
+// profiles/expert_tiles.txt); fitted to one half of them they do as well on the other.  876 are taken, in 12 % less time; of all 24 are more than 5 % slower than the better choice, and
+// together they take 0.2 % more than with it (1650 tokens of width 1024, 8 experts of 1024 with GELUs, top 6 103 / 114 us).  By rows per expert alone 99 were, 2612 tokens of width 1024, 32 gated experts of 512,
+// top 4 86 / 94, 377 of width 2048, 8 of 256 40 / 51.
 bool moe_wide_pays(int64_t N, int64_t E, int64_t W, int64_t ff, bool glu) {
   if (E < 1 || N < 48 * E || N > INT32_MAX || W % 128 != 0 || ff % 128 != 0 || W < 256 || ff < 256) return false;
   const int B = N >= 96 * E ? 128 : 64;
@@ -397,12 +398,13 @@ bool moe_wide_pays(int64_t N, int64_t E, int64_t W, int64_t ff, bool glu) {
     full += E * p * (row_tiles(n, WIDE_ROWS) - h), half += E * p * h, other += E * p * row_tiles(std::max(n, 1), B);
   }
   double wide = 0.0, narrow = 0.0;
-  for (const auto& [cols, K] : {std::pair{glu ? 2 * ff : ff, W}, {W, ff}}) {
-    const double steps = (double)K / 64, nt = (double)cols / 128, cf = 0.24 * steps + 8.5, ch = 0.377 * steps + 2.15;
+  for (const bool down : {false, true}) {
+    const int64_t cols = down ? W : glu ? 2 * ff : ff, K = down ? ff : W;
+    const double gates = glu && !down ? 7.3 : 0.0, steps = (double)K / 64, nt = (double)cols / 128, cf = 0.42 * steps + 3.3 + gates, ch = 0.24 * steps + 2.8 + gates / 2;
     const double span = std::ceil(full * nt / 256 - 0.04) * cf, left = half * nt * ch / 256 - 0.85 * std::max(0.0, span - full * nt * cf / 256);
     wide += span + (left > 0.0 ? std::ceil(left / ch - 0.04) * ch : 0.0);
     const double items = other * std::ceil((double)cols / B);
-    narrow += steps * (B == 128 ? std::max(1.0, std::ceil(items / 768 - 0.1)) : 0.875 * items / 1024);
+    narrow += steps * (B == 128 ? std::max(1.0, std::ceil(items / 768 - 0.1)) + 0.32 * items / 768 : 1.04 * items / 1024);
   }
   return wide < narrow;
 }

@@ -4,9 +4,9 @@
 // Row tiles have 256 rows but the last one of an expert, which takes what is left, 33 to 288: a power of two of tokens gives an expert a multiple of 256 copies, give or
 // take the square root, and with tiles of 256 half of the experts had one more tile, of a few rows (2048 tokens, 8 experts, top 2: 16 row tiles for 20).  Tiles of at
 // most 128 rows are dealt out last, to the CUs that are done first.
-// us, tiles of 128 x 128 / these: width 2048, 8 experts of 1024, up (gated) and down, 459 tokens 36.5, 21.7 / 25.4, 15.0, 1021 46.9, 27.0 / 34.8, 20.3, 3035 83, 47 / 66, 39;
-// without gates 3011 tokens 49, 46 / 33, 36; width 4096, 8 of 1408, gated, 1511 tokens 118, 65 / 100, 54; 32 experts, width 1024, 1699 tokens 32, 29 / 26, 24, but gated
-// 2612 tokens, a third of whose tiles start a new round, 70, 39 / 78, 39 (which moe_wide_pays leaves to the others).
+// us, tiles of 128 x 128 / these, kernel times after the caches are written over: width 2048, 8 experts of 1024, up (gated) and down, 459 tokens 47, 26 / 39, 20, 1021 56, 31 / 50, 24, 3035 86, 49 /
+// 81, 42; erf GELUs 2911 tokens 54, 41 / 50, 42, 3011 55, 48 / 54, 42; width 4096, 8 of 1408, gated, 1511 tokens 132, 70 / 136, 58; 32 experts of 512, width 1024, top 4, 1699 tokens 28, 23 / 28, 22, but
+// gated 2612 tokens, whose tiles make two rounds of one and a half, 43, 28 / 57, 30 (moe_wide_pays leaves them to the others).
 #pragma once
 #include "wide_tiles.h"
 

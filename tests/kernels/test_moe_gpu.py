@@ -111,14 +111,15 @@ def test_tiles_that_pay():
     from llmctl.ops import hybrid as hops
 
     pays = hops.native_hybrid().moe_wide_pays
-    picks = []
+    picks, taken, best = [], 0.0, 0.0
     for line in (Path(__file__).resolve().parents[2] / "profiles" / "expert_tiles.txt").read_text().splitlines():
         if m := re.match(r"(\d+) (\d+) (\d+) (\d+) (\d+) (\w+) \| ([\d.]+) \| ([\d.]+)$", line):
             T, W, ff, E, top = map(int, m.groups()[:5])
-            if pays(T * top, E, W, ff, m[6] == "swiglu"):
-                picks.append((float(m[7]), float(m[8])))
-    assert len(picks) >= 700 and all(wide <= 1.07 * other for other, wide in picks) and sum(wide > other for other, wide in picks) <= 30
-    assert sum(wide for _, wide in picks) < 0.88 * sum(other for other, _ in picks)
+            other, wide = float(m[7]), float(m[8])
+            own = wide if pays(T * top, E, W, ff, m[6] == "swiglu") else other
+            picks.append(own / min(other, wide))
+            taken, best = taken + own, best + min(other, wide)
+    assert len(picks) == 1803 and max(picks) < 1.2 and sum(p > 1.05 for p in picks) <= 25 and taken < 1.0025 * best
     assert not any(pays(N, E, W, ff, True) for N, E, W, ff in ((0, 8, 2048, 1024), (383, 8, 2048, 1024), (4096, 8, 2048, 1000), (4096, 8, 2040, 1024), (4096, 8, 128, 1024), (4096, 0, 2048, 1024)))
 
 
