@@ -251,32 +251,30 @@ def _act_us(M: int, N: int) -> float:
 
 
 def _few_rows_form(M: int, N: int, K: int, act: bool, eager: bool) -> int:
-    """:func:`rows_form` of up to 1024 rows.  Their tiles are few, so K is cut into ranges of 256 at least.  The model of these launches is a fit to their times at 1211 sizes
-    (12 % off in the root mean square), the library's a lower bound, for its own times jump by a half from one size to the next (256 x 6144 x 2048 27.4, 288 rows 18.8): a pick is to be
-    faster wherever they fall (``profiles/few_rows_products.txt``, ``short_prompt_products.txt`` and ``prompt_products.txt``).  334 of the sizes are taken, in 19 % less time; six of these take longer,
-    291 x 256 x 8192 14.2 / 15.3 the longest of its own.
-    ``eager``: a step's launches are the host's time, and a library product takes it 24 us, this 9 (13 with the pass that adds the ranges): of up to 6 Mi outputs and 36 us also what may take
-    the chip a few us longer, 7 and a quarter of the library's lower bound by the model, 6.3 at most of the sizes timed (200 x 6144 x 2048 16.7 / 23.0; all 1000 that are taken, in 10 % less).
-    us, library / here: 600 x 2048 x 8192 47 / 36, 128 x 4096 x 11008 79 / 46; left to the library 900 x 2048 x 2048 16.3 / 20.3, 288 x 32000 x 2048 68 / 81, 128 x 12288 x 4096 45 / 53; for the
-    host's sake 256 x 2048 x 2048 11.3 / 14.9.  Prompts, us a step, with every product the library's / here: dumazen width 2048 100 tokens 1387 / 1118, 450 1331 / 1110, 900 tokens
-    1440 / 1380; lenitar 300 982 / 880; malinex 200 948 / 809."""
-    cols, stream = -(-N // 128), 4.0 + N * K * 2e-6 / 2.1
-    best, code = 1e9, 0
+    """:func:`rows_form` of up to 1024 rows.  Their tiles are few, so K is cut into ranges of 256 at least: rounds of 256 workgroups, a K-tile of 64 1.06 us on tiles of 256 rows and 0.82 on those of
+    128, 3.1 us and the fp32 sums' bytes for the pass that adds the ranges, and the weight's stream at the least; against the library's products, which K beyond 4096 makes slow.  The
+    constants are fitted to the choice, not to either time, at 1200 sizes (fitted to one half of them they do as well on the other; ``profiles/few_rows_products.txt``, ``short_prompt_products.txt``
+    and ``prompt_products.txt``): the library's own times jump by a half from one size to the next (256 x 6144 x 2048 27.4, 288 rows 18.8).  573 of the sizes timed are taken, in 18 % less
+    time; 38 of these take longer, by 3.6 us at most but for one (579 x 8448 x 6272 76 / 85), nine by more than a tenth (201 x 256 x 6144 11.2 / 14.0).  All sizes together take 3 % more than with
+    the better choice everywhere, and 9 % less than in the library.
+    ``eager``: a step's launches are the host's time, and a library product takes it 24 us, this 9 (13 with the pass that adds the ranges): of up to 6 Mi outputs and 38 us also what may take
+    the chip a few us longer, 8 and 0.3 of the library's time by the model, 5.2 at most of the sizes timed but for that one (350 x 3712 x 2048 16.3 / 21.5; all 1003 that are taken, in 11 % less).
+    us, library / here: 600 x 2048 x 8192 47 / 36, 128 x 4096 x 11008 79 / 46, 288 x 8256 x 2048 29 / 22; left to the library 900 x 2048 x 2048 16.3 / 20.3, 288 x 32000 x 2048 68 / 81, 128 x 12288 x
+    4096 45 / 53; for the host's sake 256 x 2048 x 2048 11.3 / 14.9.  Prompts, us a step, with every product the library's / here: dumazen width 2048 100 tokens 1387 / 1118, 450 1331 / 1110; lenitar 300
+    982 / 880; malinex 200 948 / 809."""
+    cols, best, code = -(-N // 128), 1e9, 0
     for splits in (1, 2, 3, 4, 6, 8, 12, 16):
         if splits > 1 and (splits > K // 256 or splits * cols * _tile_rows(M, 1) > 512):
             break
-        kt, add = K / 64 / splits, 0.0 if splits == 1 else 4.6 + splits * M * N * 4e-6 / 2.94
-        for form, (empty, full, fixed) in ((1, (0.626, 0.39, 4.9)), (2, (0.448, 0.237, 3.85))):
-            t = _rounds_us(splits * cols * _tile_rows(M, form), kt, empty, full, fixed + (act * _ACT_TILE[form] if splits == 1 else 0.0)) + add
+        for form, step in ((1, 1.06), (2, 0.82)):
+            rounds = -(-splits * cols * _tile_rows(M, form) // _CUS)
+            t = rounds * (K / 64 / splits * step + (act * _ACT_TILE[form] if splits == 1 else 0.0)) + (3.1 + splits * M * N * 4e-6 if splits > 1 else 0.0)
             if t < best:
                 best, code = t, form + 4 * (splits - 1)
-    best, gflop = max(best, stream), 2e-9 * M * N * K
-    if K < 8192:
-        library = 7.7 + 0.1 * N * K * 2e-6 + 0.96 * gflop
-    else:  # (few tiles and long chains there too: it leaves the chip idle until some 40 GFLOP)
-        library = min(13.5 + 2.9 * gflop, 60.0 + 0.85 * gflop)
-    library += act * _act_us(M, N)
-    return code if best < library or (eager and M * N <= 6 << 20 and best <= min(1.25 * library + 7.0, 36.0)) else 0
+    mb, gflop = N * K * 2e-6, 2e-9 * M * N * K
+    best = max(best, mb / 1.8)
+    library = min(7.2 + 0.22 * mb + 0.88 * gflop + 20.0 * max(0, K - 4096) / 1024, 75.0 + 0.68 * gflop) + act * _act_us(M, N)
+    return code if best < library or (eager and M * N <= 6 << 20 and best <= min(1.3 * library + 8.0, 38.0)) else 0
 
 
 def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None, act: int = 0,
@@ -321,10 +319,7 @@ def _prompt_form(M: int, N: int, K: int, act: bool) -> Optional[int]:
     if small_pays("eager", M, N, K):
         return -1
     code = rows_form(M, N, K, act, True)
-    if not code and act:
-        code = rows_form(M, N, K, False, True)
-        code = code and code + (1 << 20)
-    return None if not code and fwd64_pick(M, N, K) else code
+    return None if not code and (fwd64_pick(M, N, K) or (act and rows_form(M, N, K, False, True))) else code
 
 
 def prompt_forms(x: torch.Tensor, sizes) -> Optional[List[int]]:
