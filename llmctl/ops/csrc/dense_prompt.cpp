@@ -26,11 +26,8 @@ bool takes(const at::Tensor& t, at::IntArrayRef sizes, c10::Device dev) {
   return t.defined() && t.device() == dev && t.scalar_type() == at::kBFloat16 && t.sizes() == sizes && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
-constexpr int64_t ACT_APART = 1 << 20;
-
-// form: -1 gemm_small, 0 the library, else gemm_rows' (tiles + 4 (ranges - 1), ACT_APART: the activation in a pass of its own); act: 0 none, 2 tanh GELU
+// form: -1 gemm_small, 0 the library, else gemm_rows' (tiles + 4 (ranges - 1)); act: 0 none, 2 tanh GELU
 at::Tensor product(const at::Tensor& x, const at::Tensor& w, const at::Tensor& b, int64_t form, int64_t act) {
-  if (form >= ACT_APART) return gelu_fwd(product(x, w, b, form - ACT_APART, 0));
   if (form > 0) return gemm_rows(x, w, b, form & 3, (form >> 2) + 1, act);
   if (form < 0) {
     at::Tensor y = at::empty({x.size(0), w.size(0)}, x.options());

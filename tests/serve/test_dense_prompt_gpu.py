@@ -50,18 +50,17 @@ def test_same_bits_as_the_loop(tmp_path, lens, kw):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("kw,lens,route", [({}, (100,), "small"), ({}, (1000,), "tiles"), ({}, (1000, 900, 850), "library"),
-                                           (dict(hidden=2048, heads=16, kv_heads=16, ffn=7680), (614,), "apart")])
-def test_routes_of_the_gelu(tmp_path, kw, lens, route):
-    """The up projection on gemm_small, on the prompt tiles, as the library's product with a pass for the GELU, and on the tiles with a pass (where the epilogue costs more than it)."""
+@pytest.mark.parametrize("lens,route", [((100,), "small"), ((1000,), "tiles"), ((1000, 900, 850), "library")])
+def test_routes_of_the_gelu(tmp_path, lens, route):
+    """The up projection on gemm_small, on the prompt tiles, and as the library's product with a pass for the GELU."""
     from llmctl.exec.linear import prompt_forms
 
-    eng = _engine(tmp_path, **kw)
+    eng = _engine(tmp_path)
     x = torch.empty(sum(lens), eng.cfg.hidden, device="cuda", dtype=torch.bfloat16)
     with torch.inference_mode():
         form, = prompt_forms(x, ((eng.cfg.ffn, eng.cfg.hidden, True),))
-    assert route == ("small" if form < 0 else "library" if form == 0 else "apart" if form >= 1 << 20 else "tiles")
-    test_same_bits_as_the_loop(tmp_path, lens, kw)
+    assert route == ("small" if form < 0 else "tiles" if form else "library")
+    test_same_bits_as_the_loop(tmp_path, lens, {})
 
 
 def test_patched_methods_and_ops_keep_the_loop(tmp_path, monkeypatch):
