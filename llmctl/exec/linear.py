@@ -262,6 +262,9 @@ def _few_rows_form(M: int, N: int, K: int, act: bool, eager: bool) -> int:
     us, library / here: 600 x 2048 x 8192 47 / 36, 128 x 4096 x 11008 79 / 46, 288 x 8256 x 2048 29 / 22; left to the library 900 x 2048 x 2048 16.3 / 20.3, 288 x 32000 x 2048 68 / 81, 128 x 12288 x
     4096 45 / 53; for the host's sake 256 x 2048 x 2048 11.3 / 14.9.  Prompts, us a step, with every product the library's / here: dumazen width 2048 100 tokens 1387 / 1118, 450 1331 / 1110; lenitar 300
     982 / 880; malinex 200 948 / 809."""
+    # Of nine sizes of as many outputs six are the library's, by 4 to 33 %; three of K up to 512 would be faster here (1000 x 11008 x 512 43 / 27) and stay where the rule of large products had them.
+    if not act and M * N > 10 << 20:
+        return 0
     cols, best, code = -(-N // 128), 1e9, 0
     for splits in (1, 2, 3, 4, 6, 8, 12, 16):
         if splits > 1 and (splits > K // 256 or splits * cols * _tile_rows(M, 1) > 512):

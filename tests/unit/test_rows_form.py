@@ -53,7 +53,7 @@ def test_what_the_host_saves_costs_the_chip_little():
     assert sum(own for *_, own in picks) < 0.9 * sum(library for *_, library, _ in picks)
 
 
-@pytest.mark.parametrize("M,N,K", [(900, 2048, 2048), (450, 3712, 2048), (350, 5136, 2048), (288, 6144, 2048), (288, 5136, 2048), (288, 32000, 2048), (100, 4096, 4096), (200, 8192, 2048)])
+@pytest.mark.parametrize("M,N,K", [(900, 2048, 2048), (450, 3712, 2048), (350, 5136, 2048), (288, 6144, 2048), (288, 5136, 2048), (288, 32000, 2048), (100, 4096, 4096), (200, 8192, 2048), (1000, 11008, 512)])
 def test_the_librarys(M, N, K):
     """(288 x 32000 x 2048 is more than the host's sake allows)"""
     assert L.rows_form(M, N, K) == 0 and (N < 32000 or L.rows_form(M, N, K, False, True) == 0)
