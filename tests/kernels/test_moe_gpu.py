@@ -85,8 +85,8 @@ def test_wide_tiles_at_their_edges(counts, W, ff, top, act):
 
 @pytest.mark.parametrize("T,top,E", [(8192, 2, 8), (8193, 2, 8), (9000, 2, 9), (16385, 1, 3), (11000, 3, 40), (20000, 2, 8)])
 @pytest.mark.parametrize("form", [1, 2])
-def test_copies_of_more_than_a_chunk(T, top, E, form):
-    """16384 copies are placed at a time, and the wide tiles' lanes hold 64 row tiles; unlike shares, an expert that nobody chose and copies of none between."""
+def test_more_copies_than_the_registers_hold(T, top, E, form):
+    """The grouping keeps 16384 copies in registers and reads the rest again, and the wide tiles' lanes hold 64 row tiles; unlike shares, an expert that nobody chose and copies of none between."""
     from llmctl.ops import hybrid as hops
 
     W = ff = 256
