@@ -3,7 +3,7 @@
 // A few hundred rows are 16 to 128 tiles, and a tile's K-tiles from HBM take a workgroup 0.5 to 0.8 us each whatever the others do (the lines that one CU can have on
 // their way): such products are cut into ranges of K, one workgroup each, whose fp32 sums gemm_rows_sum adds in the order of K.
 // us, one range / the best: 128 x 4096 x 11008 124 / 46 (2 TB/s), 200 x 2048 x 2048 19.0 / 13.7 (the adding pass and its launch are 6 of them), 200 x 2048 x 8192 68.7 / 22.9.
-// GELUs in the epilogue: 3.9 us a tile of 256 rows, which nothing overlaps, so large products leave them to a pass (3379 x 8192: 27 us).
+// GELUs in the epilogue: 3.9 us a tile of 256 rows, which nothing overlaps, so large products leave them to a pass (3379 x 8192: 21 us).
 //
 // y's columns may lie in groups apart (a latent prompt's keys and values beside a shared rotary key: the copy into place took 9.4 us for 2048 tokens of 16 heads).
 // Tiles of 256 rows, the last one 33 to 288 (a few rows more are no tile of their own), or of 128; which, and whether at all, rows_form of exec/linear.py says.
