@@ -23,7 +23,9 @@ step.  The down projection's data gradient can carry the SwiGLU backward in its 
 
 from __future__ import annotations
 
+import contextlib
 import functools
+import threading
 from typing import Callable, List, Optional, Tuple
 
 import torch
@@ -114,6 +116,25 @@ def forward_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] =
     return F.linear(x, w, b)
 
 
+class _Steps(threading.local):
+    recorded = False
+
+
+_steps = _Steps()
+
+
+@contextlib.contextmanager
+def recorded_step():
+    """This thread's products are those of a step that is recorded, or of the eager ones ahead of the recording: launches that the host does not feed, so the ``eager`` rules take
+    nothing for its sake.  Said by who records, not asked of the stream: a recording has to take the routes of the steps ahead of it, where the library makes its handle and loads its kernels (a
+    library product that a recording is the first to call ends the process)."""
+    was, _steps.recorded = _steps.recorded, True
+    try:
+        yield
+    finally:
+        _steps.recorded = was
+
+
 @functools.lru_cache(maxsize=4096)
 def small_pays(layout: str, M: int, N: int, K: int, bias: bool = False) -> bool:
     """Is ``gemm_small`` (csrc/gemm_small.hip) the fastest form of this product of a training step?  ``fwd``: M tokens, N outputs; ``dgrad``: K
@@ -178,7 +199,7 @@ def small_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = N
     M = x.numel() // K if K and x.shape[-1] == K else 0
     if not M or type(M * N) is not int or not small_pays(layout, M, N, K) or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
         return None  # (symbolic and traced sizes are no ints)
-    if layout == "eager" and not small_pays("fwd", M, N, K) and torch.cuda.is_current_stream_capturing():
+    if layout == "eager" and not small_pays("fwd", M, N, K) and _steps.recorded:
         return None
     if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not x.is_contiguous() or _any_autocast()
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad or (b is not None and b.requires_grad)))
@@ -199,7 +220,7 @@ def small_linear_f32(x: torch.Tensor, w: torch.Tensor) -> Optional[torch.Tensor]
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or type(x.shape[0]) is not int or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
         return None
     M, (N, K) = x.shape[0], w.shape
-    if (M * N > 2 << 20 or not small_pays("eager", M, N, K) or torch.cuda.is_current_stream_capturing() or _any_autocast() or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
+    if (M * N > 2 << 20 or not small_pays("eager", M, N, K) or _steps.recorded or _any_autocast() or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
             or _forward_ad._current_level >= 0 or torch.compiler.is_compiling() or not _small_ok("fwd", M, N, K, x, w)):
         return None
     y = torch.empty(M, N, dtype=torch.float32, device=x.device)
@@ -289,7 +310,7 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
         return None
     N, K = w.shape
     M = x.numel() // K if K and x.shape[-1] == K else 0
-    code = rows_form(M, N, K, act != 0, eager) if M and type(M * N) is int else 0  # (symbolic and traced sizes are no ints)
+    code = rows_form(M, N, K, act != 0, eager and not _steps.recorded) if M and type(M * N) is int else 0  # (symbolic and traced sizes are no ints)
     if not code or _calls_are_seen() or not w.is_cuda or knobs().fwd64 != "auto":
         return None
     if (type(x) is not torch.Tensor or _is_legacy_batched(x) or not (x.dim() == 2 or x.is_contiguous()) or _any_autocast()
@@ -300,10 +321,6 @@ def rows_linear(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = No
     if (not _small_ok("fwd", M, N, K, x2, w) or not (b is None or (_small_bias(b, N) and b.data_ptr() & 15 == 0))
             or 512 * x2.stride(0) >= 1 << 30 or 512 * w.stride(0) >= 1 << 30):
         return None
-    if eager and M <= 1024 and torch.cuda.is_current_stream_capturing():
-        code = rows_form(M, N, K, act != 0)
-        if not code:
-            return None
     if out is not None:
         if not (type(out) is torch.Tensor and out.dtype is torch.bfloat16 and out.shape[2] & 7 == 0 and out.stride(2) == 1 and out.stride(0) & 7 == 0
                 and out.stride(1) & 7 == 0 and out.data_ptr() & 15 == 0):
@@ -331,7 +348,7 @@ def prompt_forms(x: torch.Tensor, sizes) -> Optional[List[int]]:
     if (type(x) is not torch.Tensor or M <= 32 or type(M) is not int or not x.is_cuda or x.dtype is not torch.bfloat16 or _calls_are_seen() or _any_autocast()
             or _is_legacy_batched(x) or _is_wrapped(x) or torch.is_grad_enabled() or _forward_ad._current_level >= 0 or torch.compiler.is_compiling()
             or kn.fwd64 != "auto" or kn.skinny_gemm != "auto" or not _gemm64_enabled() or GEMM64_CONFIGS or GEMM64_SHAPE_CONFIGS or not use_native(x)
-            or torch.cuda.is_current_stream_capturing()):
+            or _steps.recorded or torch.cuda.is_current_stream_capturing()):
         return None
     forms = [_prompt_form(M, *s) for s in sizes]
     return None if None in forms else forms

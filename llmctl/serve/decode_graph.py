@@ -22,6 +22,7 @@ from typing import Callable, Dict, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from llmctl.exec.linear import recorded_step
 from llmctl.utils.env import graph_capture_gc_guard
 
 WARM_STEPS = 2  # eager steps of a shape before it is captured
@@ -82,7 +83,7 @@ class DecodeGraph:
     def capture(self, model, cache, pool) -> None:
         """Record the step.  Nothing runs, so a failure (raised) leaves caches and states as they were."""
         g = torch.cuda.CUDAGraph()
-        with _capturing, graph_capture_gc_guard(collect=False), torch.cuda.stream(_capture_stream(self.buf.device)):
+        with _capturing, recorded_step(), graph_capture_gc_guard(collect=False), torch.cuda.stream(_capture_stream(self.buf.device)):
             # other threads go on working meanwhile: only this thread's calls are held to what a capture allows
             g.capture_begin(pool=pool, capture_error_mode="thread_local")
             try:
@@ -149,6 +150,10 @@ class GraphTable:
         """Whether the next step of ``shape`` may be replayed or recorded."""
         e = self._shapes.get(shape, 0)
         return e is not None and (not isinstance(e, int) or e >= WARM_STEPS)
+
+    def warming(self, shape: Tuple[int, int]) -> bool:
+        """Whether ``shape`` is to be recorded after some more eager steps."""
+        return isinstance(self._shapes.get(shape), int)
 
     def step(self, shape: Tuple[int, int], record: Callable[[Tuple[int, int]], Optional[DecodeGraph]]) -> Optional[DecodeGraph]:
         """The graph that runs the next step of ``shape``; None: it runs eagerly.  ``record(shape)``: its graph, or None where it

@@ -23,6 +23,7 @@ prompts), and sampled with a host sync per request per token.  Here:
 
 from __future__ import annotations
 
+import contextlib
 import logging
 import math
 import time
@@ -35,7 +36,7 @@ import torch.nn.functional as F
 from llmctl import ops
 from llmctl.config.knobs import use as use_knobs
 from llmctl.io.artifact import load_model
-from llmctl.exec.linear import prompt_forms
+from llmctl.exec.linear import prompt_forms, recorded_step
 from llmctl.models import DecoderLM
 from llmctl.models.transformer import DecoderLayer
 from llmctl.ops._lib import native
@@ -309,17 +310,18 @@ class InferenceEngine:
         """One decode step of a hybrid-mixer model: the first steps of a shape run eagerly, then its captured graph is
         replayed (:mod:`llmctl.serve.decode_graph`).  ``ids_on_device``: the rows' input tokens as a device tensor."""
         n = len(dp["positions"])
-        g = None
+        g, shape = None, (n, 1 << max(int(max(dp["ctx"])) - 1, 0).bit_length() if n else 0)
         if self._decode_capture and n and np.shape(dp["bt"])[1:] == (self.max_blocks_per_seq,):  # (tables of another width: eagerly)
             w = self._weights_key()
             if w != self._weights_seen:
                 self.release_graphs()
                 self._weights_seen = w
-            g = self._decode_graphs.step((n, 1 << max(int(max(dp["ctx"])) - 1, 0).bit_length()), self._record_decode)
+            g = self._decode_graphs.step(shape, self._record_decode)
         if g is None:
             if ids_on_device is not None:
                 dp = dict(dp, ids=ids_on_device.tolist())
-            return self._hybrid_exec(None, dp, count=count)
+            with recorded_step() if self._decode_graphs.warming(shape) else contextlib.nullcontext():
+                return self._hybrid_exec(None, dp, count=count)
         limit = getattr(self.model, "position_limit", None)
         if limit is not None and max(dp["positions"]) >= limit:
             raise ValueError(f"position {max(dp['positions'])} is beyond the model's {limit} learned positions")
@@ -856,12 +858,12 @@ class InferenceEngine:
         bufs = self._static(nb)
         s = torch.cuda.Stream(device=self.device)
         s.wait_stream(torch.cuda.current_stream(self.device))
-        with torch.cuda.stream(s):
+        with recorded_step(), torch.cuda.stream(s):
             for _ in range(2):  # warm-up (allocator / lazy init) outside the graph
                 self._graph_body(bufs)
         torch.cuda.current_stream(self.device).wait_stream(s)
         g = torch.cuda.CUDAGraph()
-        with graph_capture_gc_guard(), torch.cuda.graph(g):
+        with recorded_step(), graph_capture_gc_guard(), torch.cuda.graph(g):
             self._graph_body(bufs)
         self._graphs[nb] = (g, bufs)
 

@@ -383,3 +383,33 @@ def test_a_step_gives_the_same_bits_captured_or_not(name, cut):
         assert ((a - b).norm(dim=1) <= 2.0**-7 * b.norm(dim=1)).all()
     g.release()
     e.close()
+
+
+@pytest.mark.parametrize("name,rows", [("lenitar-w1024-l4", 33), ("malinex-w2048-l3-h16-g4-e4", 64), ("dumazen-w2048-l3-h16-g4", 64)])
+def test_a_recording_calls_no_library_product_first(name, rows, monkeypatch):
+    """More than 32 rows, whose products go by size: what the recorded step has the library do, the eager steps ahead of it did (it makes its handle and loads its kernels there)."""
+    from llmctl.serve.engine import InferenceEngine
+    from llmctl.serve.scheduler import PrefillChunk
+
+    e = InferenceEngine(name, device="cuda", max_batch_size=rows, num_kv_blocks=rows + 1, block_size=16, max_model_len=16, dtype=torch.bfloat16, prefix_caching=False, seed=3)
+    a, b = torch.ones(64, 256, device="cuda", dtype=torch.bfloat16), torch.ones(256, 256, device="cuda", dtype=torch.bfloat16)
+    torch.nn.functional.linear(a, b), torch.nn.functional.linear(a, b, b[0])  # (its handle, so that this test ends in any case)
+    seqs = [e.open_sequence([1 + i, 2, 3, 4, 5]) for i in range(rows)]
+    e.prefill([PrefillChunk(s, 0, 5) for s in seqs])
+    for s in seqs:
+        e.scheduler.computed(s, 5)
+    calls, lib = {False: set(), True: set()}, torch.nn.functional.linear
+
+    def linear(x, w, *rest):
+        calls[torch.cuda.is_current_stream_capturing()].add((tuple(x.shape), tuple(w.shape)))
+        return lib(x, w, *rest)
+
+    monkeypatch.setattr(torch.nn.functional, "linear", linear)
+    for t in range(3):  # contexts of 6 to 8: one shape
+        for s in seqs:
+            e.scheduler.extend(s, [6 + t])
+            s._decode_slot = int(e.kv.slots(s.seq_id, s.num_tokens - 1, 1)[0])
+        e.decode(seqs)
+        for s in seqs:
+            e.scheduler.computed(s, 1)
+    assert len(e._decode_graphs) == 1 and calls[True] and calls[True] <= calls[False]

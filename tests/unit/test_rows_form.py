@@ -81,3 +81,47 @@ def test_a_vector_is_a_weight_too():
     x, w = torch.randn(40, 16), torch.randn(16)
     for f in (hops.linear, hops.odd_linear):
         assert torch.equal(f(x, w), torch.nn.functional.linear(x, w))
+
+
+def test_a_recording_takes_the_routes_of_the_steps_ahead_of_it(monkeypatch):
+    """A library product that a recording is the first to call ends the process: the stream's state moves no product, and who records says so for the steps ahead too."""
+    import threading
+    import types
+
+    import torch
+
+    ran = []
+    fake = types.SimpleNamespace(gemm_rows=lambda x, w, b, form, splits, act: ran.append((form, splits)) or torch.empty(x.shape[0], w.shape[0]),
+                                 gemm_small=lambda x, w, y, *a: ran.append("small"))
+    monkeypatch.setattr(L, "native", lambda: fake)
+    monkeypatch.setattr(L, "_small_ok", lambda *a: True)
+
+    def routes(M, N, K):
+        x = torch.empty(M, K)
+        w = types.SimpleNamespace(shape=(N, K), dim=lambda: 2, is_cuda=True, requires_grad=False, stride=lambda i: K)
+        got = []
+        for f in (lambda: L.rows_linear(x, w), lambda: L.small_linear(x, w, None, "eager"), lambda: L.small_linear_f32(x, w)):
+            ran.clear()
+            got.append((f() is not None, *ran))
+        return got
+
+    moved = 0
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    with torch.no_grad():
+        for M, N, K in ((33, 3072, 1024), (40, 2048, 2048), (100, 1024, 1024), (256, 2048, 2048), (300, 768, 768), (300, 3072, 768), (1500, 1024, 512), (2048, 2048, 2048)):
+            plain = routes(M, N, K)
+            monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+            assert routes(M, N, K) == plain
+            with L.recorded_step():
+                recorded, other = routes(M, N, K), []
+                t = threading.Thread(target=lambda: other.append(L._steps.recorded))
+                t.start(), t.join()
+                assert other == [False]
+            monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+            with L.recorded_step():
+                assert routes(M, N, K) == recorded
+            assert routes(M, N, K) == plain
+            code = L.rows_form(M, N, K)
+            assert recorded[0] == ((True, (code & 3, (code >> 2) + 1)) if code else (False,)) and recorded[1][0] == L.small_pays("fwd", M, N, K) and not recorded[2][0]
+            moved += recorded != plain
+    assert moved >= 4
